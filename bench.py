@@ -102,9 +102,6 @@ def gemm_flops(label):
     return 2.0 * H * M * N * K * gemm_group(label)
 
 
-N_CUS = 256
-
-
 def attention_flops(label, cfg):
     """Algorithmic flops of the fused attention thunks: the causal half of Q K^T and P V in the
     forward pass (2 products of S^2/2 x Dh per head), of dV, dP, dQ and dK in the adjoint (4); what the
@@ -119,58 +116,35 @@ def gemm_dims(label):
     return (m.group(2) == "T", m.group(3) == "T") + tuple(int(m.group(i)) for i in (4, 5, 6, 7))
 
 
-def plan_tokens_product(M, N):
-    """Mirror of plan_tokens_product in csrc/gemm_mfma.hip: (tile, columns of the first launch)."""
-    best, best_cost = (4, N), None
-    for tile, bn, round_cost in ((4, 128, 32768), (5, 256, 54613)):
-        tiles_m, tiles_n = (M + 255) // 256, (N + bn - 1) // bn
-        total = tiles_m * tiles_n
-        full = total // N_CUS
-        cols_main = full * N_CUS // tiles_m
-        rest = tiles_m * (tiles_n - cols_main)
-        if full >= 1 and cols_main < tiles_n and rest * bn * 4 <= N_CUS * 128:
-            cost, main_cols = full * round_cost + 12288, cols_main * bn
-        else:
-            cost, main_cols = -(-total // N_CUS) * round_cost, N
-        if best_cost is None or cost < best_cost:
-            best, best_cost = (tile, main_cols), cost
-    return best
+def gemm_plan(M, N, K):
+    """((tile rows, columns) of the first launch, launches) of a dense product of 16-byte aligned operands."""
+    import ctypes as C
+    from cacti_amd import ffi
+    out = (C.c_int64 * 6)()
+    ffi.call("cacti_hip_gemm_plan", M, N, K, 1, out)
+    return (out[0], out[1]), out[5]
 
 
-TILE_ARGS = {0: "128, 128, 2, 2, 8, false, 2, 2, false", 4: "256, 128, 4, 2, 8, false, 1, 3, true",
-             5: "256, 256, 2, 4, 8, false, 1, 2, true", 6: "256, 192, 4, 2, 8, false, 1, 2, true"}
+TILE_ARGS = {(64, 64): "64, 64, 2, 2, 8, false, 1, 4, true", (128, 64): "128, 64, 2, 2, 8, false, 1, 3, true",
+             (128, 128): "128, 128, 2, 4, 8, false, 1, 3, true", (256, 128): "256, 128, 4, 2, 8, false, 1, 3, true",
+             (256, 192): "256, 192, 4, 2, 8, false, 1, 2, true", (256, 256): "256, 256, 2, 4, 8, false, 1, 2, true"}
 
 
 def kernel_symbol(label):
     """Name of the HIP kernel instantiation a dense GEMM label runs on (its first launch), as
-    rocprofv3 prints it.  The tile choice mirrors gemm_mfma_launch for 16-byte aligned operands
-    and K % 64 == 0: with an output of at least 1024 x 1024 and one block, A not transposed runs
-    256 x 128 or 256 x 256 / 8 waves by plan_tokens_product, A transposed 256 x 256 / 8 waves from
-    2048 x 2048 outputs on (256 x 192 where that fills the CUs markedly better), all with
-    direct-to-LDS loads; everything else 128 x 128 / 4 waves through registers."""
+    rocprofv3 prints it, for 16-byte aligned operands."""
     ta, tb, H, M, N, K = gemm_dims(label)
-    tile = 0
-    if H == 1 and M >= 1024 and N >= 1024:
-        if not ta:
-            tile = plan_tokens_product(M, N)[0]
-        elif M >= 2048 and N >= 2048:
-            fill = lambda t: t / (-(-t // N_CUS) * N_CUS)
-            tiles256 = ((M + 255) // 256) * ((N + 255) // 256)
-            tiles192 = ((M + 255) // 256) * ((N + 191) // 192)
-            tile = 6 if fill(tiles192) > 1.2 * fill(tiles256) else 5
-    return "gemm_mfma_kernel<%s, %s, %s>" % (str(ta).lower(), str(tb).lower(), TILE_ARGS[tile])
+    return "gemm_mfma_kernel<%s, %s, %s, 0, false>" % (str(ta).lower(), str(tb).lower(), TILE_ARGS[gemm_plan(M, N, K)[0]])
 
 
 def is_split(label):
     """True if the thunk issues two kernels (the columns beyond the full rounds of its tiles go to
-    a second launch of 64 x 64 tiles): its event pair then brackets both, so it is left out of a
+    a second launch of smaller tiles): its event pair then brackets both, so it is left out of a
     single kernel's roofline sample."""
     ta, tb, H, M, N, K = gemm_dims(label)
     if gemm_group(label) > 1:                              # a grouped thunk: never one launch of one product
         return True
-    if ta or H != 1 or M < 1024 or N < 1024 or K % 64:
-        return False
-    return plan_tokens_product(M, N)[1] < N
+    return H == 1 and gemm_plan(M, N, K)[1] > 1
 
 
 def label_prefix(label):

@@ -256,12 +256,13 @@ inline bool mult(int64_t v, int64_t a) { return v % a == 0; }
 
 }  // namespace
 
-CACTI_API int cacti_hip_gemm_f16_strided_batched_tri(int ta, int tb, int64_t nblk, int64_t M,
-                                                     int64_t N, int64_t K, float alpha, const void *A,
-                                                     int64_t lda, int64_t stride_a, const void *B,
-                                                     int64_t ldb, int64_t stride_b, float beta,
-                                                     void *C, int64_t ldc, int64_t stride_c, int tri,
-                                                     void *stream)
+namespace {
+
+// ws_need null: the caller has no workspace.  Otherwise *ws_need is set to the bytes the chosen way needs, and if that is
+// more than ws_bytes nothing is launched.
+int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, float alpha, const void *A, int64_t lda,
+             int64_t stride_a, const void *B, int64_t ldb, int64_t stride_b, float beta, void *C, int64_t ldc,
+             int64_t stride_c, int tri, void *ws, size_t ws_bytes, size_t *ws_need, void *stream)
 {
     CACTI_REQUIRE(tri >= 0 && tri <= 3, CACTI_E_INVALID, "gemm: tri must be 0..3");
     CACTI_REQUIRE(tri == 0 || (tri == 1 && M == N) || (tri == 2 && !ta && M == K) ||
@@ -276,7 +277,8 @@ CACTI_API int cacti_hip_gemm_f16_strided_batched_tri(int ta, int tb, int64_t nbl
                   "gemm: leading dimension smaller than the row length");
     CACTI_REQUIRE(aligned(A, 2) && aligned(B, 2) && aligned(C, 2), CACTI_E_INVALID,
                   "gemm: operands must be 2-byte aligned");
-    GemmArgs p;
+    CACTI_REQUIRE(!ws_need || aligned(ws, 16), CACTI_E_INVALID, "gemm: the workspace must be 16-byte aligned");
+    GemmArgs p = {};
     p.M = M; p.N = N; p.K = K; p.alpha = alpha; p.beta = beta;
     p.A = (const half_t *)A; p.lda = lda; p.sa = stride_a;
     p.B = (const half_t *)B; p.ldb = ldb; p.sb = stride_b;
@@ -285,23 +287,22 @@ CACTI_API int cacti_hip_gemm_f16_strided_batched_tri(int ta, int tb, int64_t nbl
     p.tiles_n = (int)((N + BN - 1) / BN);
     p.tri = tri;
     CACTI_REQUIRE((int64_t)p.tiles_m * p.tiles_n < (1LL << 31), CACTI_E_NOTIMPL, "gemm: too many tiles");
+    if (ws_need) *ws_need = 0;
 
     // widest vector every operand supports: contiguous extent, leading dimension,
     // batch stride and base address must all be multiples of it
     const int64_t ca = ta ? M : K, cb = tb ? K : N;
+    const bool multi = nblk > 1;
+    auto fits_a = [&](int v) { return mult(ca, v) && mult(lda, v) && (!multi || mult(stride_a, v)) && aligned(A, 2 * v); };
+    auto fits_b = [&](int v) { return mult(cb, v) && mult(ldb, v) && (!multi || mult(stride_b, v)) && aligned(B, 2 * v); };
+    auto fits_c = [&](int v) { return mult(N, v) && mult(ldc, v) && (!multi || mult(stride_c, v)) && aligned(C, 2 * v); };
     int vec = 1;
-    for (int v : {8, 4}) {
-        const bool multi = nblk > 1;
-        if (mult(ca, v) && mult(cb, v) && mult(N, v) && mult(lda, v) && mult(ldb, v) &&
-            mult(ldc, v) && (!multi || (mult(stride_a, v) && mult(stride_b, v) && mult(stride_c, v))) &&
-            aligned(A, 2 * v) && aligned(B, 2 * v) && aligned(C, 2 * v)) {
+    for (int v : {8, 4})
+        if (fits_a(v) && fits_b(v) && fits_c(v)) {
             vec = v;
             break;
         }
-    }
     hipStream_t st = (hipStream_t)stream;
-    p.win = 0;
-    p.ztab = 0;
     if (vec >= 4 && !ta && tb && K <= 128 && beta == 0.f && tri <= 1)
         return gemm_nt_smallk_launch(p, nblk, st);
     // one to four rows against a weight matrix (decoding): a stream over B
@@ -324,14 +325,87 @@ CACTI_API int cacti_hip_gemm_f16_strided_batched_tri(int ta, int tb, int64_t nbl
         }
         if (inside) {
             p.win = 1;
-            return gemm_mfma_launch(ta, tb, p, nblk, 8, -1, st);
+            return gemm_mfma_launch(ta, tb, p, nblk, 8, false, nullptr, st);
         }
     }
-    if (vec >= 4) return gemm_mfma_launch(ta, tb, p, nblk, vec, -1, st);
+    if (tri == 0 && vec == 8) {
+        const GemmPlan plan = gemm_plan(M, N, K, nblk, ws_need != nullptr);
+        if (plan.split > 1) {
+            p.ldp = (N + 3) / 4 * 4;
+            p.part = (float *)ws;
+            *ws_need = (size_t)plan.split * (size_t)M * (size_t)p.ldp * sizeof(float);
+            if (*ws_need > ws_bytes) return 0;
+        }
+        return gemm_mfma_launch(ta, tb, p, nblk, 8, false, &plan, st);
+    }
+    // Operands that are not 16-byte aligned, with a workspace: laid out anew (one launch for both, 3-5 us for a few MB)
+    // for the direct kernels.  Element-wise loads in the kernel cost 1.6 us (both operands contiguous in K) to 3.4 us
+    // (both strided) per 32 values of K instead, so only products with hardly any K stay on them.
+    if (ws_need && tri == 0 && nblk == 1 && K > 64) {
+        const bool ok_a = fits_a(8), ok_b = fits_b(8);
+        const int64_t ra = ta ? K : M, rb = tb ? N : K, pa = (ca + 7) / 8 * 8, pb = (cb + 7) / 8 * 8;
+        const size_t bytes_a = ok_a ? 0 : (size_t)ra * (size_t)pa * 2, bytes_b = ok_b ? 0 : (size_t)rb * (size_t)pb * 2;
+        const GemmPlan plan = gemm_plan(M, N, K, 1, true);
+        p.ldp = (N + 3) / 4 * 4;
+        const size_t bytes_part = plan.split > 1 ? (size_t)plan.split * (size_t)M * (size_t)p.ldp * sizeof(float) : 0;
+        *ws_need = bytes_a + bytes_b + bytes_part;                // each a multiple of 16
+        if (*ws_need > ws_bytes) return 0;
+        char *w = static_cast<char *>(ws);
+        const half_t *src[2] = {p.A, p.B};
+        half_t *dst[2] = {ok_a ? nullptr : (half_t *)w, ok_b ? nullptr : (half_t *)(w + bytes_a)};
+        const int64_t rows[2] = {ra, rb}, cols[2] = {ca, cb}, ld[2] = {lda, ldb};
+        if (!ok_a || !ok_b) {
+            const int rc = gemm_repack(src, dst, rows, cols, ld, st);
+            if (rc) return rc;
+        }
+        if (!ok_a) {
+            p.A = dst[0];
+            p.lda = pa;
+        }
+        if (!ok_b) {
+            p.B = dst[1];
+            p.ldb = pb;
+        }
+        p.part = (float *)(w + bytes_a + bytes_b);
+        return gemm_mfma_launch(ta, tb, p, 1, 8, !fits_c(8), &plan, st);
+    }
+    if (vec >= 4) return gemm_mfma_launch(ta, tb, p, nblk, vec, false, nullptr, st);
     if (!ta && !tb) return launch_vec<false, false>(vec, p, nblk, st);
     if (!ta && tb) return launch_vec<false, true>(vec, p, nblk, st);
     if (ta && !tb) return launch_vec<true, false>(vec, p, nblk, st);
     return launch_vec<true, true>(vec, p, nblk, st);
+}
+
+}  // namespace
+
+CACTI_API int cacti_hip_gemm_f16_strided_batched_tri(int ta, int tb, int64_t nblk, int64_t M,
+                                                     int64_t N, int64_t K, float alpha, const void *A,
+                                                     int64_t lda, int64_t stride_a, const void *B,
+                                                     int64_t ldb, int64_t stride_b, float beta,
+                                                     void *C, int64_t ldc, int64_t stride_c, int tri,
+                                                     void *stream)
+{
+    return gemm_run(ta, tb, nblk, M, N, K, alpha, A, lda, stride_a, B, ldb, stride_b, beta, C, ldc, stride_c, tri, nullptr, 0,
+                    nullptr, stream);
+}
+
+CACTI_API int cacti_hip_gemm_f16_ws(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const void *A, int64_t lda,
+                                    const void *B, int64_t ldb, float beta, void *C, int64_t ldc, void *ws, size_t ws_bytes,
+                                    size_t *ws_need, void *stream)
+{
+    CACTI_REQUIRE(ws_need, CACTI_E_INVALID, "gemm_ws: null ws_need");
+    return gemm_run(ta, tb, 1, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, 0, ws, ws_bytes, ws_need, stream);
+}
+
+CACTI_API int cacti_hip_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, int64_t out[6])
+{
+    CACTI_REQUIRE(out && M > 0 && N > 0 && K > 0 && nz > 0, CACTI_E_INVALID, "gemm_plan: bad argument");
+    const GemmPlan plan = gemm_plan(M, N, K, nz, false);
+    gemm_tile_dims(plan.tile, out, out + 1);
+    out[2] = plan.cols > 0 ? plan.cols : N;
+    gemm_tile_dims(plan.rest, out + 3, out + 4);
+    out[5] = plan.cols > 0 ? 2 : 1;
+    return 0;
 }
 
 // Pointer-array batch (cublasGemmBatchedEx shape): the products must have one shape; up to
@@ -357,15 +431,13 @@ CACTI_API int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M
             }
             continue;
         }
-        GemmArgs p;
+        GemmArgs p = {};
         p.M = M; p.N = N; p.K = K; p.alpha = alpha; p.beta = beta;
         p.A = (const half_t *)A[z0]; p.lda = lda; p.sa = 0;
         p.B = (const half_t *)B[z0]; p.ldb = ldb; p.sb = 0;
         p.C = (half_t *)C[z0]; p.ldc = ldc; p.sc = 0;
         p.tiles_m = (int)((M + BM - 1) / BM);
         p.tiles_n = (int)((N + BN - 1) / BN);
-        p.tri = 0;
-        p.win = 0;
         p.ztab = 1;
         for (int64_t z = 0; z < kMaxPtrBatch; z++) {
             const int64_t zz = z0 + (z < cnt ? z : 0);
@@ -373,7 +445,8 @@ CACTI_API int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M
             p.zb[z] = (const half_t *)B[zz] - p.B;
             p.zc[z] = (half_t *)C[zz] - p.C;
         }
-        const int rc = gemm_mfma_launch(ta, tb, p, cnt, 8, -1, (hipStream_t)stream);
+        const GemmPlan plan = gemm_plan(M, N, K, cnt, false);
+        const int rc = gemm_mfma_launch(ta, tb, p, cnt, 8, false, &plan, (hipStream_t)stream);
         if (rc) return rc;
     }
     return 0;

@@ -34,14 +34,32 @@ struct GemmArgs {
     // C + zc[z] (element offsets) instead of z times the batch strides; at most kMaxPtrBatch blocks
     int ztab;
     int64_t za[4], zb[4], zc[4];
+    // split > 1: the product in parts of K, whose fp32 sums go to part[part][M][ldp]
+    int split;
+    float *part;
+    int64_t ldp;
 };
 constexpr int kMaxPtrBatch = 4;
 constexpr int kTriPad = 256;
 
-// tile < 0: chosen by shape
-// align = 8 (16-byte aligned operands) or 4 (8-byte aligned, e.g. head_dim 100)
-int gemm_mfma_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, int align, int tile,
+// how gemm_mfma_launch cuts a product whose operands are 16-byte aligned: tile shapes as in gemm_mfma.hip
+struct GemmPlan {
+    int tile, rest;      // shape of the (first) launch; of the second
+    int64_t cols;        // > 0: columns of the first launch, the rest go to a second
+    int split;           // parts of K
+};
+// nz: products of this shape in the launch
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split);
+void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn);
+
+// align = 8 (16-byte aligned operands) or 4 (8-byte aligned, e.g. head_dim 100).  plan: null for the triangular and
+// column-window products and for align = 4; otherwise align = 8 is required of A and B, and of C unless `odd`
+// (C of any alignment and N).
+int gemm_mfma_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, int align, bool odd, const GemmPlan *plan,
                      hipStream_t st);
+
+int gemm_repack(const half_t *const src[2], half_t *const dst[2], const int64_t rows[2], const int64_t cols[2],
+                const int64_t ld[2], hipStream_t st);
 
 // C = f16(alpha A B^T) with K <= 128 (attention scores): A [M,K], B [N,K] row-major, rows
 // 8-byte aligned, K % 4 == 0, beta = 0, tri 0 or 1

@@ -46,6 +46,7 @@
 #include "common.h"
 #include "gemm_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 using namespace cacti;
@@ -53,6 +54,15 @@ using namespace cacti;
 namespace {
 
 constexpr int BK = 64;
+
+// what the lanes of a direct load beyond the end of K fetch
+__device__ __attribute__((aligned(16))) uint4 g_zero16;
+
+// 16 bytes from the lane's own address into LDS (lane l at m0 + 16 l)
+__device__ __forceinline__ void load_lds16(uint32_t m0, const void *src)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(m0), "v"(src) : "memory");
+}
 
 __device__ __forceinline__ int swz(int r) { return ((r >> 3) ^ r) & 7; }
 // The same for the direct path, whose fragments (v_mfma_f32_16x16x32_f16) are 16 rows x four 16-byte k
@@ -179,6 +189,17 @@ struct LoadKCD {
                          : "memory");
         }
     }
+    // the k tile with only `left` < BK values of k: chunks beyond them are zeros (left is a multiple of 8)
+    __device__ __forceinline__ void dma_tail(uint32_t lds, const half_t *base, int left) const
+    {
+        const uint32_t wave = lds + (threadIdx.x & ~63u) * 16;
+#pragma unroll
+        for (int it = 0; it < NL; it++) {
+            const int c = threadIdx.x + it * NT, r = c >> 3, q = (c & 7) ^ swz16(r);
+            const void *src = q * 8 < left ? (const void *)at(base, off[it]) : (const void *)&g_zero16;
+            load_lds16(__builtin_amdgcn_readfirstlane(wave + it * NT * 16), src);
+        }
+    }
     // instruction `it` of the NL alone (base = origin + k0): lets the caller place each load between MFMAs
     __device__ __forceinline__ void dma1(int it, uint32_t lds, const half_t *base) const
     {
@@ -232,6 +253,17 @@ struct LoadKSD {
                          :
                          : "s"(m0), "v"(off[it]), "s"(base)
                          : "memory");
+        }
+    }
+    // the k tile with only `left` < BK k rows: the rows beyond them are zeros
+    __device__ __forceinline__ void dma_tail(uint32_t lds, const half_t *base, int left) const
+    {
+        const uint32_t wave = lds + (threadIdx.x & ~63u) * 16;
+#pragma unroll
+        for (int it = 0; it < NL; it++) {
+            const int k = (threadIdx.x + it * NT) / CPR;
+            const void *src = k < left ? (const void *)at(base, off[it]) : (const void *)&g_zero16;
+            load_lds16(__builtin_amdgcn_readfirstlane(wave + it * NT * 16), src);
         }
     }
     __device__ __forceinline__ void dma1(int it, uint32_t lds, const half_t *base) const
@@ -547,9 +579,16 @@ __device__ __forceinline__ uint2 lds_read_tr(const unsigned char *q)
     return r;
 }
 
+// E_ROWS: f16(alpha AB + beta C) as whole rows of C, whose pieces are 16-byte (AL = 8) or 8-byte aligned;
+// E_PART: the fp32 sums of one part of K, row-major with pitch ldp, for reduce_parts_kernel; E_ODD: as E_ROWS,
+// element by element, for a C of any alignment and N.
+enum : int { E_ROWS = 0, E_PART = 1, E_ODD = 2 };
+
 // DMA = true: both operands are fetched straight into LDS, NBUF - 1 tiles ahead, no register
 // stages (STAGES is 1); DMA = false: through registers, two LDS buffers.
-template <bool TA, bool TB, int BM, int BN, int WM, int WN, int AL, bool KTAIL, int STAGES, int NBUF, bool DMA>
+// EPI: what the epilogue writes (above).  M32 (direct, one 32 x 32 block per wave): v_mfma_f32_32x32x16_f16 with k in
+// ascending order, the sums of the register path bit for bit.
+template <bool TA, bool TB, int BM, int BN, int WM, int WN, int AL, bool KTAIL, int STAGES, int NBUF, bool DMA, int EPI, bool M32>
 __global__ void __launch_bounds__(WM * WN * 64, min_waves(BM, BN, WM * WN, NBUF))
 gemm_mfma_kernel(GemmArgs p)
 {
@@ -558,6 +597,8 @@ gemm_mfma_kernel(GemmArgs p)
     asm volatile("" ::"s"(p.M), "s"(p.N), "s"(p.K), "s"(p.alpha), "s"(p.beta), "s"(p.A), "s"(p.lda), "s"(p.sa), "s"(p.B),
                  "s"(p.ldb), "s"(p.sb), "s"(p.C), "s"(p.ldc), "s"(p.sc), "s"(p.tiles_m), "s"(p.tiles_n), "s"(p.tri),
                  "s"(p.gm), "s"(p.xcd), "s"(p.pair), "s"(p.win), "s"(p.ztab));
+    static_assert(EPI == E_ROWS || (DMA && !M32), "split and odd products are direct ones");
+    static_assert(!M32 || (DMA && BM == 32 * WM && BN == 32 * WN), "one block per wave");
     static_assert(DMA ? (STAGES == 1 && AL == 8 && !KTAIL) : NBUF == 2,
                   "direct loads: 16-byte aligned operands, whole k tiles");
     constexpr bool TR_A = DMA && TA, TR_B = DMA && !TB;           // fragments by transposing reads
@@ -614,6 +655,14 @@ gemm_mfma_kernel(GemmArgs p)
     if (p.tri == 1 && n0 > m0 + BM - 1) return;                   // uniform for the block
     if (p.tri == 2) nk = min(nk, (int)((m0 + BM + BK - 1) / BK));
     if (p.tri == 3) kt0 = (int)(m0 / BK);
+    const int64_t part = bz;
+    if (EPI == E_PART) {
+        // the "blocks of the batch" are the parts of K: the same operands, a range of k tiles each
+        const int per = (nk + p.split - 1) / p.split;
+        kt0 = (int)part * per;
+        nk = min(nk, kt0 + per);
+        bz = 0;
+    }
 
     const half_t *A = p.A + (p.ztab ? p.za[bz] : bz * p.sa);
     // column window (p.win): the [k][n] operand B and C of block bz start 8 bytes off a 16-byte
@@ -657,25 +706,43 @@ gemm_mfma_kernel(GemmArgs p)
     if constexpr (UNI) {
         la.init(Ao, p.lda, p.M - m0, Bo, p.ldb, nw - n0, p.K);
     } else {
-        la.init(p.lda, p.M - m0, p.K);
-        lb.init(p.ldb, (p.win ? (nw + 7) / 8 * 8 : nw) - n0, p.K);
+        // (the columns of a strided operand end on a multiple of 8: N itself, or the padding behind it)
+        la.init(p.lda, (DMA && TA ? (p.M + 7) / 8 * 8 : p.M) - m0, p.K);
+        lb.init(p.ldb, (DMA && !TB ? (nw + 7) / 8 * 8 : nw) - n0, p.K);
     }
     uint4 ra[STAGES][LA::NREG], rb[STAGES][LB::NREG];
     // direct loads: the first NBUF tiles are requested here, before the accumulators are cleared and the
     // fragment addresses worked out (some thousand cycles of set-up that need not stand in front of them)
     if constexpr (DMA) {
+        // A tail of K goes first, so that every later load is of a whole tile: step t multiplies tile t - 1 and
+        // step 0 the last, incomplete one (only products without a triangular operand have a tail here).  M32
+        // keeps the order and loads it in its turn.
+        const int ktail = (int)(p.K % BK);
+        auto load_tail = [&](int u) __attribute__((always_inline)) {
+            const int64_t k0 = p.K - ktail;
+            la.dma_tail((uint32_t)(uintptr_t)(As + u * BM * BK), la.kbase(Ao, k0), ktail);
+            lb.dma_tail((uint32_t)(uintptr_t)(Bs + u * BN * BK), lb.kbase(Bo, k0), ktail);
+        };
+        if (!M32 && ktail) {
+            if (kt0 == 0) load_tail(0);
+            Ao = la.kbase(Ao, -BK);
+            Bo = lb.kbase(Bo, -BK);
+        }
 #pragma unroll
-        for (int u = 0; u < NBUF; u++)
-            if (kt0 + u < nk) {
+        for (int u = 0; u < NBUF; u++) {
+            if (M32 && ktail && kt0 + u == nk - 1) {
+                load_tail(u);
+            } else if (kt0 + u < nk && (M32 || kt0 + u > 0 || !ktail)) {
                 la.dma((uint32_t)(uintptr_t)(As + u * BM * BK), Ao, (int64_t)(kt0 + u) * BK);
                 lb.dma((uint32_t)(uintptr_t)(Bs + u * BN * BK), Bo, (int64_t)(kt0 + u) * BK);
             }
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
 
     // direct path: 16 x 16 results of v_mfma_f32_16x16x32_f16, [A fragment][B fragment]; lane l holds row
     // l % 16 of the fragment pair's block and columns 4 (l / 16) .. + 3
-    float4_t c16[DMA ? 2 * TM : 1][DMA ? 2 * TN : 1];
+    float4_t c16[DMA && !M32 ? 2 * TM : 1][DMA && !M32 ? 2 * TN : 1];
     const int l16 = lane & 15, kg = lane >> 4;
     float16_t acc[TM][TN];
 #pragma unroll
@@ -822,9 +889,9 @@ gemm_mfma_kernel(GemmArgs p)
         constexpr int NMH = TM * NB;                              // MFMAs of a half
         constexpr int RA = (TR_A ? 2 : 1) * TM, RB = (TR_B ? 2 : 1) * NB;   // LDS reads: A fragments of a half, all B
 #pragma unroll
-        for (int a = 0; a < NA; a++)
+        for (int a = 0; a < (M32 ? 1 : NA); a++)
 #pragma unroll
-            for (int b = 0; b < NB; b++) c16[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+            for (int b = 0; b < (M32 ? 1 : NB); b++) c16[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
         half8_t fa[2][TM], fb[2][NB];                             // A fragments of a half, B fragments of a k step
         // [row][k] tiles: halves offset of the lane's row in a block's upper / lower 16 rows, and its swizzle
         const int ar[2] = {wm * 32 + l16, wm * 32 + 16 + l16}, br[2] = {wn * 32 + l16, wn * 32 + 16 + l16};
@@ -918,6 +985,21 @@ gemm_mfma_kernel(GemmArgs p)
         half8_t ga[2][2][NA], gb[2][2][NB];
         auto read_tile = [&](auto set_c, int buf) __attribute__((always_inline)) {
             constexpr int S = decltype(set_c)::value;
+            if constexpr (M32) {
+                // fragments of the four k steps of 16: ks of ga / gb [ks / 2][ks % 2]
+#pragma unroll
+                for (int ks = 0; ks < 4; ks++) {
+                    const half_t *as = As + buf * BM * BK, *bs = Bs + buf * BN * BK;
+                    const int q = ks * 2 + lh;
+                    ga[S][ks >> 1][ks & 1] =
+                        TR_A ? frag_tr(reinterpret_cast<const unsigned char *>(as) + atr + ks * 16 * (BM * 2), BM * 2)
+                             : *reinterpret_cast<const half8_t *>(as + ar0 * BK + ((q ^ swz16(ar0)) << 3));
+                    gb[S][ks >> 1][ks & 1] =
+                        TR_B ? frag_tr(reinterpret_cast<const unsigned char *>(bs) + btr + ks * 16 * (BN * 2), BN * 2)
+                             : *reinterpret_cast<const half8_t *>(bs + br0 * BK + ((q ^ swz16(br0)) << 3));
+                }
+                return;
+            }
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
 #pragma unroll
@@ -936,9 +1018,20 @@ gemm_mfma_kernel(GemmArgs p)
                 __syncthreads();
                 read_tile(std::integral_constant<int, S ^ 1>{}, nb);
                 __builtin_amdgcn_sched_barrier(0);
-                if (MAIN || t + NBUF < nk) issue_all(t + NBUF, cb);
+                if (!MAIN && M32 && p.K % BK != 0 && t + NBUF == nk - 1) {
+                    const int64_t k0 = (int64_t)(nk - 1) * BK;
+                    la.dma_tail(lds_addr(As + cb * BM * BK), la.kbase(Ao, k0), (int)(p.K - k0));
+                    lb.dma_tail(lds_addr(Bs + cb * BN * BK), lb.kbase(Bo, k0), (int)(p.K - k0));
+                } else if (MAIN || t + NBUF < nk) {
+                    issue_all(t + NBUF, cb);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (M32) {
+#pragma unroll
+                for (int ks = 0; ks < 4; ks++)
+                    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(gb[S][ks >> 1][ks & 1], ga[S][ks >> 1][ks & 1], acc[0][0], 0, 0, 0);
+            } else
 #pragma unroll
             for (int ks = 0; ks < 2; ks++)
 #pragma unroll
@@ -951,7 +1044,8 @@ gemm_mfma_kernel(GemmArgs p)
             t++;
         };
         read_tile(std::integral_constant<int, 0>{}, 0);
-        while (t + NBUF + 1 < nk) {                               // both steps load inside K
+        const int nk_whole = M32 && p.K % BK != 0 ? nk - 1 : nk;
+        while (t + NBUF + 1 < nk_whole) {                         // both steps load whole tiles
             body(std::integral_constant<int, 0>{}, std::true_type{});
             body(std::integral_constant<int, 1>{}, std::true_type{});
         }
@@ -1038,6 +1132,20 @@ gemm_mfma_kernel(GemmArgs p)
         if (TAIL > 4 && kt + 4 < nk) { step(std::integral_constant<int, 4 % STAGES>{}, std::false_type{}, kt + 4, cb); cb = next_buf(cb); }
     }
 
+    if constexpr (EPI == E_PART) {
+        // a lane's 4 consecutive columns of a row are 16 bytes of the part, four lanes a 64-byte run
+        float *out = p.part + part * p.M * p.ldp;
+#pragma unroll
+        for (int a = 0; a < 2 * TM; a++) {
+            const int64_t m = m0 + (a >> 1) * (32 * WM) + wm * 32 + (a & 1) * 16 + l16;
+#pragma unroll
+            for (int b = 0; b < 2 * TN; b++) {
+                const int64_t n = n0 + (b >> 1) * (32 * WN) + wn * 32 + (b & 1) * 16 + kg * 4;
+                if (m < p.M && n < p.N) *reinterpret_cast<float4_t *>(out + m * p.ldp + n) = c16[a][b];
+            }
+        }
+        return;
+    }
     // Epilogue through LDS (the operand buffers are free after the last barrier): a lane
     // holds row m = .. + l32 and, per accumulator group q, the 4 consecutive columns
     // n = .. + 8 q + 4 lh + {0..3}, i.e. 8 bytes in each of 32 different rows of C; staged as
@@ -1057,7 +1165,7 @@ gemm_mfma_kernel(GemmArgs p)
     // stored (the general loop below waits for every piece in turn: 9,000 cycles more per workgroup measured)
     // (tiles of up to 256 x 128: the larger ones have no registers for it and spill in their main loop with it)
     constexpr bool C_BATCH = BM * BN <= 256 * 128 && BM * CPRC % NT == 0;
-    const bool c_inside = C_BATCH && AL == 8 && shift == 0 && m0 + BM <= p.M && n0 + BN <= nw;
+    const bool c_inside = C_BATCH && AL == 8 && EPI == E_ROWS && shift == 0 && m0 + BM <= p.M && n0 + BN <= nw;
     if (has_beta && c_inside) {
         constexpr int NC = C_BATCH ? BM * CPRC / NT : 1;
         uint4 old[NC];
@@ -1079,7 +1187,12 @@ gemm_mfma_kernel(GemmArgs p)
             const bool lo = m < p.M && n >= shift && n < nw, hi = m < p.M && n + 4 >= shift && n + 4 < nw;
             const half_t *cp = C + m * p.ldc + n;
             uint4 v = make_uint4(0, 0, 0, 0);
-            if (AL == 8 && lo && hi) {
+            if (EPI == E_ODD) {
+                half_t *e = reinterpret_cast<half_t *>(&v);
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    if (m < p.M && n + j < p.N) e[j] = cp[j];
+            } else if (AL == 8 && lo && hi) {
                 v = *reinterpret_cast<const uint4 *>(cp);
             } else {
                 if (lo) {
@@ -1097,7 +1210,7 @@ gemm_mfma_kernel(GemmArgs p)
         }
         __syncthreads();
     }
-    if constexpr (DMA) {
+    if constexpr (DMA && !M32) {
 #pragma unroll
         for (int a = 0; a < 2 * TM; a++) {
             const int row = (a >> 1) * (32 * WM) + wm * 32 + (a & 1) * 16 + l16;
@@ -1143,6 +1256,15 @@ gemm_mfma_kernel(GemmArgs p)
         }
 }
     __syncthreads();
+    if constexpr (EPI == E_ODD) {
+        // consecutive lanes take consecutive elements of a row
+        for (int c = threadIdx.x; c < BM * BN; c += NT) {
+            const int row = c / BN, col = c % BN;
+            if (m0 + row < p.M && n0 + col < p.N)
+                C[(m0 + row) * p.ldc + n0 + col] = Cs[row * BN + ((((col >> 3) ^ (row & CSW)) << 3) | (col & 7))];
+        }
+        return;
+    }
     for (int c = threadIdx.x; c < BM * CPRC; c += NT) {
         const int row = c / CPRC, cc = c % CPRC;
         const int64_t m = m0 + row, n = n0 + cc * 8;
@@ -1161,13 +1283,68 @@ gemm_mfma_kernel(GemmArgs p)
     }
 }
 
-template <bool TA, bool TB, int BM, int BN, int WM, int WN, int AL, bool KTAIL, int STAGES, int NBUF = 2, bool DMA = false>
+// C = f16(alpha sum of the parts + beta C), four columns per lane; the parts are added in order.  VEC: N and the rows
+// of C allow 8-byte accesses.
+template <bool VEC>
+__global__ void __launch_bounds__(256)
+reduce_parts_kernel(int64_t M, int64_t N, int64_t ldp, int split, const float *__restrict__ part, float alpha, float beta,
+                    half_t *__restrict__ C, int64_t ldc)
+{
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= M * ldp) return;
+    const int64_t m = i / ldp, n = i - m * ldp;
+    float4_t s = *reinterpret_cast<const float4_t *>(part + i);
+    for (int k = 1; k < split; k++) s += *reinterpret_cast<const float4_t *>(part + k * M * ldp + i);
+    half_t *cp = C + m * ldc + n;
+    half4_t o, old = {0, 0, 0, 0};
+    const bool has_beta = beta != 0.f;
+    if (VEC) {
+        if (has_beta) old = *reinterpret_cast<const half4_t *>(cp);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (has_beta && n + r < N) old[r] = cp[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) o[r] = has_beta ? f2h(alpha * s[r] + beta * h2f(old[r])) : f2h(alpha * s[r]);
+    if (VEC) {
+        *reinterpret_cast<half4_t *>(cp) = o;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (n + r < N) cp[r] = o[r];
+    }
+}
+
+// Operands of any alignment as operands the direct kernels take: rows of `cols` halves, `ld` apart, to rows of `out_cols`
+// = cols rounded up to 8 (zeros behind cols), 16-byte aligned.  One lane per 16-byte piece, both operands in one launch.
+struct RepackArgs {
+    const half_t *src[2];
+    half_t *dst[2];
+    int64_t rows[2], cols[2], ld[2];
+};
+__global__ void __launch_bounds__(256) repack_kernel(RepackArgs p)
+{
+    const int z = blockIdx.y;
+    const int64_t per_row = (p.cols[z] + 7) / 8, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (!p.dst[z] || i >= p.rows[z] * per_row) return;
+    const int64_t row = i / per_row, c = (i - row * per_row) * 8;
+    const half_t *src = p.src[z] + row * p.ld[z] + c;
+    const int64_t left = p.cols[z] - c;
+    h8 v;
+#pragma unroll
+    for (int j = 0; j < 8; j++) v.v[j] = j < left ? src[j] : (half_t)0.f;
+    st8(p.dst[z] + i * 8, v);
+}
+
+template <bool TA, bool TB, int BM, int BN, int WM, int WN, int AL, bool KTAIL, int STAGES, int NBUF = 2, bool DMA = false,
+          int EPI = E_ROWS, bool M32 = false>
 int launch_cfg(GemmArgs p, int64_t nblk, hipStream_t st)
 {
     p.tiles_m = (int)((p.M + BM - 1) / BM);
     p.tiles_n = (int)((p.N + (p.win ? 4 : 0) + BN - 1) / BN);
     const size_t smem = (size_t)NBUF * (BM + BN) * BK * sizeof(half_t);
-    auto kern = gemm_mfma_kernel<TA, TB, BM, BN, WM, WN, AL, KTAIL, STAGES, NBUF, DMA>;
+    auto kern = gemm_mfma_kernel<TA, TB, BM, BN, WM, WN, AL, KTAIL, STAGES, NBUF, DMA, EPI, M32>;
     static DeviceOnce attr_set;                   // one per instantiation
     if (!attr_set.fresh()) {
         CACTI_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1202,34 +1379,48 @@ int launch_cfg(GemmArgs p, int64_t nblk, hipStream_t st)
     return launch_status("gemm_mfma");
 }
 
-// tile: 0 = 128 x 128 on 4 waves, two register stages (every loader is branch-free on 256
-// lanes); 1 = 256 x 128 on 8 waves, two register stages; 3 = 64 x 64 on 4 waves; 4 = 256 x 128,
-// 5 = 256 x 256 (128 x 64 per wave), 6 = 256 x 192 (64 x 96 per wave) and 7 = 128 x 128 (64 x 32
-// per wave) on 8 waves with both operands loaded straight into LDS; 8 = 64 x 64 on 4 waves the same way,
-// five k tiles ahead
-template <bool TA, bool TB>
-int launch_tile(int tile, int align, const GemmArgs &p, int64_t nblk, hipStream_t st)
+// Tile shapes of the direct kernels: 64 x 64 and 128 x 64 on 4 waves (two workgroups per CU), 128 x 128, 256 x 128,
+// 256 x 256 (128 x 64 per wave) and 256 x 192 (64 x 96 per wave) on 8 waves (one per CU).
+// T64_SMALL: 64 x 64 with the 32 x 32 x 16 instruction, for outputs of up to kSmallOutput elements.
+enum Tile : int { T64, T128_64, T128, T256_128, T256_192, T256, N_TILES, T64_SMALL = N_TILES };
+
+template <bool TA, bool TB, int EPI>
+int launch_direct(int tile, const GemmArgs &p, int64_t nblk, hipStream_t st)
 {
-    const bool ktail = (p.K % BK) != 0;
-    if (align < 8) {
-        // 8-byte aligned operands (the attention blocks): 8 waves of 64 x 32 on the 128 x 128 tile;
-        // with one workgroup per CU (32 heads x 8 tile-row pairs) two waves per SIMD hide each
-        // other's LDS latency (-9..13 % against 4 waves of 64 x 64)
-        return ktail ? launch_cfg<TA, TB, 128, 128, 2, 2, 4, true, 1>(p, nblk, st)
-                     : launch_cfg<TA, TB, 128, 128, 2, 4, 4, false, 2>(p, nblk, st);
-    }
-    if (ktail) return launch_cfg<TA, TB, 128, 128, 2, 2, 8, true, 1>(p, nblk, st);
     switch (tile) {
-        case 0: return launch_cfg<TA, TB, 128, 128, 2, 2, 8, false, 2>(p, nblk, st);
-        case 3: return launch_cfg<TA, TB, 64, 64, 2, 2, 8, false, 2>(p, nblk, st);
-        case 4: return launch_cfg<TA, TB, 256, 128, 4, 2, 8, false, 1, 3, true>(p, nblk, st);
-        case 5: return launch_cfg<TA, TB, 256, 256, 2, 4, 8, false, 1, 2, true>(p, nblk, st);
-        case 6: return launch_cfg<TA, TB, 256, 192, 4, 2, 8, false, 1, 2, true>(p, nblk, st);
-        case 7: return launch_cfg<TA, TB, 128, 128, 2, 4, 8, false, 1, 3, true>(p, nblk, st);
-        case 8: return launch_cfg<TA, TB, 64, 64, 2, 2, 8, false, 1, 6, true>(p, nblk, st);
-        default: return launch_cfg<TA, TB, 256, 128, 4, 2, 8, false, 2>(p, nblk, st);
+        case T64: return launch_cfg<TA, TB, 64, 64, 2, 2, 8, false, 1, 4, true, EPI>(p, nblk, st);
+        case T128_64: return launch_cfg<TA, TB, 128, 64, 2, 2, 8, false, 1, 3, true, EPI>(p, nblk, st);
+        case T128: return launch_cfg<TA, TB, 128, 128, 2, 4, 8, false, 1, 3, true, EPI>(p, nblk, st);
     }
+    if constexpr (EPI != E_PART)                                  // (a product that needs a split has few tiles: small ones)
+        if (tile == T256_128) return launch_cfg<TA, TB, 256, 128, 4, 2, 8, false, 1, 3, true, EPI>(p, nblk, st);
+    if constexpr (EPI == E_ROWS) {
+        switch (tile) {
+            case T64_SMALL: return launch_cfg<TA, TB, 64, 64, 2, 2, 8, false, 1, 4, true, EPI, true>(p, nblk, st);
+            case T256_192: return launch_cfg<TA, TB, 256, 192, 4, 2, 8, false, 1, 2, true, EPI>(p, nblk, st);
+            case T256: return launch_cfg<TA, TB, 256, 256, 2, 4, 8, false, 1, 2, true, EPI>(p, nblk, st);
+        }
+    }
+    set_error("gemm: no tile %d", tile);
+    return CACTI_E_STATE;
 }
+
+// What a product costs on a tile, in microseconds: a start and end of `fixed`, then per k tile the time of a full
+// set of resident workgroups (`resident` per CU: `full`), for the last, partly filled set `first` + `load` x the share
+// of the CUs that are busy where no CU has more than one, and `round` for every further set.  Fitted (least squares
+// of the log) to 338 products measured on MI355X: M 33 .. 8640, N 256 .. 32000, K 37 .. 32000, the three layouts;
+// rms error 6-8 % per tile, and the tile picked by it is 1.3 % slower than the best one in the mean, 14 % at worst.
+struct TileCost {
+    int bm, bn, resident;
+    double fixed, first, load, full, round;
+};
+constexpr TileCost kTileCost[N_TILES] = {
+    {64, 64, 2, 3.947, 0.226, 0.042, 0.385, 2.187},    {128, 64, 2, 4.429, 0.277, 0.069, 0.562, 2.748},
+    {128, 128, 1, 4.677, 0.394, 0.113, 0.507, 3.479},  {256, 128, 1, 5.582, 0.621, 0.208, 0.829, 5.417},
+    {256, 192, 1, 6.801, 0.878, 0.291, 1.169, 6.229},  {256, 256, 1, 7.843, 1.094, 0.392, 1.486, 7.759},
+};
+
+constexpr int64_t kSmallOutput = 1 << 18;
 
 int cu_count()
 {
@@ -1243,112 +1434,160 @@ int cu_count()
     return cus;
 }
 
-// How a large product with A not transposed (M = tokens) is cut into workgroups.  One workgroup
-// per CU runs in rounds of `cus` tiles, and a last round that holds only a few tiles costs as
-// much as a full one (N = 8640 at 2048 tokens: 544 tiles of 256 x 128 = 2 rounds + 32 tiles).
-// The columns of the full rounds can instead go to one launch and the few remaining ones to a
-// second launch of 64 x 64 tiles, which spreads them over every CU.  The plan compares
-// 256 x 128 tiles with 256 x 256 tiles (measured 1.2 x the rate per tile area: 883 -> 1075
-// TFLOP/s on 2048 x 8192 x 3200) by rounds x tile area / rate, the second launch costing 3/8 of
-// a 256 x 128 round.  At 2048 tokens: N = 3200 -> 200 tiles of 256 x 128 (one round); N = 8640
-// -> 256 tiles of 256 x 256 + 448 columns (135 -> 122 us); N = 32000 -> 1000 tiles of 256 x 256.
-struct Plan {
-    int tile;               // 4 or 5
-    int64_t cols_main;      // columns of the first launch (N: a single launch)
-};
-Plan plan_tokens_product(int64_t M, int64_t N, bool may_split)
+double tile_cost(int tile, int64_t M, int64_t N, int64_t nz, int64_t ktiles)
 {
-    const int64_t cus = cu_count();
-    Plan best{4, N};
-    int64_t best_cost = -1;
-    const int tiles[2] = {4, 5};
-    const int64_t widths[2] = {128, 256}, round_cost[2] = {32768, 54613};   // 256 bn / rate
-    for (int c = 0; c < 2; c++) {
-        const int64_t bn = widths[c], tiles_m = (M + 255) / 256, tiles_n = (N + bn - 1) / bn;
-        const int64_t total = tiles_m * tiles_n, full = total / cus;
-        const int64_t cols_main = full * cus / tiles_m, rest = tiles_m * (tiles_n - cols_main);
-        int64_t cost, main_cols;
-        if (may_split && full >= 1 && cols_main < tiles_n && rest * bn * 4 <= cus * 128) {
-            cost = full * round_cost[c] + 12288;
-            main_cols = cols_main * bn;
-        } else {
-            cost = (total + cus - 1) / cus * round_cost[c];
-            main_cols = N;
-        }
-        if (best_cost < 0 || cost < best_cost) {
-            best_cost = cost;
-            best = Plan{tiles[c], main_cols};
-        }
-    }
-    return best;
-}
-
-template <bool TA, bool TB>
-int launch_auto(int tile, int64_t cols_main, int align, const GemmArgs &p, int64_t nblk, hipStream_t st)
-{
-    if (cols_main > 0 && cols_main < p.N) {
-        GemmArgs a = p, b = p;
-        a.N = cols_main;
-        b.N = p.N - a.N;
-        b.B = p.B + (TB ? a.N * p.ldb : a.N);
-        b.C = p.C + a.N;
-        const int rc = launch_tile<TA, TB>(tile, align, a, nblk, st);
-        // the remaining columns on 64 x 64 tiles loaded straight into LDS, six buffers: a tile this
-        // small has 4 MFMAs per wave and k tile, so a k step costs the latency of its loads unless
-        // they were issued several steps earlier (448 columns at K = 3200: register path with two
-        // stages 23.7 us, three buffers 21.4, six 15.2 .. 16.5)
-        return rc ? rc : launch_tile<TA, TB>(8, align, b, nblk, st);
-    }
-    return launch_tile<TA, TB>(tile, align, p, nblk, st);
+    const TileCost &t = kTileCost[tile];
+    const int64_t wg = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn) * nz, cus = cu_count(), set = cus * t.resident;
+    const int64_t sets = wg / set;
+    const double rest = (double)(wg - sets * set) / (double)cus;
+    const double last = rest == 0 ? 0 : rest <= 1 ? t.first + t.load * rest : t.full;
+    return t.fixed + (double)ktiles * ((double)sets * t.full + last) + t.round * (double)(sets + (rest > 0) - 1);
 }
 
 }  // namespace
 
 namespace cacti {
 
-// tile: as launch_tile; -1 = pick by shape
-int gemm_mfma_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, int align, int tile,
-                     hipStream_t st)
+void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn)
+{
+    if (tile == T64_SMALL) tile = T64;
+    *bm = kTileCost[tile].bm;
+    *bn = kTileCost[tile].bn;
+}
+
+// How a product of 16-byte aligned operands is cut.  One workgroup takes one tile; a launch runs in sets of resident
+// workgroups, and a nearly empty last set costs as much as a full one.  Considered: every tile shape by itself; for the
+// 256-wide ones also the columns of the full sets in one launch and the rest on smaller tiles in a second (2048 x 8640 x
+// 3200: 256 tiles of 256 x 256 and 448 columns); and, where the caller has a workspace (may_split), up to 8 parts of K
+// for products with fewer tiles than CUs and a long K, whose workgroups would otherwise run 100 k tiles one after
+// another on a fraction of the CUs (37 x 3200 x 8640: 50 tiles; the parts and their sum cost a launch and
+// 8 bytes per part and element).
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split)
+{
+    const int64_t kt = (K + BK - 1) / BK, cus = cu_count();
+    GemmPlan best = {T64, T64, 0, 1};
+    double best_cost = 1e30;
+    // A small output has at most 64 tiles of 64 x 64, the shape that is best for it.  The device is nowhere near its power
+    // limit there, so the instruction is free to be the one whose sums the register path has always formed.
+    const bool small = M * N <= kSmallOutput;
+    if (small) {
+        best = {T64_SMALL, T64, 0, 1};
+        best_cost = tile_cost(T64, M, N, nz, kt);
+    }
+    for (int t = 0; t < N_TILES && !small; t++) {
+        const double c = tile_cost(t, M, N, nz, kt);
+        if (c < best_cost) {
+            best_cost = c;
+            best = {t, T64, 0, 1};
+        }
+    }
+    for (int t = T256_128; t < N_TILES && !small; t++) {
+        const int64_t tiles_m = (M + 255) / 256 * nz, bn = kTileCost[t].bn, tiles_n = (N + bn - 1) / bn;
+        const int64_t cols = tiles_m * tiles_n / cus * cus / tiles_m * bn;
+        if (cols <= 0 || cols >= N) continue;
+        for (int r = T64; r <= T128; r++) {
+            const double c = tile_cost(t, M, cols, nz, kt) + tile_cost(r, M, N - cols, nz, kt);
+            if (c < best_cost) {
+                best_cost = c;
+                best = {t, r, cols, 1};
+            }
+        }
+    }
+    if (may_split && nz == 1)
+        for (int t = T64; t <= T128; t++)
+            for (int s = 2; s <= 8; s++) {
+                const int64_t per = (kt + s - 1) / s;
+                if (per < 4 || (kt + per - 1) / per != s) continue;           // parts of some length, none empty
+                const double c = tile_cost(t, M, N, s, per) + 4.0 + (double)(M * N) * s * 8.0 / 4e6;
+                if (c < best_cost) {
+                    best_cost = c;
+                    best = {t, T64, 0, s};
+                }
+            }
+    return best;
+}
+
+}  // namespace cacti
+
+namespace {
+
+template <bool TA, bool TB>
+int launch_plan(const GemmPlan &plan, const GemmArgs &p, int64_t nblk, bool odd, hipStream_t st)
+{
+    if (plan.split > 1) {
+        GemmArgs q = p;
+        q.split = plan.split;
+        const int rc = launch_direct<TA, TB, E_PART>(plan.tile, q, plan.split, st);
+        if (rc) return rc;
+        const unsigned grid = (unsigned)((p.M * p.ldp + 1023) / 1024);
+        const auto reduce = p.N % 4 == 0 && p.ldc % 4 == 0 && aligned(p.C, 8) ? reduce_parts_kernel<true> : reduce_parts_kernel<false>;
+        hipLaunchKernelGGL(reduce, dim3(grid), dim3(256), 0, st, p.M, p.N, p.ldp, plan.split, p.part, p.alpha, p.beta, p.C, p.ldc);
+        return launch_status("gemm_reduce_parts");
+    }
+    if (odd) {
+        const int tile = plan.tile == T64_SMALL ? T64 : plan.tile;
+        return launch_direct<TA, TB, E_ODD>(tile < T256_128 ? tile : (int)T256_128, p, nblk, st);
+    }
+    if (plan.cols > 0) {
+        GemmArgs a = p, b = p;
+        a.N = plan.cols;
+        b.N = p.N - a.N;
+        b.B = p.B + (TB ? a.N * p.ldb : a.N);
+        b.C = p.C + a.N;
+        const int rc = launch_direct<TA, TB, E_ROWS>(plan.tile, a, nblk, st);
+        return rc ? rc : launch_direct<TA, TB, E_ROWS>(plan.rest, b, nblk, st);
+    }
+    return launch_direct<TA, TB, E_ROWS>(plan.tile, p, nblk, st);
+}
+
+template <bool TA, bool TB>
+int launch_any(const GemmArgs &p, int64_t nblk, int align, bool odd, const GemmPlan *plan, hipStream_t st)
+{
+    if (plan) return launch_plan<TA, TB>(*plan, p, nblk, odd, st);
+    const bool ktail = (p.K % BK) != 0;
+    // Per-head slabs addressed through a column window, and the triangular products of attention: 128 x 128 tiles
+    // on 8 waves, three LDS buffers (-5 us per launch against the register path with 8 waves).
+    if (align >= 8 && (p.win || !ktail)) return launch_direct<TA, TB, E_ROWS>(T128, p, nblk, st);
+    // 8-byte aligned operands (the attention blocks): 8 waves of 64 x 32 on the 128 x 128 tile;
+    // with one workgroup per CU (32 heads x 8 tile-row pairs) two waves per SIMD hide each
+    // other's LDS latency (-9..13 % against 4 waves of 64 x 64)
+    if (align >= 8) return launch_cfg<TA, TB, 128, 128, 2, 2, 8, true, 1>(p, nblk, st);
+    return ktail ? launch_cfg<TA, TB, 128, 128, 2, 2, 4, true, 1>(p, nblk, st)
+                 : launch_cfg<TA, TB, 128, 128, 2, 4, 4, false, 2>(p, nblk, st);
+}
+
+}  // namespace
+
+namespace cacti {
+
+int gemm_mfma_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, int align, bool odd, const GemmPlan *plan, hipStream_t st)
 {
     GemmArgs q = p;
     q.gm = -1;                                    // rows of tiles per group: chosen per launch
     q.xcd = 1;                                    // consecutive tiles to the workgroups of one XCD
-    int64_t cols_main = 0;                        // > 0: a second launch takes the columns from here on
-    if (tile < 0) {
-        {
-            // measured on MI355X at the step's shapes (TFLOP/s on cold operands, register
-            // path 128 x 128 or 256 x 128 -> direct loads).  A not transposed (forward and dgrad,
-            // M = tokens): NT 661..821 -> 707..881, NN 702..787 -> 773..864 on 256 x 128, one
-            // workgroup per CU; 256 x 256 where its rounds fit (plan_tokens_product).  Wgrad (both
-            // operands strided, weight-sized outputs): 256 x 256, 558..715 -> 755..932.
-            // Small and batched products stay on 128 x 128 through registers.
-            tile = 0;
-            // the attention products on per-head slabs: 128 x 128, 8 waves of 64 x 32, three
-            // LDS buffers (-5 us per launch against the register path with 8 waves)
-            if (p.win) tile = 7;
-            // (a pointer-table batch is a handful of whole products: planned like a single one)
-            if ((nblk == 1 || p.ztab) && p.M >= 1024 && p.N >= 1024) {
-                if (!ta) {
-                    const bool direct_ok = align >= 8 && p.K % BK == 0;     // else launch_tile ignores the tile
-                    const Plan plan = plan_tokens_product(p.M, p.N, direct_ok && p.tri == 0);
-                    tile = plan.tile;
-                    cols_main = plan.cols_main;
-                } else if (p.M >= 2048 && p.N >= 2048) {
-                    // 256 x 192 where its tile count fills the CUs markedly better (3200 x 3200:
-                    // 221 tiles in one round against 169; +5 %)
-                    const int64_t cus = cu_count();
-                    const int64_t tiles256 = ((p.M + 255) / 256) * ((p.N + 255) / 256);
-                    const int64_t tiles192 = ((p.M + 255) / 256) * ((p.N + 191) / 192);
-                    auto fill = [&](int64_t tiles) { return (double)tiles / (double)((tiles + cus - 1) / cus * cus); };
-                    tile = fill(tiles192) > 1.2 * fill(tiles256) ? 6 : 5;
-                }
-            }
-        }
+    if (!ta && !tb) return launch_any<false, false>(q, nblk, align, odd, plan, st);
+    if (!ta && tb) return launch_any<false, true>(q, nblk, align, odd, plan, st);
+    if (ta && !tb) return launch_any<true, false>(q, nblk, align, odd, plan, st);
+    return launch_any<true, true>(q, nblk, align, odd, plan, st);
+}
+
+// a copy of up to two operands in the layout of the direct kernels (dst null: none of that one)
+int gemm_repack(const half_t *const src[2], half_t *const dst[2], const int64_t rows[2], const int64_t cols[2], const int64_t ld[2],
+                hipStream_t st)
+{
+    RepackArgs p;
+    int64_t most = 0;
+    for (int z = 0; z < 2; z++) {
+        p.src[z] = src[z];
+        p.dst[z] = dst[z];
+        p.rows[z] = rows[z];
+        p.cols[z] = cols[z];
+        p.ld[z] = ld[z];
+        if (dst[z]) most = std::max(most, rows[z] * ((cols[z] + 7) / 8));
     }
-    if (!ta && !tb) return launch_auto<false, false>(tile, cols_main, align, q, nblk, st);
-    if (!ta && tb) return launch_auto<false, true>(tile, cols_main, align, q, nblk, st);
-    if (ta && !tb) return launch_auto<true, false>(tile, cols_main, align, q, nblk, st);
-    return launch_auto<true, true>(tile, cols_main, align, q, nblk, st);
+    CACTI_REQUIRE((most + 255) / 256 < (int64_t)1 << 31, CACTI_E_NOTIMPL, "gemm: operand too large to lay out");
+    hipLaunchKernelGGL(repack_kernel, dim3((unsigned)((most + 255) / 256), 2), dim3(256), 0, st, p);
+    return launch_status("gemm_repack");
 }
 
 }  // namespace cacti

@@ -733,6 +733,19 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
     if (!rc) rc = c.pool_alloc((size_t)(T * V) * 2, &k->out_logit);
     if (!rc) rc = c.pool_alloc((size_t)T * 2, &k->out_tok);
     if (!rc && want_prob) rc = c.pool_alloc((size_t)(T * V) * 4, &k->out_prob);
+    // products take a workspace where they ask for one; it is theirs in stream order, so one serves them all
+    char *gws = nullptr;
+    size_t gws_bytes = 0;
+    auto product = [&](int64_t N, int64_t K, const void *a, const void *w, void *y) -> int {
+        size_t need = 0;
+        for (;;) {
+            const int r = cacti_hip_gemm_f16_ws(0, 1, T, N, K, 1.f, a, K, w, K, 0.f, y, N, gws, gws_bytes, &need, st);
+            if (r || need <= gws_bytes) return r;
+            gws = tmp((int64_t)need, 1);
+            if (!gws) return rc;
+            gws_bytes = need;
+        }
+    };
 #define STEP(call)          \
     do {                    \
         if (!rc) rc = (call); \
@@ -756,10 +769,10 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
                 STEP(cacti_hip_rows_qkv_rope_cache_f16(T, H, Dh, xa, xb, P(w.pre_norm), g.eps, xb ? x : nullptr, P(w.q), P(w.k),
                                                        P(w.v), cosr, sinr, qr, kc + prev * D * 2, vc + prev * D * 2, st));
                 STEP(cacti_hip_attn_decode_f16(T, H, Dh, next, prev, alpha, qr, D, kc, vc, D, Dh, attn, D, aws, aws_bytes, st));
-                STEP(cacti_hip_gemm_f16(0, 1, T, D, D, 1.f, attn, D, P(w.o), D, 0.f, o, D, st));
+                STEP(product(D, D, attn, P(w.o), o));
                 // x1 = stream + o; post = rms_norm(x1); h = silu(post gate^T) * (post up^T)
                 STEP(cacti_hip_rows_norm_matmul_f16(T, F, D, x, o, P(w.post_norm), g.eps, x1, P(w.gate), P(w.up), h, st));
-                STEP(cacti_hip_gemm_f16(0, 1, T, D, F, 1.f, h, F, P(w.down), F, 0.f, down, D, st));
+                STEP(product(D, F, h, P(w.down), down));
                 xa = x1;                                          // stream = x1 + down, formed by the next consumer
                 xb = down;
             }
@@ -769,13 +782,13 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
             for (size_t l = 0; l < m->layers.size() && !rc; l++) {
                 const LayerCells &w = m->layers[l];
                 char *kc = static_cast<char *>(P(k->k_cache[l])), *vc = static_cast<char *>(P(k->v_cache[l]));
-                STEP(cacti_hip_gemm_f16(0, 1, T, D, D, 1.f, pre, D, P(w.q), D, 0.f, q, D, st));
+                STEP(product(D, D, pre, P(w.q), q));
                 STEP(cacti_hip_rope_fwd(T, H, Dh, q, cosr, sinr, qr, st));
-                STEP(cacti_hip_gemm_f16(0, 1, T, D, D, 1.f, pre, D, P(w.k), D, 0.f, kk, D, st));
+                STEP(product(D, D, pre, P(w.k), kk));
                 STEP(cacti_hip_rope_fwd(T, H, Dh, kk, cosr, sinr, kr, st));
                 // k_cache[prev .. next] += k, v_cache[prev .. next] += v
                 STEP(cacti_hip_add_f16(T * D, kc + prev * D * 2, kr, kc + prev * D * 2, st));
-                STEP(cacti_hip_gemm_f16(0, 1, T, D, D, 1.f, pre, D, P(w.v), D, 0.f, v, D, st));
+                STEP(product(D, D, pre, P(w.v), v));
                 STEP(cacti_hip_add_f16(T * D, vc + prev * D * 2, v, vc + prev * D * 2, st));
                 // scores against the cache, row-causal mask + softmax (in place), P V.  Columns from
                 // `next` on are masked for every row, so only the first Cw of the cap columns are formed.
@@ -786,16 +799,16 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
                     STEP(cacti_hip_row_causal_softmax_fwd(T, H, Cw, Cw, prev, s16, s16, st));
                     STEP(cacti_hip_gemm_f16_strided_batched(0, 0, H, T, Dh, Cw, 1.f, s16, H * Cw, Cw, vc, D, Dh, 0.f, attn, D, Dh, st));
                 }
-                STEP(cacti_hip_gemm_f16(0, 1, T, D, D, 1.f, attn, D, P(w.o), D, 0.f, o, D, st));
+                STEP(product(D, D, attn, P(w.o), o));
                 STEP(cacti_hip_add_rms_norm_fwd(T, D, x, o, P(w.post_norm), g.eps, x1, post, st));
-                STEP(cacti_hip_gemm_f16(0, 1, T, F, D, 1.f, post, D, P(w.up), D, 0.f, up, F, st));
-                STEP(cacti_hip_gemm_f16(0, 1, T, F, D, 1.f, post, D, P(w.gate), D, 0.f, gate, F, st));
+                STEP(product(F, D, post, P(w.up), up));
+                STEP(product(F, D, post, P(w.gate), gate));
                 STEP(cacti_hip_silu_gate_fwd(T * F, gate, up, h, st));
-                STEP(cacti_hip_gemm_f16(0, 1, T, D, F, 1.f, h, F, P(w.down), F, 0.f, down, D, st));
+                STEP(product(D, F, h, P(w.down), down));
                 const CellPtr wn = l + 1 < m->layers.size() ? m->layers[l + 1].pre_norm : m->head_norm;
                 STEP(cacti_hip_add_rms_norm_fwd(T, D, x1, down, P(wn), g.eps, x, pre, st));
             }
-            STEP(cacti_hip_gemm_f16(0, 1, T, V, D, 1.f, pre, D, P(m->lm_head), D, 0.f, logit, V, st));
+            STEP(product(V, D, pre, P(m->lm_head), logit));
         }
         void *otok = c.dev_ptr(k->out_tok);
         STEP(cacti_hip_softmax_ce_fwd(T, V, logit, nullptr, want_prob ? c.dev_ptr(k->out_prob) : nullptr, nullptr,

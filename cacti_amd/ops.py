@@ -5,6 +5,8 @@ given) in the reference's terms (src/thunk/mod.rs:347-351), executed by the HIP 
 behind the C ABI.  torch is used only to own device memory and name the stream; every
 computation goes through libcacti_gpu_hip_ffi.so and fails if it is not built.
 """
+import ctypes
+
 import torch
 
 from . import ffi
@@ -42,14 +44,23 @@ def gemm(a, b, ta=False, tb=False, alpha=1.0, beta=0.0, out=None):
         assert beta == 0.0
         out = torch.empty((M, N), dtype=F16, device=a.device)
     assert out.shape == (M, N) and out.stride(1) == 1
-    ffi.call("cacti_hip_gemm_f16", int(ta), int(tb), M, N, K, alpha, a.data_ptr(), a.stride(0),
-             b.data_ptr(), b.stride(0), beta, out.data_ptr(), out.stride(0), _stream())
+    _gemm(ta, tb, M, N, K, alpha, a, b, beta, out)
     return out
+
+
+def _gemm(ta, tb, M, N, K, alpha, a, b, beta, out):
+    need = ctypes.c_size_t()
+    args = (ta, tb, M, N, K, alpha, a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), beta, out.data_ptr(), out.stride(0))
+    st = _stream()
+    ffi.call("cacti_hip_gemm_f16_ws", *args, None, 0, need, st)
+    if need.value:                               # not launched: the product wants a workspace
+        ws = torch.empty(need.value, dtype=torch.uint8, device=a.device)
+        ffi.call("cacti_hip_gemm_f16_ws", *args, ws.data_ptr(), need.value, need, st)
 
 
 def gemm_batched(As, Bs, ta=False, tb=False, alpha=1.0, beta=0.0, outs=None):
     """Pointer-array batch: outs[z] = f16(alpha op(As[z]) op(Bs[z]) + beta outs[z]), one shape."""
-    import ctypes as C
+    C = ctypes
     n = len(As)
     a, b = As[0], Bs[0]
     M, K = (a.shape[1], a.shape[0]) if ta else a.shape
@@ -57,6 +68,11 @@ def gemm_batched(As, Bs, ta=False, tb=False, alpha=1.0, beta=0.0, outs=None):
     if outs is None:
         assert beta == 0.0
         outs = [torch.empty((M, N), dtype=F16, device=a.device) for _ in range(n)]
+    if any(x % 8 for x in (a.shape[1], b.shape[1], N, a.stride(0), b.stride(0), outs[0].stride(0))):
+        # rows that are not 16-byte aligned run one after another; each may want a workspace
+        for x, y, z in zip(As, Bs, outs):
+            _gemm(ta, tb, M, N, K, alpha, x, y, beta, z)
+        return outs
     arr = lambda ts: C.cast((C.c_void_p * n)(*[t.data_ptr() for t in ts]), C.c_void_p)
     ffi.call("cacti_hip_gemm_f16_batched", int(ta), int(tb), n, M, N, K, alpha, arr(As), a.stride(0), arr(Bs),
              b.stride(0), beta, arr(outs), outs[0].stride(0), _stream())

@@ -313,6 +313,34 @@ def test_gemm_direct_load_kernels(ops, oracle, ta, tb, M, N, K):
         assert exact_frac(got, want) > 0.98
 
 
+# every tile shape of the direct kernels with a K that ends inside a k tile (also shorter than one), sums in parts of K
+# (few tiles, long K; the last part shorter than the others), and operands and results of any alignment
+ANY_SHAPES = [
+    (0, 1, 72, 200, 1000), (0, 0, 72, 200, 1000), (1, 0, 72, 200, 1001), (1, 1, 72, 200, 136), (1, 0, 256, 264, 8), (0, 0, 136, 72, 24),
+    (1, 0, 1032, 1096, 611), (0, 1, 776, 1104, 520), (1, 0, 2056, 2304, 129), (1, 0, 3200, 3200, 37), (0, 0, 1100, 4104, 72),
+    (0, 1, 37, 512, 4096), (0, 0, 64, 64, 8200), (1, 0, 136, 64, 3001), (0, 1, 5, 1003, 3000), (1, 0, 40, 72, 2600),
+    (0, 1, 61, 35, 127), (0, 0, 129, 257, 193), (1, 0, 130, 258, 65), (1, 1, 7, 9, 130), (0, 0, 300, 1004, 772), (0, 1, 1, 3, 333),
+    (0, 0, 33, 31, 4001), (1, 0, 1025, 1027, 67),
+]
+
+
+@pytest.mark.parametrize("ta,tb,M,N,K", ANY_SHAPES)
+def test_gemm_tails_parts_and_odd_sizes(ops, oracle, ta, tb, M, N, K):
+    say("gemm any", ta, tb, M, N, K)
+    r = rng(990 + M + N + K + 2 * ta + tb)
+    A = randn16(r, (K, M) if ta else (M, K))
+    B = randn16(r, (N, K) if tb else (K, N), 0.1)
+    C0 = randn16(r, (M, N))
+    for alpha, beta in [(1.0, 0.0), (0.5, 1.0)]:
+        want = oracle.matmul(ta, tb, A, B, alpha, beta, C0)
+        c = torch.full((M * N + 16,), 7.0, dtype=torch.float16, device="cuda")      # what lies behind C stays
+        c[:M * N] = dev(C0).view(-1)
+        got = host(ops.gemm(dev(A), dev(B), bool(ta), bool(tb), alpha, beta, c[:M * N].view(M, N)))
+        assert_parity(got, want, "gemm any")
+        assert exact_frac(got, want) > 0.97
+        assert (c[M * N:] == 7.0).all()
+
+
 # one to four rows against a weight matrix (decoding): the streaming kernel, including a row count
 # of columns that is not a multiple of its 4 rows per workgroup, a short K, and a padded weight matrix
 SKINNY_SHAPES = [(1, 3200, 3200, 0), (2, 8640, 3200, 0), (3, 3200, 8640, 8), (4, 1000, 136, 0), (1, 32000, 3200, 0),
