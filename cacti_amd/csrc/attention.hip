@@ -1736,8 +1736,8 @@ CACTI_API size_t cacti_hip_attention_bwd_workspace(int64_t S, int64_t H)
     return (S > 0 && H > 0) ? (size_t)(2 * S * H) * sizeof(float) : 0;
 }
 
-CACTI_API int cacti_hip_attention_fwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,
-                                      const void *v, int64_t ld, void *o, void *stats, void *stream)
+static int attention_fwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k, const void *v, int64_t ld, void *o,
+                         void *stats, bool exact, hipStream_t st)
 {
     int rc = check_shape("attention_fwd", S, H, Dh, ld);
     if (rc) return rc;
@@ -1750,11 +1750,27 @@ CACTI_API int cacti_hip_attention_fwd(int64_t S, int64_t H, int64_t Dh, float al
     p.out = (half_t *)o;
     p.m = (float *)stats;
     p.l = p.m + S * H;
-    hipStream_t st = (hipStream_t)stream;
     int64_t span;
     const bool dma = direct_tiles(H, Dh, ld, {q, k, v, o}, &span);
-    return dispatch<Fwd>(span, g_exact.load(std::memory_order_relaxed) != 0, dma, p, st);
+    return dispatch<Fwd>(span, exact, dma, p, st);
 }
+
+CACTI_API int cacti_hip_attention_fwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,
+                                      const void *v, int64_t ld, void *o, void *stats, void *stream)
+{
+    return attention_fwd(S, H, Dh, alpha, q, k, v, ld, o, stats, g_exact.load(std::memory_order_relaxed) != 0, (hipStream_t)stream);
+}
+
+namespace cacti {
+
+// the exactly rounded form whatever the process-wide setting, for the cached forward pass
+int attention_fwd_exact(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k, const void *v, int64_t ld, void *o,
+                        void *stats, hipStream_t st)
+{
+    return attention_fwd(S, H, Dh, alpha, q, k, v, ld, o, stats, true, st);
+}
+
+}  // namespace cacti
 
 CACTI_API int cacti_hip_attention_bwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,
                                       const void *v, const void *o, const void *dO, int64_t ld, const void *stats,

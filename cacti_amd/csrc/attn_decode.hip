@@ -4,18 +4,19 @@
 // with the reference's rounding points (scores and probabilities are f16 values, both products
 // accumulate in fp32 and round once).
 //
-// With a single query row per head the tiled GEMM kernels cannot fill the chip (one tile per
-// head), so the cache is cut into slices of 128 positions and every (head, slice) pair is a
-// workgroup, in three launches:
-//   scores : s16[t,h,j] = f16(alpha q[t,h,:] . K[j,h,:]) for the slice's j
-//   values : the row maximum and sum over the live columns are recomputed from s16 by every
-//            workgroup (a row is a few KiB in L2), p = f16(e / sum) for the slice, partial
-//            out[t,h,:] = sum_j p[j] V[j,h,:] per slice, in fp32
-//   reduce : the slices' partial sums added in slice order and rounded once.  (Letting the last
-//            workgroup of a head do this inside the second launch needs a device-wide fence,
-//            which writes back and invalidates a whole L2 on this chip: it cost 40 us.)
-// K and V rows of a head are Dh contiguous halves, read as 8-byte pieces: consecutive lanes take
-// consecutive pieces, rows follow one another, so every wave access is a few contiguous runs.
+// A single query row per head is a few hundred KB of cache and hardly any arithmetic: what it costs is launches and
+// round trips to memory.  A workgroup takes a head and a piece of its dimension (up to 32 columns), over all positions:
+// the probabilities of a row need the sum over the whole row before the first product with V is formed, and a split
+// over positions would need that sum, and then the partial outputs, exchanged between workgroups (another launch each;
+// a device-wide fence inside the launch costs 40 us on this chip).  Every piece's workgroup forms the head's scores
+// itself, K coming out of L2 for all but the first; from kOwnScores positions on, where that would be most of the
+// time, the scores come from a launch of their own, one workgroup per head and 128 positions.  One launch instead of
+// three (scores, values per 128 positions, sum): 69 positions, 32 heads of 100: 12.9 -> 5 us.
+//
+// Eight lanes share a position, each with 8-byte pieces of the head (a head starts on a multiple of 8 bytes), 64
+// contiguous bytes per access; four positions per lane are in flight together, and the first four V pieces are
+// requested before anything else.  Loads are unconditional with clamped indices: a load inside a branch is waited for
+// at the end of the branch.
 #include "common.h"
 #include "softmax_math.h"
 
@@ -24,147 +25,139 @@ using namespace cacti;
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kSlice = 128;                // cached positions per workgroup
-constexpr int kMaxPieces = 32;             // Dh <= 128
+constexpr int kGroups = kThreads / 8;      // positions per step and lane
+constexpr int kStep = 4;                   // positions of a lane in flight
+constexpr int kSlice = kGroups * kStep;    // positions per workgroup of the scores launch
+constexpr int kOwnScores = 1024;
+constexpr int kMaxCols = 8192;             // score rows live in LDS
 
 struct __attribute__((aligned(8))) h4 {
     half_t v[4];
 };
 
-template <int T>
-__global__ void __launch_bounds__(kThreads)
-decode_scores_kernel(int C, int H, int Dh, float alpha, const half_t *__restrict__ q, int64_t ldq,
-                     const half_t *__restrict__ kc, int64_t ldk, int64_t hsk, half_t *__restrict__ s16, int64_t ld)
+__device__ __forceinline__ float dot4(const h4 &a, const h4 &b, float acc)
 {
-    __shared__ float part[T][kSlice * 25 + kSlice];        // [t][row * pieces + piece], pieces <= 26 here
-    const int tid = threadIdx.x, h = blockIdx.y, j0 = blockIdx.x * kSlice;
+    const half2_t a0 = {a.v[0], a.v[1]}, b0 = {b.v[0], b.v[1]}, a1 = {a.v[2], a.v[3]}, b1 = {b.v[2], b.v[3]};
+    return __builtin_amdgcn_fdot2(a1, b1, __builtin_amdgcn_fdot2(a0, b0, acc, false), false);
+}
+
+// The lane's query pieces: piece i8 + 8 i of head h (zeros behind the head).
+template <int T, int NP>
+__device__ __forceinline__ void load_q(h4 (&qv)[T][NP], const half_t *q, int64_t ldq, int h, int Dh, int i8)
+{
     const int pieces = Dh / 4;
-    const int nrow = min(kSlice, C - j0);
-    const int total = nrow * pieces;
-    // All of the lane's loads are issued before the first use: at most 13 pieces of K of 8 bytes,
-    // each with the matching piece of every query row (those hit in L2).  The loads are
-    // unconditional (pieces past the slice re-read its last piece): a load inside a branch is
-    // waited for at the end of the branch, which would turn the 13 loads into 13 round trips.
-    constexpr int kMaxIter = (kSlice * 25 + kThreads - 1) / kThreads;
-    h4 kv[kMaxIter], qv[kMaxIter][T];
 #pragma unroll
-    for (int it = 0; it < kMaxIter; it++) {
-        const int p = min(tid + it * kThreads, total - 1);
-        const int r = p / pieces, c = p - r * pieces;
-        kv[it] = *reinterpret_cast<const h4 *>(kc + (int64_t)(j0 + r) * ldk + h * hsk + 4 * c);
+    for (int i = 0; i < NP; i++) {
+        const int c = i8 + 8 * i;
 #pragma unroll
-        for (int t = 0; t < T; t++) qv[it][t] = *reinterpret_cast<const h4 *>(q + t * ldq + h * Dh + 4 * c);
-    }
-#pragma unroll
-    for (int it = 0; it < kMaxIter; it++) {
-        const int p = tid + it * kThreads;
-        if (p < total) {
-#pragma unroll
-            for (int t = 0; t < T; t++) {
-                float a = 0.f;
-#pragma unroll
-                for (int i = 0; i < 4; i++) a += h2f(qv[it][t].v[i]) * h2f(kv[it].v[i]);
-                part[t][p] = a;
-            }
+        for (int t = 0; t < T; t++) {
+            qv[t][i] = *reinterpret_cast<const h4 *>(q + t * ldq + h * Dh + 4 * min(c, pieces - 1));
+            if (c >= pieces) qv[t][i] = h4{};
         }
-    }
-    __syncthreads();
-    for (int idx = tid; idx < T * nrow; idx += kThreads) {
-        const int t = idx / nrow, r = idx - t * nrow;
-        float a = 0.f;
-        for (int c = 0; c < pieces; c++) a += part[t][r * pieces + c];
-        s16[((int64_t)t * H + h) * ld + j0 + r] = f2h(alpha * a);
     }
 }
 
-__device__ __forceinline__ float block_reduce(float v, bool is_max, float *scratch)
+// f16(alpha q . K[j]) for the positions j0 + g + 32 it (it < kStep) below `end`, by the first of a position's lanes to
+// out[t * ldo + j - first]
+template <int T, int NP>
+__device__ __forceinline__ void scores_step(const h4 (&qv)[T][NP], const half_t *k_head, int64_t ldk, int pieces, float alpha, int j0,
+                                            int end, half_t *out, int64_t ldo, int first)
 {
-    v = is_max ? wave_max(v) : wave_sum(v);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) scratch[wid] = v;
-    __syncthreads();
-    float r = scratch[0];
+    const int i8 = threadIdx.x & 7, g = threadIdx.x >> 3;
+    h4 kv[kStep][NP];
 #pragma unroll
-    for (int w = 1; w < kThreads / 64; w++) r = is_max ? fmaxf(r, scratch[w]) : r + scratch[w];
-    return r;
+    for (int it = 0; it < kStep; it++)
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+            kv[it][i] = *reinterpret_cast<const h4 *>(k_head + (int64_t)min(j0 + g + it * kGroups, end - 1) * ldk +
+                                                      4 * min(i8 + 8 * i, pieces - 1));
+#pragma unroll
+    for (int it = 0; it < kStep; it++)
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+            float a = 0.f;
+#pragma unroll
+            for (int i = 0; i < NP; i++) a = dot4(qv[t][i], kv[it][i], a);
+            a += dpp_f32<0xB1>(a);              // lane ^ 1
+            a += dpp_f32<0x4E>(a);              // lane ^ 2
+            a += dpp_f32<0x141>(a);             // the other four of the eight
+            const int j = j0 + g + it * kGroups;
+            if (i8 == 0 && j < end) out[t * ldo + j - first] = f2h(alpha * a);
+        }
 }
 
-constexpr int kRowIter = 4;                // 8-column pieces of a score row per lane: rows up to 8192 columns
-
-template <int T>
+template <int T, int NP>
 __global__ void __launch_bounds__(kThreads)
-decode_values_kernel(int C, int H, int Dh, int64_t row0, const half_t *__restrict__ s16, int64_t ld,
-                     const half_t *__restrict__ vc, int64_t ldv, int64_t hsv, float *__restrict__ partial)
+decode_scores_kernel(int C, int Dh, float alpha, const half_t *__restrict__ q, int64_t ldq, const half_t *__restrict__ kc, int64_t ldk,
+                     int64_t hsk, half_t *__restrict__ s16, int64_t ld)
 {
-    __shared__ float ps[T][kSlice];
-    __shared__ float red[8][T][kMaxPieces * 4];
-    __shared__ float scratch[kThreads / 64];
-    const int tid = threadIdx.x, h = blockIdx.y, split = blockIdx.x, nsplit = gridDim.x;
-    const int j0 = split * kSlice;
-    const int pieces = Dh / 4;
-    const int nrow = min(kSlice, C - j0);
-    // Every load of the workgroup is issued here, before the first wait: the slice of V (lane
-    // groups of `pieces` lanes, group g takes rows g, g + 8, ...), the score rows (8 columns per
-    // lane and step) and the lane's own column of the slice.
-    constexpr int G = 8;                       // pieces <= 25 lanes per group: 8 groups fit in 256 lanes
-    constexpr int kRowsPerGroup = kSlice / G;
-    const int g = tid / pieces, c = tid - g * pieces;
-    h4 vv[kRowsPerGroup];
-    {
-        // unconditional loads (clamped to the slice's last row and to a piece of the head): see above
-        const int cc = g < G ? c : 0;
+    const int h = blockIdx.y, j0 = blockIdx.x * kSlice;
+    h4 qv[T][NP];
+    load_q<T, NP>(qv, q, ldq, h, Dh, threadIdx.x & 7);
+    scores_step<T, NP>(qv, kc + h * hsk, ldk, Dh / 4, alpha, j0, min(C, j0 + kSlice), s16 + (int64_t)h * T * ld, ld, 0);
+}
+
+// OWN: the scores are formed here; otherwise they are s16[h][t][ld].
+template <int T, int NP, bool OWN>
+__global__ void __launch_bounds__(kThreads)
+decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__restrict__ q, int64_t ldq, const half_t *__restrict__ kc,
+                     const half_t *__restrict__ vc, int64_t ldkv, int64_t hs, const half_t *__restrict__ s16, int64_t ld,
+                     half_t *__restrict__ out, int64_t ldo)
+{
+    extern __shared__ __attribute__((aligned(16))) half_t sp[];           // [T][ld]: scores, then probabilities
+    __shared__ float scratch[2][T][kThreads / 64];
+    __shared__ float red[kThreads / 64][T][8][4];
+    const int tid = threadIdx.x, i8 = tid & 7, g = tid >> 3, lane = tid & 63, wid = tid >> 6, h = blockIdx.y;
+    const int pieces = Dh / 4, per = (pieces + gridDim.x - 1) / gridDim.x;        // pieces of this workgroup: at most 8
+    const int piece = blockIdx.x * per + i8;
+    const bool mine = i8 < per && piece < pieces;
+    const half_t *vp = vc + h * hs + 4 * (mine ? piece : 0);
+    auto load_v = [&](h4 (&v)[kStep], int j0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int it = 0; it < kRowsPerGroup; it++) {
-            const int r = min((g < G ? g : 0) + it * G, nrow - 1);
-            vv[it] = *reinterpret_cast<const h4 *>(vc + (int64_t)(j0 + r) * ldv + h * hsv + 4 * cc);
-        }
+        for (int it = 0; it < kStep; it++)
+            v[it] = *reinterpret_cast<const h4 *>(vp + (int64_t)min(j0 + g + it * kGroups, C - 1) * ldkv);
+    };
+    h4 vv[kStep];
+    load_v(vv, 0);
+    if (OWN) {
+        h4 qv[T][NP];
+        load_q<T, NP>(qv, q, ldq, h, Dh, i8);
+        for (int j0 = 0; j0 < C; j0 += kSlice) scores_step<T, NP>(qv, kc + h * hs, ldkv, pieces, alpha, j0, C, sp, ld, 0);
+    } else {
+        for (int i = tid; i < T * (int)ld / 8; i += kThreads) st8(sp + i * 8, ld8(s16 + (int64_t)h * T * ld + i * 8));
     }
-    h8 rowv[T][kRowIter];
-    half_t own[T];
+    __syncthreads();
+    // row maxima, then sums of exponentials, then the probabilities in place of the scores; row t sees live(t) positions
+    auto live = [&](int t) __attribute__((always_inline)) { return (int)min((int64_t)C, (int64_t)t + row0 + 1); };
+    float mx[T], sum[T];
 #pragma unroll
     for (int t = 0; t < T; t++) {
-        const half_t *sr = s16 + ((int64_t)t * H + h) * ld;
-        const int live = (int)min((int64_t)C, (int64_t)t + row0 + 1);
-        const int last8 = ((live - 1) / 8) * 8;                        // live >= 1
-#pragma unroll
-        for (int it = 0; it < kRowIter; it++) {
-            const int j8 = min((tid + it * kThreads) * 8, last8);      // rows are 16-byte aligned, ld % 8 == 0
-            rowv[t][it] = ld8(sr + j8);
-        }
-        own[t] = sr[min(j0 + tid, live - 1)];
+        float m = -INFINITY;
+        for (int j = tid; j < live(t); j += kThreads) m = fmaxf(m, h2f(sp[t * ld + j]));
+        m = wave_max(m);
+        if (lane == 0) scratch[0][t][wid] = m;
     }
-    // probabilities of the slice: every row's maximum and sum run over all its live columns
+    __syncthreads();
 #pragma unroll
     for (int t = 0; t < T; t++) {
-        const int live = (int)min((int64_t)C, (int64_t)t + row0 + 1);
-        float mx = -INFINITY;
+        mx[t] = scratch[0][t][0];
 #pragma unroll
-        for (int it = 0; it < kRowIter; it++) {
-            const int j8 = (tid + it * kThreads) * 8;
-            if (j8 < live) {
+        for (int w = 1; w < kThreads / 64; w++) mx[t] = fmaxf(mx[t], scratch[0][t][w]);
+        float s = 0.f;
+        for (int j = tid; j < live(t); j += kThreads) s += exp_nonpos(fmaxf(h2f(sp[t * ld + j]) - mx[t], -100.0f));
+        s = wave_sum(s);
+        if (lane == 0) scratch[1][t][wid] = s;
+    }
+    __syncthreads();
 #pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (j8 + i < live) mx = fmaxf(mx, h2f(rowv[t][it].v[i]));
-            }
-        }
-        mx = block_reduce(mx, true, scratch);
-        float sum = 0.f;
+    for (int t = 0; t < T; t++) {
+        sum[t] = scratch[1][t][0];
 #pragma unroll
-        for (int it = 0; it < kRowIter; it++) {
-            const int j8 = (tid + it * kThreads) * 8;
-            if (j8 < live) {
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (j8 + i < live) sum += exp_nonpos(fmaxf(h2f(rowv[t][it].v[i]) - mx, -100.0f));
-            }
-        }
-        sum = block_reduce(sum, false, scratch);
-        const RowDivide div(sum);
-        if (tid < kSlice) {
-            float p = 0.f;
-            if (tid < nrow && j0 + tid < live) p = h2f(f2h(div(exp_nonpos(fmaxf(h2f(own[t]) - mx, -100.0f)))));
-            ps[t][tid] = p;
+        for (int w = 1; w < kThreads / 64; w++) sum[t] += scratch[1][t][w];
+        const RowDivide div(sum[t]);
+        for (int j = tid; j < C; j += kThreads) {
+            const float e = exp_nonpos(fmaxf(h2f(sp[t * ld + j]) - mx[t], -100.0f));
+            sp[t * ld + j] = j < live(t) ? f2h(div(e)) : (half_t)0.f;
         }
     }
     __syncthreads();
@@ -173,45 +166,88 @@ decode_values_kernel(int C, int H, int Dh, int64_t row0, const half_t *__restric
     for (int t = 0; t < T; t++)
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[t][i] = 0.f;
-    if (g < G) {
+    for (int j0 = 0; j0 < C; j0 += kSlice) {
+        h4 vn[kStep];
+        load_v(vn, j0 + kSlice);                                  // (behind the last position: its row again)
 #pragma unroll
-        for (int it = 0; it < kRowsPerGroup; it++) {
-            const int r = g + it * G;
-            if (r < nrow) {
+        for (int it = 0; it < kStep; it++) {
+            const int j = j0 + g + it * kGroups;
 #pragma unroll
-                for (int t = 0; t < T; t++)
+            for (int t = 0; t < T; t++) {
+                const float p = j < C ? h2f(sp[t * ld + j]) : 0.f;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) acc[t][i] += ps[t][r] * h2f(vv[it].v[i]);
+                for (int i = 0; i < 4; i++) acc[t][i] += p * h2f(vv[it].v[i]);
             }
         }
 #pragma unroll
-        for (int t = 0; t < T; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) red[g][t][4 * c + i] = acc[t][i];
+        for (int it = 0; it < kStep; it++) vv[it] = vn[it];
     }
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float a = acc[t][i];
+            a += __shfl_xor(a, 8, 64);
+            a += swz_xor16(a);
+            a += xor32(a);
+            if (lane < 8) red[wid][t][lane][i] = a;
+        }
     __syncthreads();
-    float *mine = partial + ((int64_t)h * nsplit + split) * T * Dh;
-    for (int idx = tid; idx < T * Dh; idx += kThreads) {
-        const int t = idx / Dh, d = idx - t * Dh;
-        float a = 0.f;
-        for (int gg = 0; gg < G; gg++) a += red[gg][t][d];
-        mine[idx] = a;
+    if (tid < T * 32) {
+        const int t = tid >> 5, c = (tid >> 2) & 7, i = tid & 3;
+        if (c < per && blockIdx.x * per + c < pieces) {
+            float a = red[0][t][c][i];
+#pragma unroll
+            for (int w = 1; w < kThreads / 64; w++) a += red[w][t][c][i];
+            out[t * ldo + h * Dh + 4 * (blockIdx.x * per + c) + i] = f2h(a);
+        }
     }
 }
 
-// out[t,h,:] = f16(sum over the slices, in slice order, of the partial products)
-template <int T>
-__global__ void __launch_bounds__(128)
-decode_reduce_kernel(int nsplit, int Dh, const float *__restrict__ partial, half_t *__restrict__ out, int64_t ldo)
+struct DecodeArgs {
+    int C, H, Dh;
+    int64_t row0;
+    float alpha;
+    const half_t *q;
+    int64_t ldq;
+    const half_t *kc, *vc;
+    int64_t ldkv, hs;
+    half_t *out;
+    int64_t ldo;
+    half_t *s16;
+    hipStream_t st;
+};
+
+template <int T, int NP>
+int launch(const DecodeArgs &a)
 {
-    const int h = blockIdx.x;
-    const float *all = partial + (int64_t)h * nsplit * T * Dh;
-    for (int idx = threadIdx.x; idx < T * Dh; idx += 128) {
-        const int t = idx / Dh, d = idx - t * Dh;
-        float a = 0.f;
-        for (int s = 0; s < nsplit; s++) a += all[(int64_t)s * T * Dh + idx];
-        out[(int64_t)t * ldo + h * Dh + d] = f2h(a);
+    const int64_t ld = (a.C + 7) / 8 * 8;
+    const size_t smem = (size_t)T * (size_t)ld * sizeof(half_t);
+    const dim3 grid((unsigned)((a.Dh / 4 + 7) / 8), (unsigned)a.H), block(kThreads);
+    if (a.C <= kOwnScores) {
+        hipLaunchKernelGGL((decode_values_kernel<T, NP, true>), grid, block, smem, a.st, a.C, a.Dh, a.row0, a.alpha, a.q, a.ldq, a.kc, a.vc,
+                           a.ldkv, a.hs, (const half_t *)nullptr, ld, a.out, a.ldo);
+    } else {
+        if (smem > 48 * 1024) {
+            static DeviceOnce attr_set;
+            if (!attr_set.fresh()) {
+                CACTI_HIP(hipFuncSetAttribute((const void *)decode_values_kernel<T, NP, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              T * kMaxCols * (int)sizeof(half_t)));
+                attr_set.mark();
+            }
+        }
+        hipLaunchKernelGGL((decode_scores_kernel<T, NP>), dim3((unsigned)((a.C + kSlice - 1) / kSlice), (unsigned)a.H), block, 0, a.st, a.C,
+                           a.Dh, a.alpha, a.q, a.ldq, a.kc, a.ldkv, a.hs, a.s16, ld);
+        hipLaunchKernelGGL((decode_values_kernel<T, NP, false>), grid, block, smem, a.st, a.C, a.Dh, a.row0, a.alpha, a.q, a.ldq, a.kc, a.vc,
+                           a.ldkv, a.hs, (const half_t *)a.s16, ld, a.out, a.ldo);
     }
+    return launch_status("attn_decode");
+}
+
+template <int NP>
+int launch_rows(int64_t T, const DecodeArgs &a)
+{
+    return T == 1 ? launch<1, NP>(a) : T == 2 ? launch<2, NP>(a) : T == 3 ? launch<3, NP>(a) : launch<4, NP>(a);
 }
 
 }  // namespace
@@ -219,9 +255,7 @@ decode_reduce_kernel(int nsplit, int Dh, const float *__restrict__ partial, half
 CACTI_API size_t cacti_hip_attn_decode_workspace(int64_t T, int64_t H, int64_t Dh, int64_t C)
 {
     if (T <= 0 || H <= 0 || Dh <= 0 || C <= 0) return 0;
-    const int64_t ld = (C + 7) / 8 * 8, nsplit = (C + kSlice - 1) / kSlice;
-    // scores [T,H,ld] f16, then the per-slice partial outputs [H,nsplit,T,Dh] f32
-    return (size_t)((T * H * ld * 2 + 255) / 256 * 256 + H * nsplit * T * Dh * 4);
+    return (size_t)(T * H * ((C + 7) / 8 * 8) * 2);               // scores [H, T, C rounded up] f16
 }
 
 CACTI_API int cacti_hip_attn_decode_f16(int64_t T, int64_t H, int64_t Dh, int64_t C, int64_t initial_row, float alpha,
@@ -229,12 +263,11 @@ CACTI_API int cacti_hip_attn_decode_f16(int64_t T, int64_t H, int64_t Dh, int64_
                                         int64_t ldkv, int64_t head_stride, void *out, int64_t ldo, void *workspace,
                                         size_t workspace_bytes, void *stream)
 {
-    CACTI_REQUIRE(T >= 1 && T <= 4 && H > 0 && C > 0 && initial_row >= 0, CACTI_E_NOTIMPL,
+    CACTI_REQUIRE(T >= 1 && T <= 4 && H > 0 && H <= 65535 && C > 0 && initial_row >= 0, CACTI_E_NOTIMPL,
                   "attn_decode: 1 to 4 rows are handled here (T=%lld)", (long long)T);
-    CACTI_REQUIRE(Dh % 4 == 0 && Dh >= 4 && Dh <= 100, CACTI_E_NOTIMPL, "attn_decode: need Dh %% 4 == 0 and Dh <= 100");
+    CACTI_REQUIRE(Dh % 4 == 0 && Dh >= 4 && Dh <= 128, CACTI_E_NOTIMPL, "attn_decode: need Dh %% 4 == 0 and Dh <= 128");
     CACTI_REQUIRE(q && k_cache && v_cache && out && workspace, CACTI_E_INVALID, "attn_decode: null pointer");
-    CACTI_REQUIRE(C <= (int64_t)kRowIter * kThreads * 8, CACTI_E_NOTIMPL, "attn_decode: at most %d cached positions",
-                  kRowIter * kThreads * 8);
+    CACTI_REQUIRE(C <= kMaxCols, CACTI_E_NOTIMPL, "attn_decode: at most %d cached positions", kMaxCols);
     CACTI_REQUIRE(ldq % 4 == 0 && ldkv % 4 == 0 && head_stride % 4 == 0 && aligned(q, 8) && aligned(k_cache, 8) && aligned(v_cache, 8) &&
                       aligned(workspace, 16),
                   CACTI_E_INVALID, "attn_decode: operands must be 8-byte aligned with row pitches that are multiples of 4");
@@ -242,26 +275,7 @@ CACTI_API int cacti_hip_attn_decode_f16(int64_t T, int64_t H, int64_t Dh, int64_
                   "attn_decode: workspace too small");
     // columns beyond the last row's position are masked for every row: they are not formed
     const int64_t live = C < T + initial_row ? C : T + initial_row;
-    const int64_t ld = (C + 7) / 8 * 8;
-    half_t *s16 = static_cast<half_t *>(workspace);
-    float *partial = reinterpret_cast<float *>(static_cast<char *>(workspace) + (T * H * ld * 2 + 255) / 256 * 256);
-    const dim3 grid((unsigned)((live + kSlice - 1) / kSlice), (unsigned)H), block(kThreads);
-    hipStream_t st = (hipStream_t)stream;
-#define LAUNCH(TT)                                                                                                     \
-    do {                                                                                                               \
-        hipLaunchKernelGGL((decode_scores_kernel<TT>), grid, block, 0, st, (int)live, (int)H, (int)Dh, alpha,          \
-                           (const half_t *)q, ldq, (const half_t *)k_cache, ldkv, head_stride, s16, ld);               \
-        hipLaunchKernelGGL((decode_values_kernel<TT>), grid, block, 0, st, (int)live, (int)H, (int)Dh, initial_row, s16, \
-                           ld, (const half_t *)v_cache, ldkv, head_stride, partial);                                   \
-        hipLaunchKernelGGL((decode_reduce_kernel<TT>), dim3((unsigned)H), dim3(128), 0, st, (int)grid.x, (int)Dh,      \
-                           (const float *)partial, (half_t *)out, ldo);                                                \
-    } while (0)
-    switch (T) {
-        case 1: LAUNCH(1); break;
-        case 2: LAUNCH(2); break;
-        case 3: LAUNCH(3); break;
-        default: LAUNCH(4); break;
-    }
-#undef LAUNCH
-    return launch_status("attn_decode");
+    const DecodeArgs a = {(int)live, (int)H, (int)Dh, initial_row, alpha, (const half_t *)q, ldq, (const half_t *)k_cache,
+                          (const half_t *)v_cache, ldkv, head_stride, (half_t *)out, ldo, (half_t *)workspace, (hipStream_t)stream};
+    return Dh <= 64 ? launch_rows<2>(T, a) : launch_rows<4>(T, a);
 }

@@ -171,6 +171,51 @@ rope_pair_kernel(int64_t S, int H, int Dh, const half_t *__restrict__ in0,
     }
 }
 
+// The new rows of a prompt on their way to attention, in one launch: blockIdx.y = 0 rotates the queries, 1 adds the
+// rotated keys to their cache rows, 2 adds the values to theirs, with the rounding points of the separate thunks.
+__global__ void __launch_bounds__(kThreads)
+rope_cache_kernel(int64_t S, int H, int Dh, const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v,
+                  const half_t *__restrict__ cos16, const half_t *__restrict__ sin16, half_t *qr, half_t *kc, half_t *vc)
+{
+    const int z = blockIdx.y;
+    const half_t *__restrict__ in = z == 0 ? q : z == 1 ? k : v;
+    half_t *out = z == 0 ? qr : z == 1 ? kc : vc;
+    const int hf = Dh / 2, pph = hf / 2;
+    const int64_t per_tok = (int64_t)H * pph, total = S * per_tok;
+    for (int64_t it = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; it < total; it += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t s = it / per_tok;
+        const int r = (int)(it - s * per_tok);
+        const int h = r / pph, d = (r - h * pph) * 2;
+        const int64_t eL = (s * H + h) * Dh + d, eR = eL + hf;
+        const int64_t tL = s * Dh + d, tR = tL + hf;
+        half2_t oL = *reinterpret_cast<const half2_t *>(in + eL), oR = *reinterpret_cast<const half2_t *>(in + eR);
+        half2_t qL, qR;
+        if (z > 0) {
+            qL = *reinterpret_cast<const half2_t *>(out + eL);
+            qR = *reinterpret_cast<const half2_t *>(out + eR);
+        }
+        if (z < 2) {
+            const half2_t cL = *reinterpret_cast<const half2_t *>(cos16 + tL), cR = *reinterpret_cast<const half2_t *>(cos16 + tR);
+            const half2_t sL = *reinterpret_cast<const half2_t *>(sin16 + tL), sR = *reinterpret_cast<const half2_t *>(sin16 + tR);
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const float xl = h2f(oL[i]), xr = h2f(oR[i]);
+                oL[i] = f2h(rnd16(xl * h2f(cL[i])) - rnd16(xr * h2f(sL[i])));
+                oR[i] = f2h(rnd16(xr * h2f(cR[i])) + rnd16(xl * h2f(sR[i])));
+            }
+        }
+        if (z > 0) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                oL[i] = f2h(h2f(qL[i]) + h2f(oL[i]));
+                oR[i] = f2h(h2f(qR[i]) + h2f(oR[i]));
+            }
+        }
+        *reinterpret_cast<half2_t *>(out + eL) = oL;
+        *reinterpret_cast<half2_t *>(out + eR) = oR;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // SiLU gate.  forward: y = f16(g / (1 + exp(-g))); h = f16(y u).
 __global__ void __launch_bounds__(kThreads)
@@ -411,6 +456,21 @@ static int rope_launch(bool bwd, int64_t S, int64_t H, int64_t Dh, const void *i
                            (const half_t *)c, (const half_t *)s, (half_t *)out, 0);
     return launch_status("rope");
 }
+
+namespace cacti {
+
+// Dh % 4 == 0; every pointer 4-byte aligned
+int rope_cache_launch(int64_t S, int64_t H, int64_t Dh, const void *q, const void *k, const void *v, const void *cos16, const void *sin16,
+                      void *q_rot, void *k_cache_rows, void *v_cache_rows, hipStream_t st)
+{
+    const dim3 grid((unsigned)grid_for(S * H * (Dh / 4), kThreads, 4096), 3);
+    hipLaunchKernelGGL(rope_cache_kernel, grid, dim3(kThreads), 0, st, S, (int)H, (int)Dh, (const half_t *)q, (const half_t *)k,
+                       (const half_t *)v, (const half_t *)cos16, (const half_t *)sin16, (half_t *)q_rot, (half_t *)k_cache_rows,
+                       (half_t *)v_cache_rows);
+    return launch_status("rope_cache");
+}
+
+}  // namespace cacti
 
 CACTI_API int cacti_hip_rope_fwd(int64_t S, int64_t H, int64_t Dh, const void *x,
                                  const void *cos16, const void *sin16, void *y, void *stream)

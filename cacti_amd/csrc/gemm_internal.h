@@ -70,4 +70,24 @@ int gemm_nt_smallk_launch(const GemmArgs &p, int64_t nblk, hipStream_t st);
 int gemm_skinny_nt_launch(int64_t M, int64_t N, int64_t K, float alpha, const half_t *A, int64_t lda,
                           const half_t *B, int64_t ldb, half_t *C, int64_t ldc, hipStream_t st);
 
+// The decoding kernels of gemm_skinny.hip as the cached forward pass uses them (1 to 4 rows of K <= 8192 elements,
+// K % 8 == 0, everything 16-byte aligned).  The rows are rms_norm(x or f16(x + x2), w_norm); with tok, row m of x is row
+// tok[m] of a table of `vocab` rows (an id out of range raises *status to m + 1).
+struct RowSource {
+    const void *x, *x2, *w_norm;
+    float eps;
+    const uint16_t *tok;
+    int64_t vocab;
+    int *status;
+};
+int rows_qkv_launch(int64_t M, int64_t H, int64_t Dh, const RowSource &x, void *sum_out, const void *Wq, const void *Wk, const void *Wv,
+                    const void *cos16, const void *sin16, void *q_rot, void *k_cache_rows, void *v_cache_rows, hipStream_t st);
+int rows_gate_launch(int64_t M, int64_t N, int64_t K, const RowSource &x, void *sum_out, const void *B, const void *B_mul, void *C,
+                     hipStream_t st);
+int rows_norm_launch(int64_t M, int64_t N, int64_t K, const RowSource &x, const void *B, void *C, hipStream_t st);
+// logit = rows B^T and the arg max of each row in out_tok; the last row's token is added to in_tok[pos] where pos >= 0
+size_t rows_head_scratch_bytes(int64_t M, int64_t N);
+int rows_head_launch(int64_t M, int64_t N, int64_t K, const RowSource &x, const void *B, void *logit, void *scratch, void *out_tok,
+                     void *in_tok, int64_t pos, hipStream_t st);
+
 }  // namespace cacti

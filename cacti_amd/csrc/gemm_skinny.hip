@@ -49,13 +49,30 @@ struct SkinnyArgs {
     const half_t *cos16, *sin16;
     half_t *kc, *vc;
     int H, Dh;
+    // NORM: with tok, row m of x is row tok[m] of A (the embedding of `vocab` rows); an id out of range raises
+    // *status to m + 1 and reads the last row
+    const uint16_t *tok;
+    int64_t vocab;
+    int *status;
+    // E_PLAIN: with cand, the largest result of the workgroup's columns, cand[m * workgroups + workgroup] (arg_key)
+    uint32_t *cand;
 };
 enum : int { E_PLAIN = 0, E_GATE = 1, E_QKV = 2 };
 
+// An f16 result and its column (below 65536) as one number that orders as the arg max does: by value, the first
+// column of equal values (+0 and -0 are equal), no NaN.
+__device__ __forceinline__ uint32_t arg_key(half_t v, int64_t n)
+{
+    uint16_t b = __builtin_bit_cast(uint16_t, v);
+    if ((b & 0x7fff) > 0x7c00) return 0;
+    if (b == 0x8000) b = 0;
+    const uint32_t o = b & 0x8000 ? (uint16_t)~b : b | 0x8000u;
+    return o << 16 | (uint32_t)(0xffff - n);
+}
+
 __device__ __forceinline__ float block_sum(float v, float *scratch)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    v = wave_sum(v);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     __syncthreads();
     if (lane == 0) scratch[wid] = v;
@@ -117,6 +134,19 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
             if (GATE) brow[NB - 1][r] = p.B2 + n * p.ldb;
         }
     }
+    const half_t *arow[M];
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+        arow[m] = p.A + m * p.lda;
+        if (NORM && p.tok) {
+            int64_t id = p.tok[m];
+            if (id >= p.vocab) {
+                if (tid == 0 && blockIdx.x == 0 && blockIdx.y == 0 && p.status) atomicMax(p.status, m + 1);
+                id = p.vocab - 1;
+            }
+            arow[m] = p.A + id * p.lda;
+        }
+    }
     const int64_t chunks = p.K / 8;
     for (int64_t base = 0; base < chunks; base += (int64_t)kPre * kThreads) {
         half8_t b[kPre][NB][kRows];
@@ -132,7 +162,7 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
                 for (int r = 0; r < kRows; r++)
                     b[j][q][r] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(brow[q][r]) + c);
 #pragma unroll
-            for (int m = 0; m < M; m++) a[j][m] = ld8(p.A + m * p.lda + c * 8);
+            for (int m = 0; m < M; m++) a[j][m] = ld8(arow[m] + c * 8);
         }
         if (NORM) {
             // the whole row is in this one batch (K <= 8 * kPre * kThreads, seen to by the launcher)
@@ -200,9 +230,7 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
         for (int m = 0; m < M; m++)
 #pragma unroll
             for (int r = 0; r < kRows; r++) {
-                float v = acc[q][m][r];
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+                const float v = wave_sum(acc[q][m][r]);
                 if (lane == 0) part[wid][(q * M + m) * kRows + r] = v;
             }
     __syncthreads();
@@ -245,6 +273,12 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
 #pragma unroll
             for (int w = 0; w < kThreads / 64; w++) v[q] += part[w][(q * M + m) * kRows + r];
         }
+        if (EPI == E_PLAIN && p.cand) {
+            uint32_t k = n0 + r < p.N ? arg_key(f2h(p.alpha * v[0]), n0 + r) : 0u;
+            k = max(k, (uint32_t)__shfl_xor((int)k, 1, 64));
+            k = max(k, (uint32_t)__shfl_xor((int)k, 2, 64));
+            if (r == 0) p.cand[(int64_t)m * gridDim.x + blockIdx.x] = k;
+        }
         if (n0 + r < p.N) {
             if (GATE) {
                 // g = f16(alpha dot_g), u = f16(alpha dot_u); h = f16(f16(silu g) * u)
@@ -254,6 +288,29 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
             } else {
                 p.C[m * p.ldc + n0 + r] = f2h(p.alpha * v[0]);
             }
+        }
+    }
+}
+
+// The arg max of each row from the workgroups' candidates, in out_tok; the last row's token is added to in_tok[pos]
+// (pos < 0: nowhere), src/librarium/llama.rs:953-959.
+__global__ void __launch_bounds__(1024)
+finish_rows_kernel(int M, int count, const uint32_t *__restrict__ cand, uint16_t *out_tok, uint16_t *in_tok, int64_t pos)
+{
+    __shared__ uint32_t best[16];
+    for (int m = 0; m < M; m++) {
+        uint32_t k = 0;
+        for (int i = threadIdx.x; i < count; i += 1024) k = max(k, cand[(int64_t)m * count + i]);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) k = max(k, (uint32_t)__shfl_xor((int)k, off, 64));
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0) best[threadIdx.x >> 6] = k;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < 16; w++) k = max(k, best[w]);
+            const uint16_t id = (uint16_t)(0xffff - (k & 0xffff));
+            out_tok[m] = id;
+            if (m == M - 1 && pos >= 0) in_tok[pos] = (uint16_t)(in_tok[pos] + id);
         }
     }
 }
@@ -284,9 +341,77 @@ int launch(int64_t M, const SkinnyArgs &p, hipStream_t st)
 int gemm_skinny_nt_launch(int64_t M, int64_t N, int64_t K, float alpha, const half_t *A, int64_t lda,
                           const half_t *B, int64_t ldb, half_t *C, int64_t ldc, hipStream_t st)
 {
-    SkinnyArgs p = {N, K, alpha, A, lda, nullptr, nullptr, 0.f, nullptr, B, nullptr, ldb, C, ldc,
-                    nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
+    SkinnyArgs p = {};
+    p.N = N; p.K = K; p.alpha = alpha;
+    p.A = A; p.lda = lda;
+    p.B = B; p.ldb = ldb;
+    p.C = C; p.ldc = ldc;
     return launch<false, E_PLAIN>(M, p, st);
+}
+
+namespace {
+
+SkinnyArgs norm_args(const RowSource &x, int64_t N, int64_t K, void *sum_out)
+{
+    SkinnyArgs p = {};
+    p.N = N; p.K = K; p.alpha = 1.0f;
+    p.A = (const half_t *)x.x; p.lda = K;
+    p.x2 = (const half_t *)x.x2;
+    p.w = (const half_t *)x.w_norm; p.eps = x.eps;
+    p.tok = x.tok; p.vocab = x.vocab; p.status = x.status;
+    p.sum_out = (half_t *)sum_out;
+    p.ldb = K;
+    p.ldc = N;
+    return p;
+}
+
+}  // namespace
+
+int rows_qkv_launch(int64_t M, int64_t H, int64_t Dh, const RowSource &x, void *sum_out, const void *Wq, const void *Wk, const void *Wv,
+                    const void *cos16, const void *sin16, void *q_rot, void *k_cache_rows, void *v_cache_rows, hipStream_t st)
+{
+    const int64_t D = H * Dh;
+    SkinnyArgs p = norm_args(x, D, D, sum_out);
+    p.B = (const half_t *)Wq; p.B2 = (const half_t *)Wk; p.B3 = (const half_t *)Wv;
+    p.C = (half_t *)q_rot;
+    p.cos16 = (const half_t *)cos16; p.sin16 = (const half_t *)sin16;
+    p.kc = (half_t *)k_cache_rows; p.vc = (half_t *)v_cache_rows;
+    p.H = (int)H; p.Dh = (int)Dh;
+    return launch<true, E_QKV>(M, p, st);
+}
+
+int rows_gate_launch(int64_t M, int64_t N, int64_t K, const RowSource &x, void *sum_out, const void *B, const void *B_mul, void *C,
+                     hipStream_t st)
+{
+    SkinnyArgs p = norm_args(x, N, K, sum_out);
+    p.B = (const half_t *)B; p.B2 = (const half_t *)B_mul;
+    p.C = (half_t *)C;
+    return launch<true, E_GATE>(M, p, st);
+}
+
+int rows_norm_launch(int64_t M, int64_t N, int64_t K, const RowSource &x, const void *B, void *C, hipStream_t st)
+{
+    SkinnyArgs p = norm_args(x, N, K, nullptr);
+    p.B = (const half_t *)B;
+    p.C = (half_t *)C;
+    return launch<true, E_PLAIN>(M, p, st);
+}
+
+size_t rows_head_scratch_bytes(int64_t M, int64_t N) { return (size_t)M * (size_t)((N + kRows - 1) / kRows) * sizeof(uint32_t); }
+
+int rows_head_launch(int64_t M, int64_t N, int64_t K, const RowSource &x, const void *B, void *logit, void *scratch, void *out_tok,
+                     void *in_tok, int64_t pos, hipStream_t st)
+{
+    CACTI_REQUIRE(N <= 65536, CACTI_E_NOTIMPL, "rows_head: more than 65536 tokens");
+    SkinnyArgs p = norm_args(x, N, K, nullptr);
+    p.B = (const half_t *)B;
+    p.C = (half_t *)logit;
+    p.cand = (uint32_t *)scratch;
+    const int rc = launch<true, E_PLAIN>(M, p, st);
+    if (rc) return rc;
+    hipLaunchKernelGGL(finish_rows_kernel, dim3(1), dim3(1024), 0, st, (int)M, (int)((N + kRows - 1) / kRows), (const uint32_t *)scratch,
+                       (uint16_t *)out_tok, (uint16_t *)in_tok, pos);
+    return launch_status("finish_rows");
 }
 
 }  // namespace cacti
@@ -304,9 +429,9 @@ CACTI_API int cacti_hip_rows_norm_matmul_f16(int64_t M, int64_t N, int64_t K, co
     CACTI_REQUIRE(aligned(x, 16) && aligned(x2, 16) && aligned(w_norm, 16) && aligned(sum_out, 16) && aligned(B, 16) &&
                       aligned(B_mul, 16) && aligned(C, 2),
                   CACTI_E_INVALID, "rows_norm_matmul: operands must be 16-byte aligned");
-    SkinnyArgs p = {N, K, 1.0f, (const half_t *)x, K, (const half_t *)x2, (const half_t *)w_norm, eps,
-                    (half_t *)sum_out, (const half_t *)B, (const half_t *)B_mul, K, (half_t *)C, N,
-                    nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
+    SkinnyArgs p = norm_args(RowSource{x, x2, w_norm, eps, nullptr, 0, nullptr}, N, K, sum_out);
+    p.B = (const half_t *)B; p.B2 = (const half_t *)B_mul;
+    p.C = (half_t *)C;
     hipStream_t st = (hipStream_t)stream;
     if (w_norm) return B_mul ? launch<true, E_GATE>(M, p, st) : launch<true, E_PLAIN>(M, p, st);
     return B_mul ? launch<false, E_GATE>(M, p, st) : launch<false, E_PLAIN>(M, p, st);
@@ -327,9 +452,6 @@ CACTI_API int cacti_hip_rows_qkv_rope_cache_f16(int64_t M, int64_t H, int64_t Dh
                       aligned(Wk, 16) && aligned(Wv, 16) && aligned(cos16, 2) && aligned(sin16, 2) && aligned(q_rot, 2) &&
                       aligned(k_cache_rows, 2) && aligned(v_cache_rows, 2),
                   CACTI_E_INVALID, "rows_qkv: rows and weights must be 16-byte aligned");
-    SkinnyArgs p = {D, D, 1.0f, (const half_t *)x, D, (const half_t *)x2, (const half_t *)w_norm, eps,
-                    (half_t *)sum_out, (const half_t *)Wq, (const half_t *)Wk, D, (half_t *)q_rot, D,
-                    (const half_t *)Wv, (const half_t *)cos16, (const half_t *)sin16, (half_t *)k_cache_rows,
-                    (half_t *)v_cache_rows, (int)H, (int)Dh};
-    return launch<true, E_QKV>(M, p, (hipStream_t)stream);
+    return rows_qkv_launch(M, H, Dh, RowSource{x, x2, w_norm, eps, nullptr, 0, nullptr}, sum_out, Wq, Wk, Wv, cos16, sin16, q_rot,
+                           k_cache_rows, v_cache_rows, (hipStream_t)stream);
 }

@@ -1,0 +1,36 @@
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+
+namespace cacti {
+
+// A device region (16-byte aligned; the whole last 16 bytes are readable) and where it goes in page-locked memory.
+struct HostRegion {
+    const void *src;
+    void *dst;
+    size_t bytes;
+};
+constexpr int kMaxRegions = 8;
+constexpr size_t kStagingBytes = 4u << 20;
+
+// Page-locked memory regions are gathered into, with the words their arrival is announced in.  One gather at a time.
+struct Staging {
+    char *base = nullptr;
+    unsigned epoch = 0;
+    char *data() const { return base + kFlagBytes; }
+    size_t room() const { return kStagingBytes - kFlagBytes; }
+    static constexpr size_t kFlagBytes = 4096;
+};
+// n <= kMaxRegions regions, in one launch on `st`, to places in s.data(); returns when they are there.  The launch comes
+// behind all work queued on `st`, so this waits for it like a stream synchronisation.
+int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st);
+// one region of any size to pageable memory, likewise
+int read_large(void *dst, const void *src, size_t bytes, hipStream_t st);
+// n regions of `bytes` (a multiple of 16), 16-byte aligned, set to zero
+int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st);
+
+// Up to four buffers that were given back are kept for later takers (page-locking costs hundreds of microseconds).
+bool staging_take(Staging *s);
+void staging_give_back(Staging *s);
+
+}  // namespace cacti

@@ -1,0 +1,220 @@
+// Data on its way from the device to the host program, and many small regions cleared at once.
+//
+// A read-back of a few KB costs its round trips, not its bytes: hipMemcpyAsync into pageable memory is staged by the
+// runtime and a stream synchronisation takes some 15 us to notice that the stream is empty.  Here one kernel writes the
+// regions straight into page-locked host memory, each workgroup followed by a word that says its part is there, and the
+// host polls those words.  A large read is the same in pieces, several of them on the link while the host's threads copy
+// earlier ones to their place (the runtime's copy to pageable memory: 16 GB/s).
+#include <emmintrin.h>
+#include <string.h>
+
+#include <algorithm>
+#include <atomic>
+#include <chrono>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "common.h"
+#include "hostcopy.h"
+
+namespace cacti {
+
+namespace {
+
+constexpr int kGatherBlocks = 64;              // workgroups per region at most: 4 KB and more each
+constexpr int kFlagsPerGather = kGatherBlocks * kMaxRegions;
+static_assert(kFlagsPerGather * sizeof(unsigned) <= Staging::kFlagBytes, "a word per workgroup");
+
+struct GatherArgs {
+    const uint4 *src[kMaxRegions];
+    uint4 *dst[kMaxRegions];
+    int64_t n16[kMaxRegions];
+    unsigned *flags;
+    unsigned epoch;
+};
+
+__global__ void __launch_bounds__(256) gather_kernel(GatherArgs p)
+{
+    const int z = blockIdx.y;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < p.n16[z]; i += (int64_t)gridDim.x * 256) p.dst[z][i] = p.src[z][i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_store(p.flags + z * gridDim.x + blockIdx.x, p.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+struct ZeroArgs {
+    uint4 *p[kMaxRegions];
+    int64_t n16;
+};
+
+__global__ void __launch_bounds__(256) zero_regions_kernel(ZeroArgs a)
+{
+    uint4 *p = a.p[blockIdx.y];
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < a.n16; i += (int64_t)gridDim.x * 256) p[i] = make_uint4(0, 0, 0, 0);
+}
+
+int launch_gather(const HostRegion *r, int n, unsigned *flags, unsigned epoch, int *nflags, hipStream_t st)
+{
+    GatherArgs p = {};
+    int64_t most = 1;
+    for (int i = 0; i < n; i++) {
+        p.src[i] = static_cast<const uint4 *>(r[i].src);
+        p.dst[i] = static_cast<uint4 *>(r[i].dst);
+        p.n16[i] = (int64_t)((r[i].bytes + 15) / 16);
+        most = std::max(most, p.n16[i]);
+    }
+    p.flags = flags;
+    p.epoch = epoch;
+    const int blocks = (int)std::min<int64_t>((most + 255) / 256, kGatherBlocks);
+    *nflags = blocks * n;
+    hipLaunchKernelGGL(gather_kernel, dim3((unsigned)blocks, (unsigned)n), dim3(256), 0, st, p);
+    return launch_status("gather_to_host");
+}
+
+// until all words hold `epoch`; a stream that is busy for longer than polling is worth is waited for by the runtime,
+// which also reports a failed one
+int wait_flags(const unsigned *flags, int n, unsigned epoch, hipStream_t st)
+{
+    const auto begin = std::chrono::steady_clock::now();
+    int i = 0;
+    for (unsigned polls = 1;; polls++) {
+        while (i < n && __atomic_load_n(flags + i, __ATOMIC_ACQUIRE) == epoch) i++;
+        if (i == n) return 0;
+        _mm_pause();
+        if ((polls & 255) == 0 && std::chrono::steady_clock::now() - begin > std::chrono::milliseconds(50)) break;
+    }
+    CACTI_HIP(hipStreamSynchronize(st));
+    for (; i < n; i++)
+        CACTI_REQUIRE(__atomic_load_n(flags + i, __ATOMIC_ACQUIRE) == epoch, CACTI_E_STATE, "gather_to_host: a part did not arrive");
+    return 0;
+}
+
+std::mutex g_mutex;
+std::vector<Staging> g_free;                   // staging buffers of contexts that are gone, for the next ones
+
+// large reads, one at a time: page-locked memory for kPieces pieces
+constexpr size_t kPiece = 1u << 20;
+constexpr int kPieces = 16, kReadThreads = 4;
+std::mutex g_large_mutex;
+char *g_large = nullptr;
+unsigned g_large_epoch = 0;
+
+}  // namespace
+
+int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st)
+{
+    CACTI_REQUIRE(n >= 1 && n <= kMaxRegions, CACTI_E_INVALID, "gather_to_host: %d regions", n);
+    unsigned *flags = reinterpret_cast<unsigned *>(s.base);
+    int nflags = 0;
+    if (++s.epoch == 0) s.epoch = 1;
+    const int rc = launch_gather(r, n, flags, s.epoch, &nflags, st);
+    return rc ? rc : wait_flags(flags, nflags, s.epoch, st);
+}
+
+int read_large(void *dst, const void *src, size_t bytes, hipStream_t st)
+{
+    std::lock_guard<std::mutex> lock(g_large_mutex);
+    constexpr size_t flag_bytes = (size_t)kPieces * kGatherBlocks * sizeof(unsigned);
+    if (!g_large) {
+        void *p = nullptr;
+        if (hipHostMalloc(&p, flag_bytes + kPieces * kPiece, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            CACTI_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+            CACTI_HIP(hipStreamSynchronize(st));
+            return 0;
+        }
+        g_large = static_cast<char *>(p);
+        memset(g_large, 0, flag_bytes);
+    }
+    unsigned *const flags = reinterpret_cast<unsigned *>(g_large);
+    char *const data = g_large + flag_bytes;
+    int dev = 0;
+    CACTI_HIP(hipGetDevice(&dev));
+    for (size_t done = 0; done < bytes;) {                        // windows of kPieces pieces
+        const size_t window = std::min(bytes - done, kPieces * kPiece);
+        const int pieces = (int)((window + kPiece - 1) / kPiece);
+        if (++g_large_epoch == 0) g_large_epoch = 1;
+        const unsigned epoch = g_large_epoch;
+        int nflags[kPieces];
+        for (int i = 0; i < pieces; i++) {
+            const HostRegion r = {static_cast<const char *>(src) + done + (size_t)i * kPiece, data + (size_t)i * kPiece,
+                                  std::min(kPiece, window - (size_t)i * kPiece)};
+            const int rc = launch_gather(&r, 1, flags + i * kGatherBlocks, epoch, &nflags[i], st);
+            if (rc) return rc;
+        }
+        std::atomic<int> next{0}, failed{0};
+        auto work = [&]() {
+            for (int i; !failed.load() && (i = next.fetch_add(1)) < pieces;) {
+                const int rc = wait_flags(flags + i * kGatherBlocks, nflags[i], epoch, st);
+                if (rc) failed.store(rc);
+                else memcpy(static_cast<char *>(dst) + done + (size_t)i * kPiece, data + (size_t)i * kPiece,
+                            std::min(kPiece, window - (size_t)i * kPiece));
+            }
+        };
+        std::vector<std::thread> th;
+        for (int t = 1; t < std::min(kReadThreads, pieces); t++)
+            th.emplace_back([&]() {
+                (void)hipSetDevice(dev);
+                work();
+            });
+        work();
+        for (std::thread &t : th) t.join();
+        if (failed.load()) return failed.load();
+        done += window;
+    }
+    return 0;
+}
+
+int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st)
+{
+    for (int i0 = 0; i0 < n; i0 += kMaxRegions) {
+        ZeroArgs a = {};
+        const int m = std::min(n - i0, kMaxRegions);
+        for (int i = 0; i < m; i++) a.p[i] = static_cast<uint4 *>(ptrs[i0 + i]);
+        a.n16 = (int64_t)(bytes / 16);
+        const unsigned blocks = (unsigned)std::min<int64_t>((a.n16 + 255) / 256, 512);
+        hipLaunchKernelGGL(zero_regions_kernel, dim3(blocks, (unsigned)m), dim3(256), 0, st, a);
+        const int rc = launch_status("zero_regions");
+        if (rc) return rc;
+    }
+    return 0;
+}
+
+bool staging_take(Staging *s)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        if (!g_free.empty()) {
+            *s = g_free.back();
+            g_free.pop_back();
+            return true;
+        }
+    }
+    void *p = nullptr;
+    if (hipHostMalloc(&p, kStagingBytes, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    memset(p, 0, Staging::kFlagBytes);
+    *s = Staging{static_cast<char *>(p), 0};
+    return true;
+}
+
+void staging_give_back(Staging *s)
+{
+    if (!s->base) return;
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        if (g_free.size() < 4) {
+            g_free.push_back(*s);
+            *s = Staging{};
+            return;
+        }
+    }
+    hipHostFree(s->base);
+    *s = Staging{};
+}
+
+}  // namespace cacti

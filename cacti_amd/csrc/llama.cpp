@@ -4,10 +4,12 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <string>
 
 #include "../../include/cacti_hip_runtime.h"
 #include "common.h"
+#include "gemm_internal.h"
 #include "thunks.h"
 
 using namespace cacti;
@@ -577,8 +579,13 @@ CACTI_API int cacti_llama_step(cacti_llama *m, const uint16_t *tok, const uint16
     // (the next cycle's staging then overlaps it); an out-of-range token id is reported by
     // the next synchronizing call (cacti_ctx_sync, or a step that reads the loss).
     if (!loss_out) return 0;
-    TRY(c.check_status());
-    return c.cell_get(m->out_loss, loss_out, S * 4);
+    Cell &l = c.cell(m->out_loss);
+    if (!l.v_valid || l.v_ready) {                                // (spilled: through its host replica)
+        TRY(c.check_status());
+        return c.cell_get(m->out_loss, loss_out, S * 4);
+    }
+    const Ctx::Fetch f = {c.dev_ptr(l.voff), loss_out, S * 4};
+    return c.fetch(&f, 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -593,7 +600,17 @@ struct cacti_llama_cached {
     // outputs of the last apply (pool regions kept until the next apply or destroy)
     size_t out_logit = kNoOffset, out_prob = kNoOffset, out_tok = kNoOffset;
     int64_t out_rows = 0;
+    int64_t rows;                            // cache rows below this may hold values
 };
+
+namespace cacti {
+// csrc/elementwise.hip
+int rope_cache_launch(int64_t S, int64_t H, int64_t Dh, const void *q, const void *k, const void *v, const void *cos16, const void *sin16,
+                      void *q_rot, void *k_cache_rows, void *v_cache_rows, hipStream_t st);
+// csrc/attention.hip
+int attention_fwd_exact(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k, const void *v, int64_t ld, void *o,
+                        void *stats, hipStream_t st);
+}  // namespace cacti
 
 namespace {
 
@@ -620,7 +637,7 @@ CACTI_API int cacti_llama_cached_create(cacti_llama *model, int64_t seq_cap, cac
     Ctx &c = model->ctx->c;
     cacti_llama_cached *k = new cacti_llama_cached();
     k->base = model;
-    k->cap = seq_cap;
+    k->cap = k->rows = seq_cap;
     for (int64_t l = 0; l < model->cfg.L; l++) {
         const std::string p = "l" + std::to_string(l) + ".";
         k->k_cache.push_back(c.cell_new(CellType({seq_cap, model->cfg.H, model->cfg.Dh}, F16), true, (p + "k_cache").c_str()));
@@ -659,11 +676,13 @@ CACTI_API int cacti_llama_cached_reset_state(cacti_llama_cached *k)
 {
     CACTI_REQUIRE(k, CACTI_E_INVALID, "llama_cached_reset_state: null model");
     Ctx &c = k->base->ctx->c;
-    for (size_t l = 0; l < k->k_cache.size(); l++) {
-        int rc = c.cell_zero(k->k_cache[l]);
-        if (!rc) rc = c.cell_zero(k->v_cache[l]);
-        if (rc) return rc;
-    }
+    // only the rows written since the last time hold anything
+    std::vector<CellPtr> all = k->k_cache;
+    all.insert(all.end(), k->v_cache.begin(), k->v_cache.end());
+    const size_t row = (size_t)k->base->cfg.D * 2;
+    const int rc = c.cells_zero_rows(all.data(), (int)all.size(), std::min((size_t)k->cap * row, ((size_t)k->rows * row + 15) / 16 * 16));
+    if (rc) return rc;
+    k->rows = 0;
     return 0;
 }
 
@@ -696,6 +715,7 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
     const float alpha = 1.0f / sqrtf((float)Dh);
     hipStream_t st = c.stream();
     cached_drop_outputs(k);
+    k->rows = std::max(k->rows, next);
 
     // every cell the pass touches is made resident and pinned for the duration of the call
     std::vector<CellPtr> used = m->params;
@@ -722,13 +742,17 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
     auto P = [&](CellPtr x) { return c.dev_ptr(c.cell(x).voff); };
     char *x = tmp(T * D, 2), *pre = tmp(T * D, 2), *q = tmp(T * D, 2), *qr = tmp(T * D, 2), *kk = tmp(T * D, 2),
          *kr = tmp(T * D, 2), *v = tmp(T * D, 2), *attn = tmp(T * D, 2), *o = tmp(T * D, 2), *x1 = tmp(T * D, 2),
-         *post = tmp(T * D, 2), *up = tmp(T * F, 2), *gate = tmp(T * F, 2), *h = tmp(T * F, 2), *down = tmp(T * D, 2),
-         *s16 = nullptr, *aws = nullptr;
-    // one to four rows: the fused decoding attention; more: scores, softmax and P V as three products
-    const bool fused_attn = T <= 4 && Dh % 4 == 0 && Dh <= 100 && next <= 8192;
-    const size_t aws_bytes = fused_attn ? cacti_hip_attn_decode_workspace(T, H, Dh, next) : 0;
-    if (fused_attn) aws = tmp((int64_t)aws_bytes, 1);
-    else s16 = tmp(T * H * Cw, 2);
+         *post = tmp(T * D, 2), *up = tmp(T * F, 2), *gate = tmp(T * F, 2), *h = tmp(T * F, 2), *down = tmp(T * D, 2);
+    // one to four rows: the decoding kernels, one launch per weight matrix (or pair, or triple) and one or two for
+    // attention.  More rows: the training kernels; a long prompt from position 0 is causal attention over its own rows of
+    // the cache in one kernel (1531 rows, 16 heads of 128: 93 -> 40 us per layer), other rows take scores, softmax and P V
+    // as three (up to 128 rows they are one tile of scores per head, 17 against 11 us, and the numbers of the training
+    // pass with separate thunks bit for bit).
+    const bool few = T <= 4 && Dh % 4 == 0 && Dh <= 128 && next <= 8192 && D % 8 == 0 && D <= 8192;
+    const bool causal = !few && prev == 0 && T > 128 && Dh % 4 == 0 && Dh <= 128 && T <= 65536;
+    const size_t aws_bytes = few ? cacti_hip_attn_decode_workspace(T, H, Dh, next)
+                                 : causal ? cacti_hip_attention_stats_bytes(T, H) : (size_t)(T * H * Cw) * 2;
+    char *aws = tmp((int64_t)aws_bytes, 1), *head_ws = few && !want_prob ? tmp((int64_t)rows_head_scratch_bytes(T, V), 1) : nullptr;
     // outputs
     if (!rc) rc = c.pool_alloc((size_t)(T * V) * 2, &k->out_logit);
     if (!rc) rc = c.pool_alloc((size_t)T * 2, &k->out_tok);
@@ -746,6 +770,19 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
             gws_bytes = need;
         }
     };
+    // products that share their input in one launch, where their sizes allow it: a prompt of a few rows leaves most CUs
+    // without a tile otherwise (37 rows, 3200 x 3200: 50 tiles each)
+    auto products = [&](int n, int64_t N, int64_t K, const void *a, std::vector<void *> w, std::vector<void *> y) -> int {
+        if (N % 8 == 0 && K % 8 == 0 && K > 128) {
+            const std::vector<const void *> as((size_t)n, a), bs(w.begin(), w.end());
+            return cacti_hip_gemm_f16_batched(0, 1, n, T, N, K, 1.f, as.data(), K, bs.data(), K, 0.f, y.data(), N, st);
+        }
+        for (int i = 0; i < n; i++) {
+            const int r = product(N, K, a, w[(size_t)i], y[(size_t)i]);
+            if (r) return r;
+        }
+        return 0;
+    };
 #define STEP(call)          \
     do {                    \
         if (!rc) rc = (call); \
@@ -754,55 +791,72 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
         const char *cosr = static_cast<const char *>(P(m->cos)) + prev * Dh * 2;
         const char *sinr = static_cast<const char *>(P(m->sin)) + prev * Dh * 2;
         char *tok = static_cast<char *>(P(k->in_tok));
-        // stream = embed.outer_select(in_tok[prev .. next])
-        STEP(cacti_hip_embed_fwd(V, D, P(m->embed), T, tok + prev * 2, x, c.status_ptr(), st));
-        void *logit = c.dev_ptr(k->out_logit);
-        if (fused_attn && D <= 8192) {
-            // One to four rows: the norms, the residual adds and the SiLU gate ride in the product
-            // kernels (cacti_hip_rows_norm_matmul_f16), which stream each weight matrix once.
-            // The residual stream is (xa) or the pending sum f16(xa + xb).
-            const char *xa = x, *xb = nullptr;
+        void *logit = c.dev_ptr(k->out_logit), *otok = c.dev_ptr(k->out_tok);
+        bool finished = false;                                    // the arg max has been taken and appended
+        if (few) {
+            // The norms, the residual adds and the SiLU gate ride in the product kernels, which stream each weight
+            // matrix once.  The residual stream is xa or the pending sum f16(xa + xb); the first layer's is gathered
+            // from the embedding by its kernels (stream = embed.outer_select(in_tok[prev .. next])).
+            RowSource xs = {P(m->embed), nullptr, nullptr, g.eps, reinterpret_cast<const uint16_t *>(tok + prev * 2), V,
+                            static_cast<int *>(c.status_ptr())};
+            auto normed = [&](const void *xb, CellPtr w) {
+                RowSource r = xs;
+                r.x2 = xb;
+                r.w_norm = P(w);
+                return r;
+            };
+            const char *xb = nullptr;
             for (size_t l = 0; l < m->layers.size() && !rc; l++) {
                 const LayerCells &w = m->layers[l];
                 char *kc = static_cast<char *>(P(k->k_cache[l])), *vc = static_cast<char *>(P(k->v_cache[l]));
                 // q, k, v projections of the normed stream, rotation, k_cache[prev ..] += k, v_cache[prev ..] += v
-                STEP(cacti_hip_rows_qkv_rope_cache_f16(T, H, Dh, xa, xb, P(w.pre_norm), g.eps, xb ? x : nullptr, P(w.q), P(w.k),
-                                                       P(w.v), cosr, sinr, qr, kc + prev * D * 2, vc + prev * D * 2, st));
+                STEP(rows_qkv_launch(T, H, Dh, normed(xb, w.pre_norm), xb ? x : nullptr, P(w.q), P(w.k), P(w.v), cosr, sinr, qr,
+                                     kc + prev * D * 2, vc + prev * D * 2, st));
+                if (xb) xs = RowSource{x, nullptr, nullptr, g.eps, nullptr, 0, nullptr};
                 STEP(cacti_hip_attn_decode_f16(T, H, Dh, next, prev, alpha, qr, D, kc, vc, D, Dh, attn, D, aws, aws_bytes, st));
                 STEP(product(D, D, attn, P(w.o), o));
                 // x1 = stream + o; post = rms_norm(x1); h = silu(post gate^T) * (post up^T)
-                STEP(cacti_hip_rows_norm_matmul_f16(T, F, D, x, o, P(w.post_norm), g.eps, x1, P(w.gate), P(w.up), h, st));
+                STEP(rows_gate_launch(T, F, D, normed(o, w.post_norm), x1, P(w.gate), P(w.up), h, st));
                 STEP(product(D, F, h, P(w.down), down));
-                xa = x1;                                          // stream = x1 + down, formed by the next consumer
-                xb = down;
+                xs = RowSource{x1, nullptr, nullptr, g.eps, nullptr, 0, nullptr};
+                xb = down;                                        // stream = x1 + down, formed by the next consumer
             }
-            STEP(cacti_hip_rows_norm_matmul_f16(T, V, D, xa, xb, P(m->head_norm), g.eps, nullptr, P(m->lm_head), nullptr, logit, st));
+            if (head_ws) {
+                STEP(rows_head_launch(T, V, D, normed(xb, m->head_norm), P(m->lm_head), logit, head_ws, otok, tok, next < cap ? next : -1,
+                                      st));
+                finished = true;
+            } else {
+                STEP(rows_norm_launch(T, V, D, normed(xb, m->head_norm), P(m->lm_head), logit, st));
+            }
         } else {
+            // stream = embed.outer_select(in_tok[prev .. next])
+            STEP(cacti_hip_embed_fwd(V, D, P(m->embed), T, tok + prev * 2, x, c.status_ptr(), st));
             STEP(cacti_hip_rms_norm_fwd(T, D, x, P(m->layers.empty() ? m->head_norm : m->layers[0].pre_norm), g.eps, pre, st));
             for (size_t l = 0; l < m->layers.size() && !rc; l++) {
                 const LayerCells &w = m->layers[l];
                 char *kc = static_cast<char *>(P(k->k_cache[l])), *vc = static_cast<char *>(P(k->v_cache[l]));
-                STEP(product(D, D, pre, P(w.q), q));
-                STEP(cacti_hip_rope_fwd(T, H, Dh, q, cosr, sinr, qr, st));
-                STEP(product(D, D, pre, P(w.k), kk));
-                STEP(cacti_hip_rope_fwd(T, H, Dh, kk, cosr, sinr, kr, st));
-                // k_cache[prev .. next] += k, v_cache[prev .. next] += v
-                STEP(cacti_hip_add_f16(T * D, kc + prev * D * 2, kr, kc + prev * D * 2, st));
-                STEP(product(D, D, pre, P(w.v), v));
-                STEP(cacti_hip_add_f16(T * D, vc + prev * D * 2, v, vc + prev * D * 2, st));
-                // scores against the cache, row-causal mask + softmax (in place), P V.  Columns from
-                // `next` on are masked for every row, so only the first Cw of the cap columns are formed.
-                if (fused_attn) {
-                    STEP(cacti_hip_attn_decode_f16(T, H, Dh, next, prev, alpha, qr, D, kc, vc, D, Dh, attn, D, aws, aws_bytes, st));
+                STEP(products(3, D, D, pre, {P(w.q), P(w.k), P(w.v)}, {q, kk, v}));
+                // rotation, k_cache[prev .. next] += k, v_cache[prev .. next] += v
+                if (Dh % 4 == 0) {
+                    STEP(rope_cache_launch(T, H, Dh, q, kk, v, cosr, sinr, qr, kc + prev * D * 2, vc + prev * D * 2, st));
                 } else {
-                    STEP(cacti_hip_gemm_f16_strided_batched(0, 1, H, T, Cw, Dh, alpha, qr, D, Dh, kc, D, Dh, 0.f, s16, H * Cw, Cw, st));
-                    STEP(cacti_hip_row_causal_softmax_fwd(T, H, Cw, Cw, prev, s16, s16, st));
-                    STEP(cacti_hip_gemm_f16_strided_batched(0, 0, H, T, Dh, Cw, 1.f, s16, H * Cw, Cw, vc, D, Dh, 0.f, attn, D, Dh, st));
+                    STEP(cacti_hip_rope_fwd(T, H, Dh, q, cosr, sinr, qr, st));
+                    STEP(cacti_hip_rope_fwd(T, H, Dh, kk, cosr, sinr, kr, st));
+                    STEP(cacti_hip_add_f16(T * D, kc + prev * D * 2, kr, kc + prev * D * 2, st));
+                    STEP(cacti_hip_add_f16(T * D, vc + prev * D * 2, v, vc + prev * D * 2, st));
+                }
+                if (causal) {
+                    STEP(attention_fwd_exact(T, H, Dh, alpha, qr, kc, vc, D, attn, aws, st));
+                } else {
+                    // scores against the cache, row-causal mask + softmax (in place), P V.  Columns from
+                    // `next` on are masked for every row, so only the first Cw of the cap columns are formed.
+                    STEP(cacti_hip_gemm_f16_strided_batched(0, 1, H, T, Cw, Dh, alpha, qr, D, Dh, kc, D, Dh, 0.f, aws, H * Cw, Cw, st));
+                    STEP(cacti_hip_row_causal_softmax_fwd(T, H, Cw, Cw, prev, aws, aws, st));
+                    STEP(cacti_hip_gemm_f16_strided_batched(0, 0, H, T, Dh, Cw, 1.f, aws, H * Cw, Cw, vc, D, Dh, 0.f, attn, D, Dh, st));
                 }
                 STEP(product(D, D, attn, P(w.o), o));
                 STEP(cacti_hip_add_rms_norm_fwd(T, D, x, o, P(w.post_norm), g.eps, x1, post, st));
-                STEP(product(F, D, post, P(w.up), up));
-                STEP(product(F, D, post, P(w.gate), gate));
+                STEP(products(2, F, D, post, {P(w.up), P(w.gate)}, {up, gate}));
                 STEP(cacti_hip_silu_gate_fwd(T * F, gate, up, h, st));
                 STEP(product(D, F, h, P(w.down), down));
                 const CellPtr wn = l + 1 < m->layers.size() ? m->layers[l + 1].pre_norm : m->head_norm;
@@ -810,11 +864,12 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
             }
             STEP(product(V, D, pre, P(m->lm_head), logit));
         }
-        void *otok = c.dev_ptr(k->out_tok);
-        STEP(cacti_hip_softmax_ce_fwd(T, V, logit, nullptr, want_prob ? c.dev_ptr(k->out_prob) : nullptr, nullptr,
-                                      otok, nullptr, st));
-        // in_tok[next] += out_lm_tok[T - 1]
-        if (next < cap) STEP(cacti_hip_append_token_u16(tok, next, otok, T - 1, st));
+        if (!finished) {
+            STEP(cacti_hip_softmax_ce_fwd(T, V, logit, nullptr, want_prob ? c.dev_ptr(k->out_prob) : nullptr, nullptr,
+                                          otok, nullptr, st));
+            // in_tok[next] += out_lm_tok[T - 1]
+            if (next < cap) STEP(cacti_hip_append_token_u16(tok, next, otok, T - 1, st));
+        }
         if (!rc) {
             c.cell(k->in_tok).h_valid = false;
             for (size_t l = 0; l < m->layers.size(); l++)
@@ -834,11 +889,12 @@ CACTI_API int cacti_llama_cached_outputs(cacti_llama_cached *k, void *logit_f16,
     CACTI_REQUIRE(k && k->out_rows > 0, CACTI_E_STATE, "llama_cached_outputs: no apply has run");
     CACTI_REQUIRE(!prob || k->out_prob != kNoOffset, CACTI_E_STATE, "llama_cached_outputs: the last apply kept no probabilities");
     Ctx &c = k->base->ctx->c;
-    hipStream_t st = c.stream();
     const int64_t T = k->out_rows, V = k->base->cfg.V;
-    if (logit_f16) CACTI_HIP(hipMemcpyAsync(logit_f16, c.dev_ptr(k->out_logit), (size_t)(T * V) * 2, hipMemcpyDeviceToHost, st));
-    if (prob) CACTI_HIP(hipMemcpyAsync(prob, c.dev_ptr(k->out_prob), (size_t)(T * V) * 4, hipMemcpyDeviceToHost, st));
-    if (tok) CACTI_HIP(hipMemcpyAsync(tok, c.dev_ptr(k->out_tok), (size_t)T * 2, hipMemcpyDeviceToHost, st));
-    return c.check_status();                                     // syncs; raises a token id out of range
+    Ctx::Fetch f[3];
+    int n = 0;
+    if (tok) f[n++] = {c.dev_ptr(k->out_tok), tok, (size_t)T * 2};
+    if (logit_f16) f[n++] = {c.dev_ptr(k->out_logit), logit_f16, (size_t)(T * V) * 2};
+    if (prob) f[n++] = {c.dev_ptr(k->out_prob), prob, (size_t)(T * V) * 4};
+    return c.fetch(f, n);                                         // syncs; raises a token id out of range
 }
 

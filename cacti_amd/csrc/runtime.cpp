@@ -150,6 +150,7 @@ Ctx::~Ctx()
         if (ingest_host_[k]) hipHostFree(ingest_host_[k]);
         if (ingest_ev_[k]) hipEventDestroy(ingest_ev_[k]);
     }
+    staging_give_back(&staging_);
     if (base_) hipFree(base_);
     if (own_stream_ && stream_) hipStreamDestroy(stream_);
     if (counted_) live_contexts_add(dev_, -1);
@@ -199,6 +200,7 @@ int Ctx::init(int dev, size_t pool_bytes, int host_pagelocked)
     }
     CACTI_HIP(hipEventCreate(&ev0_));
     CACTI_HIP(hipEventCreate(&ev1_));
+    (void)staging_take(&staging_);             // (without it read-backs go through the runtime's copies)
     return 0;
 }
 
@@ -233,14 +235,41 @@ int Ctx::order_after_compute(hipStream_t st)
     return 0;
 }
 
-int Ctx::check_status()
+int Ctx::check_status() { return fetch(nullptr, 0); }
+
+int Ctx::fetch(const Fetch *f, int n)
 {
-    int v = 0;
-    CACTI_HIP(hipMemcpyAsync(&v, status_ptr(), sizeof(int), hipMemcpyDeviceToHost, stream_));
-    CACTI_HIP(hipStreamSynchronize(stream_));
-    if (v) {
+    int status = 0;
+    HostRegion r[kMaxRegions];
+    const Fetch *staged[kMaxRegions] = {};
+    int m = 0;
+    size_t used = 256;                         // behind the status word's place
+    const bool stage = staging_.base != nullptr;
+    if (stage) r[m++] = {status_ptr(), staging_.data(), sizeof(int)};
+    else CACTI_HIP(hipMemcpyAsync(&status, status_ptr(), sizeof(int), hipMemcpyDeviceToHost, stream_));
+    for (int i = 0; i < n; i++) {
+        bytes_d2h_ += f[i].bytes;
+        const size_t room = (f[i].bytes + 255) / 256 * 256;
+        if (stage && m < kMaxRegions && used + room <= staging_.room()) {
+            staged[m] = &f[i];
+            r[m++] = {f[i].src, staging_.data() + used, f[i].bytes};
+            used += room;
+        } else {
+            const int rc = read_large(f[i].dst, f[i].src, f[i].bytes, stream_);
+            if (rc) return rc;
+        }
+    }
+    if (stage) {
+        const int rc = gather_to_host(staging_, r, m, stream_);
+        if (rc) return rc;
+        memcpy(&status, staging_.data(), sizeof(int));
+        for (int i = 1; i < m; i++) memcpy(staged[i]->dst, r[i].dst, staged[i]->bytes);
+    } else {
+        CACTI_HIP(hipStreamSynchronize(stream_));
+    }
+    if (status) {
         CACTI_HIP(hipMemsetAsync(status_ptr(), 0, sizeof(int), stream_));
-        set_error("token id out of range at position %d", v - 1);
+        set_error("token id out of range at position %d", status - 1);
         return CACTI_E_INDEX;
     }
     return 0;
@@ -359,8 +388,15 @@ int Ctx::cell_get(CellPtr ci, void *host, size_t bytes)
             ev_put(c.v_ready);
             c.v_ready = nullptr;
         }
-        CACTI_HIP(hipMemcpyAsync(host, dev_ptr(c.voff), bytes, hipMemcpyDeviceToHost, stream_));
-        CACTI_HIP(hipStreamSynchronize(stream_));
+        int rc;
+        if (staging_.base && bytes <= staging_.room()) {
+            const HostRegion r = {dev_ptr(c.voff), staging_.data(), bytes};
+            rc = gather_to_host(staging_, &r, 1, stream_);
+            if (!rc) memcpy(host, staging_.data(), bytes);
+        } else {
+            rc = read_large(host, dev_ptr(c.voff), bytes, stream_);
+        }
+        if (rc) return rc;
         bytes_d2h_ += bytes;
         return 0;
     }
@@ -543,6 +579,25 @@ int Ctx::cell_zero(CellPtr c)
     cells_[c].v_valid = true;
     cells_[c].h_valid = false;
     return 0;
+}
+
+int Ctx::cells_zero_rows(const CellPtr *cells, int n, size_t bytes)
+{
+    if (bytes == 0) return 0;
+    std::vector<void *> p;
+    int rc = 0, done = 0;
+    for (; done < n && !rc; done++) {
+        cells_[cells[done]].pin++;
+        rc = ensure_vmem(cells[done], bytes < cells_[cells[done]].ty.bytes());
+    }
+    for (int i = 0; i < n && !rc; i++) p.push_back(dev_ptr(cells_[cells[i]].voff));
+    if (!rc) rc = zero_regions(p.data(), n, bytes, stream_);
+    for (int i = 0; i < done; i++) cells_[cells[i]].pin--;
+    for (int i = 0; i < n && !rc; i++) {
+        cells_[cells[i]].v_valid = true;
+        cells_[cells[i]].h_valid = false;
+    }
+    return rc;
 }
 
 // The five cells of a tensor must be resident together; with a capped pool the list is cut into

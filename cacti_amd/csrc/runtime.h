@@ -17,6 +17,8 @@
 #include <unordered_map>
 #include <vector>
 
+#include "hostcopy.h"
+
 namespace cacti {
 
 enum Dtype : int { F16 = 0, F32 = 1, U16 = 2, I32 = 3 };
@@ -213,6 +215,11 @@ class Ctx {
     // reference asserts inside the kernel, src/thunk/op.rs:3538); checked at sync points
     void *status_ptr() { return base_ + status_off_; }
     int check_status();
+    // Device regions (256-byte aligned, as the pool hands them out) to host arrays, and the status word with them: one
+    // launch and one synchronisation for what fits the staging buffer.  Returns the status word's error.
+    struct Fetch { const void *src; void *dst; size_t bytes; };
+    int fetch(const Fetch *f, int n);
+    int cells_zero_rows(const CellPtr *cells, int n, size_t bytes);    // the first `bytes` (a multiple of 16) of every cell
     void stats(Stats *s) const;
     // the pool's usage by class of cell, as text (NvGpuPCtx::_dump_usage / _dump_sizes / _dump_free,
     // src/pctx/nvgpu.rs:690-742): what an exhausted pool prints, and the per-cycle report
@@ -301,6 +308,7 @@ class Ctx {
     std::map<std::string, std::pair<double, uint64_t>> times_;
     std::map<std::string, uint64_t> op_bytes_;                   // label -> operand bytes of one launch
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
+    Staging staging_;                                            // for read-backs
     // cell_ingest: two page-locked staging buffers and the event after the last upload from each
     void *ingest_host_[2] = {nullptr, nullptr};
     hipEvent_t ingest_ev_[2] = {nullptr, nullptr};
