@@ -5,12 +5,14 @@
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "lib")
 LIB = os.path.join(OUT_DIR, "libcacti_gpu_hip_ffi.so")
+FAST = os.path.join(OUT_DIR, "_fast.so")       # CPython functions over LIB (pysrc/fast.cpp)
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -45,13 +47,16 @@ def build(jobs=4):
         objs = list(ex.map(_compile, sources()))
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs
     subprocess.check_call(cmd)
+    subprocess.check_call(["g++", "-O2", "-shared", "-fPIC", "-std=c++17", "-Wall", "-I" + sysconfig.get_paths()["include"],
+                           os.path.join(HERE, "pysrc", "fast.cpp"), "-o", FAST, "-L" + OUT_DIR, "-l:" + os.path.basename(LIB),
+                           "-Wl,-rpath,$ORIGIN"])
     return LIB
 
 
 def ensure():
     """The library's path, built first if no built library is there (tests, the smoke run and the
     benchmark call this; the loader itself never builds and never falls back)."""
-    return LIB if os.path.exists(LIB) else build()
+    return LIB if os.path.exists(LIB) and os.path.exists(FAST) else build()
 
 
 if __name__ == "__main__":

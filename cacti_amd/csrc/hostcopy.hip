@@ -218,3 +218,28 @@ void staging_give_back(Staging *s)
 }
 
 }  // namespace cacti
+
+using namespace cacti;
+
+namespace {
+// a calling thread's own, given back when the thread ends
+struct ThreadStaging {
+    Staging s;
+    ~ThreadStaging() { staging_give_back(&s); }
+};
+}  // namespace
+
+CACTI_API int cacti_hip_read_i32(const void *dev, int32_t *value, void *stream)
+{
+    CACTI_REQUIRE(dev && value && aligned(dev, 16), CACTI_E_INVALID, "read_i32: null or misaligned pointer");
+    static thread_local ThreadStaging t;
+    if (!t.s.base && !staging_take(&t.s)) {
+        CACTI_HIP(hipMemcpyAsync(value, dev, sizeof(*value), hipMemcpyDeviceToHost, (hipStream_t)stream));
+        CACTI_HIP(hipStreamSynchronize((hipStream_t)stream));
+        return 0;
+    }
+    const HostRegion r = {dev, t.s.data(), sizeof(*value)};
+    const int rc = gather_to_host(t.s, &r, 1, (hipStream_t)stream);
+    if (!rc) memcpy(value, t.s.data(), sizeof(*value));
+    return rc;
+}

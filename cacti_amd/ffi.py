@@ -3,6 +3,8 @@
 Loading fails loudly when the library has not been built: there is no CPU fallback.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -48,6 +50,7 @@ SIGNATURES = {
     "cacti_hip_event_query": (ci, [vp]),
     "cacti_hip_event_sync": (ci, [vp]),
     "cacti_hip_event_elapsed_ms": (ci, [vp, vp, C.POINTER(f32)]),
+    "cacti_hip_read_i32": (ci, [vp, C.POINTER(C.c_int32), vp]),
     "cacti_hip_gemm_f16": (ci, [ci, ci, i64, i64, i64, f32, vp, i64, vp, i64, f32, vp, i64, vp]),
     "cacti_hip_gemm_f16_ws": (ci, [ci, ci, i64, i64, i64, f32, vp, i64, vp, i64, f32, vp, i64, vp, sz, C.POINTER(sz), vp]),
     "cacti_hip_gemm_plan": (ci, [i64, i64, i64, i64, C.POINTER(i64)]),
@@ -208,6 +211,23 @@ def lib():
             fn.argtypes = args
         _lib = L
     return _lib
+
+
+_fast = None
+
+
+def fast():
+    """The operator entry points as CPython functions (pysrc/fast.cpp), built beside the library."""
+    global _fast
+    if _fast is None:
+        lib()                                    # the same library, by its path
+        path = os.path.join(os.path.dirname(LIB_PATH), "_fast.so")
+        if not os.path.exists(path):
+            raise RuntimeError("%s is missing: build it with `python -m cacti_amd.build`" % path)
+        loader = importlib.machinery.ExtensionFileLoader("_fast", path)
+        _fast = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fast", loader))
+        loader.exec_module(_fast)
+    return _fast
 
 
 def check(rc):

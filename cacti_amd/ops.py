@@ -12,18 +12,47 @@ import torch
 from . import ffi
 
 F16 = torch.float16
+F32 = torch.float32
+
+# A small operator is host work: 8 us of it in Python against some 3 us on the device.  So the entry points are called as
+# CPython functions (ffi.fast), the stream is read without building a torch.cuda.Stream (2.7 us), and each operator
+# checks its tensors in one expression.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device()) if _raw_stream else torch.cuda.current_stream().cuda_stream
+
+
+class _Calls:
+    """The library's entry points without their prefix, raising on a status that is not 0."""
+
+    def __getattr__(self, name):
+        f = getattr(ffi.fast(), name)
+
+        def call(*args):
+            rc = f(*args)
+            if rc:
+                ffi.check(rc)
+
+        setattr(self, name, call)
+        return call
+
+
+_do = _Calls()
+
+
+def _size(name, *args):
+    return getattr(ffi.fast(), name)(*args)
 
 
 def _p(t):
-    return 0 if t is None else t.data_ptr()
+    return None if t is None else t.data_ptr()
 
 
 def _chk(t, dtype=F16):
-    assert t.is_cuda and t.is_contiguous() and t.dtype == dtype, (t.dtype, t.device, t.shape)
+    assert t.is_cuda and t.is_contiguous() and t.dtype is dtype, (t.dtype, t.device, t.shape)
     return t
 
 
@@ -36,26 +65,30 @@ def selftest_wave_reduce():
 # ---------------------------------------------------------------- GEMM
 def gemm(a, b, ta=False, tb=False, alpha=1.0, beta=0.0, out=None):
     """out = f16(alpha op(a) op(b) + beta out); a, b 2-d row-major f16 (rows may be strided)."""
-    assert a.dim() == 2 and b.dim() == 2 and a.stride(1) == 1 and b.stride(1) == 1
-    M, K = (a.shape[1], a.shape[0]) if ta else a.shape
-    K2, N = (b.shape[1], b.shape[0]) if tb else b.shape
+    (ra, ca), (rb, cb) = a.shape, b.shape
+    assert a.stride(1) == 1 and b.stride(1) == 1
+    M, K = (ca, ra) if ta else (ra, ca)
+    K2, N = (cb, rb) if tb else (rb, cb)
     assert K == K2, (a.shape, b.shape, ta, tb)
     if out is None:
         assert beta == 0.0
         out = torch.empty((M, N), dtype=F16, device=a.device)
-    assert out.shape == (M, N) and out.stride(1) == 1
+    else:
+        assert out.shape == (M, N) and out.stride(1) == 1
     _gemm(ta, tb, M, N, K, alpha, a, b, beta, out)
     return out
 
 
 def _gemm(ta, tb, M, N, K, alpha, a, b, beta, out):
-    need = ctypes.c_size_t()
+    f = ffi.fast().gemm_f16_ws
     args = (ta, tb, M, N, K, alpha, a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), beta, out.data_ptr(), out.stride(0))
     st = _stream()
-    ffi.call("cacti_hip_gemm_f16_ws", *args, None, 0, need, st)
-    if need.value:                               # not launched: the product wants a workspace
-        ws = torch.empty(need.value, dtype=torch.uint8, device=a.device)
-        ffi.call("cacti_hip_gemm_f16_ws", *args, ws.data_ptr(), need.value, need, st)
+    need = f(*args, None, 0, st)
+    if need > 0:                                 # not launched: the product wants a workspace
+        ws = torch.empty(need, dtype=torch.uint8, device=a.device)
+        need = f(*args, ws.data_ptr(), need, st)
+    if need < 0:
+        ffi.check(-1000000 - need)
 
 
 def gemm_batched(As, Bs, ta=False, tb=False, alpha=1.0, beta=0.0, outs=None):
@@ -82,7 +115,7 @@ def gemm_batched(As, Bs, ta=False, tb=False, alpha=1.0, beta=0.0, outs=None):
 def gemm_strided_batched(ta, tb, nblk, M, N, K, alpha, a, lda, sa, b, ldb, sb, beta, c, ldc, sc,
                          tri=0):
     """tri: 0 dense; 1 only tril(C) wanted (rest unwritten); 2 A = tril; 3 A^T with A = tril."""
-    ffi.call("cacti_hip_gemm_f16_strided_batched_tri", int(ta), int(tb), nblk, M, N, K, alpha,
+    _do.gemm_f16_strided_batched_tri(int(ta), int(tb), nblk, M, N, K, alpha,
              a.data_ptr(), lda, sa, b.data_ptr(), ldb, sb, beta, c.data_ptr(), ldc, sc, int(tri),
              _stream())
     return c
@@ -112,8 +145,8 @@ def attention_fwd(q, k, v, alpha):
     _chk(q), _chk(k), _chk(v)
     S, H, Dh = q.shape
     o = torch.empty_like(q)
-    stats = torch.empty(ffi.lib().cacti_hip_attention_stats_bytes(S, H) // 4, dtype=torch.float32, device=q.device)
-    ffi.call("cacti_hip_attention_fwd", S, H, Dh, alpha, q.data_ptr(), k.data_ptr(), v.data_ptr(), H * Dh,
+    stats = torch.empty(_size("attention_stats_bytes", S, H) // 4, dtype=torch.float32, device=q.device)
+    _do.attention_fwd(S, H, Dh, alpha, q.data_ptr(), k.data_ptr(), v.data_ptr(), H * Dh,
              o.data_ptr(), stats.data_ptr(), _stream())
     return o, stats
 
@@ -127,10 +160,10 @@ def attention_bwd(q, k, v, dO, stats, alpha, acc=None, o=None):
     S, H, Dh = q.shape
     dq, dk, dv = acc if acc is not None else (torch.empty_like(q), torch.empty_like(q), torch.empty_like(q))
     a = int(acc is not None)
-    nbytes = ffi.lib().cacti_hip_attention_bwd_workspace(S, H)
+    nbytes = _size("attention_bwd_workspace", S, H)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-    ffi.call("cacti_hip_attention_bwd", S, H, Dh, alpha, q.data_ptr(), k.data_ptr(), v.data_ptr(),
-             0 if o is None else o.data_ptr(), dO.data_ptr(), H * Dh, stats.data_ptr(), dq.data_ptr(), a,
+    _do.attention_bwd(S, H, Dh, alpha, q.data_ptr(), k.data_ptr(), v.data_ptr(),
+             _p(o), dO.data_ptr(), H * Dh, stats.data_ptr(), dq.data_ptr(), a,
              dk.data_ptr(), a, dv.data_ptr(), a,
              ws.data_ptr(), nbytes, _stream())
     return dq, dk, dv
@@ -141,7 +174,7 @@ def rms_norm_fwd(x, w, eps):
     _chk(x), _chk(w)
     N, D = x.shape
     y = torch.empty_like(x)
-    ffi.call("cacti_hip_rms_norm_fwd", N, D, x.data_ptr(), w.data_ptr(), eps, y.data_ptr(),
+    _do.rms_norm_fwd(N, D, x.data_ptr(), w.data_ptr(), eps, y.data_ptr(),
              _stream())
     return y
 
@@ -151,7 +184,7 @@ def add_rms_norm_fwd(a, b, w, eps):
     _chk(a), _chk(b), _chk(w)
     N, D = a.shape
     s, y = torch.empty_like(a), torch.empty_like(a)
-    ffi.call("cacti_hip_add_rms_norm_fwd", N, D, a.data_ptr(), b.data_ptr(), w.data_ptr(), eps,
+    _do.add_rms_norm_fwd(N, D, a.data_ptr(), b.data_ptr(), w.data_ptr(), eps,
              s.data_ptr(), y.data_ptr(), _stream())
     return s, y
 
@@ -162,9 +195,9 @@ def rms_norm_bwd(x, w, eps, dy, dx_acc=None, dw_acc=None):
     N, D = x.shape
     dx = torch.empty_like(x) if dx_acc is None else _chk(dx_acc)
     dw = torch.empty_like(w) if dw_acc is None else _chk(dw_acc)
-    nbytes = ffi.lib().cacti_hip_rms_norm_bwd_workspace(N, D)
+    nbytes = _size("rms_norm_bwd_workspace", N, D)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    ffi.call("cacti_hip_rms_norm_bwd", N, D, x.data_ptr(), w.data_ptr(), eps, dy.data_ptr(),
+    _do.rms_norm_bwd(N, D, x.data_ptr(), w.data_ptr(), eps, dy.data_ptr(),
              dx.data_ptr(), int(dx_acc is not None), dw.data_ptr(), int(dw_acc is not None),
              ws.data_ptr(), nbytes, _stream())
     return dx, dw
@@ -173,7 +206,7 @@ def rms_norm_bwd(x, w, eps, dy, dx_acc=None, dw_acc=None):
 def rope_tables(S, Dh, device="cuda"):
     cos = torch.empty((S, Dh), dtype=F16, device=device)
     sin = torch.empty((S, Dh), dtype=F16, device=device)
-    ffi.call("cacti_hip_rope_tables", S, Dh, cos.data_ptr(), sin.data_ptr(), _stream())
+    _do.rope_tables(S, Dh, cos.data_ptr(), sin.data_ptr(), _stream())
     return cos, sin
 
 
@@ -181,7 +214,7 @@ def rope_fwd(x, cos, sin):
     _chk(x), _chk(cos), _chk(sin)
     S, H, Dh = x.shape
     y = torch.empty_like(x)
-    ffi.call("cacti_hip_rope_fwd", S, H, Dh, x.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+    _do.rope_fwd(S, H, Dh, x.data_ptr(), cos.data_ptr(), sin.data_ptr(),
              y.data_ptr(), _stream())
     return y
 
@@ -190,7 +223,7 @@ def rope_bwd(dy, cos, sin, dx_acc=None):
     _chk(dy), _chk(cos), _chk(sin)
     S, H, Dh = dy.shape
     dx = torch.empty_like(dy) if dx_acc is None else _chk(dx_acc)
-    ffi.call("cacti_hip_rope_bwd", S, H, Dh, dy.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+    _do.rope_bwd(S, H, Dh, dy.data_ptr(), cos.data_ptr(), sin.data_ptr(),
              dx.data_ptr(), int(dx_acc is not None), _stream())
     return dx
 
@@ -198,7 +231,7 @@ def rope_bwd(dy, cos, sin, dx_acc=None):
 def silu_gate_fwd(g, u):
     _chk(g), _chk(u)
     h = torch.empty_like(g)
-    ffi.call("cacti_hip_silu_gate_fwd", g.numel(), g.data_ptr(), u.data_ptr(), h.data_ptr(),
+    _do.silu_gate_fwd(g.numel(), g.data_ptr(), u.data_ptr(), h.data_ptr(),
              _stream())
     return h
 
@@ -207,7 +240,7 @@ def silu_gate_bwd(g, u, dh, dg_acc=None, du_acc=None):
     _chk(g), _chk(u), _chk(dh)
     dg = torch.empty_like(g) if dg_acc is None else _chk(dg_acc)
     du = torch.empty_like(g) if du_acc is None else _chk(du_acc)
-    ffi.call("cacti_hip_silu_gate_bwd", g.numel(), g.data_ptr(), u.data_ptr(), dh.data_ptr(),
+    _do.silu_gate_bwd(g.numel(), g.data_ptr(), u.data_ptr(), dh.data_ptr(),
              dg.data_ptr(), int(dg_acc is not None), du.data_ptr(), int(du_acc is not None),
              _stream())
     return dg, du
@@ -220,7 +253,7 @@ def causal_softmax_fwd(s16):
     # the kernel writes j <= i and zeros only up to the next multiple of 256 columns:
     # start from zeros so that dense consumers may read the whole row
     p = torch.zeros_like(s16)
-    ffi.call("cacti_hip_causal_softmax_fwd", S, H, s16.data_ptr(), p.data_ptr(), _stream())
+    _do.causal_softmax_fwd(S, H, s16.data_ptr(), p.data_ptr(), _stream())
     return p
 
 
@@ -228,13 +261,15 @@ def causal_softmax_bwd(s16, dp16):
     _chk(s16), _chk(dp16)
     S, H, _ = s16.shape
     ds = torch.zeros_like(s16)
-    ffi.call("cacti_hip_causal_softmax_bwd", S, H, s16.data_ptr(), dp16.data_ptr(), ds.data_ptr(),
+    _do.causal_softmax_bwd(S, H, s16.data_ptr(), dp16.data_ptr(), ds.data_ptr(),
              _stream())
     return ds
 
 
 def _raise_index(status, what):
-    v = int(status.item())
+    rc, v = ffi.fast().read_i32(status.data_ptr(), _stream())
+    if rc:
+        ffi.check(rc)
     if v:
         raise IndexError("%s: id out of range at row %d" % (what, v - 1))
 
@@ -247,7 +282,7 @@ def softmax_ce_fwd(logit, tok, want_prob=True):
     loss = torch.empty((N,), dtype=torch.float32, device=logit.device)
     amax = torch.empty((N,), dtype=torch.int16, device=logit.device)
     status = torch.zeros(1, dtype=torch.int32, device=logit.device)
-    ffi.call("cacti_hip_softmax_ce_fwd", N, V, logit.data_ptr(), tok.data_ptr(), _p(prob),
+    _do.softmax_ce_fwd(N, V, logit.data_ptr(), tok.data_ptr(), _p(prob),
              loss.data_ptr(), amax.data_ptr(), status.data_ptr(), _stream())
     _raise_index(status, "softmax_ce_fwd")
     return prob, loss, amax
@@ -257,7 +292,7 @@ def softmax_ce_bwd(logit, tok, scale, acc=None):
     _chk(logit), _chk(scale, torch.float32)
     N, V = logit.shape
     d = torch.empty_like(logit) if acc is None else _chk(acc)
-    ffi.call("cacti_hip_softmax_ce_bwd", N, V, logit.data_ptr(), tok.data_ptr(), scale.data_ptr(),
+    _do.softmax_ce_bwd(N, V, logit.data_ptr(), tok.data_ptr(), scale.data_ptr(),
              d.data_ptr(), int(acc is not None), _stream())
     return d
 
@@ -268,7 +303,7 @@ def embed_fwd(W, tok):
     S = tok.numel()
     y = torch.empty((S, D), dtype=F16, device=W.device)
     status = torch.zeros(1, dtype=torch.int32, device=W.device)
-    ffi.call("cacti_hip_embed_fwd", V, D, W.data_ptr(), S, tok.data_ptr(), y.data_ptr(),
+    _do.embed_fwd(V, D, W.data_ptr(), S, tok.data_ptr(), y.data_ptr(),
              status.data_ptr(), _stream())
     _raise_index(status, "embed_fwd")
     return y
@@ -278,20 +313,20 @@ def embed_bwd(V, tok, dy, acc=None):
     _chk(dy)
     S, D = dy.shape
     dW = torch.empty((V, D), dtype=F16, device=dy.device) if acc is None else _chk(acc)
-    ffi.call("cacti_hip_embed_bwd", V, D, S, tok.data_ptr(), dy.data_ptr(), dW.data_ptr(),
+    _do.embed_bwd(V, D, S, tok.data_ptr(), dy.data_ptr(), dW.data_ptr(),
              int(acc is not None), _stream())
     return dW
 
 
 def add_f16(a, b, out=None):
     out = torch.empty_like(a) if out is None else out
-    ffi.call("cacti_hip_add_f16", a.numel(), a.data_ptr(), b.data_ptr(), out.data_ptr(), _stream())
+    _do.add_f16(a.numel(), a.data_ptr(), b.data_ptr(), out.data_ptr(), _stream())
     return out
 
 
 def accumulate_1d(dst, src):
     name = {torch.float32: "f32", torch.float16: "f16", torch.int16: "u16"}[dst.dtype]
-    ffi.call("cacti_hip_accumulate_1d_" + name, dst.data_ptr(), src.data_ptr(), dst.numel(),
+    getattr(_do, "accumulate_1d_" + name)(dst.data_ptr(), src.data_ptr(), dst.numel(),
              _stream())
     return dst
 
@@ -301,7 +336,7 @@ def nan_count(x):
     """Number of NaNs of an f16 tensor as a 0-d int64 device tensor (src/thunk/op.rs:273-349)."""
     _chk(x)
     out = torch.empty((), dtype=torch.int64, device=x.device)
-    ffi.call("cacti_hip_nan_count_f16", x.numel(), x.data_ptr(), out.data_ptr(), _stream())
+    _do.nan_count_f16(x.numel(), x.data_ptr(), out.data_ptr(), _stream())
     return out
 
 
@@ -309,7 +344,7 @@ def abs_log2_hist8(x):
     """int64[256] histogram of the floor(log2 |x|) classes of an f16 tensor (src/thunk/op.rs:351-441)."""
     _chk(x)
     out = torch.empty(256, dtype=torch.int64, device=x.device)
-    ffi.call("cacti_hip_abs_log2_hist8_f16", x.numel(), x.data_ptr(), out.data_ptr(), _stream())
+    _do.abs_log2_hist8_f16(x.numel(), x.data_ptr(), out.data_ptr(), _stream())
     return out
 
 
@@ -324,7 +359,7 @@ def digests(xs):
     out = torch.empty((n, 257), dtype=torch.int64, device=dev)
     if n == 0:
         return out[:, :256], out[:, 256]
-    scratch = torch.empty(ffi.lib().cacti_hip_digests_scratch_bytes(n), dtype=torch.uint8, device=dev)
+    scratch = torch.empty(_size("digests_scratch_bytes", n), dtype=torch.uint8, device=dev)
     ptrs = (C.c_void_p * n)(*[x.data_ptr() for x in xs])
     ns = (C.c_int64 * n)(*[x.numel() for x in xs])
     ffi.call("cacti_hip_digests_f16_batch", n, C.cast(ptrs, C.c_void_p), C.cast(ns, C.c_void_p),
@@ -341,7 +376,7 @@ def online_average_scale_(u, v, src_scale, rate):
     """v += rate * (src_scale * f32(u) - v) in place (src/thunk/op.rs:3884-3939)."""
     _chk(u), _f(v)
     assert u.numel() == v.numel()
-    ffi.call("cacti_hip_online_average_scale_f16_f32", u.numel(), u.data_ptr(), v.data_ptr(), src_scale, rate,
+    _do.online_average_scale_f16_f32(u.numel(), u.data_ptr(), v.data_ptr(), src_scale, rate,
              _stream())
     return v
 
@@ -350,7 +385,7 @@ def online_average_square_scale_(u, v, src_scale, rate):
     """v += rate * ((src_scale * f32(u))^2 - v) in place (src/thunk/op.rs:3941-4002)."""
     _chk(u), _f(v)
     assert u.numel() == v.numel()
-    ffi.call("cacti_hip_online_average_square_scale_f16_f32", u.numel(), u.data_ptr(), v.data_ptr(), src_scale,
+    _do.online_average_square_scale_f16_f32(u.numel(), u.data_ptr(), v.data_ptr(), src_scale,
              rate, _stream())
     return v
 
@@ -360,7 +395,7 @@ def online_adamw_update_(g1, g2, w, signed_lr, lr_unbias, lamda, eps):
     (src/thunk/op.rs:4004-4062)."""
     _f(g1), _f(g2), _f(w)
     assert g1.numel() == g2.numel() == w.numel()
-    ffi.call("cacti_hip_online_adamw_update_f32", w.numel(), g1.data_ptr(), g2.data_ptr(), w.data_ptr(),
+    _do.online_adamw_update_f32(w.numel(), g1.data_ptr(), g2.data_ptr(), w.data_ptr(),
              signed_lr, lr_unbias, lamda, eps, _stream())
     return w
 
@@ -368,14 +403,14 @@ def online_adamw_update_(g1, g2, w, signed_lr, lr_unbias, lamda, eps):
 def cast_f32_f16(x):
     _f(x)
     y = torch.empty(x.shape, dtype=torch.float16, device=x.device)
-    ffi.call("cacti_hip_cast_f32_f16", x.numel(), x.data_ptr(), y.data_ptr(), _stream())
+    _do.cast_f32_f16(x.numel(), x.data_ptr(), y.data_ptr(), _stream())
     return y
 
 
 def cast_f16_f32(x):
     _chk(x)
     y = torch.empty(x.shape, dtype=torch.float32, device=x.device)
-    ffi.call("cacti_hip_cast_f16_f32", x.numel(), x.data_ptr(), y.data_ptr(), _stream())
+    _do.cast_f16_f32(x.numel(), x.data_ptr(), y.data_ptr(), _stream())
     return y
 
 
@@ -402,7 +437,7 @@ def adamw32_step_(grads, avgs, avg2s, masters, params, scalars):
     arr = lambda ts: C.cast((C.c_void_p * n)(*[t.data_ptr() for t in ts]), C.c_void_p)
     ns = (C.c_int64 * n)(*[g.numel() for g in grads])
     sc = (C.c_float * 7)(*scalars)
-    scratch = torch.empty(ffi.lib().cacti_hip_adamw32_scratch_bytes(n), dtype=torch.uint8, device=grads[0].device)
+    scratch = torch.empty(_size("adamw32_scratch_bytes", n), dtype=torch.uint8, device=grads[0].device)
     ffi.call("cacti_hip_adamw32_step_f16_batch", n, arr(grads), arr(avgs), arr(avg2s), arr(masters), arr(params),
              C.cast(ns, C.c_void_p), C.cast(sc, C.c_void_p), scratch.data_ptr(), _stream())
 
@@ -411,23 +446,23 @@ def adamw32_step_(grads, avgs, avg2s, masters, params, scalars):
 def _raw_cast(name, x, in_dtype, out_dtype):
     _chk(x, in_dtype)
     y = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    ffi.call(name, x.numel(), x.data_ptr(), y.data_ptr(), _stream())
+    getattr(_do, name)(x.numel(), x.data_ptr(), y.data_ptr(), _stream())
     return y
 
 
 def raw_cast_bf16_f16(u):
     """bf16 bit patterns (int16 tensor) -> f16."""
-    return _raw_cast("cacti_hip_raw_cast_bf16_f16", u, torch.int16, torch.float16)
+    return _raw_cast("raw_cast_bf16_f16", u, torch.int16, torch.float16)
 
 
 def raw_cast_bf16_f32(u):
-    return _raw_cast("cacti_hip_raw_cast_bf16_f32", u, torch.int16, torch.float32)
+    return _raw_cast("raw_cast_bf16_f32", u, torch.int16, torch.float32)
 
 
 def raw_cast_f32_bf16(x):
     """f32 -> bf16 bit patterns (int16 tensor), truncating."""
-    return _raw_cast("cacti_hip_raw_cast_f32_bf16", x, torch.float32, torch.int16)
+    return _raw_cast("raw_cast_f32_bf16", x, torch.float32, torch.int16)
 
 
 def raw_cast_f16_bf16(x):
-    return _raw_cast("cacti_hip_raw_cast_f16_bf16", x, torch.float16, torch.int16)
+    return _raw_cast("raw_cast_f16_bf16", x, torch.float16, torch.int16)

@@ -89,6 +89,9 @@ int cacti_hip_event_query(void *event);                         /* lib.rs:453   
 int cacti_hip_event_sync(void *event);                          /* lib.rs:461       */
 int cacti_hip_event_elapsed_ms(void *start, void *stop, float *ms);
 
+/* One 32-bit word of device memory (16-byte aligned) behind everything queued on the stream; returns when it is there. */
+int cacti_hip_read_i32(const void *dev, int32_t *value, void *stream);
+
 /* ------------------------------------------------------------------------- */
 /* GEMM: C = alpha * op(A) op(B) + beta * C, f16 x f16 -> fp32 accumulate ->   */
 /* f16 out, hand-written MFMA kernels.                                         */
