@@ -24,11 +24,15 @@ using namespace cacti;
 
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kGroups = kThreads / 8;      // positions per step and lane
+constexpr int kThreads = 256;              // of the scores launch; the values launch has kThreads or kWide
+constexpr int kWide = 512;
 constexpr int kStep = 4;                   // positions of a lane in flight
-constexpr int kSlice = kGroups * kStep;    // positions per workgroup of the scores launch
-constexpr int kOwnScores = 1024;
+constexpr int kSlice = kThreads / 8 * kStep;   // positions per workgroup of the scores launch
+// Measured, us at 70 / 300 / 600 / 1000 / 1540 positions, 16 heads of 128: own scores on 256 lanes 4.6 / 6.8 / 10.0 / 13.7 /
+// 19.6, on 512 lanes 5.4 / 7.1 / 8.7 / 10.5 / 14.3, on 1024 7.2 / 7.4 / 10.2 / 11.1 / 16.0; scores apart and 512 lanes 7.2 / 7.8 / 8.4
+// / 9.7 / 11.2.  32 heads of 100 cross at the same places.
+constexpr int kNarrow = 320;               // up to here kThreads lanes, own scores
+constexpr int kOwnScores = 512;            // up to here kWide lanes, own scores; beyond, a scores launch
 constexpr int kMaxCols = 8192;             // score rows live in LDS
 
 struct __attribute__((aligned(8))) h4 {
@@ -59,10 +63,11 @@ __device__ __forceinline__ void load_q(h4 (&qv)[T][NP], const half_t *q, int64_t
 
 // f16(alpha q . K[j]) for the positions j0 + g + 32 it (it < kStep) below `end`, by the first of a position's lanes to
 // out[t * ldo + j - first]
-template <int T, int NP>
+template <int T, int NP, int NT>
 __device__ __forceinline__ void scores_step(const h4 (&qv)[T][NP], const half_t *k_head, int64_t ldk, int pieces, float alpha, int j0,
                                             int end, half_t *out, int64_t ldo, int first)
 {
+    constexpr int kGroups = NT / 8;
     const int i8 = threadIdx.x & 7, g = threadIdx.x >> 3;
     h4 kv[kStep][NP];
 #pragma unroll
@@ -94,19 +99,20 @@ decode_scores_kernel(int C, int Dh, float alpha, const half_t *__restrict__ q, i
     const int h = blockIdx.y, j0 = blockIdx.x * kSlice;
     h4 qv[T][NP];
     load_q<T, NP>(qv, q, ldq, h, Dh, threadIdx.x & 7);
-    scores_step<T, NP>(qv, kc + h * hsk, ldk, Dh / 4, alpha, j0, min(C, j0 + kSlice), s16 + (int64_t)h * T * ld, ld, 0);
+    scores_step<T, NP, kThreads>(qv, kc + h * hsk, ldk, Dh / 4, alpha, j0, min(C, j0 + kSlice), s16 + (int64_t)h * T * ld, ld, 0);
 }
 
 // OWN: the scores are formed here; otherwise they are s16[h][t][ld].
-template <int T, int NP, bool OWN>
-__global__ void __launch_bounds__(kThreads)
+template <int T, int NP, bool OWN, int NT>
+__global__ void __launch_bounds__(NT)
 decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__restrict__ q, int64_t ldq, const half_t *__restrict__ kc,
                      const half_t *__restrict__ vc, int64_t ldkv, int64_t hs, const half_t *__restrict__ s16, int64_t ld,
                      half_t *__restrict__ out, int64_t ldo)
 {
     extern __shared__ __attribute__((aligned(16))) half_t sp[];           // [T][ld]: scores, then probabilities
-    __shared__ float scratch[2][T][kThreads / 64];
-    __shared__ float red[kThreads / 64][T][8][4];
+    __shared__ float scratch[2][T][NT / 64];
+    __shared__ float red[NT / 64][T][8][4];
+    constexpr int kGroups = NT / 8;            // positions per step and lane
     const int tid = threadIdx.x, i8 = tid & 7, g = tid >> 3, lane = tid & 63, wid = tid >> 6, h = blockIdx.y;
     const int pieces = Dh / 4, per = (pieces + gridDim.x - 1) / gridDim.x;        // pieces of this workgroup: at most 8
     const int piece = blockIdx.x * per + i8;
@@ -122,9 +128,9 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
     if (OWN) {
         h4 qv[T][NP];
         load_q<T, NP>(qv, q, ldq, h, Dh, i8);
-        for (int j0 = 0; j0 < C; j0 += kSlice) scores_step<T, NP>(qv, kc + h * hs, ldkv, pieces, alpha, j0, C, sp, ld, 0);
+        for (int j0 = 0; j0 < C; j0 += kGroups * kStep) scores_step<T, NP, NT>(qv, kc + h * hs, ldkv, pieces, alpha, j0, C, sp, ld, 0);
     } else {
-        for (int i = tid; i < T * (int)ld / 8; i += kThreads) st8(sp + i * 8, ld8(s16 + (int64_t)h * T * ld + i * 8));
+        for (int i = tid; i < T * (int)ld / 8; i += NT) st8(sp + i * 8, ld8(s16 + (int64_t)h * T * ld + i * 8));
     }
     __syncthreads();
     // row maxima, then sums of exponentials, then the probabilities in place of the scores; row t sees live(t) positions
@@ -133,7 +139,7 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
 #pragma unroll
     for (int t = 0; t < T; t++) {
         float m = -INFINITY;
-        for (int j = tid; j < live(t); j += kThreads) m = fmaxf(m, h2f(sp[t * ld + j]));
+        for (int j = tid; j < live(t); j += NT) m = fmaxf(m, h2f(sp[t * ld + j]));
         m = wave_max(m);
         if (lane == 0) scratch[0][t][wid] = m;
     }
@@ -142,9 +148,9 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
     for (int t = 0; t < T; t++) {
         mx[t] = scratch[0][t][0];
 #pragma unroll
-        for (int w = 1; w < kThreads / 64; w++) mx[t] = fmaxf(mx[t], scratch[0][t][w]);
+        for (int w = 1; w < NT / 64; w++) mx[t] = fmaxf(mx[t], scratch[0][t][w]);
         float s = 0.f;
-        for (int j = tid; j < live(t); j += kThreads) s += exp_nonpos(fmaxf(h2f(sp[t * ld + j]) - mx[t], -100.0f));
+        for (int j = tid; j < live(t); j += NT) s += exp_nonpos(fmaxf(h2f(sp[t * ld + j]) - mx[t], -100.0f));
         s = wave_sum(s);
         if (lane == 0) scratch[1][t][wid] = s;
     }
@@ -153,9 +159,9 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
     for (int t = 0; t < T; t++) {
         sum[t] = scratch[1][t][0];
 #pragma unroll
-        for (int w = 1; w < kThreads / 64; w++) sum[t] += scratch[1][t][w];
+        for (int w = 1; w < NT / 64; w++) sum[t] += scratch[1][t][w];
         const RowDivide div(sum[t]);
-        for (int j = tid; j < C; j += kThreads) {
+        for (int j = tid; j < C; j += NT) {
             const float e = exp_nonpos(fmaxf(h2f(sp[t * ld + j]) - mx[t], -100.0f));
             sp[t * ld + j] = j < live(t) ? f2h(div(e)) : (half_t)0.f;
         }
@@ -166,9 +172,9 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
     for (int t = 0; t < T; t++)
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[t][i] = 0.f;
-    for (int j0 = 0; j0 < C; j0 += kSlice) {
+    for (int j0 = 0; j0 < C; j0 += kGroups * kStep) {
         h4 vn[kStep];
-        load_v(vn, j0 + kSlice);                                  // (behind the last position: its row again)
+        load_v(vn, j0 + kGroups * kStep);                                  // (behind the last position: its row again)
 #pragma unroll
         for (int it = 0; it < kStep; it++) {
             const int j = j0 + g + it * kGroups;
@@ -198,7 +204,7 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
         if (c < per && blockIdx.x * per + c < pieces) {
             float a = red[0][t][c][i];
 #pragma unroll
-            for (int w = 1; w < kThreads / 64; w++) a += red[w][t][c][i];
+            for (int w = 1; w < NT / 64; w++) a += red[w][t][c][i];
             out[t * ldo + h * Dh + 4 * (blockIdx.x * per + c) + i] = f2h(a);
         }
     }
@@ -218,30 +224,32 @@ struct DecodeArgs {
     hipStream_t st;
 };
 
+template <int T, int NP, bool OWN, int NT>
+int launch_values(const DecodeArgs &a, int64_t ld)
+{
+    const size_t smem = (size_t)T * (size_t)ld * sizeof(half_t);
+    auto kern = decode_values_kernel<T, NP, OWN, NT>;
+    if (smem > 32 * 1024) {
+        static DeviceOnce attr_set;
+        if (!attr_set.fresh()) {
+            CACTI_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, T * kMaxCols * (int)sizeof(half_t)));
+            attr_set.mark();
+        }
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)((a.Dh / 4 + 7) / 8), (unsigned)a.H), dim3(NT), smem, a.st, a.C, a.Dh, a.row0, a.alpha, a.q,
+                       a.ldq, a.kc, a.vc, a.ldkv, a.hs, (const half_t *)a.s16, ld, a.out, a.ldo);
+    return launch_status("attn_decode");
+}
+
 template <int T, int NP>
 int launch(const DecodeArgs &a)
 {
     const int64_t ld = (a.C + 7) / 8 * 8;
-    const size_t smem = (size_t)T * (size_t)ld * sizeof(half_t);
-    const dim3 grid((unsigned)((a.Dh / 4 + 7) / 8), (unsigned)a.H), block(kThreads);
-    if (a.C <= kOwnScores) {
-        hipLaunchKernelGGL((decode_values_kernel<T, NP, true>), grid, block, smem, a.st, a.C, a.Dh, a.row0, a.alpha, a.q, a.ldq, a.kc, a.vc,
-                           a.ldkv, a.hs, (const half_t *)nullptr, ld, a.out, a.ldo);
-    } else {
-        if (smem > 48 * 1024) {
-            static DeviceOnce attr_set;
-            if (!attr_set.fresh()) {
-                CACTI_HIP(hipFuncSetAttribute((const void *)decode_values_kernel<T, NP, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                              T * kMaxCols * (int)sizeof(half_t)));
-                attr_set.mark();
-            }
-        }
-        hipLaunchKernelGGL((decode_scores_kernel<T, NP>), dim3((unsigned)((a.C + kSlice - 1) / kSlice), (unsigned)a.H), block, 0, a.st, a.C,
-                           a.Dh, a.alpha, a.q, a.ldq, a.kc, a.ldkv, a.hs, a.s16, ld);
-        hipLaunchKernelGGL((decode_values_kernel<T, NP, false>), grid, block, smem, a.st, a.C, a.Dh, a.row0, a.alpha, a.q, a.ldq, a.kc, a.vc,
-                           a.ldkv, a.hs, (const half_t *)a.s16, ld, a.out, a.ldo);
-    }
-    return launch_status("attn_decode");
+    if (a.C <= kNarrow) return launch_values<T, NP, true, kThreads>(a, ld);
+    if (a.C <= kOwnScores) return launch_values<T, NP, true, kWide>(a, ld);
+    hipLaunchKernelGGL((decode_scores_kernel<T, NP>), dim3((unsigned)((a.C + kSlice - 1) / kSlice), (unsigned)a.H), dim3(kThreads), 0, a.st,
+                       a.C, a.Dh, a.alpha, a.q, a.ldq, a.kc, a.ldkv, a.hs, a.s16, ld);
+    return launch_values<T, NP, false, kWide>(a, ld);
 }
 
 template <int NP>

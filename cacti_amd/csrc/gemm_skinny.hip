@@ -2,12 +2,13 @@
 // a weight matrix).  The product is a stream over B: every byte of the weights is read once and
 // used M times, so the kernel is built for HBM, not for the matrix cores.
 //
-// A workgroup of 256 lanes owns R = 4 rows of B (4 output columns) and splits K over its lanes
-// in 16-byte pieces; a lane issues the loads of 2 or 4 pieces x 4 rows before it uses the first,
+// A workgroup of 64 or 256 lanes owns R = 4 rows of B (4 output columns) and splits K over its lanes
+// in 16-byte pieces; a lane issues the loads of its 1 to 5 pieces x 4 rows before it uses the first,
 // accumulates M x 4 fp32 sums with v_dot2_f32_f16 (the scalar form, 3 instructions per product
 // with the conversions, made the kernel compute-bound), and the sums are reduced over the wave (cross-lane adds) and
-// over the 4 waves (LDS).  N / 4 workgroups: 800 for N = 3200, 8 resident per CU.  A (a few KiB)
-// is re-read from L2 by every workgroup.
+// over the waves (LDS).  N / 4 workgroups: 800 for N = 3200, 8 resident per CU.  A (a few KiB)
+// is re-read from L2 by every workgroup.  What a launch costs beyond its bytes at 6 TB/s is some 4 us: start, the first
+// loads' latency, the norm and the reductions.
 //
 // Two fusions keep a decoding step from paying a launch for every small thunk:
 //  * NORM: A is not read but formed per workgroup as the RMSNorm of a row x (optionally of the
@@ -25,9 +26,8 @@ namespace cacti {
 
 namespace {
 
-constexpr int kThreads = 256;
 constexpr int kRows = 4;
-constexpr int kMaxPre = 4;                 // pieces of K per lane whose loads are in flight together (2 or 4)
+constexpr int kMaxNorm = 1024;             // 16-byte pieces of a row that NORM takes (4 waves x 4 pieces per lane)
 
 struct SkinnyArgs {
     int64_t N, K;
@@ -70,16 +70,18 @@ __device__ __forceinline__ uint32_t arg_key(half_t v, int64_t n)
     return o << 16 | (uint32_t)(0xffff - n);
 }
 
+template <int W>
 __device__ __forceinline__ float block_sum(float v, float *scratch)
 {
     v = wave_sum(v);
+    if (W == 1) return v;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     __syncthreads();
     if (lane == 0) scratch[wid] = v;
     __syncthreads();
     float r = scratch[0];
 #pragma unroll
-    for (int w = 1; w < kThreads / 64; w++) r += scratch[w];
+    for (int w = 1; w < W; w++) r += scratch[w];
     return r;
 }
 
@@ -94,14 +96,16 @@ __device__ __forceinline__ float dot8(const half8_t &a, const half8_t &b, float 
     return acc;
 }
 
-template <int M, bool NORM, int EPI, int kPre>
-__global__ void __launch_bounds__(kThreads)
+// W waves split K, kPre pieces per lane and pass.
+template <int M, bool NORM, int EPI, int W, int kPre>
+__global__ void __launch_bounds__(W * 64)
 gemm_skinny_nt_kernel(SkinnyArgs p)
 {
+    constexpr int kThreads = W * 64;
     constexpr bool GATE = EPI == E_GATE;
     constexpr int NB = GATE ? 2 : 1;
-    __shared__ float part[kThreads / 64][NB * M * kRows];
-    __shared__ float scratch[kThreads / 64];
+    __shared__ float part[W][NB * M * kRows];
+    __shared__ float scratch[W];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int64_t n0 = (int64_t)blockIdx.x * kRows;
     float acc[NB][M][kRows];
@@ -115,14 +119,14 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
     const half_t *brow[NB][kRows];
     int64_t col[kRows];
     if (EPI == E_QKV) {
-        // the workgroup owns two rotation pairs of one head: columns d, d + 1, d + Dh/2, d + 1 + Dh/2;
-        // blockIdx.y picks the query, key or value projection
-        const int hf = p.Dh / 2, per_head = hf / 2;
-        const int head = blockIdx.x / per_head, d0 = 2 * (blockIdx.x - head * per_head);
+        // the workgroup owns kRows / 2 consecutive rotation pairs (columns d and d + Dh/2 of a head), the left columns
+        // in the first half of its rows; blockIdx.y picks the query, key or value projection
+        const int hf = p.Dh / 2;
         const half_t *Bsel = blockIdx.y == 0 ? p.B : blockIdx.y == 1 ? p.B2 : p.B3;
 #pragma unroll
         for (int r = 0; r < kRows; r++) {
-            col[r] = (int64_t)head * p.Dh + d0 + (r & 1) + (r >> 1) * hf;
+            const int pair = blockIdx.x * (kRows / 2) + r % (kRows / 2), head = pair / hf;
+            col[r] = (int64_t)head * p.Dh + (pair - head * hf) + (r / (kRows / 2)) * hf;
             brow[0][r] = Bsel + col[r] * p.ldb;
         }
     } else {
@@ -195,7 +199,7 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
                         }
                     }
                 }
-                ss = block_sum(ss, scratch);
+                ss = block_sum<W>(ss, scratch);
                 const float rinv = 1.0f / sqrtf(ss / (float)p.K + p.eps);
 #pragma unroll
                 for (int j = 0; j < kPre; j++) {
@@ -242,15 +246,15 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
         if (tid < M * kRows) {
             float v = 0.f;
 #pragma unroll
-            for (int w = 0; w < kThreads / 64; w++) v += part[w][m * kRows + r];
+            for (int w = 0; w < W; w++) v += part[w][m * kRows + r];
             xr[m][r] = rnd16(p.alpha * v);
         }
         __syncthreads();
         if (tid < M * kRows) {
             float y = xr[m][r];
             if (blockIdx.y < 2) {
-                const bool left = r < 2;
-                const float xp = xr[m][r ^ 2];
+                const bool left = r < kRows / 2;
+                const float xp = xr[m][left ? r + kRows / 2 : r - kRows / 2];
                 const int64_t d = col[r] % p.Dh;
                 const float cs = h2f(p.cos16[m * p.Dh + d]), sn = h2f(p.sin16[m * p.Dh + d]);
                 y = rnd16(rnd16(y * cs) + rnd16((left ? -xp : xp) * sn));
@@ -271,7 +275,7 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
         for (int q = 0; q < NB; q++) {
             v[q] = 0.f;
 #pragma unroll
-            for (int w = 0; w < kThreads / 64; w++) v[q] += part[w][(q * M + m) * kRows + r];
+            for (int w = 0; w < W; w++) v[q] += part[w][(q * M + m) * kRows + r];
         }
         if (EPI == E_PLAIN && p.cand) {
             uint32_t k = n0 + r < p.N ? arg_key(f2h(p.alpha * v[0]), n0 + r) : 0u;
@@ -315,24 +319,40 @@ finish_rows_kernel(int M, int count, const uint32_t *__restrict__ cand, uint16_t
     }
 }
 
-template <bool NORM, int EPI, int kPre>
-int launch_pre(int64_t M, const SkinnyArgs &p, hipStream_t st)
+template <int M, bool NORM, int EPI, int W, int kPre>
+void launch_cfg(const SkinnyArgs &p, hipStream_t st)
 {
-    const dim3 grid((unsigned)((p.N + kRows - 1) / kRows), EPI == E_QKV ? 3 : 1), block(kThreads);
-    switch (M) {
-        case 1: hipLaunchKernelGGL((gemm_skinny_nt_kernel<1, NORM, EPI, kPre>), grid, block, 0, st, p); break;
-        case 2: hipLaunchKernelGGL((gemm_skinny_nt_kernel<2, NORM, EPI, kPre>), grid, block, 0, st, p); break;
-        case 3: hipLaunchKernelGGL((gemm_skinny_nt_kernel<3, NORM, EPI, kPre>), grid, block, 0, st, p); break;
-        default: hipLaunchKernelGGL((gemm_skinny_nt_kernel<4, NORM, EPI, kPre>), grid, block, 0, st, p); break;
-    }
-    return launch_status("gemm_skinny_nt");
+    const dim3 grid((unsigned)((p.N + kRows - 1) / kRows), EPI == E_QKV ? 3 : 1), block(W * 64);
+    hipLaunchKernelGGL((gemm_skinny_nt_kernel<M, NORM, EPI, W, kPre>), grid, block, 0, st, p);
 }
 
-// rows of at most 4096 elements fit two pieces per lane: fewer registers, more workgroups per CU
+// A row of K is cut over the lanes of the workgroup with as little left over as may be (lanes without a piece of their
+// own still load): K = 2048 is one piece per lane of 4 waves (two: gate and up 11.5 against 10.3 us, a head of 32000 25.5
+// against 22.0), K = 8640 five in one pass (four in two: 13.2 against 11.5).  Few pieces: one wave, so that no barrier stands
+// between its loads and its result.  Eight columns per workgroup instead of four changed nothing (13.9 and 14.1 us for q,
+// k, v of 3200).
 template <bool NORM, int EPI>
 int launch(int64_t M, const SkinnyArgs &p, hipStream_t st)
 {
-    return p.K <= 8 * 2 * kThreads ? launch_pre<NORM, EPI, 2>(M, p, st) : launch_pre<NORM, EPI, kMaxPre>(M, p, st);
+    const int64_t pieces = p.K / 8;
+    if (M == 1) {
+        if (pieces <= 64) launch_cfg<1, NORM, EPI, 1, 1>(p, st);
+        else if (pieces <= 128) launch_cfg<1, NORM, EPI, 1, 2>(p, st);
+        else if (pieces <= 256) launch_cfg<1, NORM, EPI, 4, 1>(p, st);
+        else if (pieces <= 512) launch_cfg<1, NORM, EPI, 4, 2>(p, st);
+        else if (pieces <= 768) launch_cfg<1, NORM, EPI, 4, 3>(p, st);
+        else if (!NORM && EPI == E_PLAIN && pieces > 1024 && pieces <= 1280) launch_cfg<1, false, E_PLAIN, 4, 5>(p, st);
+        else launch_cfg<1, NORM, EPI, 4, 4>(p, st);
+    } else if (pieces <= 512) {
+        if (M == 2) launch_cfg<2, NORM, EPI, 4, 2>(p, st);
+        else if (M == 3) launch_cfg<3, NORM, EPI, 4, 2>(p, st);
+        else launch_cfg<4, NORM, EPI, 4, 2>(p, st);
+    } else {
+        if (M == 2) launch_cfg<2, NORM, EPI, 4, 4>(p, st);
+        else if (M == 3) launch_cfg<3, NORM, EPI, 4, 4>(p, st);
+        else launch_cfg<4, NORM, EPI, 4, 4>(p, st);
+    }
+    return launch_status("gemm_skinny_nt");
 }
 
 }  // namespace
@@ -423,8 +443,8 @@ CACTI_API int cacti_hip_rows_norm_matmul_f16(int64_t M, int64_t N, int64_t K, co
                                              const void *B_mul, void *C, void *stream)
 {
     CACTI_REQUIRE(M >= 1 && M <= 4, CACTI_E_NOTIMPL, "rows_norm_matmul: 1 to 4 rows are handled here (M=%lld)", (long long)M);
-    CACTI_REQUIRE(N > 0 && K > 0 && K % 8 == 0 && K <= 8 * kMaxPre * kThreads, CACTI_E_NOTIMPL,
-                  "rows_norm_matmul: need K %% 8 == 0 and K <= %d (K=%lld)", 8 * kMaxPre * kThreads, (long long)K);
+    CACTI_REQUIRE(N > 0 && K > 0 && K % 8 == 0 && K <= 8 * kMaxNorm, CACTI_E_NOTIMPL,
+                  "rows_norm_matmul: need K %% 8 == 0 and K <= %d (K=%lld)", 8 * kMaxNorm, (long long)K);
     CACTI_REQUIRE(x && B && C && (w_norm || (!x2 && !sum_out)), CACTI_E_INVALID, "rows_norm_matmul: null pointer");
     CACTI_REQUIRE(aligned(x, 16) && aligned(x2, 16) && aligned(w_norm, 16) && aligned(sum_out, 16) && aligned(B, 16) &&
                       aligned(B_mul, 16) && aligned(C, 2),
@@ -444,8 +464,8 @@ CACTI_API int cacti_hip_rows_qkv_rope_cache_f16(int64_t M, int64_t H, int64_t Dh
 {
     const int64_t D = H * Dh;
     CACTI_REQUIRE(M >= 1 && M <= 4, CACTI_E_NOTIMPL, "rows_qkv: 1 to 4 rows are handled here (M=%lld)", (long long)M);
-    CACTI_REQUIRE(H > 0 && Dh > 0 && Dh % 4 == 0 && D % 8 == 0 && D <= 8 * kMaxPre * kThreads, CACTI_E_NOTIMPL,
-                  "rows_qkv: need Dh %% 4 == 0, H*Dh %% 8 == 0 and H*Dh <= %d", 8 * kMaxPre * kThreads);
+    CACTI_REQUIRE(H > 0 && Dh > 0 && Dh % 4 == 0 && D % 8 == 0 && D <= 8 * kMaxNorm, CACTI_E_NOTIMPL,
+                  "rows_qkv: need Dh %% 4 == 0, H*Dh %% 8 == 0 and H*Dh <= %d", 8 * kMaxNorm);
     CACTI_REQUIRE(x && w_norm && Wq && Wk && Wv && cos16 && sin16 && q_rot && k_cache_rows && v_cache_rows, CACTI_E_INVALID,
                   "rows_qkv: null pointer");
     CACTI_REQUIRE(aligned(x, 16) && aligned(x2, 16) && aligned(w_norm, 16) && aligned(sum_out, 16) && aligned(Wq, 16) &&
