@@ -3,32 +3,24 @@
 // gradient each cycle (NanCountFutThunkSpec, src/thunk/op.rs:273-349; AbsLog2Hist8FutThunkSpec,
 // src/thunk/op.rs:351-441; used at examples/open_llama_3b_train.rs:409-424).
 //
-// Both stream the tensor once, 16 bytes per lane per step.  The histogram is kept in LDS
-// (ds_add_u32).  An f16 tensor of weights or gradients falls into a dozen adjacent bins, so the
-// 64 adds of a wave would pile up on a few addresses; every bin therefore has 16 counters, one
-// per lane & 15 (16 different banks), which are summed at the end and flushed with one 64-bit
-// atomic per non-empty bin and workgroup.  Counts are integers: the order of the adds does not
-// matter.
+// Both stream the tensor once, 16 bytes per lane per step.  One LDS add per element, into the dozen adjacent bins that the
+// values of a weight or gradient tensor fall into, was as much a bound as memory (3.7 TB/s).  A lane now counts pairs: the
+// two exponent fields of a 32-bit word are one of 1024 bins, so there are half as many adds and they spread over a hundred
+// addresses (four sets of bins, by lane & 3).  What an exponent field does not say, the subnormals' highest mantissa bit
+// and the NaNs, is looked for in two halves at a time and counted apart where there is any; zeros are the zero exponents
+// that were not subnormal.  At the end of a workgroup the pairs are summed to exponents and each non-empty class is
+// flushed with one 64-bit atomic.  Counts are integers: the order of the adds does not matter.
 #include "common.h"
-#include <vector>
+
+#include <type_traits>
 
 using namespace cacti;
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kSub = 16;                   // counters per bin
-
-// bin of one f16 bit pattern: 255 for inf / nan, 0 for +-0, floor(log2 |x|) + 127 otherwise
-// (the reference: exponent field - 15 for normal numbers, -24 + floor(log2 mantissa) for
-// subnormal ones, shifted by 0x7f into a u8; src/thunk/op.rs:417-432)
-__device__ __forceinline__ int abs_log2_bin(uint32_t u)
-{
-    const uint32_t b = (u >> 10) & 0x1f, m = u & 0x3ff;
-    if (b == 0x1f) return 255;
-    if (b == 0) return m == 0 ? 0 : 103 + (31 - __builtin_clz(m));   // -24 + log2 m + 127
-    return (int)b + 112;                                              // b - 15 + 127
-}
+constexpr int kSets = 4;                   // sets of pair bins
+constexpr int kSetPitch = 1024 + 16;       // their distance: the sets start in different banks
 
 __device__ __forceinline__ int is_nan16(uint32_t u) { return (u & 0x7c00) == 0x7c00 && (u & 0x3ff) != 0; }
 
@@ -37,12 +29,14 @@ __global__ void __launch_bounds__(64) zero_i64_kernel(unsigned long long *p, int
     for (int i = blockIdx.x * 64 + threadIdx.x; i < n; i += gridDim.x * 64) p[i] = 0;
 }
 
-// one tensor of a launch: workgroups first_block .. first_block + ceil(n / 8 / chunk) - 1 (at
-// least one) read it; out[0..255] += histogram (HIST), out[HIST ? 256 : 0] += NaN count (NANS)
+// one tensor of a launch: workgroups first_block .. first_block + blocks - 1 read it, sweep by sweep in turn (workgroup b
+// takes sweeps b, b + blocks, ..: what the launch reads at a time is contiguous.  With a contiguous 128 KiB for each
+// workgroup all of them walked the same addresses modulo 128 KiB, and so the same memory channels, at once: 3.4 TB/s);
+// out[0..255] += histogram (HIST), out[HIST ? 256 : 0] += NaN count (NANS)
 struct DigestSeg {
     const uint16_t *x;
     int64_t n;
-    int64_t first_block;
+    int32_t first_block, blocks;
     unsigned long long *out;
 };
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -64,69 +58,138 @@ inline int chunk_for(int64_t n)
     return (int)(sweeps < 1 ? 1 : sweeps > 8 ? 8 : sweeps) * kSweep;
 }
 
-template <bool HIST, bool NANS>
-__device__ __forceinline__ void digest_unit(const u32x4 v, uint32_t *wh, uint32_t &nans)
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+// Classes of the reference (src/thunk/op.rs:417-432): 255 for inf / nan, 0 for +-0, floor(log2 |x|) + 127 otherwise: exponent
+// field + 112 for normal numbers, 103 + the index of the highest mantissa bit for subnormal ones.
+struct Hist {
+    uint32_t pair[kSets * kSetPitch];      // [set][exponent of the low half | exponent of the high half << 5]
+    uint32_t expo[32], sub[10];
+};
+
+// subnormal halves and NaNs of a piece, one element at a time
+template <bool NANS>
+__device__ __forceinline__ void digest_rare(const uint32_t (&w)[4], Hist *h, uint32_t &nans)
 {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t lo = w[i] & 0xffff, hi = w[i] >> 16;
-        if (HIST) {
-            atomicAdd(&wh[abs_log2_bin(lo) * kSub], 1u);
-            atomicAdd(&wh[abs_log2_bin(hi) * kSub], 1u);
-        }
-        if (NANS) nans += is_nan16(lo) + is_nan16(hi);
+    for (int i = 0; i < 8; i++) {
+        const uint32_t x = w[i >> 1] >> (i & 1 ? 16 : 0) & 0x7fff;
+        if (x - 1 < 0x3ff) atomicAdd(&h->sub[31 - __builtin_clz(x)], 1u);
+        if (NANS) nans += x > 0x7c00;
     }
 }
 
-// segs == nullptr: the one tensor `one`; otherwise nseg tensors, segs[] sorted by first_block
+template <bool NANS>
+__device__ __forceinline__ void digest_unit(const u32x4 v, uint32_t *pairs, Hist *h, uint32_t &nans)
+{
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    u16x2 least = {0xffff, 0xffff}, most = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t x = w[i] & 0x7fff7fff, t = x >> 10 & 0x001f001f;
+        atomicAdd(pairs + ((t | t >> 11) & 0x3ff), 1u);
+        const u16x2 xv = __builtin_bit_cast(u16x2, x), one = {1, 1};
+        most = __builtin_elementwise_max(most, xv);
+        least = __builtin_elementwise_min(least, (u16x2)(xv - one));          // a zero wraps to the largest value
+    }
+    if (least.x < 0x3ff || least.y < 0x3ff || most.x > 0x7c00 || most.y > 0x7c00) digest_rare<NANS>(w, h, nans);
+}
+
+// The tensors of a launch, in the kernel's arguments: a table in device memory is a copy in front of the launch.
+constexpr int kSegsPerLaunch = 64;
+struct DigestArgs {
+    int nseg;
+    DigestSeg seg[kSegsPerLaunch];         // by first_block
+};
+
 template <bool HIST, bool NANS>
 __global__ void __launch_bounds__(kThreads)
-digest_kernel(DigestSeg one, const DigestSeg *__restrict__ segs, int nseg, int chunk)
+digest_kernel(DigestArgs args)
 {
-    __shared__ uint32_t hist[HIST ? 256 * kSub : 1];          // [bin][lane & 15]
+    __shared__ typename std::conditional<HIST, Hist, int>::type hist_mem;
+    Hist *const hist = reinterpret_cast<Hist *>(&hist_mem);
     const int lane = threadIdx.x & 63;
     if (HIST) {
-        for (int i = threadIdx.x; i < 256 * kSub; i += kThreads) hist[i] = 0;
+        for (int i = threadIdx.x; i < (int)(sizeof(Hist) / 4); i += kThreads) reinterpret_cast<uint32_t *>(hist)[i] = 0;
     }
-    DigestSeg sg = one;
-    if (segs) {
-        int lo = 0, hi = nseg - 1;                            // last segment starting at or before this block
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (segs[mid].first_block <= (int64_t)blockIdx.x) lo = mid;
-            else hi = mid - 1;
-        }
-        sg = segs[lo];
+    int seg = 0;
+    for (int hi = args.nseg - 1; seg < hi;) {                 // last segment starting at or before this block
+        const int mid = (seg + hi + 1) >> 1;
+        if (args.seg[mid].first_block <= (int)blockIdx.x) seg = mid;
+        else hi = mid - 1;
     }
+    const DigestSeg sg = args.seg[seg];
     if (HIST) __syncthreads();
-    const int64_t lb = (int64_t)blockIdx.x - sg.first_block;
-    uint32_t *wh = hist + (HIST ? (lane & (kSub - 1)) : 0);
+    const int lb = (int)blockIdx.x - sg.first_block;
+    uint32_t *pairs = hist->pair + (lane & (kSets - 1)) * kSetPitch;
     uint32_t nans = 0;
     const int64_t n8 = sg.n / 8;                                  // whole 16-byte units (x is 16-byte aligned)
-    const int64_t u0 = lb * chunk, u1 = u0 + chunk < n8 ? u0 + chunk : n8;
     const u32x4 *xv = reinterpret_cast<const u32x4 *>(sg.x);
-    int64_t u = u0 + threadIdx.x;
-    for (; u + (kUnroll - 1) * kThreads < u1; u += kUnroll * kThreads) {
-        u32x4 v[kUnroll];
+    auto nan_unit = [&](const u32x4 v) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-        for (int j = 0; j < kUnroll; j++) v[j] = __builtin_nontemporal_load(xv + u + j * kThreads);
+        for (int i = 0; i < 4; i++) nans += is_nan16(w[i] & 0xffff) + is_nan16(w[i] >> 16);
+    };
+    int64_t u = (int64_t)lb * kSweep;                             // the sweep's first unit
+    const int64_t stride = (int64_t)sg.blocks * kSweep;
+    u32x4 v[kUnroll], vn[kUnroll];
+    auto load = [&](u32x4 (&d)[kUnroll], int64_t at) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < kUnroll; j++) digest_unit<HIST, NANS>(v[j], wh, nans);
+        for (int j = 0; j < kUnroll; j++) d[j] = __builtin_nontemporal_load(xv + at + j * kThreads + threadIdx.x);
+    };
+    if (u + kSweep <= n8) load(v, u);
+    for (; u + kSweep <= n8; u += stride) {
+        load(vn, u + stride + kSweep <= n8 ? u + stride : u);     // the next sweep is on its way while this one is counted
+#pragma unroll
+        for (int j = 0; j < kUnroll; j++) {
+            if (HIST) digest_unit<NANS>(v[j], pairs, hist, nans);
+            else nan_unit(v[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < kUnroll; j++) v[j] = vn[j];
     }
-    for (; u < u1; u += kThreads) digest_unit<HIST, NANS>(xv[u], wh, nans);
+    for (u += threadIdx.x; u < n8; u += kThreads) {               // the tensor's last, incomplete sweep
+        const u32x4 t = xv[u];
+        if (HIST) digest_unit<NANS>(t, pairs, hist, nans);
+        else nan_unit(t);
+    }
     // the last n % 8 elements: one lane each of the tensor's first workgroup
     if (lb == 0 && threadIdx.x < (int)(sg.n - n8 * 8)) {
-        const uint32_t e = sg.x[n8 * 8 + threadIdx.x];
-        if (HIST) atomicAdd(&wh[abs_log2_bin(e) * kSub], 1u);
-        if (NANS) nans += is_nan16(e);
+        const uint32_t x = sg.x[n8 * 8 + threadIdx.x] & 0x7fff;
+        if (HIST) {
+            atomicAdd(&hist->expo[x >> 10], 1u);
+            if (x - 1 < 0x3ff) atomicAdd(&hist->sub[31 - __builtin_clz(x)], 1u);
+        }
+        nans += x > 0x7c00;
     }
     if (HIST) {
         __syncthreads();
-        uint32_t s = 0;
 #pragma unroll
-        for (int w = 0; w < kSub; w++) s += hist[threadIdx.x * kSub + ((w + threadIdx.x) & (kSub - 1))];   // kThreads == 256 bins
-        if (s) atomicAdd(&sg.out[threadIdx.x], (unsigned long long)s);
+        for (int k = 0; k < 1024 / kThreads; k++) {
+            const int p = threadIdx.x + k * kThreads;
+            uint32_t s = 0;
+#pragma unroll
+            for (int set = 0; set < kSets; set++) s += hist->pair[set * kSetPitch + p];
+            if (s) {
+                atomicAdd(&hist->expo[p & 31], s);
+                atomicAdd(&hist->expo[p >> 5], s);
+            }
+        }
+        __syncthreads();
+        uint32_t s = 0;
+        int bin = 0;
+        if (threadIdx.x < 32) {
+            s = hist->expo[threadIdx.x];
+            bin = threadIdx.x == 31 ? 255 : (int)threadIdx.x + 112;
+            if (threadIdx.x == 0) {
+                bin = 0;
+                for (int i = 0; i < 10; i++) s -= hist->sub[i];
+            }
+        } else if (threadIdx.x < 42) {
+            s = hist->sub[threadIdx.x - 32];
+            bin = 103 + (int)threadIdx.x - 32;
+        }
+        if (s) atomicAdd(&sg.out[bin], (unsigned long long)s);
     }
     if (NANS) {
         // wave sum of the lane counts, then one atomic per wave
@@ -141,10 +204,12 @@ int run(int64_t n, const void *x, void *out, hipStream_t st)
     hipLaunchKernelGGL(zero_i64_kernel, dim3(1), dim3(64), 0, st, (unsigned long long *)out,
                        (HIST ? 256 : 0) + (NANS ? 1 : 0));
     if (n > 0) {
-        const DigestSeg one = {(const uint16_t *)x, n, 0, (unsigned long long *)out};
-        const int chunk = chunk_for(n);
-        hipLaunchKernelGGL((digest_kernel<HIST, NANS>), dim3((unsigned)seg_blocks(n, chunk)), dim3(kThreads), 0,
-                           st, one, (const DigestSeg *)nullptr, 0, chunk);
+        DigestArgs args;
+        args.nseg = 1;
+        const int64_t blocks = seg_blocks(n, chunk_for(n));
+        CACTI_REQUIRE(blocks < (int64_t)1 << 31, CACTI_E_INVALID, "digest: tensor too large for one launch");
+        args.seg[0] = {(const uint16_t *)x, n, 0, (int32_t)blocks, (unsigned long long *)out};
+        hipLaunchKernelGGL((digest_kernel<HIST, NANS>), dim3((unsigned)blocks), dim3(kThreads), 0, st, args);
     }
     return launch_status(HIST ? "abs_log2_hist8" : "nan_count");
 }
@@ -184,36 +249,36 @@ CACTI_API int cacti_hip_digests_f16_batch(int count, const void *const *xs, cons
 {
     CACTI_REQUIRE(count >= 0, CACTI_E_INVALID, "digests_batch: negative count");
     if (count == 0) return 0;
-    CACTI_REQUIRE(xs && ns && out_i64 && scratch && aligned(out_i64, 8) && aligned(scratch, 8), CACTI_E_INVALID,
+    CACTI_REQUIRE(xs && ns && out_i64 && aligned(out_i64, 8), CACTI_E_INVALID,
                   "digests_batch: null or misaligned argument");
     return cacti::digest_batch_f16(count, xs, ns, out_i64, scratch, (hipStream_t)stream);
 }
 
 namespace cacti {
 
-// Both digests of `count` tensors in ONE launch: out[257 * i + 0..255] = histogram and
-// out[257 * i + 256] = NaN count of tensor i.  `segs_dev` is device scratch of
-// digest_batch_scratch_bytes(count) bytes (8-byte aligned); xs[i] 16-byte aligned, ns[i] >= 0.
-size_t digest_batch_scratch_bytes(int count) { return (size_t)count * sizeof(DigestSeg); }
+// Both digests of `count` tensors, up to kSegsPerLaunch of them in a launch: out[257 * i + 0..255] = histogram and
+// out[257 * i + 256] = NaN count of tensor i.  xs[i] 16-byte aligned, ns[i] >= 0.
+size_t digest_batch_scratch_bytes(int) { return 16; }           // (not used any more; callers allocate it)
 
-int digest_batch_f16(int count, const void *const *xs, const int64_t *ns, void *out, void *segs_dev,
-                     hipStream_t st)
+int digest_batch_f16(int count, const void *const *xs, const int64_t *ns, void *out, void *, hipStream_t st)
 {
     if (count <= 0) return 0;
-    std::vector<DigestSeg> segs((size_t)count);
-    int64_t blocks = 0;
-    for (int i = 0; i < count; i++) {
-        CACTI_REQUIRE(ns[i] >= 0 && (xs[i] || ns[i] == 0) && aligned(xs[i], 16), CACTI_E_INVALID,
-                      "digest_batch: tensor %d: null, negative size or not 16-byte aligned", i);
-        segs[i] = {(const uint16_t *)xs[i], ns[i], blocks, (unsigned long long *)out + (size_t)i * 257};
-        blocks += seg_blocks(ns[i], kChunk);
-    }
-    CACTI_REQUIRE(blocks < (int64_t)1 << 31, CACTI_E_INVALID, "digest_batch: too many workgroups");
-    // pageable source: the copy has left the host vector when the call returns
-    CACTI_HIP(hipMemcpyAsync(segs_dev, segs.data(), segs.size() * sizeof(DigestSeg), hipMemcpyHostToDevice, st));
+    for (int i = 0; i < count; i++)
+        CACTI_REQUIRE(ns[i] >= 0 && ns[i] < (int64_t)1 << 44 && (xs[i] || ns[i] == 0) && aligned(xs[i], 16), CACTI_E_INVALID,
+                      "digest_batch: tensor %d: null, bad size or not 16-byte aligned", i);
     hipLaunchKernelGGL(zero_i64_kernel, dim3(64), dim3(64), 0, st, (unsigned long long *)out, count * 257);
-    hipLaunchKernelGGL((digest_kernel<true, true>), dim3((unsigned)blocks), dim3(kThreads), 0, st, DigestSeg{},
-                       (const DigestSeg *)segs_dev, count, kChunk);
+    for (int i0 = 0; i0 < count; i0 += kSegsPerLaunch) {
+        DigestArgs args;
+        args.nseg = count - i0 < kSegsPerLaunch ? count - i0 : kSegsPerLaunch;
+        int64_t blocks = 0;
+        for (int i = 0; i < args.nseg; i++) {
+            const int64_t nb = seg_blocks(ns[i0 + i], kChunk);
+            CACTI_REQUIRE(blocks + nb < (int64_t)1 << 31, CACTI_E_INVALID, "digest_batch: too many workgroups");
+            args.seg[i] = {(const uint16_t *)xs[i0 + i], ns[i0 + i], (int32_t)blocks, (int32_t)nb, (unsigned long long *)out + (size_t)(i0 + i) * 257};
+            blocks += nb;
+        }
+        hipLaunchKernelGGL((digest_kernel<true, true>), dim3((unsigned)blocks), dim3(kThreads), 0, st, args);
+    }
     return launch_status("digest_batch");
 }
 

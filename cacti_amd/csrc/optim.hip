@@ -13,7 +13,6 @@
 // 16-byte access per f32 tensor), so every wave instruction covers one contiguous 512-byte or
 // 1-KiB run; non-temporal both ways since nothing is read twice.
 #include "common.h"
-#include <vector>
 
 using namespace cacti;
 
@@ -127,22 +126,28 @@ __device__ __forceinline__ void store4(float *dst, const float (&d)[4])
     __builtin_nontemporal_store(v, reinterpret_cast<f32x4 *>(dst));
 }
 
-// segs == nullptr: the one tensor `one`; otherwise nseg tensors, segs[] sorted by first_block
+// The tensors of a launch, in the kernel's arguments: a table in device memory is a copy in front of the launch.
+constexpr int kSegsPerLaunch = 64;
+struct OptArgs {
+    OptScalars sc;
+    int nseg;
+    OptSeg seg[kSegsPerLaunch];                     // by first_block
+};
+static_assert(sizeof(OptArgs) <= 4096, "kernel arguments");
+
 template <int MODE>
 __global__ void __launch_bounds__(kThreads)
-optim_kernel(OptSeg one, const OptSeg *__restrict__ segs, int nseg, OptScalars sc)
+optim_kernel(OptArgs args)
 {
     using U = Uses<MODE>;
-    OptSeg sg = one;
-    if (segs) {
-        int lo = 0, hi = nseg - 1;                            // last segment starting at or before this block
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (segs[mid].first_block <= (int64_t)blockIdx.x) lo = mid;
-            else hi = mid - 1;
-        }
-        sg = segs[lo];
+    const OptScalars sc = args.sc;
+    int seg = 0;
+    for (int hi = args.nseg - 1; seg < hi;) {                 // last segment starting at or before this block
+        const int mid = (seg + hi + 1) >> 1;
+        if (args.seg[mid].first_block <= (int64_t)blockIdx.x) seg = mid;
+        else hi = mid - 1;
     }
+    const OptSeg sg = args.seg[seg];
     const int64_t lb = (int64_t)blockIdx.x - sg.first_block;
     const int64_t n4 = sg.n / 4;
     const int64_t u0 = lb * kChunk;
@@ -210,8 +215,11 @@ int run_one(const char *what, const OptSeg &sg, const OptScalars &sc, hipStream_
     if (sg.n > 0) {
         const int64_t blocks = seg_blocks(sg.n);
         CACTI_REQUIRE(blocks < (int64_t)1 << 31, CACTI_E_INVALID, "%s: tensor too large for one launch", what);
-        hipLaunchKernelGGL((optim_kernel<MODE>), dim3((unsigned)blocks), dim3(kThreads), 0, st, sg,
-                           (const OptSeg *)nullptr, 0, sc);
+        OptArgs args;
+        args.sc = sc;
+        args.nseg = 1;
+        args.seg[0] = sg;
+        hipLaunchKernelGGL((optim_kernel<MODE>), dim3((unsigned)blocks), dim3(kThreads), 0, st, args);
     }
     return launch_status(what);
 }
@@ -306,7 +314,7 @@ CACTI_API int cacti_adamw32_scalars(int iter_nr, float grad_scale, float lr, flo
     return 0;
 }
 
-CACTI_API size_t cacti_hip_adamw32_scratch_bytes(int count) { return count > 0 ? (size_t)count * sizeof(OptSeg) : 0; }
+CACTI_API size_t cacti_hip_adamw32_scratch_bytes(int count) { return count > 0 ? 16 : 0; }   // (not used any more)
 
 CACTI_API int cacti_hip_adamw32_step_f16_batch(int count, const void *const *grads_f16, void *const *avgs_f32,
                                                void *const *avg2s_f32, void *const *masters_f32,
@@ -315,11 +323,8 @@ CACTI_API int cacti_hip_adamw32_step_f16_batch(int count, const void *const *gra
 {
     CACTI_REQUIRE(count >= 0, CACTI_E_INVALID, "adamw32_step: negative count");
     if (count == 0) return 0;
-    CACTI_REQUIRE(grads_f16 && avgs_f32 && avg2s_f32 && masters_f32 && params_f16 && ns && scalars7 && scratch &&
-                      aligned(scratch, 8),
-                  CACTI_E_INVALID, "adamw32_step: null or misaligned argument");
-    std::vector<OptSeg> segs((size_t)count);
-    int64_t blocks = 0;
+    CACTI_REQUIRE(grads_f16 && avgs_f32 && avg2s_f32 && masters_f32 && params_f16 && ns && scalars7,
+                  CACTI_E_INVALID, "adamw32_step: null argument");
     for (int i = 0; i < count; i++) {
         CACTI_REQUIRE(ns[i] >= 0, CACTI_E_INVALID, "adamw32_step: tensor %d has a negative size", i);
         CACTI_REQUIRE(ns[i] == 0 || (grads_f16[i] && avgs_f32[i] && avg2s_f32[i] && masters_f32[i] && params_f16[i]),
@@ -327,17 +332,20 @@ CACTI_API int cacti_hip_adamw32_step_f16_batch(int count, const void *const *gra
         CACTI_REQUIRE(aligned(grads_f16[i], 16) && aligned(avgs_f32[i], 16) && aligned(avg2s_f32[i], 16) &&
                           aligned(masters_f32[i], 16) && aligned(params_f16[i], 16),
                       CACTI_E_INVALID, "adamw32_step: tensor %d is not 16-byte aligned", i);
-        segs[i] = {(const uint16_t *)grads_f16[i], (float *)avgs_f32[i], (float *)avg2s_f32[i],
-                   (float *)masters_f32[i], (uint16_t *)params_f16[i], ns[i], blocks};
-        blocks += seg_blocks(ns[i]);
     }
-    CACTI_REQUIRE(blocks < (int64_t)1 << 31, CACTI_E_INVALID, "adamw32_step: too many workgroups");
-    hipStream_t st = (hipStream_t)stream;
-    // pageable source: the copy has left the host vector when the call returns
-    CACTI_HIP(hipMemcpyAsync(scratch, segs.data(), segs.size() * sizeof(OptSeg), hipMemcpyHostToDevice, st));
-    OptScalars sc;
-    for (int k = 0; k < 7; k++) sc.s[k] = scalars7[k];
-    hipLaunchKernelGGL((optim_kernel<M_STEP>), dim3((unsigned)blocks), dim3(kThreads), 0, st, OptSeg{},
-                       (const OptSeg *)scratch, count, sc);
+    OptArgs args;
+    for (int k = 0; k < 7; k++) args.sc.s[k] = scalars7[k];
+    for (int i0 = 0; i0 < count; i0 += kSegsPerLaunch) {
+        args.nseg = count - i0 < kSegsPerLaunch ? count - i0 : kSegsPerLaunch;
+        int64_t blocks = 0;
+        for (int k = 0; k < args.nseg; k++) {
+            const int i = i0 + k;
+            args.seg[k] = {(const uint16_t *)grads_f16[i], (float *)avgs_f32[i], (float *)avg2s_f32[i],
+                           (float *)masters_f32[i], (uint16_t *)params_f16[i], ns[i], blocks};
+            blocks += seg_blocks(ns[i]);
+        }
+        CACTI_REQUIRE(blocks < (int64_t)1 << 31, CACTI_E_INVALID, "adamw32_step: too many workgroups");
+        hipLaunchKernelGGL((optim_kernel<M_STEP>), dim3((unsigned)blocks), dim3(kThreads), 0, (hipStream_t)stream, args);
+    }
     return launch_status("adamw32_step");
 }
