@@ -28,7 +28,7 @@ struct cacti_llama {
     std::vector<CellPtr> params, grads;
     bool grads_written = false;                                 // a gradient cycle has been staged
     int attention_mode = 0;                                     // 0 fused thunk, 1 the chain of separate thunks
-    int group_products = 1;                                     // 0 none, 1 up + gate forward, 2 also q, k, v and the weight gradients
+    int group_products = 2;                                     // 0 none, 1 up + gate forward, 2 also q, k, v and the weight gradients
     std::vector<CellPtr> master, grad_avg, grad2_avg;           // f32 optimiser state (adamw_init)
     std::vector<std::string> names;
     CellPtr embed, head_norm, lm_head;
