@@ -24,8 +24,9 @@ struct Staging {
 // n <= kMaxRegions regions, in one launch on `st`, to places in s.data(); returns when they are there.  The launch comes
 // behind all work queued on `st`, so this waits for it like a stream synchronisation.
 int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st);
-// one region of any size to pageable memory, likewise
-int read_large(void *dst, const void *src, size_t bytes, hipStream_t st);
+// one region of any size to pageable memory, likewise, and (not null) a word of device memory with it
+int read_large(void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st);
+constexpr size_t kLargeRead = 512u << 10;      // from here on it is the better one
 // n regions of `bytes` (a multiple of 16), 16-byte aligned, set to zero
 int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st);
 

@@ -2,9 +2,9 @@
 //
 // A read-back of a few KB costs its round trips, not its bytes: hipMemcpyAsync into pageable memory is staged by the
 // runtime and a stream synchronisation takes some 15 us to notice that the stream is empty.  Here one kernel writes the
-// regions straight into page-locked host memory, each workgroup followed by a word that says its part is there, and the
-// host polls those words.  A large read is the same in pieces, several of them on the link while the host's threads copy
-// earlier ones to their place (the runtime's copy to pageable memory: 16 GB/s).
+// regions straight into page-locked host memory in chunks, each followed by a word that says it is there, and the host
+// polls those words.  Of a large read the host copies the chunks that have arrived to their place while the others are on
+// the link (the runtime's copy to pageable memory: 16 GB/s).
 #include <emmintrin.h>
 #include <string.h>
 
@@ -22,7 +22,7 @@ namespace cacti {
 
 namespace {
 
-constexpr int kGatherBlocks = 64;              // workgroups per region at most: 4 KB and more each
+constexpr int kGatherBlocks = 64;              // chunks per region of a small read at most: 4 KB and more each
 constexpr int kFlagsPerGather = kGatherBlocks * kMaxRegions;
 static_assert(kFlagsPerGather * sizeof(unsigned) <= Staging::kFlagBytes, "a word per workgroup");
 
@@ -34,14 +34,32 @@ struct GatherArgs {
     unsigned epoch;
 };
 
+__device__ __forceinline__ void chunk_arrived(unsigned *flag, unsigned epoch)
+{
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ void __launch_bounds__(256) gather_kernel(GatherArgs p)
 {
     const int z = blockIdx.y;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < p.n16[z]; i += (int64_t)gridDim.x * 256) p.dst[z][i] = p.src[z][i];
-    __threadfence_system();
-    __syncthreads();
-    if (threadIdx.x == 0)
-        __hip_atomic_store(p.flags + z * gridDim.x + blockIdx.x, p.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    chunk_arrived(p.flags + z * gridDim.x + blockIdx.x, p.epoch);
+}
+
+// One large region.  The link is full with a few workgroups (16: 52 GB/s); more of them would only make the chunks
+// arrive all together at the end, and the host wants them one after another.
+__global__ void __launch_bounds__(256)
+stream_kernel(const uint4 *src, uint4 *dst, int64_t n16, int64_t chunk16, const int *word, int *word_dst, unsigned *flags, unsigned epoch)
+{
+    const int64_t chunks = (n16 + chunk16 - 1) / chunk16;
+    for (int64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+        if (word && c == 0 && threadIdx.x == 0) *word_dst = *word;
+        const int64_t end = min((c + 1) * chunk16, n16);
+        for (int64_t i = c * chunk16 + threadIdx.x; i < end; i += 256) dst[i] = src[i];
+        chunk_arrived(flags + c, epoch);
+    }
 }
 
 struct ZeroArgs {
@@ -94,9 +112,9 @@ int wait_flags(const unsigned *flags, int n, unsigned epoch, hipStream_t st)
 std::mutex g_mutex;
 std::vector<Staging> g_free;                   // staging buffers of contexts that are gone, for the next ones
 
-// large reads, one at a time: page-locked memory for kPieces pieces
-constexpr size_t kPiece = 1u << 20;
-constexpr int kPieces = 16, kReadThreads = 4;
+// large reads, one at a time: page-locked memory for a window of chunks
+constexpr size_t kWindow = 16u << 20, kLeastChunk = 32u << 10, kLargeFlagBytes = kWindow / kLeastChunk * sizeof(unsigned) + 64;
+constexpr int kStreamBlocks = 16, kReadThreads = 4;
 std::mutex g_large_mutex;
 char *g_large = nullptr;
 unsigned g_large_epoch = 0;
@@ -113,48 +131,50 @@ int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st)
     return rc ? rc : wait_flags(flags, nflags, s.epoch, st);
 }
 
-int read_large(void *dst, const void *src, size_t bytes, hipStream_t st)
+// Measured, us, one gather and one copy behind it / 1 MiB pieces before -> chunks: 2 MiB 119 -> 76, 20 MiB 569 -> 473.  A
+// helper thread costs some 10 us to start: worth it from several MiB on, where the copying host (12 .. 30 GB/s) and not
+// the link (52) is what one thread would wait for.  Below 512 KiB chunks bring nothing (32 us at 512 KiB either way).
+int read_large(void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st)
 {
     std::lock_guard<std::mutex> lock(g_large_mutex);
-    constexpr size_t flag_bytes = (size_t)kPieces * kGatherBlocks * sizeof(unsigned);
     if (!g_large) {
         void *p = nullptr;
-        if (hipHostMalloc(&p, flag_bytes + kPieces * kPiece, hipHostMallocPortable) != hipSuccess) {
+        if (hipHostMalloc(&p, kLargeFlagBytes + kWindow, hipHostMallocPortable) != hipSuccess) {
             (void)hipGetLastError();
             CACTI_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+            if (word) CACTI_HIP(hipMemcpyAsync(word_dst, word, sizeof(int), hipMemcpyDeviceToHost, st));
             CACTI_HIP(hipStreamSynchronize(st));
             return 0;
         }
         g_large = static_cast<char *>(p);
-        memset(g_large, 0, flag_bytes);
+        memset(g_large, 0, kLargeFlagBytes);
     }
-    unsigned *const flags = reinterpret_cast<unsigned *>(g_large);
-    char *const data = g_large + flag_bytes;
+    int *const word_here = reinterpret_cast<int *>(g_large);       // 64 bytes for it, then the flags, then the data
+    unsigned *const flags = reinterpret_cast<unsigned *>(g_large + 64);
+    char *const data = g_large + kLargeFlagBytes;
     int dev = 0;
     CACTI_HIP(hipGetDevice(&dev));
-    for (size_t done = 0; done < bytes;) {                        // windows of kPieces pieces
-        const size_t window = std::min(bytes - done, kPieces * kPiece);
-        const int pieces = (int)((window + kPiece - 1) / kPiece);
+    for (size_t done = 0; done < bytes;) {
+        const size_t window = std::min(bytes - done, kWindow), chunk = window < (4u << 20) ? kLeastChunk : 2 * kLeastChunk;
+        const int chunks = (int)((window + chunk - 1) / chunk), threads = (int)std::min<size_t>(kReadThreads, 1 + window / (4u << 20));
         if (++g_large_epoch == 0) g_large_epoch = 1;
         const unsigned epoch = g_large_epoch;
-        int nflags[kPieces];
-        for (int i = 0; i < pieces; i++) {
-            const HostRegion r = {static_cast<const char *>(src) + done + (size_t)i * kPiece, data + (size_t)i * kPiece,
-                                  std::min(kPiece, window - (size_t)i * kPiece)};
-            const int rc = launch_gather(&r, 1, flags + i * kGatherBlocks, epoch, &nflags[i], st);
-            if (rc) return rc;
-        }
+        hipLaunchKernelGGL(stream_kernel, dim3((unsigned)std::min(chunks, kStreamBlocks)), dim3(256), 0, st,
+                           reinterpret_cast<const uint4 *>(static_cast<const char *>(src) + done), reinterpret_cast<uint4 *>(data),
+                           (int64_t)((window + 15) / 16), (int64_t)(chunk / 16), word, word_here, flags, epoch);
+        const int rc = launch_status("read_large");
+        if (rc) return rc;
         std::atomic<int> next{0}, failed{0};
         auto work = [&]() {
-            for (int i; !failed.load() && (i = next.fetch_add(1)) < pieces;) {
-                const int rc = wait_flags(flags + i * kGatherBlocks, nflags[i], epoch, st);
+            for (int i; !failed.load() && (i = next.fetch_add(1)) < chunks;) {
+                const int rc = wait_flags(flags + i, 1, epoch, st);
                 if (rc) failed.store(rc);
-                else memcpy(static_cast<char *>(dst) + done + (size_t)i * kPiece, data + (size_t)i * kPiece,
-                            std::min(kPiece, window - (size_t)i * kPiece));
+                else memcpy(static_cast<char *>(dst) + done + (size_t)i * chunk, data + (size_t)i * chunk,
+                            std::min(chunk, window - (size_t)i * chunk));
             }
         };
         std::vector<std::thread> th;
-        for (int t = 1; t < std::min(kReadThreads, pieces); t++)
+        for (int t = 1; t < threads; t++)
             th.emplace_back([&]() {
                 (void)hipSetDevice(dev);
                 work();
@@ -164,6 +184,7 @@ int read_large(void *dst, const void *src, size_t bytes, hipStream_t st)
         if (failed.load()) return failed.load();
         done += window;
     }
+    if (word) *word_dst = *word_here;
     return 0;
 }
 

@@ -245,26 +245,28 @@ int Ctx::fetch(const Fetch *f, int n)
     int m = 0;
     size_t used = 256;                         // behind the status word's place
     const bool stage = staging_.base != nullptr;
+    bool have_status = false;
     if (stage) r[m++] = {status_ptr(), staging_.data(), sizeof(int)};
-    else CACTI_HIP(hipMemcpyAsync(&status, status_ptr(), sizeof(int), hipMemcpyDeviceToHost, stream_));
     for (int i = 0; i < n; i++) {
         bytes_d2h_ += f[i].bytes;
         const size_t room = (f[i].bytes + 255) / 256 * 256;
-        if (stage && m < kMaxRegions && used + room <= staging_.room()) {
+        if (stage && m < kMaxRegions && f[i].bytes <= kLargeRead && used + room <= staging_.room()) {
             staged[m] = &f[i];
             r[m++] = {f[i].src, staging_.data() + used, f[i].bytes};
             used += room;
         } else {
-            const int rc = read_large(f[i].dst, f[i].src, f[i].bytes, stream_);
+            const int rc = read_large(f[i].dst, f[i].src, f[i].bytes, static_cast<int *>(status_ptr()), &status, stream_);
             if (rc) return rc;
+            have_status = true;
         }
     }
-    if (stage) {
+    if (stage && (m > 1 || !have_status)) {
         const int rc = gather_to_host(staging_, r, m, stream_);
         if (rc) return rc;
         memcpy(&status, staging_.data(), sizeof(int));
         for (int i = 1; i < m; i++) memcpy(staged[i]->dst, r[i].dst, staged[i]->bytes);
-    } else {
+    } else if (!have_status) {
+        CACTI_HIP(hipMemcpyAsync(&status, status_ptr(), sizeof(int), hipMemcpyDeviceToHost, stream_));
         CACTI_HIP(hipStreamSynchronize(stream_));
     }
     if (status) {
@@ -389,12 +391,12 @@ int Ctx::cell_get(CellPtr ci, void *host, size_t bytes)
             c.v_ready = nullptr;
         }
         int rc;
-        if (staging_.base && bytes <= staging_.room()) {
+        if (staging_.base && bytes <= kLargeRead) {
             const HostRegion r = {dev_ptr(c.voff), staging_.data(), bytes};
             rc = gather_to_host(staging_, &r, 1, stream_);
             if (!rc) memcpy(host, staging_.data(), bytes);
         } else {
-            rc = read_large(host, dev_ptr(c.voff), bytes, stream_);
+            rc = read_large(host, dev_ptr(c.voff), bytes, nullptr, nullptr, stream_);
         }
         if (rc) return rc;
         bytes_d2h_ += bytes;
