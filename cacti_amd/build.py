@@ -47,9 +47,16 @@ def build(jobs=4):
         objs = list(ex.map(_compile, sources()))
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs
     subprocess.check_call(cmd)
-    subprocess.check_call(["g++", "-O2", "-shared", "-fPIC", "-std=c++17", "-Wall", "-I" + sysconfig.get_paths()["include"],
-                           os.path.join(HERE, "pysrc", "fast.cpp"), "-o", FAST, "-L" + OUT_DIR, "-l:" + os.path.basename(LIB),
-                           "-Wl,-rpath,$ORIGIN"])
+    import torch
+    from torch.utils import cpp_extension
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    subprocess.check_call(
+        ["g++", "-O2", "-shared", "-fPIC", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+         "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I" + sysconfig.get_paths()["include"]] +
+        [f for d in cpp_extension.include_paths() + [os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")]
+         for f in ("-isystem", d)] +
+        [os.path.join(HERE, "pysrc", "fast.cpp"), "-o", FAST, "-L" + OUT_DIR, "-l:" + os.path.basename(LIB), "-L" + torch_lib,
+         "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python", "-Wl,-rpath,$ORIGIN"])
     return LIB
 
 

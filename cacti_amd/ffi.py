@@ -217,16 +217,19 @@ _fast = None
 
 
 def fast():
-    """The operator entry points as CPython functions (pysrc/fast.cpp), built beside the library."""
+    """The operators as CPython functions (pysrc/fast.cpp), built beside the library."""
     global _fast
     if _fast is None:
+        import torch                             # noqa: F401 (whose libraries the module is linked to)
         lib()                                    # the same library, by its path
         path = os.path.join(os.path.dirname(LIB_PATH), "_fast.so")
         if not os.path.exists(path):
             raise RuntimeError("%s is missing: build it with `python -m cacti_amd.build`" % path)
         loader = importlib.machinery.ExtensionFileLoader("_fast", path)
-        _fast = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fast", loader))
-        loader.exec_module(_fast)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fast", loader))
+        loader.exec_module(module)
+        module.set_check(check)
+        _fast = module
     return _fast
 
 

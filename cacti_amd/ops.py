@@ -5,8 +5,6 @@ given) in the reference's terms (src/thunk/mod.rs:347-351), executed by the HIP 
 behind the C ABI.  torch is used only to own device memory and name the stream; every
 computation goes through libcacti_gpu_hip_ffi.so and fails if it is not built.
 """
-import ctypes
-
 import torch
 
 from . import ffi
@@ -14,9 +12,9 @@ from . import ffi
 F16 = torch.float16
 F32 = torch.float32
 
-# A small operator is host work: 8 us of it in Python against some 3 us on the device.  So the entry points are called as
-# CPython functions (ffi.fast), the stream is read without building a torch.cuda.Stream (2.7 us), and each operator
-# checks its tensors in one expression.
+# A small operator is host work (8 us of it in Python against some 3 us on the device), so the operators of the model's path
+# are CPython functions that take the tensors themselves (ffi.fast, pysrc/fast.cpp); the others reach the C ABI through it
+# with pointers and a stream that is read without building a torch.cuda.Stream (2.7 us).
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _current_device = getattr(torch._C, "_cuda_getDevice", None)
 
@@ -40,11 +38,17 @@ class _Calls:
         return call
 
 
+class _Operators:
+    """The operators of pysrc/fast.cpp."""
+
+    def __getattr__(self, name):
+        f = getattr(ffi.fast(), name)
+        setattr(self, name, f)
+        return f
+
+
 _do = _Calls()
-
-
-def _size(name, *args):
-    return getattr(ffi.fast(), name)(*args)
+_op = _Operators()
 
 
 def _p(t):
@@ -65,50 +69,16 @@ def selftest_wave_reduce():
 # ---------------------------------------------------------------- GEMM
 def gemm(a, b, ta=False, tb=False, alpha=1.0, beta=0.0, out=None):
     """out = f16(alpha op(a) op(b) + beta out); a, b 2-d row-major f16 (rows may be strided)."""
-    (ra, ca), (rb, cb) = a.shape, b.shape
-    assert a.stride(1) == 1 and b.stride(1) == 1
-    M, K = (ca, ra) if ta else (ra, ca)
-    K2, N = (cb, rb) if tb else (rb, cb)
-    assert K == K2, (a.shape, b.shape, ta, tb)
-    if out is None:
-        assert beta == 0.0
-        out = torch.empty((M, N), dtype=F16, device=a.device)
-    else:
-        assert out.shape == (M, N) and out.stride(1) == 1
-    _gemm(ta, tb, M, N, K, alpha, a, b, beta, out)
-    return out
-
-
-def _gemm(ta, tb, M, N, K, alpha, a, b, beta, out):
-    f = ffi.fast().gemm_f16_ws
-    args = (ta, tb, M, N, K, alpha, a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), beta, out.data_ptr(), out.stride(0))
-    st = _stream()
-    need = f(*args, None, 0, st)
-    if need > 0:                                 # not launched: the product wants a workspace
-        ws = torch.empty(need, dtype=torch.uint8, device=a.device)
-        need = f(*args, ws.data_ptr(), need, st)
-    if need < 0:
-        ffi.check(-1000000 - need)
+    return _op.gemm(a, b, ta, tb, alpha, beta, out)
 
 
 def gemm_batched(As, Bs, ta=False, tb=False, alpha=1.0, beta=0.0, outs=None):
     """Pointer-array batch: outs[z] = f16(alpha op(As[z]) op(Bs[z]) + beta outs[z]), one shape."""
-    C = ctypes
-    n = len(As)
-    a, b = As[0], Bs[0]
-    M, K = (a.shape[1], a.shape[0]) if ta else a.shape
-    N = b.shape[0] if tb else b.shape[1]
     if outs is None:
         assert beta == 0.0
-        outs = [torch.empty((M, N), dtype=F16, device=a.device) for _ in range(n)]
-    if any(x % 8 for x in (a.shape[1], b.shape[1], N, a.stride(0), b.stride(0), outs[0].stride(0))):
-        # rows that are not 16-byte aligned run one after another; each may want a workspace
-        for x, y, z in zip(As, Bs, outs):
-            _gemm(ta, tb, M, N, K, alpha, x, y, beta, z)
-        return outs
-    arr = lambda ts: C.cast((C.c_void_p * n)(*[t.data_ptr() for t in ts]), C.c_void_p)
-    ffi.call("cacti_hip_gemm_f16_batched", int(ta), int(tb), n, M, N, K, alpha, arr(As), a.stride(0), arr(Bs),
-             b.stride(0), beta, arr(outs), outs[0].stride(0), _stream())
+        shape = (As[0].shape[1 if ta else 0], Bs[0].shape[0 if tb else 1])
+        outs = [torch.empty(shape, dtype=F16, device=As[0].device) for _ in As]
+    _op.gemm_batched(As, Bs, outs, ta, tb, alpha, beta)
     return outs
 
 
@@ -142,65 +112,28 @@ def block_matmul_pv(p16, v, causal=False):
 
 def attention_fwd(q, k, v, alpha):
     """Fused causal attention on [S,H,Dh] tensors: returns (o, stats); stats feeds attention_bwd."""
-    _chk(q), _chk(k), _chk(v)
-    S, H, Dh = q.shape
-    o = torch.empty_like(q)
-    stats = torch.empty(_size("attention_stats_bytes", S, H) // 4, dtype=torch.float32, device=q.device)
-    _do.attention_fwd(S, H, Dh, alpha, q.data_ptr(), k.data_ptr(), v.data_ptr(), H * Dh,
-             o.data_ptr(), stats.data_ptr(), _stream())
-    return o, stats
+    return _op.attention_fwd(q, k, v, alpha)
 
 
 def attention_bwd(q, k, v, dO, stats, alpha, acc=None, o=None):
     """Adjoint of attention_fwd: returns (dq, dk, dv); acc = (dq, dk, dv) to accumulate into; o = the forward
     output (lets blocks of queries with spread probabilities skip the pass that forms the row sums)."""
-    _chk(q), _chk(k), _chk(v), _chk(dO)
-    if o is not None:
-        _chk(o)
-    S, H, Dh = q.shape
-    dq, dk, dv = acc if acc is not None else (torch.empty_like(q), torch.empty_like(q), torch.empty_like(q))
-    a = int(acc is not None)
-    nbytes = _size("attention_bwd_workspace", S, H)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-    _do.attention_bwd(S, H, Dh, alpha, q.data_ptr(), k.data_ptr(), v.data_ptr(),
-             _p(o), dO.data_ptr(), H * Dh, stats.data_ptr(), dq.data_ptr(), a,
-             dk.data_ptr(), a, dv.data_ptr(), a,
-             ws.data_ptr(), nbytes, _stream())
-    return dq, dk, dv
+    return _op.attention_bwd(q, k, v, dO, stats, alpha, acc, o)
 
 
 # ---------------------------------------------------------------- fused thunks
 def rms_norm_fwd(x, w, eps):
-    _chk(x), _chk(w)
-    N, D = x.shape
-    y = torch.empty_like(x)
-    _do.rms_norm_fwd(N, D, x.data_ptr(), w.data_ptr(), eps, y.data_ptr(),
-             _stream())
-    return y
+    return _op.rms_norm_fwd(x, w, eps)
 
 
 def add_rms_norm_fwd(a, b, w, eps):
     """(f16(a + b), rms_norm of it): the residual add and the norm that follows, one launch."""
-    _chk(a), _chk(b), _chk(w)
-    N, D = a.shape
-    s, y = torch.empty_like(a), torch.empty_like(a)
-    _do.add_rms_norm_fwd(N, D, a.data_ptr(), b.data_ptr(), w.data_ptr(), eps,
-             s.data_ptr(), y.data_ptr(), _stream())
-    return s, y
+    return _op.add_rms_norm_fwd(a, b, w, eps)
 
 
 def rms_norm_bwd(x, w, eps, dy, dx_acc=None, dw_acc=None):
     """Returns (dx, dw).  dx_acc / dw_acc: tensors to accumulate into (updated in place)."""
-    _chk(x), _chk(w), _chk(dy)
-    N, D = x.shape
-    dx = torch.empty_like(x) if dx_acc is None else _chk(dx_acc)
-    dw = torch.empty_like(w) if dw_acc is None else _chk(dw_acc)
-    nbytes = _size("rms_norm_bwd_workspace", N, D)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    _do.rms_norm_bwd(N, D, x.data_ptr(), w.data_ptr(), eps, dy.data_ptr(),
-             dx.data_ptr(), int(dx_acc is not None), dw.data_ptr(), int(dw_acc is not None),
-             ws.data_ptr(), nbytes, _stream())
-    return dx, dw
+    return _op.rms_norm_bwd(x, w, eps, dy, dx_acc, dw_acc)
 
 
 def rope_tables(S, Dh, device="cuda"):
@@ -211,39 +144,19 @@ def rope_tables(S, Dh, device="cuda"):
 
 
 def rope_fwd(x, cos, sin):
-    _chk(x), _chk(cos), _chk(sin)
-    S, H, Dh = x.shape
-    y = torch.empty_like(x)
-    _do.rope_fwd(S, H, Dh, x.data_ptr(), cos.data_ptr(), sin.data_ptr(),
-             y.data_ptr(), _stream())
-    return y
+    return _op.rope_fwd(x, cos, sin)
 
 
 def rope_bwd(dy, cos, sin, dx_acc=None):
-    _chk(dy), _chk(cos), _chk(sin)
-    S, H, Dh = dy.shape
-    dx = torch.empty_like(dy) if dx_acc is None else _chk(dx_acc)
-    _do.rope_bwd(S, H, Dh, dy.data_ptr(), cos.data_ptr(), sin.data_ptr(),
-             dx.data_ptr(), int(dx_acc is not None), _stream())
-    return dx
+    return _op.rope_bwd(dy, cos, sin, dx_acc)
 
 
 def silu_gate_fwd(g, u):
-    _chk(g), _chk(u)
-    h = torch.empty_like(g)
-    _do.silu_gate_fwd(g.numel(), g.data_ptr(), u.data_ptr(), h.data_ptr(),
-             _stream())
-    return h
+    return _op.silu_gate_fwd(g, u)
 
 
 def silu_gate_bwd(g, u, dh, dg_acc=None, du_acc=None):
-    _chk(g), _chk(u), _chk(dh)
-    dg = torch.empty_like(g) if dg_acc is None else _chk(dg_acc)
-    du = torch.empty_like(g) if du_acc is None else _chk(du_acc)
-    _do.silu_gate_bwd(g.numel(), g.data_ptr(), u.data_ptr(), dh.data_ptr(),
-             dg.data_ptr(), int(dg_acc is not None), du.data_ptr(), int(du_acc is not None),
-             _stream())
-    return dg, du
+    return _op.silu_gate_bwd(g, u, dh, dg_acc, du_acc)
 
 
 def causal_softmax_fwd(s16):
@@ -289,12 +202,7 @@ def softmax_ce_fwd(logit, tok, want_prob=True):
 
 
 def softmax_ce_bwd(logit, tok, scale, acc=None):
-    _chk(logit), _chk(scale, torch.float32)
-    N, V = logit.shape
-    d = torch.empty_like(logit) if acc is None else _chk(acc)
-    _do.softmax_ce_bwd(N, V, logit.data_ptr(), tok.data_ptr(), scale.data_ptr(),
-             d.data_ptr(), int(acc is not None), _stream())
-    return d
+    return _op.softmax_ce_bwd(logit, tok, scale, acc)
 
 
 def embed_fwd(W, tok):
@@ -319,9 +227,7 @@ def embed_bwd(V, tok, dy, acc=None):
 
 
 def add_f16(a, b, out=None):
-    out = torch.empty_like(a) if out is None else out
-    _do.add_f16(a.numel(), a.data_ptr(), b.data_ptr(), out.data_ptr(), _stream())
-    return out
+    return _op.add_f16(a, b, out)
 
 
 def accumulate_1d(dst, src):
@@ -351,20 +257,10 @@ def abs_log2_hist8(x):
 def digests(xs):
     """Both digests of a list of f16 tensors in one launch: (hist int64[n,256], nan int64[n])
     (the per-cycle loop of examples/open_llama_3b_train.rs:409-424)."""
-    import ctypes as C
-    n = len(xs)
-    for x in xs:
-        _chk(x)
-    dev = xs[0].device if n else torch.device("cuda")
-    out = torch.empty((n, 257), dtype=torch.int64, device=dev)
-    if n == 0:
+    if len(xs) == 0:
+        out = torch.empty((0, 257), dtype=torch.int64, device="cuda")
         return out[:, :256], out[:, 256]
-    scratch = torch.empty(_size("digests_scratch_bytes", n), dtype=torch.uint8, device=dev)
-    ptrs = (C.c_void_p * n)(*[x.data_ptr() for x in xs])
-    ns = (C.c_int64 * n)(*[x.numel() for x in xs])
-    ffi.call("cacti_hip_digests_f16_batch", n, C.cast(ptrs, C.c_void_p), C.cast(ns, C.c_void_p),
-             out.data_ptr(), scratch.data_ptr(), _stream())
-    return out[:, :256], out[:, 256]
+    return _op.digests(xs)
 
 
 # ---------------------------------------------------------------- optimiser thunks (AdamW32)
@@ -417,29 +313,13 @@ def cast_f16_f32(x):
 def adamw32_scalars(iter_nr, grad_scale, lr, wd, a1, a2, eps):
     """The seven f32 scalars of one AdamW32 step (host arithmetic of src/librarium/adamw.rs:45-60 and
     src/op.rs:984-1023) as a list; raises for iter_nr <= 0."""
-    import ctypes as C
-    out = (C.c_float * 7)()
-    ffi.call("cacti_adamw32_scalars", int(iter_nr), grad_scale or 0.0, lr, wd, a1, a2, eps, C.cast(out, C.c_void_p))
-    return list(out)
+    return _op.adamw32_scalars(int(iter_nr), grad_scale or 0.0, lr, wd, a1, a2, eps)
 
 
 def adamw32_step_(grads, avgs, avg2s, masters, params, scalars):
     """One AdamW32 step of a list of tensors in one launch, in place (avgs, avg2s, masters updated,
     params overwritten with f16(master))."""
-    import ctypes as C
-    n = len(grads)
-    assert len(avgs) == len(avg2s) == len(masters) == len(params) == n
-    if n == 0:
-        return
-    for g, a, b, w, p in zip(grads, avgs, avg2s, masters, params):
-        _chk(g), _f(a), _f(b), _f(w), _chk(p)
-        assert g.numel() == a.numel() == b.numel() == w.numel() == p.numel()
-    arr = lambda ts: C.cast((C.c_void_p * n)(*[t.data_ptr() for t in ts]), C.c_void_p)
-    ns = (C.c_int64 * n)(*[g.numel() for g in grads])
-    sc = (C.c_float * 7)(*scalars)
-    scratch = torch.empty(_size("adamw32_scratch_bytes", n), dtype=torch.uint8, device=grads[0].device)
-    ffi.call("cacti_hip_adamw32_step_f16_batch", n, arr(grads), arr(avgs), arr(avg2s), arr(masters), arr(params),
-             C.cast(ns, C.c_void_p), C.cast(sc, C.c_void_p), scratch.data_ptr(), _stream())
+    _op.adamw32_step(grads, avgs, avg2s, masters, params, scalars)
 
 
 # ---------------------------------------------------------------- bf16 raw casts (src/thunk/op.rs:665-803)
