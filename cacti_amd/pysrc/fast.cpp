@@ -2,7 +2,7 @@
 // over the C ABI some 2 were the launch (which the device needs as well, 2.3 us from one small kernel to the next); the
 // rest went into allocating the results (torch.empty: 1.5 us each from Python, a third of it here), a Python call for
 // every property of a tensor that is looked at, and the conversion of arguments.  us per call from Python, before ->
-// here: gemm 6.3 -> @g, rms_norm 4.8 -> @r, its adjoint 10.6 -> @b, silu_gate 4.8 -> @s.
+// here: gemm 6.3 -> 4.0, rms_norm 4.8 -> 3.7, its adjoint (two kernels) 10.6 -> 8.0, silu_gate 4.8 -> 3.7.
 //
 // Tensors come as torch hands them over; what an operator wants of them is checked as before (AssertionError), a status of
 // the C ABI that is not 0 is raised by ffi.check.  The other entry points (FN) take pointers as integers or None and
@@ -124,14 +124,17 @@ int truth(PyObject *o)
     return v;
 }
 
-// the call itself runs without the interpreter lock; a status that is not 0 becomes the exception ffi.check raises
+// the call itself runs without the interpreter lock (taken again also where it throws: a tensor without storage does); a
+// status that is not 0 becomes the exception ffi.check raises
+struct Unlocked {
+    PyThreadState *st = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(st); }
+};
 template <class F>
 auto unlocked(F f)
 {
-    PyThreadState *st = PyEval_SaveThread();
-    const auto r = f();
-    PyEval_RestoreThread(st);
-    return r;
+    const Unlocked u;
+    return f();
 }
 void raise_status(int rc)
 {
@@ -179,12 +182,12 @@ PyObject *take2(const Result &a, const Result &b)
     return r;
 }
 
-// the tensors of a list or tuple
+// The tensors of a list or tuple, held: another thread may change the list while a call runs without the interpreter lock.
 struct Tensors {
-    PyObject *seq;
-    std::vector<const at::Tensor *> t;
-    explicit Tensors(PyObject *o) : seq(PySequence_Fast(o, "a sequence of tensors expected"))
+    std::vector<at::Tensor> t;
+    explicit Tensors(PyObject *o)
     {
+        PyObject *seq = PySequence_Fast(o, "a sequence of tensors expected");
         if (!seq) throw PyFailed();
         const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
         t.reserve(n);
@@ -194,17 +197,16 @@ struct Tensors {
                 Py_DECREF(seq);
                 fail(PyExc_TypeError, "a tensor expected");
             }
-            t.push_back(&THPVariable_Unpack(e));
+            t.push_back(THPVariable_Unpack(e));
         }
+        Py_DECREF(seq);
     }
-    Tensors(const Tensors &) = delete;
-    ~Tensors() { Py_DECREF(seq); }
     size_t size() const { return t.size(); }
-    const at::Tensor &operator[](size_t i) const { return *t[i]; }
+    const at::Tensor &operator[](size_t i) const { return t[i]; }
     std::vector<void *> pointers() const
     {
         std::vector<void *> p(t.size());
-        for (size_t i = 0; i < t.size(); i++) p[i] = t[i]->data_ptr();
+        for (size_t i = 0; i < t.size(); i++) p[i] = t[i].data_ptr();
         return p;
     }
 };
@@ -304,31 +306,23 @@ PyObject *attention_bwd(PyObject *const *v)
     const void *o = v[7] == Py_None ? nullptr : f16(v[7]).data_ptr();
     require(q.dim() == 3, "attention: [S, H, Dh] expected");
     const int64_t S = q.size(0), H = q.size(1), Dh = q.size(2);
-    PyObject *acc[3] = {Py_None, Py_None, Py_None};
-    if (v[6] != Py_None) {
-        require(PySequence_Check(v[6]) && PySequence_Size(v[6]) == 3, "attention_bwd: acc = (dq, dk, dv)");
-        for (int i = 0; i < 3; i++) {
-            acc[i] = PySequence_GetItem(v[6], i);
-            if (!acc[i]) throw PyFailed();
-            Py_DECREF(acc[i]);                   // (the sequence holds it)
-        }
-    }
-    auto target = [&](int i) -> Result {
-        if (acc[i] == Py_None) return {new_like(q), nullptr};
-        return {tensor(acc[i]), acc[i]};
+    const bool into = v[6] != Py_None;
+    auto given = [&]() {
+        const Tensors acc(v[6]);
+        require(acc.size() == 3, "attention_bwd: acc = (dq, dk, dv)");
+        return acc.t;
     };
-    const Result dq = target(0), dk = target(1), dv = target(2);
+    const std::vector<at::Tensor> d = into ? given() : std::vector<at::Tensor>{new_like(q), new_like(q), new_like(q)};
     const size_t bytes = cacti_hip_attention_bwd_workspace(S, H);
     const at::Tensor ws = empty({(int64_t)bytes}, q, at::kByte);
     void *st = stream();
     run([&] {
         return cacti_hip_attention_bwd(S, H, Dh, alpha, q.data_ptr(), k.data_ptr(), w.data_ptr(), o, dO.data_ptr(), H * Dh, stats.data_ptr(),
-                                       dq.ptr(), dq.acc(), dk.ptr(), dk.acc(), dv.ptr(), dv.acc(), ws.data_ptr(), bytes, st);
+                                       d[0].data_ptr(), into, d[1].data_ptr(), into, d[2].data_ptr(), into, ws.data_ptr(), bytes, st);
     });
-    PyObject *x = dq.take(), *y = dk.take(), *z = dv.take(), *r = PyTuple_New(3);
-    PyTuple_SET_ITEM(r, 0, x);
-    PyTuple_SET_ITEM(r, 1, y);
-    PyTuple_SET_ITEM(r, 2, z);
+    PyObject *r = PyTuple_New(3);
+    if (!r) throw PyFailed();
+    for (int i = 0; i < 3; i++) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(d[i]));     // (a tensor that was given: its own object)
     return r;
 }
 
@@ -427,7 +421,8 @@ PyObject *silu_gate_bwd(PyObject *const *v)
 PyObject *add_f16(PyObject *const *v)
 {
     const at::Tensor &a = tensor(v[0]), &b = tensor(v[1]);
-    const Result out = v[2] == Py_None ? Result{new_like(a), nullptr} : Result{tensor(v[2]), v[2]};
+    // (element for element in memory order: the result has a's strides, whatever they are)
+    const Result out = v[2] == Py_None ? Result{at::empty_like(a), nullptr} : Result{tensor(v[2]), v[2]};
     void *st = stream();
     run([&] { return cacti_hip_add_f16(a.numel(), a.data_ptr(), b.data_ptr(), out.ptr(), st); });
     return out.take();

@@ -258,6 +258,43 @@ def test_accumulate_and_add(ops, oracle):
     assert (host(t).view(np.uint16) == (u + v).astype(np.uint16)).all()
 
 
+def test_add_of_transposed_operands(ops):
+    # element for element in memory order: the result has the operands' strides
+    a, b = (torch.randn(33, 50, device="cuda").half().t() for _ in range(2))
+    got = ops.add_f16(a, b)
+    assert got.stride() == a.stride()
+    assert torch.equal(got, a + b)
+
+
+def test_operators_run_on_the_current_stream(ops):
+    """A chain of operators, with a product that wants a workspace, captured on another stream and replayed on new inputs."""
+    x, y = (torch.empty(64, 250, dtype=torch.float16, device="cuda") for _ in range(2))
+    W = torch.randn(35, 250, device="cuda").half()
+    chain = lambda: ops.gemm(ops.silu_gate_fwd(ops.add_f16(x, y), y), W, tb=True)
+    eager = []
+    inputs = [[torch.randn_like(x) for _ in range(2)] for _ in range(3)]
+    for u, v in inputs:
+        x.copy_(u), y.copy_(v)
+        eager.append(chain())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = chain()
+    for (u, v), want in zip(inputs, eager):
+        x.copy_(u), y.copy_(v)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
+def test_operators_refuse_tensors_without_memory(ops):
+    # a batched tensor has no pointer; the error leaves the operators usable
+    x = torch.randn(3, 16, device="cuda").half()
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda a: ops.add_f16(a, a))(x)
+    assert torch.equal(ops.add_f16(x, x), x + x)
+
+
 # ---------------------------------------------------------------- GEMM
 GEMM_SHAPES = [
     (128, 128, 32), (256, 384, 192), (100, 72, 40), (128, 688, 256), (128, 256, 688),
