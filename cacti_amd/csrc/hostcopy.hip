@@ -12,6 +12,7 @@
 #include <atomic>
 #include <chrono>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -173,14 +174,19 @@ int read_large(void *dst, const void *src, size_t bytes, const int *word, int *w
                             std::min(chunk, window - (size_t)i * chunk));
             }
         };
-        std::vector<std::thread> th;
-        for (int t = 1; t < threads; t++)
-            th.emplace_back([&]() {
-                (void)hipSetDevice(dev);
-                work();
-            });
+        std::thread th[kReadThreads];
+        try {
+            for (int t = 1; t < threads; t++)
+                th[t] = std::thread([&]() {
+                    (void)hipSetDevice(dev);
+                    work();
+                });
+        } catch (const std::system_error &) {
+            // no more threads to be had: those that started and this one take the chunks
+        }
         work();
-        for (std::thread &t : th) t.join();
+        for (std::thread &t : th)
+            if (t.joinable()) t.join();
         if (failed.load()) return failed.load();
         done += window;
     }
