@@ -312,7 +312,7 @@ finish_rows_kernel(int M, int count, const uint32_t *__restrict__ cand, uint16_t
         __syncthreads();
         if (threadIdx.x == 0) {
             for (int w = 1; w < 16; w++) k = max(k, best[w]);
-            const uint16_t id = (uint16_t)(0xffff - (k & 0xffff));
+            const uint16_t id = k ? (uint16_t)(0xffff - (k & 0xffff)) : 0;     // (a row of NaNs alone has no candidate)
             out_tok[m] = id;
             if (m == M - 1 && pos >= 0) in_tok[pos] = (uint16_t)(in_tok[pos] + id);
         }
