@@ -67,6 +67,7 @@ constexpr int kTileRows = 64;
 constexpr int kTileB = kTileRows * kRowB;   // 16 KB
 constexpr int kNT = 256;                 // threads of a wave group (4 waves): the unit that loads a tile
 constexpr int kBM = 128;                 // rows of the fixed operand per wave group (32 per wave)
+constexpr int kCus = 256;
 constexpr float kSpread = 8.f;           // least row sum of exponentials for the short form of sigma (dQ kernel)
 
 struct AttnArgs {
@@ -80,6 +81,8 @@ struct AttnArgs {
     float *y, *sig;                      // [H][S] adjoint scratch: sigma, and 1 / l (exact arithmetic) or the
                                          // exponent offset m log2(e) + log2(l) (fast arithmetic) of each row
     int acc_dq, acc_dk, acc_dv;
+    int split, per;                      // dK / dV in parts (SPLIT): the parts' number, and the query tiles of each
+    float *part;                         // [split][2: dK, dV][H][S][Dh] sums of the parts
 };
 
 typedef __fp16 fp16x4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
@@ -1273,7 +1276,8 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
 
 constexpr int kDkvBufs = 3;                      // tile buffers per tensor (Q, dO) and sets of row statistics
 
-template <int KS, int DT, bool FAST, bool DMA>
+// SPLIT: a workgroup takes p.per of the query tiles of its keys and leaves its sums in p.part (dkv_parts).
+template <int KS, int DT, bool FAST, bool DMA, bool SPLIT>
 __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
 {
     // the whole argument block in scalar registers at once (read field by field where the control flow first
@@ -1289,7 +1293,9 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
               lh = lane >> 5;
     const int S = p.S, Dh = p.Dh;
     const int64_t ld = p.ld;
-    const int h = blockIdx.x % p.H, pr = blockIdx.x / p.H;
+    const int h = blockIdx.x % p.H, pz = blockIdx.x / p.H, pr = SPLIT ? pz / p.split : pz, z = SPLIT ? pz - pr * p.split : 0;
+    const int first_tile = pr * (kBM / kTileRows) + z * (SPLIT ? p.per : 0);
+    if (SPLIT && first_tile * kTileRows >= S) return;                   // no query tile left for this part
     const int64_t hoff = (int64_t)h * Dh;
     const int shift = DMA ? (int)(hoff & 7) : 0;                        // the head's first column in its window
     gptr_t Q = gp(p.q) + hoff - shift, G = gp(p.dO) + hoff - shift;
@@ -1320,7 +1326,7 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
                 kacc[dt][r] = 0.f;
                 vacc[dt][r] = 0.f;
             }
-        const int iq0 = c00 / kTileRows, niq = (S + kTileRows - 1) / kTileRows;
+        const int iq0 = first_tile, ntiles = (S + kTileRows - 1) / kTileRows, niq = SPLIT ? min(ntiles, iq0 + p.per) : ntiles;
         typedef typename std::conditional<DMA, DmaTileMap, FastTileMap>::type Map;
         typedef typename std::conditional<DMA, DmaTileLoader, FastTileLoader>::type Loader;
         const Map tm(ld, Dh, shift);
@@ -1402,12 +1408,14 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
             prod_tr<DT>(vacc, Gs + bf * kTileB, 32 * qb, pack8(pe), pack8(pe + 8), lane);
             prod_tr<DT>(kacc, Qs + bf * kTileB, 32 * qb, pack8(de), pack8(de + 8), lane);
         };
-        // tiles [a, b), tile a in LDS and published
+        // tiles [a, b), tile a in LDS and published.  The two blocks are one piece of code, and there are two call sites
+        // and not three: a workgroup meets most of its instructions once, coming from memory (51 -> 36 KB of them; 777
+        // positions, 16 heads of 128, in parts: 27.1 -> 24.8 us).
         auto run_tiles = [&](int a, int b) __attribute__((always_inline)) {
             for (int iq = a; iq < b; iq++) {
                 if (iq + 1 < niq) fetch(iq + 1);
-                block(iq, 0);
-                block(iq, 1);
+#pragma unroll 1
+                for (int qb = 0; qb < 2; qb++) block(iq, qb);
                 if (iq + 1 < niq) land(iq + 1);
                 tile_sync<DMA>();
             }
@@ -1436,9 +1444,10 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
         // (fast arithmetic, tiles loaded straight into LDS): while the vector unit forms P and dS of block b, the
         // matrix unit forms S and dP of block b + 1 and adds block b - 1 to dV and dK.  A wave has its SIMD to
         // itself here, so nothing else would fill the one unit while the other works.
-        const int iqB = iq0 + 2, iqE = S / kTileRows;
-        if (FAST && DMA && iqE > iqB) {
-            run_tiles(iq0, iqB);
+        const int iqB = SPLIT && z > 0 ? iq0 : iq0 + 2, iqE = SPLIT ? min(niq, S / kTileRows) : S / kTileRows;
+        const bool pipe = FAST && DMA && iqE > iqB;
+        run_tiles(iq0, pipe ? iqB : niq);
+        if (pipe) {
             if constexpr (FAST && DMA) {
                 const int a4 = (lane >> 2) & 3, b4 = lane & 3, n16 = (lane >> 4) & 1;
                 const int colb = 16 * n16 + 4 * b4;
@@ -1588,8 +1597,25 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
                 prod_tr<DT>(kacc, Qs + buf_of(iqE - 1) * kTileB, 32, PD[1][2], PD[1][3], lane);
             }
             run_tiles(iqE, niq);
-        } else {
-            run_tiles(iq0, niq);
+        }
+        if constexpr (SPLIT) {
+            if (mykey < S) {
+                const int64_t plane = (int64_t)p.H * S * Dh;
+                float *krow = p.part + z * 2 * plane + ((int64_t)h * S + mykey) * Dh, *vrow = krow + plane;
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const int d0 = 32 * dt + 8 * q + 4 * lh - shift;
+                        if (d0 >= 0 && d0 < Dh) {
+                            *reinterpret_cast<float4_t *>(krow + d0) =
+                                float4_t{kacc[dt][4 * q], kacc[dt][4 * q + 1], kacc[dt][4 * q + 2], kacc[dt][4 * q + 3]};
+                            *reinterpret_cast<float4_t *>(vrow + d0) =
+                                float4_t{vacc[dt][4 * q], vacc[dt][4 * q + 1], vacc[dt][4 * q + 2], vacc[dt][4 * q + 3]};
+                        }
+                    }
+            }
+            return;
         }
         const bool staged_v = DMA && !p.acc_dv, staged_k = DMA && !p.acc_dk;
         if (staged_v || staged_k) {
@@ -1620,6 +1646,42 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
         }
     }
 }
+
+// dK and dV from the sums of their parts, added in order; four columns per lane, blockIdx.y = 0 dK, 1 dV
+__global__ void __launch_bounds__(256) attn_bwd_dkv_sum_kernel(AttnArgs p)
+{
+    const int per_row = p.Dh / 4;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, plane = (int64_t)p.H * p.S * p.Dh;
+    if (i >= plane / 4) return;
+    const int64_t row = i / per_row;                                    // h * S + key
+    const int h = (int)(row / p.S), key = (int)(row - (int64_t)h * p.S), d = (int)(i - row * per_row) * 4;
+    const int tiles = (p.S + kTileRows - 1) / kTileRows - key / kBM * (kBM / kTileRows), parts = (tiles + p.per - 1) / p.per;
+    const float *src = p.part + blockIdx.y * plane + 4 * i;
+    float4_t a = *reinterpret_cast<const float4_t *>(src);
+    for (int z = 1; z < parts; z++) a += *reinterpret_cast<const float4_t *>(src + z * 2 * plane);
+    half_t *dst = (blockIdx.y ? p.dv : p.dk) + key * p.ld + (int64_t)h * p.Dh + d;
+    store_row4(dst, a[0], a[1], a[2], a[3], blockIdx.y ? 1.0f : p.alpha, blockIdx.y ? p.acc_dv : p.acc_dk);
+}
+
+// A workgroup of the dK / dV kernel walks all query tiles from its keys on, 1.4 us each behind some 10 us of start, and
+// a short sequence has few workgroups for it (611 positions of 16 heads: 80 of up to 10 tiles, on 256 CUs).  There the
+// query tiles of 128 keys go to several workgroups, as many as the device has room for, whose fp32 sums a second launch of
+// 4.6 to 6.6 us adds up: worth it from five tiles saved on.  Measured, us, one walk -> parts and their sum: 611 positions,
+// 16 heads of 64, 24.9 -> 15.6 + 4.6; 777 positions, 16 heads of 128, 35.6 -> 24.8 + 6.6; forward and adjoint together: 611 x 16 x 64 67.1 -> 64.6, 449 x 8 x 128
+// 63.8 -> 60.3, 1000 x 4 x 100 94.2 -> 77.6.  split = 1: not.
+struct DkvParts {
+    int split, per;
+};
+DkvParts dkv_parts(int64_t S, int64_t H)
+{
+    const int64_t groups = (S + kBM - 1) / kBM * H, tiles = (S + kTileRows - 1) / kTileRows;
+    int64_t split = std::min<int64_t>(kCus / groups, 8);
+    if (split < 2) return {1, (int)tiles};
+    const int64_t per = std::max<int64_t>(2, (tiles + split - 1) / split);
+    if (tiles - per < 5) return {1, (int)tiles};
+    return {(int)((tiles + per - 1) / per), (int)per};
+}
+size_t stats_part_bytes(int64_t S, int64_t H) { return ((size_t)(2 * S * H) * sizeof(float) + 15) / 16 * 16; }
 
 constexpr size_t kDkvSmem = 2 * kDkvBufs * kTileB + kDkvBufs * 4 * 64 * sizeof(float);
 
@@ -1653,18 +1715,29 @@ int launch_fwd(const AttnArgs &p, hipStream_t st)
 template <int KS, int DT, bool FAST, bool DMA>
 int launch_bwd(const AttnArgs &p, hipStream_t st)
 {
+    constexpr bool PARTS = FAST && DMA;
     static DeviceOnce ready;
     if (!ready.fresh()) {
         int rc = set_smem(attn_bwd_dq_kernel<KS, DT, FAST, DMA>, kQmSmem);
         if (rc) return rc;
-        if ((rc = set_smem(attn_bwd_dkv_kernel<KS, DT, FAST, DMA>, kDkvSmem))) return rc;
+        if ((rc = set_smem(attn_bwd_dkv_kernel<KS, DT, FAST, DMA, false>, kDkvSmem))) return rc;
+        if constexpr (PARTS)
+            if ((rc = set_smem(attn_bwd_dkv_kernel<KS, DT, FAST, DMA, true>, kDkvSmem))) return rc;
         ready.mark();
     }
     const int nqt = (p.S + kBM - 1) / kBM;
     hipLaunchKernelGGL((attn_bwd_dq_kernel<KS, DT, FAST, DMA>), dim3((unsigned)(nqt * p.H)), dim3(kNT2), kQmSmem, st, p);
     int rc = launch_status("attention_bwd_dq");
     if (rc) return rc;
-    hipLaunchKernelGGL((attn_bwd_dkv_kernel<KS, DT, FAST, DMA>), dim3((unsigned)(nqt * p.H)), dim3(kNT), kDkvSmem, st, p);
+    if constexpr (PARTS)
+        if (p.split > 1) {
+            hipLaunchKernelGGL((attn_bwd_dkv_kernel<KS, DT, FAST, DMA, true>), dim3((unsigned)(nqt * p.split * p.H)), dim3(kNT),
+                               kDkvSmem, st, p);
+            const int64_t lanes = (int64_t)p.H * p.S * (p.Dh / 4);
+            hipLaunchKernelGGL(attn_bwd_dkv_sum_kernel, dim3((unsigned)((lanes + 255) / 256), 2), dim3(256), 0, st, p);
+            return launch_status("attention_bwd_dkv");
+        }
+    hipLaunchKernelGGL((attn_bwd_dkv_kernel<KS, DT, FAST, DMA, false>), dim3((unsigned)(nqt * p.H)), dim3(kNT), kDkvSmem, st, p);
     return launch_status("attention_bwd_dkv");
 }
 
@@ -1772,6 +1845,14 @@ int attention_fwd_exact(int64_t S, int64_t H, int64_t Dh, float alpha, const voi
 
 }  // namespace cacti
 
+CACTI_API size_t cacti_hip_attention_bwd_workspace_best(int64_t S, int64_t H, int64_t Dh)
+{
+    if (S <= 0 || H <= 0 || Dh <= 0 || Dh > kDP) return cacti_hip_attention_bwd_workspace(S, H);
+    const DkvParts parts = dkv_parts(S, H);
+    if (parts.split < 2) return cacti_hip_attention_bwd_workspace(S, H);
+    return stats_part_bytes(S, H) + (size_t)parts.split * 2 * (size_t)H * (size_t)S * (size_t)Dh * sizeof(float);
+}
+
 CACTI_API int cacti_hip_attention_bwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,
                                       const void *v, const void *o, const void *dO, int64_t ld, const void *stats,
                                       void *dq, int dq_acc, void *dk, int dk_acc, void *dv, int dv_acc,
@@ -1798,6 +1879,12 @@ CACTI_API int cacti_hip_attention_bwd(int64_t S, int64_t H, int64_t Dh, float al
     p.l = p.m + S * H;
     p.y = (float *)workspace;
     p.sig = p.y + S * H;
+    const DkvParts parts = dkv_parts(S, H);
+    if (parts.split > 1 && aligned(workspace, 16) && workspace_bytes >= cacti_hip_attention_bwd_workspace_best(S, H, Dh)) {
+        p.split = parts.split;
+        p.per = parts.per;
+        p.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + stats_part_bytes(S, H));
+    }
     hipStream_t st = (hipStream_t)stream;
     int64_t span;
     const bool dma = direct_tiles(H, Dh, ld, {q, k, v, dO, o, dq, dk, dv}, &span);     // o may be null: passes

@@ -313,7 +313,7 @@ PyObject *attention_bwd(PyObject *const *v)
         return acc.t;
     };
     const std::vector<at::Tensor> d = into ? given() : std::vector<at::Tensor>{new_like(q), new_like(q), new_like(q)};
-    const size_t bytes = cacti_hip_attention_bwd_workspace(S, H);
+    const size_t bytes = cacti_hip_attention_bwd_workspace_best(S, H, Dh);
     const at::Tensor ws = empty({(int64_t)bytes}, q, at::kByte);
     void *st = stream();
     run([&] {

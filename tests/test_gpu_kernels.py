@@ -678,3 +678,33 @@ def test_rope_on_two_tensors_in_one_launch(S, H, Dh):
     w0 = a0.clone()
     ffi.call("cacti_hip_rope_bwd", S, H, Dh, x0.data_ptr(), cos.data_ptr(), sin.data_ptr(), w0.data_ptr(), 1, st)
     assert torch.equal(d0, w0) and torch.equal(d1, ops.rope_bwd(x1, cos, sin))
+
+
+# dK / dV in parts of the queries (the workspace of ops) against one walk over all of them (the least workspace): parts that
+# begin on the diagonal or past it, of whole tiles and of a ragged last one alone, and accumulation
+PART_SHAPES = [(611, 16, 64, False), (777, 16, 128, True), (449, 3, 100, False), (1000, 2, 128, False), (385, 5, 36, True),
+               (449, 1, 64, False), (1025, 8, 100, False), (640, 12, 100, True)]
+
+
+@pytest.mark.parametrize("S,H,Dh,acc", PART_SHAPES)
+def test_attention_bwd_in_parts(ops, S, H, Dh, acc):
+    from cacti_amd import ffi
+    from tests.util import rel_l2
+    least, best = ffi.lib().cacti_hip_attention_bwd_workspace(S, H), ffi.lib().cacti_hip_attention_bwd_workspace_best(S, H, Dh)
+    say("attention_bwd in parts", S, H, Dh, acc, least, best)
+    assert best > least
+    g = torch.Generator(device="cuda")
+    g.manual_seed(S + H + Dh)
+    q, k, v, dO, d0 = (torch.randn(S, H, Dh, generator=g, device="cuda").half() for _ in range(5))
+    alpha = Dh ** -0.5
+    o, stats = ops.attention_fwd(q, k, v, alpha)
+    got = ops.attention_bwd(q, k, v, dO, stats, alpha, acc=tuple(d0.clone() for _ in range(3)) if acc else None, o=o)
+    want = [d0.clone() for _ in range(3)]
+    ws = torch.empty(least, dtype=torch.uint8, device="cuda")
+    ffi.call("cacti_hip_attention_bwd", S, H, Dh, alpha, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dO.data_ptr(), H * Dh,
+             stats.data_ptr(), want[0].data_ptr(), int(acc), want[1].data_ptr(), int(acc), want[2].data_ptr(), int(acc),
+             ws.data_ptr(), least, torch.cuda.current_stream().cuda_stream)
+    assert_bits(host(got[0]), host(want[0]), "dq")
+    for a, b in zip(got[1:], want[1:]):
+        # fp32 sums of the same terms in another order, rounded once: a last place (2^-11 of it) here and there
+        assert rel_l2(host(a), host(b)) < 2e-4 and exact_frac(host(a), host(b)) > 0.95
