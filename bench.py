@@ -1037,7 +1037,7 @@ def run_decode(args):
            "roofline": {"bound": "hbm", "achieved": (wbytes + kvbytes) / dt / 1e9, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                         "frac": (wbytes + kvbytes) / dt / 1e9 / PEAK_HBM_GBS, "traffic": None,
                         "note": "whole position: %.2f GB of weights + %.2f GB of cached keys and values over the "
-                                "wall time of a call (about 15 launches per layer); per-kernel figures are in "
+                                "wall time of a call (6 launches per layer at this context); per-kernel figures are in "
                                 "profiles/" % (wbytes / 1e9, kvbytes / 1e9)}}
     k.close()
     model.close()
