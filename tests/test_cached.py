@@ -365,6 +365,26 @@ def test_cached_pass_error_paths(oracle):
 
 
 @pytest.mark.gpu
+def test_a_row_of_nans_decodes_to_a_token_of_the_vocabulary():
+    from cacti_amd.runtime import LlamaCached
+    cfg, flat, tok, lm_tok, scale = _inputs(seed=6)
+    ctx, m = _gpu_model(cfg, flat)
+    names = [n for n, _ in m.params]
+    i = names.index("lm_head")
+    m.put_param(i, np.full(m.params[i][1], np.nan, np.float16))
+    k = LlamaCached(m, 64)
+    k.reset_state()
+    t = np.zeros(64, np.uint16)
+    t[:2] = tok[:2]
+    k.set_tokens(t)
+    k.apply(0, 2)
+    assert (k.outputs()["tok"] == 0).all() and np.array_equal(k.tokens(), t)
+    k.apply(2, 3)                                          # its successor is fed back
+    k.outputs()
+    k.close(); m.close(); ctx.close()
+
+
+@pytest.mark.gpu
 def test_full_size_decode_agrees_with_one_call_over_the_same_tokens():
     """3B shapes (hidden 3200, 32 heads x 100, ffn 8640, vocabulary 32000), 2 layers, capacity 2048,
     no oracle run: a 515-token sequence processed as prompt + three single-token cycles (the
