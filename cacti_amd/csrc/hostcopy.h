@@ -11,16 +11,18 @@ struct HostRegion {
     size_t bytes;
 };
 constexpr int kMaxRegions = 8;
-constexpr size_t kStagingBytes = 4u << 20;
 
 // Page-locked memory regions are gathered into, with the words their arrival is announced in.  One gather at a time.
 struct Staging {
     char *base = nullptr;
+    size_t bytes = 0;
     unsigned epoch = 0;
     char *data() const { return base + kFlagBytes; }
-    size_t room() const { return kStagingBytes - kFlagBytes; }
+    size_t room() const { return bytes - kFlagBytes; }
     static constexpr size_t kFlagBytes = 4096;
 };
+constexpr size_t kStagingBytes = 4u << 20;     // of a context
+constexpr size_t kWordBytes = 8u << 10;        // of a call that reads one word
 // n <= kMaxRegions regions, in one launch on `st`, to places in s.data(); returns when they are there.  The launch comes
 // behind all work queued on `st`, so this waits for it like a stream synchronisation.
 int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st);
@@ -30,8 +32,9 @@ constexpr size_t kLargeRead = 512u << 10;      // from here on it is the better 
 // n regions of `bytes` (a multiple of 16), 16-byte aligned, set to zero
 int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st);
 
-// Up to four buffers that were given back are kept for later takers (page-locking costs hundreds of microseconds).
-bool staging_take(Staging *s);
+// A buffer of kStagingBytes or kWordBytes.  A few of each size that were given back are kept for later takers
+// (page-locking costs hundreds of microseconds).
+bool staging_take(Staging *s, size_t bytes);
 void staging_give_back(Staging *s);
 
 }  // namespace cacti

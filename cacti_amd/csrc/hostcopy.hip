@@ -110,8 +110,38 @@ int wait_flags(const unsigned *flags, int n, unsigned epoch, hipStream_t st)
     return 0;
 }
 
+// Buffers nobody uses at the moment, by size: at most 4 of a context's, for the next contexts, and 16 of a word's, one for
+// every thread that reads at the same time.
+struct Kept {
+    size_t bytes, most;
+    std::vector<Staging> free;
+};
 std::mutex g_mutex;
-std::vector<Staging> g_free;                   // staging buffers of contexts that are gone, for the next ones
+Kept g_kept[] = {{kStagingBytes, 4, {}}, {kWordBytes, 16, {}}};
+std::atomic<size_t> g_pinned{0};               // bytes page-locked here, kept or in use
+
+Kept *kept_of(size_t bytes)
+{
+    for (Kept &k : g_kept)
+        if (k.bytes == bytes) return &k;
+    return nullptr;
+}
+
+void *pinned_alloc(size_t bytes)
+{
+    void *p = nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    g_pinned += bytes;
+    return p;
+}
+void pinned_free(void *p, size_t bytes)
+{
+    hipHostFree(p);
+    g_pinned -= bytes;
+}
 
 // large reads, one at a time: page-locked memory for a window of chunks
 constexpr size_t kWindow = 16u << 20, kLeastChunk = 32u << 10, kLargeFlagBytes = kWindow / kLeastChunk * sizeof(unsigned) + 64;
@@ -139,9 +169,8 @@ int read_large(void *dst, const void *src, size_t bytes, const int *word, int *w
 {
     std::lock_guard<std::mutex> lock(g_large_mutex);
     if (!g_large) {
-        void *p = nullptr;
-        if (hipHostMalloc(&p, kLargeFlagBytes + kWindow, hipHostMallocPortable) != hipSuccess) {
-            (void)hipGetLastError();
+        void *p = pinned_alloc(kLargeFlagBytes + kWindow);
+        if (!p) {
             CACTI_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
             if (word) CACTI_HIP(hipMemcpyAsync(word_dst, word, sizeof(int), hipMemcpyDeviceToHost, st));
             CACTI_HIP(hipStreamSynchronize(st));
@@ -209,38 +238,35 @@ int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st)
     return 0;
 }
 
-bool staging_take(Staging *s)
+bool staging_take(Staging *s, size_t bytes)
 {
+    Kept *k = kept_of(bytes);
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        if (!g_free.empty()) {
-            *s = g_free.back();
-            g_free.pop_back();
+        if (!k->free.empty()) {
+            *s = k->free.back();
+            k->free.pop_back();
             return true;
         }
     }
-    void *p = nullptr;
-    if (hipHostMalloc(&p, kStagingBytes, hipHostMallocPortable) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
+    void *p = pinned_alloc(bytes);
+    if (!p) return false;
     memset(p, 0, Staging::kFlagBytes);
-    *s = Staging{static_cast<char *>(p), 0};
+    *s = Staging{static_cast<char *>(p), bytes, 0};
     return true;
 }
 
 void staging_give_back(Staging *s)
 {
     if (!s->base) return;
+    Kept *k = kept_of(s->bytes);
+    bool keep;
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        if (g_free.size() < 4) {
-            g_free.push_back(*s);
-            *s = Staging{};
-            return;
-        }
+        keep = k->free.size() < k->most;
+        if (keep) k->free.push_back(*s);
     }
-    hipHostFree(s->base);
+    if (!keep) pinned_free(s->base, s->bytes);
     *s = Staging{};
 }
 
@@ -248,25 +274,29 @@ void staging_give_back(Staging *s)
 
 using namespace cacti;
 
-namespace {
-// a calling thread's own, given back when the thread ends
-struct ThreadStaging {
-    Staging s;
-    ~ThreadStaging() { staging_give_back(&s); }
-};
-}  // namespace
-
+// The buffer is the call's, not the thread's: threads that live on after a read hold nothing.
 CACTI_API int cacti_hip_read_i32(const void *dev, int32_t *value, void *stream)
 {
     CACTI_REQUIRE(dev && value && aligned(dev, 16), CACTI_E_INVALID, "read_i32: null or misaligned pointer");
-    static thread_local ThreadStaging t;
-    if (!t.s.base && !staging_take(&t.s)) {
+    Staging s;
+    if (!staging_take(&s, kWordBytes)) {
         CACTI_HIP(hipMemcpyAsync(value, dev, sizeof(*value), hipMemcpyDeviceToHost, (hipStream_t)stream));
         CACTI_HIP(hipStreamSynchronize((hipStream_t)stream));
         return 0;
     }
-    const HostRegion r = {dev, t.s.data(), sizeof(*value)};
-    const int rc = gather_to_host(t.s, &r, 1, (hipStream_t)stream);
-    if (!rc) memcpy(value, t.s.data(), sizeof(*value));
+    const HostRegion r = {dev, s.data(), sizeof(*value)};
+    const int rc = gather_to_host(s, &r, 1, (hipStream_t)stream);
+    if (!rc) memcpy(value, s.data(), sizeof(*value));
+    staging_give_back(&s);
     return rc;
+}
+
+CACTI_API int cacti_hip_pinned_bytes(size_t *held, size_t *kept)
+{
+    CACTI_REQUIRE(held && kept, CACTI_E_INVALID, "pinned_bytes: null out pointer");
+    std::lock_guard<std::mutex> lock(g_mutex);
+    *held = g_pinned.load();
+    *kept = 0;
+    for (const Kept &k : g_kept) *kept += k.bytes * k.free.size();
+    return 0;
 }

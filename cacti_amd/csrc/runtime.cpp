@@ -200,7 +200,7 @@ int Ctx::init(int dev, size_t pool_bytes, int host_pagelocked)
     }
     CACTI_HIP(hipEventCreate(&ev0_));
     CACTI_HIP(hipEventCreate(&ev1_));
-    (void)staging_take(&staging_);             // (without it read-backs go through the runtime's copies)
+    (void)staging_take(&staging_, kStagingBytes);             // (without it read-backs go through the runtime's copies)
     return 0;
 }
 

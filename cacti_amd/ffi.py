@@ -51,6 +51,7 @@ SIGNATURES = {
     "cacti_hip_event_sync": (ci, [vp]),
     "cacti_hip_event_elapsed_ms": (ci, [vp, vp, C.POINTER(f32)]),
     "cacti_hip_read_i32": (ci, [vp, C.POINTER(C.c_int32), vp]),
+    "cacti_hip_pinned_bytes": (ci, [C.POINTER(sz), C.POINTER(sz)]),
     "cacti_hip_gemm_f16": (ci, [ci, ci, i64, i64, i64, f32, vp, i64, vp, i64, f32, vp, i64, vp]),
     "cacti_hip_gemm_f16_ws": (ci, [ci, ci, i64, i64, i64, f32, vp, i64, vp, i64, f32, vp, i64, vp, sz, C.POINTER(sz), vp]),
     "cacti_hip_gemm_plan": (ci, [i64, i64, i64, i64, C.POINTER(i64)]),

@@ -91,6 +91,9 @@ int cacti_hip_event_elapsed_ms(void *start, void *stop, float *ms);
 
 /* One 32-bit word of device memory (16-byte aligned) behind everything queued on the stream; returns when it is there. */
 int cacti_hip_read_i32(const void *dev, int32_t *value, void *stream);
+/* Page-locked host memory the library holds for read-backs: all of it, and the part that no context or call uses at
+ * the moment and that is kept for the next one. */
+int cacti_hip_pinned_bytes(size_t *held, size_t *kept);
 
 /* ------------------------------------------------------------------------- */
 /* GEMM: C = alpha * op(A) op(B) + beta * C, f16 x f16 -> fp32 accumulate ->   */
