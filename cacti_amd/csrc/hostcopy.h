@@ -23,16 +23,18 @@ struct Staging {
 };
 constexpr size_t kStagingBytes = 4u << 20;     // of a context
 constexpr size_t kWordBytes = 8u << 10;        // of a call that reads one word
+constexpr size_t kWindowBytes = Staging::kFlagBytes + (16u << 20);   // of a large read: a window of it at a time
 // n <= kMaxRegions regions, in one launch on `st`, to places in s.data(); returns when they are there.  The launch comes
 // behind all work queued on `st`, so this waits for it like a stream synchronisation.
 int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st);
-// one region of any size to pageable memory, likewise, and (not null) a word of device memory with it
+// one region of any size to pageable memory, likewise, and (not null) a word of device memory with it; readers on other
+// threads and streams go on meanwhile
 int read_large(void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st);
 constexpr size_t kLargeRead = 512u << 10;      // from here on it is the better one
 // n regions of `bytes` (a multiple of 16), 16-byte aligned, set to zero
 int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st);
 
-// A buffer of kStagingBytes or kWordBytes.  A few of each size that were given back are kept for later takers
+// A buffer of one of the sizes above.  A few of each size that were given back are kept for later takers
 // (page-locking costs hundreds of microseconds).
 bool staging_take(Staging *s, size_t bytes);
 void staging_give_back(Staging *s);

@@ -110,14 +110,15 @@ int wait_flags(const unsigned *flags, int n, unsigned epoch, hipStream_t st)
     return 0;
 }
 
-// Buffers nobody uses at the moment, by size: at most 4 of a context's, for the next contexts, and 16 of a word's, one for
-// every thread that reads at the same time.
+// Buffers nobody uses at the moment, by size: at most 4 of a context's, for the next contexts, 16 of a word's, one for
+// every thread that reads at the same time, and two windows of large reads (a third reader at the same time page-locks
+// its own and frees it again).
 struct Kept {
     size_t bytes, most;
     std::vector<Staging> free;
 };
 std::mutex g_mutex;
-Kept g_kept[] = {{kStagingBytes, 4, {}}, {kWordBytes, 16, {}}};
+Kept g_kept[] = {{kStagingBytes, 4, {}}, {kWordBytes, 16, {}}, {kWindowBytes, 2, {}}};
 std::atomic<size_t> g_pinned{0};               // bytes page-locked here, kept or in use
 
 Kept *kept_of(size_t bytes)
@@ -143,12 +144,10 @@ void pinned_free(void *p, size_t bytes)
     g_pinned -= bytes;
 }
 
-// large reads, one at a time: page-locked memory for a window of chunks
-constexpr size_t kWindow = 16u << 20, kLeastChunk = 32u << 10, kLargeFlagBytes = kWindow / kLeastChunk * sizeof(unsigned) + 64;
+// a large read's buffer: 64 bytes for the word, then the flags, then the window of chunks
+constexpr size_t kWindow = kWindowBytes - Staging::kFlagBytes, kLeastChunk = 32u << 10;
+static_assert(64 + kWindow / kLeastChunk * sizeof(unsigned) <= Staging::kFlagBytes, "a word per chunk");
 constexpr int kStreamBlocks = 16, kReadThreads = 4;
-std::mutex g_large_mutex;
-char *g_large = nullptr;
-unsigned g_large_epoch = 0;
 
 }  // namespace
 
@@ -162,33 +161,18 @@ int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st)
     return rc ? rc : wait_flags(flags, nflags, s.epoch, st);
 }
 
-// Measured, us, one gather and one copy behind it / 1 MiB pieces before -> chunks: 2 MiB 119 -> 76, 20 MiB 569 -> 473.  A
-// helper thread costs some 10 us to start: worth it from several MiB on, where the copying host (12 .. 30 GB/s) and not
-// the link (52) is what one thread would wait for.  Below 512 KiB chunks bring nothing (32 us at 512 KiB either way).
-int read_large(void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st)
+static int read_windows(Staging &s, void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st)
 {
-    std::lock_guard<std::mutex> lock(g_large_mutex);
-    if (!g_large) {
-        void *p = pinned_alloc(kLargeFlagBytes + kWindow);
-        if (!p) {
-            CACTI_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
-            if (word) CACTI_HIP(hipMemcpyAsync(word_dst, word, sizeof(int), hipMemcpyDeviceToHost, st));
-            CACTI_HIP(hipStreamSynchronize(st));
-            return 0;
-        }
-        g_large = static_cast<char *>(p);
-        memset(g_large, 0, kLargeFlagBytes);
-    }
-    int *const word_here = reinterpret_cast<int *>(g_large);       // 64 bytes for it, then the flags, then the data
-    unsigned *const flags = reinterpret_cast<unsigned *>(g_large + 64);
-    char *const data = g_large + kLargeFlagBytes;
+    int *const word_here = reinterpret_cast<int *>(s.base);
+    unsigned *const flags = reinterpret_cast<unsigned *>(s.base + 64);
+    char *const data = s.data();
     int dev = 0;
     CACTI_HIP(hipGetDevice(&dev));
     for (size_t done = 0; done < bytes;) {
         const size_t window = std::min(bytes - done, kWindow), chunk = window < (4u << 20) ? kLeastChunk : 2 * kLeastChunk;
         const int chunks = (int)((window + chunk - 1) / chunk), threads = (int)std::min<size_t>(kReadThreads, 1 + window / (4u << 20));
-        if (++g_large_epoch == 0) g_large_epoch = 1;
-        const unsigned epoch = g_large_epoch;
+        if (++s.epoch == 0) s.epoch = 1;
+        const unsigned epoch = s.epoch;
         hipLaunchKernelGGL(stream_kernel, dim3((unsigned)std::min(chunks, kStreamBlocks)), dim3(256), 0, st,
                            reinterpret_cast<const uint4 *>(static_cast<const char *>(src) + done), reinterpret_cast<uint4 *>(data),
                            (int64_t)((window + 15) / 16), (int64_t)(chunk / 16), word, word_here, flags, epoch);
@@ -221,6 +205,23 @@ int read_large(void *dst, const void *src, size_t bytes, const int *word, int *w
     }
     if (word) *word_dst = *word_here;
     return 0;
+}
+
+// Measured, us, one gather and one copy behind it / 1 MiB pieces before -> chunks: 2 MiB 119 -> 76, 20 MiB 569 -> 473.  A
+// helper thread costs some 10 us to start: worth it from several MiB on, where the copying host (12 .. 30 GB/s) and not
+// the link (52) is what one thread would wait for.  Below 512 KiB chunks bring nothing (32 us at 512 KiB either way).
+int read_large(void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st)
+{
+    Staging s;
+    if (!staging_take(&s, kWindowBytes)) {
+        CACTI_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+        if (word) CACTI_HIP(hipMemcpyAsync(word_dst, word, sizeof(int), hipMemcpyDeviceToHost, st));
+        CACTI_HIP(hipStreamSynchronize(st));
+        return 0;
+    }
+    const int rc = read_windows(s, dst, src, bytes, word, word_dst, st);
+    staging_give_back(&s);
+    return rc;
 }
 
 int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st)

@@ -4,6 +4,7 @@ import threading
 
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -18,7 +19,6 @@ def pinned():
 def test_reading_a_word_holds_no_memory_per_thread():
     """Threads that stay alive after a read of one word hold nothing, and what is kept for later reads stays small however
     many threads read at once."""
-    import torch
     from cacti_amd import ffi
     words = torch.arange(0, 48 * 4, 4, dtype=torch.int32, device="cuda").view(48, 1).repeat(1, 4).contiguous()
     torch.cuda.synchronize()
@@ -42,3 +42,57 @@ def test_reading_a_word_holds_no_memory_per_thread():
         t.join()
     assert got == [4 * i for i in range(48)]
     assert after[0] - before[0] <= 16 * 8192 and after[0] - after[1] == before[0] - before[1]
+
+
+SMALL = dict(S=32, D=256, H=4, F=512, L=1, eps=1e-6)
+
+
+def model(V=4096):
+    from cacti_amd.runtime import Ctx, Llama
+    ctx = Ctx(0, 256 << 20, True)
+    m = Llama(ctx, SMALL["S"], SMALL["D"], SMALL["H"], SMALL["D"] // SMALL["H"], SMALL["F"], V, SMALL["L"], SMALL["eps"])
+    r = np.random.default_rng(3)
+    for i, (name, shape) in enumerate(m.params):
+        m.put_param(i, (r.standard_normal(shape) * 0.05).astype(np.float16))
+    tok = r.integers(0, V, SMALL["S"]).astype(np.uint16)
+    m.step(tok, tok, np.full(SMALL["S"], 8.0, np.float32))
+    return ctx, m
+
+
+def busy(stream, ms):
+    """Keeps a stream busy for about that long (a kernel that counts clock cycles)."""
+    st = torch.cuda.ExternalStream(stream, device="cuda:0")
+    with torch.cuda.stream(st):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        torch.cuda._sleep(1000)
+        a.record()
+        torch.cuda._sleep(1000000)
+        b.record()
+        b.synchronize()
+        torch.cuda._sleep(int(min(ms / a.elapsed_time(b), 2000) * 1000000))
+
+
+def test_a_large_read_does_not_wait_for_another_contexts_stream():
+    """One context's large read waits for what is queued on its stream; a read of another context, on another thread, is
+    through before that."""
+    from cacti_amd import ffi
+    torch.cuda.init()
+    (ctx_a, a), (ctx_b, b) = model(), model()
+    i = [n for n, _ in a.params].index("lm_head")
+    want = a.grad(i)
+    assert want.nbytes >= 2 << 20 and np.array_equal(want, b.grad(i))
+    got = {}
+
+    def slow():
+        got["a"] = a.grad(i)
+
+    busy(ffi.lib().cacti_ctx_stream(ctx_a._c), 1500.0)
+    t = threading.Thread(target=slow)
+    t.start()
+    t.join(0.1)                                            # it is inside its read by now
+    got["b"] = b.grad(i)
+    first = t.is_alive()
+    t.join()
+    assert first and np.array_equal(got["a"], want) and np.array_equal(got["b"], want)
+    for x in (a, b, ctx_a, ctx_b):
+        x.close()
