@@ -17,6 +17,7 @@ struct Staging {
     char *base = nullptr;
     size_t bytes = 0;
     unsigned epoch = 0;
+    bool lost = false;                         // a failed read may still be writing it
     char *data() const { return base + kFlagBytes; }
     size_t room() const { return bytes - kFlagBytes; }
     static constexpr size_t kFlagBytes = 4096;

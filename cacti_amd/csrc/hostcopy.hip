@@ -12,10 +12,9 @@
 #include <atomic>
 #include <chrono>
 #include <mutex>
-#include <system_error>
-#include <thread>
 #include <vector>
 
+#include "chunks.h"
 #include "common.h"
 #include "hostcopy.h"
 
@@ -144,10 +143,19 @@ void pinned_free(void *p, size_t bytes)
     g_pinned -= bytes;
 }
 
+// After a failure: the kernel may still be writing the buffer.  Where not even waiting for it works, the buffer is never
+// handed out again.
+void settle(Staging &s, hipStream_t st)
+{
+    if (hipStreamSynchronize(st) == hipSuccess) return;
+    (void)hipGetLastError();
+    s.lost = true;
+}
+
 // a large read's buffer: 64 bytes for the word, then the flags, then the window of chunks
 constexpr size_t kWindow = kWindowBytes - Staging::kFlagBytes, kLeastChunk = 32u << 10;
 static_assert(64 + kWindow / kLeastChunk * sizeof(unsigned) <= Staging::kFlagBytes, "a word per chunk");
-constexpr int kStreamBlocks = 16, kReadThreads = 4;
+constexpr int kStreamBlocks = 16;
 
 }  // namespace
 
@@ -157,8 +165,11 @@ int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st)
     unsigned *flags = reinterpret_cast<unsigned *>(s.base);
     int nflags = 0;
     if (++s.epoch == 0) s.epoch = 1;
-    const int rc = launch_gather(r, n, flags, s.epoch, &nflags, st);
-    return rc ? rc : wait_flags(flags, nflags, s.epoch, st);
+    int rc = launch_gather(r, n, flags, s.epoch, &nflags, st);
+    if (rc) return rc;
+    rc = wait_flags(flags, nflags, s.epoch, st);
+    if (rc) settle(s, st);
+    return rc;
 }
 
 static int read_windows(Staging &s, void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st)
@@ -170,7 +181,7 @@ static int read_windows(Staging &s, void *dst, const void *src, size_t bytes, co
     CACTI_HIP(hipGetDevice(&dev));
     for (size_t done = 0; done < bytes;) {
         const size_t window = std::min(bytes - done, kWindow), chunk = window < (4u << 20) ? kLeastChunk : 2 * kLeastChunk;
-        const int chunks = (int)((window + chunk - 1) / chunk), threads = (int)std::min<size_t>(kReadThreads, 1 + window / (4u << 20));
+        const int chunks = (int)((window + chunk - 1) / chunk), threads = (int)std::min<size_t>(kCopyThreads, 1 + window / (4u << 20));
         if (++s.epoch == 0) s.epoch = 1;
         const unsigned epoch = s.epoch;
         hipLaunchKernelGGL(stream_kernel, dim3((unsigned)std::min(chunks, kStreamBlocks)), dim3(256), 0, st,
@@ -178,29 +189,14 @@ static int read_windows(Staging &s, void *dst, const void *src, size_t bytes, co
                            (int64_t)((window + 15) / 16), (int64_t)(chunk / 16), word, word_here, flags, epoch);
         const int rc = launch_status("read_large");
         if (rc) return rc;
-        std::atomic<int> next{0}, failed{0};
-        auto work = [&]() {
-            for (int i; !failed.load() && (i = next.fetch_add(1)) < chunks;) {
-                const int rc = wait_flags(flags + i, 1, epoch, st);
-                if (rc) failed.store(rc);
-                else memcpy(static_cast<char *>(dst) + done + (size_t)i * chunk, data + (size_t)i * chunk,
-                            std::min(chunk, window - (size_t)i * chunk));
-            }
-        };
-        std::thread th[kReadThreads];
-        try {
-            for (int t = 1; t < threads; t++)
-                th[t] = std::thread([&]() {
-                    (void)hipSetDevice(dev);
-                    work();
-                });
-        } catch (const std::system_error &) {
-            // no more threads to be had: those that started and this one take the chunks
+        const ChunkError e = copy_chunks(
+            static_cast<char *>(dst) + done, data, window, chunk, threads, [&]() { (void)hipSetDevice(dev); },
+            [&](int i) { return wait_flags(flags + i, 1, epoch, st); }, []() { return cacti_hip_last_error(); });
+        if (e.rc) {
+            settle(s, st);
+            set_error("%s", e.text);
+            return e.rc;
         }
-        work();
-        for (std::thread &t : th)
-            if (t.joinable()) t.join();
-        if (failed.load()) return failed.load();
         done += window;
     }
     if (word) *word_dst = *word_here;
@@ -253,13 +249,19 @@ bool staging_take(Staging *s, size_t bytes)
     void *p = pinned_alloc(bytes);
     if (!p) return false;
     memset(p, 0, Staging::kFlagBytes);
-    *s = Staging{static_cast<char *>(p), bytes, 0};
+    *s = Staging{};
+    s->base = static_cast<char *>(p);
+    s->bytes = bytes;
     return true;
 }
 
 void staging_give_back(Staging *s)
 {
     if (!s->base) return;
+    if (s->lost) {                             // (neither kept nor freed: something may still write it)
+        *s = Staging{};
+        return;
+    }
     Kept *k = kept_of(s->bytes);
     bool keep;
     {
