@@ -15,6 +15,7 @@
 
 #include "../../include/cacti_hip_runtime.h"
 #include "common.h"
+#include "hostcopy.h"
 
 namespace {
 
@@ -175,6 +176,7 @@ CACTI_API int cacti_hip_primary_ctx_reset(int dev)
     CACTI_REQUIRE(live_contexts(dev) == 0, CACTI_E_STATE,
                   "primary_ctx_reset: %d device context(s) of this library are alive on device %d; destroy "
                   "them first (a reset frees their pool, streams and events)", live_contexts(dev), dev);
+    staging_release(dev);          // page-locked buffers kept for later read-backs
     CACTI_HIP(hipDevicePrimaryCtxReset(dev));
     module_epoch_advance();        // function attributes and symbol addresses are looked up again
     return 0;

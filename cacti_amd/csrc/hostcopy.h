@@ -17,6 +17,8 @@ struct Staging {
     char *base = nullptr;
     size_t bytes = 0;
     unsigned epoch = 0;
+    int dev = 0;                               // the device that was current when it was page-locked
+    unsigned resets = 0;                       // and how often that had been reset
     bool lost = false;                         // a failed read may still be writing it
     char *data() const { return base + kFlagBytes; }
     size_t room() const { return bytes - kFlagBytes; }
@@ -35,9 +37,12 @@ constexpr size_t kLargeRead = 512u << 10;      // from here on it is the better 
 // n regions of `bytes` (a multiple of 16), 16-byte aligned, set to zero
 int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st);
 
-// A buffer of one of the sizes above.  A few of each size that were given back are kept for later takers
-// (page-locking costs hundreds of microseconds).
+// A buffer of one of the sizes above, for the current device.  A few of each size that were given back are kept for later
+// takers (page-locking costs hundreds of microseconds).
 bool staging_take(Staging *s, size_t bytes);
 void staging_give_back(Staging *s);
+// Before a reset of the device, which deletes its page-locked memory too: frees what is kept, and what is in use then is
+// not kept later.
+void staging_release(int dev);
 
 }  // namespace cacti

@@ -119,6 +119,7 @@ struct Kept {
 std::mutex g_mutex;
 Kept g_kept[] = {{kStagingBytes, 4, {}}, {kWordBytes, 16, {}}, {kWindowBytes, 2, {}}};
 std::atomic<size_t> g_pinned{0};               // bytes page-locked here, kept or in use
+unsigned g_resets[64];                         // per device, under g_mutex
 
 Kept *kept_of(size_t bytes)
 {
@@ -238,39 +239,59 @@ int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st)
 bool staging_take(Staging *s, size_t bytes)
 {
     Kept *k = kept_of(bytes);
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
+        (void)hipGetLastError();
+        return false;
+    }
+    *s = Staging{};
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        if (!k->free.empty()) {
-            *s = k->free.back();
-            k->free.pop_back();
-            return true;
-        }
+        for (size_t i = k->free.size(); i-- > 0;)
+            if (k->free[i].dev == dev) {
+                *s = k->free[i];
+                k->free.erase(k->free.begin() + (std::ptrdiff_t)i);
+                return true;
+            }
+        s->resets = g_resets[dev];
     }
     void *p = pinned_alloc(bytes);
     if (!p) return false;
     memset(p, 0, Staging::kFlagBytes);
-    *s = Staging{};
     s->base = static_cast<char *>(p);
     s->bytes = bytes;
+    s->dev = dev;
     return true;
 }
 
 void staging_give_back(Staging *s)
 {
     if (!s->base) return;
-    if (s->lost) {                             // (neither kept nor freed: something may still write it)
-        *s = Staging{};
-        return;
-    }
-    Kept *k = kept_of(s->bytes);
-    bool keep;
+    bool keep = false, ours;
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        keep = k->free.size() < k->most;
+        Kept *k = kept_of(s->bytes);
+        ours = !s->lost && s->resets == g_resets[s->dev];
+        keep = ours && k->free.size() < k->most;
         if (keep) k->free.push_back(*s);
     }
-    if (!keep) pinned_free(s->base, s->bytes);
+    // (one that may still be written, or that a reset has deleted, is neither kept nor freed)
+    if (ours && !keep) pinned_free(s->base, s->bytes);
+    else if (!ours) g_pinned -= s->bytes;
     *s = Staging{};
+}
+
+void staging_release(int dev)
+{
+    if (dev < 0 || dev >= 64) return;
+    std::lock_guard<std::mutex> lock(g_mutex);
+    for (Kept &k : g_kept)
+        for (size_t i = k.free.size(); i-- > 0;)
+            if (k.free[i].dev == dev) {
+                pinned_free(k.free[i].base, k.bytes);
+                k.free.erase(k.free.begin() + (std::ptrdiff_t)i);
+            }
+    g_resets[dev]++;
 }
 
 }  // namespace cacti

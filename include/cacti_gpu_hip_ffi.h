@@ -73,6 +73,7 @@ int cacti_hip_primary_ctx_release(int dev);                     /* lib.rs:159   
  * hipError_t (a status, never an abort).  reset destroys everything on the device, so it is refused with CACTI_E_STATE
  * while a cacti_ctx of this library exists on `dev`; after a reset the library looks its per-device
  * state (kernel attributes, the address of its built-in scratch array) up again on the next launch.
+ * The page-locked buffers it keeps for read-backs are given back before the reset.
  * Memory, streams and events the caller created on the device are the caller's to forget. */
 int cacti_hip_primary_ctx_set_flags(int dev, unsigned flags);   /* lib.rs:186       */
 int cacti_hip_primary_ctx_reset(int dev);                       /* lib.rs:169       */

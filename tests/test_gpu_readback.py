@@ -96,3 +96,29 @@ def test_a_large_read_does_not_wait_for_another_contexts_stream():
     assert first and np.array_equal(got["a"], want) and np.array_equal(got["b"], want)
     for x in (a, b, ctx_a, ctx_b):
         x.close()
+
+
+def test_a_device_reset_leaves_no_page_locked_buffer(tmp_path):
+    """The buffers kept for later contexts go before the reset that would delete them under the library (a child process:
+    the reset takes everything on the device with it)."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = (
+        "import sys\n"
+        "sys.path.insert(0, %r)\n"
+        "import torch\n"
+        "torch.cuda.init()\n"
+        "from cacti_amd import ffi\n"
+        "from tests.test_gpu_readback import model, pinned\n"
+        "ctx, m = model()\n"
+        "m.grads()\n"
+        "m.close(); ctx.close()\n"
+        "held, kept = pinned()\n"
+        "assert held == kept >= (16 << 20), (held, kept)\n"
+        "ffi.call('cacti_hip_primary_ctx_reset', 0)\n"
+        "assert pinned() == (0, 0), pinned()\n"
+        "print('released')\n" % root)
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "released" in r.stdout, r.stdout + r.stderr[-2000:]
