@@ -929,28 +929,36 @@ int Ctx::spill_eagerly(const Entry &e)
     return 0;
 }
 
-int Ctx::pool_alloc(size_t bytes, size_t *off, bool high)
+size_t Ctx::pinned_bytes() const
+{
+    size_t n = 0;
+    for (const Cell &c : cells_)
+        if (c.alive && c.voff != kNoOffset && c.pin > 0) n += c.ty.bytes();
+    return n;
+}
+
+size_t Ctx::pool_try(size_t bytes, bool high)
 {
     size_t o = pool_.alloc(bytes, high);
+    if (o == kNoOffset && try_soft_oom(bytes) == 0) o = pool_.alloc(bytes, high);
+    if (o != kNoOffset) n_alloc_++;
+    return o;
+}
+
+int Ctx::pool_alloc(size_t bytes, size_t *off, bool high)
+{
+    const size_t o = pool_try(bytes, high);
     if (o == kNoOffset) {
-        int rc = try_soft_oom(bytes);
-        if (rc == 0) o = pool_.alloc(bytes, high);
-        if (o == kNoOffset) {
-            // the reference dumps the pool's usage before it panics (src/pctx/nvgpu.rs:2424-2440); here the
-            // full table goes to stderr and the status message carries the pool's line of it
-            const std::string rep = usage_report();
-            fprintf(stderr, "cacti: device pool exhausted, request of %zu bytes does not fit after eviction\n%s", bytes,
-                    rep.c_str());
-            size_t pinned = 0;
-            for (const Cell &c : cells_)
-                if (c.alive && c.voff != kNoOffset && c.pin > 0) pinned += c.ty.bytes();
-            set_error("device pool exhausted: request %zu bytes, cap %zu, used %zu, front %zu, largest free %zu, "
-                      "pinned by the running thunk %zu, downloads in flight %zu (usage by class of cell on stderr)",
-                      bytes, pool_.cap(), pool_.used(), pool_.front(), pool_.largest_free(), pinned, pending_bytes_);
-            return CACTI_E_OOM;
-        }
+        // the reference dumps the pool's usage before it panics (src/pctx/nvgpu.rs:2424-2440); here the
+        // full table goes to stderr and the status message carries the pool's line of it
+        const std::string rep = usage_report();
+        fprintf(stderr, "cacti: device pool exhausted, request of %zu bytes does not fit after eviction\n%s", bytes,
+                rep.c_str());
+        set_error("device pool exhausted: request %zu bytes, cap %zu, used %zu, front %zu, largest free %zu, "
+                  "pinned by the running thunk %zu, downloads in flight %zu (usage by class of cell on stderr)",
+                  bytes, pool_.cap(), pool_.used(), pool_.front(), pool_.largest_free(), pinned_bytes(), pending_bytes_);
+        return CACTI_E_OOM;
     }
-    n_alloc_++;
     *off = o;
     return 0;
 }
@@ -1328,8 +1336,12 @@ int Ctx::run_entry(const Entry &e)
     }
     size_t ws_off = kNoOffset, ws_bytes = 0;
     if (!rc) {
-        ws_bytes = sp.workspace(aty);
-        if (ws_bytes) rc = pool_alloc(ws_bytes, &ws_off);
+        const size_t least = sp.workspace(aty);
+        ws_bytes = sp.workspace_best(aty);
+        // (nothing is evicted for scratch that the running thunk's own cells leave no room for)
+        if (ws_bytes > least && ws_bytes + pinned_bytes() <= pool_.cap()) ws_off = pool_try(ws_bytes);
+        if (ws_off == kNoOffset) ws_bytes = least;
+        if (ws_off == kNoOffset && ws_bytes) rc = pool_alloc(ws_bytes, &ws_off);
     }
     if (!rc) {
         // resolve pointers only now: eviction during allocation cannot move pinned cells

@@ -110,7 +110,9 @@ struct ThunkSpec {
     // source that dies at this entry instead of copying it)
     virtual bool is_copy() const { return false; }
     virtual int out_ty(const std::vector<CellType> &arg, std::vector<CellType> &out) const = 0;
+    // device scratch of `run`: what it cannot do without, and what it is fastest with (taken where the pool has it)
     virtual size_t workspace(const std::vector<CellType> &) const { return 0; }
+    virtual size_t workspace_best(const std::vector<CellType> &a) const { return workspace(a); }
     // label under which launches are grouped in the timing report (name + shape for GEMMs)
     virtual std::string key(const std::vector<CellType> &, uint32_t) const { return name(); }
     virtual int run(Ctx &ctx, const std::vector<CellType> &aty, void *const *a,
@@ -168,7 +170,9 @@ class Ctx {
     // the current version (uploading from the host replica)
     int ensure_vmem(CellPtr c, bool need_value);
     int pool_alloc(size_t bytes, size_t *off, bool high = false);                   // with soft-OOM eviction
+    size_t pool_try(size_t bytes, bool high = false);            // likewise; kNoOffset and no report when it does not fit
     void pool_free(size_t off) { pool_.free(off); }              // later reuse is ordered on the stream
+    size_t pinned_bytes() const;                                 // of the cells of the running thunk
     int try_soft_oom(size_t need);
     int evict(CellPtr c);                                        // VMem -> Mem, drop VMem
     // Overlapped spilling (page-locked host memory only).  Downloads and uploads run on two further

@@ -600,7 +600,8 @@ struct AttentionBwdSpec : ThunkSpec {
         o = {a[0], a[0], a[0]};
         return 0;
     }
-    size_t workspace(const std::vector<CellType> &a) const override
+    size_t workspace(const std::vector<CellType> &a) const override { return cacti_hip_attention_bwd_workspace(a[0].shape[0], H); }
+    size_t workspace_best(const std::vector<CellType> &a) const override
     {
         return cacti_hip_attention_bwd_workspace_best(a[0].shape[0], H, a[0].shape[1] / H);
     }
