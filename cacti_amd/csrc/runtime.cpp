@@ -951,9 +951,9 @@ int Ctx::pool_alloc(size_t bytes, size_t *off, bool high)
     if (o == kNoOffset) {
         // the reference dumps the pool's usage before it panics (src/pctx/nvgpu.rs:2424-2440); here the
         // full table goes to stderr and the status message carries the pool's line of it
-        const std::string rep = usage_report();
-        fprintf(stderr, "cacti: device pool exhausted, request of %zu bytes does not fit after eviction\n%s", bytes,
-                rep.c_str());
+        if (!quiet_oom_)
+            fprintf(stderr, "cacti: device pool exhausted, request of %zu bytes does not fit after eviction\n%s", bytes,
+                    usage_report().c_str());
         set_error("device pool exhausted: request %zu bytes, cap %zu, used %zu, front %zu, largest free %zu, "
                   "pinned by the running thunk %zu, downloads in flight %zu (usage by class of cell on stderr)",
                   bytes, pool_.cap(), pool_.used(), pool_.front(), pool_.largest_free(), pinned_bytes(), pending_bytes_);
@@ -1321,18 +1321,35 @@ int Ctx::run_entry(const Entry &e)
         return 0;
     }
     const ThunkSpec &sp = *thunks_[e.thunk];
+    const int n = sp.pieces();
+    quiet_oom_ = n > 1;
+    int rc = run_thunk(sp, e.args, e.outs, e.acc_mask);
+    quiet_oom_ = false;
+    if (n <= 1 || rc != CACTI_E_OOM) return rc;
+    for (int i = 0; i < n; i++) {
+        std::vector<CellPtr> args;
+        const std::unique_ptr<ThunkSpec> one = sp.piece(i, e.args, &args);
+        rc = run_thunk(*one, args, {e.outs[(size_t)i]}, (e.acc_mask >> i) & 1);
+        if (rc) return rc;
+    }
+    return 0;
+}
+
+// CACTI_E_OOM: nothing has been launched
+int Ctx::run_thunk(const ThunkSpec &sp, const std::vector<CellPtr> &args, const std::vector<CellPtr> &outs, uint32_t acc_mask)
+{
     std::vector<CellType> aty, oty;
-    for (CellPtr a : e.args) cells_[a].pin++;
-    for (CellPtr o : e.outs) cells_[o].pin++;
+    for (CellPtr a : args) cells_[a].pin++;
+    for (CellPtr o : outs) cells_[o].pin++;
     int rc = 0;
     std::vector<void *> ap, op;
-    for (CellPtr a : e.args) {
+    for (CellPtr a : args) {
         if ((rc = ensure_vmem(a, true))) break;
         aty.push_back(cells_[a].ty);
     }
-    for (size_t k = 0; !rc && k < e.outs.size(); k++) {
-        if ((rc = ensure_vmem(e.outs[k], (e.acc_mask >> k) & 1))) break;
-        oty.push_back(cells_[e.outs[k]].ty);
+    for (size_t k = 0; !rc && k < outs.size(); k++) {
+        if ((rc = ensure_vmem(outs[k], (acc_mask >> k) & 1))) break;
+        oty.push_back(cells_[outs[k]].ty);
     }
     size_t ws_off = kNoOffset, ws_bytes = 0;
     if (!rc) {
@@ -1345,13 +1362,13 @@ int Ctx::run_entry(const Entry &e)
     }
     if (!rc) {
         // resolve pointers only now: eviction during allocation cannot move pinned cells
-        for (CellPtr a : e.args) ap.push_back(dev_ptr(cells_[a].voff));
-        for (CellPtr o : e.outs) op.push_back(dev_ptr(cells_[o].voff));
+        for (CellPtr a : args) ap.push_back(dev_ptr(cells_[a].voff));
+        for (CellPtr o : outs) op.push_back(dev_ptr(cells_[o].voff));
         hipEvent_t e0 = ev0_, e1 = ev1_;
         int timing = timing_;
         std::string key;
         if (timing == 2) {
-            key = sp.key(aty, e.acc_mask);
+            key = sp.key(aty, acc_mask);
             if (!timing_filter_.empty() && key.compare(0, timing_filter_.size(), timing_filter_) != 0)
                 timing = 0;
             else if (timing_seen_++ % (uint64_t)timing_every_ != 0)
@@ -1378,18 +1395,18 @@ int Ctx::run_entry(const Entry &e)
             // an output that is accumulated into read as well
             uint64_t b = 0;
             for (auto &t : aty) b += t.bytes();
-            for (size_t k = 0; k < oty.size(); k++) b += oty[k].bytes() * (((e.acc_mask >> k) & 1) ? 2 : 1);
-            op_bytes_[timing == 2 ? key : sp.key(aty, e.acc_mask)] = b;
+            for (size_t k = 0; k < oty.size(); k++) b += oty[k].bytes() * (((acc_mask >> k) & 1) ? 2 : 1);
+            op_bytes_[timing == 2 ? key : sp.key(aty, acc_mask)] = b;
         }
         if (timing) hipEventRecord(e0, stream_);
-        rc = sp.run(*this, aty, ap.data(), oty, op.data(), e.acc_mask,
+        rc = sp.run(*this, aty, ap.data(), oty, op.data(), acc_mask,
                     ws_off == kNoOffset ? nullptr : dev_ptr(ws_off), ws_bytes);
         if (timing) hipEventRecord(e1, stream_);
         if (timing == 1 && !rc) {
             hipEventSynchronize(e1);
             float ms = 0;
             hipEventElapsedTime(&ms, e0, e1);
-            auto &t = times_[sp.key(aty, e.acc_mask)];
+            auto &t = times_[sp.key(aty, acc_mask)];
             t.first += ms;
             t.second++;
         }
@@ -1397,12 +1414,12 @@ int Ctx::run_entry(const Entry &e)
     }
     if (ws_off != kNoOffset) pool_.free(ws_off);      // reuse is ordered on the stream
     if (!rc)
-        for (CellPtr o : e.outs) {
+        for (CellPtr o : outs) {
             cells_[o].v_valid = true;
             cells_[o].h_valid = false;
         }
-    for (CellPtr a : e.args) cells_[a].pin--;
-    for (CellPtr o : e.outs) cells_[o].pin--;
+    for (CellPtr a : args) cells_[a].pin--;
+    for (CellPtr o : outs) cells_[o].pin--;
     return rc;
 }
 

@@ -118,6 +118,10 @@ struct ThunkSpec {
     virtual int run(Ctx &ctx, const std::vector<CellType> &aty, void *const *a,
                     const std::vector<CellType> &oty, void *const *o, uint32_t acc_mask,
                     void *ws, size_t ws_bytes) const = 0;
+    // A thunk of several independent products: how many, and product i as a thunk by itself with the arguments it reads
+    // (its output is output i).  They run one after another where the pool has no room for the cells of all.
+    virtual int pieces() const { return 1; }
+    virtual std::unique_ptr<ThunkSpec> piece(int, const std::vector<CellPtr> &, std::vector<CellPtr> *) const { return nullptr; }
     // out_adj[k] = adjoint cell of output k or 0; stage contributions through ctx.adj_*
     virtual int pop_adj(Ctx &, const Entry &, const std::vector<CellPtr> &) const { return 0; }
 };
@@ -251,6 +255,7 @@ class Ctx {
 
    private:
     int run_entry(const Entry &e);
+    int run_thunk(const ThunkSpec &sp, const std::vector<CellPtr> &args, const std::vector<CellPtr> &outs, uint32_t acc_mask);
     int host_alloc(Cell &c);
     void host_free(Cell &c);
     hipEvent_t ev_get();
@@ -271,6 +276,7 @@ class Ctx {
     size_t eager_left_ = 0, cyc_eager_ = 0, prev_eager_ = 0, cyc_demand_down_ = 0, cyc_dropped_ = 0;
     bool in_eager_ = false;
     size_t stable_end_ = 0;                                      // one past the largest id a stable cell has had
+    bool quiet_oom_ = false;                                     // an exhausted pool is not the last word: no report
     size_t pf_cursor_ = 0;                                       // entries before it have had their far prefetch
     int spill_eagerly(const Entry &e);
     int upload_ahead(Cell &c, bool *ordered);                    // one cell, on the upload stream

@@ -358,6 +358,12 @@ struct WgradNSpec : ThunkSpec {
         }
         return cacti_hip_gemm_f16_batched(1, 0, n, N, K, Sq, 1.f, A, N, B, K, (acc & 1) ? 1.f : 0.f, C, K, S(c));
     }
+    int pieces() const override { return n; }
+    std::unique_ptr<ThunkSpec> piece(int i, const std::vector<CellPtr> &a, std::vector<CellPtr> *in) const override
+    {
+        *in = {a[(size_t)i], a[(size_t)n]};
+        return make_matmul(true, false, 1.f);
+    }
     std::string key(const std::vector<CellType> &aty, uint32_t acc) const override
     {
         char buf[128];
@@ -398,6 +404,12 @@ struct ProjNSpec : ThunkSpec {
             C[i] = o[i];
         }
         return cacti_hip_gemm_f16_batched(0, 1, n, Sq, N, K, 1.f, A, K, B, K, 0.f, C, N, S(c));
+    }
+    int pieces() const override { return n; }
+    std::unique_ptr<ThunkSpec> piece(int i, const std::vector<CellPtr> &a, std::vector<CellPtr> *in) const override
+    {
+        *in = {a[0], a[(size_t)(1 + i)]};
+        return make_matmul(false, true, 1.f);
     }
     std::string key(const std::vector<CellType> &aty, uint32_t) const override
     {

@@ -142,6 +142,22 @@ def test_capped_pool_spills_and_matches(oracle, pagelocked):
     m.close(); ctx.close()
 
 
+def test_grouped_products_run_one_by_one_in_a_pool_too_small_for_the_group():
+    """The three projections of a layer and their weight gradients are one thunk each by default; a pool with room for
+    one weight matrix of 2 MiB at a time, but not for three, runs them one after another, with the same bits."""
+    wide = dict(S=136, D=1024, H=8, Dh=128, F=1024, V=1024, L=1, eps=1e-6)
+    cfg, flat, tok, lm_tok, scale = make_inputs(wide, seed=8, norm_mean=1.0, grad_scale=1024.0)
+    got = []
+    for pool in (1 << 30, 5 << 20):
+        ctx, m = _model(cfg, pool_bytes=pool)
+        m.put_params_flat(flat)
+        got.append((m.step(tok, lm_tok, scale), m.grads()))
+        m.close(); ctx.close()
+    assert np.array_equal(got[0][0], got[1][0])
+    for n, g in got[1][1].items():
+        assert np.array_equal(g.view(np.uint16), got[0][1][n].view(np.uint16)), n
+
+
 def test_attention_scratch_gives_way_to_a_capped_pool(oracle):
     """A pool with room for the least scratch of the attention adjoint, but not for what it is fastest with (26 MB of fp32
     partial sums at 1024 positions, 4 heads of 100): the cycle runs, with the results of the larger pool up to the
