@@ -1810,7 +1810,7 @@ CACTI_API size_t cacti_hip_attention_bwd_workspace(int64_t S, int64_t H)
 }
 
 static int attention_fwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k, const void *v, int64_t ld, void *o,
-                         void *stats, bool exact, hipStream_t st)
+                         void *stats, bool exact, bool windows, hipStream_t st)
 {
     int rc = check_shape("attention_fwd", S, H, Dh, ld);
     if (rc) return rc;
@@ -1823,24 +1823,27 @@ static int attention_fwd(int64_t S, int64_t H, int64_t Dh, float alpha, const vo
     p.out = (half_t *)o;
     p.m = (float *)stats;
     p.l = p.m + S * H;
-    int64_t span;
-    const bool dma = direct_tiles(H, Dh, ld, {q, k, v, o}, &span);
+    int64_t span = Dh;
+    const bool dma = (windows || Dh % 8 == 0) && direct_tiles(H, Dh, ld, {q, k, v, o}, &span);
     return dispatch<Fwd>(span, exact, dma, p, st);
 }
 
 CACTI_API int cacti_hip_attention_fwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,
                                       const void *v, int64_t ld, void *o, void *stats, void *stream)
 {
-    return attention_fwd(S, H, Dh, alpha, q, k, v, ld, o, stats, g_exact.load(std::memory_order_relaxed) != 0, (hipStream_t)stream);
+    return attention_fwd(S, H, Dh, alpha, q, k, v, ld, o, stats, g_exact.load(std::memory_order_relaxed) != 0, true, (hipStream_t)stream);
 }
 
 namespace cacti {
 
-// the exactly rounded form whatever the process-wide setting, for the cached forward pass
+// For the cached forward pass: the exactly rounded form whatever the process-wide setting, and every head by its own
+// elements alone, as with scores, softmax and P V apart.  Heads that start between 16-byte boundaries then come through
+// registers: a window of 16-byte pieces holds 4 elements of the next head, and a key of -infinity there (a score of
+// -infinity, a probability of 0 in its own head) would make this head's scores NaN.
 int attention_fwd_exact(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k, const void *v, int64_t ld, void *o,
                         void *stats, hipStream_t st)
 {
-    return attention_fwd(S, H, Dh, alpha, q, k, v, ld, o, stats, true, st);
+    return attention_fwd(S, H, Dh, alpha, q, k, v, ld, o, stats, true, false, st);
 }
 
 }  // namespace cacti

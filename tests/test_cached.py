@@ -291,6 +291,33 @@ def test_cached_pass_in_one_call_matches_the_training_forward_pass(oracle):
 
 
 @pytest.mark.gpu
+def test_an_infinite_key_stays_in_its_head(oracle):
+    """A long prompt on heads of 100 (every other head starts between two 16-byte boundaries), one key of which is -infinity
+    in the last column of head 0, 4 columns from head 1: its scores are -infinity and its probability 0 in head 0, and
+    no other head sees it, as in the oracle's chain of separate products."""
+    from cacti_amd.runtime import LlamaCached
+    from tests.llama_ref import make_inputs
+    cfg, flat, tok, lm_tok, scale = make_inputs(dict(S=200, D=400, H=4, Dh=100, F=416, V=256, L=1, eps=1e-6), seed=3, norm_mean=1.0)
+    p = {n: w.copy() for n, w in oracle.split_params(cfg, flat).items()}
+    p["embed"][:, 0], p["embed"][:, 399] = 1.0, 0.0
+    p["embed"][7, 399] = 8.0                                       # token 7 alone has a key beyond the range of f16
+    p["l0.q"][[49, 99]], p["l0.k"][99] = 0.0, 0.0
+    p["l0.q"][49, 0], p["l0.q"][99, 0], p["l0.k"][99, 399] = -1.0, 1.0, -60000.0
+    tok[tok == 7] = 8
+    tok[3] = 7
+    flat = np.concatenate([p[n].ravel() for n in p])
+    kc, vc = oracle.llama_cached_state(cfg)
+    want = oracle.llama_cached_apply(cfg, flat, kc, vc, tok.copy(), 0, cfg.S)["logit"]
+    assert np.isinf(kc).sum() == 2 and np.isfinite(want.astype(np.float32)).all()
+    ctx, m = _gpu_model(cfg, flat)
+    k = LlamaCached(m, cfg.S)
+    k.set_tokens(tok)
+    k.apply(0, cfg.S)
+    assert_parity(k.outputs()["logit"], want, "logit")
+    k.close(); m.close(); ctx.close()
+
+
+@pytest.mark.gpu
 def test_greedy_generation_feeds_its_own_tokens(oracle):
     """The deploy loop (examples/open_llama_3b_deploy.rs:195-206): prompt, then one position per
     cycle; every cycle's input token is the previous cycle's arg max (asserted by the example), the
