@@ -1467,9 +1467,14 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split)
     const int64_t kt = (K + BK - 1) / BK, cus = cu_count();
     GemmPlan best = {T64, T64, 0, 1};
     double best_cost = 1e30;
-    // A small output has at most 64 tiles of 64 x 64, the shape that is best for it.  The device is nowhere near its power
-    // limit there, so the instruction is free to be the one whose sums the register path has always formed.
-    const bool small = M * N <= kSmallOutput;
+    // A small output has about 64 tiles of 64 x 64 (or one row or column of them), the shape that is best for it while they
+    // run on the device all at once; more of them are cut by cost like any other product (measured, 64 x 64 -> by cost: 16
+    // products of 512 x 512 x 1024 19.3 -> 13.6 us, 32 of them 37.2 -> 23.0, 64 of 512 x 512 x 192 30.8 -> 18.9; at 8, 512
+    // tiles, both are 10.4).  The device is nowhere near its power limit with a small output, so the instruction is free to be
+    // the one whose sums the register path has always formed.  Up to kMaxPtrBatch products in a launch go by the
+    // single product alone: a group has the bits of separate launches.
+    const int64_t tiles64 = (M + 63) / 64 * ((N + 63) / 64);
+    const bool small = M * N <= kSmallOutput && (nz <= kMaxPtrBatch || tiles64 * nz <= kTileCost[T64].resident * cus);
     if (small) {
         best = {T64_SMALL, T64, 0, 1};
         best_cost = tile_cost(T64, M, N, nz, kt);

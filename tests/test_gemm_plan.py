@@ -1,0 +1,33 @@
+"""How products are cut into tiles (cacti_hip_gemm_plan; no GPU: the device is taken to have 256 CUs then)."""
+import ctypes as C
+
+import pytest
+
+from cacti_amd import ffi
+
+
+def plan(M, N, K, nz):
+    out = (C.c_int64 * 6)()
+    assert ffi.lib().cacti_hip_gemm_plan(M, N, K, nz, out) == 0
+    return list(out)
+
+
+@pytest.mark.parametrize("nz", [1, 2, 3, 4, 8])
+def test_small_outputs_take_64_by_64_tiles_while_those_fit_the_device(nz):
+    assert plan(512, 512, 1024, nz)[:2] == [64, 64]
+    assert plan(1024, 256, 128, nz)[:2] == [64, 64]
+    assert plan(128, 256, 688, nz)[:2] == [64, 64]
+
+
+@pytest.mark.parametrize("M,N,K,nz", [(512, 512, 1024, 16), (512, 512, 1024, 32), (512, 512, 192, 64), (256, 1024, 4096, 32)])
+def test_many_small_outputs_are_cut_by_cost(M, N, K, nz):
+    """More 64 x 64 tiles than the device runs at once: tiles of twice the side need fewer rounds per k tile."""
+    p = plan(M, N, K, nz)
+    assert p[0] * p[1] > 64 * 64 and p[5] == 1
+
+
+def test_a_group_is_cut_by_the_same_rule_as_its_products():
+    """Small or not is decided for one product where up to four share a launch, so that a group has the bits of its
+    products' own launches."""
+    for M, N in ((128, 688), (688, 256), (1024, 256), (5, 20000), (512, 512)):
+        assert all(plan(M, N, 256, nz)[:2] == [64, 64] for nz in (1, 2, 3, 4))

@@ -428,6 +428,24 @@ def test_gemm_pointer_array_batch(ops, oracle, ta, tb, n, M, N, K, off):
             assert np.array_equal(host(dC[z]).view(np.uint16), single.view(np.uint16)), z
 
 
+@pytest.mark.parametrize("tb,n,M,N,K", [(1, 16, 264, 520, 200), (0, 16, 264, 520, 200), (1, 33, 512, 512, 192), (0, 70, 128, 256, 136)])
+def test_gemm_batch_of_many_small_outputs(ops, tb, n, M, N, K):
+    """More 64 x 64 tiles than run at once, against fp32 torch (the bar of the random shapes above: f16 rounding of the result)."""
+    say("gemm batch of small outputs", tb, n, M, N, K)
+    torch.manual_seed(n + M)
+    A = torch.randn(n, M, K, device="cuda").half()
+    B = (torch.randn((n, N, K) if tb else (n, K, N), device="cuda") * 0.1).half()
+    for beta in (0.0, 1.0):
+        C0 = torch.randn(n, M, N, device="cuda").half()
+        got = C0.clone()
+        ops.gemm_strided_batched(False, bool(tb), n, M, N, K, 1.0, A, K, M * K, B, K if tb else N, N * K, beta, got, N, M * N)
+        for z in range(n):
+            ref = A[z].float() @ (B[z].float().T if tb else B[z].float()) + beta * C0[z].float()
+            err = ((got[z].float() - ref).norm() / ref.norm()).item()
+            mx = ((got[z].float() - ref).abs().max() / ref.abs().max()).item()
+            assert err < 6e-4 and mx < 4e-3, (z, beta, err, mx)
+
+
 @pytest.mark.parametrize("case", ["fwd", "dgrad", "wgrad"])
 def test_gemm_projection_shapes(ops, oracle, case):
     """The three GEMMs of one projection at a reduced token count (oracle finishes in seconds)."""
