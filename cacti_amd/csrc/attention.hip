@@ -67,7 +67,6 @@ constexpr int kTileRows = 64;
 constexpr int kTileB = kTileRows * kRowB;   // 16 KB
 constexpr int kNT = 256;                 // threads of a wave group (4 waves): the unit that loads a tile
 constexpr int kBM = 128;                 // rows of the fixed operand per wave group (32 per wave)
-constexpr int kCus = 256;
 constexpr float kSpread = 8.f;           // least row sum of exponentials for the short form of sigma (dQ kernel)
 
 struct AttnArgs {
@@ -1675,7 +1674,7 @@ struct DkvParts {
 DkvParts dkv_parts(int64_t S, int64_t H)
 {
     const int64_t groups = (S + kBM - 1) / kBM * H, tiles = (S + kTileRows - 1) / kTileRows;
-    int64_t split = std::min<int64_t>(kCus / groups, 8);
+    int64_t split = std::min<int64_t>(device_cus() / groups, 8);
     if (split < 2) return {1, (int)tiles};
     const int64_t per = std::max<int64_t>(2, (tiles + split - 1) / split);
     if (tiles - per < 5) return {1, (int)tiles};

@@ -39,6 +39,8 @@ void module_epoch_advance();
 // streams and events behind its back, so the reset entry point refuses while any exists
 int live_contexts(int dev);
 void live_contexts_add(int dev, int n);
+// compute units of the current device (256 where there is none)
+int device_cus();
 struct DeviceOnce {
     int dev = -1;
     unsigned epoch = 0;

@@ -28,6 +28,19 @@ void live_contexts_add(int dev, int n)
     if (dev >= 0 && dev < 64) g_live_contexts[dev].fetch_add(n);
 }
 
+int device_cus()
+{
+    static std::atomic<int> known[64];
+    int dev = -1, n = 0;
+    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) {
+        n = known[dev].load(std::memory_order_relaxed);
+        if (!n && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) known[dev].store(n);
+    }
+    if (n > 0) return n;
+    (void)hipGetLastError();
+    return 256;
+}
+
 int hip_status(hipError_t e, const char *what)
 {
     if (e == hipSuccess) return 0;

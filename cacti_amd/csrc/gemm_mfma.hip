@@ -1422,22 +1422,10 @@ constexpr TileCost kTileCost[N_TILES] = {
 
 constexpr int64_t kSmallOutput = 1 << 18;
 
-int cu_count()
-{
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-            cus = 256;
-    }
-    return cus;
-}
-
-double tile_cost(int tile, int64_t M, int64_t N, int64_t nz, int64_t ktiles)
+double tile_cost(int64_t cus, int tile, int64_t M, int64_t N, int64_t nz, int64_t ktiles)
 {
     const TileCost &t = kTileCost[tile];
-    const int64_t wg = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn) * nz, cus = cu_count(), set = cus * t.resident;
+    const int64_t wg = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn) * nz, set = cus * t.resident;
     const int64_t sets = wg / set;
     const double rest = (double)(wg - sets * set) / (double)cus;
     const double last = rest == 0 ? 0 : rest <= 1 ? t.first + t.load * rest : t.full;
@@ -1464,7 +1452,7 @@ void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn)
 // 8 bytes per part and element).
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split)
 {
-    const int64_t kt = (K + BK - 1) / BK, cus = cu_count();
+    const int64_t kt = (K + BK - 1) / BK, cus = device_cus();
     GemmPlan best = {T64, T64, 0, 1};
     double best_cost = 1e30;
     // A small output has about 64 tiles of 64 x 64 (or one row or column of them), the shape that is best for it while they
@@ -1477,10 +1465,10 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split)
     const bool small = M * N <= kSmallOutput && (nz <= kMaxPtrBatch || tiles64 * nz <= kTileCost[T64].resident * cus);
     if (small) {
         best = {T64_SMALL, T64, 0, 1};
-        best_cost = tile_cost(T64, M, N, nz, kt);
+        best_cost = tile_cost(cus, T64, M, N, nz, kt);
     }
     for (int t = 0; t < N_TILES && !small; t++) {
-        const double c = tile_cost(t, M, N, nz, kt);
+        const double c = tile_cost(cus, t, M, N, nz, kt);
         if (c < best_cost) {
             best_cost = c;
             best = {t, T64, 0, 1};
@@ -1491,7 +1479,7 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split)
         const int64_t cols = tiles_m * tiles_n / cus * cus / tiles_m * bn;
         if (cols <= 0 || cols >= N) continue;
         for (int r = T64; r <= T128; r++) {
-            const double c = tile_cost(t, M, cols, nz, kt) + tile_cost(r, M, N - cols, nz, kt);
+            const double c = tile_cost(cus, t, M, cols, nz, kt) + tile_cost(cus, r, M, N - cols, nz, kt);
             if (c < best_cost) {
                 best_cost = c;
                 best = {t, r, cols, 1};
@@ -1503,7 +1491,7 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split)
             for (int s = 2; s <= 8; s++) {
                 const int64_t per = (kt + s - 1) / s;
                 if (per < 4 || (kt + per - 1) / per != s) continue;           // parts of some length, none empty
-                const double c = tile_cost(t, M, N, s, per) + 4.0 + (double)(M * N) * s * 8.0 / 4e6;
+                const double c = tile_cost(cus, t, M, N, s, per) + 4.0 + (double)(M * N) * s * 8.0 / 4e6;
                 if (c < best_cost) {
                     best_cost = c;
                     best = {t, T64, 0, s};

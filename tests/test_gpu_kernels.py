@@ -726,3 +726,18 @@ def test_attention_bwd_in_parts(ops, S, H, Dh, acc):
     for a, b in zip(got[1:], want[1:]):
         # fp32 sums of the same terms in another order, rounded once: a last place (2^-11 of it) here and there
         assert rel_l2(host(a), host(b)) < 2e-4 and exact_frac(host(a), host(b)) > 0.95
+
+
+@pytest.mark.parametrize("S,H,Dh", [(611, 16, 64), (449, 3, 100), (1000, 2, 128), (1025, 8, 100), (2048, 32, 100), (128, 4, 64)])
+def test_attention_bwd_parts_fill_this_device(S, H, Dh):
+    """As many parts as this device has compute units for, whatever their number, and at most 8."""
+    from cacti_amd import ffi
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    tiles, split = -(-S // 64), min(cus // (-(-S // 128) * H), 8)
+    least = ffi.lib().cacti_hip_attention_bwd_workspace(S, H)
+    want = least
+    if split >= 2:
+        per = max(2, -(-tiles // split))
+        if tiles - per >= 5:
+            want = -(-least // 16) * 16 + -(-tiles // per) * 2 * H * S * Dh * 4
+    assert ffi.lib().cacti_hip_attention_bwd_workspace_best(S, H, Dh) == want
