@@ -269,13 +269,16 @@ PyObject *gemm_batched(PyObject *const *v)
     require(n > 0 && bs.size() == n && outs.size() == n, "gemm_batched: lists of one length expected");
     const at::Tensor &a = as[0], &b = bs[0], &o = outs[0];
     const Shape s = product_shape(a, b, ta, tb);
-    for (int64_t x : {a.size(1), b.size(1), s.N, a.stride(0), b.stride(0), o.stride(0)})
-        if (x % 8) {
-            // rows that are not 16-byte aligned run one after another; each may want a workspace
-            for (size_t z = 0; z < n; z++) gemm_into(ta, tb, s.M, s.N, s.K, alpha, as[z], bs[z], beta, outs[z]);
-            Py_RETURN_NONE;
-        }
     const std::vector<void *> pa = as.pointers(), pb = bs.pointers(), po = outs.pointers();
+    bool aligned = true;
+    for (int64_t x : {a.size(1), b.size(1), s.N, a.stride(0), b.stride(0), o.stride(0)}) aligned = aligned && x % 8 == 0;
+    for (const std::vector<void *> *v : {&pa, &pb, &po})
+        for (void *p : *v) aligned = aligned && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+    if (!aligned) {
+        // operands whose rows are not all 16-byte aligned run one after another; each may want a workspace
+        for (size_t z = 0; z < n; z++) gemm_into(ta, tb, s.M, s.N, s.K, alpha, as[z], bs[z], beta, outs[z]);
+        Py_RETURN_NONE;
+    }
     void *st = stream();
     run([&] {
         return cacti_hip_gemm_f16_batched(ta, tb, (int64_t)n, s.M, s.N, s.K, alpha, pa.data(), a.stride(0), pb.data(), b.stride(0), beta,

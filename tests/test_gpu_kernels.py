@@ -428,6 +428,38 @@ def test_gemm_pointer_array_batch(ops, oracle, ta, tb, n, M, N, K, off):
             assert np.array_equal(host(dC[z]).view(np.uint16), single.view(np.uint16)), z
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0), (0, 0)])
+@pytest.mark.parametrize("off", [1, 4])
+def test_gemm_operands_that_start_between_16_byte_boundaries(ops, oracle, ta, tb, off):
+    """Rows that are multiples of 8 elements, every array `off` elements past a boundary (slices of larger tensors): a batch
+    takes the way of its single products, an aligned copy and the direct kernels, bit for bit; C is written where it
+    is, with nothing beside it touched."""
+    say("gemm odd bases", ta, tb, off)
+    n, M, N, K = 2, 520, 616, 264
+    r = rng(310 + 2 * ta + tb + off)
+    As = [randn16(r, (K, M) if ta else (M, K)) for _ in range(n)]
+    Bs = [randn16(r, (N, K) if tb else (K, N), 0.1) for _ in range(n)]
+    C0 = randn16(r, (M, N))
+
+    def place(x):
+        buf = torch.full((x.size + 16,), 7.0, dtype=torch.float16, device="cuda")
+        buf[off:off + x.size] = dev(x).view(-1)
+        return buf, buf[off:off + x.size].view(x.shape)
+    dA, dB = [place(x)[1] for x in As], [place(x)[1] for x in Bs]
+    assert dA[0].data_ptr() % 16 == 2 * off
+    for alpha, beta in [(1.0, 0.0), (0.5, 1.0)]:
+        dC = [place(C0) for _ in range(n)]
+        ops.gemm_batched(dA, dB, bool(ta), bool(tb), alpha, beta, [c for _, c in dC])
+        for z in range(n):
+            want = oracle.matmul(ta, tb, As[z], Bs[z], alpha, beta, C0)
+            assert_parity(host(dC[z][1]), want, "odd base %d" % z)
+            assert exact_frac(host(dC[z][1]), want) > 0.97
+            one = place(C0)[1]
+            ops.gemm(dA[z], dB[z], bool(ta), bool(tb), alpha, beta, one)
+            assert_bits(host(dC[z][1]), host(one), "batch and single product")
+            assert (dC[z][0][:off] == 7.0).all() and (dC[z][0][off + M * N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("tb,n,M,N,K", [(1, 16, 264, 520, 200), (0, 16, 264, 520, 200), (1, 33, 512, 512, 192), (0, 70, 128, 256, 136)])
 def test_gemm_batch_of_many_small_outputs(ops, tb, n, M, N, K):
     """More 64 x 64 tiles than run at once, against fp32 torch (the bar of the random shapes above: f16 rounding of the result)."""
