@@ -217,9 +217,7 @@ int run(int64_t n, const void *x, void *out, hipStream_t st)
 }  // namespace
 
 namespace cacti {
-size_t digest_batch_scratch_bytes(int count);
-int digest_batch_f16(int count, const void *const *xs, const int64_t *ns, void *out, void *segs_dev,
-                     hipStream_t st);
+int digest_batch_f16(int count, const void *const *xs, const int64_t *ns, void *out, hipStream_t st);
 }  // namespace cacti
 
 CACTI_API int cacti_hip_nan_count_f16(int64_t n, const void *x, void *count_i64, void *stream)
@@ -239,28 +237,23 @@ CACTI_API int cacti_hip_abs_log2_hist8_f16(int64_t n, const void *x, void *hist_
     return run<true, false>(n, x, hist_i64_256, (hipStream_t)stream);
 }
 
-CACTI_API size_t cacti_hip_digests_scratch_bytes(int count)
-{
-    return count > 0 ? cacti::digest_batch_scratch_bytes(count) : 0;
-}
+CACTI_API size_t cacti_hip_digests_scratch_bytes(int) { return 0; }
 
 CACTI_API int cacti_hip_digests_f16_batch(int count, const void *const *xs, const int64_t *ns, void *out_i64,
-                                          void *scratch, void *stream)
+                                          void *, void *stream)
 {
     CACTI_REQUIRE(count >= 0, CACTI_E_INVALID, "digests_batch: negative count");
     if (count == 0) return 0;
     CACTI_REQUIRE(xs && ns && out_i64 && aligned(out_i64, 8), CACTI_E_INVALID,
                   "digests_batch: null or misaligned argument");
-    return cacti::digest_batch_f16(count, xs, ns, out_i64, scratch, (hipStream_t)stream);
+    return cacti::digest_batch_f16(count, xs, ns, out_i64, (hipStream_t)stream);
 }
 
 namespace cacti {
 
 // Both digests of `count` tensors, up to kSegsPerLaunch of them in a launch: out[257 * i + 0..255] = histogram and
 // out[257 * i + 256] = NaN count of tensor i.  xs[i] 16-byte aligned, ns[i] >= 0.
-size_t digest_batch_scratch_bytes(int) { return 16; }           // (not used any more; callers allocate it)
-
-int digest_batch_f16(int count, const void *const *xs, const int64_t *ns, void *out, void *, hipStream_t st)
+int digest_batch_f16(int count, const void *const *xs, const int64_t *ns, void *out, hipStream_t st)
 {
     if (count <= 0) return 0;
     for (int i = 0; i < count; i++)

@@ -314,12 +314,12 @@ CACTI_API int cacti_adamw32_scalars(int iter_nr, float grad_scale, float lr, flo
     return 0;
 }
 
-CACTI_API size_t cacti_hip_adamw32_scratch_bytes(int count) { return count > 0 ? 16 : 0; }   // (not used any more)
+CACTI_API size_t cacti_hip_adamw32_scratch_bytes(int) { return 0; }
 
 CACTI_API int cacti_hip_adamw32_step_f16_batch(int count, const void *const *grads_f16, void *const *avgs_f32,
                                                void *const *avg2s_f32, void *const *masters_f32,
                                                void *const *params_f16, const int64_t *ns, const float *scalars7,
-                                               void *scratch, void *stream)
+                                               void *, void *stream)
 {
     CACTI_REQUIRE(count >= 0, CACTI_E_INVALID, "adamw32_step: negative count");
     if (count == 0) return 0;

@@ -409,9 +409,7 @@ int Ctx::cell_get(CellPtr ci, void *host, size_t bytes)
 }
 
 // csrc/digest.hip
-size_t digest_batch_scratch_bytes(int count);
-int digest_batch_f16(int count, const void *const *xs, const int64_t *ns, void *out, void *segs_dev,
-                     hipStream_t st);
+int digest_batch_f16(int count, const void *const *xs, const int64_t *ns, void *out, hipStream_t st);
 
 // One launch digests every cell: all of them are made resident first (a cell that cannot be
 // held beside the others fails the call with the pool's error).
@@ -419,10 +417,10 @@ int Ctx::cells_digest(const CellPtr *cells, int n, int64_t *hist, int64_t *nan)
 {
     CACTI_REQUIRE(n >= 0 && (n == 0 || (cells && hist && nan)), CACTI_E_INVALID, "cells_digest: null argument");
     if (n == 0) return 0;
-    // device scratch: per cell 256 histogram bins + the NaN count, then the launch's descriptors
+    // device scratch: per cell 256 histogram bins + the NaN count
     const size_t out_bytes = (size_t)n * 257 * sizeof(int64_t);
     size_t off;
-    int rc = pool_alloc(out_bytes + digest_batch_scratch_bytes(n), &off);
+    int rc = pool_alloc(out_bytes, &off);
     if (rc) return rc;
     char *scratch = static_cast<char *>(dev_ptr(off));
     std::vector<const void *> xs((size_t)n);
@@ -451,8 +449,7 @@ int Ctx::cells_digest(const CellPtr *cells, int n, int64_t *hist, int64_t *nan)
             m++;
         }
         if (rc == 0 && m > 0)
-            rc = digest_batch_f16(m, xs.data(), ns.data(), scratch + (size_t)done * 257 * sizeof(int64_t),
-                                  scratch + out_bytes, stream_);
+            rc = digest_batch_f16(m, xs.data(), ns.data(), scratch + (size_t)done * 257 * sizeof(int64_t), stream_);
         for (int i = done; i < done + m; i++) cells_[cells[i]].pin--;
         if (rc == 0 && m == 0) rc = CACTI_E_OOM;
         done += m;
@@ -610,9 +607,7 @@ int Ctx::cells_adamw32(int n, const CellPtr *grads, const CellPtr *avgs, const C
     CACTI_REQUIRE(n >= 0 && (n == 0 || (grads && avgs && avg2s && masters && params && sc)), CACTI_E_INVALID,
                   "cells_adamw32: null argument");
     if (n == 0) return 0;
-    size_t off;
-    int rc = pool_alloc(cacti_hip_adamw32_scratch_bytes(n), &off);
-    if (rc) return rc;
+    int rc = 0;
     std::vector<const void *> g((size_t)n);
     std::vector<void *> a((size_t)n), b((size_t)n), w((size_t)n), p((size_t)n);
     std::vector<int64_t> ns((size_t)n);
@@ -654,7 +649,7 @@ int Ctx::cells_adamw32(int n, const CellPtr *grads, const CellPtr *avgs, const C
         }
         if (rc == 0 && m > 0)
             rc = cacti_hip_adamw32_step_f16_batch(m, g.data(), a.data(), b.data(), w.data(), p.data(), ns.data(), sc,
-                                                  dev_ptr(off), stream_);
+                                                  nullptr, stream_);
         for (int i = done; i < done + m; i++) {
             const CellPtr five[5] = {grads[i], avgs[i], avg2s[i], masters[i], params[i]};
             for (int k = 0; k < 5; k++) cells_[five[k]].pin--;
@@ -667,7 +662,6 @@ int Ctx::cells_adamw32(int n, const CellPtr *grads, const CellPtr *avgs, const C
         if (rc == 0 && m == 0) rc = CACTI_E_OOM;
         done += m;
     }
-    pool_.free(off);                                             // reuse is ordered on the stream
     return rc;
 }
 

@@ -426,8 +426,8 @@ int cacti_hip_abs_log2_hist8_f16(int64_t n, const void *x, void *hist_i64_256, v
  * over all parameters and gradients, examples/open_llama_3b_train.rs:409-424, as one call):
  * out_i64[257 * i + b] = abs_log2_hist8 class b of tensor i, out_i64[257 * i + 256] = its NaN
  * count.  xs[i] (device, 16-byte aligned) holds ns[i] >= 0 f16 elements; xs and ns are host
- * arrays read before the call returns.  out_i64 (count * 257 values) and scratch
- * (cacti_hip_digests_scratch_bytes(count) bytes) are device memory, 8-byte aligned. */
+ * arrays read before the call returns.  out_i64 (count * 257 values) is device memory, 8-byte aligned.  The tensors'
+ * table travels with the launch: scratch is not looked at (null will do) and takes 0 bytes. */
 size_t cacti_hip_digests_scratch_bytes(int count);
 int cacti_hip_digests_f16_batch(int count, const void *const *xs, const int64_t *ns, void *out_i64,
                                 void *scratch, void *stream);
@@ -467,8 +467,8 @@ int cacti_adamw32_scalars(int iter_nr, float grad_scale, float lr, float wd, flo
  * examples/open_llama_3b_train.rs:252-268), each element read and written once; bit-identical to
  * the four separate thunks.  grads (f16, read), avgs, avg2s, masters (f32, updated), params (f16,
  * written), ns (element counts) are host arrays of device pointers / sizes, read before the call
- * returns; scalars7 as cacti_adamw32_scalars fills it; scratch: device memory of
- * cacti_hip_adamw32_scratch_bytes(count) bytes, 8-byte aligned. */
+ * returns; scalars7 as cacti_adamw32_scalars fills it.  scratch is not looked at (null will
+ * do) and takes 0 bytes. */
 size_t cacti_hip_adamw32_scratch_bytes(int count);
 int cacti_hip_adamw32_step_f16_batch(int count, const void *const *grads_f16, void *const *avgs_f32,
                                      void *const *avg2s_f32, void *const *masters_f32,

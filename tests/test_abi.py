@@ -60,3 +60,10 @@ def test_edge_shapes_are_rejected_with_a_message():
     assert L.cacti_hip_rope_fwd(4, 2, 7, 16, 16, 16, 16, None) < 0                         # odd head dim
     assert L.cacti_hip_softmax_ce_bwd(0, 8, 16, 16, 16, 16, 0, None) == -1
     assert L.cacti_hip_embed_fwd(8, 8, 16, 0, 16, 16, 16, None) == -1                      # no positions
+
+
+def test_digests_and_adamw_need_no_scratch():
+    """Their tensor tables travel in the kernel arguments."""
+    L = ffi.lib()
+    for n in (0, 1, 64, 1000):
+        assert L.cacti_hip_digests_scratch_bytes(n) == 0 and L.cacti_hip_adamw32_scratch_bytes(n) == 0
