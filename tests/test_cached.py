@@ -135,6 +135,17 @@ def test_decoding_attention_matches_the_oracle_chain(oracle, T, H, Dh, Cc, row0)
         out.zero_()
 
 
+# Each way the positions and heads are cut: heads above 100; up to 320 positions on 256 lanes, up to 512 on 512 lanes with
+# their own scores (both edges), a scores launch beyond, for one row and for two to four; score rows of more than 32 KiB of
+# LDS (four rows from 4097 positions on) up to the most there can be; columns beyond the last row's position
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,Dh,Cc,row0", [(1, 16, 128, 69, 68), (2, 3, 104, 320, 318), (3, 2, 128, 321, 318), (1, 4, 128, 512, 511),
+                                            (1, 4, 100, 400, 399), (4, 2, 64, 513, 509), (2, 4, 128, 1540, 1538), (3, 2, 112, 700, 697),
+                                            (4, 2, 128, 4097, 4093), (4, 1, 128, 8192, 8188), (3, 1, 36, 8192, 8189), (2, 2, 120, 640, 333)])
+def test_decoding_attention_over_its_ranges(oracle, T, H, Dh, Cc, row0):
+    test_decoding_attention_matches_the_oracle_chain(oracle, T, H, Dh, Cc, row0)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,add,gate", [(1, 3200, 3200, False, False), (1, 8640, 3200, True, True), (2, 96, 256, True, False),
                                             (4, 250, 1024, False, True), (3, 32000, 3200, True, False), (1, 64, 8192, True, True),
@@ -181,6 +192,18 @@ def test_rows_norm_matmul_matches_the_separate_thunks(oracle, M, N, K, add, gate
     if not add and not gate:
         ffi.call("cacti_hip_rows_norm_matmul_f16", M, N, K, ptr(dx), None, None, 0.0, None, ptr(dB), None, out.data_ptr(), None)
         assert_parity(out.cpu().numpy().view(np.float16), oracle.matmul(0, 1, x, B), "rows matmul")
+
+
+# each way a row is cut over lanes and pieces (K / 8 pieces: up to 64, 128, 256, 512, 768 and more for one row, 512 for
+# two to four), at both edges
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,add,gate", [(1, 72, 512, True, False), (1, 72, 520, False, True), (1, 100, 1024, False, False),
+                                            (1, 100, 1032, True, True), (1, 64, 2048, False, True), (1, 130, 2056, False, False),
+                                            (1, 40, 4096, True, False), (1, 72, 4104, True, False), (1, 64, 6144, True, True),
+                                            (1, 64, 6152, False, True), (2, 64, 4096, True, True), (3, 40, 4104, False, True),
+                                            (4, 66, 8192, True, False)])
+def test_rows_norm_matmul_over_its_ranges(oracle, M, N, K, add, gate):
+    test_rows_norm_matmul_matches_the_separate_thunks(oracle, M, N, K, add, gate)
 
 
 @pytest.mark.gpu
@@ -230,6 +253,12 @@ def test_rows_qkv_rope_cache_matches_the_separate_thunks(oracle, M, H, Dh, add):
     assert np.mean(h16(out).view(np.uint16) == qr.view(np.uint16)) > 0.95
     if add:
         assert np.array_equal(sout.cpu().numpy().view(np.uint16), rsum.view(np.uint16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,H,Dh,add", [(1, 16, 128, True), (1, 12, 100, False), (1, 33, 128, True), (1, 50, 124, False), (3, 34, 124, True)])
+def test_rows_qkv_rope_cache_over_its_ranges(oracle, M, H, Dh, add):
+    test_rows_qkv_rope_cache_matches_the_separate_thunks(oracle, M, H, Dh, add)
 
 
 def _gpu_model(cfg, flat):
@@ -353,6 +382,36 @@ def test_greedy_generation_feeds_its_own_tokens(oracle):
         a, b = b, b + 1
     assert i >= 2
     k.close(); m.close(); ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first", [13, 20, 64])
+def test_reset_clears_every_row_that_was_written(oracle, first):
+    """A reset after part of the rows, then a longer pass over them: the bits of a model whose caches were never used (the
+    pass adds to the cache rows, so a row left behind would show)."""
+    from cacti_amd.runtime import LlamaCached
+    cfg, flat, tok, lm_tok, scale = _inputs(seed=8)
+    ctx, m = _gpu_model(cfg, flat)
+    used, fresh = LlamaCached(m, cfg.S), LlamaCached(m, cfg.S)
+
+    def passes(k):
+        out = []
+        for a, b in ((0, 33), (33, 34), (34, 38), (38, 80)):
+            k.set_tokens(tok[:80])                         # (teacher-forced: the appended token is overwritten)
+            k.apply(a, b)
+            out.append(k.outputs()["logit"])
+        return np.concatenate(out)
+
+    for _ in range(2):
+        for a, b in ((0, first - 1), (first - 1, first)):
+            used.set_tokens(np.roll(tok, 5)[:first])
+            used.apply(a, b)
+        used.outputs()
+        used.reset_state()
+    want = passes(fresh)
+    assert np.array_equal(passes(used).view(np.uint16), want.view(np.uint16))
+    for x in (used, fresh, m, ctx):
+        x.close()
 
 
 @pytest.mark.gpu

@@ -398,6 +398,16 @@ def test_gemm_few_rows_streams_the_weights(ops, oracle, M, N, K, pad):
         assert exact_frac(got, want) > 0.98
 
 
+# each way a row of K is cut over the lanes, at both edges (one row: 1 to 5 pieces per lane, then passes of four; two to four
+# rows: passes of two or four).  400 columns and more: fp32 sums of 10^4 terms in another order differ by some 1e-6 of a
+# typical result, which moves one f16 rounding (5e-4 apart) in 250; of 40 columns a single pair is 5 %.
+@pytest.mark.parametrize("M,N,K", [(1, 400, 8), (1, 400, 512), (1, 472, 520), (1, 500, 1032), (1, 466, 2048), (1, 464, 2056),
+                                   (1, 464, 4104), (1, 430, 6144), (1, 464, 6152), (1, 464, 8200), (1, 440, 10240), (1, 440, 10248),
+                                   (1, 424, 16392), (2, 464, 4096), (2, 464, 4104), (3, 440, 8200), (4, 466, 10248)])
+def test_gemm_few_rows_over_their_ranges(ops, oracle, M, N, K):
+    test_gemm_few_rows_streams_the_weights(ops, oracle, M, N, K, 0)
+
+
 @pytest.mark.parametrize("ta,tb,n,M,N,K,off", [(0, 1, 3, 1032, 1096, 192, 0), (1, 0, 2, 1096, 1032, 128, 0), (0, 0, 5, 1024, 1024, 192, 0),
                                              (0, 1, 3, 1032, 1096, 192, 4), (0, 1, 2, 64, 72, 40, 0)])
 def test_gemm_pointer_array_batch(ops, oracle, ta, tb, n, M, N, K, off):
@@ -426,6 +436,15 @@ def test_gemm_pointer_array_batch(ops, oracle, ta, tb, n, M, N, K, off):
             assert_parity(host(dC[z]), want, "gemm batched %d" % z)
             single = host(ops.gemm(dA[z], dB[z], bool(ta), bool(tb), alpha, beta, dev(C0[z])))
             assert np.array_equal(host(dC[z]).view(np.uint16), single.view(np.uint16)), z
+
+
+# a K that ends inside a k tile, as the weight gradients of a ragged sequence have it (any K where both operands are strided
+# in it); the smallest K the shared launch takes; outputs below and above the line of the small ones
+@pytest.mark.parametrize("ta,tb,n,M,N,K", [(1, 0, 3, 1032, 1096, 611), (1, 0, 2, 2056, 1032, 129), (0, 1, 3, 1032, 1096, 200),
+                                           (0, 0, 4, 520, 1024, 136), (1, 0, 3, 688, 256, 203), (1, 1, 2, 1032, 520, 264),
+                                           (0, 1, 5, 203, 1376, 520)])
+def test_gemm_pointer_array_batch_with_a_k_tail(ops, oracle, ta, tb, n, M, N, K):
+    test_gemm_pointer_array_batch(ops, oracle, ta, tb, n, M, N, K, 0)
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0), (0, 0)])

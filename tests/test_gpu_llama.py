@@ -65,10 +65,43 @@ def test_tiny_llama_step_all_gradients(oracle, attention):
 
 
 def test_grouped_products_are_the_separate_thunks_bit_for_bit():
-    """Small shapes (every product through the register path): the grouped stagings of the projections and
+    """Small shapes (outputs of at most 2^18 elements): the grouped stagings of the projections and
     of their weight gradients (modes 1 and 2) give the loss and all gradients of the separate matmul thunks
     (mode 0), bit for bit."""
     cfg, flat, tok, lm_tok, scale = make_inputs(TINY, seed=3, norm_mean=1.0, grad_scale=1024.0)
+    got = {}
+    for groups in (0, 1, 2):
+        ctx, m = _model(cfg)
+        m.set_product_groups(groups)
+        m.put_params_flat(flat)
+        got[groups] = (m.step(tok, lm_tok, scale), m.grads())
+        m.close(); ctx.close()
+    for groups in (1, 2):
+        assert np.array_equal(got[groups][0], got[0][0])
+        for n, g in got[groups][1].items():
+            assert np.array_equal(g.view(np.uint16), got[0][1][n].view(np.uint16)), (groups, n)
+
+
+# a sequence of odd length and products of more than 2^18 outputs: the weight gradients sum over 203 positions (a k tile of 64
+# ends inside them), and the forward products of the FFN and the head, and all weight gradients but the norms', are past the
+# line up to which the tiny model's products keep the instruction of the register path
+RAGGED = dict(S=203, D=544, H=8, Dh=68, F=1376, V=2048, L=1, eps=1e-6)
+
+
+def test_ragged_llama_step_all_gradients(oracle):
+    from tests.envelope import order_envelope
+    cfg, flat, tok, lm_tok, scale = make_inputs(RAGGED, seed=12, norm_mean=1.0, grad_scale=1024.0)
+    ref = oracle.llama_step(cfg, flat, tok, lm_tok, scale)
+    ctx, m = _model(cfg)
+    m.put_params_flat(flat)
+    assert_parity(m.step(tok, lm_tok, scale), ref["loss"], "loss", l2=1e-4, mx=1e-3)
+    _, env = order_envelope(oracle, cfg, flat, tok, lm_tok, scale)
+    _compare(oracle, cfg, m, ref, env, "ragged")
+    m.close(); ctx.close()
+
+
+def test_grouped_products_of_a_ragged_sequence_are_the_separate_thunks_bit_for_bit():
+    cfg, flat, tok, lm_tok, scale = make_inputs(RAGGED, seed=13, norm_mean=1.0, grad_scale=1024.0)
     got = {}
     for groups in (0, 1, 2):
         ctx, m = _model(cfg)

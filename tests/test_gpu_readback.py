@@ -98,6 +98,28 @@ def test_a_large_read_does_not_wait_for_another_contexts_stream():
         x.close()
 
 
+@pytest.mark.parametrize("V,D", [(20000, 1024), (8200, 1032), (24, 264)])
+def test_reads_of_several_windows_come_back_whole(V, D):
+    """41 MB in three windows of 16 MiB; 16.9 MB, a window and a few pieces, the last of them short; 13 KB in one gather.
+    Right behind an update on the device, so that the bytes are not the host's own copy."""
+    from cacti_amd.runtime import Ctx, Llama
+    ctx = Ctx(0, 1 << 30, True)
+    m = Llama(ctx, 16, D, 4, D // 4, 64, V, 0, 1e-6)
+    r = np.random.default_rng(V)
+    for i, (name, shape) in enumerate(m.params):
+        m.put_param(i, (r.standard_normal(shape) * 0.05).astype(np.float16))
+    tok = r.integers(0, V, 16).astype(np.uint16)
+    m.adamw_init()
+    m.step(tok, tok, np.full(16, 8.0, np.float32))
+    m.adamw_step(1, lr=1e-2)
+    for i, (name, shape) in enumerate(m.params):
+        # the f16 parameter is the rounded master, which comes back through another read of twice the bytes
+        got, master = m.param(i), m.adamw_state(i, "master")
+        assert np.array_equal(got.view(np.uint16), master.astype(np.float16).view(np.uint16)), name
+        assert np.isfinite(master).all() and len(np.unique(got.view(np.uint16))) > min(got.size, 100) // 4
+    m.close(); ctx.close()
+
+
 def test_a_device_reset_leaves_no_page_locked_buffer(tmp_path):
     """The buffers kept for later contexts go before the reset that would delete them under the library (a child process:
     the reset takes everything on the device with it)."""
