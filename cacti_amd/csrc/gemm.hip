@@ -421,6 +421,7 @@ CACTI_API int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M
     const int64_t ca = ta ? M : K, cb = tb ? K : N;
     bool fast = M > 0 && N > 0 && K > 0 && (beta == 0.f || beta == 1.f) && mult(ca, 8) && mult(cb, 8) && mult(N, 8) &&
                 mult(lda, 8) && mult(ldb, 8) && mult(ldc, 8) && lda >= ca && ldb >= cb && ldc >= N && K > 128;
+    if (!ta && tb && M <= 4 && beta == 0.f) fast = false;         // a stream over B each, as alone (gemm_run)
     for (int64_t z = 0; z < nblk && fast; z++) fast = aligned(A[z], 16) && aligned(B[z], 16) && aligned(C[z], 16);
     for (int64_t z0 = 0; z0 < nblk; z0 += kMaxPtrBatch) {
         const int64_t cnt = nblk - z0 < kMaxPtrBatch ? nblk - z0 : kMaxPtrBatch;

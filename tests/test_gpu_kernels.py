@@ -447,6 +447,13 @@ def test_gemm_pointer_array_batch_with_a_k_tail(ops, oracle, ta, tb, n, M, N, K)
     test_gemm_pointer_array_batch(ops, oracle, ta, tb, n, M, N, K, 0)
 
 
+@pytest.mark.parametrize("n,M,N,K", [(3, 1, 1096, 264), (2, 4, 1096, 264), (4, 5, 1096, 264)])
+def test_gemm_pointer_array_batch_of_few_rows(ops, oracle, n, M, N, K):
+    """One to four rows take the streaming kernel in a batch as they do alone: the bits of the single products.  (K = 264:
+    ops.gemm lends a workspace, with which an accumulating product of few rows and a longer K is summed in parts.)"""
+    test_gemm_pointer_array_batch(ops, oracle, 0, 1, n, M, N, K, 0)
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0), (0, 0)])
 @pytest.mark.parametrize("off", [1, 4])
 def test_gemm_operands_that_start_between_16_byte_boundaries(ops, oracle, ta, tb, off):
