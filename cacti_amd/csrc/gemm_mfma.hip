@@ -7,15 +7,15 @@
 // blocks that are interleaved with those of the other waves (32 WM rows / 32 WN columns apart).
 // The register path forms a block with v_mfma_f32_32x32x16_f16; the direct path, which carries the
 // large products of the step, as four 16 x 16 results of v_mfma_f32_16x16x32_f16: under a sustained
-// load the device is limited by power, and that instruction needs less of it per flop.  Shapes
-// instantiated: 128 x 128 on 4 waves (two workgroups per CU), 256 x 128 and 256 x 256 on 8
-// waves (one per CU), 64 x 64 on 4 waves (remainder columns).
+// load the device is limited by power, and that instruction needs less of it per flop.  Shapes: the
+// direct path's are listed at enum Tile; the register path has 128 x 128 on 4 or 8 waves.
 //
-// Two ways from global memory to LDS.  Through registers (any alignment >= 8 bytes, k tails):
-// described below.  Direct (16-byte aligned operands, K a multiple of 64; the large dense
-// products): global_load_lds_dwordx4 writes each wave's 1 KB straight into LDS, NBUF - 1 k
-// tiles ahead, with no staging registers, no LDS store instructions and no transposes in
-// registers; a k-contiguous operand lands in the swizzled [row][k] layout below (the swizzle
+// Two ways from global memory to LDS.  Through registers (any alignment >= 8 bytes; the attention
+// products of separate thunks on heads that start between 16-byte boundaries): described below.
+// Direct (16-byte aligned operands, any K: a tail of K is loaded first, its lanes beyond the end
+// fetching zeros; all other products): global_load_lds_dwordx4 writes each wave's 1 KB straight into
+// LDS, NBUF - 1 k tiles ahead, with no staging registers, no LDS store instructions and no
+// transposes in registers; a k-contiguous operand lands in the swizzled [row][k] layout below (the swizzle
 // is applied to the global address), a k-strided one in its own [k][row] layout and is
 // transposed on the way out of LDS by ds_read_b64_tr_b16.
 //
@@ -600,7 +600,7 @@ gemm_mfma_kernel(GemmArgs p)
     static_assert(EPI == E_ROWS || (DMA && !M32), "split and odd products are direct ones");
     static_assert(!M32 || (DMA && BM == 32 * WM && BN == 32 * WN), "one block per wave");
     static_assert(DMA ? (STAGES == 1 && AL == 8 && !KTAIL) : NBUF == 2,
-                  "direct loads: 16-byte aligned operands, whole k tiles");
+                  "direct loads: 16-byte aligned operands, one register stage, their own k tail");
     constexpr bool TR_A = DMA && TA, TR_B = DMA && !TB;           // fragments by transposing reads
     static_assert((WM % 2 == 0 || BM / WM == 32) && (WN % 2 == 0 || BN / WN == 32),
                   "tiles of a wave lie 32 WM rows apart: a multiple of 64 keeps their swizzle equal");
@@ -1409,7 +1409,10 @@ int launch_direct(int tile, const GemmArgs &p, int64_t nblk, hipStream_t st)
 // set of resident workgroups (`resident` per CU: `full`), for the last, partly filled set `first` + `load` x the share
 // of the CUs that are busy where no CU has more than one, and `round` for every further set.  Fitted (least squares
 // of the log) to 338 products measured on MI355X: M 33 .. 8640, N 256 .. 32000, K 37 .. 32000, the three layouts;
-// rms error 6-8 % per tile, and the tile picked by it is 1.3 % slower than the best one in the mean, 14 % at worst.
+// rms error 6-8 % per tile.  On 322 others of the same ranges (profiles/gemm_tile_times_by_shape.txt has the times of every
+// tile) it is 9-11 % for the tiles of 128 x 128 and more and 18-21 % for the smaller two, whose worst products stream
+// operands of hundreds of MB through few tiles; the tile picked by it is 0.8 % slower than the best one in the mean
+// and 34 % at worst (41 x 18096 x 28216).
 struct TileCost {
     int bm, bn, resident;
     double fixed, first, load, full, round;

@@ -3,7 +3,8 @@
 // used M times, so the kernel is built for HBM, not for the matrix cores.
 //
 // A workgroup of 64 or 256 lanes owns R = 4 rows of B (4 output columns) and splits K over its lanes
-// in 16-byte pieces; a lane issues the loads of its 1 to 5 pieces x 4 rows before it uses the first,
+// in 16-byte pieces; a lane issues the loads of its 1 to 5 pieces x 4 rows before it uses the first (a longer row
+// takes several such passes),
 // accumulates M x 4 fp32 sums with v_dot2_f32_f16 (the scalar form, 3 instructions per product
 // with the conversions, made the kernel compute-bound), and the sums are reduced over the wave (cross-lane adds) and
 // over the waves (LDS).  N / 4 workgroups: 800 for N = 3200, 8 resident per CU.  A (a few KiB)
@@ -14,7 +15,9 @@
 //  * NORM: A is not read but formed per workgroup as the RMSNorm of a row x (optionally of the
 //    residual sum f16(x + x2), which workgroup 0 also writes out): the lanes' own pieces of the
 //    row give the sum of squares (every piece of the row belongs to exactly one lane), one
-//    workgroup reduction, then a = f16(w * (x * rinv)) exactly as the RMSNorm kernel rounds it.
+//    workgroup reduction, then a = f16(w * (x * rinv)).  The RMSNorm kernel sums in fp64 and divides;
+//    here the sum is fp32 and rinv a rounded reciprocal, which moves 8 elements of 100,000 to
+//    the neighbouring f16.
 //  * GATE: two weight matrices share the rows (gate and up projection); the epilogue stores
 //    f16(f16(silu(g)) * u) of the two rounded products, as the SiLU-gate kernel computes it.
 //  * QKV: one launch covers the query, key and value projections; a workgroup owns two rotation
@@ -326,11 +329,13 @@ void launch_cfg(const SkinnyArgs &p, hipStream_t st)
     hipLaunchKernelGGL((gemm_skinny_nt_kernel<M, NORM, EPI, W, kPre>), grid, block, 0, st, p);
 }
 
-// A row of K is cut over the lanes of the workgroup with as little left over as may be (lanes without a piece of their
-// own still load): K = 2048 is one piece per lane of 4 waves (two: gate and up 11.5 against 10.3 us, a head of 32000 25.5
-// against 22.0), K = 8640 five in one pass (four in two: 13.2 against 11.5).  Few pieces: one wave, so that no barrier stands
-// between its loads and its result.  Eight columns per workgroup instead of four changed nothing (13.9 and 14.1 us for q,
-// k, v of 3200).
+// How a row of K is cut over lanes.  Lanes without a piece of their own still load (a duplicate), so one row takes as many
+// pieces per lane as it needs: K = 2048 is one piece per lane of 4 waves (with two: gate and up 11.5 against 10.3 us, a
+// head of 32000 25.5 against 22.0), and up to 1024 one wave does, so that no barrier stands between its loads and its
+// result.  A plain product of 8200 to 10240 elements is five pieces in one pass (K = 8640: four in two passes 13.2
+// against 11.5); every longer row is passes of four, the last of them partly duplicates, and two to four rows have
+// passes of two (K <= 4096) or four pieces only: no other cut of those has been measured.  Eight columns per
+// workgroup instead of four changed nothing (13.9 and 14.1 us for q, k, v of 3200).
 template <bool NORM, int EPI>
 int launch(int64_t M, const SkinnyArgs &p, hipStream_t st)
 {

@@ -313,9 +313,9 @@ struct MatMulSpec : ThunkSpec {
 // cacti_hip_gemm_f16_batched: the shape of the reference's cublasGemmBatchedEx call,
 // cacti_gpu_cu_ffi/src/lib.rs:793-885).  The reference stages the query, key and value projections of a layer
 // (and the gate and up projections) as separate matmul thunks on the same input (src/librarium/llama.rs:
-// 478-497); each product here is computed by the same tiles in the same order as its own launch would, so the
-// results are those of the separate thunks bit for bit, and the adjoint stages what their adjoints would have
-// staged, in their order: the weight gradients (one grouped thunk), then the input gradients one after the other
+// 478-497); each output here is summed over the same values in the same order as in a launch of its own (the tiles
+// may be others), so the results are those of the separate thunks bit for bit, and the adjoint stages what their
+// adjoints would have staged, in their order: the weight gradients (one grouped thunk), then the input gradients one after the other
 // (they accumulate into one cell: last product first, as the reverse sweep over separate thunks meets them).
 constexpr int kMaxGroup = 4;
 

@@ -255,7 +255,7 @@ def abs_log2_hist8(x):
 
 
 def digests(xs):
-    """Both digests of a list of f16 tensors in one launch: (hist int64[n,256], nan int64[n])
+    """Both digests of a list of f16 tensors, up to 64 in a launch: (hist int64[n,256], nan int64[n])
     (the per-cycle loop of examples/open_llama_3b_train.rs:409-424)."""
     if len(xs) == 0:
         out = torch.empty((0, 257), dtype=torch.int64, device="cuda")
@@ -317,7 +317,7 @@ def adamw32_scalars(iter_nr, grad_scale, lr, wd, a1, a2, eps):
 
 
 def adamw32_step_(grads, avgs, avg2s, masters, params, scalars):
-    """One AdamW32 step of a list of tensors in one launch, in place (avgs, avg2s, masters updated,
+    """One AdamW32 step of a list of tensors, up to 64 in a launch, in place (avgs, avg2s, masters updated,
     params overwritten with f16(master))."""
     _op.adamw32_step(grads, avgs, avg2s, masters, params, scalars)
 

@@ -149,10 +149,11 @@ int cacti_hip_mfma_probe(int shape, int lds_reads, int random_operands, int bloc
 
 /* Pointer-array batch, the shape of cublasGemmBatchedEx (cacti_gpu_cu_ffi/src/lib.rs:793-885):
  * nblk products of one shape, block z on A[z], B[z], C[z] (host arrays of device pointers, read
- * before the call returns).  With every operand 16-byte aligned up to four products share a launch,
- * otherwise they run one after another.  (Sharing a launch saves launches, not time: measured on the
- * three 2048 x 3200 x 3200 projections of a layer, 600 whole tiles on 256 CUs take three tile times
- * either way.)  Results equal those of nblk calls of cacti_hip_gemm_f16. */
+ * before the call returns).  With every operand 16-byte aligned and K > 128 up to four products share a
+ * launch, otherwise (and for one to four rows against a transposed B) they run one after another.  Sharing
+ * saves launches, and time where the products alone leave CUs idle; the three 2048 x 3200 x 3200 projections
+ * of a layer, 600 whole tiles on 256 CUs, take three tile times either way.  Results equal those of nblk
+ * calls of cacti_hip_gemm_f16 bit for bit. */
 int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K,
                                float alpha, const void *const *A, int64_t lda, const void *const *B,
                                int64_t ldb, float beta, void *const *C, int64_t ldc, void *stream);
@@ -422,7 +423,7 @@ int cacti_hip_selftest_wave_reduce(void *out4, void *stream);
 int cacti_hip_nan_count_f16(int64_t n, const void *x, void *count_i64, void *stream);
 int cacti_hip_abs_log2_hist8_f16(int64_t n, const void *x, void *hist_i64_256, void *stream);
 
-/* Both digests of `count` tensors in one launch and one read of each tensor (the example's loop
+/* Both digests of `count` tensors, up to 64 in a launch, in one read of each tensor (the example's loop
  * over all parameters and gradients, examples/open_llama_3b_train.rs:409-424, as one call):
  * out_i64[257 * i + b] = abs_log2_hist8 class b of tensor i, out_i64[257 * i + 256] = its NaN
  * count.  xs[i] (device, 16-byte aligned) holds ns[i] >= 0 f16 elements; xs and ns are host
@@ -462,7 +463,7 @@ int cacti_hip_cast_f16_f32(int64_t n, const void *src_f16, void *dst_f32, void *
 int cacti_adamw32_scalars(int iter_nr, float grad_scale, float lr, float wd, float a1, float a2,
                           float eps, float *out7);
 
-/* One AdamW32 step of `count` tensors in one launch: for each tensor the three thunks above and the
+/* One AdamW32 step of `count` tensors, up to 64 in a launch: for each tensor the three thunks above and the
  * cast of the master weights back to the f16 parameter (the loop of
  * examples/open_llama_3b_train.rs:252-268), each element read and written once; bit-identical to
  * the four separate thunks.  grads (f16, read), avgs, avg2s, masters (f32, updated), params (f16,
