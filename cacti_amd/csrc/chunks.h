@@ -6,8 +6,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace cacti {
@@ -52,8 +52,8 @@ ChunkError copy_chunks(char *dst, const char *src, size_t bytes, size_t chunk, i
                 start();
                 work();
             });
-    } catch (const std::system_error &) {
-        // no more threads to be had: those that started and this one take the pieces
+    } catch (const std::exception &) {
+        // no more threads (or memory for one) to be had: those that started and this one take the pieces
     }
     work();
     for (std::thread &t : th)

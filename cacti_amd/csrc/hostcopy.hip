@@ -12,7 +12,6 @@
 #include <atomic>
 #include <chrono>
 #include <mutex>
-#include <vector>
 
 #include "chunks.h"
 #include "common.h"
@@ -113,11 +112,18 @@ int wait_flags(const unsigned *flags, int n, unsigned epoch, hipStream_t st)
 // every thread that reads at the same time, and two windows of large reads (a third reader at the same time page-locks
 // its own and frees it again).
 struct Kept {
-    size_t bytes, most;
-    std::vector<Staging> free;
+    size_t bytes;
+    int most, n;
+    Staging free[16];
+    Staging take(int i)
+    {
+        const Staging s = free[i];
+        free[i] = free[--n];
+        return s;
+    }
 };
 std::mutex g_mutex;
-Kept g_kept[] = {{kStagingBytes, 4, {}}, {kWordBytes, 16, {}}, {kWindowBytes, 2, {}}};
+Kept g_kept[] = {{kStagingBytes, 4, 0, {}}, {kWordBytes, 16, 0, {}}, {kWindowBytes, 2, 0, {}}};
 std::atomic<size_t> g_pinned{0};               // bytes page-locked here, kept or in use
 unsigned g_resets[64];                         // per device, under g_mutex
 
@@ -247,10 +253,9 @@ bool staging_take(Staging *s, size_t bytes)
     *s = Staging{};
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        for (size_t i = k->free.size(); i-- > 0;)
+        for (int i = k->n; i-- > 0;)
             if (k->free[i].dev == dev) {
-                *s = k->free[i];
-                k->free.erase(k->free.begin() + (std::ptrdiff_t)i);
+                *s = k->take(i);
                 return true;
             }
         s->resets = g_resets[dev];
@@ -272,12 +277,12 @@ void staging_give_back(Staging *s)
         std::lock_guard<std::mutex> lock(g_mutex);
         Kept *k = kept_of(s->bytes);
         ours = !s->lost && s->resets == g_resets[s->dev];
-        keep = ours && k->free.size() < k->most;
-        if (keep) k->free.push_back(*s);
+        keep = ours && k->n < k->most;
+        if (keep) k->free[k->n++] = *s;
     }
     // (one that may still be written, or that a reset has deleted, is neither kept nor freed)
     if (ours && !keep) pinned_free(s->base, s->bytes);
-    else if (!ours) g_pinned -= s->bytes;
+    else if (!ours && !s->lost) g_pinned -= s->bytes;
     *s = Staging{};
 }
 
@@ -286,11 +291,8 @@ void staging_release(int dev)
     if (dev < 0 || dev >= 64) return;
     std::lock_guard<std::mutex> lock(g_mutex);
     for (Kept &k : g_kept)
-        for (size_t i = k.free.size(); i-- > 0;)
-            if (k.free[i].dev == dev) {
-                pinned_free(k.free[i].base, k.bytes);
-                k.free.erase(k.free.begin() + (std::ptrdiff_t)i);
-            }
+        for (int i = k.n; i-- > 0;)
+            if (k.free[i].dev == dev) pinned_free(k.take(i).base, k.bytes);
     g_resets[dev]++;
 }
 
@@ -321,6 +323,6 @@ CACTI_API int cacti_hip_pinned_bytes(size_t *held, size_t *kept)
     std::lock_guard<std::mutex> lock(g_mutex);
     *held = g_pinned.load();
     *kept = 0;
-    for (const Kept &k : g_kept) *kept += k.bytes * k.free.size();
+    for (const Kept &k : g_kept) *kept += k.bytes * (size_t)k.n;
     return 0;
 }

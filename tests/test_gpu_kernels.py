@@ -1,6 +1,6 @@
 """Parity of every HIP kernel against the CPU oracle on the same seeded inputs (MI355X).
 
-All calls go through the C ABI (cacti_amd.ops is a thin ctypes layer).  Tolerances:
+All calls go through the C ABI (cacti_amd.ops is a thin layer over it).  Tolerances:
 tests/util.py (rel-L2 <= 1e-3, max element relative error <= 2e-2); gather / argmax /
 index results bit-exact.  Elementwise kernels reproduce the oracle's rounding points, so
 most of them are in fact compared bit for bit (`exact_frac`).
