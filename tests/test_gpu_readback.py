@@ -1,5 +1,8 @@
 """Read-backs: page-locked memory the library holds for them, and readers that do not get in each other's way (MI355X)."""
 import ctypes as C
+import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -47,9 +50,9 @@ def test_reading_a_word_holds_no_memory_per_thread():
 SMALL = dict(S=32, D=256, H=4, F=512, L=1, eps=1e-6)
 
 
-def model(V=4096):
+def model(V=4096, pagelocked=True):
     from cacti_amd.runtime import Ctx, Llama
-    ctx = Ctx(0, 256 << 20, True)
+    ctx = Ctx(0, 256 << 20, pagelocked)
     m = Llama(ctx, SMALL["S"], SMALL["D"], SMALL["H"], SMALL["D"] // SMALL["H"], SMALL["F"], V, SMALL["L"], SMALL["eps"])
     r = np.random.default_rng(3)
     for i, (name, shape) in enumerate(m.params):
@@ -72,12 +75,11 @@ def busy(stream, ms):
         torch.cuda._sleep(int(min(ms / a.elapsed_time(b), 2000) * 1000000))
 
 
-def test_a_large_read_does_not_wait_for_another_contexts_stream():
-    """One context's large read waits for what is queued on its stream; a read of another context, on another thread, is
-    through before that."""
+def concurrent_reads():
     from cacti_amd import ffi
     torch.cuda.init()
-    (ctx_a, a), (ctx_b, b) = model(), model()
+    # (no streams for spilling: two streams and the null stream are fewer than the hardware queues, so none shares one)
+    (ctx_a, a), (ctx_b, b) = model(pagelocked=False), model(pagelocked=False)
     i = [n for n, _ in a.params].index("lm_head")
     want = a.grad(i)
     assert want.nbytes >= 2 << 20 and np.array_equal(want, b.grad(i))
@@ -93,9 +95,25 @@ def test_a_large_read_does_not_wait_for_another_contexts_stream():
     got["b"] = b.grad(i)
     first = t.is_alive()
     t.join()
-    assert first and np.array_equal(got["a"], want) and np.array_equal(got["b"], want)
+    assert np.array_equal(got["a"], want) and np.array_equal(got["b"], want)
     for x in (a, b, ctx_a, ctx_b):
         x.close()
+    print("the other context's read was first:", first)
+
+
+def child(code):
+    """Runs in a process of its own: with its own hardware queues, and its own device state."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", "import sys; sys.path.insert(0, %r); import torch; torch.cuda.init()\n%s" % (root, code)],
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr[-2000:]
+    return r.stdout
+
+
+def test_a_large_read_does_not_wait_for_another_contexts_stream():
+    """One context's large read waits for what is queued on its stream; a read of another context, on another thread, is
+    through before that."""
+    assert "first: True" in child("from tests.test_gpu_readback import concurrent_reads; concurrent_reads()")
 
 
 @pytest.mark.parametrize("V,D", [(20000, 1024), (8200, 1032), (24, 264)])
@@ -120,18 +138,10 @@ def test_reads_of_several_windows_come_back_whole(V, D):
     m.close(); ctx.close()
 
 
-def test_a_device_reset_leaves_no_page_locked_buffer(tmp_path):
+def test_a_device_reset_leaves_no_page_locked_buffer():
     """The buffers kept for later contexts go before the reset that would delete them under the library (a child process:
     the reset takes everything on the device with it)."""
-    import os
-    import subprocess
-    import sys
-    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    code = (
-        "import sys\n"
-        "sys.path.insert(0, %r)\n"
-        "import torch\n"
-        "torch.cuda.init()\n"
+    assert "released" in child(
         "from cacti_amd import ffi\n"
         "from tests.test_gpu_readback import model, pinned\n"
         "ctx, m = model()\n"
@@ -141,6 +151,4 @@ def test_a_device_reset_leaves_no_page_locked_buffer(tmp_path):
         "assert held == kept >= (16 << 20), (held, kept)\n"
         "ffi.call('cacti_hip_primary_ctx_reset', 0)\n"
         "assert pinned() == (0, 0), pinned()\n"
-        "print('released')\n" % root)
-    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
-    assert r.returncode == 0 and "released" in r.stdout, r.stdout + r.stderr[-2000:]
+        "print('released')\n")
