@@ -10,10 +10,10 @@
 // load the device is limited by power, and that instruction needs less of it per flop.  Shapes: the
 // direct path's are listed at enum Tile; the register path has 128 x 128 on 4 or 8 waves.
 //
-// Two ways from global memory to LDS.  Through registers (any alignment >= 8 bytes; the attention
-// products of separate thunks on heads that start between 16-byte boundaries): described below.
-// Direct (16-byte aligned operands, any K: a tail of K is loaded first, its lanes beyond the end
-// fetching zeros; all other products): global_load_lds_dwordx4 writes each wave's 1 KB straight into
+// Two ways from global memory to LDS.  Through registers (any alignment >= 8 bytes, k tails; what is left for it
+// are operands aligned to 8 bytes only, where no workspace is lent for a copy, and triangular products
+// with a k tail): described below.  Direct (16-byte aligned operands, any K: a tail of K is loaded first, its
+// lanes beyond the end fetching zeros; all other products): global_load_lds_dwordx4 writes each wave's 1 KB straight into
 // LDS, NBUF - 1 k tiles ahead, with no staging registers, no LDS store instructions and no
 // transposes in registers; a k-contiguous operand lands in the swizzled [row][k] layout below (the swizzle
 // is applied to the global address), a k-strided one in its own [k][row] layout and is
