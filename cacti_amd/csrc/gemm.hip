@@ -254,6 +254,10 @@ int launch_vec(int vec, const GemmArgs &p, int64_t nblk, hipStream_t st)
 
 inline bool mult(int64_t v, int64_t a) { return v % a == 0; }
 
+// The tile kernels keep a lane's place inside a tile (up to 256 rows) as a 32-bit byte offset; operands whose rows lie
+// farther apart go to the kernel above, which addresses each element in 64 bits.
+constexpr int64_t kMaxPitch = (int64_t)1 << 23;
+
 }  // namespace
 
 namespace {
@@ -303,6 +307,7 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
             break;
         }
     hipStream_t st = (hipStream_t)stream;
+    const bool near = lda < kMaxPitch && ldb < kMaxPitch;
     if (vec >= 4 && !ta && tb && K <= 128 && beta == 0.f && tri <= 1)
         return gemm_nt_smallk_launch(p, nblk, st);
     // one to four rows against a weight matrix (decoding): a stream over B
@@ -313,7 +318,7 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
     // is only a multiple of 8 bytes.  Addressed from the 16-byte boundary below each slab they
     // take the direct-load path; the extra columns read stay inside the columns the blocks
     // cover in one row of B (checked here).
-    if (vec == 4 && !tb && nblk > 1 && mult(K, 64) && mult(ta ? M : K, 8) && mult(lda, 8) &&
+    if (near && vec == 4 && !tb && nblk > 1 && mult(K, 64) && mult(ta ? M : K, 8) && mult(lda, 8) &&
         mult(stride_a, 8) && aligned(A, 16) && mult(ldb, 8) && mult(ldc, 8) && aligned(B, 16) &&
         aligned(C, 16) && (stride_b & 7) == (stride_c & 7)) {
         const int64_t row_end = (nblk - 1) * stride_b + N;
@@ -328,7 +333,7 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
             return gemm_mfma_launch(ta, tb, p, nblk, 8, false, nullptr, st);
         }
     }
-    if (tri == 0 && vec == 8) {
+    if (near && tri == 0 && vec == 8) {
         const GemmPlan plan = gemm_plan(M, N, K, nblk, ws_need != nullptr);
         if (plan.split > 1) {
             p.ldp = (N + 3) / 4 * 4;
@@ -341,9 +346,9 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
     // Operands that are not 16-byte aligned, with a workspace: laid out anew (one launch for both, 3-5 us for a few MB)
     // for the direct kernels.  Element-wise loads in the kernel cost 1.6 us (both operands contiguous in K) to 3.4 us
     // (both strided) per 32 values of K instead, so only products with hardly any K stay on them.
-    if (ws_need && tri == 0 && nblk == 1 && K > 64) {
-        const bool ok_a = fits_a(8), ok_b = fits_b(8);
-        const int64_t ra = ta ? K : M, rb = tb ? N : K, pa = (ca + 7) / 8 * 8, pb = (cb + 7) / 8 * 8;
+    const int64_t ra = ta ? K : M, rb = tb ? N : K, pa = (ca + 7) / 8 * 8, pb = (cb + 7) / 8 * 8;
+    if (ws_need && tri == 0 && nblk == 1 && K > 64 && pa < kMaxPitch && pb < kMaxPitch) {
+        const bool ok_a = fits_a(8) && lda < kMaxPitch, ok_b = fits_b(8) && ldb < kMaxPitch;
         const size_t bytes_a = ok_a ? 0 : (size_t)ra * (size_t)pa * 2, bytes_b = ok_b ? 0 : (size_t)rb * (size_t)pb * 2;
         const GemmPlan plan = gemm_plan(M, N, K, 1, true);
         p.ldp = (N + 3) / 4 * 4;
@@ -369,7 +374,7 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
         p.part = (float *)(w + bytes_a + bytes_b);
         return gemm_mfma_launch(ta, tb, p, 1, 8, !fits_c(8), &plan, st);
     }
-    if (vec >= 4) return gemm_mfma_launch(ta, tb, p, nblk, vec, false, nullptr, st);
+    if (near && vec >= 4) return gemm_mfma_launch(ta, tb, p, nblk, vec, false, nullptr, st);
     if (!ta && !tb) return launch_vec<false, false>(vec, p, nblk, st);
     if (!ta && tb) return launch_vec<false, true>(vec, p, nblk, st);
     if (ta && !tb) return launch_vec<true, false>(vec, p, nblk, st);
@@ -420,7 +425,8 @@ CACTI_API int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M
         CACTI_REQUIRE(A[z] && B[z] && C[z], CACTI_E_INVALID, "gemm_batched: null operand in block %lld", (long long)z);
     const int64_t ca = ta ? M : K, cb = tb ? K : N;
     bool fast = M > 0 && N > 0 && K > 0 && (beta == 0.f || beta == 1.f) && mult(ca, 8) && mult(cb, 8) && mult(N, 8) &&
-                mult(lda, 8) && mult(ldb, 8) && mult(ldc, 8) && lda >= ca && ldb >= cb && ldc >= N && K > 128;
+                mult(lda, 8) && mult(ldb, 8) && mult(ldc, 8) && lda >= ca && ldb >= cb && ldc >= N && K > 128 &&
+                lda < kMaxPitch && ldb < kMaxPitch;
     if (!ta && tb && M <= 4 && beta == 0.f) fast = false;         // a stream over B each, as alone (gemm_run)
     for (int64_t z = 0; z < nblk && fast; z++) fast = aligned(A[z], 16) && aligned(B[z], 16) && aligned(C[z], 16);
     for (int64_t z0 = 0; z0 < nblk; z0 += kMaxPtrBatch) {

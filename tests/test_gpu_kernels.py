@@ -454,6 +454,31 @@ def test_gemm_pointer_array_batch_of_few_rows(ops, oracle, n, M, N, K):
     test_gemm_pointer_array_batch(ops, oracle, 0, 1, n, M, N, K, 0)
 
 
+@pytest.mark.parametrize("ta,tb,M,N,K", [(0, 1, 64, 264, 520), (0, 0, 64, 264, 520), (1, 0, 72, 264, 64), (1, 0, 72, 264, 61), (0, 1, 63, 100, 40)])
+@pytest.mark.parametrize("ws", [False, True])
+def test_gemm_rows_gigabytes_apart(ops, oracle, ta, tb, M, N, K, ws):
+    """Rows of A 2^26 elements apart (a column slice of a very wide matrix): beyond a 32-bit offset inside one tile.  Through
+    the entry point without a workspace, and with one."""
+    from cacti_amd import ffi
+    say("gemm far rows", ta, tb, M, N, K, ws)
+    r = rng(320 + M + K + ta + 2 * tb)
+    A, B = randn16(r, (K, M) if ta else (M, K)), randn16(r, (N, K) if tb else (K, N), 0.1)
+    ld = (1 << 26) + 8
+    wide = torch.empty((A.shape[0] - 1) * ld + A.shape[1], dtype=torch.float16, device="cuda")
+    dA = wide.as_strided(A.shape, (ld, 1))
+    dA.copy_(dev(A))
+    dB, want = dev(B), oracle.matmul(ta, tb, A, B)
+    if ws:
+        got = ops.gemm(dA, dB, bool(ta), bool(tb))
+    else:
+        got = torch.empty((M, N), dtype=torch.float16, device="cuda")
+        ffi.call("cacti_hip_gemm_f16", ta, tb, M, N, K, 1.0, dA.data_ptr(), ld, dB.data_ptr(), dB.stride(0), 0.0, got.data_ptr(), N,
+                 torch.cuda.current_stream().cuda_stream)
+    assert_parity(host(got), want, "far rows")
+    del wide, dA
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0), (0, 0)])
 @pytest.mark.parametrize("off", [1, 4])
 def test_gemm_operands_that_start_between_16_byte_boundaries(ops, oracle, ta, tb, off):
