@@ -70,7 +70,7 @@ def synth_inputs(cfg, seed=1, grad_scale=1024.0):
 # L2-miss traffic per launch of the GEMM kernels at the step's shapes: measured, not assumed, and tied to
 # the kernels it was measured on.  cacti_amd/gemm_traffic.json is written by `python -m cacti_amd.gemm_traffic`
 # from two rocprofv3 --pmc passes (FETCH_SIZE, WRITE_SIZE) over `bench.py --workload gemm-traffic` and
-# records the hash of csrc/gemm_mfma.hip it was taken on; with any other build of the kernels the roofline
+# records the hash of csrc/gemm_direct.hip it was taken on; with any other build of the kernels the roofline
 # line carries "traffic": null instead of figures that no longer describe what runs.
 def _traffic_table():
     from cacti_amd import gemm_traffic
@@ -125,16 +125,12 @@ def gemm_plan(M, N, K):
     return (out[0], out[1]), out[5]
 
 
-TILE_ARGS = {(64, 64): "64, 64, 2, 2, 8, false, 1, 4, true", (128, 64): "128, 64, 2, 2, 8, false, 1, 3, true",
-             (128, 128): "128, 128, 2, 4, 8, false, 1, 3, true", (256, 128): "256, 128, 4, 2, 8, false, 1, 3, true",
-             (256, 192): "256, 192, 4, 2, 8, false, 1, 2, true", (256, 256): "256, 256, 2, 4, 8, false, 1, 2, true"}
-
-
 def kernel_symbol(label):
     """Name of the HIP kernel instantiation a dense GEMM label runs on (its first launch), as
-    rocprofv3 prints it, for 16-byte aligned operands."""
+    rocprofv3 prints it, for 16-byte aligned operands (tiles of 64 columns run two workgroups to a CU)."""
     ta, tb, H, M, N, K = gemm_dims(label)
-    return "gemm_mfma_kernel<%s, %s, %s, 0, false>" % (str(ta).lower(), str(tb).lower(), TILE_ARGS[gemm_plan(M, N, K)[0]])
+    bm, bn = gemm_plan(M, N, K)[0]
+    return "gemm_direct_kernel<%s, %s, %d, %d, %d, false>" % (str(ta).lower(), str(tb).lower(), bm, bn, 2 if bn == 64 or (bm, bn) == (64, 128) else 1)
 
 
 def is_split(label):

@@ -330,7 +330,7 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
         }
         if (inside) {
             p.win = 1;
-            return gemm_mfma_launch(ta, tb, p, nblk, 8, false, nullptr, st);
+            return gemm_mfma_launch(ta, tb, p, nblk, 8, st);
         }
     }
     if (near && tri == 0 && vec == 8) {
@@ -341,7 +341,7 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
             *ws_need = (size_t)plan.split * (size_t)M * (size_t)p.ldp * sizeof(float);
             if (*ws_need > ws_bytes) return 0;
         }
-        return gemm_mfma_launch(ta, tb, p, nblk, 8, false, &plan, st);
+        return gemm_direct_launch(ta, tb, p, nblk, plan, st);
     }
     // Operands that are not 16-byte aligned, with a workspace: laid out anew (one launch for both, 3-5 us for a few MB)
     // for the direct kernels.  Element-wise loads in the kernel cost 1.6 us (both operands contiguous in K) to 3.4 us
@@ -372,9 +372,10 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
             p.ldb = pb;
         }
         p.part = (float *)(w + bytes_a + bytes_b);
-        return gemm_mfma_launch(ta, tb, p, 1, 8, !fits_c(8), &plan, st);
+        p.odd = !fits_c(8);
+        return gemm_direct_launch(ta, tb, p, 1, plan, st);
     }
-    if (near && vec >= 4) return gemm_mfma_launch(ta, tb, p, nblk, vec, false, nullptr, st);
+    if (near && vec >= 4) return gemm_mfma_launch(ta, tb, p, nblk, vec, st);
     if (!ta && !tb) return launch_vec<false, false>(vec, p, nblk, st);
     if (!ta && tb) return launch_vec<false, true>(vec, p, nblk, st);
     if (ta && !tb) return launch_vec<true, false>(vec, p, nblk, st);
@@ -443,8 +444,6 @@ CACTI_API int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M
         p.A = (const half_t *)A[z0]; p.lda = lda; p.sa = 0;
         p.B = (const half_t *)B[z0]; p.ldb = ldb; p.sb = 0;
         p.C = (half_t *)C[z0]; p.ldc = ldc; p.sc = 0;
-        p.tiles_m = (int)((M + BM - 1) / BM);
-        p.tiles_n = (int)((N + BN - 1) / BN);
         p.ztab = 1;
         for (int64_t z = 0; z < kMaxPtrBatch; z++) {
             const int64_t zz = z0 + (z < cnt ? z : 0);
@@ -453,7 +452,7 @@ CACTI_API int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M
             p.zc[z] = (half_t *)C[zz] - p.C;
         }
         const GemmPlan plan = gemm_plan(M, N, K, cnt, false);
-        const int rc = gemm_mfma_launch(ta, tb, p, cnt, 8, false, &plan, (hipStream_t)stream);
+        const int rc = gemm_direct_launch(ta, tb, p, cnt, plan, (hipStream_t)stream);
         if (rc) return rc;
     }
     return 0;

@@ -4,6 +4,67 @@
 
 namespace cacti {
 
+// n / d for n < 2^31 by a multiplication: with m = ceil(2^(31 + s) / d) and 2^(s - 1) < d <= 2^s, m d exceeds 2^(31 + s) by
+// less than 2^s, so n m exceeds n 2^(31 + s) / d by less than 2^(31 + s) / d.  (A division by a kernel argument is some
+// 40 vector instructions, one after another, in front of a workgroup's first load.)
+struct FastDiv {
+    uint32_t m, shift;
+    void set(uint32_t d)
+    {
+        uint32_t s = 0;
+        while ((uint64_t)1 << s < d) s++;
+        shift = 31 + s;
+        m = (uint32_t)((((uint64_t)1 << shift) + d - 1) / d);
+    }
+    __host__ __device__ __forceinline__ uint32_t div(uint32_t n) const { return (uint32_t)((uint64_t)n * m >> shift); }
+};
+
+// From a workgroup's number to its tile.  Dispatch order i lands on XCD i % 8: each XCD is given a contiguous band of the
+// flattened (block of the batch, tile) sequence.  Within a block the tiles are walked in groups of `rows` tile rows x all
+// tile columns, row fastest, so that the workgroups resident together on an XCD form a patch of C and share the operand
+// panels fetched into its L2.  A pointer-table batch is a handful of whole products that share an operand (the projections
+// of one input, the weight gradients against one input): product fastest, so that the workgroups resident together work on
+// the same tile of every product and fetch the shared panel once.
+struct TileWalk {
+    int wgs, nz, ztab, tiles, rows, full, rest, per_group;        // full, rest: tile rows in whole groups, and others
+    FastDiv by_tiles, by_nz, by_group, by_rows, by_rest;
+    void set(int tiles_m, int tiles_n, int rows_, int64_t nblk, int ztab_)
+    {
+        tiles = tiles_m * tiles_n;
+        nz = (int)nblk;
+        wgs = (int)(tiles * nblk);
+        ztab = ztab_;
+        rows = rows_;
+        full = tiles_m / rows * rows;
+        by_tiles.set(tiles);
+        by_nz.set(nz);
+        rest = tiles_m - full;
+        per_group = rows * tiles_n;
+        by_group.set(per_group);
+        by_rows.set(rows);
+        by_rest.set(rest ? rest : 1);
+    }
+    __host__ __device__ __forceinline__ void locate(uint32_t wg, int &tm, int &tn, int &bz) const
+    {
+        const uint32_t per = (uint32_t)wgs >> 3, rem = wgs & 7, xcd = wg & 7;
+        uint32_t id = xcd * per + (xcd < rem ? xcd : rem) + (wg >> 3);
+        bz = 0;
+        if (ztab) {
+            const uint32_t q = by_nz.div(id);
+            bz = (int)(id - q * nz);
+            id = q;
+        } else if (nz > 1) {
+            bz = (int)by_tiles.div(id);
+            id -= (uint32_t)bz * tiles;
+        }
+        const uint32_t group = by_group.div(id), in = id - group * per_group;
+        const int first = (int)group * rows;
+        const uint32_t col = first < full ? by_rows.div(in) : by_rest.div(in);
+        tn = (int)col;
+        tm = first + (int)(in - col * (first < full ? rows : rest));
+    }
+};
+
 struct GemmArgs {
     int64_t M, N, K;
     float alpha, beta;
@@ -13,7 +74,8 @@ struct GemmArgs {
     int64_t ldb, sb;
     half_t *C;
     int64_t ldc, sc;
-    int tiles_m, tiles_n;
+    int tiles_m, tiles_n;  // (gemm_direct.hip: in `walk` only)
+    TileWalk walk;
     // triangular structure of square attention operands (0 = none):
     //  1: only the lower triangle (n <= m) of C is wanted: tiles wholly above it are skipped
     //     and left unwritten;
@@ -24,7 +86,6 @@ struct GemmArgs {
     // For 2 and 3 the entries of A above the diagonal must be zero up to the next multiple
     // of 256 columns; beyond that they are never read.
     int tri;
-    int gm, xcd;          // tile walk: rows per group; 1 = XCD-banded numbering
     int pair;             // 1: a workgroup computes tile rows r and tiles_m - 1 - r (tri 2 / 3)
     // 1: B ([K][N] row-major) and C are addressed per block from the 16-byte boundary at or
     // below their first column (column window); set by the entry point when A is 16-byte
@@ -34,15 +95,16 @@ struct GemmArgs {
     // C + zc[z] (element offsets) instead of z times the batch strides; at most kMaxPtrBatch blocks
     int ztab;
     int64_t za[4], zb[4], zc[4];
-    // split > 1: the product in parts of K, whose fp32 sums go to part[part][M][ldp]
-    int split;
+    // part: the product in parts of K of split_tiles k tiles each, whose fp32 sums go to part[part][M][ldp]
+    int split_tiles;
     float *part;
     int64_t ldp;
+    int odd;              // C of any alignment and N: element by element
 };
 constexpr int kMaxPtrBatch = 4;
 constexpr int kTriPad = 256;
 
-// how gemm_mfma_launch cuts a product whose operands are 16-byte aligned: tile shapes as in gemm_mfma.hip
+// how gemm_direct_launch cuts a product whose operands are 16-byte aligned: tile shapes as in gemm_direct.hip
 struct GemmPlan {
     int tile, rest;      // shape of the (first) launch; of the second
     int64_t cols;        // > 0: columns of the first launch, the rest go to a second
@@ -52,11 +114,16 @@ struct GemmPlan {
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split);
 void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn);
 
-// align = 8 (16-byte aligned operands) or 4 (8-byte aligned, e.g. head_dim 100).  plan: null for the triangular and
-// column-window products and for align = 4; otherwise align = 8 is required of A and B, and of C unless `odd`
-// (C of any alignment and N).
-int gemm_mfma_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, int align, bool odd, const GemmPlan *plan,
-                     hipStream_t st);
+// Products of operands whose rows are at least 8-byte aligned (align = 4; 8: 16-byte aligned), with a triangular operand or
+// a column window among them.
+int gemm_mfma_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, int align, hipStream_t st);
+
+// Products of 16-byte aligned operands, cut by `plan` (p.part lent for its parts; p.odd: C of any alignment and N; tri and win
+// are not for these).
+int gemm_direct_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, const GemmPlan &plan, hipStream_t st);
+
+// tile rows per group of the walk of a launch of tiles_m x tiles_n tiles of bm x bn
+int gemm_walk_rows(int tiles_m, int tiles_n, int bm, int bn, int64_t nblk);
 
 int gemm_repack(const half_t *const src[2], half_t *const dst[2], const int64_t rows[2], const int64_t cols[2],
                 const int64_t ld[2], hipStream_t st);

@@ -1,19 +1,16 @@
-// Fast path of the f16 GEMM for operands whose rows are at least 8-byte aligned (every
-// projection, LM-head and attention GEMM of the step; head_dim 100 gives 8-byte alignment).
+// The f16 GEMM for operands whose rows are at least 8-byte aligned, where gemm_direct.hip does not take them: the products of
+// attention written as separate thunks (a triangular operand, per-head slabs addressed through a column window) and
+// operands aligned to 8 bytes only, where no workspace is lent for a copy.
 //
 //   C[M,N] = alpha op(A) op(B) + beta C,   f16 in, fp32 MFMA accumulate, f16 out.
 //
-// Block tile BM x BN x 64, WM x WN wavefronts, each owning BM / WM x BN / WN outputs as 32 x 32
+// Block tile 128 x 128 x 64, WM x WN wavefronts, each owning BM / WM x BN / WN outputs as 32 x 32
 // blocks that are interleaved with those of the other waves (32 WM rows / 32 WN columns apart).
-// The register path forms a block with v_mfma_f32_32x32x16_f16; the direct path, which carries the
-// large products of the step, as four 16 x 16 results of v_mfma_f32_16x16x32_f16: under a sustained
-// load the device is limited by power, and that instruction needs less of it per flop.  Shapes: the
-// direct path's are listed at enum Tile; the register path has 128 x 128 on 4 or 8 waves.
+// The register path forms a block with v_mfma_f32_32x32x16_f16, the direct path as four 16 x 16 results of
+// v_mfma_f32_16x16x32_f16.
 //
-// Two ways from global memory to LDS.  Through registers (any alignment >= 8 bytes, k tails; what is left for it
-// are operands aligned to 8 bytes only, where no workspace is lent for a copy, and triangular products
-// with a k tail): described below.  Direct (16-byte aligned operands, any K: a tail of K is loaded first, its
-// lanes beyond the end fetching zeros; all other products): global_load_lds_dwordx4 writes each wave's 1 KB straight into
+// Two ways from global memory to LDS.  Through registers (any alignment >= 8 bytes, k tails): described below.  Direct
+// (16-byte aligned operands, K a multiple of 64): global_load_lds_dwordx4 writes each wave's 1 KB straight into
 // LDS, NBUF - 1 k tiles ahead, with no staging registers, no LDS store instructions and no
 // transposes in registers; a k-contiguous operand lands in the swizzled [row][k] layout below (the swizzle
 // is applied to the global address), a k-strided one in its own [k][row] layout and is
@@ -45,6 +42,7 @@
 // the operand panels in their own L2.
 #include "common.h"
 #include "gemm_internal.h"
+#include "gemm_tile.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -53,30 +51,9 @@ using namespace cacti;
 
 namespace {
 
-constexpr int BK = 64;
-
-// what the lanes of a direct load beyond the end of K fetch
-__device__ __attribute__((aligned(16))) uint4 g_zero16;
-
-// 16 bytes from the lane's own address into LDS (lane l at m0 + 16 l)
-__device__ __forceinline__ void load_lds16(uint32_t m0, const void *src)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(m0), "v"(src) : "memory");
-}
-
 __device__ __forceinline__ int swz(int r) { return ((r >> 3) ^ r) & 7; }
-// The same for the direct path, whose fragments (v_mfma_f32_16x16x32_f16) are 16 rows x four 16-byte k
-// chunks per wave instruction instead of 32 rows x two: with swz() those reads take two passes through
-// LDS (measured: 286 against 493 GB/s per CU), with this one a single pass (484).  Period 32 rows.
-__device__ __forceinline__ int swz16(int r) { return ((r >> 2) ^ r) & 7; }
-
 // 16-byte chunk q (0..7) of tile row r
 __device__ __forceinline__ int lds_off(int r, int q) { return r * BK + ((q ^ swz(r)) << 3); }
-
-__device__ __forceinline__ const half_t *at(const half_t *base, uint32_t byte_off)
-{
-    return reinterpret_cast<const half_t *>(reinterpret_cast<const char *>(base) + byte_off);
-}
 
 // 8 halves as one 16-byte load (AL = 8) or two 8-byte loads (AL = 4: operands that are only
 // 8-byte aligned, whose extents are multiples of 4); off1 = offset of the second half
@@ -150,135 +127,6 @@ struct LoadKC {
     static constexpr int NREG = NL;
     static constexpr int NDMA = 0;
     __device__ __forceinline__ void dma(uint32_t, const half_t *, int64_t) const {}
-};
-
-// ---- k-contiguous operand fetched straight into LDS (global_load_lds_dwordx4: the 16 bytes
-// of lane l land at LDS address M0 + 16 l, no register staging and no LDS store instruction).
-// A wave fills 1 KB = 8 consecutive tile rows per instruction; the chunk swizzle of the LDS
-// layout is applied on the global side: the lane at chunk position p of row r fetches k chunk
-// p ^ f(r), which stays inside the row's 128-byte segment.  The loads are issued from inline
-// assembly, so the compiler neither counts them nor knows that they write LDS: the kernel
-// waits for them itself (vmcnt) before the barrier that publishes the tile.
-template <int ROWS, int NT>
-struct LoadKCD {
-    static_assert(ROWS * 8 % NT == 0, "whole instructions per wave");
-    static constexpr int NL = ROWS * 8 / NT;
-    uint32_t off[NL];              // byte offset of the lane's chunk from (row0, k = 0)
-
-    __device__ __forceinline__ void init(int64_t ld, int64_t rows_left, int64_t)
-    {
-#pragma unroll
-        for (int it = 0; it < NL; it++) {
-            const int c = threadIdx.x + it * NT;
-            const int r = c >> 3, q = (c & 7) ^ swz16(r);
-            const int64_t row = r < rows_left ? r : rows_left - 1;
-            off[it] = (uint32_t)((row * ld + q * 8) * 2);
-        }
-    }
-    // lds = byte address in LDS of the tile buffer to fill; origin = &op[row0][0]
-    __device__ __forceinline__ void dma(uint32_t lds, const half_t *origin, int64_t k0) const
-    {
-        const half_t *base = origin + k0;
-        const uint32_t wave = lds + (threadIdx.x & ~63u) * 16;
-#pragma unroll
-        for (int it = 0; it < NL; it++) {
-            const uint32_t m0 = __builtin_amdgcn_readfirstlane(wave + it * NT * 16);
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                         :
-                         : "s"(m0), "v"(off[it]), "s"(base)
-                         : "memory");
-        }
-    }
-    // the k tile with only `left` < BK values of k: chunks beyond them are zeros (left is a multiple of 8)
-    __device__ __forceinline__ void dma_tail(uint32_t lds, const half_t *base, int left) const
-    {
-        const uint32_t wave = lds + (threadIdx.x & ~63u) * 16;
-#pragma unroll
-        for (int it = 0; it < NL; it++) {
-            const int c = threadIdx.x + it * NT, r = c >> 3, q = (c & 7) ^ swz16(r);
-            const void *src = q * 8 < left ? (const void *)at(base, off[it]) : (const void *)&g_zero16;
-            load_lds16(__builtin_amdgcn_readfirstlane(wave + it * NT * 16), src);
-        }
-    }
-    // instruction `it` of the NL alone (base = origin + k0): lets the caller place each load between MFMAs
-    __device__ __forceinline__ void dma1(int it, uint32_t lds, const half_t *base) const
-    {
-        const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds + (threadIdx.x & ~63u) * 16 + it * NT * 16);
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     :
-                     : "s"(m0), "v"(off[it]), "s"(base)
-                     : "memory");
-    }
-    __device__ __forceinline__ const half_t *kbase(const half_t *origin, int64_t k0) const { return origin + k0; }
-    __device__ __forceinline__ void load(uint4 *, const half_t *, int64_t) const {}
-    __device__ __forceinline__ void store(const uint4 *, half_t *) const {}
-    static constexpr int NREG = 1;
-    static constexpr int NDMA = NL;
-};
-
-// ---- k-strided operand (memory [k][row]) fetched straight into LDS in its own layout,
-// [64 k][ROWS] with the 16-byte chunks of k row k swizzled by 2 (k & 3); the MFMA fragments
-// come out of it through ds_read_b64_tr_b16, which hands each lane of a 16-lane group 4
-// consecutive k of one row from a 4 k x 16 rows block (the swizzle spreads the 4 k rows of such
-// a block over all banks).  A wave fills 1 KB = 1024 / (2 ROWS) whole k rows per instruction.
-template <int ROWS, int NT>
-struct LoadKSD {
-    static constexpr int CPR = ROWS / 8;           // 16-byte chunks per k row
-    static_assert(BK * CPR % NT == 0 && CPR >= 8, "whole instructions per wave");
-    static constexpr int NL = BK * CPR / NT;
-    uint32_t off[NL];              // byte offset of the lane's chunk from (k = 0, row0)
-    int64_t ld;
-
-    __device__ __forceinline__ void init(int64_t ld_, int64_t rows_left, int64_t)
-    {
-        ld = ld_;
-#pragma unroll
-        for (int it = 0; it < NL; it++) {
-            const int c = threadIdx.x + it * NT;
-            const int k = c / CPR, q = (c % CPR) ^ (2 * (k & 3));
-            int64_t col = q * 8;
-            if (col > rows_left - 8) col = rows_left - 8;          // rows_left is a multiple of 8
-            off[it] = (uint32_t)((k * ld_ + col) * 2);
-        }
-    }
-    // lds = byte address in LDS of the tile buffer to fill; origin = &op[0][row0]
-    __device__ __forceinline__ void dma(uint32_t lds, const half_t *origin, int64_t k0) const
-    {
-        const half_t *base = origin + k0 * ld;
-        const uint32_t wave = lds + (threadIdx.x & ~63u) * 16;
-#pragma unroll
-        for (int it = 0; it < NL; it++) {
-            const uint32_t m0 = __builtin_amdgcn_readfirstlane(wave + it * NT * 16);
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                         :
-                         : "s"(m0), "v"(off[it]), "s"(base)
-                         : "memory");
-        }
-    }
-    // the k tile with only `left` < BK k rows: the rows beyond them are zeros
-    __device__ __forceinline__ void dma_tail(uint32_t lds, const half_t *base, int left) const
-    {
-        const uint32_t wave = lds + (threadIdx.x & ~63u) * 16;
-#pragma unroll
-        for (int it = 0; it < NL; it++) {
-            const int k = (threadIdx.x + it * NT) / CPR;
-            const void *src = k < left ? (const void *)at(base, off[it]) : (const void *)&g_zero16;
-            load_lds16(__builtin_amdgcn_readfirstlane(wave + it * NT * 16), src);
-        }
-    }
-    __device__ __forceinline__ void dma1(int it, uint32_t lds, const half_t *base) const
-    {
-        const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds + (threadIdx.x & ~63u) * 16 + it * NT * 16);
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     :
-                     : "s"(m0), "v"(off[it]), "s"(base)
-                     : "memory");
-    }
-    __device__ __forceinline__ const half_t *kbase(const half_t *origin, int64_t k0) const { return origin + k0 * ld; }
-    __device__ __forceinline__ void load(uint4 *, const half_t *, int64_t) const {}
-    __device__ __forceinline__ void store(const uint4 *, half_t *) const {}
-    static constexpr int NREG = 1;
-    static constexpr int NDMA = NL;
 };
 
 // ---- k-strided operand (memory [k][row]): item c -> row chunk c % (ROWS/8), k group
@@ -559,46 +407,16 @@ constexpr int min_waves(int bm, int bn, int waves, int nbuf)
     return w >= 2 ? 2 : 1;
 }
 
-// wait until at most n vector memory loads are outstanding (s_waitcnt vmcnt only)
-template <int N>
-__device__ __forceinline__ void wait_vmem()
-{
-    static_assert(N >= 0 && N < 64, "vmcnt has 6 bits");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-typedef __fp16 fp16x4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
-
-// 4 consecutive k of this lane's row out of a [k][row] tile (ds_read_b64_tr_b16)
-__device__ __forceinline__ uint2 lds_read_tr(const unsigned char *q)
-{
-    typedef __attribute__((address_space(3))) fp16x4_t *lds_ptr;
-    const fp16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_ptr)q);
-    uint2 r;
-    __builtin_memcpy(&r, &v, 8);
-    return r;
-}
-
-// E_ROWS: f16(alpha AB + beta C) as whole rows of C, whose pieces are 16-byte (AL = 8) or 8-byte aligned;
-// E_PART: the fp32 sums of one part of K, row-major with pitch ldp, for reduce_parts_kernel; E_ODD: as E_ROWS,
-// element by element, for a C of any alignment and N.
-enum : int { E_ROWS = 0, E_PART = 1, E_ODD = 2 };
-
 // DMA = true: both operands are fetched straight into LDS, NBUF - 1 tiles ahead, no register
 // stages (STAGES is 1); DMA = false: through registers, two LDS buffers.
-// EPI: what the epilogue writes (above).  M32 (direct, one 32 x 32 block per wave): v_mfma_f32_32x32x16_f16 with k in
-// ascending order, the sums of the register path bit for bit.
-template <bool TA, bool TB, int BM, int BN, int WM, int WN, int AL, bool KTAIL, int STAGES, int NBUF, bool DMA, int EPI, bool M32>
+template <bool TA, bool TB, int BM, int BN, int WM, int WN, int AL, bool KTAIL, int STAGES, int NBUF, bool DMA>
 __global__ void __launch_bounds__(WM * WN * 64, min_waves(BM, BN, WM * WN, NBUF))
 gemm_mfma_kernel(GemmArgs p)
 {
     // the whole argument block in scalar registers before anything else: read field by field where the control
     // flow first wants it, it costs five dependent round trips to memory before the first operand load
     asm volatile("" ::"s"(p.M), "s"(p.N), "s"(p.K), "s"(p.alpha), "s"(p.beta), "s"(p.A), "s"(p.lda), "s"(p.sa), "s"(p.B),
-                 "s"(p.ldb), "s"(p.sb), "s"(p.C), "s"(p.ldc), "s"(p.sc), "s"(p.tiles_m), "s"(p.tiles_n), "s"(p.tri),
-                 "s"(p.gm), "s"(p.xcd), "s"(p.pair), "s"(p.win), "s"(p.ztab));
-    static_assert(EPI == E_ROWS || (DMA && !M32), "split and odd products are direct ones");
-    static_assert(!M32 || (DMA && BM == 32 * WM && BN == 32 * WN), "one block per wave");
+                 "s"(p.ldb), "s"(p.sb), "s"(p.C), "s"(p.ldc), "s"(p.sc), "s"(p.tiles_m), "s"(p.tri), "s"(p.pair), "s"(p.win));
     static_assert(DMA ? (STAGES == 1 && AL == 8 && !KTAIL) : NBUF == 2,
                   "direct loads: 16-byte aligned operands, one register stage, their own k tail");
     constexpr bool TR_A = DMA && TA, TR_B = DMA && !TB;           // fragments by transposing reads
@@ -610,42 +428,11 @@ gemm_mfma_kernel(GemmArgs p)
     half_t *As = reinterpret_cast<half_t *>(smem_raw);            // [NBUF][BM*BK]
     half_t *Bs = As + NBUF * BM * BK;                             // [NBUF][BN*BK]
 
-    // XCD-aware numbering over the flattened (block of the batch, tile) sequence: dispatch
-    // order i lands on XCD i % 8; give each XCD a contiguous band.  With a batch that is a
-    // multiple of 8 an XCD then owns whole blocks of the batch, which also balances the
-    // triangular modes (their work per tile row grows or shrinks along M).
-    const int nb = gridDim.x;
-    int bid = blockIdx.x;
-    if (p.xcd) {
-        const int per = nb >> 3, rem = nb & 7;
-        const int xcd = bid & 7, idx = bid >> 3;
-        bid = xcd * per + (xcd < rem ? xcd : rem) + idx;
-    }
-    // pair mode (triangular operands): a workgroup takes tile row r and then tile row
-    // tiles_m - 1 - r, whose k ranges add up to the same length for every r
-    const int rows_m = p.pair ? p.tiles_m / 2 : p.tiles_m;
-    const int tiles = rows_m * p.tiles_n;
-    int64_t bz;
-    if (p.ztab) {
-        // a pointer-table batch is a handful of whole products that share an operand (the projections of one
-        // input, the weight gradients against one input): product fastest, so that the workgroups resident
-        // together on an XCD work on the same tile of every product and fetch the shared panel once
-        const int nz = nb / tiles;
-        bz = bid % nz;
-        bid /= nz;
-    } else {
-        bz = bid / tiles;
-        bid -= (int)bz * tiles;
-    }
-    // within a block of the batch, tiles are walked in groups of 8 tile rows x all tile
-    // columns, row fastest: the ~64 blocks resident on an XCD then form an 8 x 8 patch of C
-    // and each operand panel fetched into its L2 is shared by 8 blocks
-    const int GM = p.gm;
-    const int per_group = GM * p.tiles_n;
-    const int first_m = (bid / per_group) * GM;
-    const int gsz = min(GM, rows_m - first_m);
-    const int tm_base = first_m + (bid % per_group) % gsz;
-    const int tn = (bid % per_group) / gsz;
+    // A batch that is a multiple of 8 gives an XCD whole blocks of it, which also balances the triangular modes (their work
+    // per tile row grows or shrinks along M).  Pair mode (triangular operands): a workgroup takes tile row r and then tile
+    // row tiles_m - 1 - r, whose k ranges add up to the same length for every r.
+    int tm_base, tn, bz;
+    p.walk.locate(blockIdx.x, tm_base, tn, bz);
     for (int rep = 0; rep <= p.pair; rep++) {
     int tm = rep ? p.tiles_m - 1 - tm_base : tm_base;
     if (p.tri == 2 && !p.pair) tm = p.tiles_m - 1 - tm;           // longest k ranges first
@@ -655,16 +442,8 @@ gemm_mfma_kernel(GemmArgs p)
     if (p.tri == 1 && n0 > m0 + BM - 1) return;                   // uniform for the block
     if (p.tri == 2) nk = min(nk, (int)((m0 + BM + BK - 1) / BK));
     if (p.tri == 3) kt0 = (int)(m0 / BK);
-    const int64_t part = bz;
-    if (EPI == E_PART) {
-        // the "blocks of the batch" are the parts of K: the same operands, a range of k tiles each
-        const int per = (nk + p.split - 1) / p.split;
-        kt0 = (int)part * per;
-        nk = min(nk, kt0 + per);
-        bz = 0;
-    }
 
-    const half_t *A = p.A + (p.ztab ? p.za[bz] : bz * p.sa);
+    const half_t *A = p.A + (int64_t)bz * p.sa;
     // column window (p.win): the [k][n] operand B and C of block bz start 8 bytes off a 16-byte
     // boundary when bz * sb is an odd multiple of 4 (head_dim 100).  Both are then addressed
     // from the boundary before: column `shift` of this view is the block's column 0, columns
@@ -672,8 +451,8 @@ gemm_mfma_kernel(GemmArgs p)
     // and never stored.
     const int shift = p.win ? (int)((bz * p.sb) & 7) : 0;
     const int64_t nw = p.N + shift;                               // end of the window
-    const half_t *B = p.B + (p.ztab ? p.zb[bz] : bz * p.sb) - shift;
-    half_t *C = p.C + (p.ztab ? p.zc[bz] : bz * p.sc) - shift;
+    const half_t *B = p.B + (int64_t)bz * p.sb - shift;
+    half_t *C = p.C + (int64_t)bz * p.sc - shift;
     // tile origins: &op[row0][0] for a k-contiguous operand, &op[0][row0] for a strided one
     const half_t *Ao = TA ? A + m0 : A + m0 * p.lda;
     const half_t *Bo = TB ? B + n0 * p.ldb : B + n0;
@@ -714,35 +493,18 @@ gemm_mfma_kernel(GemmArgs p)
     // direct loads: the first NBUF tiles are requested here, before the accumulators are cleared and the
     // fragment addresses worked out (some thousand cycles of set-up that need not stand in front of them)
     if constexpr (DMA) {
-        // A tail of K goes first, so that every later load is of a whole tile: step t multiplies tile t - 1 and
-        // step 0 the last, incomplete one (only products without a triangular operand have a tail here).  M32
-        // keeps the order and loads it in its turn.
-        const int ktail = (int)(p.K % BK);
-        auto load_tail = [&](int u) __attribute__((always_inline)) {
-            const int64_t k0 = p.K - ktail;
-            la.dma_tail((uint32_t)(uintptr_t)(As + u * BM * BK), la.kbase(Ao, k0), ktail);
-            lb.dma_tail((uint32_t)(uintptr_t)(Bs + u * BN * BK), lb.kbase(Bo, k0), ktail);
-        };
-        if (!M32 && ktail) {
-            if (kt0 == 0) load_tail(0);
-            Ao = la.kbase(Ao, -BK);
-            Bo = lb.kbase(Bo, -BK);
-        }
 #pragma unroll
-        for (int u = 0; u < NBUF; u++) {
-            if (M32 && ktail && kt0 + u == nk - 1) {
-                load_tail(u);
-            } else if (kt0 + u < nk && (M32 || kt0 + u > 0 || !ktail)) {
+        for (int u = 0; u < NBUF; u++)
+            if (kt0 + u < nk) {
                 la.dma((uint32_t)(uintptr_t)(As + u * BM * BK), Ao, (int64_t)(kt0 + u) * BK);
                 lb.dma((uint32_t)(uintptr_t)(Bs + u * BN * BK), Bo, (int64_t)(kt0 + u) * BK);
             }
-        }
         __builtin_amdgcn_sched_barrier(0);
     }
 
     // direct path: 16 x 16 results of v_mfma_f32_16x16x32_f16, [A fragment][B fragment]; lane l holds row
     // l % 16 of the fragment pair's block and columns 4 (l / 16) .. + 3
-    float4_t c16[DMA && !M32 ? 2 * TM : 1][DMA && !M32 ? 2 * TN : 1];
+    float4_t c16[DMA ? 2 * TM : 1][DMA ? 2 * TN : 1];
     const int l16 = lane & 15, kg = lane >> 4;
     float16_t acc[TM][TN];
 #pragma unroll
@@ -889,9 +651,9 @@ gemm_mfma_kernel(GemmArgs p)
         constexpr int NMH = TM * NB;                              // MFMAs of a half
         constexpr int RA = (TR_A ? 2 : 1) * TM, RB = (TR_B ? 2 : 1) * NB;   // LDS reads: A fragments of a half, all B
 #pragma unroll
-        for (int a = 0; a < (M32 ? 1 : NA); a++)
+        for (int a = 0; a < NA; a++)
 #pragma unroll
-            for (int b = 0; b < (M32 ? 1 : NB); b++) c16[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+            for (int b = 0; b < NB; b++) c16[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
         half8_t fa[2][TM], fb[2][NB];                             // A fragments of a half, B fragments of a k step
         // [row][k] tiles: halves offset of the lane's row in a block's upper / lower 16 rows, and its swizzle
         const int ar[2] = {wm * 32 + l16, wm * 32 + 16 + l16}, br[2] = {wn * 32 + l16, wn * 32 + 16 + l16};
@@ -975,86 +737,6 @@ gemm_mfma_kernel(GemmArgs p)
         else wait_vmem<0>();
         __syncthreads();
         int t = kt0, cb = 0;
-        if constexpr (TM * TN == 1) {
-        // One 32 x 32 block per wave: a half is two MFMAs (32 cycles), far less than an LDS read takes, so
-        // reads issued one half ahead leave the wave waiting in every half.  Here the fragments of a whole
-        // k tile (two register sets) are read while the eight MFMAs of the tile before run: behind the
-        // barrier of tile t (tile t + 1 has landed; every wave holds tile t in registers, the barrier's own
-        // wait for LDS sees to that) come the reads of tile t + 1, the loads of tile t + NBUF into the
-        // buffer of tile t, and then the MFMAs of tile t.
-        half8_t ga[2][2][NA], gb[2][2][NB];
-        auto read_tile = [&](auto set_c, int buf) __attribute__((always_inline)) {
-            constexpr int S = decltype(set_c)::value;
-            if constexpr (M32) {
-                // fragments of the four k steps of 16: ks of ga / gb [ks / 2][ks % 2]
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) {
-                    const half_t *as = As + buf * BM * BK, *bs = Bs + buf * BN * BK;
-                    const int q = ks * 2 + lh;
-                    ga[S][ks >> 1][ks & 1] =
-                        TR_A ? frag_tr(reinterpret_cast<const unsigned char *>(as) + atr + ks * 16 * (BM * 2), BM * 2)
-                             : *reinterpret_cast<const half8_t *>(as + ar0 * BK + ((q ^ swz16(ar0)) << 3));
-                    gb[S][ks >> 1][ks & 1] =
-                        TR_B ? frag_tr(reinterpret_cast<const unsigned char *>(bs) + btr + ks * 16 * (BN * 2), BN * 2)
-                             : *reinterpret_cast<const half8_t *>(bs + br0 * BK + ((q ^ swz16(br0)) << 3));
-                }
-                return;
-            }
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++) {
-#pragma unroll
-                for (int a = 0; a < NA; a++) ga[S][ks][a] = read_a(buf, ks, a);
-#pragma unroll
-                for (int b = 0; b < NB; b++) gb[S][ks][b] = read_b(buf, ks, b);
-            }
-        };
-        auto body = [&](auto set_c, auto main_c) __attribute__((always_inline)) {
-            constexpr int S = decltype(set_c)::value;
-            constexpr bool MAIN = decltype(main_c)::value;
-            const int nb = next_buf(cb);
-            if (MAIN || t + 1 < nk) {
-                if (MAIN) wait_vmem<(NBUF - 2) * ND>();
-                else wait_vmem<0>();
-                __syncthreads();
-                read_tile(std::integral_constant<int, S ^ 1>{}, nb);
-                __builtin_amdgcn_sched_barrier(0);
-                if (!MAIN && M32 && p.K % BK != 0 && t + NBUF == nk - 1) {
-                    const int64_t k0 = (int64_t)(nk - 1) * BK;
-                    la.dma_tail(lds_addr(As + cb * BM * BK), la.kbase(Ao, k0), (int)(p.K - k0));
-                    lb.dma_tail(lds_addr(Bs + cb * BN * BK), lb.kbase(Bo, k0), (int)(p.K - k0));
-                } else if (MAIN || t + NBUF < nk) {
-                    issue_all(t + NBUF, cb);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (M32) {
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++)
-                    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(gb[S][ks >> 1][ks & 1], ga[S][ks >> 1][ks & 1], acc[0][0], 0, 0, 0);
-            } else
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-                for (int a = 0; a < NA; a++)
-#pragma unroll
-                    for (int b = 0; b < NB; b++)
-                        c16[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(gb[S][ks][b], ga[S][ks][a], c16[a][b], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            cb = nb;
-            t++;
-        };
-        read_tile(std::integral_constant<int, 0>{}, 0);
-        const int nk_whole = M32 && p.K % BK != 0 ? nk - 1 : nk;
-        while (t + NBUF + 1 < nk_whole) {                         // both steps load whole tiles
-            body(std::integral_constant<int, 0>{}, std::true_type{});
-            body(std::integral_constant<int, 1>{}, std::true_type{});
-        }
-        while (t < nk) {
-            body(std::integral_constant<int, 0>{}, std::false_type{});
-            if (t < nk) body(std::integral_constant<int, 1>{}, std::false_type{});
-        }
-        __syncthreads();
-        } else {
 #pragma unroll
         for (int u = 0; u < TM + NB; u++) next_read(u, 0, 0, 0);
         for (; t + NBUF < nk; t++) {                              // every load of the body lies inside K
@@ -1097,7 +779,6 @@ gemm_mfma_kernel(GemmArgs p)
             cb = nb;
         }
         __syncthreads();                                          // every wave is done with the operand buffers
-        }
     } else {
         la.load(ra[0], Ao, (int64_t)kt0 * BK);
         lb.load(rb[0], Bo, (int64_t)kt0 * BK);
@@ -1132,20 +813,6 @@ gemm_mfma_kernel(GemmArgs p)
         if (TAIL > 4 && kt + 4 < nk) { step(std::integral_constant<int, 4 % STAGES>{}, std::false_type{}, kt + 4, cb); cb = next_buf(cb); }
     }
 
-    if constexpr (EPI == E_PART) {
-        // a lane's 4 consecutive columns of a row are 16 bytes of the part, four lanes a 64-byte run
-        float *out = p.part + part * p.M * p.ldp;
-#pragma unroll
-        for (int a = 0; a < 2 * TM; a++) {
-            const int64_t m = m0 + (a >> 1) * (32 * WM) + wm * 32 + (a & 1) * 16 + l16;
-#pragma unroll
-            for (int b = 0; b < 2 * TN; b++) {
-                const int64_t n = n0 + (b >> 1) * (32 * WN) + wn * 32 + (b & 1) * 16 + kg * 4;
-                if (m < p.M && n < p.N) *reinterpret_cast<float4_t *>(out + m * p.ldp + n) = c16[a][b];
-            }
-        }
-        return;
-    }
     // Epilogue through LDS (the operand buffers are free after the last barrier): a lane
     // holds row m = .. + l32 and, per accumulator group q, the 4 consecutive columns
     // n = .. + 8 q + 4 lh + {0..3}, i.e. 8 bytes in each of 32 different rows of C; staged as
@@ -1165,7 +832,7 @@ gemm_mfma_kernel(GemmArgs p)
     // stored (the general loop below waits for every piece in turn: 9,000 cycles more per workgroup measured)
     // (tiles of up to 256 x 128: the larger ones have no registers for it and spill in their main loop with it)
     constexpr bool C_BATCH = BM * BN <= 256 * 128 && BM * CPRC % NT == 0;
-    const bool c_inside = C_BATCH && AL == 8 && EPI == E_ROWS && shift == 0 && m0 + BM <= p.M && n0 + BN <= nw;
+    const bool c_inside = C_BATCH && AL == 8 && shift == 0 && m0 + BM <= p.M && n0 + BN <= nw;
     if (has_beta && c_inside) {
         constexpr int NC = C_BATCH ? BM * CPRC / NT : 1;
         uint4 old[NC];
@@ -1187,12 +854,7 @@ gemm_mfma_kernel(GemmArgs p)
             const bool lo = m < p.M && n >= shift && n < nw, hi = m < p.M && n + 4 >= shift && n + 4 < nw;
             const half_t *cp = C + m * p.ldc + n;
             uint4 v = make_uint4(0, 0, 0, 0);
-            if (EPI == E_ODD) {
-                half_t *e = reinterpret_cast<half_t *>(&v);
-#pragma unroll
-                for (int j = 0; j < 8; j++)
-                    if (m < p.M && n + j < p.N) e[j] = cp[j];
-            } else if (AL == 8 && lo && hi) {
+            if (AL == 8 && lo && hi) {
                 v = *reinterpret_cast<const uint4 *>(cp);
             } else {
                 if (lo) {
@@ -1210,7 +872,7 @@ gemm_mfma_kernel(GemmArgs p)
         }
         __syncthreads();
     }
-    if constexpr (DMA && !M32) {
+    if constexpr (DMA) {
 #pragma unroll
         for (int a = 0; a < 2 * TM; a++) {
             const int row = (a >> 1) * (32 * WM) + wm * 32 + (a & 1) * 16 + l16;
@@ -1256,15 +918,6 @@ gemm_mfma_kernel(GemmArgs p)
         }
 }
     __syncthreads();
-    if constexpr (EPI == E_ODD) {
-        // consecutive lanes take consecutive elements of a row
-        for (int c = threadIdx.x; c < BM * BN; c += NT) {
-            const int row = c / BN, col = c % BN;
-            if (m0 + row < p.M && n0 + col < p.N)
-                C[(m0 + row) * p.ldc + n0 + col] = Cs[row * BN + ((((col >> 3) ^ (row & CSW)) << 3) | (col & 7))];
-        }
-        return;
-    }
     for (int c = threadIdx.x; c < BM * CPRC; c += NT) {
         const int row = c / CPRC, cc = c % CPRC;
         const int64_t m = m0 + row, n = n0 + cc * 8;
@@ -1283,267 +936,37 @@ gemm_mfma_kernel(GemmArgs p)
     }
 }
 
-// C = f16(alpha sum of the parts + beta C), four columns per lane; the parts are added in order.  VEC: N and the rows
-// of C allow 8-byte accesses.
-template <bool VEC>
-__global__ void __launch_bounds__(256)
-reduce_parts_kernel(int64_t M, int64_t N, int64_t ldp, int split, const float *__restrict__ part, float alpha, float beta,
-                    half_t *__restrict__ C, int64_t ldc)
-{
-    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (i >= M * ldp) return;
-    const int64_t m = i / ldp, n = i - m * ldp;
-    float4_t s = *reinterpret_cast<const float4_t *>(part + i);
-    for (int k = 1; k < split; k++) s += *reinterpret_cast<const float4_t *>(part + k * M * ldp + i);
-    half_t *cp = C + m * ldc + n;
-    half4_t o, old = {0, 0, 0, 0};
-    const bool has_beta = beta != 0.f;
-    if (VEC) {
-        if (has_beta) old = *reinterpret_cast<const half4_t *>(cp);
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (has_beta && n + r < N) old[r] = cp[r];
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++) o[r] = has_beta ? f2h(alpha * s[r] + beta * h2f(old[r])) : f2h(alpha * s[r]);
-    if (VEC) {
-        *reinterpret_cast<half4_t *>(cp) = o;
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (n + r < N) cp[r] = o[r];
-    }
-}
-
-// Operands of any alignment as operands the direct kernels take: rows of `cols` halves, `ld` apart, to rows of `out_cols`
-// = cols rounded up to 8 (zeros behind cols), 16-byte aligned.  One lane per 16-byte piece, both operands in one launch.
-struct RepackArgs {
-    const half_t *src[2];
-    half_t *dst[2];
-    int64_t rows[2], cols[2], ld[2];
-};
-__global__ void __launch_bounds__(256) repack_kernel(RepackArgs p)
-{
-    const int z = blockIdx.y;
-    const int64_t per_row = (p.cols[z] + 7) / 8, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (!p.dst[z] || i >= p.rows[z] * per_row) return;
-    const int64_t row = i / per_row, c = (i - row * per_row) * 8;
-    const half_t *src = p.src[z] + row * p.ld[z] + c;
-    const int64_t left = p.cols[z] - c;
-    h8 v;
-#pragma unroll
-    for (int j = 0; j < 8; j++) v.v[j] = j < left ? src[j] : (half_t)0.f;
-    st8(p.dst[z] + i * 8, v);
-}
-
-template <bool TA, bool TB, int BM, int BN, int WM, int WN, int AL, bool KTAIL, int STAGES, int NBUF = 2, bool DMA = false,
-          int EPI = E_ROWS, bool M32 = false>
+template <bool TA, bool TB, int BM, int BN, int WM, int WN, int AL, bool KTAIL, int STAGES, int NBUF = 2, bool DMA = false>
 int launch_cfg(GemmArgs p, int64_t nblk, hipStream_t st)
 {
     p.tiles_m = (int)((p.M + BM - 1) / BM);
-    p.tiles_n = (int)((p.N + (p.win ? 4 : 0) + BN - 1) / BN);
+    const int tiles_n = (int)((p.N + (p.win ? 4 : 0) + BN - 1) / BN);
     const size_t smem = (size_t)NBUF * (BM + BN) * BK * sizeof(half_t);
-    auto kern = gemm_mfma_kernel<TA, TB, BM, BN, WM, WN, AL, KTAIL, STAGES, NBUF, DMA, EPI, M32>;
+    auto kern = gemm_mfma_kernel<TA, TB, BM, BN, WM, WN, AL, KTAIL, STAGES, NBUF, DMA>;
     static DeviceOnce attr_set;                   // one per instantiation
     if (!attr_set.fresh()) {
         CACTI_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                       (int)smem));
         attr_set.mark();
     }
-    if (p.gm <= 0) {
-        // tile rows per group of the walk.  An XCD works on a band of tiles / 8 consecutive tiles,
-        // i.e. on gm tile rows x band / gm tile columns at a time, and fetches gm A panels and
-        // band / gm B panels per k tile into its L2: the power of two with the fewest rows fetched.  (Run
-        // time hardly reacts, the re-reads being served by the MALL; the L2-miss traffic does:
-        // -25 % at 2048 x 3200 x 8640.)
-        p.gm = 8;
-        if (nblk == 1) {
-            const double band = (double)p.tiles_m * p.tiles_n / 8.0;
-            double best = 0;
-            for (int g = 8; g >= 2; g /= 2) {             // ties: the larger group
-                const double fetched = g * (double)BM + band / g * (double)BN;
-                if (best == 0 || fetched < best) {
-                    best = fetched;
-                    p.gm = g;
-                }
-            }
-        }
-    }
     p.pair = (p.tri >= 2 && p.tiles_m % 2 == 0) ? 1 : 0;
-    const int64_t nwg = (int64_t)(p.pair ? p.tiles_m / 2 : p.tiles_m) * p.tiles_n * nblk;
+    const int rows_m = p.pair ? p.tiles_m / 2 : p.tiles_m;
+    const int64_t nwg = (int64_t)rows_m * tiles_n * nblk;
     CACTI_REQUIRE(nwg < (int64_t)1 << 31, CACTI_E_NOTIMPL, "gemm: %lld workgroups exceed the grid limit",
                   (long long)nwg);
+    p.walk.set(rows_m, tiles_n, gemm_walk_rows(rows_m, tiles_n, BM, BN, nblk), nblk, 0);
     dim3 grid((unsigned)nwg), block(WM * WN * 64);
     hipLaunchKernelGGL(kern, grid, block, smem, st, p);
     return launch_status("gemm_mfma");
 }
 
-// Tile shapes of the direct kernels: 64 x 64 and 128 x 64 on 4 waves (two workgroups per CU), 128 x 128, 256 x 128,
-// 256 x 256 (128 x 64 per wave) and 256 x 192 (64 x 96 per wave) on 8 waves (one per CU).
-// T64_SMALL: 64 x 64 with the 32 x 32 x 16 instruction, for outputs of up to kSmallOutput elements.
-enum Tile : int { T64, T128_64, T128, T256_128, T256_192, T256, N_TILES, T64_SMALL = N_TILES };
-
-template <bool TA, bool TB, int EPI>
-int launch_direct(int tile, const GemmArgs &p, int64_t nblk, hipStream_t st)
-{
-    switch (tile) {
-        case T64: return launch_cfg<TA, TB, 64, 64, 2, 2, 8, false, 1, 4, true, EPI>(p, nblk, st);
-        case T128_64: return launch_cfg<TA, TB, 128, 64, 2, 2, 8, false, 1, 3, true, EPI>(p, nblk, st);
-        case T128: return launch_cfg<TA, TB, 128, 128, 2, 4, 8, false, 1, 3, true, EPI>(p, nblk, st);
-    }
-    if constexpr (EPI != E_PART)                                  // (a product that needs a split has few tiles: small ones)
-        if (tile == T256_128) return launch_cfg<TA, TB, 256, 128, 4, 2, 8, false, 1, 3, true, EPI>(p, nblk, st);
-    if constexpr (EPI == E_ROWS) {
-        switch (tile) {
-            case T64_SMALL: return launch_cfg<TA, TB, 64, 64, 2, 2, 8, false, 1, 4, true, EPI, true>(p, nblk, st);
-            case T256_192: return launch_cfg<TA, TB, 256, 192, 4, 2, 8, false, 1, 2, true, EPI>(p, nblk, st);
-            case T256: return launch_cfg<TA, TB, 256, 256, 2, 4, 8, false, 1, 2, true, EPI>(p, nblk, st);
-        }
-    }
-    set_error("gemm: no tile %d", tile);
-    return CACTI_E_STATE;
-}
-
-// What a product costs on a tile, in microseconds: a start and end of `fixed`, then per k tile the time of a full
-// set of resident workgroups (`resident` per CU: `full`), for the last, partly filled set `first` + `load` x the share
-// of the CUs that are busy where no CU has more than one, and `round` for every further set.  Fitted (least squares
-// of the log) to 338 products measured on MI355X: M 33 .. 8640, N 256 .. 32000, K 37 .. 32000, the three layouts;
-// rms error 6-8 % per tile.  On 322 others of the same ranges (profiles/gemm_tile_times_by_shape.txt has the times of every
-// tile) it is 9-11 % for the tiles of 128 x 128 and more and 18-21 % for the smaller two, whose worst products stream
-// operands of hundreds of MB through few tiles; the tile picked by it is 0.8 % slower than the best one in the mean
-// and 34 % at worst (41 x 18096 x 28216).
-struct TileCost {
-    int bm, bn, resident;
-    double fixed, first, load, full, round;
-};
-constexpr TileCost kTileCost[N_TILES] = {
-    {64, 64, 2, 3.947, 0.226, 0.042, 0.385, 2.187},    {128, 64, 2, 4.429, 0.277, 0.069, 0.562, 2.748},
-    {128, 128, 1, 4.677, 0.394, 0.113, 0.507, 3.479},  {256, 128, 1, 5.582, 0.621, 0.208, 0.829, 5.417},
-    {256, 192, 1, 6.801, 0.878, 0.291, 1.169, 6.229},  {256, 256, 1, 7.843, 1.094, 0.392, 1.486, 7.759},
-};
-
-constexpr int64_t kSmallOutput = 1 << 18;
-
-double tile_cost(int64_t cus, int tile, int64_t M, int64_t N, int64_t nz, int64_t ktiles)
-{
-    const TileCost &t = kTileCost[tile];
-    const int64_t wg = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn) * nz, set = cus * t.resident;
-    const int64_t sets = wg / set;
-    const double rest = (double)(wg - sets * set) / (double)cus;
-    const double last = rest == 0 ? 0 : rest <= 1 ? t.first + t.load * rest : t.full;
-    return t.fixed + (double)ktiles * ((double)sets * t.full + last) + t.round * (double)(sets + (rest > 0) - 1);
-}
-
-}  // namespace
-
-namespace cacti {
-
-void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn)
-{
-    if (tile == T64_SMALL) tile = T64;
-    *bm = kTileCost[tile].bm;
-    *bn = kTileCost[tile].bn;
-}
-
-// How a product of 16-byte aligned operands is cut.  One workgroup takes one tile; a launch runs in sets of resident
-// workgroups, and a nearly empty last set costs as much as a full one.  Considered: every tile shape by itself; for the
-// 256-wide ones also the columns of the full sets in one launch and the rest on smaller tiles in a second (2048 x 8640 x
-// 3200: 256 tiles of 256 x 256 and 448 columns); and, where the caller has a workspace (may_split), up to 8 parts of K
-// for products with fewer tiles than CUs and a long K, whose workgroups would otherwise run 100 k tiles one after
-// another on a fraction of the CUs (37 x 3200 x 8640: 50 tiles; the parts and their sum cost a launch and
-// 8 bytes per part and element).
-GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split)
-{
-    const int64_t kt = (K + BK - 1) / BK, cus = device_cus();
-    GemmPlan best = {T64, T64, 0, 1};
-    double best_cost = 1e30;
-    // A small output has about 64 tiles of 64 x 64 (or one row or column of them), the shape that is best for it while they
-    // run on the device all at once; more of them are cut by cost like any other product (measured, 64 x 64 -> by cost: 16
-    // products of 512 x 512 x 1024 19.3 -> 13.6 us, 32 of them 37.2 -> 23.0, 64 of 512 x 512 x 192 30.8 -> 18.9; at 8, 512
-    // tiles, both are 10.4).  The device is nowhere near its power limit with a small output, so the instruction is free to be
-    // the one whose sums the register path has always formed.  Up to kMaxPtrBatch products in a launch go by the
-    // single product alone: a group has the bits of separate launches.
-    const int64_t tiles64 = (M + 63) / 64 * ((N + 63) / 64);
-    const bool small = M * N <= kSmallOutput && (nz <= kMaxPtrBatch || tiles64 * nz <= kTileCost[T64].resident * cus);
-    if (small) {
-        best = {T64_SMALL, T64, 0, 1};
-        best_cost = tile_cost(cus, T64, M, N, nz, kt);
-    }
-    for (int t = 0; t < N_TILES && !small; t++) {
-        const double c = tile_cost(cus, t, M, N, nz, kt);
-        if (c < best_cost) {
-            best_cost = c;
-            best = {t, T64, 0, 1};
-        }
-    }
-    for (int t = T256_128; t < N_TILES && !small; t++) {
-        const int64_t tiles_m = (M + 255) / 256 * nz, bn = kTileCost[t].bn, tiles_n = (N + bn - 1) / bn;
-        const int64_t cols = tiles_m * tiles_n / cus * cus / tiles_m * bn;
-        if (cols <= 0 || cols >= N) continue;
-        for (int r = T64; r <= T128; r++) {
-            const double c = tile_cost(cus, t, M, cols, nz, kt) + tile_cost(cus, r, M, N - cols, nz, kt);
-            if (c < best_cost) {
-                best_cost = c;
-                best = {t, r, cols, 1};
-            }
-        }
-    }
-    if (may_split && nz == 1)
-        for (int t = T64; t <= T128; t++)
-            for (int s = 2; s <= 8; s++) {
-                const int64_t per = (kt + s - 1) / s;
-                if (per < 4 || (kt + per - 1) / per != s) continue;           // parts of some length, none empty
-                const double c = tile_cost(cus, t, M, N, s, per) + 4.0 + (double)(M * N) * s * 8.0 / 4e6;
-                if (c < best_cost) {
-                    best_cost = c;
-                    best = {t, T64, 0, s};
-                }
-            }
-    return best;
-}
-
-}  // namespace cacti
-
-namespace {
-
 template <bool TA, bool TB>
-int launch_plan(const GemmPlan &plan, const GemmArgs &p, int64_t nblk, bool odd, hipStream_t st)
+int launch_any(const GemmArgs &p, int64_t nblk, int align, hipStream_t st)
 {
-    if (plan.split > 1) {
-        GemmArgs q = p;
-        q.split = plan.split;
-        const int rc = launch_direct<TA, TB, E_PART>(plan.tile, q, plan.split, st);
-        if (rc) return rc;
-        const unsigned grid = (unsigned)((p.M * p.ldp + 1023) / 1024);
-        const auto reduce = p.N % 4 == 0 && p.ldc % 4 == 0 && aligned(p.C, 8) ? reduce_parts_kernel<true> : reduce_parts_kernel<false>;
-        hipLaunchKernelGGL(reduce, dim3(grid), dim3(256), 0, st, p.M, p.N, p.ldp, plan.split, p.part, p.alpha, p.beta, p.C, p.ldc);
-        return launch_status("gemm_reduce_parts");
-    }
-    if (odd) {
-        const int tile = plan.tile == T64_SMALL ? T64 : plan.tile;
-        return launch_direct<TA, TB, E_ODD>(tile < T256_128 ? tile : (int)T256_128, p, nblk, st);
-    }
-    if (plan.cols > 0) {
-        GemmArgs a = p, b = p;
-        a.N = plan.cols;
-        b.N = p.N - a.N;
-        b.B = p.B + (TB ? a.N * p.ldb : a.N);
-        b.C = p.C + a.N;
-        const int rc = launch_direct<TA, TB, E_ROWS>(plan.tile, a, nblk, st);
-        return rc ? rc : launch_direct<TA, TB, E_ROWS>(plan.rest, b, nblk, st);
-    }
-    return launch_direct<TA, TB, E_ROWS>(plan.tile, p, nblk, st);
-}
-
-template <bool TA, bool TB>
-int launch_any(const GemmArgs &p, int64_t nblk, int align, bool odd, const GemmPlan *plan, hipStream_t st)
-{
-    if (plan) return launch_plan<TA, TB>(*plan, p, nblk, odd, st);
     const bool ktail = (p.K % BK) != 0;
     // Per-head slabs addressed through a column window, and the triangular products of attention: 128 x 128 tiles
     // on 8 waves, three LDS buffers (-5 us per launch against the register path with 8 waves).
-    if (align >= 8 && (p.win || !ktail)) return launch_direct<TA, TB, E_ROWS>(T128, p, nblk, st);
+    if (align >= 8 && (p.win || !ktail)) return launch_cfg<TA, TB, 128, 128, 2, 4, 8, false, 1, 3, true>(p, nblk, st);
     // 8-byte aligned operands (the attention blocks): 8 waves of 64 x 32 on the 128 x 128 tile;
     // with one workgroup per CU (32 heads x 8 tile-row pairs) two waves per SIMD hide each
     // other's LDS latency (-9..13 % against 4 waves of 64 x 64)
@@ -1556,34 +979,12 @@ int launch_any(const GemmArgs &p, int64_t nblk, int align, bool odd, const GemmP
 
 namespace cacti {
 
-int gemm_mfma_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, int align, bool odd, const GemmPlan *plan, hipStream_t st)
+int gemm_mfma_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, int align, hipStream_t st)
 {
-    GemmArgs q = p;
-    q.gm = -1;                                    // rows of tiles per group: chosen per launch
-    q.xcd = 1;                                    // consecutive tiles to the workgroups of one XCD
-    if (!ta && !tb) return launch_any<false, false>(q, nblk, align, odd, plan, st);
-    if (!ta && tb) return launch_any<false, true>(q, nblk, align, odd, plan, st);
-    if (ta && !tb) return launch_any<true, false>(q, nblk, align, odd, plan, st);
-    return launch_any<true, true>(q, nblk, align, odd, plan, st);
-}
-
-// a copy of up to two operands in the layout of the direct kernels (dst null: none of that one)
-int gemm_repack(const half_t *const src[2], half_t *const dst[2], const int64_t rows[2], const int64_t cols[2], const int64_t ld[2],
-                hipStream_t st)
-{
-    RepackArgs p;
-    int64_t most = 0;
-    for (int z = 0; z < 2; z++) {
-        p.src[z] = src[z];
-        p.dst[z] = dst[z];
-        p.rows[z] = rows[z];
-        p.cols[z] = cols[z];
-        p.ld[z] = ld[z];
-        if (dst[z]) most = std::max(most, rows[z] * ((cols[z] + 7) / 8));
-    }
-    CACTI_REQUIRE((most + 255) / 256 < (int64_t)1 << 31, CACTI_E_NOTIMPL, "gemm: operand too large to lay out");
-    hipLaunchKernelGGL(repack_kernel, dim3((unsigned)((most + 255) / 256), 2), dim3(256), 0, st, p);
-    return launch_status("gemm_repack");
+    if (!ta && !tb) return launch_any<false, false>(p, nblk, align, st);
+    if (!ta && tb) return launch_any<false, true>(p, nblk, align, st);
+    if (ta && !tb) return launch_any<true, false>(p, nblk, align, st);
+    return launch_any<true, true>(p, nblk, align, st);
 }
 
 }  // namespace cacti

@@ -7,7 +7,7 @@ writes cacti_amd/gemm_traffic.json: per timing label of a product the mean FETCH
 its launches (KiB per dispatch; a product that runs as two launches adds them) and the bytes they stand
 for, bytes = (FETCH_FACTOR * FETCH_SIZE + WRITE_FACTOR * WRITE_SIZE) * 1024: a streaming copy kernel of
 known size reads FETCH_SIZE = half its bytes and WRITE_SIZE = its bytes on this device.  The file also
-records the SHA-256 of csrc/gemm_mfma.hip; load_current() returns the table only while that source is
+records the SHA-256 of csrc/gemm_direct.hip; load_current() returns the table only while that source is
 the one the figures were taken on.
 """
 import csv
@@ -18,7 +18,7 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 TABLE = os.path.join(HERE, "gemm_traffic.json")
-KERNEL_SOURCE = os.path.join(HERE, "csrc", "gemm_mfma.hip")
+KERNEL_SOURCE = os.path.join(HERE, "csrc", "gemm_direct.hip")
 LAUNCHES = 4
 FETCH_FACTOR, WRITE_FACTOR = 2.0, 1.0
 
@@ -53,7 +53,7 @@ def _dispatches(path):
     rows = []
     with open(path) as f:
         for r in csv.DictReader(f):
-            if "gemm_mfma_kernel" in r["Kernel_Name"]:
+            if "gemm_direct_kernel" in r["Kernel_Name"]:
                 rows.append((int(r["Dispatch_Id"]), float(r["Counter_Value"]), r["Kernel_Name"]))
     rows.sort()
     return rows
