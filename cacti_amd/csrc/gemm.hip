@@ -343,7 +343,7 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
         }
         return gemm_direct_launch(ta, tb, p, nblk, plan, st);
     }
-    // Operands that are not 16-byte aligned, with a workspace: laid out anew (one launch for both, 3-5 us for a few MB)
+    // Operands that are not 16-byte aligned, with a workspace: laid out anew (one launch for both, 2-4 us for a few MB)
     // for the direct kernels.  Element-wise loads in the kernel cost 1.6 us (both operands contiguous in K) to 3.4 us
     // (both strided) per 32 values of K instead, so only products with hardly any K stay on them.
     const int64_t ra = ta ? K : M, rb = tb ? N : K, pa = (ca + 7) / 8 * 8, pb = (cb + 7) / 8 * 8;

@@ -48,6 +48,8 @@ using namespace cacti;
 namespace {
 
 typedef int int4_t __attribute__((ext_vector_type(4)));
+// the same at any address of a half (global memory serves it in one instruction)
+typedef int int4_any __attribute__((ext_vector_type(4), aligned(2)));
 
 // The largest tile that parts of K are formed on (a product that needs a split has few tiles: small ones).
 constexpr int kMaxPartTile = 128 * 128;
@@ -58,6 +60,29 @@ constexpr int buffers(int bm, int bn, int res)
     const int room = 160 * 1024 / res / (BK * 2), least = bm < bn ? bm : bn;
     const int d = (room - least) / (bm + bn);
     return d > 4 ? 4 : d;
+}
+
+// 8 halves of a row of C that starts at any address and has `left` of them from here on
+__device__ __forceinline__ void store_odd(half_t *c, const int4_t &v, int64_t left)
+{
+    if (left >= 8) {
+        *reinterpret_cast<int4_any *>(c) = v;
+    } else {
+        const half_t *h = reinterpret_cast<const half_t *>(&v);
+#pragma unroll
+        for (int j = 0; j < 7; j++)
+            if (j < left) c[j] = h[j];
+    }
+}
+__device__ __forceinline__ void load_odd(half_t *lds, const half_t *c, int64_t left)
+{
+    if (left >= 8) {
+        *reinterpret_cast<int4_t *>(lds) = *reinterpret_cast<const int4_any *>(c);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 7; j++)
+            if (j < left) lds[j] = c[j];
+    }
 }
 
 // BM x BN x 64 per workgroup; wave (wm, wn) has the 16-row fragments f of op(A) at 32 f + 16 wm and of op(B) at 32 f + 16 wn.
@@ -334,10 +359,10 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     const bool inside = m0 + BM <= p.M && n0 + BN <= p.N;
     half_t *const Ct = C + m0 * p.ldc + n0;
     if (p.beta != 0.f && p.odd) {
-        for (int i = tid; i < BM * BN; i += NT) {
-            const int row = i / BN, col = i % BN;
-            if (m0 + row < p.M && n0 + col < p.N)
-                Cs[row * BN + ((((col >> 3) ^ (row & CSW)) << 3) | (col & 7))] = Ct[row * p.ldc + col];
+#pragma unroll 4
+        for (int i = 0; i < NC; i++) {
+            const int q = tid + i * NT, row = q / CPRC, cc = q % CPRC;
+            if (m0 + row < p.M) load_odd(Cs + row * BN + ((cc ^ (row & CSW)) << 3), Ct + row * p.ldc + cc * 8, p.N - n0 - cc * 8);
         }
         __syncthreads();
     } else if (p.beta != 0.f) {
@@ -393,15 +418,6 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
             }
     }
     __syncthreads();
-    if (p.odd) {
-        // consecutive lanes take consecutive elements of a row
-        for (int i = tid; i < BM * BN; i += NT) {
-            const int row = i / BN, col = i % BN;
-            if (m0 + row < p.M && n0 + col < p.N)
-                Ct[row * p.ldc + col] = Cs[row * BN + ((((col >> 3) ^ (row & CSW)) << 3) | (col & 7))];
-        }
-        return;
-    }
     // a round of the workgroup copies RSTEP rows of LPR chunks, NV rounds are under way together
     constexpr int LPR = NT % CPRC == 0 ? CPRC : 8, RSTEP = NT / LPR, NR = BM / RSTEP;
     constexpr int NV = NR % 8 == 0 ? 8 : NR % 6 == 0 ? 6 : NR;
@@ -409,7 +425,8 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     const int r0 = tid / LPR, cc = tid % LPR;
     const unsigned char *const co = smem_raw + r0 * (BN * 2);
     const int cx = (cc ^ (r0 & CSW)) << 4;
-    auto copy_out = [&](auto inside_c) __attribute__((always_inline)) {
+    // INSIDE: the tile lies wholly in C, 16-byte aligned; ODD: rows at any address, N of any length
+    auto copy_out = [&](auto inside_c, auto odd_c) __attribute__((always_inline)) {
         half_t *dst = Ct + r0 * p.ldc + cc * 8;
         const int64_t step = RSTEP * p.ldc;
 #pragma unroll 1
@@ -424,15 +441,19 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
                                                             (cx ^ ((((i0 + i) * RSTEP) & CSW) << 4)));
 #pragma unroll
                 for (int i = 0; i < NV; i++) {
-                    if (decltype(inside_c)::value || (m0 + r0 + (i0 + i) * RSTEP < p.M && n0 + (g * LPR + cc) * 8 < p.N))
+                    if (decltype(odd_c)::value) {
+                        if (m0 + r0 + (i0 + i) * RSTEP < p.M) store_odd(d, v[i], p.N - n0 - (g * LPR + cc) * 8);
+                    } else if (decltype(inside_c)::value || (m0 + r0 + (i0 + i) * RSTEP < p.M && n0 + (g * LPR + cc) * 8 < p.N)) {
                         *reinterpret_cast<int4_t *>(d) = v[i];
+                    }
                     d += step;
                 }
             }
         }
     };
-    if (inside) copy_out(std::true_type{});
-    else copy_out(std::false_type{});
+    if (p.odd) copy_out(std::false_type{}, std::true_type{});
+    else if (inside) copy_out(std::true_type{}, std::false_type{});
+    else copy_out(std::false_type{}, std::false_type{});
 }
 
 // C = f16(alpha sum of the parts + beta C), four columns per lane; the parts are added in order.  VEC: N and the rows
@@ -470,6 +491,8 @@ reduce_parts_kernel(int64_t M, int64_t N, int64_t ldp, int split, const float *_
 
 // Operands of any alignment as operands the direct kernels take: rows of `cols` halves, `ld` apart, to rows of `out_cols`
 // = cols rounded up to 8 (zeros behind cols), 16-byte aligned.  One lane per 16-byte piece, both operands in one launch.
+// (One load per piece at whatever address, and results that leave in the same way: 509 x 1003 x 770 in three layouts 39.8 ->
+// 32.2 us, 1999 x 3001 x 2003 152 -> 126 with the tiles of this file; half by half before.)
 struct RepackArgs {
     const half_t *src[2];
     half_t *dst[2];
@@ -483,10 +506,16 @@ __global__ void __launch_bounds__(256) repack_kernel(RepackArgs p)
     const int64_t row = i / per_row, c = (i - row * per_row) * 8;
     const half_t *src = p.src[z] + row * p.ld[z] + c;
     const int64_t left = p.cols[z] - c;
-    h8 v;
+    int4_t v = {0, 0, 0, 0};
+    if (left >= 8) {
+        v = *reinterpret_cast<const int4_any *>(src);
+    } else {
+        half_t h[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) v.v[j] = j < left ? src[j] : (half_t)0.f;
-    st8(p.dst[z] + i * 8, v);
+        for (int j = 0; j < 8; j++) h[j] = j < left ? src[j] : (half_t)0.f;
+        __builtin_memcpy(&v, h, 16);
+    }
+    *reinterpret_cast<int4_t *>(p.dst[z] + i * 8) = v;
 }
 
 template <bool TA, bool TB, int BM, int BN, int RES, bool M32 = false>
