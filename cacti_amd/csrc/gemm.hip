@@ -343,31 +343,42 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
         }
         return gemm_direct_launch(ta, tb, p, nblk, plan, st);
     }
-    // Operands that are not 16-byte aligned, with a workspace: laid out anew (one launch for both, 2-4 us for a few MB)
-    // for the direct kernels.  Element-wise loads in the kernel cost 1.6 us (both operands contiguous in K) to 3.4 us
-    // (both strided) per 32 values of K instead, so only products with hardly any K stay on them.
+    // Operands that are not 16-byte aligned, with a workspace: loaded as they are through registers on 64 x 64 tiles, or laid
+    // out anew for the direct kernels (one launch for both, some 3.5 us and 0.4 us per MB), whichever is expected to take
+    // less.  Over 85 products of M 9 .. 4000, N 50 .. 5000, K 66 .. 5000 in three layouts the copy takes 28 % longer in the mean than
+    // the better of the two, registers 3 %, this rule 0.2 % (19 % at worst: 687 x 3731 x 410).  Element-wise loads in the kernel cost 1.6 us (both operands contiguous in K) to
+    // 3.4 us (both strided) per 32 values of K instead, so only products with hardly any K stay on them.
     const int64_t ra = ta ? K : M, rb = tb ? N : K, pa = (ca + 7) / 8 * 8, pb = (cb + 7) / 8 * 8;
     if (ws_need && tri == 0 && nblk == 1 && K > 64 && pa < kMaxPitch && pb < kMaxPitch) {
         const bool ok_a = fits_a(8) && lda < kMaxPitch, ok_b = fits_b(8) && ldb < kMaxPitch;
-        const size_t bytes_a = ok_a ? 0 : (size_t)ra * (size_t)pa * 2, bytes_b = ok_b ? 0 : (size_t)rb * (size_t)pb * 2;
-        const GemmPlan plan = gemm_plan(M, N, K, 1, true);
+        size_t bytes_a = ok_a ? 0 : (size_t)ra * (size_t)pa * 2, bytes_b = ok_b ? 0 : (size_t)rb * (size_t)pb * 2;
+        GemmPlan plan = gemm_plan(M, N, K, 1, true);
+        if (near && ca >= 8 && cb >= 8) {
+            const GemmPlan as_is = gemm_plan_any(M, N, K);
+            const double copy = bytes_a + bytes_b > 0 ? 3.5 + (double)(bytes_a + bytes_b) / 2.5e6 : 0;
+            if (as_is.us < plan.us + copy) {
+                plan = as_is;
+                p.any = 1;
+                bytes_a = bytes_b = 0;
+            }
+        }
         p.ldp = (N + 3) / 4 * 4;
         const size_t bytes_part = plan.split > 1 ? (size_t)plan.split * (size_t)M * (size_t)p.ldp * sizeof(float) : 0;
         *ws_need = bytes_a + bytes_b + bytes_part;                // each a multiple of 16
         if (*ws_need > ws_bytes) return 0;
         char *w = static_cast<char *>(ws);
         const half_t *src[2] = {p.A, p.B};
-        half_t *dst[2] = {ok_a ? nullptr : (half_t *)w, ok_b ? nullptr : (half_t *)(w + bytes_a)};
+        half_t *dst[2] = {bytes_a ? (half_t *)w : nullptr, bytes_b ? (half_t *)(w + bytes_a) : nullptr};
         const int64_t rows[2] = {ra, rb}, cols[2] = {ca, cb}, ld[2] = {lda, ldb};
-        if (!ok_a || !ok_b) {
+        if (bytes_a + bytes_b > 0) {
             const int rc = gemm_repack(src, dst, rows, cols, ld, st);
             if (rc) return rc;
         }
-        if (!ok_a) {
+        if (bytes_a) {
             p.A = dst[0];
             p.lda = pa;
         }
-        if (!ok_b) {
+        if (bytes_b) {
             p.B = dst[1];
             p.ldb = pb;
         }

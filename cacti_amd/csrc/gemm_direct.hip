@@ -47,10 +47,6 @@ using namespace cacti;
 
 namespace {
 
-typedef int int4_t __attribute__((ext_vector_type(4)));
-// the same at any address of a half (global memory serves it in one instruction)
-typedef int int4_any __attribute__((ext_vector_type(4), aligned(2)));
-
 // The largest tile that parts of K are formed on (a product that needs a split has few tiles: small ones).
 constexpr int kMaxPartTile = 128 * 128;
 
@@ -87,16 +83,19 @@ __device__ __forceinline__ void load_odd(half_t *lds, const half_t *c, int64_t l
 
 // BM x BN x 64 per workgroup; wave (wm, wn) has the 16-row fragments f of op(A) at 32 f + 16 wm and of op(B) at 32 f + 16 wn.
 // M32 (64 x 64): v_mfma_f32_32x32x16_f16 on one 32 x 32 block per wave and k in ascending order, its tail last.
-template <bool TA, bool TB, int BM, int BN, int RES, bool M32>
+// ANY: operands of any alignment, through registers (LoadKCR, LoadKSR), two tile buffers of each; three tiles ahead in
+// registers, which is what a k tile of 64 x 64 (a quarter of a microsecond) needs to have its loads back in time.  509 x 1003 x
+// 770 in three layouts: 32.2 -> 26 us against a copy to aligned rows in front.
+template <bool TA, bool TB, int BM, int BN, int RES, bool M32, bool ANY>
 __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
 {
     // the whole argument block in scalar registers before anything else: read field by field where the control
     // flow first wants it, it costs five dependent round trips to memory before the first operand load
     asm volatile("" ::"s"(p.M), "s"(p.N), "s"(p.K), "s"(p.alpha), "s"(p.beta), "s"(p.A), "s"(p.lda), "s"(p.sa), "s"(p.B),
                  "s"(p.ldb), "s"(p.sb), "s"(p.C), "s"(p.ldc), "s"(p.sc), "s"(p.ztab), "s"(p.odd), "s"(p.part));
-    constexpr int NT = 256, D = buffers(BM, BN, RES);             // D: tiles between a load and its use
+    constexpr int NT = 256, D = ANY ? 2 : buffers(BM, BN, RES);   // D: tiles between a load and its use
     constexpr bool EARLY_A = BM <= BN;                            // the operand with the spare buffer
-    constexpr int NBA = D + EARLY_A, NBB = D + !EARLY_A;
+    constexpr int NBA = ANY ? 2 : D + EARLY_A, NBB = ANY ? 2 : D + !EARLY_A;
     static_assert(D >= 2 && BM % 32 == 0 && BN % 64 == 0 && (!M32 || (BM == 64 && BN == 64)), "tile shape");
     constexpr bool TR_A = TA, TR_B = !TB;                         // fragments by transposing reads
     constexpr int NA = BM / 32, NB = BN / 32;                     // fragments of a wave
@@ -126,15 +125,44 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
 
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wid & 1, wn = wid >> 1;
-    typename std::conditional<TA, LoadKSD<BM, NT>, LoadKCD<BM, NT>>::type la;
-    typename std::conditional<TB, LoadKCD<BN, NT>, LoadKSD<BN, NT>>::type lb;
+    typedef typename std::conditional<TA, LoadKSD<BM, NT>, LoadKCD<BM, NT>>::type LAD;
+    typedef typename std::conditional<TB, LoadKCD<BN, NT>, LoadKSD<BN, NT>>::type LBD;
+    typedef typename std::conditional<TA, LoadKSR<BM, NT>, LoadKCR<BM, NT>>::type LAR;
+    typedef typename std::conditional<TB, LoadKCR<BN, NT>, LoadKSR<BN, NT>>::type LBR;
+    typename std::conditional<ANY, LAR, LAD>::type la;
+    typename std::conditional<ANY, LBR, LBD>::type lb;
     constexpr int NLA = la.NL, NLB = lb.NL, NE = EARLY_A ? NLA : NLB, NL = EARLY_A ? NLB : NLA;
     // (the columns of a strided operand end on a multiple of 8: its width, or the padding behind it)
-    la.init(p.lda, (TA ? (p.M + 7) / 8 * 8 : p.M) - m0, p.K);
-    lb.init(p.ldb, (TB ? p.N : (p.N + 7) / 8 * 8) - n0, p.K);
+    la.init(p.lda, (TA && !ANY ? (p.M + 7) / 8 * 8 : p.M) - m0, p.K);
+    lb.init(p.ldb, (TB || ANY ? p.N : (p.N + 7) / 8 * 8) - n0, p.K);
     const int ktail = (int)(p.K % BK);
     auto lds_addr = [](const half_t *q) __attribute__((always_inline)) { return (uint32_t)(uintptr_t)q; };
-    {
+    // ANY: G sets of registers, one tile of both operands each; tile t in set (t - kt0) % G
+    constexpr int G = 3;
+    int4_t ra[ANY ? G : 1][ANY ? NLA : 1], rb[ANY ? G : 1][ANY ? NLB : 1];
+    if constexpr (ANY) {
+        const bool tail = ktail && kt0 == 0;
+        if (ktail) {
+            if (tail) {
+                la.load_tail(ra[0], la.kbase(Ao, p.K - ktail), ktail);
+                lb.load_tail(rb[0], lb.kbase(Bo, p.K - ktail), ktail);
+            }
+            Ao = la.kbase(Ao, -BK);
+            Bo = lb.kbase(Bo, -BK);
+        }
+        if (!tail) {
+            la.load(ra[0], la.kbase(Ao, (int64_t)kt0 * BK));
+            lb.load(rb[0], lb.kbase(Bo, (int64_t)kt0 * BK));
+        }
+#pragma unroll
+        for (int u = 1; u < G; u++) {
+            // (a tile that is none loads the last one again: a load inside a branch is waited for at its end)
+            const int64_t k0 = (int64_t)min(kt0 + u, nk - 1) * BK;
+            if (k0 == 0 && ktail) continue;
+            la.load(ra[u], la.kbase(Ao, k0));
+            lb.load(rb[u], lb.kbase(Bo, k0));
+        }
+    } else {
         // The first D tiles.  A tail of K goes first, so that every later load is of a whole tile: step t multiplies tile
         // t - 1 and step 0 the last, incomplete one.  (M32 loads it in its turn.)
         if (!M32 && ktail) {
@@ -269,16 +297,68 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     typedef std::integral_constant<int, 0> K0;
     typedef std::integral_constant<int, 1> K1;
 
+    constexpr int TA_BYTES = BM * BK * 2, TB_BYTES = BN * BK * 2, B0 = NBA * TA_BYTES;
+    int ta = 0, tb = B0;                                          // byte offsets in LDS of tile t
+    auto next_a = [&](int q) __attribute__((always_inline)) { return q == (NBA - 1) * TA_BYTES ? 0 : q + TA_BYTES; };
+    auto next_b = [&](int q) __attribute__((always_inline)) { return q == B0 + (NBB - 1) * TB_BYTES ? B0 : q + TB_BYTES; };
+    if constexpr (ANY) {
+        auto store = [&](int set, int ta, int tb) __attribute__((always_inline)) {
+#pragma unroll
+            for (int it = 0; it < NLA; it++) {
+                int4_t v = ra[set][it];
+                if constexpr (TA) v = la.in_place(v, it);
+                *reinterpret_cast<int4_t *>(smem_raw + ta + (threadIdx.x + it * NT) * 16) = v;
+            }
+#pragma unroll
+            for (int it = 0; it < NLB; it++) {
+                int4_t v = rb[set][it];
+                if constexpr (!TB) v = lb.in_place(v, it);
+                *reinterpret_cast<int4_t *>(smem_raw + tb + (threadIdx.x + it * NT) * 16) = v;
+            }
+        };
+        // tile t + 1 moves from its set to the buffers of tile t - 1, whose fragments every wave has held since the last
+        // barrier, and tile t + 1 + G is requested into the set
+        auto body = [&](int set, int t, bool more) __attribute__((always_inline)) {
+            const int na = next_a(ta), nb = next_b(tb);
+            store(set, na, nb);
+            if (more) {
+                const int64_t k0 = (int64_t)(t + 1 + G) * BK;
+                la.load(ra[set], la.kbase(Ao, k0));
+                lb.load(rb[set], lb.kbase(Bo, k0));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            step(K0{}, std::integral_constant<int, 0>{}, std::false_type{}, ta, tb, nullptr, 0);
+            __syncthreads();
+            step(K1{}, std::integral_constant<int, 0>{}, std::false_type{}, na, nb, nullptr, 0);
+            ta = na;
+            tb = nb;
+        };
+        store(0, ta, tb);
+        if (kt0 + G < nk) {
+            la.load(ra[0], la.kbase(Ao, (int64_t)(kt0 + G) * BK));
+            lb.load(rb[0], lb.kbase(Bo, (int64_t)(kt0 + G) * BK));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NU; u++) read_u(u, ta, tb, 0);
+        int t = kt0;
+        for (; t + 2 * G < nk; t += G)
+#pragma unroll
+            for (int u = 0; u < G; u++) body((u + 1) % G, t + u, true);
+        for (; t + 1 < nk; t += G)
+#pragma unroll
+            for (int u = 0; u < G; u++)
+                if (t + u + 1 < nk) body((u + 1) % G, t + u, t + u + 1 + G < nk);
+        step(K0{}, std::integral_constant<int, 0>{}, std::false_type{}, ta, tb, nullptr, 0);
+#pragma unroll
+        for (int m = 0; m < NM; m++) mfma(1, m);
+    } else {
     if (kt0 + D <= nk) wait_vmem<(D - 1) * (NLA + NLB)>();        // the first tile; the others stay in flight
     else wait_vmem<0>();
     __syncthreads();
-    constexpr int TA_BYTES = BM * BK * 2, TB_BYTES = BN * BK * 2, B0 = NBA * TA_BYTES;
-    int ta = 0, tb = B0;                                          // byte offsets in LDS of tile t
 #pragma unroll
     for (int u = 0; u < NU; u++) read_u(u, ta, tb, 0);
     const uint32_t wave16 = lds_addr(As) + wid * 1024;
-    auto next_a = [&](int q) __attribute__((always_inline)) { return q == (NBA - 1) * TA_BYTES ? 0 : q + TA_BYTES; };
-    auto next_b = [&](int q) __attribute__((always_inline)) { return q == B0 + (NBB - 1) * TB_BYTES ? B0 : q + TB_BYTES; };
     int t = kt0;
     const half_t *asrc = la.kbase(Ao, (int64_t)(kt0 + D) * BK), *bsrc = lb.kbase(Bo, (int64_t)(kt0 + D) * BK);
     const int64_t astep = TA ? BK * p.lda : BK, bstep = TB ? BK : BK * p.ldb;
@@ -319,6 +399,7 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     step(K0{}, std::integral_constant<int, 0>{}, std::false_type{}, ta, tb, nullptr, 0);
 #pragma unroll
     for (int m = 0; m < NM; m++) mfma(1, m);
+    }
     // the accumulators are read by vector instructions from here on, which do not wait for a product by themselves
     asm volatile("s_nop 15\n\ts_nop 15");
     if constexpr (M32) {
@@ -518,13 +599,12 @@ __global__ void __launch_bounds__(256) repack_kernel(RepackArgs p)
     *reinterpret_cast<int4_t *>(p.dst[z] + i * 8) = v;
 }
 
-template <bool TA, bool TB, int BM, int BN, int RES, bool M32 = false>
+template <bool TA, bool TB, int BM, int BN, int RES, bool M32 = false, bool ANY = false>
 int launch(GemmArgs p, int64_t nblk, hipStream_t st)
 {
     const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
-    constexpr int D = buffers(BM, BN, RES);
-    constexpr size_t smem = (size_t)(D * (BM + BN) + (BM < BN ? BM : BN)) * BK * sizeof(half_t);
-    auto kern = gemm_direct_kernel<TA, TB, BM, BN, RES, M32>;
+    constexpr size_t smem = (size_t)(ANY ? 2 * (BM + BN) : buffers(BM, BN, RES) * (BM + BN) + (BM < BN ? BM : BN)) * BK * sizeof(half_t);
+    auto kern = gemm_direct_kernel<TA, TB, BM, BN, RES, M32, ANY>;
     static DeviceOnce attr_set;                   // one per instantiation
     if (!attr_set.fresh()) {
         CACTI_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
@@ -574,6 +654,7 @@ template <bool TA, bool TB, int... I>
 int launch_shape(int shape, const GemmArgs &p, int64_t nblk, hipStream_t st, std::integer_sequence<int, I...>)
 {
     if (shape == T64_SMALL) return launch<TA, TB, 64, 64, 2, true>(p, nblk, st);
+    if (p.any) return launch<TA, TB, 64, 64, 2, false, true>(p, nblk, st);
     int rc = CACTI_E_STATE;
     (void)((shape == I && (rc = launch<TA, TB, kShapes[I].bm, kShapes[I].bn, kShapes[I].res>(p, nblk, st), true)) || ...);
     return rc;
@@ -599,6 +680,23 @@ double tile_cost(int64_t cus, int tile, int64_t M, int64_t N, int64_t nz, int64_
 }
 
 constexpr int64_t kSmallOutput = 1 << 18;
+constexpr double kAnyPerTile = 1.45;
+
+// `best` in up to 8 parts of K on tile t, if that costs less; per_tile: factor on the time per k tile
+void split_k(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, double per_tile, GemmPlan &best, double &best_cost)
+{
+    for (int s = 2; s <= 8; s++) {
+        const int64_t per = (kt + s - 1) / s;
+        if (per < 4 || (kt + per - 1) / per != s) continue;               // parts of some length, none empty
+        const double fixed = kShapes[t].fixed;
+        const double c = fixed + per_tile * (tile_cost(cus, t, M, N, s, per) - fixed) + 4.0 + (double)(M * N) * s * 8.0 / 4e6;
+        if (c < best_cost) {
+            best_cost = c;
+            const double us = c;
+            best = {t, T64, 0, s, us};
+        }
+    }
+}
 
 // How a product is cut.  One workgroup takes one tile; a launch runs in sets of resident workgroups, and a nearly empty
 // last set costs as much as a full one.  Considered: every tile shape by itself; for those of one workgroup per CU also the
@@ -616,13 +714,13 @@ GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, boo
     // launches.
     const int64_t tiles64 = (M + 63) / 64 * ((N + 63) / 64);
     const bool small = M * N <= kSmallOutput && (nz <= kMaxPtrBatch || tiles64 * nz <= kShapes[T64].res * cus);
-    GemmPlan best = {small ? T64_SMALL : T64, T64, 0, 1};
     double best_cost = tile_cost(cus, T64, M, N, nz, kt);
+    GemmPlan best = {small ? T64_SMALL : T64, T64, 0, 1, 0};
     for (int t = T64 + 1; t < kNumShapes && !small; t++) {
         const double c = tile_cost(cus, t, M, N, nz, kt);
         if (c < best_cost) {
             best_cost = c;
-            best = {t, T64, 0, 1};
+            best = {t, T64, 0, 1, 0};
         }
     }
     for (int t = T64 + 1; t < kNumShapes && !small; t++) {
@@ -635,21 +733,14 @@ GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, boo
             const double c = first + tile_cost(cus, r, M, N - cols, nz, kt);
             if (c < best_cost) {
                 best_cost = c;
-                best = {t, r, cols, 1};
+                best = {t, r, cols, 1, 0};
             }
         }
     }
     if (may_split && nz == 1)
         for (int t = T64; t < kNumShapes; t++)
-            for (int s = 2; s <= 8 && kShapes[t].bm * kShapes[t].bn <= kMaxPartTile; s++) {
-                const int64_t per = (kt + s - 1) / s;
-                if (per < 4 || (kt + per - 1) / per != s) continue;           // parts of some length, none empty
-                const double c = tile_cost(cus, t, M, N, s, per) + 4.0 + (double)(M * N) * s * 8.0 / 4e6;
-                if (c < best_cost) {
-                    best_cost = c;
-                    best = {t, T64, 0, s};
-                }
-            }
+            if (kShapes[t].bm * kShapes[t].bn <= kMaxPartTile) split_k(cus, t, M, N, kt, 1.0, best, best_cost);
+    best.us = best_cost;
     return best;
 }
 
@@ -700,6 +791,19 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split)
     if (k.how != how || k.M != M || k.N != N || k.K != K || k.nz != nz)
         k = {M, N, K, nz, how, make_plan(cus, M, N, K, nz, may_split)};
     return k.plan;
+}
+
+// The same for operands that are loaded through registers whatever their alignment: 64 x 64 tiles, whose k tiles take some
+// half longer than the direct ones' (64 x 128 and 128 x 128 took twice and three times as long as that: their loads have
+// no room in the registers to be far enough ahead).
+GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K)
+{
+    const int64_t kt = (K + BK - 1) / BK, cus = device_cus();
+    const double fixed = kShapes[T64].fixed;
+    GemmPlan best = {T64, T64, 0, 1, 0};
+    best.us = fixed + kAnyPerTile * (tile_cost(cus, T64, M, N, 1, kt) - fixed);
+    split_k(cus, T64, M, N, kt, kAnyPerTile, best, best.us);
+    return best;
 }
 
 int gemm_direct_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, const GemmPlan &plan, hipStream_t st)

@@ -99,7 +99,8 @@ struct GemmArgs {
     int split_tiles;
     float *part;
     int64_t ldp;
-    int odd;              // C of any alignment and N: element by element
+    int odd;              // C of any alignment and N
+    int any;              // A and B of any alignment (strided operands with rows of 8 elements and more)
 };
 constexpr int kMaxPtrBatch = 4;
 constexpr int kTriPad = 256;
@@ -109,9 +110,11 @@ struct GemmPlan {
     int tile, rest;      // shape of the (first) launch; of the second
     int64_t cols;        // > 0: columns of the first launch, the rest go to a second
     int split;           // parts of K
+    double us;           // what it is expected to take
 };
 // nz: products of this shape in the launch
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split);
+GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K);        // for GemmArgs::any (with parts of K)
 void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn);
 
 // Products of operands whose rows are at least 8-byte aligned (align = 4; 8: 16-byte aligned), with a triangular operand or

@@ -159,6 +159,94 @@ struct LoadKSD {
     static constexpr int NDMA = NL;
 };
 
+typedef int int4_t __attribute__((ext_vector_type(4)));
+// the same at any address of a half (global memory serves it in one instruction)
+typedef int int4_any __attribute__((ext_vector_type(4), aligned(2)));
+
+// the 8 halves of v moved down by s places (s >= 0), zeros behind them
+__device__ __forceinline__ int4_t halves_down(const int4_t &v, int s)
+{
+    typedef unsigned long long u64;
+    const u64 lo = (u64)(uint32_t)v.y << 32 | (uint32_t)v.x, hi = (u64)(uint32_t)v.w << 32 | (uint32_t)v.z;
+    const int b = (s & 3) * 16;
+    const u64 l = lo >> b | (hi << 1) << (63 - b), h = hi >> b;
+    const u64 x = s >= 8 ? 0 : s >= 4 ? h : l, y = s >= 4 ? 0 : h;
+    return int4_t{(int)(uint32_t)x, (int)(x >> 32), (int)(uint32_t)y, (int)(y >> 32)};
+}
+
+// ---- operands of any alignment, through registers into the same layouts: lane l of the workgroup's load `it` holds what the
+// direct loads bring to LDS byte 16 (l + it NT) of the tile.  What would reach beyond a row's end is read from 8 halves
+// before it and moved down (rows of at least 8 halves), so that nothing outside the operand is touched.
+template <int ROWS, int NT>
+struct LoadKCR {
+    static constexpr int NL = ROWS * 8 / NT;
+    uint32_t off[NL];
+    __device__ __forceinline__ void init(int64_t ld, int64_t rows_left, int64_t)
+    {
+        const uint32_t ld2 = (uint32_t)ld * 2;
+        const int last = (int)(rows_left < ROWS ? rows_left : ROWS) - 1;
+#pragma unroll
+        for (int it = 0; it < NL; it++) {
+            const int c = threadIdx.x + it * NT, r = c >> 3;
+            off[it] = (uint32_t)min(r, last) * ld2 + ((c & 7) ^ swz16(r)) * 16;
+        }
+    }
+    __device__ __forceinline__ void load(int4_t *v, const half_t *base) const
+    {
+#pragma unroll
+        for (int it = 0; it < NL; it++) v[it] = *reinterpret_cast<const int4_any *>(at(base, off[it]));
+    }
+    // the k tile with only `left` < BK values of k, which end the row
+    __device__ __forceinline__ void load_tail(int4_t *v, const half_t *base, int left) const
+    {
+#pragma unroll
+        for (int it = 0; it < NL; it++) {
+            const int c = threadIdx.x + it * NT, q = ((c & 7) ^ swz16(c >> 3)) * 8, s = max(q + 8 - left, 0);
+            v[it] = halves_down(*reinterpret_cast<const int4_any *>(at(base, off[it]) - s), s);
+        }
+    }
+    __device__ __forceinline__ const half_t *kbase(const half_t *origin, int64_t k0) const { return origin + k0; }
+};
+template <int ROWS, int NT>
+struct LoadKSR {
+    static constexpr int CPR = ROWS / 8, SWK = CPR % 8 == 0 ? 3 : 1, NL = BK * CPR / NT;
+    uint32_t off[NL];
+    int64_t ld;
+    int down[NL];
+    bool edge;
+    __device__ __forceinline__ void init(int64_t ld_, int64_t rows_left, int64_t)
+    {
+        ld = ld_;
+        edge = rows_left < ROWS;
+        const uint32_t ld2 = (uint32_t)ld_ * 2;
+        const int left = (int)(rows_left < ROWS ? rows_left : ROWS);
+#pragma unroll
+        for (int it = 0; it < NL; it++) {
+            const int c = threadIdx.x + it * NT, k = c / CPR, q = ((c % CPR) ^ (2 * (k & SWK))) * 8;
+            down[it] = max(q + 8 - left, 0);
+            off[it] = k * ld2 + (q - down[it]) * 2;               // (may lie before the tile's first column: inside the row)
+        }
+    }
+    __device__ __forceinline__ int4_t in_place(const int4_t &v, int it) const { return edge ? halves_down(v, down[it]) : v; }
+    __device__ __forceinline__ void load(int4_t *v, const half_t *base) const
+    {
+#pragma unroll
+        for (int it = 0; it < NL; it++)
+            v[it] = *reinterpret_cast<const int4_any *>(reinterpret_cast<const char *>(base) + (int32_t)off[it]);
+    }
+    __device__ __forceinline__ void load_tail(int4_t *v, const half_t *base, int left) const
+    {
+#pragma unroll
+        for (int it = 0; it < NL; it++) {
+            const int k = (threadIdx.x + it * NT) / CPR;
+            const int64_t back = (int64_t)max(k - left + 1, 0) * ld;
+            v[it] = *reinterpret_cast<const int4_any *>(reinterpret_cast<const char *>(base - back) + (int32_t)off[it]);
+            if (back) v[it] = int4_t{0, 0, 0, 0};
+        }
+    }
+    __device__ __forceinline__ const half_t *kbase(const half_t *origin, int64_t k0) const { return origin + k0 * ld; }
+};
+
 // wait until at most n vector memory loads are outstanding (s_waitcnt vmcnt only)
 template <int N>
 __device__ __forceinline__ void wait_vmem()

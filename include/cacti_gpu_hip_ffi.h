@@ -111,8 +111,8 @@ int cacti_hip_gemm_f16(int ta, int tb, int64_t M, int64_t N, int64_t K, float al
 /* The same for callers that can lend device memory for the duration of the product (in stream order).  *ws_need is
  * set to the bytes the chosen way of computing it takes; if that is more than ws_bytes nothing is launched and the
  * call is to be repeated with that much (ws 16-byte aligned; null with ws_bytes = 0 to ask).  With a workspace, operands
- * of any alignment take the direct kernels through an aligned copy, and products with few output tiles and a long K
- * are summed in parts of K. */
+ * of any alignment take the tile kernels, as they are or through an aligned copy, and products with few output tiles and a
+ * long K are summed in parts of K. */
 int cacti_hip_gemm_f16_ws(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const void *A, int64_t lda,
                           const void *B, int64_t ldb, float beta, void *C, int64_t ldc, void *ws, size_t ws_bytes,
                           size_t *ws_need, void *stream);

@@ -113,6 +113,22 @@ def test_products_of_any_alignment(M, N, K, ta, tb):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 65), (9, 15, 127), (63, 65, 128), (71, 130, 129), (64, 9, 193), (200, 77, 257), (66, 74, 1999),
+                                   (5, 3, 200), (7, 300, 77)])
+def test_operands_that_start_at_any_half(M, N, K, ta, tb):
+    """Edges of tiles and of K with operands between 16-byte boundaries, up to the last half of their memory; strided ones of
+    fewer than 8 columns too."""
+    A, B, a, b = operands(M, N, K, ta, tb)
+    for shift in (1, 3):
+        place = lambda t: torch.cat([t.new_full((shift,), float("nan")), t.reshape(-1)])[shift:].view(t.shape)
+        got = ops.gemm(place(a), place(b), ta=ta, tb=tb)
+        check(A, B, False, True, got)
+        old = torch.randn(M, N, device="cuda", dtype=torch.float16)
+        check(A, B, False, True, ops.gemm(place(a), place(b), ta=ta, tb=tb, beta=1.0, out=place(old)), old)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(37, 3200, 8640), (5, 2048, 5504), (100, 1000, 9001), (33, 4104, 6000)])
 def test_parts_of_k(M, N, K):
     A, B, _, _ = operands(M, N, K, False, True)
