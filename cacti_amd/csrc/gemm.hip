@@ -308,7 +308,9 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
         }
     hipStream_t st = (hipStream_t)stream;
     const bool near = lda < kMaxPitch && ldb < kMaxPitch;
-    if (vec >= 4 && !ta && tb && K <= 128 && beta == 0.f && tri <= 1)
+    // Scores: a batch of heads, or the lower triangle of one.  (A single product with a short K is no score: 149 x 8280 x 96
+    // takes 43 us there, whose workgroups walk tile rows of a square, and 4.3 on the tiles below; 2048 x 2048 x 128 17 and 5.9.)
+    if (vec >= 4 && !ta && tb && K <= 128 && beta == 0.f && tri <= 1 && (nblk > 1 || tri == 1 || (vec < 8 && !ws_need)))
         return gemm_nt_smallk_launch(p, nblk, st);
     // one to four rows against a weight matrix (decoding): a stream over B
     if (vec == 8 && !ta && tb && M <= 4 && nblk == 1 && beta == 0.f && tri == 0)
@@ -347,9 +349,9 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
     // out anew for the direct kernels (one launch for both, some 3.5 us and 0.4 us per MB), whichever is expected to take
     // less.  Over 85 products of M 9 .. 4000, N 50 .. 5000, K 66 .. 5000 in three layouts the copy takes 28 % longer in the mean than
     // the better of the two, registers 3 %, this rule 0.2 % (19 % at worst: 687 x 3731 x 410).  Element-wise loads in the kernel cost 1.6 us (both operands contiguous in K) to
-    // 3.4 us (both strided) per 32 values of K instead, so only products with hardly any K stay on them.
+    // 3.4 us (both strided) per 32 values of K instead.
     const int64_t ra = ta ? K : M, rb = tb ? N : K, pa = (ca + 7) / 8 * 8, pb = (cb + 7) / 8 * 8;
-    if (ws_need && tri == 0 && nblk == 1 && K > 64 && pa < kMaxPitch && pb < kMaxPitch) {
+    if (ws_need && tri == 0 && nblk == 1 && K >= 8 && pa < kMaxPitch && pb < kMaxPitch) {
         const bool ok_a = fits_a(8) && lda < kMaxPitch, ok_b = fits_b(8) && ldb < kMaxPitch;
         size_t bytes_a = ok_a ? 0 : (size_t)ra * (size_t)pa * 2, bytes_b = ok_b ? 0 : (size_t)rb * (size_t)pb * 2;
         GemmPlan plan = gemm_plan(M, N, K, 1, true);

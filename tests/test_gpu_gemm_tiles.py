@@ -66,12 +66,9 @@ def test_direct_tiles_at_their_edges(tile):
         old = torch.randn(M, N, device="cuda", dtype=torch.float16)
         acc = ops.gemm(A, Bt, beta=1.0, out=old.clone())
         check(A, B, False, True, acc, old)
-        # the sums are formed in one order whatever the layout: the same bits (a transposed A has rows of 8 elements and more;
-        # A B^T of K <= 128 is another kernel's)
+        # the sums are formed in one order whatever the layout: the same bits (a transposed A has rows of 8 elements and more)
         M8 = M // 8 * 8
         for ta, tb in ((False, True), (True, False), (True, True)):
-            if tb and not ta and K <= 128:
-                continue
             a, b = (A[:M8].T.contiguous() if ta else A), (B if tb else Bt)
             m = M8 if ta else M
             if plan(m, N, K) == plan(M, N, K):
@@ -115,7 +112,7 @@ def test_products_of_any_alignment(M, N, K, ta, tb):
 @pytest.mark.gpu
 @pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
 @pytest.mark.parametrize("M,N,K", [(8, 8, 65), (9, 15, 127), (63, 65, 128), (71, 130, 129), (64, 9, 193), (200, 77, 257), (66, 74, 1999),
-                                   (5, 3, 200), (7, 300, 77)])
+                                   (5, 3, 200), (7, 300, 77), (9, 11, 8), (33, 70, 13), (130, 9, 63)])
 def test_operands_that_start_at_any_half(M, N, K, ta, tb):
     """Edges of tiles and of K with operands between 16-byte boundaries, up to the last half of their memory; strided ones of
     fewer than 8 columns too."""
