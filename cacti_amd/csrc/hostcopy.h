@@ -33,7 +33,7 @@ int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st);
 // one region of any size to pageable memory, likewise, and (not null) a word of device memory with it; readers on other
 // threads and streams go on meanwhile
 int read_large(void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st);
-constexpr size_t kLargeRead = 512u << 10;      // from here on it is the better one
+constexpr size_t kLargeRead = 192u << 10;      // from here on it is the better one
 // n regions of `bytes` (a multiple of 16), 16-byte aligned, set to zero
 int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st);
 

@@ -33,17 +33,33 @@ struct GatherArgs {
     unsigned epoch;
 };
 
+// Sixteen bytes to host memory at system scope: through both caches, like a relaxed atomic of that scope (which the language
+// has for eight bytes at most).  So there is nothing in the caches for a system fence to write back before the word that
+// announces the chunk, only stores to wait for; the fence, once per wave, was a third of the read (64 KiB 12.0 -> 9.0 us,
+// 344 KiB 24.7 -> 18.2 from launch to copied, 64 bytes 6.9 -> 5.8).
+__device__ __forceinline__ void store_host(uint4 *dst, const uint4 &v)
+{
+    typedef unsigned uint4_v __attribute__((ext_vector_type(4)));
+    const uint4_v w = {v.x, v.y, v.z, v.w};
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(dst), "v"(w) : "memory");
+}
+__device__ __forceinline__ void store_host(int *dst, int v)
+{
+    __hip_atomic_store(dst, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// every wave's stores have been acknowledged, then the word
 __device__ __forceinline__ void chunk_arrived(unsigned *flag, unsigned epoch)
 {
-    __threadfence_system();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(flag, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (threadIdx.x == 0) __hip_atomic_store(flag, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ void __launch_bounds__(256) gather_kernel(GatherArgs p)
 {
     const int z = blockIdx.y;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < p.n16[z]; i += (int64_t)gridDim.x * 256) p.dst[z][i] = p.src[z][i];
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < p.n16[z]; i += (int64_t)gridDim.x * 256) store_host(p.dst[z] + i, p.src[z][i]);
     chunk_arrived(p.flags + z * gridDim.x + blockIdx.x, p.epoch);
 }
 
@@ -54,9 +70,9 @@ stream_kernel(const uint4 *src, uint4 *dst, int64_t n16, int64_t chunk16, const 
 {
     const int64_t chunks = (n16 + chunk16 - 1) / chunk16;
     for (int64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
-        if (word && c == 0 && threadIdx.x == 0) *word_dst = *word;
+        if (word && c == 0 && threadIdx.x == 0) store_host(word_dst, *word);
         const int64_t end = min((c + 1) * chunk16, n16);
-        for (int64_t i = c * chunk16 + threadIdx.x; i < end; i += 256) dst[i] = src[i];
+        for (int64_t i = c * chunk16 + threadIdx.x; i < end; i += 256) store_host(dst + i, src[i]);
         chunk_arrived(flags + c, epoch);
     }
 }
@@ -212,7 +228,8 @@ static int read_windows(Staging &s, void *dst, const void *src, size_t bytes, co
 
 // Measured, us, one gather and one copy behind it / 1 MiB pieces before -> chunks: 2 MiB 119 -> 76, 20 MiB 569 -> 473.  A
 // helper thread costs some 10 us to start: worth it from several MiB on, where the copying host (12 .. 30 GB/s) and not
-// the link (52) is what one thread would wait for.  Below 512 KiB chunks bring nothing (32 us at 512 KiB either way).
+// the link (52) is what one thread would wait for.  One gather and one copy behind it against chunks, since the chunks are
+// announced without a fence: 128 KiB 15.3 and 15.7, 344 KiB 24.4 and 22.3, 512 KiB 30.2 and 29.6.
 int read_large(void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st)
 {
     Staging s;
