@@ -5,7 +5,7 @@
 // accumulate in fp32 and round once).
 //
 // A single query row per head is a few hundred KB of cache and hardly any arithmetic: what it costs is launches and
-// round trips to memory.  A workgroup takes a head and a piece of its dimension (up to 32 columns), over all positions:
+// round trips to memory.  A workgroup takes a head and a piece of its dimension (8 to 32 columns), over all positions:
 // the probabilities of a row need the sum over the whole row before the first product with V is formed, and a split
 // over positions would need that sum, and then the partial outputs, exchanged between workgroups (another launch each;
 // a device-wide fence inside the launch costs 40 us on this chip).  Every piece's workgroup forms the head's scores
@@ -13,10 +13,16 @@
 // time, the scores come from a launch of their own, one workgroup per head and 128 positions.  One launch instead of
 // three (scores, values per 128 positions, sum): 69 positions, 32 heads of 100: 12.9 -> 5 us.
 //
-// Eight lanes share a position, each with 8-byte pieces of the head (a head starts on a multiple of 8 bytes), 64
-// contiguous bytes per access; four positions per lane are in flight together, and the first four V pieces are
-// requested before anything else.  Loads are unconditional with clamped indices: a load inside a branch is waited for
-// at the end of the branch.
+// In the scores eight lanes share a position, each with 8-byte pieces of the head (a head starts on a multiple of 8
+// bytes), 64 contiguous bytes per access; in the product with V it is LP lanes with a piece each: fewer columns per
+// workgroup are more workgroups, each with fewer steps over the positions behind one another.  (The head is the fast
+// index of the grid: where their number is a multiple of 8, all workgroups of a head are on one XCD and share a row's
+// bytes in its L2.)  Four positions per lane are in flight together; the first V pieces are requested once the scores'
+// own loads are, which would otherwise be returned behind them, and arrive during the softmax.  Loads are unconditional
+// with clamped indices: a load inside a branch is waited for at the end of the branch.
+// Eight lanes throughout and V first -> now, us: one row, 16 heads of 128, 200 / 480 / 1540 / 4000 positions 5.7 / 6.8 /
+// 10.7 / 18.5 -> 5.0 / 6.1 / 8.9 / 15.4; 32 heads of 100 6.5 / 9.3 / 16.2 / 31.6 -> 5.6 / 7.2 / 12.5 / 23.0; four rows of
+// 16 x 128 10.9 / 13.3 / 20.1 / 35.7 -> 10.4 / 12.6 / 16.9 / 26.7.
 #include "common.h"
 #include "softmax_math.h"
 
@@ -28,11 +34,15 @@ constexpr int kThreads = 256;              // of the scores launch; the values l
 constexpr int kWide = 512;
 constexpr int kStep = 4;                   // positions of a lane in flight
 constexpr int kSlice = kThreads / 8 * kStep;   // positions per workgroup of the scores launch
-// Measured, us at 70 / 300 / 600 / 1000 / 1540 positions, 16 heads of 128: own scores on 256 lanes 4.6 / 6.8 / 10.0 / 13.7 /
-// 19.6, on 512 lanes 5.4 / 7.1 / 8.7 / 10.5 / 14.3, on 1024 7.2 / 7.4 / 10.2 / 11.1 / 16.0; scores apart and 512 lanes 7.2 / 7.8 / 8.4
-// / 9.7 / 11.2.  32 heads of 100 cross at the same places.
-constexpr int kNarrow = 320;               // up to here kThreads lanes, own scores
-constexpr int kOwnScores = 512;            // up to here kWide lanes, own scores; beyond, a scores launch
+// Up to here kThreads lanes, eight to a position, own scores: one step over the positions, which more lanes cannot make
+// shorter (70 positions, 32 heads of 100: 4.6 against 4.9 us; 300 positions 6.8 against 6.5).
+constexpr int kNarrow = 128;
+// Up to here kWide lanes, four to a position, own scores; beyond, a scores launch: 16 heads of 128, 400 / 520 / 800
+// positions 6.1 / 7.5 / 8.6 against 6.8 / 7.0 / 7.3 us, 32 heads of 100 6.8 / 8.2 / 9.7 against 6.9 / 7.8 / 8.6.
+constexpr int kOwnScores = 480;
+// The same for one or two rows of heads to 64, which have half of the keys' bytes to read: 32 heads of 64, 800 / 1200
+// positions 6.9 / 8.3 against 7.7 / 8.1 us; four rows of 16 such heads at 520 13.0 against 12.9.
+constexpr int kOwnScoresShort = 960;
 constexpr int kMaxCols = 8192;             // score rows live in LDS
 
 struct __attribute__((aligned(8))) h4 {
@@ -102,8 +112,8 @@ decode_scores_kernel(int C, int Dh, float alpha, const half_t *__restrict__ q, i
     scores_step<T, NP, kThreads>(qv, kc + h * hsk, ldk, Dh / 4, alpha, j0, min(C, j0 + kSlice), s16 + (int64_t)h * T * ld, ld, 0);
 }
 
-// OWN: the scores are formed here; otherwise they are s16[h][t][ld].
-template <int T, int NP, bool OWN, int NT>
+// OWN: the scores are formed here; otherwise they are s16[h][t][ld].  LP: lanes per position in the product with V.
+template <int T, int NP, bool OWN, int NT, int LP>
 __global__ void __launch_bounds__(NT)
 decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__restrict__ q, int64_t ldq, const half_t *__restrict__ kc,
                      const half_t *__restrict__ vc, int64_t ldkv, int64_t hs, const half_t *__restrict__ s16, int64_t ld,
@@ -111,12 +121,12 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
 {
     extern __shared__ __attribute__((aligned(16))) half_t sp[];           // [T][ld]: scores, then probabilities
     __shared__ float scratch[2][T][NT / 64];
-    __shared__ float red[NT / 64][T][8][4];
-    constexpr int kGroups = NT / 8;            // positions per step and lane
-    const int tid = threadIdx.x, i8 = tid & 7, g = tid >> 3, lane = tid & 63, wid = tid >> 6, h = blockIdx.y;
-    const int pieces = Dh / 4, per = (pieces + gridDim.x - 1) / gridDim.x;        // pieces of this workgroup: at most 8
-    const int piece = blockIdx.x * per + i8;
-    const bool mine = i8 < per && piece < pieces;
+    __shared__ float red[NT / 64][T][LP][4];
+    constexpr int kGroups = NT / LP;           // positions per step and lane
+    const int tid = threadIdx.x, ip = tid & (LP - 1), g = tid / LP, lane = tid & 63, wid = tid >> 6, h = blockIdx.x;
+    const int pieces = Dh / 4, per = (pieces + gridDim.y - 1) / gridDim.y;        // pieces of this workgroup: at most LP
+    const int piece = blockIdx.y * per + ip;
+    const bool mine = ip < per && piece < pieces;
     const half_t *vp = vc + h * hs + 4 * (mine ? piece : 0);
     auto load_v = [&](h4 (&v)[kStep], int j0) __attribute__((always_inline)) {
 #pragma unroll
@@ -124,14 +134,15 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
             v[it] = *reinterpret_cast<const h4 *>(vp + (int64_t)min(j0 + g + it * kGroups, C - 1) * ldkv);
     };
     h4 vv[kStep];
-    load_v(vv, 0);
     if (OWN) {
         h4 qv[T][NP];
-        load_q<T, NP>(qv, q, ldq, h, Dh, i8);
-        for (int j0 = 0; j0 < C; j0 += kGroups * kStep) scores_step<T, NP, NT>(qv, kc + h * hs, ldkv, pieces, alpha, j0, C, sp, ld, 0);
+        load_q<T, NP>(qv, q, ldq, h, Dh, tid & 7);
+        for (int j0 = 0; j0 < C; j0 += NT / 8 * kStep) scores_step<T, NP, NT>(qv, kc + h * hs, ldkv, pieces, alpha, j0, C, sp, ld, 0);
     } else {
         for (int i = tid; i < T * (int)ld / 8; i += NT) st8(sp + i * 8, ld8(s16 + (int64_t)h * T * ld + i * 8));
     }
+    // (not before the scores' own loads, which would be returned behind them; the softmax covers these)
+    load_v(vv, 0);
     __syncthreads();
     // row maxima, then sums of exponentials, then the probabilities in place of the scores; row t sees live(t) positions
     auto live = [&](int t) __attribute__((always_inline)) { return (int)min((int64_t)C, (int64_t)t + row0 + 1); };
@@ -193,19 +204,21 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             float a = acc[t][i];
+            if (LP <= 2) a += __shfl_xor(a, 2, 64);
+            if (LP <= 4) a += __shfl_xor(a, 4, 64);
             a += __shfl_xor(a, 8, 64);
             a += swz_xor16(a);
             a += xor32(a);
-            if (lane < 8) red[wid][t][lane][i] = a;
+            if (lane < LP) red[wid][t][lane][i] = a;
         }
     __syncthreads();
-    if (tid < T * 32) {
-        const int t = tid >> 5, c = (tid >> 2) & 7, i = tid & 3;
-        if (c < per && blockIdx.x * per + c < pieces) {
+    if (tid < T * LP * 4) {
+        const int t = tid / (LP * 4), c = (tid >> 2) & (LP - 1), i = tid & 3;
+        if (c < per && blockIdx.y * per + c < pieces) {
             float a = red[0][t][c][i];
 #pragma unroll
             for (int w = 1; w < NT / 64; w++) a += red[w][t][c][i];
-            out[t * ldo + h * Dh + 4 * (blockIdx.x * per + c) + i] = f2h(a);
+            out[t * ldo + h * Dh + 4 * (blockIdx.y * per + c) + i] = f2h(a);
         }
     }
 }
@@ -224,11 +237,11 @@ struct DecodeArgs {
     hipStream_t st;
 };
 
-template <int T, int NP, bool OWN, int NT>
+template <int T, int NP, bool OWN, int NT, int LP>
 int launch_values(const DecodeArgs &a, int64_t ld)
 {
     const size_t smem = (size_t)T * (size_t)ld * sizeof(half_t);
-    auto kern = decode_values_kernel<T, NP, OWN, NT>;
+    auto kern = decode_values_kernel<T, NP, OWN, NT, LP>;
     if (smem > 32 * 1024) {
         static DeviceOnce attr_set;
         if (!attr_set.fresh()) {
@@ -236,7 +249,7 @@ int launch_values(const DecodeArgs &a, int64_t ld)
             attr_set.mark();
         }
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)((a.Dh / 4 + 7) / 8), (unsigned)a.H), dim3(NT), smem, a.st, a.C, a.Dh, a.row0, a.alpha, a.q,
+    hipLaunchKernelGGL(kern, dim3((unsigned)a.H, (unsigned)((a.Dh / 4 + LP - 1) / LP)), dim3(NT), smem, a.st, a.C, a.Dh, a.row0, a.alpha, a.q,
                        a.ldq, a.kc, a.vc, a.ldkv, a.hs, (const half_t *)a.s16, ld, a.out, a.ldo);
     return launch_status("attn_decode");
 }
@@ -245,11 +258,14 @@ template <int T, int NP>
 int launch(const DecodeArgs &a)
 {
     const int64_t ld = (a.C + 7) / 8 * 8;
-    if (a.C <= kNarrow) return launch_values<T, NP, true, kThreads>(a, ld);
-    if (a.C <= kOwnScores) return launch_values<T, NP, true, kWide>(a, ld);
+    if (a.C <= kNarrow) return launch_values<T, NP, true, kThreads, 8>(a, ld);
+    if (a.C <= (NP == 2 && T <= 2 ? kOwnScoresShort : kOwnScores)) return launch_values<T, NP, true, kWide, 4>(a, ld);
     hipLaunchKernelGGL((decode_scores_kernel<T, NP>), dim3((unsigned)((a.C + kSlice - 1) / kSlice), (unsigned)a.H), dim3(kThreads), 0, a.st,
                        a.C, a.Dh, a.alpha, a.q, a.ldq, a.kc, a.ldkv, a.hs, a.s16, ld);
-    return launch_values<T, NP, false, kWide>(a, ld);
+    // two lanes to a position while every workgroup of theirs has a CU (1540 positions, 16 heads of 128, two / four: 8.8 /
+    // 9.3 us, 32 of 64 8.9 / 9.6; 32 of 100, 416 workgroups, 14.0 / 12.2)
+    if ((int64_t)a.H * ((a.Dh / 4 + 1) / 2) <= device_cus()) return launch_values<T, NP, false, kWide, 2>(a, ld);
+    return launch_values<T, NP, false, kWide, 4>(a, ld);
 }
 
 template <int NP>

@@ -135,14 +135,27 @@ def test_decoding_attention_matches_the_oracle_chain(oracle, T, H, Dh, Cc, row0)
         out.zero_()
 
 
-# Each way the positions and heads are cut: heads above 100; up to 320 positions on 256 lanes, up to 512 on 512 lanes with
-# their own scores (both edges), a scores launch beyond, for one row and for two to four; score rows of more than 32 KiB of
+# Each way the positions and heads are cut: heads above 100; few positions on 256 lanes, more on 512 lanes with their own
+# scores, a scores launch beyond, for one row and for two to four (the edges of the cut are below); score rows of more than 32 KiB of
 # LDS (four rows from 4097 positions on) up to the most there can be; columns beyond the last row's position
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,H,Dh,Cc,row0", [(1, 16, 128, 69, 68), (2, 3, 104, 320, 318), (3, 2, 128, 321, 318), (1, 4, 128, 512, 511),
                                             (1, 4, 100, 400, 399), (4, 2, 64, 513, 509), (2, 4, 128, 1540, 1538), (3, 2, 112, 700, 697),
                                             (4, 2, 128, 4097, 4093), (4, 1, 128, 8192, 8188), (3, 1, 36, 8192, 8189), (2, 2, 120, 640, 333)])
 def test_decoding_attention_over_its_ranges(oracle, T, H, Dh, Cc, row0):
+    test_decoding_attention_matches_the_oracle_chain(oracle, T, H, Dh, Cc, row0)
+
+
+# How the lanes are dealt out since: 128 positions and one more, 480 and 960 (heads to 64, one or two rows) and one more;
+# behind the scores launch two lanes to a position (few workgroups) or four (32 heads of 100), and heads whose columns the
+# last workgroup of either does not fill (100, 36, 20) or that are less than one workgroup's (4); a step over the positions
+# less one, exactly one and one more (512 positions of two lanes, 1024 of one)
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,Dh,Cc,row0", [(1, 8, 128, 128, 127), (1, 8, 100, 129, 128), (4, 3, 36, 129, 125), (1, 5, 128, 480, 479),
+                                            (1, 32, 100, 481, 480), (2, 4, 64, 960, 958), (1, 3, 64, 961, 960), (3, 4, 64, 480, 477),
+                                            (3, 4, 64, 481, 478), (1, 3, 4, 961, 960), (2, 3, 20, 1024, 1022), (1, 32, 100, 1025, 1024),
+                                            (4, 32, 100, 513, 509), (1, 32, 128, 511, 510), (1, 2, 36, 2049, 2048)])
+def test_decoding_attention_where_its_cut_changes(oracle, T, H, Dh, Cc, row0):
     test_decoding_attention_matches_the_oracle_chain(oracle, T, H, Dh, Cc, row0)
 
 
