@@ -52,6 +52,7 @@ struct SkinnyArgs {
     const half_t *cos16, *sin16;
     half_t *kc, *vc;
     int H, Dh;
+    FastDiv half_head;       // by Dh / 2
     // NORM: with tok, row m of x is row tok[m] of A (the embedding of `vocab` rows); an id out of range raises
     // *status to m + 1 and reads the last row
     const uint16_t *tok;
@@ -104,6 +105,13 @@ template <int M, bool NORM, int EPI, int W, int kPre>
 __global__ void __launch_bounds__(W * 64)
 gemm_skinny_nt_kernel(SkinnyArgs p)
 {
+    // the argument block in scalar registers at once: field by field where the control flow first wants it, it is several
+    // round trips to memory before the weights are requested
+    if (NORM)
+        asm volatile("" ::"s"(p.N), "s"(p.K), "s"(p.alpha), "s"(p.A), "s"(p.lda), "s"(p.B), "s"(p.ldb), "s"(p.C), "s"(p.ldc),
+                     "s"(p.x2), "s"(p.w), "s"(p.eps), "s"(p.sum_out), "s"(p.tok), "s"(p.vocab));
+    if (NORM && EPI != E_PLAIN) asm volatile("" ::"s"(p.B2));
+    if (EPI == E_QKV) asm volatile("" ::"s"(p.B3), "s"(p.cos16), "s"(p.sin16), "s"(p.kc), "s"(p.vc), "s"(p.H), "s"(p.Dh), "s"(p.half_head.m), "s"(p.half_head.shift));
     constexpr int kThreads = W * 64;
     constexpr bool GATE = EPI == E_GATE;
     constexpr int NB = GATE ? 2 : 1;
@@ -118,29 +126,6 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
         for (int m = 0; m < M; m++)
 #pragma unroll
             for (int r = 0; r < kRows; r++) acc[b][m][r] = 0.f;
-    // rows past N re-read the last row (their sums are dropped)
-    const half_t *brow[NB][kRows];
-    int64_t col[kRows];
-    if (EPI == E_QKV) {
-        // the workgroup owns kRows / 2 consecutive rotation pairs (columns d and d + Dh/2 of a head), the left columns
-        // in the first half of its rows; blockIdx.y picks the query, key or value projection
-        const int hf = p.Dh / 2;
-        const half_t *Bsel = blockIdx.y == 0 ? p.B : blockIdx.y == 1 ? p.B2 : p.B3;
-#pragma unroll
-        for (int r = 0; r < kRows; r++) {
-            const int pair = blockIdx.x * (kRows / 2) + r % (kRows / 2), head = pair / hf;
-            col[r] = (int64_t)head * p.Dh + (pair - head * hf) + (r / (kRows / 2)) * hf;
-            brow[0][r] = Bsel + col[r] * p.ldb;
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < kRows; r++) {
-            col[r] = n0 + r;
-            const int64_t n = n0 + r < p.N ? n0 + r : p.N - 1;
-            brow[0][r] = p.B + n * p.ldb;
-            if (GATE) brow[NB - 1][r] = p.B2 + n * p.ldb;
-        }
-    }
     const half_t *arow[M];
 #pragma unroll
     for (int m = 0; m < M; m++) {
@@ -155,26 +140,60 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
         }
     }
     const int64_t chunks = p.K / 8;
-    for (int64_t base = 0; base < chunks; base += (int64_t)kPre * kThreads) {
-        half8_t b[kPre][NB][kRows];
-        h8 a[kPre][M], wv[NORM ? kPre : 1], x2v[NORM ? kPre : 1][M];
-        // Every load of the batch is issued before the first use, unconditionally (pieces past the row re-read its last
-        // piece): a load inside a branch is waited for at the end of the branch.  Loads return in order, so with NORM the row
-        // and its norm weights go first and the norm is worked out while the weights stream (gate and up of 5504 x 2048 10.5
-        // -> 10.0 us, q, k, v of 2048 8.0 -> 7.7; without a norm the row goes last: first it costs 3 % at 3200 x 8640).
-        if (NORM) {
+    h8 a[kPre][M], wv[NORM ? kPre : 1], x2v[NORM ? kPre : 1][M];
+    // Loads return in order, so with NORM (the whole row in one batch) the row and its norm weights go first, and the norm
+    // is worked out while the weights stream (gate and up of 5504 x 2048 10.5 -> 10.0 us; without a norm the row goes last:
+    // first it costs 3 % at 3200 x 8640).  They are requested before the weights' addresses are worked out, and the one batch
+    // is said to be one: in a loop over batches the compiler moves the first steps of the norm in front of it, i.e. in front
+    // of the weights' requests.  With that, q, k, v's cells and angles requested here and the arguments read at once: q, k, v
+    // of 2048 8.1 -> 6.9 us, gate and up 10.0 -> 9.6, a head of 32000 x 2048 22.3 -> 20.6; four rows of 3200: q, k, v
+    // 52 -> 28, gate and up 57 -> 36, head 142 -> 71.
+    if (NORM) {
 #pragma unroll
-            for (int j = 0; j < kPre; j++) {
-                const int64_t cr = base + j * kThreads + tid, c = cr < chunks ? cr : chunks - 1;
+        for (int j = 0; j < kPre; j++) {
+            const int64_t cr = j * kThreads + tid, c = cr < chunks ? cr : chunks - 1;
 #pragma unroll
-                for (int m = 0; m < M; m++) {
-                    a[j][m] = ld8(arow[m] + c * 8);
-                    x2v[j][m] = ld8((p.x2 ? p.x2 + m * p.lda : arow[m]) + c * 8);
-                }
-                wv[j] = ld8(p.w + c * 8);
+            for (int m = 0; m < M; m++) {
+                a[j][m] = ld8(arow[m] + c * 8);
+                x2v[j][m] = ld8((p.x2 ? p.x2 + m * p.lda : arow[m]) + c * 8);
             }
-            __builtin_amdgcn_sched_barrier(0);
+            wv[j] = ld8(p.w + c * 8);
         }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // rows past N re-read the last row (their sums are dropped)
+    const half_t *brow[NB][kRows];
+    int64_t col[kRows];
+    int dcol[kRows];                                         // QKV: the column inside its head
+    if (EPI == E_QKV) {
+        // the workgroup owns kRows / 2 consecutive rotation pairs (columns d and d + Dh/2 of a head), the left columns
+        // in the first half of its rows; blockIdx.y picks the query, key or value projection
+        // (Dh / 2 is even: both pairs are of one head)
+        const int hf = p.Dh / 2, head = p.half_head.div(blockIdx.x * (kRows / 2)), d0 = blockIdx.x * (kRows / 2) - head * hf;
+        const half_t *Bsel = blockIdx.y == 0 ? p.B : blockIdx.y == 1 ? p.B2 : p.B3;
+#pragma unroll
+        for (int r = 0; r < kRows; r++) {
+            dcol[r] = d0 + r % (kRows / 2) + (r / (kRows / 2)) * hf;
+            col[r] = (int64_t)head * p.Dh + dcol[r];
+            brow[0][r] = Bsel + col[r] * p.ldb;
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < kRows; r++) {
+            col[r] = n0 + r;
+            const int64_t n = n0 + r < p.N ? n0 + r : p.N - 1;
+            brow[0][r] = p.B + n * p.ldb;
+            if (GATE) brow[NB - 1][r] = p.B2 + n * p.ldb;
+        }
+    }
+    // QKV: what the epilogue needs from memory, lane (m, r); requested with the weights
+    const int er = tid % kRows, em = tid / kRows < M ? tid / kRows : M - 1;
+    int64_t ecol = 0;
+    half_t ecos = 0, esin = 0, ecell = 0;
+    for (int64_t base = 0; base < (NORM ? 1 : chunks); base += (int64_t)kPre * kThreads) {
+        half8_t b[kPre][NB][kRows];
+        // Every load of the batch is issued before the first use, unconditionally (pieces past the row re-read its last
+        // piece): a load inside a branch is waited for at the end of the branch.
 #pragma unroll
         for (int j = 0; j < kPre; j++) {
             const int64_t cr = base + j * kThreads + tid, c = cr < chunks ? cr : chunks - 1;
@@ -187,6 +206,18 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
 #pragma unroll
                 for (int m = 0; m < M; m++) a[j][m] = ld8(arow[m] + c * 8);
             }
+        }
+        if (EPI == E_QKV) {
+            int d = dcol[0];
+            ecol = col[0];
+#pragma unroll
+            for (int r = 1; r < kRows; r++) {
+                d = er == r ? dcol[r] : d;
+                ecol = er == r ? col[r] : ecol;
+            }
+            ecos = p.cos16[em * p.Dh + d];
+            esin = p.sin16[em * p.Dh + d];
+            ecell = (blockIdx.y == 1 ? p.kc : p.vc)[em * p.ldc + ecol];
         }
         if (NORM) __builtin_amdgcn_sched_barrier(0);
         if (NORM) {
@@ -266,15 +297,12 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
             if (blockIdx.y < 2) {
                 const bool left = r < kRows / 2;
                 const float xp = xr[m][left ? r + kRows / 2 : r - kRows / 2];
-                const int64_t d = col[r] % p.Dh;
-                const float cs = h2f(p.cos16[m * p.Dh + d]), sn = h2f(p.sin16[m * p.Dh + d]);
-                y = rnd16(rnd16(y * cs) + rnd16((left ? -xp : xp) * sn));
+                y = rnd16(rnd16(y * h2f(ecos)) + rnd16((left ? -xp : xp) * h2f(esin)));
             }
             if (blockIdx.y == 0) {
-                p.C[m * p.ldc + col[r]] = f2h(y);
+                p.C[m * p.ldc + ecol] = f2h(y);
             } else {
-                half_t *dst = (blockIdx.y == 1 ? p.kc : p.vc) + m * p.ldc + col[r];
-                *dst = f2h(h2f(*dst) + y);
+                (blockIdx.y == 1 ? p.kc : p.vc)[m * p.ldc + ecol] = f2h(h2f(ecell) + y);
             }
         }
         return;
@@ -412,6 +440,7 @@ int rows_qkv_launch(int64_t M, int64_t H, int64_t Dh, const RowSource &x, void *
     p.cos16 = (const half_t *)cos16; p.sin16 = (const half_t *)sin16;
     p.kc = (half_t *)k_cache_rows; p.vc = (half_t *)v_cache_rows;
     p.H = (int)H; p.Dh = (int)Dh;
+    p.half_head.set((uint32_t)(Dh / 2));
     return launch<true, E_QKV>(M, p, st);
 }
 
