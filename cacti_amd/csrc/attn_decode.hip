@@ -55,37 +55,45 @@ __device__ __forceinline__ float dot4(const h4 &a, const h4 &b, float acc)
     return __builtin_amdgcn_fdot2(a1, b1, __builtin_amdgcn_fdot2(a0, b0, acc, false), false);
 }
 
-// The lane's query pieces: piece i8 + 8 i of head h (zeros behind the head).
+// The lane's query pieces: piece i8 + 8 i of head h (the last one again behind the head).
 template <int T, int NP>
 __device__ __forceinline__ void load_q(h4 (&qv)[T][NP], const half_t *q, int64_t ldq, int h, int Dh, int i8)
 {
-    const int pieces = Dh / 4;
 #pragma unroll
-    for (int i = 0; i < NP; i++) {
-        const int c = i8 + 8 * i;
+    for (int i = 0; i < NP; i++)
 #pragma unroll
-        for (int t = 0; t < T; t++) {
-            qv[t][i] = *reinterpret_cast<const h4 *>(q + t * ldq + h * Dh + 4 * min(c, pieces - 1));
-            if (c >= pieces) qv[t][i] = h4{};
-        }
-    }
+        for (int t = 0; t < T; t++) qv[t][i] = *reinterpret_cast<const h4 *>(q + t * ldq + h * Dh + 4 * min(i8 + 8 * i, Dh / 4 - 1));
+}
+// ... and zeros there, once the first keys are on their way too
+template <int T, int NP>
+__device__ __forceinline__ void clear_q(h4 (&qv)[T][NP], int pieces, int i8)
+{
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+#pragma unroll
+        for (int t = 0; t < T; t++)
+            if (i8 + 8 * i >= pieces) qv[t][i] = h4{};
 }
 
-// f16(alpha q . K[j]) for the positions j0 + g + 32 it (it < kStep) below `end`, by the first of a position's lanes to
-// out[t * ldo + j - first]
-template <int T, int NP, int NT>
-__device__ __forceinline__ void scores_step(const h4 (&qv)[T][NP], const half_t *k_head, int64_t ldk, int pieces, float alpha, int j0,
-                                            int end, half_t *out, int64_t ldo, int first)
+// The lane's pieces of the keys j0 + g + NT / 8 it (it < kStep), of the last one before `end` behind it
+template <int NP, int NT>
+__device__ __forceinline__ void load_k(h4 (&kv)[kStep][NP], const half_t *k_head, int64_t ldk, int pieces, int j0, int end)
 {
-    constexpr int kGroups = NT / 8;
     const int i8 = threadIdx.x & 7, g = threadIdx.x >> 3;
-    h4 kv[kStep][NP];
 #pragma unroll
     for (int it = 0; it < kStep; it++)
 #pragma unroll
         for (int i = 0; i < NP; i++)
-            kv[it][i] = *reinterpret_cast<const h4 *>(k_head + (int64_t)min(j0 + g + it * kGroups, end - 1) * ldk +
+            kv[it][i] = *reinterpret_cast<const h4 *>(k_head + (int64_t)min(j0 + g + it * (NT / 8), end - 1) * ldk +
                                                       4 * min(i8 + 8 * i, pieces - 1));
+}
+// f16(alpha q . K[j]) for those positions, by the first of a position's lanes to out[t * ldo + j]
+template <int T, int NP, int NT>
+__device__ __forceinline__ void scores_step(const h4 (&qv)[T][NP], const h4 (&kv)[kStep][NP], float alpha, int j0, int end, half_t *out,
+                                            int64_t ldo)
+{
+    const int i8 = threadIdx.x & 7, g = threadIdx.x >> 3;
 #pragma unroll
     for (int it = 0; it < kStep; it++)
 #pragma unroll
@@ -96,8 +104,8 @@ __device__ __forceinline__ void scores_step(const h4 (&qv)[T][NP], const half_t 
             a += dpp_f32<0xB1>(a);              // lane ^ 1
             a += dpp_f32<0x4E>(a);              // lane ^ 2
             a += dpp_f32<0x141>(a);             // the other four of the eight
-            const int j = j0 + g + it * kGroups;
-            if (i8 == 0 && j < end) out[t * ldo + j - first] = f2h(alpha * a);
+            const int j = j0 + g + it * (NT / 8);
+            if (i8 == 0 && j < end) out[t * ldo + j] = f2h(alpha * a);
         }
 }
 
@@ -106,10 +114,13 @@ __global__ void __launch_bounds__(kThreads)
 decode_scores_kernel(int C, int Dh, float alpha, const half_t *__restrict__ q, int64_t ldq, const half_t *__restrict__ kc, int64_t ldk,
                      int64_t hsk, half_t *__restrict__ s16, int64_t ld)
 {
-    const int h = blockIdx.y, j0 = blockIdx.x * kSlice;
-    h4 qv[T][NP];
+    asm volatile("" ::"s"(C), "s"(Dh), "s"(alpha), "s"(q), "s"(ldq), "s"(kc), "s"(ldk), "s"(hsk), "s"(s16), "s"(ld));
+    const int h = blockIdx.y, j0 = blockIdx.x * kSlice, end = min(C, j0 + kSlice);
+    h4 qv[T][NP], kv[kStep][NP];
     load_q<T, NP>(qv, q, ldq, h, Dh, threadIdx.x & 7);
-    scores_step<T, NP, kThreads>(qv, kc + h * hsk, ldk, Dh / 4, alpha, j0, min(C, j0 + kSlice), s16 + (int64_t)h * T * ld, ld, 0);
+    load_k<NP, kThreads>(kv, kc + h * hsk, ldk, Dh / 4, j0, end);
+    clear_q<T, NP>(qv, Dh / 4, threadIdx.x & 7);
+    scores_step<T, NP, kThreads>(qv, kv, alpha, j0, end, s16 + (int64_t)h * T * ld, ld);
 }
 
 // OWN: the scores are formed here; otherwise they are s16[h][t][ld].  LP: lanes per position in the product with V.
@@ -119,6 +130,9 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
                      const half_t *__restrict__ vc, int64_t ldkv, int64_t hs, const half_t *__restrict__ s16, int64_t ld,
                      half_t *__restrict__ out, int64_t ldo)
 {
+    // the arguments in scalar registers at once (one by one, where first wanted, they are three round trips to memory)
+    asm volatile("" ::"s"(C), "s"(Dh), "s"(row0), "s"(alpha), "s"(q), "s"(ldq), "s"(kc), "s"(vc), "s"(ldkv), "s"(hs), "s"(s16), "s"(ld),
+                 "s"(out), "s"(ldo));
     extern __shared__ __attribute__((aligned(16))) half_t sp[];           // [T][ld]: scores, then probabilities
     __shared__ float scratch[2][T][NT / 64];
     __shared__ float red[NT / 64][T][LP][4];
@@ -135,14 +149,20 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
     };
     h4 vv[kStep];
     if (OWN) {
-        h4 qv[T][NP];
+        h4 qv[T][NP], kv[kStep][NP];
         load_q<T, NP>(qv, q, ldq, h, Dh, tid & 7);
-        for (int j0 = 0; j0 < C; j0 += NT / 8 * kStep) scores_step<T, NP, NT>(qv, kc + h * hs, ldkv, pieces, alpha, j0, C, sp, ld, 0);
+        load_k<NP, NT>(kv, kc + h * hs, ldkv, pieces, 0, C);
+        load_v(vv, 0);
+        clear_q<T, NP>(qv, pieces, tid & 7);
+        scores_step<T, NP, NT>(qv, kv, alpha, 0, C, sp, ld);
+        for (int j0 = NT / 8 * kStep; j0 < C; j0 += NT / 8 * kStep) {
+            load_k<NP, NT>(kv, kc + h * hs, ldkv, pieces, j0, C);
+            scores_step<T, NP, NT>(qv, kv, alpha, j0, C, sp, ld);
+        }
     } else {
         for (int i = tid; i < T * (int)ld / 8; i += NT) st8(sp + i * 8, ld8(s16 + (int64_t)h * T * ld + i * 8));
+        load_v(vv, 0);
     }
-    // (not before the scores' own loads, which would be returned behind them; the softmax covers these)
-    load_v(vv, 0);
     __syncthreads();
     // row maxima, then sums of exponentials, then the probabilities in place of the scores; row t sees live(t) positions
     auto live = [&](int t) __attribute__((always_inline)) { return (int)min((int64_t)C, (int64_t)t + row0 + 1); };
@@ -183,9 +203,7 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
     for (int t = 0; t < T; t++)
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[t][i] = 0.f;
-    for (int j0 = 0; j0 < C; j0 += kGroups * kStep) {
-        h4 vn[kStep];
-        load_v(vn, j0 + kGroups * kStep);                                  // (behind the last position: its row again)
+    auto add = [&](int j0) __attribute__((always_inline)) {
 #pragma unroll
         for (int it = 0; it < kStep; it++) {
             const int j = j0 + g + it * kGroups;
@@ -196,9 +214,16 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
                 for (int i = 0; i < 4; i++) acc[t][i] += p * h2f(vv[it].v[i]);
             }
         }
+    };
+    int j0 = 0;
+    for (; j0 + kGroups * kStep < C; j0 += kGroups * kStep) {
+        h4 vn[kStep];
+        load_v(vn, j0 + kGroups * kStep);
+        add(j0);
 #pragma unroll
         for (int it = 0; it < kStep; it++) vv[it] = vn[it];
     }
+    add(j0);                                  // (without a request behind it, which would be waited for)
 #pragma unroll
     for (int t = 0; t < T; t++)
 #pragma unroll
