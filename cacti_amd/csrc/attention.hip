@@ -11,7 +11,7 @@
 //
 // Layout: q, k, v, o and their adjoints are [S, H, Dh] (row stride ld), 8-byte aligned.
 //
-// Forward (a workgroup = 128 query rows of one head, 4 waves x 32 rows; keys in tiles of 64):
+// Forward (a workgroup = 128 or 64 query rows of one head, 32 rows to a wave; keys in tiles of 64):
 // the scores are computed twice.  Pass 1 keeps a running row maximum m and sum l of exp(S16 - m);
 // pass 2 recomputes S16 (same instructions, same bits), forms P16 = f16(exp(S16 - m) / l) -- the
 // reference's probabilities, not an unnormalised stand-in -- and accumulates O += P16 V.  Only
@@ -685,38 +685,54 @@ __device__ __forceinline__ void write_rows(const unsigned char *stage, half_t *d
 }
 
 // Work split of the query-major kernels (forward, dQ).  A workgroup is two wave groups of 4 waves on
-// the same 128 query rows; group g takes the key tiles g, g + 2, ... with its own LDS buffers, and the
-// two partial results (row statistics, output tile) meet in LDS at the end: the 2 waves a SIMD holds
-// have the same amount of work from start to end.
+// the same QR query rows; group g takes the key tiles g, g + 2, ... with its own LDS buffers, and the
+// partial results (row statistics, output tile) meet in LDS at the end: the 2 waves a SIMD holds
+// have the same amount of work from start to end.  With 128 rows each wave of a group has rows of its own
+// and takes whole key tiles, with 64 two of them share 32 rows and take half of the keys of a tile each
+// (which of the two: query_rows).
 constexpr int kNT2 = 2 * kNT;
 constexpr int kGroupLds = 4 * kTileB;                   // K and V tiles, two buffers each
 constexpr int kXsOff = 2 * kGroupLds;                   // float [2 groups][2][128]: statistics exchange
 constexpr size_t kQmSmem = 2 * kGroupLds + 2 * 2 * kBM * sizeof(float);
 
-// partial output tiles (DT x 16 floats per lane) of wave group 1 -> LDS -> added onto group 0's
-template <int DT>
-__device__ __forceinline__ void merge_partials(float16_t (&acc)[DT], unsigned char *region, int g, int tig)
+// What a wave takes with QR query rows per workgroup: query block qb and, of a group's four waves, part kp of the keys of
+// every tile (KP parts); its partial results are number `part` of 2 KP.
+template <int QR>
+struct WaveShare {
+    static constexpr int QB = QR / 32, KP = 4 / QB;
+    int qb, kp, part;
+    __device__ __forceinline__ WaveShare(int wid, int g) : qb(KP == 1 ? wid : wid % QB), kp(KP == 1 ? 0 : wid / QB), part(g * KP + kp) {}
+};
+
+// partial output tiles (DT x 16 floats per lane) 1 .. -> LDS -> added onto partial 0's; `region` ends at 2 kGroupLds
+template <int QR, int DT>
+__device__ __forceinline__ void merge_partials(float16_t (&acc)[DT], unsigned char *smem, const WaveShare<QR> &w, int lane)
 {
-    float *x = reinterpret_cast<float *>(region);
-    if (g == 1) {
+    constexpr int NP = 2 * WaveShare<QR>::KP, NL = WaveShare<QR>::QB * 64, ONE = DT * 16 * NL;
+    static_assert((NP - 1) * ONE * 4 <= 2 * kGroupLds - QR * kRowB, "beside the staged rows");
+    float *x = reinterpret_cast<float *>(smem + 2 * kGroupLds - (NP - 1) * ONE * 4) + w.qb * 64 + lane;
+    if (w.part > 0) {
+        float *mine = NP == 2 ? x : x + (w.part - 1) * ONE;
 #pragma unroll
         for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) x[(dt * 16 + r) * kNT + tig] = acc[dt][r];
+            for (int r = 0; r < 16; r++) mine[(dt * 16 + r) * NL] = acc[dt][r];
     }
     __syncthreads();
-    if (g == 0) {
+    if (w.part == 0) {
 #pragma unroll
-        for (int dt = 0; dt < DT; dt++)
+        for (int n = 0; n < NP - 1; n++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[dt][r] += x[(dt * 16 + r) * kNT + tig];
+            for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[dt][r] += x[n * ONE + (dt * 16 + r) * NL];
     }
 }
 
 // ---------------------------------------------------------------------------------------------
 // Workgroups take the tiles in descending order of their key count; a CU holds one workgroup at a
 // time (LDS), so the dispatcher hands the next tile to whichever CU is done first.
-template <int KS, int DT, bool FAST, bool DMA>
+template <int KS, int DT, bool FAST, bool DMA, int QR>
 __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
 {
     // the whole argument block in scalar registers at once (read field by field where the control flow first
@@ -734,19 +750,21 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
     const int lane = tig & 63, wid = __builtin_amdgcn_readfirstlane(tig >> 6), l32 = lane & 31, lh = lane >> 5;
     const int S = p.S, Dh = p.Dh;
     const int64_t ld = p.ld;
-    const int nqt = (S + kBM - 1) / kBM;
+    const int nqt = (S + QR - 1) / QR;
+    const WaveShare<QR> ws(wid, g);
+    constexpr int KP = WaveShare<QR>::KP, NP = 2 * KP;
     const int h = blockIdx.x % p.H, qt = nqt - 1 - blockIdx.x / p.H;
     const int shift = DMA ? (int)(((int64_t)h * Dh) & 7) : 0;          // the head's first column in its window
     gptr_t Q = gp(p.q) + (int64_t)h * Dh, K = gp(p.k) + (int64_t)h * Dh - shift, V = gp(p.v) + (int64_t)h * Dh - shift;
     {
-        const int i0 = qt * kBM, r0 = i0 + wid * 32, myrow = r0 + l32;
+        const int i0 = qt * QR, qrow = ws.qb * 32 + l32, r0 = i0 + ws.qb * 32, myrow = r0 + l32;
 
         // the queries: with direct tiles they come as two tiles straight into LDS below, beside the first key
         // and value tiles (a load in which every lane addresses its own row is served at one lane per clock)
         half8_t qf[KS];
         if constexpr (!DMA) load_frags<KS>(qf, Q, ld, myrow, S, Dh, lh, shift);
 
-        const int kend = min(i0 + kBM, S);                 // keys [0, kend) are visible to the tile
+        const int kend = min(i0 + QR, S);                 // keys [0, kend) are visible to the tile
         const int njt = (kend + kTileRows - 1) / kTileRows, niter = (njt + 1) / 2;
         typedef typename std::conditional<DMA, DmaTileMap, FastTileMap>::type Map;
         typedef typename std::conditional<DMA, DmaTileLoader, FastTileLoader>::type Loader;
@@ -764,14 +782,15 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
         if constexpr (DMA) {
             // rows 64 g .. 64 g + 63 of the workgroup's queries into this group's second V buffer, which idles
             // until the second pass; every wave then takes its fragments from the tile that holds its rows
-            tv.load(tm, Q - shift + (int64_t)(i0 + g * kTileRows) * ld, S - (i0 + g * kTileRows), Vs + kTileB);
+            if (QR > 64 || g == 0)
+                tv.load(tm, Q - shift + (int64_t)(i0 + g * kTileRows) * ld, S - (i0 + g * kTileRows), Vs + kTileB);
             zero_pads(smem, 2 * kGroupLds / kRowB, (Dh + shift + 7) >> 3);
         }
         tile_sync<DMA>();
         if constexpr (DMA)
-            frags_from_tile<KS>(qf, smem + (wid >> 1) * kGroupLds + 3 * kTileB, (wid & 1) * 32 + l32, Dh, lh, shift);
+            frags_from_tile<KS>(qf, smem + (ws.qb >> 1) * kGroupLds + 3 * kTileB, (ws.qb & 1) * 32 + l32, Dh, lh, shift);
         int it0 = 0;
-        if constexpr (FAST) {
+        if constexpr (FAST && KP == 1) {
             // The key tiles wholly below the diagonal for every wave (iterations 0 .. qt - 1 of both groups) as a
             // pipeline: the products of a score tile run while the statistics of the tile before it are updated.
             // The same operations on the same values in the same order as the general loop below.
@@ -832,8 +851,8 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
             if (nxt) tk.load(tm, K + (int64_t)(jt + 2) * kTileRows * ld, S - (jt + 2) * kTileRows, Ks + (cur ^ 1) * kTileB);
             if (jt < njt) {
 #pragma unroll
-                for (int kt = 0; kt < 2; kt++) {
-                    const int kb = jt * kTileRows + 32 * kt;
+                for (int k2 = 0; k2 < 2 / KP; k2++) {
+                    const int kt = KP == 1 ? k2 : ws.kp, kb = jt * kTileRows + 32 * kt;
                     if (kb > r0 + 31) continue;          // every key of the tile is beyond every row of the wave
                     const float16_t acc = prod_direct<KS>(Ks + cur * kTileB, 32 * kt, qf, l32, lh);
                     const bool full = kb + 31 <= r0;
@@ -897,7 +916,7 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
         }
         float m, l;
         {
-            // the four partial (maximum, sum) pairs of a row -- two lanes in each of two groups -- merged
+            // the partial (maximum, sum) pairs of a row -- two lanes in each wave that holds it -- merged
             // in one fixed order by every lane that needs the result
             const float m_o = __shfl_xor(m_run, 32, 64), l_o = __shfl_xor(l_run, 32, 64);
             const float ma = lh ? m_o : m_run, la = lh ? l_o : l_run;
@@ -905,16 +924,22 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
             const float mg = fmaxf(ma, mb);
             const float lg = ((ma == -INFINITY) ? 0.f : la * M::ex(ma, mg)) + ((mb == -INFINITY) ? 0.f : lb * M::ex(mb, mg));
             if (lh == 0) {
-                xs[(g * 2 + 0) * kBM + wid * 32 + l32] = mg;
-                xs[(g * 2 + 1) * kBM + wid * 32 + l32] = lg;
+                xs[(ws.part * 2 + 0) * QR + qrow] = mg;
+                xs[(ws.part * 2 + 1) * QR + qrow] = lg;
             }
             __syncthreads();
-            const float m0 = xs[0 * kBM + wid * 32 + l32], l0 = xs[1 * kBM + wid * 32 + l32];
-            const float m1 = xs[2 * kBM + wid * 32 + l32], l1 = xs[3 * kBM + wid * 32 + l32];
-            m = fmaxf(m0, m1);
-            l = ((m0 == -INFINITY) ? 0.f : l0 * M::ex(m0, m)) + ((m1 == -INFINITY) ? 0.f : l1 * M::ex(m1, m));
+            m = xs[qrow];
+#pragma unroll
+            for (int n = 1; n < NP; n++) m = fmaxf(m, xs[2 * n * QR + qrow]);
+            l = 0.f;
+#pragma unroll
+            for (int n = 0; n < NP; n++) {
+                const float mn = xs[2 * n * QR + qrow], ln = xs[(2 * n + 1) * QR + qrow];
+                const float e = (mn == -INFINITY) ? 0.f : ln * M::ex(mn, m);
+                l = n ? l + e : e;
+            }
             if (myrow >= S) { m = 0.f; l = 1.f; }
-            if (g == 0 && lh == 0 && myrow < S) {
+            if (ws.part == 0 && lh == 0 && myrow < S) {
                 p.m[(int64_t)h * S + myrow] = m;
                 p.l[(int64_t)h * S + myrow] = l;
             }
@@ -936,7 +961,7 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
         }
         tile_sync<DMA>();
         int it2 = 0;
-        if constexpr (FAST && DMA) {
+        if constexpr (FAST && DMA && KP == 1) {
             // The key tiles wholly below the diagonal for every wave, as in pass 1, with the vector arithmetic of a
             // block between the MFMAs of its neighbours: per tile, the scores of its second block are formed while
             // the probabilities of the first are, the first block's P V products run while the second's
@@ -993,8 +1018,8 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
             }
             if (jt < njt) {
 #pragma unroll
-                for (int kt = 0; kt < 2; kt++) {
-                    const int kb = jt * kTileRows + 32 * kt;
+                for (int k2 = 0; k2 < 2 / KP; k2++) {
+                    const int kt = KP == 1 ? k2 : ws.kp, kb = jt * kTileRows + 32 * kt;
                     if (kb > r0 + 31) continue;
                     const float16_t acc = prod_direct<KS>(Ks + cur * kTileB, 32 * kt, qf, l32, lh);
                     const bool full = kb + 31 <= r0;
@@ -1030,13 +1055,13 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
             }
             tile_sync<DMA>();
         }
-        merge_partials<DT>(oacc, smem + kGroupLds, g, tig);
+        merge_partials<QR, DT>(oacc, smem, ws, lane);
         if constexpr (DMA) {
-            if (g == 0) stage_rows<DT>(smem, oacc, wid * 32 + l32, lh, 1.0f);
+            if (ws.part == 0) stage_rows<DT>(smem, oacc, qrow, lh, 1.0f);
             __syncthreads();
-            write_rows(smem, p.out + (int64_t)i0 * ld + (int64_t)h * Dh - shift, ld, min(kBM, S - i0), Dh, shift,
+            write_rows(smem, p.out + (int64_t)i0 * ld + (int64_t)h * Dh - shift, ld, min(QR, S - i0), Dh, shift,
                        threadIdx.x, kNT2);
-        } else if (g == 0 && myrow < S) {
+        } else if (ws.part == 0 && myrow < S) {
             half_t *orow = p.out + (int64_t)myrow * ld + (int64_t)h * Dh;
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
@@ -1055,7 +1080,7 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
 // dQ: queries fixed, loop over the key tiles at or before them, work split as in the forward kernel.
 // Pass 0 forms sigma = sum_j P' f32(dP16); pass 1 dS16 and dQ.  Leaves y = 1 / l and sigma per row for
 // the dK / dV kernel.
-template <int KS, int DT, bool FAST, bool DMA>
+template <int KS, int DT, bool FAST, bool DMA, int QR>
 __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
 {
     // the whole argument block in scalar registers at once (read field by field where the control flow first
@@ -1071,7 +1096,9 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
     const int lane = tig & 63, wid = __builtin_amdgcn_readfirstlane(tig >> 6), l32 = lane & 31, lh = lane >> 5;
     const int S = p.S, Dh = p.Dh;
     const int64_t ld = p.ld;
-    const int nqt = (S + kBM - 1) / kBM;
+    const int nqt = (S + QR - 1) / QR;
+    const WaveShare<QR> ws(wid, g);
+    constexpr int KP = WaveShare<QR>::KP, NP = 2 * KP;
     const int h = blockIdx.x % p.H, qt = nqt - 1 - blockIdx.x / p.H;
     const int64_t hoff = (int64_t)h * Dh;
     const int shift = DMA ? (int)(hoff & 7) : 0;                        // the head's first column in its window
@@ -1080,8 +1107,8 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
     if constexpr (!DMA) zero_lds(smem, 2 * kGroupLds);
     gptr_t K = gp(p.k) + hoff - shift, V = gp(p.v) + hoff - shift;
     {
-        const int i0 = qt * kBM, r0 = i0 + wid * 32, myrow = r0 + l32;
-        const int kend = min(i0 + kBM, S);
+        const int i0 = qt * QR, qrow = ws.qb * 32 + l32, r0 = i0 + ws.qb * 32, myrow = r0 + l32;
+        const int kend = min(i0 + QR, S);
         const int njt = (kend + kTileRows - 1) / kTileRows, niter = (njt + 1) / 2;
         typedef typename std::conditional<DMA, DmaTileMap, TileMap8>::type Map;
         typedef typename std::conditional<DMA, DmaTileLoader, TileLoader8>::type Loader;
@@ -1105,18 +1132,26 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
         bool tiles_on_the_way = false;
         float m = ((gfptr_t)p.m)[(int64_t)h * S + min(myrow, S - 1)];
         float l = ((gfptr_t)p.l)[(int64_t)h * S + min(myrow, S - 1)];
+        // the row this lane votes for on the form of sigma below: of the 128 rows the workgroup's are part of
+        const int vrow = QR == 128 ? myrow : (i0 & ~127) + (threadIdx.x & 127);
+        const float lvote = QR == 128 ? l : ((gfptr_t)p.l)[(int64_t)h * S + min(vrow, S - 1)];
         half8_t qf[KS], gf[KS], of[FAST ? KS : 1];
         if constexpr (DMA) {
-            const int64_t off = hoff - shift + (int64_t)(i0 + g * kTileRows) * ld;
-            const int left = S - (i0 + g * kTileRows);
+            const int first = i0 + (QR > 64 ? g * kTileRows : 0), left = S - first;
+            const int64_t off = hoff - shift + (int64_t)first * ld;
             const bool want_o = FAST && p.o;
-            tk.load(tm, gp(p.q) + off, left, smem + g * kTileB);
-            tk.load(tm, gp(p.dO) + off, left, smem + (2 + g) * kTileB);
-            if (want_o) tk.load(tm, gp(p.o) + off, left, smem + (4 + g) * kTileB);
+            if (QR > 64) {
+                tk.load(tm, gp(p.q) + off, left, smem + g * kTileB);
+                tk.load(tm, gp(p.dO) + off, left, smem + (2 + g) * kTileB);
+                if (want_o) tk.load(tm, gp(p.o) + off, left, smem + (4 + g) * kTileB);
+            } else {                              // three tiles, two groups
+                tk.load(tm, (g ? gp(p.dO) : gp(p.q)) + off, left, smem + 2 * g * kTileB);
+                if (want_o && g) tk.load(tm, gp(p.o) + off, left, smem + 4 * kTileB);
+            }
             zero_pads(smem, 2 * kGroupLds / kRowB, (Dh + shift + 7) >> 3);
             tile_sync<DMA>();
-            const unsigned char *mine = smem + (wid >> 1) * kTileB;
-            const int trow = (wid & 1) * 32 + l32;
+            const unsigned char *mine = smem + (ws.qb >> 1) * kTileB;
+            const int trow = (ws.qb & 1) * 32 + l32;
             frags_from_tile<KS>(qf, mine, trow, Dh, lh, shift);
             frags_from_tile<KS>(gf, mine + 2 * kTileB, trow, Dh, lh, shift);
             if constexpr (FAST) {
@@ -1156,8 +1191,8 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
                 }
                 if (jt < njt) {
 #pragma unroll
-                    for (int kt = 0; kt < 2; kt++) {
-                        const int kb = jt * kTileRows + 32 * kt;
+                    for (int k2 = 0; k2 < 2 / KP; k2++) {
+                        const int kt = KP == 1 ? k2 : ws.kp, kb = jt * kTileRows + 32 * kt;
                         if (kb > r0 + 31) continue;
                         const float16_t sacc = prod_direct<KS>(Ks + cur * kTileB, 32 * kt, qf, l32, lh);
                         const float16_t pacc = prod_direct<KS>(Vs + cur * kTileB, 32 * kt, gf, l32, lh);
@@ -1218,13 +1253,13 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
         // over the keys; in the reference's arithmetic the two differ by the f16 roundings of dP16, P16 and O,
         // about 2^-11 |dP| sqrt(sum_j P_ij^2).  Where a row's probability mass is spread that is below the
         // rounding of dS16 itself.  Where it sits on one key it is not: the reference has dP16 - sigma = 0
-        // there exactly, and rows 0 and 1 of a sequence failed the element bound with the short form.  So a
-        // workgroup takes the short form only if every one of its rows has sum_j exp(S16_ij - m_i) >= kSpread
-        // (no probability above 1 / kSpread), else the pass over the keys; the exactly rounded build always
-        // takes the pass.
+        // there exactly, and rows 0 and 1 of a sequence failed the element bound with the short form.  So
+        // 128 rows (of one workgroup or two) take the short form only if every one of them has sum_j
+        // exp(S16_ij - m_i) >= kSpread (no probability above 1 / kSpread), else the pass over the keys; the
+        // exactly rounded build always takes the pass.
         bool short_sigma = false;
         if constexpr (FAST) {
-            if (p.o) short_sigma = __syncthreads_and(myrow >= S || l >= kSpread) != 0;
+            if (p.o) short_sigma = __syncthreads_and(vrow >= S || lvote >= kSpread) != 0;
         }
         if (short_sigma) {
             float part = 0.f;
@@ -1235,12 +1270,14 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
             sig = part + __shfl_xor(part, 32, 64);                     // the two lanes of a row
         } else {
             const float part = run_pass(std::integral_constant<int, 0>{});
-            const float pg = part + __shfl_xor(part, 32, 64);         // the two lanes of a row, then the two groups
-            if (lh == 0) xs[g * kBM + wid * 32 + l32] = pg;
+            const float pg = part + __shfl_xor(part, 32, 64);         // the two lanes of a row, then the waves that hold it
+            if (lh == 0) xs[ws.part * QR + qrow] = pg;
             __syncthreads();
-            sig = xs[wid * 32 + l32] + xs[kBM + wid * 32 + l32];
+            sig = xs[qrow];
+#pragma unroll
+            for (int n = 1; n < NP; n++) sig += xs[n * QR + qrow];
         }
-        if (g == 0 && lh == 0 && myrow < S) {
+        if (ws.part == 0 && lh == 0 && myrow < S) {
             p.y[(int64_t)h * S + myrow] = FAST ? cs : y;          // what the dK / dV kernel wants per row
             p.sig[(int64_t)h * S + myrow] = sig;
         }
@@ -1249,12 +1286,12 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
 #pragma unroll
             for (int r = 0; r < 16; r++) dacc[dt][r] = 0.f;
         run_pass(std::integral_constant<int, 1>{});
-        merge_partials<DT>(dacc, smem + kGroupLds, g, tig);
+        merge_partials<QR, DT>(dacc, smem, ws, lane);
         if (DMA && !p.acc_dq) {
-            if (g == 0) stage_rows<DT>(smem, dacc, wid * 32 + l32, lh, p.alpha);
+            if (ws.part == 0) stage_rows<DT>(smem, dacc, qrow, lh, p.alpha);
             __syncthreads();
-            write_rows(smem, p.dq + (int64_t)i0 * ld + hoff - shift, ld, min(kBM, S - i0), Dh, shift, threadIdx.x, kNT2);
-        } else if (g == 0 && myrow < S) {
+            write_rows(smem, p.dq + (int64_t)i0 * ld + hoff - shift, ld, min(QR, S - i0), Dh, shift, threadIdx.x, kNT2);
+        } else if (ws.part == 0 && myrow < S) {
             half_t *drow = p.dq + (int64_t)myrow * ld + hoff;
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
@@ -1697,17 +1734,36 @@ int set_smem(K kern, size_t bytes)
 // the CPU restatement of the reference to 4.9e-5 .. 7.1e-5.
 std::atomic<int> g_exact{0};             // cacti_hip_attention_set_exact: launch the exactly rounded forms
 
+// Query rows per workgroup of the forward and the dQ kernel, 64 or 128.  A workgroup has a CU to itself and walks its keys
+// 128 at a time; with 64 rows two waves share a tile's keys, so a step takes less time (one head of 128: 2.1 us against 2.85
+// forward) and there are twice as many workgroups, each of which reads all keys.  Worth it until they need a third round
+// over the CUs: 128 -> 64 rows, us, forward and adjoint, 611 positions, 16 heads of 64 19.2 -> 16.1 and 42.3 -> 35.4; 777,
+// 16 of 128 26.0 -> 20.7 and 62 -> 53; 1534, 16 of 100 41.3 -> 32.2 and 92 -> 85; 1984, 16 of 128 (496 workgroups) 50.8 ->
+// 46.2 and 115 -> 107; 1422, 24 of 100 (552) 38.4 -> 47.5 and 90 -> 94; 2048, 32 of 100 (1024) 68 -> 95 and 156 -> 168.
+// Exact arithmetic: 1531, 16 of 128 71.8 -> 43.7 and 172 -> 134.  The forward kernel's second round is short only if there
+// are long sequences in the first: 901, 32 of 100 (480 workgroups) 28.1 -> 29.2, 786 (416) 25.4 -> 25.6.
+int query_rows(int64_t S, int64_t H, bool forward, bool fast)
+{
+    const int64_t cus = device_cus(), wgs = (S + 63) / 64 * H;
+    return wgs <= (forward && fast && S <= 1024 ? cus + cus * 3 / 4 : 2 * cus) ? 64 : 128;
+}
+
 template <int KS, int DT, bool FAST, bool DMA>
 int launch_fwd(const AttnArgs &p, hipStream_t st)
 {
     static DeviceOnce ready;
     if (!ready.fresh()) {
-        int rc = set_smem(attn_fwd_kernel<KS, DT, FAST, DMA>, kQmSmem);
+        int rc = set_smem(attn_fwd_kernel<KS, DT, FAST, DMA, 128>, kQmSmem);
         if (rc) return rc;
+        if constexpr (DMA)
+            if ((rc = set_smem(attn_fwd_kernel<KS, DT, FAST, DMA, 64>, kQmSmem))) return rc;
         ready.mark();
     }
-    const int nqt = (p.S + kBM - 1) / kBM;
-    hipLaunchKernelGGL((attn_fwd_kernel<KS, DT, FAST, DMA>), dim3((unsigned)(nqt * p.H)), dim3(kNT2), kQmSmem, st, p);
+    const int rows = DMA ? query_rows(p.S, p.H, true, FAST) : 128, nqt = (p.S + rows - 1) / rows;
+    const dim3 grid((unsigned)(nqt * p.H));
+    if constexpr (DMA)
+        if (rows == 64) hipLaunchKernelGGL((attn_fwd_kernel<KS, DT, FAST, DMA, 64>), grid, dim3(kNT2), kQmSmem, st, p);
+    if (rows == 128) hipLaunchKernelGGL((attn_fwd_kernel<KS, DT, FAST, DMA, 128>), grid, dim3(kNT2), kQmSmem, st, p);
     return launch_status("attention_fwd");
 }
 
@@ -1717,15 +1773,21 @@ int launch_bwd(const AttnArgs &p, hipStream_t st)
     constexpr bool PARTS = FAST && DMA;
     static DeviceOnce ready;
     if (!ready.fresh()) {
-        int rc = set_smem(attn_bwd_dq_kernel<KS, DT, FAST, DMA>, kQmSmem);
+        int rc = set_smem(attn_bwd_dq_kernel<KS, DT, FAST, DMA, 128>, kQmSmem);
         if (rc) return rc;
+        if constexpr (DMA)
+            if ((rc = set_smem(attn_bwd_dq_kernel<KS, DT, FAST, DMA, 64>, kQmSmem))) return rc;
         if ((rc = set_smem(attn_bwd_dkv_kernel<KS, DT, FAST, DMA, false>, kDkvSmem))) return rc;
         if constexpr (PARTS)
             if ((rc = set_smem(attn_bwd_dkv_kernel<KS, DT, FAST, DMA, true>, kDkvSmem))) return rc;
         ready.mark();
     }
     const int nqt = (p.S + kBM - 1) / kBM;
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<KS, DT, FAST, DMA>), dim3((unsigned)(nqt * p.H)), dim3(kNT2), kQmSmem, st, p);
+    const int rows = DMA ? query_rows(p.S, p.H, false, FAST) : 128;
+    const dim3 grid((unsigned)((p.S + rows - 1) / rows * p.H));
+    if constexpr (DMA)
+        if (rows == 64) hipLaunchKernelGGL((attn_bwd_dq_kernel<KS, DT, FAST, DMA, 64>), grid, dim3(kNT2), kQmSmem, st, p);
+    if (rows == 128) hipLaunchKernelGGL((attn_bwd_dq_kernel<KS, DT, FAST, DMA, 128>), grid, dim3(kNT2), kQmSmem, st, p);
     int rc = launch_status("attention_bwd_dq");
     if (rc) return rc;
     if constexpr (PARTS)

@@ -717,6 +717,23 @@ def test_fused_attention(ops, oracle, S, H, Dh):
         assert_bits(host(a), host(b), "repeat")
 
 
+# The forward and the dQ kernel take 64 query rows per workgroup where their number is at most twice (forward, fast, up to
+# 1024 positions: 7/4 of) the CUs' of an MI355X, 256, and 128 beyond: rows one short of, on and one past the edges of both
+# at few heads, and the 128 rows' form at many small heads (480 workgroups of 64 rows: forward only; 528, 640: both), with
+# tiles straight into LDS, in windows (heads of 12, 100) and, exact, in the other arithmetic
+@pytest.mark.gpu
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("S,H,Dh", [(63, 2, 64), (64, 1, 128), (65, 2, 100), (127, 2, 128), (129, 4, 64), (191, 2, 100), (193, 1, 128),
+                                    (130, 160, 8), (130, 176, 8), (257, 128, 12), (321, 86, 16)])
+def test_fused_attention_by_query_rows(ops, oracle, S, H, Dh, exact):
+    from cacti_amd import ffi
+    ffi.call("cacti_hip_attention_set_exact", int(exact))
+    try:
+        test_fused_attention(ops, oracle, S, H, Dh)
+    finally:
+        ffi.call("cacti_hip_attention_set_exact", 0)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("gain,exact", [(8.0, False), (24.0, True), (2.0, True)])
 def test_fused_attention_with_large_scores(ops, oracle, gain, exact):
