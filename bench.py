@@ -130,7 +130,7 @@ def kernel_symbol(label):
     rocprofv3 prints it, for 16-byte aligned operands (tiles of 64 columns run two workgroups to a CU)."""
     ta, tb, H, M, N, K = gemm_dims(label)
     bm, bn = gemm_plan(M, N, K)[0]
-    return "gemm_direct_kernel<%s, %s, %d, %d, %d, false>" % (str(ta).lower(), str(tb).lower(), bm, bn, 2 if bn == 64 or (bm, bn) == (64, 128) else 1)
+    return "gemm_direct_kernel<%s, %s, %d, %d, %d, false, false>" % (str(ta).lower(), str(tb).lower(), bm, bn, 2 if bn == 64 or (bm, bn) == (64, 128) else 1)
 
 
 def is_split(label):
