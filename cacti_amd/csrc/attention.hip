@@ -706,11 +706,11 @@ struct WaveShare {
 
 // partial output tiles (DT x 16 floats per lane) 1 .. -> LDS -> added onto partial 0's; `region` ends at 2 kGroupLds
 template <int QR, int DT>
-__device__ __forceinline__ void merge_partials(float16_t (&acc)[DT], unsigned char *smem, const WaveShare<QR> &w, int lane)
+__device__ __forceinline__ void merge_partials(float16_t (&acc)[DT], unsigned char *smem, const WaveShare<QR> &w, int tig)
 {
     constexpr int NP = 2 * WaveShare<QR>::KP, NL = WaveShare<QR>::QB * 64, ONE = DT * 16 * NL;
     static_assert((NP - 1) * ONE * 4 <= 2 * kGroupLds - QR * kRowB, "beside the staged rows");
-    float *x = reinterpret_cast<float *>(smem + 2 * kGroupLds - (NP - 1) * ONE * 4) + w.qb * 64 + lane;
+    float *x = reinterpret_cast<float *>(smem + 2 * kGroupLds - (NP - 1) * ONE * 4) + (tig & (NL - 1));
     if (w.part > 0) {
         float *mine = NP == 2 ? x : x + (w.part - 1) * ONE;
 #pragma unroll
@@ -1055,7 +1055,7 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
             }
             tile_sync<DMA>();
         }
-        merge_partials<QR, DT>(oacc, smem, ws, lane);
+        merge_partials<QR, DT>(oacc, smem, ws, tig);
         if constexpr (DMA) {
             if (ws.part == 0) stage_rows<DT>(smem, oacc, qrow, lh, 1.0f);
             __syncthreads();
@@ -1286,7 +1286,7 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
 #pragma unroll
             for (int r = 0; r < 16; r++) dacc[dt][r] = 0.f;
         run_pass(std::integral_constant<int, 1>{});
-        merge_partials<QR, DT>(dacc, smem, ws, lane);
+        merge_partials<QR, DT>(dacc, smem, ws, tig);
         if (DMA && !p.acc_dq) {
             if (ws.part == 0) stage_rows<DT>(smem, dacc, qrow, lh, p.alpha);
             __syncthreads();
@@ -1307,14 +1307,16 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
 }
 
 // ---------------------------------------------------------------------------------------------
-// dK, dV: keys fixed (128 per workgroup of 4 waves, a lane owns one), loop over the query tiles at or
+// dK, dV: keys fixed (128 or 64 per workgroup of 4 waves, a lane owns one), loop over the query tiles at or
 // after them; the key tiles with the most queries first.
 
-constexpr int kDkvBufs = 3;                      // tile buffers per tensor (Q, dO) and sets of row statistics
+// tile buffers per tensor (Q, dO) and sets of row statistics
+constexpr int dkv_bufs(int keys) { return keys == 128 ? 3 : 2; }
 
 // SPLIT: a workgroup takes p.per of the query tiles of its keys and leaves its sums in p.part (dkv_parts).
-template <int KS, int DT, bool FAST, bool DMA, bool SPLIT>
-__global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
+// KR: keys per workgroup.  With 64 two waves share 32 keys and take one 32-query block of every tile each.
+template <int KS, int DT, bool FAST, bool DMA, bool SPLIT, int KR>
+__global__ void __launch_bounds__(kNT, KR == 64 && KS == 4 ? 2 : 1) attn_bwd_dkv_kernel(AttnArgs p)
 {
     // the whole argument block in scalar registers at once (read field by field where the control flow first
     // wants it, it costs several dependent round trips to memory before the first tile is requested)
@@ -1322,29 +1324,32 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
                  "s"(p.o), "s"(p.out), "s"(p.dq), "s"(p.dk), "s"(p.dv), "s"(p.m), "s"(p.l), "s"(p.y), "s"(p.sig),
                  "s"(p.acc_dq), "s"(p.acc_dk), "s"(p.acc_dv));
     typedef AttnMath<FAST> M;
+    constexpr int BUFS = dkv_bufs(KR);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    unsigned char *Qs = smem, *Gs = smem + kDkvBufs * kTileB;
-    float *St = reinterpret_cast<float *>(smem + 2 * kDkvBufs * kTileB);   // [3][4][64]: m, l, y, sigma of a tile's rows
+    unsigned char *Qs = smem, *Gs = smem + BUFS * kTileB;
+    float *St = reinterpret_cast<float *>(smem + 2 * BUFS * kTileB);   // [3][4][64]: m, l, y, sigma of a tile's rows
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = lane & 31,
               lh = lane >> 5;
     const int S = p.S, Dh = p.Dh;
     const int64_t ld = p.ld;
     const int h = blockIdx.x % p.H, pz = blockIdx.x / p.H, pr = SPLIT ? pz / p.split : pz, z = SPLIT ? pz - pr * p.split : 0;
-    const int first_tile = pr * (kBM / kTileRows) + z * (SPLIT ? p.per : 0);
+    static_assert(KR == 128 || (KR == 64 && DMA && !SPLIT), "keys of a workgroup");
+    const int kb = KR == 128 ? wid : wid & 1, qh = KR == 128 ? 0 : wid >> 1;
+    const int first_tile = pr * (KR / kTileRows) + z * (SPLIT ? p.per : 0);
     if (SPLIT && first_tile * kTileRows >= S) return;                   // no query tile left for this part
     const int64_t hoff = (int64_t)h * Dh;
     const int shift = DMA ? (int)(hoff & 7) : 0;                        // the head's first column in its window
     gptr_t Q = gp(p.q) + hoff - shift, G = gp(p.dO) + hoff - shift;
     // the pad columns of the tile buffers: zero from the first tile's barrier on (direct tiles: cleared below,
     // behind the first loads)
-    if constexpr (!DMA) zero_lds(smem, 2 * kDkvBufs * kTileB);
+    if constexpr (!DMA) zero_lds(smem, 2 * BUFS * kTileB);
     // the four per-row statistics of a 64-query tile: lane t of wave w fetches array w, row t
     gfptr_t stat_src = (gfptr_t)(wid == 0 ? p.m : wid == 1 ? p.l : wid == 2 ? p.y : p.sig) + (int64_t)h * S;
     const float stat_pad = (wid == 1 || wid == 2) ? 1.f : 0.f;
 
     {
         const int kt_ = pr;                                             // low key tiles see the most queries
-        const int c00 = kt_ * kBM, c0 = c00 + wid * 32, mykey = c0 + l32;
+        const int c00 = kt_ * KR, c0 = c00 + kb * 32, mykey = c0 + l32;
 
         // the keys and values of the workgroup: with direct tiles they come as tiles straight into LDS, beside the
         // first query tile (below)
@@ -1373,7 +1378,7 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
             const float t = stat_src[row < S ? row : S - 1];
             st = row < S ? t : stat_pad;          // rows beyond S are masked; the pad only has to be finite
         };
-        auto buf_of = [&](int iq) __attribute__((always_inline)) { return (iq - iq0) % kDkvBufs; };
+        auto buf_of = [&](int iq) __attribute__((always_inline)) { return (iq - iq0) % BUFS; };
         auto fetch = [&](int iq) __attribute__((always_inline)) {        // tile iq on its way (registers or LDS)
             const int bf = buf_of(iq);
             tq.load(tm, Q + (int64_t)iq * kTileRows * ld, S - iq * kTileRows, Qs + bf * kTileB);
@@ -1451,7 +1456,7 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
             for (int iq = a; iq < b; iq++) {
                 if (iq + 1 < niq) fetch(iq + 1);
 #pragma unroll 1
-                for (int qb = 0; qb < 2; qb++) block(iq, qb);
+                for (int qb = qh; qb < (KR == 128 ? 2 : qh + 1); qb++) block(iq, qb);
                 if (iq + 1 < niq) land(iq + 1);
                 tile_sync<DMA>();
             }
@@ -1460,19 +1465,19 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
         fetch(iq0);
         land(iq0);
         if constexpr (DMA) {
-            // the 128 key and value rows into the second and third buffers, idle until the first tile is worked on
+            // the key and value rows into the second (and third) buffers, idle until the first tile is worked on
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < KR / kTileRows; t++) {
                 const int64_t off = hoff - shift + (int64_t)(c00 + t * kTileRows) * ld;
                 tq.load(tm, gp(p.k) + off, S - (c00 + t * kTileRows), Qs + (1 + t) * kTileB);
                 tg.load(tm, gp(p.v) + off, S - (c00 + t * kTileRows), Gs + (1 + t) * kTileB);
             }
-            zero_pads(smem, 2 * kDkvBufs * kTileB / kRowB, (Dh + shift + 7) >> 3);
+            zero_pads(smem, 2 * BUFS * kTileB / kRowB, (Dh + shift + 7) >> 3);
         }
         tile_sync<DMA>();
         if constexpr (DMA) {
-            frags_from_tile<KS>(kf, Qs + (1 + (wid >> 1)) * kTileB, (wid & 1) * 32 + l32, Dh, lh, shift);
-            frags_from_tile<KS>(vf, Gs + (1 + (wid >> 1)) * kTileB, (wid & 1) * 32 + l32, Dh, lh, shift);
+            frags_from_tile<KS>(kf, Qs + (1 + (kb >> 1)) * kTileB, (kb & 1) * 32 + l32, Dh, lh, shift);
+            frags_from_tile<KS>(vf, Gs + (1 + (kb >> 1)) * kTileB, (kb & 1) * 32 + l32, Dh, lh, shift);
             __syncthreads();                      // every wave holds its fragments: the buffers take query tiles now
         }
         // The tiles that hold the diagonal (two: 128 keys) and a ragged last tile run block by block.  The tiles
@@ -1481,10 +1486,10 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
         // matrix unit forms S and dP of block b + 1 and adds block b - 1 to dV and dK.  A wave has its SIMD to
         // itself here, so nothing else would fill the one unit while the other works.
         const int iqB = SPLIT && z > 0 ? iq0 : iq0 + 2, iqE = SPLIT ? min(niq, S / kTileRows) : S / kTileRows;
-        const bool pipe = FAST && DMA && iqE > iqB;
+        const bool pipe = FAST && DMA && KR == 128 && iqE > iqB;
         run_tiles(iq0, pipe ? iqB : niq);
         if (pipe) {
-            if constexpr (FAST && DMA) {
+            if constexpr (FAST && DMA && KR == 128) {
                 const int a4 = (lane >> 2) & 3, b4 = lane & 3, n16 = (lane >> 4) & 1;
                 const int colb = 16 * n16 + 4 * b4;
                 // blocks alternate between two register sets: SP = the S and dP accumulators (formed in one
@@ -1653,17 +1658,40 @@ __global__ void __launch_bounds__(kNT, 1) attn_bwd_dkv_kernel(AttnArgs p)
             }
             return;
         }
-        const bool staged_v = DMA && !p.acc_dv, staged_k = DMA && !p.acc_dk;
+        if constexpr (KR == 64) {
+            // the sums over the second 32 queries of every tile onto those over the first
+            float *x = reinterpret_cast<float *>(smem) + kb * 64 + lane;
+            if (qh == 1) {
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        x[(dt * 16 + r) * 128] = kacc[dt][r];
+                        x[((DT + dt) * 16 + r) * 128] = vacc[dt][r];
+                    }
+            }
+            __syncthreads();
+            if (qh == 0) {
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        kacc[dt][r] += x[(dt * 16 + r) * 128];
+                        vacc[dt][r] += x[((DT + dt) * 16 + r) * 128];
+                    }
+            }
+        }
+        const bool mine = qh == 0, staged_v = DMA && !p.acc_dv, staged_k = DMA && !p.acc_dk;
         if (staged_v || staged_k) {
             __syncthreads();                              // the last products have read their tiles
-            if (staged_k) stage_rows<DT>(Qs, kacc, wid * 32 + l32, lh, p.alpha);
-            if (staged_v) stage_rows<DT>(Gs, vacc, wid * 32 + l32, lh, 1.0f);
+            if (staged_k && mine) stage_rows<DT>(Qs, kacc, kb * 32 + l32, lh, p.alpha);
+            if (staged_v && mine) stage_rows<DT>(Gs, vacc, kb * 32 + l32, lh, 1.0f);
             __syncthreads();
             const int64_t off = (int64_t)c00 * ld + hoff - shift;
-            if (staged_k) write_rows(Qs, p.dk + off, ld, min(kBM, S - c00), Dh, shift, threadIdx.x, kNT);
-            if (staged_v) write_rows(Gs, p.dv + off, ld, min(kBM, S - c00), Dh, shift, threadIdx.x, kNT);
+            if (staged_k) write_rows(Qs, p.dk + off, ld, min(KR, S - c00), Dh, shift, threadIdx.x, kNT);
+            if (staged_v) write_rows(Gs, p.dv + off, ld, min(KR, S - c00), Dh, shift, threadIdx.x, kNT);
         }
-        if (mykey < S && !(staged_v && staged_k)) {
+        if (mine && mykey < S && !(staged_v && staged_k)) {
             half_t *krow = p.dk + (int64_t)mykey * ld + hoff, *vrow = p.dv + (int64_t)mykey * ld + hoff;
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
@@ -1702,9 +1730,9 @@ __global__ void __launch_bounds__(256) attn_bwd_dkv_sum_kernel(AttnArgs p)
 // A workgroup of the dK / dV kernel walks all query tiles from its keys on, 1.4 us each behind some 10 us of start, and
 // a short sequence has few workgroups for it (611 positions of 16 heads: 80 of up to 10 tiles, on 256 CUs).  There the
 // query tiles of 128 keys go to several workgroups, as many as the device has room for, whose fp32 sums a second launch of
-// 4.6 to 6.6 us adds up: worth it from five tiles saved on.  Measured, us, one walk -> parts and their sum: 611 positions,
-// 16 heads of 64, 24.9 -> 15.6 + 4.6; 777 positions, 16 heads of 128, 35.6 -> 24.8 + 6.6; forward and adjoint together: 611 x 16 x 64 67.1 -> 64.6, 449 x 8 x 128
-// 63.8 -> 60.3, 1000 x 4 x 100 94.2 -> 77.6.  split = 1: not.
+// 4.6 to 6.6 us adds up: worth it from five tiles saved on where the alternative is 128 keys and one walk (24.9 -> 15.6 +
+// 4.6 us there), from eight on where it is 64 keys (few_keys).  Forward and adjoint together, one walk -> parts: 1000
+// positions, 4 heads of 100, 94.2 -> 77.6 us.  split = 1: not.
 struct DkvParts {
     int split, per;
 };
@@ -1719,7 +1747,7 @@ DkvParts dkv_parts(int64_t S, int64_t H)
 }
 size_t stats_part_bytes(int64_t S, int64_t H) { return ((size_t)(2 * S * H) * sizeof(float) + 15) / 16 * 16; }
 
-constexpr size_t kDkvSmem = 2 * kDkvBufs * kTileB + kDkvBufs * 4 * 64 * sizeof(float);
+constexpr size_t dkv_smem(int keys) { return (2 * kTileB + 4 * 64 * sizeof(float)) * dkv_bufs(keys); }
 
 template <class K>
 int set_smem(K kern, size_t bytes)
@@ -1740,12 +1768,25 @@ std::atomic<int> g_exact{0};             // cacti_hip_attention_set_exact: launc
 // over the CUs: 128 -> 64 rows, us, forward and adjoint, 611 positions, 16 heads of 64 19.2 -> 16.1 and 42.3 -> 35.4; 777,
 // 16 of 128 26.0 -> 20.7 and 62 -> 53; 1534, 16 of 100 41.3 -> 32.2 and 92 -> 85; 1984, 16 of 128 (496 workgroups) 50.8 ->
 // 46.2 and 115 -> 107; 1422, 24 of 100 (552) 38.4 -> 47.5 and 90 -> 94; 2048, 32 of 100 (1024) 68 -> 95 and 156 -> 168.
-// Exact arithmetic: 1531, 16 of 128 71.8 -> 43.7 and 172 -> 134.  The forward kernel's second round is short only if there
+// Exact arithmetic: 1531, 16 of 128 71.8 -> 43.7 and 172 -> 134.  Up to 128 positions there is a step or two either way.  The forward kernel's second round is short only if there
 // are long sequences in the first: 901, 32 of 100 (480 workgroups) 28.1 -> 29.2, 786 (416) 25.4 -> 25.6.
 int query_rows(int64_t S, int64_t H, bool forward, bool fast)
 {
     const int64_t cus = device_cus(), wgs = (S + 63) / 64 * H;
-    return wgs <= (forward && fast && S <= 1024 ? cus + cus * 3 / 4 : 2 * cus) ? 64 : 128;
+    return S > 128 && wgs <= (forward && fast && S <= 1024 ? cus + cus * 3 / 4 : 2 * cus) ? 64 : 128;
+}
+
+// Whether the dK / dV kernel takes 64 keys per workgroup instead of 128: its workgroups then walk the same query tiles with
+// half of the work in each (two waves to 32 keys), but without the in-wave pipeline.  Adjoint with 128 -> 64 keys, us: 611
+// positions, 16 heads of 64 37.3 -> 32.2; 777, 16 of 128 53 -> 47; 1531, 16 of 128 (384 workgroups) 86 -> 75; 2048, 16 of 128
+// (512) 113 -> 108; 1051, 32 of 100 (544) 80 -> 87.  Heads to 64 leave registers for two workgroups per CU: 2048, 16 of 64
+// 94 -> 78; 2048, 32 of 64 (1024) 125 -> 117.  Against parts of the query tiles it is the better one unless a part is more
+// than 7 tiles shorter than the walk: 449, 8 of 64 (6 shorter) 28.5 -> 27.7, 611, 4 of 64 (8) 27.8 -> 29.2, 1000, 4 of 100
+// (14) 44.6 -> 52.
+bool few_keys(const AttnArgs &p, bool narrow)
+{
+    const int64_t tiles = (p.S + kTileRows - 1) / kTileRows;
+    return p.S > 128 && tiles * p.H <= (narrow ? 4 : 2) * (int64_t)device_cus() && !(p.split > 1 && tiles - p.per > 7);
 }
 
 template <int KS, int DT, bool FAST, bool DMA>
@@ -1777,9 +1818,11 @@ int launch_bwd(const AttnArgs &p, hipStream_t st)
         if (rc) return rc;
         if constexpr (DMA)
             if ((rc = set_smem(attn_bwd_dq_kernel<KS, DT, FAST, DMA, 64>, kQmSmem))) return rc;
-        if ((rc = set_smem(attn_bwd_dkv_kernel<KS, DT, FAST, DMA, false>, kDkvSmem))) return rc;
+        if ((rc = set_smem(attn_bwd_dkv_kernel<KS, DT, FAST, DMA, false, 128>, dkv_smem(128)))) return rc;
+        if constexpr (DMA)
+            if ((rc = set_smem(attn_bwd_dkv_kernel<KS, DT, FAST, DMA, false, 64>, dkv_smem(64)))) return rc;
         if constexpr (PARTS)
-            if ((rc = set_smem(attn_bwd_dkv_kernel<KS, DT, FAST, DMA, true>, kDkvSmem))) return rc;
+            if ((rc = set_smem(attn_bwd_dkv_kernel<KS, DT, FAST, DMA, true, 128>, dkv_smem(128)))) return rc;
         ready.mark();
     }
     const int nqt = (p.S + kBM - 1) / kBM;
@@ -1790,15 +1833,21 @@ int launch_bwd(const AttnArgs &p, hipStream_t st)
     if (rows == 128) hipLaunchKernelGGL((attn_bwd_dq_kernel<KS, DT, FAST, DMA, 128>), grid, dim3(kNT2), kQmSmem, st, p);
     int rc = launch_status("attention_bwd_dq");
     if (rc) return rc;
+    if constexpr (DMA)
+        if (few_keys(p, KS == 4)) {
+            hipLaunchKernelGGL((attn_bwd_dkv_kernel<KS, DT, FAST, DMA, false, 64>), dim3((unsigned)((p.S + 63) / 64 * p.H)), dim3(kNT),
+                               dkv_smem(64), st, p);
+            return launch_status("attention_bwd_dkv");
+        }
     if constexpr (PARTS)
         if (p.split > 1) {
-            hipLaunchKernelGGL((attn_bwd_dkv_kernel<KS, DT, FAST, DMA, true>), dim3((unsigned)(nqt * p.split * p.H)), dim3(kNT),
-                               kDkvSmem, st, p);
+            hipLaunchKernelGGL((attn_bwd_dkv_kernel<KS, DT, FAST, DMA, true, 128>), dim3((unsigned)(nqt * p.split * p.H)), dim3(kNT),
+                               dkv_smem(128), st, p);
             const int64_t lanes = (int64_t)p.H * p.S * (p.Dh / 4);
             hipLaunchKernelGGL(attn_bwd_dkv_sum_kernel, dim3((unsigned)((lanes + 255) / 256), 2), dim3(256), 0, st, p);
             return launch_status("attention_bwd_dkv");
         }
-    hipLaunchKernelGGL((attn_bwd_dkv_kernel<KS, DT, FAST, DMA, false>), dim3((unsigned)(nqt * p.H)), dim3(kNT), kDkvSmem, st, p);
+    hipLaunchKernelGGL((attn_bwd_dkv_kernel<KS, DT, FAST, DMA, false, 128>), dim3((unsigned)(nqt * p.H)), dim3(kNT), dkv_smem(128), st, p);
     return launch_status("attention_bwd_dkv");
 }
 
