@@ -1189,56 +1189,67 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
                     tk.load(tm, K + (int64_t)(jt + 2) * kTileRows * ld, S - (jt + 2) * kTileRows, Ks + (cur ^ 1) * kTileB);
                     tv.load(tm, V + (int64_t)(jt + 2) * kTileRows * ld, S - (jt + 2) * kTileRows, Vs + (cur ^ 1) * kTileB);
                 }
-                if (jt < njt) {
-#pragma unroll
-                    for (int k2 = 0; k2 < 2 / KP; k2++) {
-                        const int kt = KP == 1 ? k2 : ws.kp, kb = jt * kTileRows + 32 * kt;
-                        if (kb > r0 + 31) continue;
-                        const float16_t sacc = prod_direct<KS>(Ks + cur * kTileB, 32 * kt, qf, l32, lh);
-                        const float16_t pacc = prod_direct<KS>(Vs + cur * kTileB, 32 * kt, gf, l32, lh);
-                        const bool full = kb + 31 <= r0;
-                        float de[16];
-                        if constexpr (FAST) {
-                            // sigma and dS with the f16 value of dP read by the fused multiply-add
-                            half_t dph[16];
-                            round16(dph, pacc);
-                            if (full) {
-#pragma unroll
-                                for (int e = 0; e < 16; e++) {
-                                    const float pr_ = exp2_mix(f2h(scaled(p.alpha, sacc[e])), cs);
-                                    const half_t dp = dph[e];
-                                    if (PASS == 0) part = __builtin_fmaf((float)dp, pr_, part);
-                                    else de[e] = __builtin_fmaf((float)dp, pr_, -(sig * pr_));
-                                }
-                            } else {
-#pragma unroll
-                                for (int e = 0; e < 16; e++) {
-                                    const bool live = kb + 8 * (e >> 2) + 4 * lh + (e & 3) <= myrow;
-                                    const float pr_ = exp2_mix(f2h(scaled(p.alpha, sacc[e])), cs);
-                                    const half_t dp = dph[e];
-                                    if (PASS == 0) part += live ? (float)dp * pr_ : 0.f;
-                                    else de[e] = live ? __builtin_fmaf((float)dp, pr_, -(sig * pr_)) : 0.f;
-                                }
-                            }
-                        } else if (full) {
+                // 32 keys of the tile
+                auto block = [&](int kt) __attribute__((always_inline)) {
+                    const int kb = jt * kTileRows + 32 * kt;
+                    if (kb > r0 + 31) return;
+                    const float16_t sacc = prod_direct<KS>(Ks + cur * kTileB, 32 * kt, qf, l32, lh);
+                    const float16_t pacc = prod_direct<KS>(Vs + cur * kTileB, 32 * kt, gf, l32, lh);
+                    const bool full = kb + 31 <= r0;
+                    float de[16];
+                    if constexpr (FAST) {
+                        // sigma and dS with the f16 value of dP read by the fused multiply-add
+                        half_t dph[16];
+                        round16(dph, pacc);
+                        if (full) {
 #pragma unroll
                             for (int e = 0; e < 16; e++) {
-                                const float pr_ = M::prob(rnd16(scaled(p.alpha, sacc[e])), m, l, y);
-                                const float tt = pr_ * rnd16(pacc[e]);
-                                if (PASS == 0) part += tt;
-                                else de[e] = tt - sig * pr_;
+                                const float pr_ = exp2_mix(f2h(scaled(p.alpha, sacc[e])), cs);
+                                const half_t dp = dph[e];
+                                if (PASS == 0) part = __builtin_fmaf((float)dp, pr_, part);
+                                else de[e] = __builtin_fmaf((float)dp, pr_, -(sig * pr_));
                             }
                         } else {
 #pragma unroll
                             for (int e = 0; e < 16; e++) {
                                 const bool live = kb + 8 * (e >> 2) + 4 * lh + (e & 3) <= myrow;
-                                const float pr_ = M::prob(rnd16(scaled(p.alpha, sacc[e])), m, l, y);
-                                const float tt = pr_ * rnd16(pacc[e]);
-                                if (PASS == 0) part += live ? tt : 0.f;
-                                else de[e] = live ? tt - sig * pr_ : 0.f;
+                                const float pr_ = exp2_mix(f2h(scaled(p.alpha, sacc[e])), cs);
+                                const half_t dp = dph[e];
+                                if (PASS == 0) part += live ? (float)dp * pr_ : 0.f;
+                                else de[e] = live ? __builtin_fmaf((float)dp, pr_, -(sig * pr_)) : 0.f;
                             }
                         }
-                        if (PASS == 1) prod_tr<DT>(dacc, Ks + cur * kTileB, 32 * kt, pack8(de), pack8(de + 8), lane);
+                    } else if (full) {
+#pragma unroll
+                        for (int e = 0; e < 16; e++) {
+                            const float pr_ = M::prob(rnd16(scaled(p.alpha, sacc[e])), m, l, y);
+                            const float tt = pr_ * rnd16(pacc[e]);
+                            if (PASS == 0) part += tt;
+                            else de[e] = tt - sig * pr_;
+                        }
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 16; e++) {
+                            const bool live = kb + 8 * (e >> 2) + 4 * lh + (e & 3) <= myrow;
+                            const float pr_ = M::prob(rnd16(scaled(p.alpha, sacc[e])), m, l, y);
+                            const float tt = pr_ * rnd16(pacc[e]);
+                            if (PASS == 0) part += live ? tt : 0.f;
+                            else de[e] = live ? tt - sig * pr_ : 0.f;
+                        }
+                    }
+                    if (PASS == 1) prod_tr<DT>(dacc, Ks + cur * kTileB, 32 * kt, pack8(de), pack8(de + 8), lane);
+                };
+                if (jt < njt) {
+                    if constexpr (KP == 2) {
+                        block(ws.kp);
+                    } else if constexpr (PASS == 0) {
+                        // one piece of code for both: only the first workgroup of a head runs this pass, and meets every
+                        // instruction of it once
+#pragma unroll 1
+                        for (int kt = 0; kt < 2; kt++) block(kt);
+                    } else {
+#pragma unroll
+                        for (int kt = 0; kt < 2; kt++) block(kt);
                     }
                 }
                 if (nxt) {
