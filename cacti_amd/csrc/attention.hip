@@ -1739,11 +1739,11 @@ __global__ void __launch_bounds__(256) attn_bwd_dkv_sum_kernel(AttnArgs p)
 }
 
 // A workgroup of the dK / dV kernel walks all query tiles from its keys on, 1.4 us each behind some 10 us of start, and
-// a short sequence has few workgroups for it (611 positions of 16 heads: 80 of up to 10 tiles, on 256 CUs).  There the
+// a short sequence has few workgroups for it (1000 positions of 4 heads: 32 of up to 16 tiles, on 256 CUs).  There the
 // query tiles of 128 keys go to several workgroups, as many as the device has room for, whose fp32 sums a second launch of
-// 4.6 to 6.6 us adds up: worth it from five tiles saved on where the alternative is 128 keys and one walk (24.9 -> 15.6 +
-// 4.6 us there), from eight on where it is 64 keys (few_keys).  Forward and adjoint together, one walk -> parts: 1000
-// positions, 4 heads of 100, 94.2 -> 77.6 us.  split = 1: not.
+// 4.6 to 6.6 us adds up.  What it is weighed against is one walk with 64 keys (few_keys: half the work per tile), so a part
+// has to be at least 8 tiles shorter than the walk.  Adjoint with 64 keys -> parts, us: 449 positions, 8 heads of 64 (6
+// tiles shorter) 27.7 -> 28.5; 611, 4 of 64 (8) 29.2 -> 27.8; 1000, 4 of 100 (14) 52 -> 44.6.  split = 1: not.
 struct DkvParts {
     int split, per;
 };
@@ -1753,7 +1753,7 @@ DkvParts dkv_parts(int64_t S, int64_t H)
     int64_t split = std::min<int64_t>(device_cus() / groups, 8);
     if (split < 2) return {1, (int)tiles};
     const int64_t per = std::max<int64_t>(2, (tiles + split - 1) / split);
-    if (tiles - per < 5) return {1, (int)tiles};
+    if (tiles - per < 8) return {1, (int)tiles};
     return {(int)((tiles + per - 1) / per), (int)per};
 }
 size_t stats_part_bytes(int64_t S, int64_t H) { return ((size_t)(2 * S * H) * sizeof(float) + 15) / 16 * 16; }
@@ -1791,13 +1791,11 @@ int query_rows(int64_t S, int64_t H, bool forward, bool fast)
 // half of the work in each (two waves to 32 keys), but without the in-wave pipeline.  Adjoint with 128 -> 64 keys, us: 611
 // positions, 16 heads of 64 37.3 -> 32.2; 777, 16 of 128 53 -> 47; 1531, 16 of 128 (384 workgroups) 86 -> 75; 2048, 16 of 128
 // (512) 113 -> 108; 1051, 32 of 100 (544) 80 -> 87.  Heads to 64 leave registers for two workgroups per CU: 2048, 16 of 64
-// 94 -> 78; 2048, 32 of 64 (1024) 125 -> 117.  Against parts of the query tiles it is the better one unless a part is more
-// than 7 tiles shorter than the walk: 449, 8 of 64 (6 shorter) 28.5 -> 27.7, 611, 4 of 64 (8) 27.8 -> 29.2, 1000, 4 of 100
-// (14) 44.6 -> 52.
+// 94 -> 78; 2048, 32 of 64 (1024) 125 -> 117.  Parts of the query tiles, where there are any, are better (dkv_parts).
 bool few_keys(const AttnArgs &p, bool narrow)
 {
     const int64_t tiles = (p.S + kTileRows - 1) / kTileRows;
-    return p.S > 128 && tiles * p.H <= (narrow ? 4 : 2) * (int64_t)device_cus() && !(p.split > 1 && tiles - p.per > 7);
+    return p.S > 128 && tiles * p.H <= (narrow ? 4 : 2) * (int64_t)device_cus() && p.split < 2;
 }
 
 template <int KS, int DT, bool FAST, bool DMA>
