@@ -1743,20 +1743,25 @@ __global__ void __launch_bounds__(256) attn_bwd_dkv_sum_kernel(AttnArgs p)
 // query tiles of 128 keys go to several workgroups, as many as the device has room for, whose fp32 sums a second launch of
 // 4.6 to 6.6 us adds up.  What it is weighed against is one walk with 64 keys (few_keys: half the work per tile), so a part
 // has to be at least 8 tiles shorter than the walk.  Adjoint with 64 keys -> parts, us: 449 positions, 8 heads of 64 (6
-// tiles shorter) 27.7 -> 28.5; 611, 4 of 64 (8) 29.2 -> 27.8; 1000, 4 of 100 (14) 52 -> 44.6.  split = 1: not.
+// tiles shorter) 27.7 -> 28.5; 611, 4 of 64 (8) 29.2 -> 27.8; 1000, 4 of 100 (14) 52 -> 44.6.  split = 1: not.  The exact
+// arithmetic has no parts, and is better with 64 keys than with 128 everywhere there (1000, 4 of 100: 91.5 -> 72.4 us).
 struct DkvParts {
     int split, per;
 };
-DkvParts dkv_parts(int64_t S, int64_t H)
+DkvParts dkv_parts(int64_t S, int64_t H, bool exact)
 {
     const int64_t groups = (S + kBM - 1) / kBM * H, tiles = (S + kTileRows - 1) / kTileRows;
     int64_t split = std::min<int64_t>(device_cus() / groups, 8);
-    if (split < 2) return {1, (int)tiles};
+    if (exact || split < 2) return {1, (int)tiles};
     const int64_t per = std::max<int64_t>(2, (tiles + split - 1) / split);
     if (tiles - per < 8) return {1, (int)tiles};
     return {(int)((tiles + per - 1) / per), (int)per};
 }
 size_t stats_part_bytes(int64_t S, int64_t H) { return ((size_t)(2 * S * H) * sizeof(float) + 15) / 16 * 16; }
+size_t parts_bytes(const DkvParts &parts, int64_t S, int64_t H, int64_t Dh)
+{
+    return (size_t)parts.split * 2 * (size_t)H * (size_t)S * (size_t)Dh * sizeof(float);
+}
 
 constexpr size_t dkv_smem(int keys) { return (2 * kTileB + 4 * 64 * sizeof(float)) * dkv_bufs(keys); }
 
@@ -1970,9 +1975,9 @@ int attention_fwd_exact(int64_t S, int64_t H, int64_t Dh, float alpha, const voi
 CACTI_API size_t cacti_hip_attention_bwd_workspace_best(int64_t S, int64_t H, int64_t Dh)
 {
     if (S <= 0 || H <= 0 || Dh <= 0 || Dh > kDP) return cacti_hip_attention_bwd_workspace(S, H);
-    const DkvParts parts = dkv_parts(S, H);
+    const DkvParts parts = dkv_parts(S, H, g_exact.load(std::memory_order_relaxed) != 0);
     if (parts.split < 2) return cacti_hip_attention_bwd_workspace(S, H);
-    return stats_part_bytes(S, H) + (size_t)parts.split * 2 * (size_t)H * (size_t)S * (size_t)Dh * sizeof(float);
+    return stats_part_bytes(S, H) + parts_bytes(parts, S, H, Dh);
 }
 
 CACTI_API int cacti_hip_attention_bwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,
@@ -2001,8 +2006,9 @@ CACTI_API int cacti_hip_attention_bwd(int64_t S, int64_t H, int64_t Dh, float al
     p.l = p.m + S * H;
     p.y = (float *)workspace;
     p.sig = p.y + S * H;
-    const DkvParts parts = dkv_parts(S, H);
-    if (parts.split > 1 && aligned(workspace, 16) && workspace_bytes >= cacti_hip_attention_bwd_workspace_best(S, H, Dh)) {
+    const bool exact = g_exact.load(std::memory_order_relaxed) != 0;
+    const DkvParts parts = dkv_parts(S, H, exact);
+    if (parts.split > 1 && aligned(workspace, 16) && workspace_bytes >= stats_part_bytes(S, H) + parts_bytes(parts, S, H, Dh)) {
         p.split = parts.split;
         p.per = parts.per;
         p.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + stats_part_bytes(S, H));
@@ -2010,5 +2016,5 @@ CACTI_API int cacti_hip_attention_bwd(int64_t S, int64_t H, int64_t Dh, float al
     hipStream_t st = (hipStream_t)stream;
     int64_t span;
     const bool dma = direct_tiles(H, Dh, ld, {q, k, v, dO, o, dq, dk, dv}, &span);     // o may be null: passes
-    return dispatch<Bwd>(span, g_exact.load(std::memory_order_relaxed) != 0, dma, p, st);
+    return dispatch<Bwd>(span, exact, dma, p, st);
 }

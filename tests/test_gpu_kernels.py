@@ -829,6 +829,36 @@ def test_attention_bwd_in_parts(ops, S, H, Dh, acc):
         assert rel_l2(host(a), host(b)) < 2e-4 and exact_frac(host(a), host(b)) > 0.95
 
 
+@pytest.mark.parametrize("S,H,Dh", [(577, 2, 128), (1000, 4, 100), (705, 4, 64)])
+def test_attention_bwd_exact_has_no_parts(ops, S, H, Dh):
+    """The exact arithmetic asks for no scratch for parts and takes the same kernels whatever the workspace: the same bits
+    with the least one and with one that the default arithmetic has parts in."""
+    from cacti_amd import ffi
+    best = ffi.lib().cacti_hip_attention_bwd_workspace_best(S, H, Dh)
+    least = ffi.lib().cacti_hip_attention_bwd_workspace(S, H)
+    assert best > least
+    say("attention_bwd, exact", S, H, Dh)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(S + H + Dh)
+    q, k, v, dO = (torch.randn(S, H, Dh, generator=g, device="cuda").half() for _ in range(4))
+    alpha, st = Dh ** -0.5, torch.cuda.current_stream().cuda_stream
+    ffi.call("cacti_hip_attention_set_exact", 1)
+    try:
+        o, stats = ops.attention_fwd(q, k, v, alpha)
+        assert ffi.lib().cacti_hip_attention_bwd_workspace_best(S, H, Dh) == least
+        got = []
+        for size in (least, best):
+            ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+            d = [torch.empty_like(q) for _ in range(3)]
+            ffi.call("cacti_hip_attention_bwd", S, H, Dh, alpha, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dO.data_ptr(),
+                     H * Dh, stats.data_ptr(), d[0].data_ptr(), 0, d[1].data_ptr(), 0, d[2].data_ptr(), 0, ws.data_ptr(), size, st)
+            got.append([host(t) for t in d])
+    finally:
+        ffi.call("cacti_hip_attention_set_exact", 0)
+    for name, a, b in zip(("dq", "dk", "dv"), *got):
+        assert_bits(a, b, name)
+
+
 @pytest.mark.parametrize("S,H,Dh", [(577, 2, 128), (576, 2, 128), (611, 16, 64), (777, 16, 128), (449, 3, 100), (1000, 2, 128),
                                     (1025, 8, 100), (2048, 32, 100), (128, 4, 64)])
 def test_attention_bwd_parts_fill_this_device(S, H, Dh):
