@@ -859,6 +859,20 @@ def test_attention_bwd_exact_has_no_parts(ops, S, H, Dh):
         assert_bits(a, b, name)
 
 
+def test_attention_bwd_scratch_of_rows_without_parts(ops):
+    """1000 positions of 3 heads of 100: rows of 300 elements, which no kernel with parts takes; the operator allocates its
+    results and the least workspace (each rounded up by the allocator), not 19 MB of fp32 planes."""
+    S, H, Dh = 1000, 3, 100
+    q, k, v, dO = (torch.randn(S, H, Dh, device="cuda").half() for _ in range(4))
+    o, stats = ops.attention_fwd(q, k, v, 0.1)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    ops.attention_bwd(q, k, v, dO, stats, 0.1, o=o)
+    taken, room = torch.cuda.max_memory_allocated() - before, 3 * q.nbytes + 8 * S * H + 4 * 512
+    assert taken <= room
+
+
 @pytest.mark.parametrize("S,H,Dh", [(577, 2, 128), (576, 2, 128), (611, 16, 64), (777, 16, 128), (449, 3, 100), (1000, 2, 128),
                                     (1025, 8, 100), (2048, 32, 100), (128, 4, 64)])
 def test_attention_bwd_parts_fill_this_device(S, H, Dh):
