@@ -30,10 +30,13 @@ constexpr size_t kWindowBytes = Staging::kFlagBytes + (16u << 20);   // of a lar
 // n <= kMaxRegions regions, in one launch on `st`, to places in s.data(); returns when they are there.  The launch comes
 // behind all work queued on `st`, so this waits for it like a stream synchronisation.
 int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st);
-// one region of any size to pageable memory, likewise, and (not null) a word of device memory with it; readers on other
-// threads and streams go on meanwhile
-int read_large(void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st);
+// one region of any size to pageable memory, likewise, and (not null) a word of device memory with it: up to kOwnRead bytes
+// through `own`, the caller's, which no other reader waits for or takes; beyond through a borrowed window.  Readers on
+// other threads and streams go on meanwhile.
+int read_large(Staging &own, void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st);
 constexpr size_t kLargeRead = 192u << 10;      // from here on it is the better one
+constexpr size_t kOwnRead = 512u << 10;
+static_assert(kOwnRead <= kStagingBytes - Staging::kFlagBytes, "a context's buffer holds it");
 // n regions of `bytes` (a multiple of 16), 16-byte aligned, set to zero
 int zero_regions(void *const *ptrs, int n, size_t bytes, hipStream_t st);
 

@@ -125,8 +125,8 @@ int wait_flags(const unsigned *flags, int n, unsigned epoch, hipStream_t st)
 }
 
 // Buffers nobody uses at the moment, by size: at most 4 of a context's, for the next contexts, 16 of a word's, one for
-// every thread that reads at the same time, and two windows of large reads (a third reader at the same time page-locks
-// its own and frees it again).
+// every thread that reads at the same time, and two windows of reads above kOwnRead (a third such reader at the same time
+// page-locks its own and frees it again).
 struct Kept {
     size_t bytes;
     int most, n;
@@ -175,9 +175,11 @@ void settle(Staging &s, hipStream_t st)
     s.lost = true;
 }
 
-// a large read's buffer: 64 bytes for the word, then the flags, then the window of chunks
-constexpr size_t kWindow = kWindowBytes - Staging::kFlagBytes, kLeastChunk = 32u << 10;
-static_assert(64 + kWindow / kLeastChunk * sizeof(unsigned) <= Staging::kFlagBytes, "a word per chunk");
+// a large read's buffer: a word per chunk, at the end of their place the word that is read with it (a gather's words, in the
+// same buffer, do not reach there), then the window of chunks
+constexpr size_t kWindow = kWindowBytes - Staging::kFlagBytes, kLeastChunk = 32u << 10, kWordPlace = Staging::kFlagBytes - 64;
+static_assert(kWindow / kLeastChunk * sizeof(unsigned) <= kWordPlace && kFlagsPerGather * sizeof(unsigned) <= kWordPlace,
+              "a word per chunk");
 constexpr int kStreamBlocks = 16;
 
 }  // namespace
@@ -197,13 +199,13 @@ int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st)
 
 static int read_windows(Staging &s, void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st)
 {
-    int *const word_here = reinterpret_cast<int *>(s.base);
-    unsigned *const flags = reinterpret_cast<unsigned *>(s.base + 64);
+    int *const word_here = reinterpret_cast<int *>(s.base + kWordPlace);
+    unsigned *const flags = reinterpret_cast<unsigned *>(s.base);
     char *const data = s.data();
     int dev = 0;
     CACTI_HIP(hipGetDevice(&dev));
     for (size_t done = 0; done < bytes;) {
-        const size_t window = std::min(bytes - done, kWindow), chunk = window < (4u << 20) ? kLeastChunk : 2 * kLeastChunk;
+        const size_t window = std::min(bytes - done, s.room()), chunk = window < (4u << 20) ? kLeastChunk : 2 * kLeastChunk;
         const int chunks = (int)((window + chunk - 1) / chunk), threads = (int)std::min<size_t>(kCopyThreads, 1 + window / (4u << 20));
         if (++s.epoch == 0) s.epoch = 1;
         const unsigned epoch = s.epoch;
@@ -230,8 +232,9 @@ static int read_windows(Staging &s, void *dst, const void *src, size_t bytes, co
 // helper thread costs some 10 us to start: worth it from several MiB on, where the copying host (12 .. 30 GB/s) and not
 // the link (52) is what one thread would wait for.  One gather and one copy behind it against chunks, since the chunks are
 // announced without a fence: 128 KiB 15.3 and 15.7, 344 KiB 24.4 and 22.3, 512 KiB 30.2 and 29.6.
-int read_large(void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st)
+int read_large(Staging &own, void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st)
 {
+    if (own.base && !own.lost && bytes <= kOwnRead) return read_windows(own, dst, src, bytes, word, word_dst, st);
     Staging s;
     if (!staging_take(&s, kWindowBytes)) {
         CACTI_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));

@@ -255,7 +255,7 @@ int Ctx::fetch(const Fetch *f, int n)
             r[m++] = {f[i].src, staging_.data() + used, f[i].bytes};
             used += room;
         } else {
-            const int rc = read_large(f[i].dst, f[i].src, f[i].bytes, static_cast<int *>(status_ptr()), &status, stream_);
+            const int rc = read_large(staging_, f[i].dst, f[i].src, f[i].bytes, static_cast<int *>(status_ptr()), &status, stream_);
             if (rc) return rc;
             have_status = true;
         }
@@ -396,7 +396,7 @@ int Ctx::cell_get(CellPtr ci, void *host, size_t bytes)
             rc = gather_to_host(staging_, &r, 1, stream_);
             if (!rc) memcpy(host, staging_.data(), bytes);
         } else {
-            rc = read_large(host, dev_ptr(c.voff), bytes, nullptr, nullptr, stream_);
+            rc = read_large(staging_, host, dev_ptr(c.voff), bytes, nullptr, nullptr, stream_);
         }
         if (rc) return rc;
         bytes_d2h_ += bytes;

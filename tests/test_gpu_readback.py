@@ -116,6 +116,57 @@ def test_a_large_read_does_not_wait_for_another_contexts_stream():
     assert "first: True" in child("from tests.test_gpu_readback import concurrent_reads; concurrent_reads()")
 
 
+def test_reads_of_some_hundred_kb_at_once_page_lock_nothing():
+    """Three contexts read a gradient of 300 KB at the same time, each waiting for what is queued on its own stream: each
+    goes through the buffer its context has anyway."""
+    from cacti_amd import ffi
+    contexts = [model(V=600, pagelocked=False) for _ in range(3)]
+    i = [n for n, _ in contexts[0][1].params].index("lm_head")
+    want = contexts[0][1].grad(i)
+    assert 192 << 10 < want.nbytes < 512 << 10
+    got = [None] * 3
+
+    def read(j):
+        got[j] = contexts[j][1].grad(i)
+
+    torch.cuda.synchronize()
+    before = pinned()
+    for ctx, _ in contexts:
+        busy(ffi.lib().cacti_ctx_stream(ctx._c), 400.0)
+    threads = [threading.Thread(target=read, args=(j,)) for j in range(3)]
+    for t in threads:
+        t.start()
+    threads[0].join(0.1)                                   # all three are inside their reads by now
+    during = pinned()
+    for t in threads:
+        t.join()
+    for g in got:
+        assert np.array_equal(g, want)
+    assert during[0] == pinned()[0] == before[0]
+    for ctx, m in contexts:
+        m.close(); ctx.close()
+
+
+def test_a_context_reads_large_and_small_through_one_buffer():
+    """Reads in chunks (300 KB, with the status word behind it) and in one gather, in turn: the words that announce them
+    share their place in the context's buffer."""
+    ctx, m = model(V=600)
+    names = [n for n, _ in m.params]
+    big, small = names.index("lm_head"), names.index("head_norm")
+    want = None
+    r = np.random.default_rng(4)
+    tok = r.integers(0, 600, SMALL["S"]).astype(np.uint16)
+    for _ in range(40):
+        m.step(tok, tok, np.full(SMALL["S"], 8.0, np.float32))
+        now = m.grad(big), m.grad(small)
+        want = want or now
+        for _ in range(3):
+            again = m.grad(small), m.grad(big)
+            assert np.array_equal(again[0], now[1]) and np.array_equal(again[1], now[0])
+        assert np.array_equal(now[0], want[0]) and np.array_equal(now[1], want[1])
+    m.close(); ctx.close()
+
+
 @pytest.mark.parametrize("V,D", [(20000, 1024), (8200, 1032), (24, 264)])
 def test_reads_of_several_windows_come_back_whole(V, D):
     """41 MB in three windows of 16 MiB; 16.9 MB, a window and a few pieces, the last of them short; 13 KB in one gather.
