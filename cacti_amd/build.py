@@ -3,10 +3,14 @@
     python -m cacti_amd.build            # compile every source and link
 """
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
+import tempfile
 from concurrent.futures import ThreadPoolExecutor
+
+from cacti_amd import asm_check
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -21,6 +25,9 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function", "-Wno-unused-value", "-Wno-unused-result", "-Wno-unknown-warning-option",
 ]
+# Sources with matrix instructions or loads into LDS in inline assembly: what the compiler made of them is checked.  In
+# gemm_direct.hip, whose kernels hold all of a wave's registers, a spill and a product rounded only once are faults too.
+CHECKED = ("attention.hip", "gemm_direct.hip", "gemm_mfma.hip")
 
 
 def sources():
@@ -28,9 +35,25 @@ def sources():
 
 
 def _compile(src):
-    obj = os.path.join(OUT_DIR, os.path.splitext(src)[0] + ".o")
+    name = os.path.splitext(src)[0]
+    obj = os.path.join(OUT_DIR, name + ".o")
+    if src not in CHECKED:
+        _hipcc(src, obj)
+        return obj
+    with tempfile.TemporaryDirectory() as tmp:
+        made = os.path.join(tmp, name + ".o")
+        _hipcc(src, made, "--save-temps=obj")
+        with open(os.path.join(tmp, name + "-hip-amdgcn-amd-amdhsa-gfx950.s")) as f:
+            faults = asm_check.check(f.read(), spills=src == "gemm_direct.hip", fused=src == "gemm_direct.hip")
+        if faults:
+            raise RuntimeError("%s: %d faults around inline assembly\n%s" % (src, len(faults), "\n".join(faults[:20])))
+        shutil.move(made, obj)
+    return obj
+
+
+def _hipcc(src, obj, *more):
     cmd = [HIPCC] + FLAGS + (["-x", "hip"] if src.endswith(".cpp") else []) + \
-          ["-c", os.path.join(CSRC, src), "-o", obj]
+          ["-c", os.path.join(CSRC, src), "-o", obj] + list(more)
     p = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     out = "\n".join(l for l in p.stdout.splitlines()
                     if "is not a recognized feature for this target" not in l)
@@ -38,7 +61,6 @@ def _compile(src):
         raise RuntimeError("hipcc failed on %s:\n%s" % (src, out))
     if out.strip():
         sys.stderr.write(out + "\n")
-    return obj
 
 
 def build(jobs=4):

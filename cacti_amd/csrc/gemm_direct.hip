@@ -19,6 +19,8 @@
 // a burst of loads off (all 16 loads of a wave and k tile behind its barrier: 1.70 us per k tile of 256 x 256, spread over
 // the k tile's products: 1.00).  So the products are inline assembly with their operands' register classes named, and the
 // order in the source is the order in the binary: between any two products stand at most one load and one fragment read.
+// The compiler counts no wait states from or to inline assembly: the build checks in its assembly that no accumulator is
+// touched before its product is through, that no operand comes too late, and that nothing is spilled (asm_check.py).
 //
 // The k loop.  A k tile is two k steps of 32, its fragments two sets of registers: while the products of one step run, the
 // fragments of the next are read.  One barrier per k tile, between its two steps: behind it every wave holds the tile's
@@ -274,7 +276,7 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
         for (int m = 0; m < NM; m++) {
             const int d = N > 0 && (m + 1) * N / NM > m * N / NM ? m * N / NM : -1;
             if (d >= 0) {
-                const uint32_t off = IS_A ? la.off[d < NLA ? d : 0] : lb.off[d < NLB ? d : 0];
+                const uint32_t off = IS_A ? la.off[d > 0 && d < NLA ? d : 0] : lb.off[d > 0 && d < NLB ? d : 0];
                 if constexpr (M32)
                     asm volatile("s_add_u32 m0, %5, %6\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %3, %4"
                                  : "+a"(c32)
