@@ -164,7 +164,7 @@ typedef int int4_t __attribute__((ext_vector_type(4)));
 typedef int int4_any __attribute__((ext_vector_type(4), aligned(2)));
 
 // the 8 halves of v moved down by s places (s >= 0), zeros behind them
-__device__ __forceinline__ int4_t halves_down(const int4_t &v, int s)
+__device__ __forceinline__ int4_t halves_down(int4_t v, int s)
 {
     typedef unsigned long long u64;
     const u64 lo = (u64)(uint32_t)v.y << 32 | (uint32_t)v.x, hi = (u64)(uint32_t)v.w << 32 | (uint32_t)v.z;
