@@ -127,10 +127,13 @@ def gemm_plan(M, N, K):
 
 def kernel_symbol(label):
     """Name of the HIP kernel instantiation a dense GEMM label runs on (its first launch), as
-    rocprofv3 prints it, for 16-byte aligned operands (tiles of 64 columns run two workgroups to a CU)."""
+    rocprofv3 prints it, for 16-byte aligned operands."""
+    import ctypes as C
+    from cacti_amd import ffi
     ta, tb, H, M, N, K = gemm_dims(label)
-    bm, bn = gemm_plan(M, N, K)[0]
-    return "gemm_direct_kernel<%s, %s, %d, %d, %d, false, false>" % (str(ta).lower(), str(tb).lower(), bm, bn, 2 if bn == 64 or (bm, bn) == (64, 128) else 1)
+    name = C.create_string_buffer(128)
+    ffi.call("cacti_hip_gemm_kernel_name", int(ta), int(tb), M, N, K, 1, name, len(name))
+    return name.value.decode()
 
 
 def is_split(label):

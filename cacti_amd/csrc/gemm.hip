@@ -427,6 +427,14 @@ CACTI_API int cacti_hip_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, i
     return 0;
 }
 
+CACTI_API int cacti_hip_gemm_kernel_name(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t nz, char *name, size_t bytes)
+{
+    CACTI_REQUIRE(name && M > 0 && N > 0 && K > 0 && nz > 0, CACTI_E_INVALID, "gemm_kernel_name: bad argument");
+    const int n = gemm_kernel_name(ta, tb, gemm_plan(M, N, K, nz, false), name, bytes);
+    CACTI_REQUIRE(n >= 0 && (size_t)n < bytes, CACTI_E_INVALID, "gemm_kernel_name: %zu bytes are too few for the name", bytes);
+    return 0;
+}
+
 // Pointer-array batch (cublasGemmBatchedEx shape): the products must have one shape; up to
 // kMaxPtrBatch of them share a launch when every operand is 16-byte aligned, otherwise they run
 // one after another.

@@ -41,6 +41,8 @@
 #include "gemm_internal.h"
 #include "gemm_tile.h"
 
+#include <stdio.h>
+
 #include <algorithm>
 #include <type_traits>
 #include <utility>
@@ -775,6 +777,14 @@ void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn)
     const Shape &s = kShapes[tile == T64_SMALL ? T64 : tile];
     *bm = s.bm;
     *bn = s.bn;
+}
+
+int gemm_kernel_name(int ta, int tb, const GemmPlan &plan, char *name, size_t bytes)
+{
+    const bool small = plan.tile == T64_SMALL;
+    const Shape &s = kShapes[small ? T64 : plan.tile];
+    return snprintf(name, bytes, "gemm_direct_kernel<%s, %s, %d, %d, %d, %s, false>", ta ? "true" : "false", tb ? "true" : "false", s.bm, s.bn,
+                    s.res, small ? "true" : "false");
 }
 
 // A program has few shapes and calls them over and over; working one out takes some microseconds (hundreds of costs), so

@@ -116,6 +116,8 @@ struct GemmPlan {
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split);
 GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K);        // for GemmArgs::any (with parts of K)
 void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn);
+// the kernel of the plan's (first) launch as a profiler prints it; returns what snprintf does
+int gemm_kernel_name(int ta, int tb, const GemmPlan &plan, char *name, size_t bytes);
 
 // Products of operands whose rows are at least 8-byte aligned (align = 4; 8: 16-byte aligned), with a triangular operand or
 // a column window among them.

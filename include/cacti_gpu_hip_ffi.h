@@ -121,6 +121,8 @@ int cacti_hip_gemm_f16_ws(int ta, int tb, int64_t M, int64_t N, int64_t K, float
  * launch): out = rows and columns of the output tile of the first launch, its columns of C, rows and columns of the
  * tile of the second launch, launches (1 or 2). */
 int cacti_hip_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, int64_t out[6]);
+/* The kernel of the first launch of such a product, as a profiler prints it (a tile shape can have more than one). */
+int cacti_hip_gemm_kernel_name(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t nz, char *name, size_t bytes);
 
 /* `nblk` independent blocks, block h at A + h*stride_a etc. (strides in
  * elements).  This is how the per-head blocks of [B,S,H,Dh] / [B,S,H,S]

@@ -31,3 +31,18 @@ def test_a_group_is_cut_by_the_same_rule_as_its_products():
     products' own launches."""
     for M, N in ((128, 688), (688, 256), (1024, 256), (5, 20000), (512, 512)):
         assert all(plan(M, N, 256, nz)[:2] == [64, 64] for nz in (1, 2, 3, 4))
+
+
+@pytest.mark.parametrize("M,N,K,how", [(300, 8640, 256, "128, 128, 2, false"), (300, 8640, 1024, "128, 128, 1, false"),
+                                       (64, 5504, 256, "64, 64, 2, false"), (64, 256, 256, "64, 64, 2, true")])
+def test_kernel_names_tell_the_kernels_of_one_tile_shape_apart(M, N, K, how):
+    """128 x 128 exists with one and with two workgroups to a CU, 64 x 64 with either instruction."""
+    import bench
+    assert bench.kernel_symbol("matmul[NT,1x%dx%dx%d]" % (M, N, K)) == "gemm_direct_kernel<false, true, %s, false>" % how
+
+
+def test_a_kernel_name_needs_its_room():
+    name = C.create_string_buffer(128)
+    assert ffi.lib().cacti_hip_gemm_kernel_name(1, 0, 2048, 8640, 3200, 1, name, 20) == -1
+    assert ffi.lib().cacti_hip_gemm_kernel_name(1, 0, 2048, 8640, 3200, 1, name, 128) == 0
+    assert name.value == b"gemm_direct_kernel<true, false, 256, 256, 1, false, false>"
