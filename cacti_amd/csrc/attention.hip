@@ -18,12 +18,13 @@
 // (m, l) per row are kept for the adjoint.
 //
 // Adjoint: two kernels, each deterministic (no atomics).  The dQ kernel has the forward's shape
-// (queries fixed, loop over keys); the dK/dV kernel fixes 128 keys and loops over the queries at
+// (queries fixed, loop over keys); the dK/dV kernel fixes 128 or 64 keys and loops over the queries at
 // or after them.  Both recompute S16, P' and dP16 per tile.  The row sums sigma_i = sum_j P'_ij
 // f32(dP16_ij) are formed as the reference forms them, from the rounded dP16, by a first pass of the
-// dQ kernel over its key tiles (the shortcut sum_d dO_id O_id is the same number only in exact
-// arithmetic: it misses the cancellation between dP16 and sigma in rows whose probability sits on
-// one key, where the reference's dS is exactly zero).
+// dQ kernel over its key tiles, unless the probability of every row of a block of 128 queries is spread
+// (kSpread): the shortcut sum_d dO_id O_id is the same number only in exact arithmetic, and misses the
+// cancellation between dP16 and sigma in rows whose probability sits on one key, where the reference's
+// dS is exactly zero.
 //
 // MFMA data flow (v_mfma_f32_32x32x16_f16, D = X Y^T: lane <-> row of Y, registers <-> rows of X).
 // With the fixed operand as Y, a lane owns one query (key) and 16 of a 32-key (query) tile's
@@ -1784,8 +1785,9 @@ std::atomic<int> g_exact{0};             // cacti_hip_attention_set_exact: launc
 // over the CUs: 128 -> 64 rows, us, forward and adjoint, 611 positions, 16 heads of 64 19.2 -> 16.1 and 42.3 -> 35.4; 777,
 // 16 of 128 26.0 -> 20.7 and 62 -> 53; 1534, 16 of 100 41.3 -> 32.2 and 92 -> 85; 1984, 16 of 128 (496 workgroups) 50.8 ->
 // 46.2 and 115 -> 107; 1422, 24 of 100 (552) 38.4 -> 47.5 and 90 -> 94; 2048, 32 of 100 (1024) 68 -> 95 and 156 -> 168.
-// Exact arithmetic: 1531, 16 of 128 71.8 -> 43.7 and 172 -> 134.  Up to 128 positions there is a step or two either way.  The forward kernel's second round is short only if there
-// are long sequences in the first: 901, 32 of 100 (480 workgroups) 28.1 -> 29.2, 786 (416) 25.4 -> 25.6.
+// Exact arithmetic: 1531, 16 of 128 71.8 -> 43.7 and 172 -> 134.  Up to 128 positions there is a step or two either way.
+// The forward kernel's second round is short only if there are long sequences in the first: 901, 32 of 100 (480 workgroups)
+// 28.1 -> 29.2, 786 (416) 25.4 -> 25.6.
 int query_rows(int64_t S, int64_t H, bool forward, bool fast)
 {
     const int64_t cus = device_cus(), wgs = (S + 63) / 64 * H;

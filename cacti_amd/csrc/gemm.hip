@@ -347,9 +347,9 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
     }
     // Operands that are not 16-byte aligned, with a workspace: loaded as they are through registers on 64 x 64 tiles, or laid
     // out anew for the direct kernels (one launch for both, some 3.5 us and 0.4 us per MB), whichever is expected to take
-    // less.  Over 85 products of M 9 .. 4000, N 50 .. 5000, K 66 .. 5000 in three layouts the copy takes 28 % longer in the mean than
-    // the better of the two, registers 3 %, this rule 0.2 % (19 % at worst: 687 x 3731 x 410).  Element-wise loads in the kernel cost 1.6 us (both operands contiguous in K) to
-    // 3.4 us (both strided) per 32 values of K instead.
+    // less.  Over 85 products of M 9 .. 4000, N 50 .. 5000, K 66 .. 5000 in three layouts the copy takes 28 % longer in the
+    // mean than the better of the two, registers 3 %, this rule 0.2 % (19 % at worst: 687 x 3731 x 410).  Element-wise loads
+    // in the kernel cost 1.6 us (both operands contiguous in K) to 3.4 us (both strided) per 32 values of K instead.
     const int64_t ra = ta ? K : M, rb = tb ? N : K, pa = (ca + 7) / 8 * 8, pb = (cb + 7) / 8 * 8;
     if (ws_need && tri == 0 && nblk == 1 && K >= 8 && pa < kMaxPitch && pb < kMaxPitch) {
         const bool ok_a = fits_a(8) && lda < kMaxPitch, ok_b = fits_b(8) && ldb < kMaxPitch;

@@ -111,7 +111,9 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
         asm volatile("" ::"s"(p.N), "s"(p.K), "s"(p.alpha), "s"(p.A), "s"(p.lda), "s"(p.B), "s"(p.ldb), "s"(p.C), "s"(p.ldc),
                      "s"(p.x2), "s"(p.w), "s"(p.eps), "s"(p.sum_out), "s"(p.tok), "s"(p.vocab));
     if (NORM && EPI != E_PLAIN) asm volatile("" ::"s"(p.B2));
-    if (EPI == E_QKV) asm volatile("" ::"s"(p.B3), "s"(p.cos16), "s"(p.sin16), "s"(p.kc), "s"(p.vc), "s"(p.H), "s"(p.Dh), "s"(p.half_head.m), "s"(p.half_head.shift));
+    if (EPI == E_QKV)
+        asm volatile("" ::"s"(p.B3), "s"(p.cos16), "s"(p.sin16), "s"(p.kc), "s"(p.vc), "s"(p.H), "s"(p.Dh), "s"(p.half_head.m),
+                     "s"(p.half_head.shift));
     constexpr int kThreads = W * 64;
     constexpr bool GATE = EPI == E_GATE;
     constexpr int NB = GATE ? 2 : 1;
