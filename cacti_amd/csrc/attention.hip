@@ -1773,10 +1773,10 @@ int set_smem(K kern, size_t bytes)
     return 0;
 }
 
-// Which arithmetic the kernels are launched with (AttnMath).  Measured at 32 heads x 2048 x 100 on MI355X, in a
-// hot loop with the register loaders: forward 93 us / adjoint 232 us with the fast form, 123 / 305 us with the exact one; the two
-// differ by 3e-5 .. 4e-5 relative L2 in O, dQ, dK, dV, and O, dQ, dK, dV of the fast form agree with
-// the CPU restatement of the reference to 4.9e-5 .. 7.1e-5.
+// Which arithmetic the kernels are launched with (AttnMath).  Measured at 32 heads x 2048 x 100 on MI355X, in a hot loop:
+// forward 64 us / adjoint 145 us with the fast form, 101 / 251 us with the exact one, which has no in-wave pipelines, no short
+// form of sigma and no parts; the two differ by 3e-5 .. 4e-5 relative L2 in O, dQ, dK, dV, and O, dQ, dK, dV of the fast form
+// agree with the CPU restatement of the reference to 4.9e-5 .. 7.1e-5.
 std::atomic<int> g_exact{0};             // cacti_hip_attention_set_exact: launch the exactly rounded forms
 
 // Query rows per workgroup of the forward and the dQ kernel, 64 or 128.  A workgroup has a CU to itself and walks its keys

@@ -12,7 +12,7 @@
 // read feeds BM / 32 or BN / 32 products; eight waves on a 256 x 256 tile read half as many bytes again.  From 192 x 192
 // on the matrix pipes are the longest of the three, and with every CU at work the power limit is in front of them: 1616
 // TFLOP/s is what this mix of products, reads and loads sustains on random operands with no dependences (256 CUs; 872 on
-// 104, where it is the matrix pipes), 4096 x 4096 x 6400 runs at 1460.
+// 104, where it is the matrix pipes), 4096 x 4096 x 6400 runs at 1435 to 1460 by box, 8192 x 8192 x 8192 at 1465 to 1480.
 //
 // The compiler does not find this schedule by itself: left alone it spills (70 to 100 registers at 128 x 128 results per
 // wave) and moves the loads together, and a wave that is alone on its SIMD stands still while the vector memory path works
