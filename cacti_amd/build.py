@@ -43,7 +43,10 @@ def _compile(src):
     with tempfile.TemporaryDirectory() as tmp:
         made = os.path.join(tmp, name + ".o")
         _hipcc(src, made, "--save-temps=obj")
-        with open(os.path.join(tmp, name + "-hip-amdgcn-amd-amdhsa-gfx950.s")) as f:
+        asm = [f for f in os.listdir(tmp) if f.endswith("gfx950.s")]
+        if len(asm) != 1:
+            raise RuntimeError("%s: no assembly to check among %s" % (src, sorted(os.listdir(tmp))))
+        with open(os.path.join(tmp, asm[0])) as f:
             faults = asm_check.check(f.read(), spills=src == "gemm_direct.hip", fused=src == "gemm_direct.hip")
         if faults:
             raise RuntimeError("%s: %d faults around inline assembly\n%s" % (src, len(faults), "\n".join(faults[:20])))
