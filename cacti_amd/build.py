@@ -27,7 +27,7 @@ FLAGS = [
 ]
 # Sources with matrix instructions or loads into LDS in inline assembly: what the compiler made of them is checked.  In
 # gemm_direct.hip, whose kernels hold all of a wave's registers, a spill and a product rounded only once are faults too.
-CHECKED = ("attention.hip", "gemm_direct.hip", "gemm_mfma.hip")
+CHECKED = ("attention.hip", "attention_short.hip", "gemm_direct.hip", "gemm_mfma.hip")
 
 
 def sources():

@@ -317,9 +317,9 @@ size_t cacti_hip_attention_stats_bytes(int64_t S, int64_t H);
 int cacti_hip_attention_fwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,
                             const void *v, int64_t ld, void *o, void *stats, void *stream);
 size_t cacti_hip_attention_bwd_workspace(int64_t S, int64_t H);
-/* As much as the adjoint has a use for in the arithmetic that is set: with it (16-byte aligned) the default arithmetic sums the
- * dK / dV of short sequences in parts of the queries, on more of the device, where the tensors allow the faster form above
- * (ld % 8 == 0 and the rest).  Any workspace of at least
+/* As much as the adjoint can have a use for in the arithmetic that is set: with it (16-byte aligned) the default arithmetic sums
+ * the dK / dV of few heads in parts of the queries, on more of the device, where the tensors allow the faster form above
+ * (ld % 8 == 0 and the rest) and a walk over all queries takes longer.  Any workspace of at least
  * cacti_hip_attention_bwd_workspace(S, H) bytes is enough in either. */
 size_t cacti_hip_attention_bwd_workspace_best(int64_t S, int64_t H, int64_t Dh);
 int cacti_hip_attention_bwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,

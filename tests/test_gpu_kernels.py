@@ -717,6 +717,74 @@ def test_fused_attention(ops, oracle, S, H, Dh):
         assert_bits(host(a), host(b), "repeat")
 
 
+# Edges of the kernels of 32 rows per workgroup (attention_short.hip): of their blocks of 32 (a single position, one short of, on
+# and one past it), of what 4 and 8 waves split (128, 256), of the forms by length (1024, 2048) and by workgroups on 256 CUs (256,
+# 512; 768 and 1024 forward), and of the adjoint's other half (2048, 2 of 128: dK, dV in parts; 2080, 4 of 64: no forward; the
+# last ones: forward only, and neither); windows, rows longer than the heads, accumulation
+SHORT_SHAPES = [(1, 1, 8, 0), (31, 2, 100, 0), (32, 1, 64, 24), (33, 4, 60, 0), (127, 1, 128, 0), (129, 3, 64, 0), (255, 2, 68, 8),
+                (257, 1, 32, 0), (512, 16, 100, 0), (513, 16, 64, 0), (1023, 2, 12, 0), (1024, 8, 64, 0), (1025, 2, 128, 0), (2047, 8, 64, 0),
+                (2048, 2, 128, 8), (2080, 4, 64, 0), (97, 192, 12, 0), (128, 256, 72, 0), (128, 257, 72, 0)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("S,H,Dh,gap", SHORT_SHAPES)
+def test_attention_of_short_sequences_against_the_register_path(ops, S, H, Dh, gap, exact):
+    """Tensors on 16-byte boundaries against the same ones 8 bytes off (tiles through registers, 128 rows): relative L2 to the
+    chain in 64 bits of O, dQ, dK, dV no larger, but for the output's own rounding falling otherwise here and there (two sums of
+    the same terms in another order: a few of 2^-11 steps, 2e-5 of the norm, measured 1e-6); gap: columns between rows."""
+    import torch
+    from cacti_amd import ffi
+    say("attention of short sequences", S, H, Dh, gap, exact)
+    ld, alpha, st = H * Dh + gap, Dh ** -0.5, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(S + H + Dh)
+    def tensor(off, like=None):
+        x = torch.full((S * ld + 8,), 7.0, dtype=torch.float16, device="cuda")[off:off + S * ld].view(S, ld)
+        x[:, :H * Dh] = torch.randn(S, H * Dh, device="cuda", generator=g).half() if like is None else like[:, :H * Dh]
+        return x
+    q, k, v, dO, base = (tensor(0) for _ in range(5))
+    ffi.call("cacti_hip_attention_set_exact", int(exact))
+    try:
+        size = ffi.lib().cacti_hip_attention_bwd_workspace_best(S, H, Dh)
+        got = []
+        for off in (0, 4):
+            Q, K, V, DO, o = (tensor(off, like) for like in (q, k, v, dO, base))
+            stats, ws = torch.empty(2 * S * H, device="cuda"), torch.empty(size, dtype=torch.uint8, device="cuda")
+            ffi.call("cacti_hip_attention_fwd", S, H, Dh, alpha, Q.data_ptr(), K.data_ptr(), V.data_ptr(), ld, o.data_ptr(), stats.data_ptr(), st)
+            out = [o]
+            for with_o, acc in ((1, 0), (0, 0), (1, 1)):
+                d = [tensor(off, base) for _ in range(3)]
+                ffi.call("cacti_hip_attention_bwd", S, H, Dh, alpha, Q.data_ptr(), K.data_ptr(), V.data_ptr(), o.data_ptr() if with_o else None,
+                         DO.data_ptr(), ld, stats.data_ptr(), d[0].data_ptr(), acc, d[1].data_ptr(), acc, d[2].data_ptr(), acc, ws.data_ptr(),
+                         size, st)
+                out += d
+            assert all(bool((x[:, H * Dh:] == 7.0).all()) for x in out), "columns between rows"
+            got.append([x[:, :H * Dh].double() for x in out] + [stats.double()])
+    finally:
+        ffi.call("cacti_hip_attention_set_exact", 0)
+    sums = [0.0] * 4, [[0.0] * 10, [0.0] * 10]
+    for h in range(H):                              # the chain in 64 bits, a head at a time
+        hq, hk, hv, hd, hb = (t[:, h * Dh:(h + 1) * Dh].double() for t in (q, k, v, dO, base))
+        low = torch.ones(S, S, dtype=torch.bool, device="cuda").tril()
+        p = torch.softmax((alpha * hq @ hk.T.contiguous()).masked_fill(~low, float("-inf")), 1)
+        dp = hd @ hv.T.contiguous()
+        ds = p * (dp - (p * dp).sum(1, keepdim=True))
+        d = [alpha * ds @ hk, alpha * ds.T.contiguous() @ hq, p.T.contiguous() @ hd]
+        want = [p @ hv] + d + d + [x + hb for x in d]
+        for i, w in enumerate([p @ hv] + d): sums[0][i] += float(w.square().sum())
+        for side in (0, 1):
+            for i, w in enumerate(want):
+                sums[1][side][i] += float((got[side][i][:, h * Dh:(h + 1) * Dh] - w).square().sum())
+    for i in range(10):
+        norm = max(sums[0][(0, 1, 2, 3)[0 if i == 0 else (i - 1) % 3 + 1]], 1e-30 * S * H * Dh)
+        new, old = (sums[1][side][i] ** 0.5 / norm ** 0.5 for side in (0, 1))
+        say("  result %d: rel_l2 %.3e, through registers %.3e" % (i, new, old))
+        assert new <= old + 2e-5, (i, new, old)
+    # the statistics: maxima and sums of the rounded scores, of which a few round otherwise in the other order of summation
+    m, l = (torch.stack([got[side][10].view(2, H, S)[j] for side in (0, 1)]) for j in (0, 1))
+    assert float((m[0] - m[1]).abs().max()) <= 2e-3 * max(1.0, float(m.abs().max())) and float((l[0] / l[1] - 1).abs().max()) < 2e-3
+
+
 # The forward and the dQ kernel take 64 query rows per workgroup where their number is at most twice (forward, fast, up to
 # 1024 positions: 7/4 of) the CUs' of an MI355X, 256, and 128 beyond: rows one short of, on and one past the edges of both
 # at few heads, and the 128 rows' form at many small heads (480 workgroups of 64 rows: forward only; 528, 640: both), with
