@@ -91,8 +91,13 @@ __device__ __forceinline__ void load_odd(half_t *lds, const half_t *c, int64_t l
 // ANY: operands of any alignment, through registers (LoadKCR, LoadKSR), two tile buffers of each; three tiles ahead in
 // registers, which is what a k tile of 64 x 64 (a quarter of a microsecond) needs to have its loads back in time.  509 x 1003 x
 // 770 in three layouts: 32.2 -> 26 us against a copy to aligned rows in front.
-template <bool TA, bool TB, int BM, int BN, int RES, bool M32, bool ANY>
-__global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
+// CHAIN: the sum of p.chain products (offsets za, zb; K a multiple of 64, at least 256), each rounded to f16 with what the ones
+// before it came to, as launches one after another that accumulate into C round it, with the sum so far in registers and the
+// next product's tiles on their way while the last one's are multiplied.  Launches apart cost a start and an end each (3.7 us
+// with 64 x 64, 5.7 with 160 x 192), the sum's way through memory and the gap between them: three of 611 x 1024 x 1024 21.0 ->
+// 14.2 us, of 777 x 2048 x 2048 41.0 -> 31.6, of 2048 x 3200 x 3200 132 -> 114; two of 2048 x 3200 x 8640 199 -> 195.
+template <bool TA, bool TB, int BM, int BN, int RES, bool M32, bool ANY, bool CHAIN>
+__device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p)
 {
     // the whole argument block in scalar registers before anything else: read field by field where the control
     // flow first wants it, it costs five dependent round trips to memory before the first operand load
@@ -104,7 +109,8 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     static_assert(D >= 2 && BM % 32 == 0 && BN % 64 == 0 && (!M32 || (BM == 64 && BN == 64)), "tile shape");
     constexpr bool TR_A = TA, TR_B = !TB;                         // fragments by transposing reads
     constexpr int NA = BM / 32, NB = BN / 32;                     // fragments of a wave
-    constexpr bool PARTS = BM * BN <= kMaxPartTile && !M32;
+    constexpr bool PARTS = BM * BN <= kMaxPartTile && !M32 && !CHAIN;
+    static_assert(!CHAIN || (!ANY && D <= 4), "the first D tiles are of the first product");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     half_t *As = reinterpret_cast<half_t *>(smem_raw);            // [NBA][BM * BK]
     half_t *Bs = As + NBA * BM * BK;                              // [NBB][BN * BK]
@@ -113,6 +119,8 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     p.walk.locate(blockIdx.x, tm, tn, bz);
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
     int nk = (int)((p.K + BK - 1) / BK), kt0 = 0;
+    const int product = nk;                                       // CHAIN: k tiles of one
+    if constexpr (CHAIN) nk *= p.chain;
     const int part = bz;
     if (PARTS && p.part) {
         // the "blocks of the batch" are the parts of K: the same operands, a range of k tiles each
@@ -140,7 +148,7 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     // (the columns of a strided operand end on a multiple of 8: its width, or the padding behind it)
     la.init(p.lda, (TA && !ANY ? (p.M + 7) / 8 * 8 : p.M) - m0, p.K);
     lb.init(p.ldb, (TB || ANY ? p.N : (p.N + 7) / 8 * 8) - n0, p.K);
-    const int ktail = (int)(p.K % BK);
+    const int ktail = CHAIN ? 0 : (int)(p.K % BK);
     auto lds_addr = [](const half_t *q) __attribute__((always_inline)) { return (uint32_t)(uintptr_t)q; };
     // ANY: G sets of registers, one tile of both operands each; tile t in set (t - kt0) % G
     constexpr int G = 3;
@@ -302,6 +310,64 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     typedef std::integral_constant<int, 0> K0;
     typedef std::integral_constant<int, 1> K1;
 
+    // alpha times the sum, rounded to fp32 (the empty asm keeps the compiler from fusing the product with the conversion
+    // behind it in some of the kernels and not in others)
+    auto scaled = [&](int a, int b, int r) __attribute__((always_inline)) {
+        float v;
+        if constexpr (M32) v = p.alpha * c32[b * 4 + r];
+        else v = p.alpha * c[a][b][r];
+        asm("" : "+v"(v));
+        return v;
+    };
+    // M32: four groups q of a lane's columns in place of the fragments
+    constexpr int EA = M32 ? 1 : NA, EB = M32 ? 4 : NB;
+    // the accumulators are read by vector instructions from here on, which do not wait for a product by themselves
+    auto sums_done = [&]() __attribute__((always_inline)) {
+        asm volatile("s_nop 15\n\ts_nop 15");
+        if constexpr (M32) {
+            asm volatile("" : "+a"(c32));
+        } else {
+#pragma unroll
+            for (int a = 0; a < NA; a++)
+#pragma unroll
+                for (int b = 0; b < NB; b++) asm volatile("" : "+a"(c[a][b]));
+        }
+    };
+    // CHAIN: what the products before came to (at first -0, to which anything adds as itself)
+    half4_t sum[CHAIN ? EA : 1][CHAIN ? EB : 1];
+    if constexpr (CHAIN)
+#pragma unroll
+        for (int a = 0; a < EA; a++)
+#pragma unroll
+            for (int b = 0; b < EB; b++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) sum[a][b][r] = (half_t)-0.0f;
+    auto fold = [&]() __attribute__((always_inline)) {
+        sums_done();
+#pragma unroll
+        for (int a = 0; a < EA; a++)
+#pragma unroll
+            for (int b = 0; b < EB; b++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    sum[CHAIN ? a : 0][CHAIN ? b : 0][r] = f2h(scaled(a, b, r) + h2f(sum[CHAIN ? a : 0][CHAIN ? b : 0][r]));
+        // zeroed where they are, by a product of zeros: as values that the compiler assigns they get registers of their own, which
+        // the loop's are copied into on its other path.  (Behind it the compiler may still move one.)
+        half8_t zero;
+#pragma unroll
+        for (int i = 0; i < 8; i++) zero[i] = (half_t)0.0f;
+        asm volatile("s_nop 4" : "+v"(zero));
+        if constexpr (M32) {
+            asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %1, 0" : "+a"(c32) : "v"(zero));
+        } else {
+#pragma unroll
+            for (int a = 0; a < NA; a++)
+#pragma unroll
+                for (int b = 0; b < NB; b++) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %1, 0" : "+a"(c[a][b]) : "v"(zero));
+        }
+        sums_done();
+    };
+
     constexpr int TA_BYTES = BM * BK * 2, TB_BYTES = BN * BK * 2, B0 = NBA * TA_BYTES;
     int ta = 0, tb = B0;                                          // byte offsets in LDS of tile t
     auto next_a = [&](int q) __attribute__((always_inline)) { return q == (NBA - 1) * TA_BYTES ? 0 : q + TA_BYTES; };
@@ -368,6 +434,17 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     const half_t *asrc = la.kbase(Ao, (int64_t)(kt0 + D) * BK), *bsrc = lb.kbase(Bo, (int64_t)(kt0 + D) * BK);
     const int64_t astep = TA ? BK * p.lda : BK, bstep = TB ? BK : BK * p.ldb;
     int te = EARLY_A ? D * TA_BYTES : B0 + D * TB_BYTES;          // buffer of tile t + D of the early operand
+    // CHAIN: tiles of the present product that are still to be loaded and to be multiplied
+    int to_load = product - D, to_sum = product, next = 0;
+    auto next_product = [&]() __attribute__((always_inline)) {
+        next++;
+        to_load = product;
+        if (next < p.chain) {
+            asrc = Ao + p.za[next];
+            bsrc = Bo + p.zb[next];
+        }
+    };
+    if (CHAIN && to_load == 0) next_product();
     const int nk_whole = M32 && ktail ? nk - 1 : nk;
     for (; t + D < nk_whole; t++) {
         step(K0{}, std::integral_constant<int, NE>{}, std::integral_constant<bool, EARLY_A>{}, ta, tb, EARLY_A ? asrc : bsrc,
@@ -382,6 +459,13 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
         te = EARLY_A ? next_a(te) : next_b(te);
         asrc += astep;
         bsrc += bstep;
+        if constexpr (CHAIN) {
+            if (--to_load == 0) next_product();
+            if (--to_sum == 0) {
+                fold();
+                to_sum = product;
+            }
+        }
     }
     for (; t + 1 < nk; t++) {                                     // the last tiles: nothing left to load but M32's tail
         const bool tail = M32 && ktail && t + D == nk - 1;
@@ -405,16 +489,7 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
 #pragma unroll
     for (int m = 0; m < NM; m++) mfma(1, m);
     }
-    // the accumulators are read by vector instructions from here on, which do not wait for a product by themselves
-    asm volatile("s_nop 15\n\ts_nop 15");
-    if constexpr (M32) {
-        asm volatile("" : "+a"(c32));
-    } else {
-#pragma unroll
-        for (int a = 0; a < NA; a++)
-#pragma unroll
-            for (int b = 0; b < NB; b++) asm volatile("" : "+a"(c[a][b]));
-    }
+    sums_done();
 
     if (PARTS && p.part) {
         // a lane's 4 consecutive columns of a row are 16 bytes of the part, four lanes a 64-byte run
@@ -470,17 +545,6 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     auto out4 = [&](int a, int b) __attribute__((always_inline)) {
         return reinterpret_cast<half4_t *>(eo + a * 32 * (BN * 2) + ((ex ^ (M32 ? b : b << 2)) << 4));
     };
-    // M32: four groups q of a lane's columns in place of the fragments
-    constexpr int EA = M32 ? 1 : NA, EB = M32 ? 4 : NB;
-    // alpha times the sum, rounded to fp32 (the empty asm keeps the compiler from fusing the product with the conversion
-    // behind it in some of the kernels and not in others)
-    auto scaled = [&](int a, int b, int r) __attribute__((always_inline)) {
-        float v;
-        if constexpr (M32) v = p.alpha * c32[b * 4 + r];
-        else v = p.alpha * c[a][b][r];
-        asm("" : "+v"(v));
-        return v;
-    };
     if (p.beta != 0.f) {
 #pragma unroll
         for (int a = 0; a < EA; a++)
@@ -499,7 +563,10 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
             for (int b = 0; b < EB; b++) {
                 half4_t o;
 #pragma unroll
-                for (int r = 0; r < 4; r++) o[r] = f2h(scaled(a, b, r));
+                for (int r = 0; r < 4; r++) {
+                    if constexpr (CHAIN) o[r] = f2h(scaled(a, b, r) + h2f(sum[a][b][r]));
+                    else o[r] = f2h(scaled(a, b, r));
+                }
                 *out4(a, b) = o;
             }
     }
@@ -540,6 +607,17 @@ __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
     if (p.odd) copy_out(std::false_type{}, std::true_type{});
     else if (inside) copy_out(std::true_type{}, std::false_type{});
     else copy_out(std::false_type{}, std::false_type{});
+}
+
+template <bool TA, bool TB, int BM, int BN, int RES, bool M32, bool ANY>
+__global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
+{
+    gemm_direct_tile<TA, TB, BM, BN, RES, M32, ANY, false>(p);
+}
+template <int BM, int BN, int RES, bool M32>
+__global__ void __launch_bounds__(256, RES) gemm_chain_kernel(GemmArgs p)
+{
+    gemm_direct_tile<false, false, BM, BN, RES, M32, false, true>(p);
 }
 
 // C = f16(alpha sum of the parts + beta C), four columns per lane; the parts are added in order.  VEC: N and the rows
@@ -604,12 +682,14 @@ __global__ void __launch_bounds__(256) repack_kernel(RepackArgs p)
     *reinterpret_cast<int4_t *>(p.dst[z] + i * 8) = v;
 }
 
-template <bool TA, bool TB, int BM, int BN, int RES, bool M32 = false, bool ANY = false>
+template <bool TA, bool TB, int BM, int BN, int RES, bool M32 = false, bool ANY = false, bool CHAIN = false>
 int launch(GemmArgs p, int64_t nblk, hipStream_t st)
 {
     const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     constexpr size_t smem = (size_t)(ANY ? 2 * (BM + BN) : buffers(BM, BN, RES) * (BM + BN) + (BM < BN ? BM : BN)) * BK * sizeof(half_t);
-    auto kern = gemm_direct_kernel<TA, TB, BM, BN, RES, M32, ANY>;
+    void (*kern)(GemmArgs);
+    if constexpr (CHAIN) kern = gemm_chain_kernel<BM, BN, RES, M32>;
+    else kern = gemm_direct_kernel<TA, TB, BM, BN, RES, M32, ANY>;
     static DeviceOnce attr_set;                   // one per instantiation
     if (!attr_set.fresh()) {
         CACTI_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
@@ -653,11 +733,20 @@ constexpr Shape kShapes[] = {
     {256, 256, 1, 8.360, 0.901, 0.592, 1.409, 7.849},
 };
 constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
+constexpr int kChainShapes = kNumShapes - 2;      // of the last two a lane has no registers for a second sum
 constexpr int T64 = 0, T64_SMALL = kNumShapes;   // T64_SMALL: 64 x 64 with M32
 
 template <bool TA, bool TB, int... I>
 int launch_shape(int shape, const GemmArgs &p, int64_t nblk, hipStream_t st, std::integer_sequence<int, I...>)
 {
+    if constexpr (!TA && !TB)
+        if (p.chain > 1) {
+            if (shape == T64_SMALL) return launch<TA, TB, 64, 64, 2, true, false, true>(p, nblk, st);
+            int rc = CACTI_E_STATE;
+            (void)((shape == I && I < kChainShapes && (rc = launch<TA, TB, kShapes[I < kChainShapes ? I : 0].bm, kShapes[I < kChainShapes ? I : 0].bn,
+                                                                  kShapes[I < kChainShapes ? I : 0].res, false, false, true>(p, nblk, st), true)) || ...);
+            return rc;
+        }
     if (shape == T64_SMALL) return launch<TA, TB, 64, 64, 2, true>(p, nblk, st);
     if (p.any) return launch<TA, TB, 64, 64, 2, false, true>(p, nblk, st);
     int rc = CACTI_E_STATE;
@@ -709,7 +798,7 @@ void split_k(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, double per_ti
 // 256 and 448 columns); and, where the caller has a workspace (may_split), up to 8 parts of K for products with fewer
 // tiles than CUs and a long K, whose workgroups would otherwise run 100 k tiles one after another on a fraction of the CUs
 // (37 x 3200 x 8640: 25 tiles; the parts and their sum cost a launch and 8 bytes per part and element).
-GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split)
+GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split, int shapes = kNumShapes)
 {
     const int64_t kt = (K + BK - 1) / BK;
     // A small output has about 64 tiles of 64 x 64 (or one row or column of them), the shape that is best for it while they
@@ -721,20 +810,20 @@ GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, boo
     const bool small = M * N <= kSmallOutput && (nz <= kMaxPtrBatch || tiles64 * nz <= kShapes[T64].res * cus);
     double best_cost = tile_cost(cus, T64, M, N, nz, kt);
     GemmPlan best = {small ? T64_SMALL : T64, T64, 0, 1, 0};
-    for (int t = T64 + 1; t < kNumShapes && !small; t++) {
+    for (int t = T64 + 1; t < shapes && !small; t++) {
         const double c = tile_cost(cus, t, M, N, nz, kt);
         if (c < best_cost) {
             best_cost = c;
             best = {t, T64, 0, 1, 0};
         }
     }
-    for (int t = T64 + 1; t < kNumShapes && !small; t++) {
+    for (int t = T64 + 1; t < shapes && !small; t++) {
         if (kShapes[t].res > 1) continue;
         const int64_t bn = kShapes[t].bn, tiles_m = (M + kShapes[t].bm - 1) / kShapes[t].bm * nz, tiles_n = (N + bn - 1) / bn;
         const int64_t cols = tiles_m * tiles_n / cus * cus / tiles_m * bn;
         if (cols <= 0 || cols >= N) continue;
         const double first = tile_cost(cus, t, M, cols, nz, kt);
-        for (int r = T64; r < kNumShapes && first < best_cost; r++) {
+        for (int r = T64; r < shapes && first < best_cost; r++) {
             const double c = first + tile_cost(cus, r, M, N - cols, nz, kt);
             if (c < best_cost) {
                 best_cost = c;
@@ -790,21 +879,23 @@ int gemm_kernel_name(int ta, int tb, const GemmPlan &plan, char *name, size_t by
 
 // A program has few shapes and calls them over and over; working one out takes some microseconds (hundreds of costs), so
 // each thread keeps the plans of the last ones by their sizes.
-GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split)
+static GemmPlan kept_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split, int chain)
 {
     struct Kept {
-        int64_t M, N, K, nz, how;                 // how: compute units and may_split; 0: none kept
+        int64_t M, N, K, nz, how;                 // how: compute units, chain and may_split; 0: none kept
         GemmPlan plan;
     };
     static thread_local Kept kept[256] = {};
-    const int64_t cus = device_cus(), how = cus * 2 + (may_split ? 1 : 0);
+    const int64_t cus = device_cus(), how = (cus * 8 + chain) * 2 + (may_split ? 1 : 0);
     const uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15u ^ (uint64_t)N * 0xc2b2ae3d27d4eb4fu ^ (uint64_t)K * 0x165667b19e3779f9u) +
-                       (uint64_t)(nz * 2 + (may_split ? 1 : 0)) * 0x27d4eb2f165667c5u;
+                       (uint64_t)(nz * 2 + (may_split ? 1 : 0) + chain * 64) * 0x27d4eb2f165667c5u;
     Kept &k = kept[h >> 56];
     if (k.how != how || k.M != M || k.N != N || k.K != K || k.nz != nz)
-        k = {M, N, K, nz, how, make_plan(cus, M, N, K, nz, may_split)};
+        k = {M, N, K, nz, how, make_plan(cus, M, N, K * chain, nz, may_split, chain > 1 ? kChainShapes : kNumShapes)};
     return k.plan;
 }
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split) { return kept_plan(M, N, K, nz, may_split, 1); }
+GemmPlan gemm_plan_chain(int64_t M, int64_t N, int64_t K, int chain) { return kept_plan(M, N, K, 1, false, chain); }
 
 // The same for operands that are loaded through registers whatever their alignment: 64 x 64 tiles, whose k tiles take some
 // half longer than the direct ones' (64 x 128 and 128 x 128 took twice and three times as long as that: their loads have

@@ -99,6 +99,8 @@ struct GemmArgs {
     int split_tiles;
     float *part;
     int64_t ldp;
+    // chain > 1: the sum of that many products A + za[z], B + zb[z], rounded to f16 with what the ones before came to (beta 0)
+    int chain;
     int odd;              // C of any alignment and N
     int any;              // A and B of any alignment (strided operands with rows of 8 elements and more)
 };
@@ -114,6 +116,7 @@ struct GemmPlan {
 };
 // nz: products of this shape in the launch
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split);
+GemmPlan gemm_plan_chain(int64_t M, int64_t N, int64_t K, int chain);       // chain <= kMaxPtrBatch products that add up
 GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K);        // for GemmArgs::any (with parts of K)
 void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn);
 // the kernel of the plan's (first) launch as a profiler prints it; returns what snprintf does

@@ -1323,7 +1323,8 @@ int Ctx::run_entry(const Entry &e)
     for (int i = 0; i < n; i++) {
         std::vector<CellPtr> args;
         const std::unique_ptr<ThunkSpec> one = sp.piece(i, e.args, &args);
-        rc = run_thunk(*one, args, {e.outs[(size_t)i]}, (e.acc_mask >> i) & 1);
+        const int o = sp.pieces_add_up() ? 0 : i;
+        rc = run_thunk(*one, args, {e.outs[(size_t)o]}, i > o ? 1 : (e.acc_mask >> o) & 1);
         if (rc) return rc;
     }
     return 0;

@@ -315,8 +315,9 @@ struct MatMulSpec : ThunkSpec {
 // (and the gate and up projections) as separate matmul thunks on the same input (src/librarium/llama.rs:
 // 478-497); each output here is summed over the same values in the same order as in a launch of its own (the tiles
 // may be others), so the results are those of the separate thunks bit for bit, and the adjoint stages what their
-// adjoints would have staged, in their order: the weight gradients (one grouped thunk), then the input gradients one after the other
-// (they accumulate into one cell: last product first, as the reverse sweep over separate thunks meets them).
+// adjoints would have staged, in their order: the weight gradients (one grouped thunk), then the input gradients (one thunk and
+// launch as well, cacti_hip_gemm_f16_chain: they accumulate into one cell, last product first, as the reverse sweep over
+// separate thunks meets them, with a rounding behind each).
 constexpr int kMaxGroup = 4;
 
 // dW_i = dy_i^T x: (dy_1 .. dy_n, x) -> (dW_1 .. dW_n)
@@ -369,6 +370,45 @@ struct WgradNSpec : ThunkSpec {
         char buf[128];
         snprintf(buf, sizeof(buf), "matmul[TN,1x%lldx%lldx%lld%s]x%d", (long long)aty[0].shape[1],
                  (long long)aty[n].shape[1], (long long)aty[0].shape[0], (acc & 1) ? ",acc" : "", n);
+        return buf;
+    }
+};
+
+// dx = dy_1 W_1 + .. + dy_n W_n, each product rounded to f16 with the sum of the ones before it:
+// (dy_1 .. dy_n, W_1 .. W_n) -> dx
+struct DgradNSpec : ThunkSpec {
+    int n;
+    explicit DgradNSpec(int n_) : n(n_) {}
+    const char *name() const override { return "matmul"; }
+    int arity() const override { return 2 * n; }
+    int out_ty(const std::vector<CellType> &a, std::vector<CellType> &o) const override
+    {
+        TY_REQUIRE(n >= 2 && n <= kMaxGroup, "chained input gradients: 2 .. %d products", kMaxGroup);
+        for (int i = 0; i < n; i++)
+            TY_REQUIRE(a[i].dtype == F16 && a[i].shape.size() == 2 && a[i] == a[0] && a[n + i] == a[n] && a[n].dtype == F16 &&
+                           a[n].shape.size() == 2 && a[n].shape[0] == a[0].shape[1],
+                       "chained input gradients: (dy f16 [S,N] x n, W f16 [N,K] x n) expected");
+        o.assign(1, CellType({a[0].shape[0], a[n].shape[1]}, F16));
+        return 0;
+    }
+    int run(Ctx &c, const std::vector<CellType> &aty, void *const *a, const std::vector<CellType> &,
+            void *const *o, uint32_t acc, void *, size_t) const override
+    {
+        const int64_t Sq = aty[0].shape[0], N = aty[0].shape[1], K = aty[n].shape[1];
+        return cacti_hip_gemm_f16_chain(n, Sq, K, N, a, N, a + n, K, (acc & 1) ? 1.f : 0.f, o[0], K, S(c));
+    }
+    int pieces() const override { return n; }
+    bool pieces_add_up() const override { return true; }
+    std::unique_ptr<ThunkSpec> piece(int i, const std::vector<CellPtr> &a, std::vector<CellPtr> *in) const override
+    {
+        *in = {a[(size_t)i], a[(size_t)(n + i)]};
+        return make_matmul(false, false, 1.f);
+    }
+    std::string key(const std::vector<CellType> &aty, uint32_t acc) const override
+    {
+        char buf[128];
+        snprintf(buf, sizeof(buf), "matmul[NN,1x%lldx%lldx%lld%s]x%d", (long long)aty[0].shape[0], (long long)aty[n].shape[1],
+                 (long long)aty[0].shape[1], (acc & 1) ? ",acc" : "", n);
         return buf;
     }
 };
@@ -428,11 +468,14 @@ struct ProjNSpec : ThunkSpec {
             std::vector<CellPtr> ws(e.args.begin() + 1, e.args.end()), in(dy.begin(), dy.begin() + n);
             in.push_back(x);
             if ((rc = c.adj_add(ws, std::unique_ptr<ThunkSpec>(new WgradNSpec(n)), in))) return rc;
+            std::vector<CellPtr> chain(dy.rend() - n, dy.rend());
+            chain.insert(chain.end(), ws.rbegin(), ws.rend());
+            return c.adj_add({x}, std::unique_ptr<ThunkSpec>(new DgradNSpec(n)), chain);
         }
         for (int i = n - 1; i >= 0; i--) {
             if (!dy[i]) continue;
             const CellPtr W = e.args[1 + i];
-            if (!all && (rc = c.adj_add({W}, std::unique_ptr<ThunkSpec>(new MatMulSpec(true, false, 1.f, 0)), {dy[i], x})))
+            if ((rc = c.adj_add({W}, std::unique_ptr<ThunkSpec>(new MatMulSpec(true, false, 1.f, 0)), {dy[i], x})))
                 return rc;                                                     // G^T A
             if ((rc = c.adj_add({x}, std::unique_ptr<ThunkSpec>(new MatMulSpec(false, false, 1.f, 0)), {dy[i], W})))
                 return rc;                                                     // G B

@@ -159,6 +159,10 @@ int cacti_hip_mfma_probe(int shape, int lds_reads, int random_operands, int bloc
 int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K,
                                float alpha, const void *const *A, int64_t lda, const void *const *B,
                                int64_t ldb, float beta, void *const *C, int64_t ldc, void *stream);
+/* C = f16(f16(A_0 B_0 + beta C) + A_1 B_1) .. : n products of row-major [M,K] and [K,N] operands that accumulate into one
+ * matrix, with the bits of n calls of cacti_hip_gemm_f16 (beta 1 from the second on). */
+int cacti_hip_gemm_f16_chain(int64_t n, int64_t M, int64_t N, int64_t K, const void *const *A, int64_t lda, const void *const *B,
+                             int64_t ldb, float beta, void *C, int64_t ldc, void *stream);
 
 /* The same with the triangular structure of causal attention made explicit, so that the
  * half of each sequence x sequence product that the causal mask discards is never computed:

@@ -592,6 +592,37 @@ def test_gemm_random_shapes_through_the_tile_choice(ops, seed):
         assert err < 6e-4 and mx < 4e-3, (ta, tb, M, N, K, alpha, beta, err, mx)
 
 
+# sums of products in one launch: small outputs (M32) and others, edges of tiles and one past them, as many k tiles as buffers
+# (256) and one more, remainders of all tiles; behind the line what is not for one launch: K below 256 or no multiple of 64, five
+# products, rows that are not 16-byte aligned
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,M,N,K,gap,beta", [
+    (2, 1, 8, 256, 0, 0), (3, 64, 64, 256, 0, 0), (4, 65, 72, 320, 8, 0), (2, 33, 264, 384, 0, 0), (3, 512, 512, 256, 0, 0),
+    (3, 513, 520, 256, 0, 0), (2, 611, 1032, 1024, 8, 0), (3, 777, 2048, 448, 0, 0), (2, 2049, 1608, 256, 0, 0), (4, 1000, 3200, 512, 0, 0),
+    (2, 2048, 8640, 320, 0, 0), (2, 4000, 4104, 256, 0, 0),
+    (1, 96, 128, 512, 0, 0), (2, 96, 128, 192, 0, 0), (3, 96, 128, 328, 0, 0), (5, 96, 640, 256, 0, 0), (2, 300, 1028, 256, 0, 0), (3, 512, 520, 256, 0, 1)])
+def test_gemm_chain_has_the_bits_of_products_one_by_one(ops, n, M, N, K, gap, beta):
+    import ctypes as C
+    import torch
+    from cacti_amd import ffi
+    say("gemm chain", n, M, N, K, gap, beta)
+    g = torch.Generator(device="cuda").manual_seed(n + M + N + K)
+    st = torch.cuda.current_stream().cuda_stream
+    rows = lambda r, c: torch.randn(r, c + gap, device="cuda", generator=g).half()
+    A, B, c0 = [rows(M, K) for _ in range(n)], [rows(K, N) for _ in range(n)], rows(M, N)
+    got, want = c0.clone(), c0.clone()
+    for z in range(n):
+        ffi.call("cacti_hip_gemm_f16", 0, 0, M, N, K, 1.0, A[z].data_ptr(), K + gap, B[z].data_ptr(), N + gap, 1.0 if z else float(beta),
+                 want.data_ptr(), N + gap, st)
+    pa, pb = ((C.c_void_p * n)(*[t.data_ptr() for t in x]) for x in (A, B))
+    ffi.call("cacti_hip_gemm_f16_chain", n, M, N, K, C.cast(pa, C.c_void_p), K + gap, C.cast(pb, C.c_void_p), N + gap, float(beta),
+             got.data_ptr(), N + gap, st)
+    assert_bits(host(got), host(want), "chain")
+    ref = sum(a[:, :K].float() @ b[:, :N].float() for a, b in zip(A, B)) + beta * c0[:, :N].float()
+    # n roundings of partial sums of the size of the result at most: n half ulps, 2^-12 of a value in the mean
+    assert ((got[:, :N].float() - ref).norm() / ref.norm()).item() < n * 3e-4
+
+
 def test_gemm_colmajor_entry(ops, oracle):
     """The cuBLAS-shaped entry: row-major callers pass operands swapped (thunk/op.rs:4469-4491)."""
     import ctypes as C
