@@ -558,7 +558,76 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
             if (!tiles_on_the_way) first_tiles();
             tiles_on_the_way = false;
             tile_sync<DMA>();
-            for (int it = 0; it < niter; it++) {
+            int it0 = 0;
+            if constexpr (FAST && DMA && KP == 1 && PASS == 1 && KS == 4) {
+                // The key tiles wholly below the diagonal for every wave, as in the forward kernel, with the vector arithmetic
+                // between MFMAs: that of a tile's first block between the score and dP products of its second, the second's
+                // between the first's products with K; the first block's scores and dP of the next tile follow the barrier
+                // that publishes it.  The same operations on the same values in the same order as the general loop below.
+                // Heads to 64: 1531 positions, 32 heads 54.4 -> 44.9 us, 1000, 40 heads 37.0 -> 30.4, 4000, 16 heads 92 -> 80.
+                // Wider ones have no registers for it: 32 heads of 100 at 2048 positions spill 23 and take 102 us instead of
+                // 91; with fragments read three ahead instead of all there is no spill in the loop, and 99.
+                const int nfull = min(qt, niter);
+                if (nfull > 0) {
+                    half2v_t sp[8], dp[8];
+                    float pr[16], de[16];
+                    half8_t pk[2][2];                           // packed dS of the tile's two blocks
+                    auto prob_piece = [&](const float16_t &sacc, const float16_t &pacc, auto i_c) __attribute__((always_inline)) {
+                        constexpr int i = decltype(i_c)::value;
+                        if constexpr (i == 1) {
+#pragma unroll
+                            for (int e = 0; e < 8; e++)
+                                sp[e] = __builtin_convertvector(float2v_t{scaled(p.alpha, sacc[2 * e]), scaled(p.alpha, sacc[2 * e + 1])}, half2v_t);
+                        } else if constexpr (i > 1) {
+#pragma unroll
+                            for (int e = 4 * (i - 2); e < 4 * (i - 1); e++) pr[e] = exp2_mix(sp[e >> 1][e & 1], cs);
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 8; e++) dp[e] = __builtin_convertvector(float2v_t{pacc[2 * e], pacc[2 * e + 1]}, half2v_t);
+                        }
+                    };
+                    auto ds_piece = [&](half8_t (&out)[2], auto i_c) __attribute__((always_inline)) {
+                        constexpr int i = decltype(i_c)::value;
+                        if constexpr (i < 4) {
+#pragma unroll
+                            for (int e = 4 * i; e < 4 * i + 4; e++) de[e] = __builtin_fmaf((float)dp[e >> 1][e & 1], pr[e], -(sig * pr[e]));
+                        } else {
+                            out[i - 4] = pack8(de + 8 * (i - 4));
+                        }
+                    };
+                    float16_t s0 = prod_direct<KS>(Ks, 0, qf, l32, lh), p0 = prod_direct<KS>(Vs, 0, gf, l32, lh);
+                    for (int it = 0; it < nfull; it++) {
+                        const int jt = 2 * it + g, cur = it & 1;
+                        const unsigned char *Kc = Ks + cur * kTileB, *Vc = Vs + cur * kTileB;
+                        if (jt + 2 < njt) {
+                            tk.load(tm, K + (int64_t)(jt + 2) * kTileRows * ld, S - (jt + 2) * kTileRows, Ks + (cur ^ 1) * kTileB);
+                            tv.load(tm, V + (int64_t)(jt + 2) * kTileRows * ld, S - (jt + 2) * kTileRows, Vs + (cur ^ 1) * kTileB);
+                        }
+                        const float16_t s1 = prod_direct_with<KS, 6>(Kc, 32, qf, l32, lh, [&](auto i_c) { prob_piece(s0, p0, i_c); });
+                        const float16_t p1 = prod_direct_with<KS, 6>(Vc, 32, gf, l32, lh, [&](auto i_c) { ds_piece(pk[0], i_c); });
+                        asm volatile("" : "+v"(pk[0][0]), "+v"(pk[0][1]));
+                        prod_tr_with<DT, 8>(dacc, Kc, 0, pk[0][0], pk[0][1], lane, [&](auto i_c) __attribute__((always_inline)) {
+                            constexpr int i = decltype(i_c)::value;
+                            if constexpr (i < 6) {
+                                prob_piece(s1, p1, i_c);
+                            } else {
+                                ds_piece(pk[1], std::integral_constant<int, 2 * (i - 6)>{});
+                                ds_piece(pk[1], std::integral_constant<int, 2 * (i - 6) + 1>{});
+                                ds_piece(pk[1], std::integral_constant<int, i - 2>{});
+                            }
+                        });
+                        asm volatile("" : "+v"(pk[1][0]), "+v"(pk[1][1]));
+                        prod_tr<DT>(dacc, Kc, 32, pk[1][0], pk[1][1], lane);
+                        tile_sync<DMA>();
+                        if (it + 1 < nfull) {
+                            s0 = prod_direct<KS>(Ks + (cur ^ 1) * kTileB, 0, qf, l32, lh);
+                            p0 = prod_direct<KS>(Vs + (cur ^ 1) * kTileB, 0, gf, l32, lh);
+                        }
+                    }
+                    it0 = nfull;
+                }
+            }
+            for (int it = it0; it < niter; it++) {
                 const int jt = 2 * it + g, cur = it & 1;
                 const bool nxt = jt + 2 < njt;
                 if (nxt) {

@@ -751,10 +751,10 @@ def test_fused_attention(ops, oracle, S, H, Dh):
 # Edges of the kernels of 32 rows per workgroup (attention_short.hip): of their blocks of 32 (a single position, one short of, on
 # and one past it), of what 4 and 8 waves split (128, 256), of the forms by length (1024, 2048) and by workgroups on 256 CUs (256,
 # 512; 768 and 1024 forward), and of the adjoint's other half (2048, 2 of 128: dK, dV in parts; 2080, 4 of 64: no forward; the
-# last ones: forward only, and neither); windows, rows longer than the heads, accumulation
+# last ones: forward only, neither, and neither with 128 rows of dQ a workgroup, heads to 64); windows, rows longer than the heads, accumulation
 SHORT_SHAPES = [(1, 1, 8, 0), (31, 2, 100, 0), (32, 1, 64, 24), (33, 4, 60, 0), (127, 1, 128, 0), (129, 3, 64, 0), (255, 2, 68, 8),
                 (257, 1, 32, 0), (512, 16, 100, 0), (513, 16, 64, 0), (1023, 2, 12, 0), (1024, 8, 64, 0), (1025, 2, 128, 0), (2047, 8, 64, 0),
-                (2048, 2, 128, 8), (2080, 4, 64, 0), (97, 192, 12, 0), (128, 256, 72, 0), (128, 257, 72, 0)]
+                (2048, 2, 128, 8), (2080, 4, 64, 0), (97, 192, 12, 0), (128, 256, 72, 0), (128, 257, 72, 0), (700, 48, 64, 0)]
 
 
 @pytest.mark.gpu
