@@ -723,10 +723,10 @@ __global__ void __launch_bounds__(kNT2, 2) attn_bwd_dq_kernel(AttnArgs p)
             for (int ks = 0; ks < (FAST ? KS : 1); ks++)
 #pragma unroll
                 for (int e = 0; e < 8; e++) part = __builtin_fmaf((float)gf[ks][e], (float)of[ks][e], part);
-            sig = part + __shfl_xor(part, 32, 64);                     // the two lanes of a row
+            sig = with32(part, OpSum());                     // the two lanes of a row
         } else {
             const float part = run_pass(std::integral_constant<int, 0>{});
-            const float pg = part + __shfl_xor(part, 32, 64);         // the two lanes of a row, then the waves that hold it
+            const float pg = with32(part, OpSum());         // the two lanes of a row, then the waves that hold it
             if (lh == 0) xs[ws.part * QR + qrow] = pg;
             __syncthreads();
             sig = xs[qrow];

@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_short_fwd_kernel(AttnArgs p)
     });
     // the row's maximum and sum over the wave's keys, then over the waves
     float m = (float)__builtin_fmaxf16(mx[0], mx[1]), l = 0.f;
-    m = fmaxf(m, __shfl_xor(m, 32, 64));
+    m = with32(m, OpMax());
     const float c = m * kLog2e;
     static_for<0, NB>([&](auto j_c) __attribute__((always_inline)) {
         constexpr int j = decltype(j_c)::value;
@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_short_fwd_kernel(AttnArgs p)
             }
         }
     });
-    l += __shfl_xor(l, 32, 64);
+    l = with32(l, OpSum());
     if (lh == 0) {
         xs[(wid * 2 + 0) * kBlk + l32] = m;
         xs[(wid * 2 + 1) * kBlk + l32] = l;
@@ -359,14 +359,14 @@ __global__ void __launch_bounds__(512, 2) attn_short_dq_kernel(AttnArgs p)
         for (int ks = 0; ks < KS; ks++)
 #pragma unroll
             for (int e = 0; e < 8; e++) part = __builtin_fmaf((float)gf[ks][e], (float)of[ks][e], part);
-        sig = part + __shfl_xor(part, 32, 64);
+        sig = with32(part, OpSum());
     } else {
         float part = run_pass(std::integral_constant<int, 0>{});
         if (n > 0) {
             issue(p.v, Vs, 0);
             issue(p.k, Ks, 0);
         }
-        part += __shfl_xor(part, 32, 64);
+        part = with32(part, OpSum());
         if (lh == 0) xs[wid * kBlk + l32] = part;
         __syncthreads();
         sig = xs[l32];

@@ -229,11 +229,10 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             float a = acc[t][i];
-            if (LP <= 2) a += __shfl_xor(a, 2, 64);
-            if (LP <= 4) a += __shfl_xor(a, 4, 64);
-            a += __shfl_xor(a, 8, 64);
-            a += swz_xor16(a);
-            a += xor32(a);
+            if (LP <= 2) a += dpp<0x4E>(a);                 // lane ^ 2
+            if (LP <= 4) a += dpp<0x1B>(dpp<0x141>(a));     // lane ^ 7 ^ 3
+            a += dpp<0x128>(a);                             // row_ror 8: lane ^ 8
+            a = with32(with16(a, OpSum()), OpSum());
             if (lane < LP) red[wid][t][lane][i] = a;
         }
     __syncthreads();

@@ -320,8 +320,8 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
         }
         if (EPI == E_PLAIN && p.cand) {
             uint32_t k = n0 + r < p.N ? arg_key(f2h(p.alpha * v[0]), n0 + r) : 0u;
-            k = max(k, (uint32_t)__shfl_xor((int)k, 1, 64));
-            k = max(k, (uint32_t)__shfl_xor((int)k, 2, 64));
+            k = max(k, dpp<0xB1>(k));
+            k = max(k, dpp<0x4E>(k));
             if (r == 0) p.cand[(int64_t)m * gridDim.x + blockIdx.x] = k;
         }
         if (n0 + r < p.N) {
@@ -348,8 +348,7 @@ finish_rows_kernel(int M, int count, const uint32_t *__restrict__ cand, uint16_t
     for (int m = 0; m < M; m++) {
         uint32_t k = 0;
         for (int i = threadIdx.x; i < count; i += 1024) k = max(k, cand[(int64_t)m * count + i]);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) k = max(k, (uint32_t)__shfl_xor((int)k, off, 64));
+        k = wave_reduce(k, [](uint32_t a, uint32_t b) { return max(a, b); });
         __syncthreads();
         if ((threadIdx.x & 63) == 0) best[threadIdx.x >> 6] = k;
         __syncthreads();
