@@ -22,7 +22,7 @@
 // with clamped indices: a load inside a branch is waited for at the end of the branch.
 // Eight lanes throughout and V first -> now, us: one row, 16 heads of 128, 200 / 480 / 1540 / 4000 positions 5.7 / 6.8 /
 // 10.7 / 18.5 -> 5.0 / 6.1 / 8.9 / 15.4; 32 heads of 100 6.5 / 9.3 / 16.2 / 31.6 -> 5.6 / 7.2 / 12.5 / 23.0; four rows of
-// 16 x 128 10.9 / 13.3 / 20.1 / 35.7 -> 10.4 / 12.6 / 16.9 / 26.7.
+// 16 x 128 10.9 / 13.3 / 20.1 / 35.7 -> 10.4 / 12.6 / 16.9 / 26.7 (before the exponentials were held by the lanes).
 #include "common.h"
 #include "softmax_math.h"
 
@@ -164,26 +164,48 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
         load_v(vv, 0);
     }
     __syncthreads();
-    // row maxima, then sums of exponentials, then the probabilities in place of the scores; row t sees live(t) positions
+    // position tid + k NT of row t, k < KMAX: its score, then its exponential, held by the lane.  They cover a whole row of own
+    // scores and one of 2048 positions; behind them the scores are read again and the exponentials formed twice, as they were
+    // everywhere: 1540 positions of 16 heads of 128 6.2 -> 5.0 us, 2000 of 32 of 100 9.1 -> 7.8, 70 4.5 -> 4.2, four rows of 16 of
+    // 128 over 200 11.0 -> 9.0.  (All that a row can have held is code that a launch fetches in vain: 700 positions of 32 heads
+    // of 100 5.0 -> 5.8 us; with four 4.4.)
+    constexpr int KMAX = !OWN ? 4 : NT == kThreads ? 1 : 2;
+    static_assert(!OWN || (NT == kThreads ? kNarrow : kOwnScoresShort) <= KMAX * NT, "a row's own scores in registers");
+    float e[T][KMAX], m[T], sum[T];
     auto live = [&](int t) __attribute__((always_inline)) { return (int)min((int64_t)C, (int64_t)t + row0 + 1); };
-    float mx[T], sum[T];
+    auto more = [&](int t, int end, auto &&f) __attribute__((always_inline)) {
+        if constexpr (!OWN)
+            for (int j = tid + KMAX * NT; j < end; j += NT) f(sp + t * ld + j, j);
+    };
+    // row maxima, then sums of exponentials, then the probabilities; row t sees live(t) positions
 #pragma unroll
     for (int t = 0; t < T; t++) {
-        float m = -INFINITY;
-        for (int j = tid; j < live(t); j += NT) m = fmaxf(m, h2f(sp[t * ld + j]));
-        m = wave_max(m);
-        if (lane == 0) scratch[0][t][wid] = m;
+        m[t] = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < KMAX; k++) {
+            const int j = tid + k * NT;
+            e[t][k] = h2f(sp[t * ld + min(j, C - 1)]);
+            if (j < live(t)) m[t] = fmaxf(m[t], e[t][k]);
+        }
+        more(t, live(t), [&](half_t *s, int) __attribute__((always_inline)) { m[t] = fmaxf(m[t], h2f(*s)); });
+        m[t] = wave_max(m[t]);
+        if (lane == 0) scratch[0][t][wid] = m[t];
     }
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < T; t++) {
-        mx[t] = scratch[0][t][0];
+        m[t] = scratch[0][t][0];
 #pragma unroll
-        for (int w = 1; w < NT / 64; w++) mx[t] = fmaxf(mx[t], scratch[0][t][w]);
-        float s = 0.f;
-        for (int j = tid; j < live(t); j += NT) s += exp_nonpos(fmaxf(h2f(sp[t * ld + j]) - mx[t], -100.0f));
-        s = wave_sum(s);
-        if (lane == 0) scratch[1][t][wid] = s;
+        for (int w = 1; w < NT / 64; w++) m[t] = fmaxf(m[t], scratch[0][t][w]);
+        sum[t] = 0.f;
+#pragma unroll
+        for (int k = 0; k < KMAX; k++) {
+            e[t][k] = exp_nonpos(fmaxf(e[t][k] - m[t], -100.0f));
+            if (tid + k * NT < live(t)) sum[t] += e[t][k];
+        }
+        more(t, live(t), [&](half_t *s, int) __attribute__((always_inline)) { sum[t] += exp_nonpos(fmaxf(h2f(*s) - m[t], -100.0f)); });
+        sum[t] = wave_sum(sum[t]);
+        if (lane == 0) scratch[1][t][wid] = sum[t];
     }
     __syncthreads();
 #pragma unroll
@@ -192,10 +214,14 @@ decode_values_kernel(int C, int Dh, int64_t row0, float alpha, const half_t *__r
 #pragma unroll
         for (int w = 1; w < NT / 64; w++) sum[t] += scratch[1][t][w];
         const RowDivide div(sum[t]);
-        for (int j = tid; j < C; j += NT) {
-            const float e = exp_nonpos(fmaxf(h2f(sp[t * ld + j]) - mx[t], -100.0f));
-            sp[t * ld + j] = j < live(t) ? f2h(div(e)) : (half_t)0.f;
+#pragma unroll
+        for (int k = 0; k < KMAX; k++) {
+            const int j = tid + k * NT;
+            if (j < C) sp[t * ld + j] = j < live(t) ? f2h(div(e[t][k])) : (half_t)0.f;
         }
+        more(t, C, [&](half_t *s, int j) __attribute__((always_inline)) {
+            *s = j < live(t) ? f2h(div(exp_nonpos(fmaxf(h2f(*s) - m[t], -100.0f)))) : (half_t)0.f;
+        });
     }
     __syncthreads();
     float acc[T][4];
