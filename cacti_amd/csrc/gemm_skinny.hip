@@ -74,21 +74,6 @@ __device__ __forceinline__ uint32_t arg_key(half_t v, int64_t n)
     return o << 16 | (uint32_t)(0xffff - n);
 }
 
-template <int W>
-__device__ __forceinline__ float block_sum(float v, float *scratch)
-{
-    v = wave_sum(v);
-    if (W == 1) return v;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) scratch[wid] = v;
-    __syncthreads();
-    float r = scratch[0];
-#pragma unroll
-    for (int w = 1; w < W; w++) r += scratch[w];
-    return r;
-}
-
 // sum of 8 products, fp32 accumulate: four v_dot2_f32_f16 (no conversions, two products each)
 __device__ __forceinline__ float dot8(const half8_t &a, const half8_t &b, float acc)
 {
@@ -118,7 +103,7 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
     constexpr bool GATE = EPI == E_GATE;
     constexpr int NB = GATE ? 2 : 1;
     __shared__ float part[W][NB * M * kRows];
-    __shared__ float scratch[W];
+    __shared__ float scratch[M][W];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int64_t n0 = (int64_t)blockIdx.x * kRows;
     float acc[NB][M][kRows];
@@ -223,10 +208,11 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
         }
         if (NORM) __builtin_amdgcn_sched_barrier(0);
         if (NORM) {
-            // the whole row is in this one batch (K <= 8 * kPre * kThreads, seen to by the launcher)
+            // the whole row is in this one batch (K <= 8 * kPre * kThreads, seen to by the launcher); one barrier for all rows
+            float ss[M];
 #pragma unroll
             for (int m = 0; m < M; m++) {
-                float ss = 0.f;
+                ss[m] = 0.f;
 #pragma unroll
                 for (int j = 0; j < kPre; j++) {
                     const int64_t c = base + j * kThreads + tid;
@@ -239,12 +225,25 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
 #pragma unroll
                         for (int i = 0; i < 8; i++) {
                             const float f = h2f(a[j][m].v[i]);
-                            ss += f * f;
+                            ss[m] += f * f;
                         }
                     }
                 }
-                ss = block_sum<W>(ss, scratch);
-                const float rinv = 1.0f / sqrtf(ss / (float)p.K + p.eps);
+                ss[m] = wave_sum(ss[m]);
+                if (W > 1 && lane == 0) scratch[m][wid] = ss[m];
+            }
+            if (W > 1) {
+                __syncthreads();
+#pragma unroll
+                for (int m = 0; m < M; m++) {
+                    ss[m] = scratch[m][0];
+#pragma unroll
+                    for (int w = 1; w < W; w++) ss[m] += scratch[m][w];
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                const float rinv = 1.0f / sqrtf(ss[m] / (float)p.K + p.eps);
 #pragma unroll
                 for (int j = 0; j < kPre; j++) {
                     const int64_t c = base + j * kThreads + tid;
@@ -285,21 +284,16 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
     if (EPI == E_QKV) {
         // rotate (queries, keys) and add to the caches (keys, values) with the rounding points of
         // the separate thunks: y = f16(f16(x cos) + f16(rot(x) sin)), cache = f16(cache + y)
-        __shared__ float xr[M][kRows];
         const int m = tid / kRows, r = tid % kRows;
         if (tid < M * kRows) {
             float v = 0.f;
 #pragma unroll
             for (int w = 0; w < W; w++) v += part[w][m * kRows + r];
-            xr[m][r] = rnd16(p.alpha * v);
-        }
-        __syncthreads();
-        if (tid < M * kRows) {
-            float y = xr[m][r];
+            float y = rnd16(p.alpha * v);
             if (blockIdx.y < 2) {
-                const bool left = r < kRows / 2;
-                const float xp = xr[m][left ? r + kRows / 2 : r - kRows / 2];
-                y = rnd16(rnd16(y * h2f(ecos)) + rnd16((left ? -xp : xp) * h2f(esin)));
+                static_assert(kRows == 4, "a column's partner is lane ^ 2");
+                const float xp = dpp<0x4E>(y);
+                y = rnd16(rnd16(y * h2f(ecos)) + rnd16((r < kRows / 2 ? -xp : xp) * h2f(esin)));
             }
             if (blockIdx.y == 0) {
                 p.C[m * p.ldc + ecol] = f2h(y);
