@@ -34,7 +34,8 @@ int gather_to_host(Staging &s, const HostRegion *r, int n, hipStream_t st);
 // through `own`, the caller's, which no other reader waits for or takes; beyond through a borrowed window.  Readers on
 // other threads and streams go on meanwhile.
 int read_large(Staging &own, void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st);
-constexpr size_t kLargeRead = 192u << 10;      // from here on it is the better one
+constexpr size_t kLargeRead = 192u << 10;      // from here on it is the better one where there is something else to gather,
+constexpr size_t kLargeAlone = 96u << 10;      // and from here on where there is not
 constexpr size_t kOwnRead = 512u << 10;
 static_assert(kOwnRead <= kStagingBytes - Staging::kFlagBytes, "a context's buffer holds it");
 // n regions of `bytes` (a multiple of 16), 16-byte aligned, set to zero

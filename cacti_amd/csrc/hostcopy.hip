@@ -177,8 +177,8 @@ void settle(Staging &s, hipStream_t st)
 
 // a large read's buffer: a word per chunk, at the end of their place the word that is read with it (a gather's words, in the
 // same buffer, do not reach there), then the window of chunks
-constexpr size_t kWindow = kWindowBytes - Staging::kFlagBytes, kLeastChunk = 32u << 10, kWordPlace = Staging::kFlagBytes - 64;
-static_assert(kWindow / kLeastChunk * sizeof(unsigned) <= kWordPlace && kFlagsPerGather * sizeof(unsigned) <= kWordPlace,
+constexpr size_t kWindow = kWindowBytes - Staging::kFlagBytes, kLeastChunk = 16u << 10, kWordPlace = Staging::kFlagBytes - 64;
+static_assert((1u << 20) / kLeastChunk * sizeof(unsigned) <= kWordPlace && kWindow / (2 * kLeastChunk) * sizeof(unsigned) <= kWordPlace && kFlagsPerGather * sizeof(unsigned) <= kWordPlace,
               "a word per chunk");
 constexpr int kStreamBlocks = 16;
 
@@ -205,7 +205,7 @@ static int read_windows(Staging &s, void *dst, const void *src, size_t bytes, co
     int dev = 0;
     CACTI_HIP(hipGetDevice(&dev));
     for (size_t done = 0; done < bytes;) {
-        const size_t window = std::min(bytes - done, s.room()), chunk = window < (4u << 20) ? kLeastChunk : 2 * kLeastChunk;
+        const size_t window = std::min(bytes - done, s.room()), chunk = window <= (1u << 20) ? kLeastChunk : window < (4u << 20) ? 2 * kLeastChunk : 4 * kLeastChunk;
         const int chunks = (int)((window + chunk - 1) / chunk), threads = (int)std::min<size_t>(kCopyThreads, 1 + window / (4u << 20));
         if (++s.epoch == 0) s.epoch = 1;
         const unsigned epoch = s.epoch;
@@ -231,7 +231,9 @@ static int read_windows(Staging &s, void *dst, const void *src, size_t bytes, co
 // Measured, us, one gather and one copy behind it / 1 MiB pieces before -> chunks: 2 MiB 119 -> 76, 20 MiB 569 -> 473.  A
 // helper thread costs some 10 us to start: worth it from several MiB on, where the copying host (12 .. 30 GB/s) and not
 // the link (52) is what one thread would wait for.  One gather and one copy behind it against chunks, since the chunks are
-// announced without a fence: 128 KiB 15.3 and 15.7, 344 KiB 24.4 and 22.3, 512 KiB 30.2 and 29.6.
+// announced without a fence: 128 KiB 15.3 and 15.7, 344 KiB 24.4 and 22.3, 512 KiB 30.2 and 29.6.  Up to 1 MiB in chunks of
+// 16 KiB, so that the 16 workgroups have some one after another and the host a copy to make meanwhile: 128 KiB (one gather
+// before) 14.4 -> 13.6, 512 KiB 29.0 -> 25.7; in chunks of 8 KiB 15.3 and 27.2, by 32 workgroups 13.6 and 30.2.
 int read_large(Staging &own, void *dst, const void *src, size_t bytes, const int *word, int *word_dst, hipStream_t st)
 {
     if (own.base && !own.lost && bytes <= kOwnRead) return read_windows(own, dst, src, bytes, word, word_dst, st);

@@ -391,7 +391,7 @@ int Ctx::cell_get(CellPtr ci, void *host, size_t bytes)
             c.v_ready = nullptr;
         }
         int rc;
-        if (staging_.base && bytes <= kLargeRead) {
+        if (staging_.base && bytes <= kLargeAlone) {
             const HostRegion r = {dev_ptr(c.voff), staging_.data(), bytes};
             rc = gather_to_host(staging_, &r, 1, stream_);
             if (!rc) memcpy(host, staging_.data(), bytes);
