@@ -148,7 +148,9 @@ constexpr int kCeThreads = 1024;
 // The row lives in registers as fp32 (CH x 8 values per lane); chunks past the row hold -inf, and
 // differences from the maximum below -100 contribute nothing to an fp32 sum that is at least 1.
 // The kernels are bound by their arithmetic as much as by HBM (per element: convert, maximum,
-// exponential, sum, quotient, one-hot, scale, round), hence exp_nonpos and RowDivide.
+// exponential, sum, quotient, one-hot, scale, round), hence exp_nonpos and RowDivide, and nothing per element that one lane of a
+// row has a use for (the place of the maximum, the label): 2048 x 32000 forward 56.6 -> 41.2 us (3.2 TB/s),
+// adjoint 66.2 -> 55.5 (4.7 TB/s).
 template <int CH>
 struct CeRow {
     float e[CH][8];
@@ -162,12 +164,15 @@ struct CeRow {
         float mx = -INFINITY;
 #pragma unroll
         for (int c = 0; c < CH; c++) {
-            const bool valid = c * kCeThreads + (int)threadIdx.x < nchunk;
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
-                e[c][k] = valid ? h2f(raw[c].v[k]) : -INFINITY;
-                mx = fmaxf(mx, e[c][k]);
+            for (int k = 0; k < 8; k++) e[c][k] = h2f(raw[c].v[k]);
+            if ((c + 1) * kCeThreads > nchunk) {               // uniform: the last chunks alone
+                const bool valid = c * kCeThreads + (int)threadIdx.x < nchunk;
+#pragma unroll
+                for (int k = 0; k < 8; k++) e[c][k] = valid ? e[c][k] : -INFINITY;
             }
+#pragma unroll
+            for (int k = 0; k < 8; k++) mx = fmaxf(mx, e[c][k]);
         }
         return mx;
     }
@@ -194,7 +199,7 @@ softmax_ce_fwd_kernel(int64_t N, int V, const half_t *__restrict__ logit,
                       float *__restrict__ loss, uint16_t *__restrict__ amax, int *status)
 {
     __shared__ float red[16];
-    __shared__ float xt_s;
+    __shared__ unsigned at;
     const int64_t n = blockIdx.x;
     const int nchunk = V / 8;
     const int t = tok ? (int)tok[n] : 0;
@@ -202,36 +207,26 @@ softmax_ce_fwd_kernel(int64_t N, int V, const half_t *__restrict__ logit,
         if (threadIdx.x == 0 && status) atomicMax(status, (int)n + 1);
         return;                                    // uniform for the block
     }
+    const float xt = loss ? h2f(logit[n * V + t]) : 0.f;       // the label's logit
+    if (threadIdx.x == 0) at = ~0u;                            // (the maximum's barriers stand between this and its use)
     CeRow<CH> row;
-    const float mx = block_reduce(row.load_max(logit + n * V, nchunk), OpMax(), -INFINITY, red);
-    if (amax) {
-        // first index holding the maximum
-        float best = 3.0e38f;
+    const float lane_mx = row.load_max(logit + n * V, nchunk);
+    const float mx = block_reduce(lane_mx, OpMax(), -INFINITY, red);
+    if (amax && lane_mx == mx) {
+        // the first index holding the maximum, looked for by the lanes that hold it
+        unsigned best = ~0u;
 #pragma unroll
-        for (int c = 0; c < CH; c++) {
-            const int ch = c * kCeThreads + threadIdx.x;
+        for (int c = CH - 1; c >= 0; c--) {
+            const unsigned first = (c * kCeThreads + threadIdx.x) * 8;
 #pragma unroll
-            for (int k = 0; k < 8; k++)
-                if (row.e[c][k] == mx) best = fminf(best, (float)(ch * 8 + k));
+            for (int k = 7; k >= 0; k--)
+                if (row.e[c][k] == mx) best = first + k;
         }
-        best = -block_reduce(-best, OpMax(), -3.0e38f, red);
-        if (threadIdx.x == 0) amax[n] = (uint16_t)best;
+        atomicMin(&at, best);
     }
-    if (loss) {
-        // the label's logit: selected in a register, stored by the one lane that holds it
-        float xt = 0.f;
-        bool mine = false;
-#pragma unroll
-        for (int c = 0; c < CH; c++) {
-            const int ch = c * kCeThreads + threadIdx.x;
-            mine = mine || ch == (t >> 3);
-#pragma unroll
-            for (int k = 0; k < 8; k++) xt = (ch * 8 + k == t) ? row.e[c][k] : xt;
-        }
-        if (mine) xt_s = xt;
-    }
-    const float sum = block_reduce(row.exp_sum(mx), OpSum(), 0.f, red);     // barriers inside publish xt_s
-    if (loss && threadIdx.x == 0) loss[n] = -logf(expf(xt_s - mx) / sum);
+    const float sum = block_reduce(row.exp_sum(mx), OpSum(), 0.f, red);     // barriers inside publish `at`
+    if (amax && threadIdx.x == 0) amax[n] = (uint16_t)at;
+    if (loss && threadIdx.x == 0) loss[n] = -logf(expf(xt - mx) / sum);
     if (prob) {
         float *pr = prob + n * V;
         const RowDivide div(sum);
@@ -274,13 +269,16 @@ softmax_ce_bwd_kernel(int64_t N, int V, const half_t *__restrict__ logit,
             // loaded here, not with the row: the accumulating form runs once per cycle at most (the
             // first write of dlogit overwrites)
             if (acc) old = ld8(dr + ch * 8);
+            float d[8];
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
-                float p = div(row.e[c][k]);
-                float z = p - ((ch * 8 + k == t) ? 1.0f : 0.0f);
-                float d = sc * z;
-                o.v[k] = acc ? f2h(h2f(old.v[k]) + rnd16(d)) : f2h(d);
+            for (int k = 0; k < 8; k++) d[k] = sc * div(row.e[c][k]);
+            if (ch == t >> 3) {                                  // one lane of the row
+#pragma unroll
+                for (int k = 0; k < 8; k++)
+                    if (k == (t & 7)) d[k] = sc * (div(row.e[c][k]) - 1.0f);
             }
+#pragma unroll
+            for (int k = 0; k < 8; k++) o.v[k] = acc ? f2h(h2f(old.v[k]) + rnd16(d[k])) : f2h(d[k]);
             st8(dr + ch * 8, o);
         }
     }

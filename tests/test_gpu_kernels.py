@@ -205,6 +205,31 @@ def test_softmax_ce(ops, oracle, N, V):
     assert_parity(ga, oracle.accumulate_f16(d0, wd), "dlogit+")
 
 
+# the label and the maximum are one lane's business each: in a row's first and last element, on both sides of a lane's eight, of
+# the block's 8192 and of the row's last, partly filled round; the maximum twice, the later one in another lane, wave and round;
+# a row of one value, of -infinity but for one
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [8, 64, 1000, 8192, 8200, 16384, 24576, 32000])
+def test_softmax_ce_places_of_label_and_maximum(ops, oracle, V):
+    say("softmax_ce places", V)
+    places = sorted({p for p in (0, 7, 8, 511, 512, 8191, 8192, 8199, V - 8, V - 1) if 0 <= p < V})
+    N = 2 * len(places) + 2
+    r = rng(660 + V)
+    logit, tok = randn16(r, (N, V)), np.zeros(N, np.uint16)
+    for i, p in enumerate(places):
+        tok[i], tok[len(places) + i] = p, places[-1 - i]
+        logit[i, p] = logit[len(places) + i, p] = logit[len(places) + i, V - 1] = 9.0
+    logit[-2], logit[-1], logit[-1, V // 2] = 1.5, -np.inf, 0.25
+    tok[-2:] = V - 1, V // 2
+    wprob, wloss, wamax = oracle.softmax_ce_fwd(logit, tok)
+    gprob, gloss, gamax = ops.softmax_ce_fwd(dev(logit), dev(tok))
+    assert (host(gamax).view(np.uint16) == wamax).all() and wamax[-2] == 0
+    assert_parity(host(gprob), wprob, "prob", l2=1e-5, mx=1e-4)
+    assert_parity(host(gloss), wloss, "loss", l2=1e-5, mx=1e-4)
+    scale = np.linspace(0.5, 2, N).astype(np.float32)
+    assert_parity(host(ops.softmax_ce_bwd(dev(logit), dev(tok), dev(scale))), oracle.softmax_ce_bwd(logit, tok, scale), "dlogit")
+
+
 def test_softmax_ce_argmax_ties_and_bad_token(ops, oracle):
     logit = np.zeros((2, 64), np.float16)
     logit[0, [9, 40]] = 2.0
