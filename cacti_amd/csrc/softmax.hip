@@ -269,16 +269,18 @@ softmax_ce_bwd_kernel(int64_t N, int V, const half_t *__restrict__ logit,
             // loaded here, not with the row: the accumulating form runs once per cycle at most (the
             // first write of dlogit overwrites)
             if (acc) old = ld8(dr + ch * 8);
-            float d[8];
+            float z[8];                                          // softmax - one_hot
 #pragma unroll
-            for (int k = 0; k < 8; k++) d[k] = sc * div(row.e[c][k]);
+            for (int k = 0; k < 8; k++) z[k] = div(row.e[c][k]);
             if (ch == t >> 3) {                                  // one lane of the row
 #pragma unroll
-                for (int k = 0; k < 8; k++)
-                    if (k == (t & 7)) d[k] = sc * (div(row.e[c][k]) - 1.0f);
+                for (int k = 0; k < 8; k++) z[k] = k == (t & 7) ? z[k] - 1.0f : z[k];
             }
 #pragma unroll
-            for (int k = 0; k < 8; k++) o.v[k] = acc ? f2h(h2f(old.v[k]) + rnd16(d[k])) : f2h(d[k]);
+            for (int k = 0; k < 8; k++) {
+                const float d = sc * z[k];
+                o.v[k] = acc ? f2h(h2f(old.v[k]) + rnd16(d)) : f2h(d);
+            }
             st8(dr + ch * 8, o);
         }
     }
