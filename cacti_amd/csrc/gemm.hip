@@ -513,6 +513,53 @@ CACTI_API int cacti_hip_gemm_f16_chain(int64_t n, int64_t M, int64_t N, int64_t 
     return 0;
 }
 
+static GemmPlan pair_plan(int64_t n, int64_t S, int64_t N, int64_t K)
+{
+    const bool fits = n >= 1 && n <= kMaxPtrBatch && S > 0 && N > 0 && K > 0 && mult(N, n > 1 ? 64 : 8) && (n == 1 || N >= 4 * 64) &&
+                      mult(K, 8) && N < kMaxPitch && K < kMaxPitch;
+    return fits ? gemm_plan_pair(S, N, K, (int)n) : GemmPlan{-1, 0, 0, 1, 0};
+}
+
+CACTI_API int cacti_hip_gemm_f16_grads_one_launch(int64_t n, int64_t S, int64_t N, int64_t K) { return pair_plan(n, S, N, K).tile >= 0 ? 1 : 0; }
+
+CACTI_API int cacti_hip_gemm_f16_grads(int64_t n, int64_t S, int64_t N, int64_t K, const void *const *dy, const void *const *W, const void *x,
+                                       float beta_x, void *dx, float beta_w, void *const *dW, void *stream)
+{
+    CACTI_REQUIRE(n > 0 && dy && W && dW && x && dx, CACTI_E_INVALID, "gemm_grads: null pointer or no product");
+    for (int64_t z = 0; z < n; z++)
+        CACTI_REQUIRE(dy[z] && W[z] && dW[z], CACTI_E_INVALID, "gemm_grads: null operand in product %lld", (long long)z);
+    CACTI_REQUIRE((beta_x == 0.f || beta_x == 1.f) && (beta_w == 0.f || beta_w == 1.f), CACTI_E_INVALID, "gemm_grads: beta must be 0 or 1");
+    const GemmPlan plan = pair_plan(n, S, N, K);
+    bool one = plan.tile >= 0 && (n == 1 || beta_x == 0.f) && aligned(x, 16) && aligned(dx, 16);
+    for (int64_t z = 0; z < n && one; z++) one = aligned(dy[z], 16) && aligned(W[z], 16) && aligned(dW[z], 16);
+    if (!one) {
+        for (int64_t z = 0; z < n; z += kMaxPtrBatch) {
+            const void *xs[kMaxPtrBatch] = {x, x, x, x};
+            const int rc = cacti_hip_gemm_f16_batched(1, 0, n - z < kMaxPtrBatch ? n - z : kMaxPtrBatch, N, K, S, 1.f, dy + z, N, xs, K, beta_w,
+                                                      dW + z, K, stream);
+            if (rc) return rc;
+        }
+        return cacti_hip_gemm_f16_chain(n, S, K, N, dy, N, W, K, beta_x, dx, K, stream);
+    }
+    GemmArgs nn = {}, tn = {};
+    nn.M = S; nn.N = K; nn.K = N; nn.alpha = 1.f; nn.beta = beta_x;
+    nn.A = (const half_t *)dy[0]; nn.lda = N;
+    nn.B = (const half_t *)W[0]; nn.ldb = K;
+    nn.C = (half_t *)dx; nn.ldc = K;
+    nn.chain = (int)n;
+    tn.M = N; tn.N = K; tn.K = S; tn.alpha = 1.f; tn.beta = beta_w;
+    tn.A = (const half_t *)dy[0]; tn.lda = N;
+    tn.B = (const half_t *)x; tn.ldb = K;
+    tn.C = (half_t *)dW[0]; tn.ldc = K;
+    tn.ztab = n > 1;
+    for (int64_t z = 0; z < n; z++) {
+        nn.za[z] = tn.za[z] = (const half_t *)dy[z] - nn.A;
+        nn.zb[z] = (const half_t *)W[z] - nn.B;
+        tn.zc[z] = (half_t *)dW[z] - tn.C;
+    }
+    return gemm_pair_launch(nn, tn, n, plan, (hipStream_t)stream);
+}
+
 CACTI_API int cacti_hip_gemm_f16_strided_batched(int ta, int tb, int64_t nblk, int64_t M, int64_t N,
                                                  int64_t K, float alpha, const void *A, int64_t lda,
                                                  int64_t stride_a, const void *B, int64_t ldb,

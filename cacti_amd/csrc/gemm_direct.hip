@@ -97,7 +97,7 @@ __device__ __forceinline__ void load_odd(half_t *lds, const half_t *c, int64_t l
 // with 64 x 64, 5.7 with 160 x 192), the sum's way through memory and the gap between them: three of 611 x 1024 x 1024 21.0 ->
 // 14.2 us, of 777 x 2048 x 2048 41.0 -> 31.6, of 2048 x 3200 x 3200 132 -> 114; two of 2048 x 3200 x 8640 199 -> 195.
 template <bool TA, bool TB, int BM, int BN, int RES, bool M32, bool ANY, bool CHAIN>
-__device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p)
+__device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
 {
     // the whole argument block in scalar registers before anything else: read field by field where the control
     // flow first wants it, it costs five dependent round trips to memory before the first operand load
@@ -116,7 +116,7 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p)
     half_t *Bs = As + NBA * BM * BK;                              // [NBB][BN * BK]
 
     int tm, tn, bz;
-    p.walk.locate(blockIdx.x, tm, tn, bz);
+    p.walk.locate(wg, tm, tn, bz);
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
     int nk = (int)((p.K + BK - 1) / BK), kt0 = 0;
     const int product = nk;                                       // CHAIN: k tiles of one
@@ -612,12 +612,31 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p)
 template <bool TA, bool TB, int BM, int BN, int RES, bool M32, bool ANY>
 __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
 {
-    gemm_direct_tile<TA, TB, BM, BN, RES, M32, ANY, false>(p);
+    gemm_direct_tile<TA, TB, BM, BN, RES, M32, ANY, false>(p, blockIdx.x);
 }
 template <int BM, int BN, int RES, bool M32>
 __global__ void __launch_bounds__(256, RES) gemm_chain_kernel(GemmArgs p)
 {
-    gemm_direct_tile<false, false, BM, BN, RES, M32, false, true>(p);
+    gemm_direct_tile<false, false, BM, BN, RES, M32, false, true>(p, blockIdx.x);
+}
+// Two products that wait for nothing of each other, in one launch: a gradient of the inputs (NN, of a chain perhaps) and those of
+// the weights (TN).  The one with the longer sums has the first workgroups, so that none of them begins when the others end; the
+// other's begin at a number that keeps their XCDs.
+struct PairArgs {
+    GemmArgs nn, tn;
+    uint32_t second;
+    int tn_first;
+};
+template <int BM, int BN, int RES, bool M32, bool CHAIN>
+__global__ void __launch_bounds__(256, RES) gemm_pair_kernel(PairArgs p)
+{
+    const bool first = blockIdx.x < p.second;
+    const uint32_t wg = first ? blockIdx.x : blockIdx.x - p.second;
+    if (first == (p.tn_first != 0)) {
+        if (wg < (uint32_t)p.tn.walk.wgs) gemm_direct_tile<true, false, BM, BN, RES, M32, false, false>(p.tn, wg);
+    } else {
+        if (wg < (uint32_t)p.nn.walk.wgs) gemm_direct_tile<false, false, BM, BN, RES, M32, false, CHAIN>(p.nn, wg);
+    }
 }
 
 // C = f16(alpha sum of the parts + beta C), four columns per lane; the parts are added in order.  VEC: N and the rows
@@ -735,6 +754,37 @@ constexpr Shape kShapes[] = {
 constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
 constexpr int kChainShapes = kNumShapes - 2;      // of the last two a lane has no registers for a second sum
 constexpr int T64 = 0, T64_SMALL = kNumShapes;   // T64_SMALL: 64 x 64 with M32
+
+template <int SHAPE>
+int launch_pair(const PairArgs &args, int64_t nblk, hipStream_t st)
+{
+    constexpr bool M32 = SHAPE == T64_SMALL;
+    constexpr Shape t = kShapes[M32 ? T64 : SHAPE];
+    constexpr size_t smem = (size_t)(buffers(t.bm, t.bn, t.res) * (t.bm + t.bn) + (t.bm < t.bn ? t.bm : t.bn)) * BK * sizeof(half_t);
+    PairArgs p = args;
+    auto kern = p.nn.chain > 1 ? gemm_pair_kernel<t.bm, t.bn, t.res, M32, true> : gemm_pair_kernel<t.bm, t.bn, t.res, M32, false>;
+    static DeviceOnce attr_set;
+    if (!attr_set.fresh()) {
+        CACTI_HIP(hipFuncSetAttribute((const void *)gemm_pair_kernel<t.bm, t.bn, t.res, M32, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+        CACTI_HIP(hipFuncSetAttribute((const void *)gemm_pair_kernel<t.bm, t.bn, t.res, M32, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+        attr_set.mark();
+    }
+    auto set = [&](GemmArgs &g, int64_t n) {
+        const int tiles_m = (int)((g.M + t.bm - 1) / t.bm), tiles_n = (int)((g.N + t.bn - 1) / t.bn);
+        g.walk.set(tiles_m, tiles_n, gemm_walk_rows(tiles_m, tiles_n, t.bm, t.bn, n), n, g.ztab);
+        return (int64_t)tiles_m * tiles_n * n;
+    };
+    p.tn_first = p.tn.K > p.nn.K * p.nn.chain;
+    const int64_t wgs_nn = set(p.nn, 1), wgs_tn = set(p.tn, nblk);
+    const int64_t first = ((p.tn_first ? wgs_tn : wgs_nn) + 7) / 8 * 8, second = p.tn_first ? wgs_nn : wgs_tn;
+    CACTI_REQUIRE(first + second < (int64_t)1 << 31, CACTI_E_NOTIMPL, "gemm: %lld workgroups exceed the grid limit", (long long)(first + second));
+    p.second = (uint32_t)first;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(first + second)), dim3(256), smem, st, p);
+    return launch_status("gemm_pair");
+}
+
+// The tiles of a pair, both products' the same.
+constexpr int kPairShapes[] = {T64_SMALL, 0, 3, 5, 7};     // 64 x 64 twice, 64 x 128, 128 x 128, 160 x 128
 
 template <bool TA, bool TB, int... I>
 int launch_shape(int shape, const GemmArgs &p, int64_t nblk, hipStream_t st, std::integer_sequence<int, I...>)
@@ -908,6 +958,45 @@ GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K)
     best.us = fixed + kAnyPerTile * (tile_cost(cus, T64, M, N, 1, kt) - fixed);
     split_k(cus, T64, M, N, kt, kAnyPerTile, best, best.us);
     return best;
+}
+
+// What a launch of both is expected to take: the workgroups that the device holds at a time share them all, unless one of the
+// longer product takes longer than that.  Separate launches -> one, us: S = 611, N = K = 1024 12.3 -> 8.0; three of those 23.0 ->
+// 16.9; two of N = 2816 35.9 -> 27.6; 2048, 2048, 2048 40.5 -> 35.0; 333, 3200, 8640 60.2 -> 48.8; three of 128, 256, 256 (four
+// launches) 17.0 -> 6.5.  Larger ones fill the device by themselves, with tiles of their own: three of 2048, 3200, 3200 are 229 us,
+// two of 777, 5504, 2048 99.
+GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n)
+{
+    const int64_t cus = device_cus(), kt_nn = (N + BK - 1) / BK * n, kt_tn = (S + BK - 1) / BK;
+    const bool small_nn = S * K <= kSmallOutput, small_tn = N * K <= kSmallOutput;
+    GemmPlan best = {-1, T64, 0, 1, 0};
+    if (small_nn != small_tn) return best;
+    for (int tile : kPairShapes) {
+        if ((tile == T64_SMALL) != small_nn) continue;
+        const Shape &t = kShapes[tile == T64_SMALL ? T64 : tile];
+        auto tiles = [&](int64_t M, int64_t C) { return (double)((M + t.bm - 1) / t.bm) * (double)((C + t.bn - 1) / t.bn); };
+        const double work = tiles(S, K) * (kt_nn * t.full + t.round) + n * tiles(N, K) * (kt_tn * t.full + t.round);
+        const double us = t.fixed + std::max(work / (double)(cus * t.res), (double)std::max(kt_nn, kt_tn) * (t.first + t.load));
+        if (best.tile < 0 || us < best.us) {
+            best.tile = tile;
+            best.us = us;
+        }
+    }
+    const GemmPlan nn = n > 1 ? gemm_plan_chain(S, K, N, n) : gemm_plan(S, K, N, 1, false), tn = gemm_plan(N, K, S, n, false);
+    if (best.us >= 0.95 * (nn.us + tn.us)) best.tile = -1;
+    return best;
+}
+
+int gemm_pair_launch(const GemmArgs &nn, const GemmArgs &tn, int64_t nblk, const GemmPlan &plan, hipStream_t st)
+{
+    const PairArgs p = {nn, tn, 0};
+    switch (plan.tile) {
+        case T64_SMALL: return launch_pair<T64_SMALL>(p, nblk, st);
+        case 0: return launch_pair<0>(p, nblk, st);
+        case 3: return launch_pair<3>(p, nblk, st);
+        case 5: return launch_pair<5>(p, nblk, st);
+        default: return launch_pair<7>(p, nblk, st);
+    }
 }
 
 int gemm_direct_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, const GemmPlan &plan, hipStream_t st)

@@ -117,6 +117,8 @@ struct GemmPlan {
 // nz: products of this shape in the launch
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split);
 GemmPlan gemm_plan_chain(int64_t M, int64_t N, int64_t K, int chain);       // chain <= kMaxPtrBatch products that add up
+// the gradients of n products x W_i^T, x [S,K], W_i [N,K], all in one launch (tile < 0: no better than two)
+GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n);
 GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K);        // for GemmArgs::any (with parts of K)
 void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn);
 // the kernel of the plan's (first) launch as a profiler prints it; returns what snprintf does
@@ -129,6 +131,8 @@ int gemm_mfma_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, int align,
 // Products of 16-byte aligned operands, cut by `plan` (p.part lent for its parts; p.odd: C of any alignment and N; tri and win
 // are not for these).
 int gemm_direct_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, const GemmPlan &plan, hipStream_t st);
+
+int gemm_pair_launch(const GemmArgs &nn, const GemmArgs &tn, int64_t nblk, const GemmPlan &plan, hipStream_t st);
 
 // tile rows per group of the walk of a launch of tiles_m x tiles_n tiles of bm x bn
 int gemm_walk_rows(int tiles_m, int tiles_n, int bm, int bn, int64_t nblk);

@@ -472,6 +472,7 @@ CACTI_API int cacti_llama_stage(cacti_llama *m, int want_prob, int want_grad)
         add_a = add_b = 0;
         return 0;
     };
+    auto linear = [&]() { return m->group_products >= 2 ? make_linear() : make_matmul(false, true, 1.f); };
     TRY(ap(c, make_embed(), {m->embed, m->in_tok}, &stream));
     for (size_t l = 0; l < m->layers.size(); l++) {
         const LayerCells &w = m->layers[l];
@@ -509,7 +510,7 @@ CACTI_API int cacti_llama_stage(cacti_llama *m, int want_prob, int want_grad)
             TRY(ap(c, make_causal_softmax(g.H), {s16}, &p16));
             TRY(ap(c, make_causal_pv(g.H), {p16, v}, &attn));
         }
-        TRY(ap(c, make_matmul(false, true, 1.f), {attn, w.o}, &o));
+        TRY(ap(c, linear(), {attn, w.o}, &o));
         add_a = stream;                                       // x1 = stream + o
         add_b = o;
         TRY(norm_of_stream(w.post_norm, &post));
@@ -523,13 +524,13 @@ CACTI_API int cacti_llama_stage(cacti_llama *m, int want_prob, int want_grad)
             TRY(ap(c, make_matmul(false, true, 1.f), {post, w.gate}, &gate));
         }
         TRY(ap(c, make_silu_gate(), {gate, up}, &h));
-        TRY(ap(c, make_matmul(false, true, 1.f), {h, w.down}, &down));
+        TRY(ap(c, linear(), {h, w.down}, &down));
         add_a = stream;                                       // x2 = x1 + down
         add_b = down;
     }
     CellPtr hn, logit;
     TRY(norm_of_stream(m->head_norm, &hn));
-    TRY(ap(c, make_matmul(false, true, 1.f), {hn, m->lm_head}, &logit));
+    TRY(ap(c, linear(), {hn, m->lm_head}, &logit));
     std::vector<CellPtr> outs;
     TRY(c.stage_apply(c.add_thunk(make_softmax_ce(want_prob != 0)), {logit, m->in_lm_tok}, &outs));
     m->out_logit = logit;

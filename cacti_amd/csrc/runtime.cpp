@@ -1320,12 +1320,14 @@ int Ctx::run_entry(const Entry &e)
     int rc = run_thunk(sp, e.args, e.outs, e.acc_mask);
     quiet_oom_ = false;
     if (n <= 1 || rc != CACTI_E_OOM) return rc;
+    uint32_t written = 0;
     for (int i = 0; i < n; i++) {
         std::vector<CellPtr> args;
         const std::unique_ptr<ThunkSpec> one = sp.piece(i, e.args, &args);
-        const int o = sp.pieces_add_up() ? 0 : i;
-        rc = run_thunk(*one, args, {e.outs[(size_t)o]}, i > o ? 1 : (e.acc_mask >> o) & 1);
+        const int o = sp.piece_out(i);
+        rc = run_thunk(*one, args, {e.outs[(size_t)o]}, ((e.acc_mask | written) >> o) & 1);
         if (rc) return rc;
+        written |= 1u << o;
     }
     return 0;
 }

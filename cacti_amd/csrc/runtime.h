@@ -118,11 +118,11 @@ struct ThunkSpec {
     virtual int run(Ctx &ctx, const std::vector<CellType> &aty, void *const *a,
                     const std::vector<CellType> &oty, void *const *o, uint32_t acc_mask,
                     void *ws, size_t ws_bytes) const = 0;
-    // A thunk of several independent products: how many, and product i as a thunk by itself with the arguments it reads
-    // (its output is output i, or the only one, which the later ones accumulate into).  They run one after another where the
-    // pool has no room for the cells of all.
+    // A thunk of several products: how many, product i as a thunk by itself with the arguments it reads, and the output it
+    // writes (accumulating into it where an earlier one has written it).  They run one after another where the pool has no room
+    // for the cells of all.
     virtual int pieces() const { return 1; }
-    virtual bool pieces_add_up() const { return false; }
+    virtual int piece_out(int i) const { return i; }
     virtual std::unique_ptr<ThunkSpec> piece(int, const std::vector<CellPtr> &, std::vector<CellPtr> *) const { return nullptr; }
     // out_adj[k] = adjoint cell of output k or 0; stage contributions through ctx.adj_*
     virtual int pop_adj(Ctx &, const Entry &, const std::vector<CellPtr> &) const { return 0; }

@@ -398,7 +398,7 @@ struct DgradNSpec : ThunkSpec {
         return cacti_hip_gemm_f16_chain(n, Sq, K, N, a, N, a + n, K, (acc & 1) ? 1.f : 0.f, o[0], K, S(c));
     }
     int pieces() const override { return n; }
-    bool pieces_add_up() const override { return true; }
+    int piece_out(int) const override { return 0; }
     std::unique_ptr<ThunkSpec> piece(int i, const std::vector<CellPtr> &a, std::vector<CellPtr> *in) const override
     {
         *in = {a[(size_t)i], a[(size_t)(n + i)]};
@@ -412,6 +412,69 @@ struct DgradNSpec : ThunkSpec {
         return buf;
     }
 };
+
+// All gradients of n products x W_i^T in one launch: (dy_1 .. dy_n, W_1 .. W_n, x) -> (dx, dW_1 .. dW_n), dx as above
+struct GradsNSpec : ThunkSpec {
+    int n;
+    explicit GradsNSpec(int n_) : n(n_) {}
+    const char *name() const override { return "matmul"; }
+    int arity() const override { return 2 * n + 1; }
+    int nout() const override { return n + 1; }
+    int out_ty(const std::vector<CellType> &a, std::vector<CellType> &o) const override
+    {
+        TY_REQUIRE(n >= 1 && n <= kMaxGroup, "gradients of products: 1 .. %d of them", kMaxGroup);
+        const CellType &x = a[(size_t)(2 * n)];
+        for (int i = 0; i < n; i++)
+            TY_REQUIRE(a[i].dtype == F16 && a[i].shape.size() == 2 && a[i] == a[0] && a[n + i] == a[n] && a[n].dtype == F16 &&
+                           a[n].shape.size() == 2 && a[n].shape[0] == a[0].shape[1] && x.dtype == F16 && x.shape.size() == 2 &&
+                           x.shape[0] == a[0].shape[0] && x.shape[1] == a[n].shape[1],
+                       "gradients of products: (dy f16 [S,N] x n, W f16 [N,K] x n, x f16 [S,K]) expected");
+        o.assign((size_t)(n + 1), a[n]);
+        o[0] = x;
+        return 0;
+    }
+    int run(Ctx &c, const std::vector<CellType> &aty, void *const *a, const std::vector<CellType> &,
+            void *const *o, uint32_t acc, void *, size_t) const override
+    {
+        const int64_t Sq = aty[0].shape[0], N = aty[0].shape[1], K = aty[n].shape[1];
+        const uint32_t all = (1u << n) - 1, dw = acc >> 1 & all;
+        if (dw != 0 && dw != all) {                            // mixed modes: one after the other
+            for (int i = 0; i < n; i++) {
+                const int rc = cacti_hip_gemm_f16(1, 0, N, K, Sq, 1.f, a[i], N, a[2 * n], K, ((dw >> i) & 1) ? 1.f : 0.f, o[1 + i], K, S(c));
+                if (rc) return rc;
+            }
+            return cacti_hip_gemm_f16_chain(n, Sq, K, N, a, N, a + n, K, (acc & 1) ? 1.f : 0.f, o[0], K, S(c));
+        }
+        return cacti_hip_gemm_f16_grads(n, Sq, N, K, a, a + n, a[2 * n], (acc & 1) ? 1.f : 0.f, o[0], dw ? 1.f : 0.f, o + 1, S(c));
+    }
+    int pieces() const override { return 2 * n; }
+    int piece_out(int i) const override { return i < n ? 1 + i : 0; }
+    std::unique_ptr<ThunkSpec> piece(int i, const std::vector<CellPtr> &a, std::vector<CellPtr> *in) const override
+    {
+        *in = {a[(size_t)(i % n)], a[(size_t)(i < n ? 2 * n : i)]};
+        return make_matmul(i < n, false, 1.f);
+    }
+    std::string key(const std::vector<CellType> &aty, uint32_t) const override
+    {
+        char buf[128];
+        snprintf(buf, sizeof(buf), "matmul_grads[%lldx%lldx%lld]x%d", (long long)aty[0].shape[0], (long long)aty[0].shape[1],
+                 (long long)aty[n].shape[1], n);
+        return buf;
+    }
+};
+// the gradients of y_i = x W_i^T for the dy in `dy`, last product first, as one thunk if one launch of them pays; *staged: it did
+static int stage_grads(Ctx &c, CellPtr x, const std::vector<CellPtr> &ws, const std::vector<CellPtr> &dy, bool *staged)
+{
+    const CellType &g = c.cell(dy[0]).ty, &w = c.cell(ws[0]).ty;
+    const int n = (int)ws.size();
+    *staged = cacti_hip_gemm_f16_grads_one_launch(n, g.shape[0], g.shape[1], w.shape[1]) != 0;
+    if (!*staged) return 0;
+    std::vector<CellPtr> primals = {x}, in(dy.rbegin(), dy.rend());
+    primals.insert(primals.end(), ws.rbegin(), ws.rend());
+    in.insert(in.end(), ws.rbegin(), ws.rend());
+    in.push_back(x);
+    return c.adj_add(primals, std::unique_ptr<ThunkSpec>(new GradsNSpec(n)), in);
+}
 
 // y_i = x W_i^T: (x, W_1 .. W_n) -> (y_1 .. y_n)
 struct ProjNSpec : ThunkSpec {
@@ -466,6 +529,8 @@ struct ProjNSpec : ThunkSpec {
         int rc;
         if (all) {
             std::vector<CellPtr> ws(e.args.begin() + 1, e.args.end()), in(dy.begin(), dy.begin() + n);
+            bool staged = false;
+            if ((rc = stage_grads(c, x, ws, in, &staged)) || staged) return rc;
             in.push_back(x);
             if ((rc = c.adj_add(ws, std::unique_ptr<ThunkSpec>(new WgradNSpec(n)), in))) return rc;
             std::vector<CellPtr> chain(dy.rend() - n, dy.rend());
@@ -481,6 +546,18 @@ struct ProjNSpec : ThunkSpec {
                 return rc;                                                     // G B
         }
         return 0;
+    }
+};
+
+// ---------------------------------------------------------------------------
+// y = x W^T whose gradients are one thunk where one launch of both pays
+struct LinearSpec : MatMulSpec {
+    LinearSpec() : MatMulSpec(false, true, 1.f, 0) {}
+    int pop_adj(Ctx &c, const Entry &e, const std::vector<CellPtr> &dy) const override
+    {
+        bool staged = false;
+        const int rc = stage_grads(c, e.args[0], {e.args[1]}, {dy[0]}, &staged);
+        return rc || staged ? rc : MatMulSpec::pop_adj(c, e, dy);
     }
 };
 
@@ -802,6 +879,7 @@ std::unique_ptr<ThunkSpec> make_matmul(bool ta, bool tb, float alpha)
 {
     return std::unique_ptr<ThunkSpec>(new MatMulSpec(ta, tb, alpha, 0));
 }
+std::unique_ptr<ThunkSpec> make_linear() { return std::unique_ptr<ThunkSpec>(new LinearSpec()); }
 std::unique_ptr<ThunkSpec> make_projections(int n, bool group_adjoints)
 {
     return std::unique_ptr<ThunkSpec>(new ProjNSpec(n, group_adjoints));

@@ -57,6 +57,8 @@ SIGNATURES = {
     "cacti_hip_gemm_plan": (ci, [i64, i64, i64, i64, C.POINTER(i64)]),
     "cacti_hip_gemm_kernel_name": (ci, [ci, ci, i64, i64, i64, i64, C.c_char_p, sz]),
     "cacti_hip_gemm_f16_batched": (ci, [ci, ci, i64, i64, i64, i64, f32, vp, i64, vp, i64, f32, vp, i64, vp]),
+    "cacti_hip_gemm_f16_grads": (ci, [i64, i64, i64, i64, vp, vp, vp, f32, vp, f32, vp, vp]),
+    "cacti_hip_gemm_f16_grads_one_launch": (ci, [i64, i64, i64, i64]),
     "cacti_hip_gemm_f16_chain": (ci, [i64, i64, i64, i64, vp, i64, vp, i64, f32, vp, i64, vp]),
     "cacti_hip_gemm_f16_strided_batched": (ci, [ci, ci, i64, i64, i64, i64, f32, vp, i64, i64, vp,
                                                 i64, i64, f32, vp, i64, i64, vp]),

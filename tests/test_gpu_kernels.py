@@ -648,6 +648,40 @@ def test_gemm_chain_has_the_bits_of_products_one_by_one(ops, n, M, N, K, gap, be
     assert ((got[:, :N].float() - ref).norm() / ref.norm()).item() < n * 3e-4
 
 
+# all gradients of products that share an input in one launch: small outputs (M32) and the four tiles of others; either one's sums the
+# longer; one k tile, a tail of either sum; behind the line what is for separate launches: one small output of two, what fills the device, a chain with a tail,
+# five products, rows that are not 16-byte aligned
+@pytest.mark.gpu
+@pytest.mark.parametrize("beta_x,beta_w", [(0, 0), (1, 1)])
+@pytest.mark.parametrize("n,S,N,K,one", [
+    (1, 1, 8, 8, 1), (1, 64, 64, 64, 1), (1, 33, 136, 72, 1), (3, 128, 256, 256, 1), (2, 200, 320, 264, 1), (1, 611, 1024, 1024, 1),
+    (1, 513, 1032, 1048, 1), (3, 611, 1024, 1024, 1), (2, 611, 2816, 1024, 1), (1, 611, 1024, 2816, 1), (1, 777, 2048, 2048, 1),
+    (4, 600, 576, 1032, 1), (1, 1300, 768, 2304, 1), (1, 2000, 1024, 1024, 1),
+    (2, 128, 688, 256, 0), (1, 128, 4096, 256, 0), (1, 1600, 2048, 6000, 0), (2, 600, 1000, 1024, 0), (5, 96, 256, 256, 0), (1, 300, 1028, 512, 0)])
+def test_gemm_grads_have_the_bits_of_products_one_by_one(ops, n, S, N, K, one, beta_x, beta_w):
+    import ctypes as C
+    import torch
+    from cacti_amd import ffi
+    say("gemm grads", n, S, N, K, beta_x, beta_w)
+    assert ffi.lib().cacti_hip_gemm_f16_grads_one_launch(n, S, N, K) == one
+    g = torch.Generator(device="cuda").manual_seed(n + S + N + K)
+    st = torch.cuda.current_stream().cuda_stream
+    new = lambda *s: torch.randn(*s, device="cuda", generator=g).half()
+    dy, W, x = [new(S, N) for _ in range(n)], [new(N, K) for _ in range(n)], new(S, K)
+    dx, dW = new(S, K), [new(N, K) for _ in range(n)]
+    want_x, want_w = dx.clone(), [t.clone() for t in dW]
+    for z in range(n):
+        ffi.call("cacti_hip_gemm_f16", 1, 0, N, K, S, 1.0, dy[z].data_ptr(), N, x.data_ptr(), K, float(beta_w), want_w[z].data_ptr(), K, st)
+        ffi.call("cacti_hip_gemm_f16", 0, 0, S, K, N, 1.0, dy[z].data_ptr(), N, W[z].data_ptr(), K, 1.0 if z else float(beta_x),
+                 want_x.data_ptr(), K, st)
+    pd, pw, pg = ((C.c_void_p * n)(*[t.data_ptr() for t in a]) for a in (dy, W, dW))
+    ffi.call("cacti_hip_gemm_f16_grads", n, S, N, K, C.cast(pd, C.c_void_p), C.cast(pw, C.c_void_p), x.data_ptr(), float(beta_x), dx.data_ptr(),
+             float(beta_w), C.cast(pg, C.c_void_p), st)
+    assert_bits(host(dx), host(want_x), "dx")
+    for z in range(n):
+        assert_bits(host(dW[z]), host(want_w[z]), "dW %d" % z)
+
+
 def test_gemm_colmajor_entry(ops, oracle):
     """The cuBLAS-shaped entry: row-major callers pass operands swapped (thunk/op.rs:4469-4491)."""
     import ctypes as C
