@@ -479,7 +479,7 @@ static int stage_grads(Ctx &c, CellPtr x, const std::vector<CellPtr> &ws, const 
 // y_i = x W_i^T: (x, W_1 .. W_n) -> (y_1 .. y_n)
 struct ProjNSpec : ThunkSpec {
     int n;
-    bool group_adj;                  // the weight gradients as one grouped thunk as well
+    bool group_adj;                  // the gradients grouped as well
     explicit ProjNSpec(int n_, bool ga = true) : n(n_), group_adj(ga) {}
     const char *name() const override { return "matmul"; }
     int arity() const override { return n + 1; }

@@ -148,7 +148,8 @@ class Llama:
 
     def set_product_groups(self, on):
         """0: one matmul thunk per product; 1: the up and gate projections of a layer as one thunk and
-        launch; 2 (default): also q, k, v, and the weight gradients of both groups.  Bit-identical results."""
+        launch; 2 (default): also q, k, v, the weight and the input gradients of both groups, and all gradients of a group or
+        a product in one launch where that pays.  Bit-identical results."""
         ffi.call("cacti_llama_set_product_groups", self._m, int(on))
 
     def put_param(self, i, arr):

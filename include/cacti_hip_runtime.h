@@ -237,7 +237,8 @@ int cacti_llama_set_attention(cacti_llama *model, int mode);
  * reference's cublasGemmBatchedEx shape, cacti_gpu_cu_ffi/src/lib.rs:793-885).  0: one matmul thunk per
  * product as src/librarium/llama.rs:478-497 stages them.  1: the up and gate projections of a layer
  * as one thunk and one launch, their adjoints as for separate thunks.  2 (default): also the query, key and value
- * projections, and the weight gradients of both groups as one thunk each.  A group may be cut into other tiles than its
+ * projections, the weight gradients of both groups as one thunk each, the input gradients of a group as one thunk and launch,
+ * and all gradients of a group, or of a product alone, where one launch of them pays.  A group may be cut into other tiles than its
  * products alone, but every output is summed over the same values in the same order in all three, and the adjoint's
  * accumulations keep their order, so the results are identical bit for bit.  Where the pool has no room for the cells
  * of a group at once, its products run one after another.  Measured on one MI355X, 1 -> 2: the 3B step 50.71 -> 50.45 ms; 4 layers of width 1024 on two
