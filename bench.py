@@ -293,7 +293,7 @@ def run_step(args):
     prefix = next(iter(prefixes))
 
     # timed region: exactly K steps, events around every EVENT_STRIDE-th launch of the dominant
-    # kernel (the stride is coprime to the 6 such launches per layer and the 157 per step, so all
+    # kernel (the stride is coprime to the 2 such launches per layer and the 52 per step, so all
     # shapes are sampled)
     ctx.set_timing(0)
     ctx.set_timing_filter(prefix, EVENT_STRIDE)
