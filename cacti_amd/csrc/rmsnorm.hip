@@ -102,11 +102,14 @@ rms_norm_bwd_kernel(int64_t N, int D, const half_t *__restrict__ x, const half_t
 
     if (live) {
         const half_t *xr = x + n * D, *gr = dy + n * D;
-        // every load of the row up front and unconditional (see the forward kernel)
+        // every load of the row up front and unconditional (see the forward kernel), but for dx of rows beyond 8 chunks: with it a
+        // lane spills 108 registers instead of 56 (2048 rows of 4608 43.0 us, 31.6 so; of 6144 55.3, 41.6; of 8192 95, 80;
+        // accumulating 44.1, 34.6)
         half_t *or_ = dx + n * D;
         // without accumulation the fourth stream re-reads dy (a cache hit) instead of dx
         const half_t *oldr = dx_acc ? or_ : gr;
-        h8 xv[CH], gv[CH], wv[CH], old[CH];
+        constexpr bool EARLY = CH <= 8;
+        h8 xv[CH], gv[CH], wv[CH], old[EARLY ? CH : 1];      // old: used only when dx accumulates
         double ss = 0.0;
 #pragma unroll
         for (int c = 0; c < CH; c++) {
@@ -114,7 +117,7 @@ rms_norm_bwd_kernel(int64_t N, int D, const half_t *__restrict__ x, const half_t
             xv[c] = ld8(xr + ch * 8);
             gv[c] = ld8(gr + ch * 8);
             wv[c] = ld8(w + ch * 8);
-            old[c] = ld8(oldr + ch * 8);                      // used only when dx accumulates
+            if constexpr (EARLY) old[c] = ld8(oldr + ch * 8);
         }
 #pragma unroll
         for (int c = 0; c < CH; c++) {
@@ -156,11 +159,14 @@ rms_norm_bwd_kernel(int64_t N, int D, const half_t *__restrict__ x, const half_t
             const int ch = c * 64 + lane;
             if (ch < nchunk) {
                 h8 o;
+                if constexpr (!EARLY) {
+                    if (dx_acc) old[0] = ld8(or_ + ch * 8);
+                }
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     const float xf = h2f(xv[c].v[i]);
                     const half_t c2 = f2h(dsq * (xf + xf)), c1 = gv[c].v[i];
-                    o.v[i] = (dx_acc ? old[c].v[i] + c1 : c1) + c2;
+                    o.v[i] = (dx_acc ? old[EARLY ? c : 0].v[i] + c1 : c1) + c2;
                 }
                 st8(or_ + ch * 8, o);
             }
