@@ -220,10 +220,12 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_short_fwd_kernel(AttnArgs p)
         constexpr int j = decltype(j_c)::value;
         if (j < n) {
             float pe[16];
+            // masked by position: a row whose every score came to -infinity has no probabilities (NaN), 0 is for the keys behind it
+            const int last = wid + NW * j < qt ? kBlk : l32 - 4 * lh;
 #pragma unroll
             for (int e = 0; e < 16; e++) {
                 const half_t s = sc[j][e >> 1][e & 1];
-                pe[e] = FAST ? exp2_mix(s, cs) : s == ninf ? 0.f : M::prob((float)s, m, l, y);
+                pe[e] = FAST ? exp2_mix(s, cs) : 8 * (e >> 2) + (e & 3) <= last ? M::prob((float)s, m, l, y) : 0.f;
             }
             const half8_t y0 = pack8(pe), y1 = pack8(pe + 8);
             if (j + 1 < n) landed<kPerBlock>();

@@ -876,6 +876,59 @@ def test_attention_of_short_sequences_against_the_register_path(ops, S, H, Dh, g
     assert float((m[0] - m[1]).abs().max()) <= 2e-3 * max(1.0, float(m.abs().max())) and float((l[0] / l[1] - 1).abs().max()) < 2e-3
 
 
+# One position, a ragged last block, 8 and 4 waves, a wave whose blocks hold no finite score of a row, windows, the form beyond 1024
+# positions; both adjoints of 32 rows, heads to 64 and beyond
+NOT_FINITE_SHAPES = [(1, 1, 64), (33, 2, 128), (61, 2, 64), (300, 4, 100), (700, 16, 64), (777, 4, 128), (1500, 4, 64)]
+
+
+def _attention_masks(q, k, v, dO, alpha, off, exact):
+    """Which elements of O, dQ, dK, dV are NaN and which infinite, with the tensors `off` elements past a 16-byte boundary (0: tiles
+    straight into LDS, 4: through registers)."""
+    import torch
+    from cacti_amd import ffi
+    S, H, Dh = q.shape
+    def at(x):
+        t = torch.empty(x.numel() + 8, dtype=torch.float16, device="cuda")[off:off + x.numel()].view(x.shape)
+        return t.copy_(x)
+    Q, K, V, G, o, dq, dk, dv = (at(x) for x in (q, k, v, dO, q, q, q, q))
+    st, size = torch.cuda.current_stream().cuda_stream, ffi.lib().cacti_hip_attention_bwd_workspace(S, H)
+    stats, ws = torch.empty(2 * S * H, device="cuda"), torch.empty(size, dtype=torch.uint8, device="cuda")
+    ffi.call("cacti_hip_attention_set_exact", int(exact))
+    try:
+        ffi.call("cacti_hip_attention_fwd", S, H, Dh, alpha, Q.data_ptr(), K.data_ptr(), V.data_ptr(), H * Dh, o.data_ptr(), stats.data_ptr(), st)
+        ffi.call("cacti_hip_attention_bwd", S, H, Dh, alpha, Q.data_ptr(), K.data_ptr(), V.data_ptr(), o.data_ptr(), G.data_ptr(), H * Dh,
+                 stats.data_ptr(), dq.data_ptr(), 0, dk.data_ptr(), 0, dv.data_ptr(), 0, ws.data_ptr(), size, st)
+    finally:
+        ffi.call("cacti_hip_attention_set_exact", 0)
+    return {n: (host(torch.isnan(x)), host(torch.isinf(x))) for n, x in (("o", o), ("dq", dq), ("dk", dk), ("dv", dv))}
+
+
+def _same_masks(q, k, v, dO, alpha, exact):
+    direct, registers = (_attention_masks(q, k, v, dO, alpha, off, exact) for off in (0, 4))
+    for n in direct:
+        assert (direct[n][0] == registers[n][0]).all(), n + ": NaN"
+        assert (direct[n][1] == registers[n][1]).all(), n + ": infinity"
+    return direct
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("S,H,Dh", NOT_FINITE_SHAPES)
+def test_attention_rows_whose_every_score_overflows(ops, S, H, Dh, exact):
+    """Every live score of a row rounds to -infinity: the row has no softmax (its sum is 0), so its output is NaN, and what
+    the adjoint makes of it is NaN where the register path has it."""
+    import torch
+    say("attention, rows of -infinity", S, H, Dh, exact)
+    g = torch.Generator(device="cuda").manual_seed(S + H + Dh)
+    q, v, dO = (torch.randn(S, H, Dh, device="cuda", generator=g).half() for _ in range(3))
+    k = torch.full((S, H, Dh), -300.0, device="cuda", dtype=torch.float16)
+    rows = sorted({0, S // 2, S - 1})
+    q[rows] = 300.0
+    masks = _same_masks(q, k, v, dO, Dh ** -0.5, exact)
+    nan = masks["o"][0]
+    assert nan[rows].all() and nan.sum() == len(rows) * H * Dh
+
+
 # The forward and the dQ kernel take 64 query rows per workgroup where their number is at most twice (forward, fast, up to
 # 1024 positions: 7/4 of) the CUs' of an MI355X, 256, and 128 beyond: rows one short of, on and one past the edges of both
 # at few heads, and the 128 rows' form at many small heads (480 workgroups of 64 rows: forward only; 528, 640: both), with
