@@ -31,8 +31,8 @@ struct BlockMap {
         pc = t & 15;
         r0 = t >> 4;
     }
-    // instruction `it` of the 8; src = the window's first element in the block's first row; rows beyond the tensor are its
-    // last row once more (they are masked, and what is masked there is masked for that row too)
+    // instruction `it` of the 8; src = the window's first element in the block's first row; rows beyond the tensor are its last
+    // row once more, so that a block is 8 loads to wait for whatever its rows (zero_rows where a product sums over them)
     __device__ __forceinline__ void load1(int it, gptr_t src, int rows, uint32_t lds) const
     {
         const int r = r0 + 4 * it, c = pc ^ gsw(r);
@@ -56,6 +56,14 @@ __device__ __forceinline__ void landed()
 __device__ __forceinline__ void reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 __device__ __forceinline__ uint32_t lds_of(const void *p) { return (uint32_t)(uintptr_t)p; }
+
+// Rows [rows, 32) of a block that has landed, by its wave.  For the operand of a product over the block's rows whose other factor
+// is 0 there: the last row is live for the queries (keys) that see it, and an infinity in it, once more times 0, would make
+// their sums NaN.
+__device__ __forceinline__ void zero_rows(unsigned char *block, int rows)
+{
+    for (int i = rows * 16 + (threadIdx.x & 63); i < kBlk * 16; i += 64) *reinterpret_cast<uint4 *>(block + i * 16) = make_uint4(0, 0, 0, 0);
+}
 
 // the chunks of a wave's blocks that no load writes
 __device__ __forceinline__ void zero_block_pads(unsigned char *blocks, int rows, int nch)
@@ -211,6 +219,7 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_short_fwd_kernel(AttnArgs p)
     }
     const float y = recip_refined(l), cs = prob_shift(m, l);
 
+    const bool ragged = S - i0 < kBlk && (qt - wid) % NW == 0;      // the wave's last value block
     float16_t oacc[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)
@@ -228,8 +237,12 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_short_fwd_kernel(AttnArgs p)
                 pe[e] = FAST ? exp2_mix(s, cs) : 8 * (e >> 2) + (e & 3) <= last ? M::prob((float)s, m, l, y) : 0.f;
             }
             const half8_t y0 = pack8(pe), y1 = pack8(pe + 8);
-            if (j + 1 < n) landed<kPerBlock>();
-            else landed<0>();
+            if (j + 1 < n) {
+                landed<kPerBlock>();
+            } else {
+                landed<0>();
+                if (ragged) zero_rows(mine + ((n + j) & 1) * kBlkB, S - i0);
+            }
             prod_tr<DT>(oacc, mine + ((n + j) & 1) * kBlkB, 0, y0, y1, lane);
             if (j + 2 < n) {
                 reads_done();
@@ -477,6 +490,7 @@ __global__ void __launch_bounds__(key_waves(DT) * 64, key_waves(DT) / 4) attn_sh
         const unsigned char *Qs = mine + j % PAIRS * 2 * kBlkB, *Gs = Qs + kBlkB;
         const float *stc = st + j % PAIRS * 4 * 64;
         const int q0 = (kt + wid + NW * j) * kBlk;
+        if (S - q0 < kBlk) zero_rows(mine + j % PAIRS * 2 * kBlkB + kBlkB, S - q0);
         const float16_t pacc = prod_direct<KS, NW == 8>(Gs, 0, vf, l32, lh);
         if (PAIRS == 1) landed<0>();
         const float16_t sacc = prod_direct<KS, NW == 8>(Qs, 0, kf, l32, lh);

@@ -929,6 +929,27 @@ def test_attention_rows_whose_every_score_overflows(ops, S, H, Dh, exact):
     assert nan[rows].all() and nan.sum() == len(rows) * H * Dh
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("S,H,Dh", NOT_FINITE_SHAPES)
+def test_attention_infinity_in_the_last_row(ops, S, H, Dh, exact):
+    """The last position's values (then its output gradient) hold an infinity, in a block of 32 that the tensor may not fill:
+    the last output row (every dV row) is infinite there and not NaN, nothing beyond the tensor being multiplied with it."""
+    import torch
+    say("attention, infinity in the last row", S, H, Dh, exact)
+    g = torch.Generator(device="cuda").manual_seed(S + H + Dh)
+    q, k, v, dO = (torch.randn(S, H, Dh, device="cuda", generator=g).half() for _ in range(4))
+    q *= 0.25                                     # (no probability of the last row below what f16 holds)
+    x = v.clone()
+    x[-1, :, 4:8] = float("inf")
+    masks = _same_masks(q, k, x, dO, Dh ** -0.5, exact)
+    assert masks["o"][1][-1, :, 4:8].all() and not masks["o"][0][-1].any()
+    x = dO.clone()
+    x[-1, :, 4:8] = float("inf")
+    masks = _same_masks(q, k, v, x, Dh ** -0.5, exact)
+    assert masks["dv"][1][:, :, 4:8].all() and not masks["dv"][0].any()
+
+
 # The forward and the dQ kernel take 64 query rows per workgroup where their number is at most twice (forward, fast, up to
 # 1024 positions: 7/4 of) the CUs' of an MI355X, 256, and 128 beyond: rows one short of, on and one past the edges of both
 # at few heads, and the 128 rows' form at many small heads (480 workgroups of 64 rows: forward only; 528, 640: both), with
