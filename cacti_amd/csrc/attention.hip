@@ -1445,6 +1445,17 @@ CACTI_API size_t cacti_hip_attention_bwd_workspace_best(int64_t S, int64_t H, in
     return stats_part_bytes(S, H) + parts_bytes(parts, S, H, Dh);
 }
 
+CACTI_API size_t cacti_hip_attention_bwd_workspace_used(int64_t S, int64_t H, int64_t Dh, int64_t ld)
+{
+    const size_t least = cacti_hip_attention_bwd_workspace(S, H);
+    if (S <= 0 || H <= 0 || Dh <= 0 || Dh > kDP) return least;
+    const DkvParts parts = dkv_parts(S, H, g_exact.load(std::memory_order_relaxed) != 0);
+    int64_t span;
+    // (parts are of tiles straight from memory, and with those a walk over all queries is the better form of most shapes)
+    if (parts.split < 2 || !direct_tiles(H, Dh, ld, {}, &span) || attention_short_dkv_takes(S, H, span, parts.per)) return least;
+    return cacti_hip_attention_bwd_workspace_best(S, H, Dh);
+}
+
 CACTI_API int cacti_hip_attention_bwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,
                                       const void *v, const void *o, const void *dO, int64_t ld, const void *stats,
                                       void *dq, int dq_acc, void *dk, int dk_acc, void *dv, int dv_acc,

@@ -735,8 +735,7 @@ struct AttentionBwdSpec : ThunkSpec {
     size_t workspace(const std::vector<CellType> &a) const override { return cacti_hip_attention_bwd_workspace(a[0].shape[0], H); }
     size_t workspace_best(const std::vector<CellType> &a) const override
     {
-        if (a[0].shape[1] % 8) return workspace(a);               // (such rows have no parts of the queries)
-        return cacti_hip_attention_bwd_workspace_best(a[0].shape[0], H, a[0].shape[1] / H);
+        return cacti_hip_attention_bwd_workspace_used(a[0].shape[0], H, a[0].shape[1] / H, a[0].shape[1]);
     }
     int run(Ctx &c, const std::vector<CellType> &aty, void *const *a, const std::vector<CellType> &,
             void *const *o, uint32_t acc, void *ws, size_t wsb) const override

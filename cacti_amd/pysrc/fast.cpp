@@ -316,8 +316,7 @@ PyObject *attention_bwd(PyObject *const *v)
         return acc.t;
     };
     const std::vector<at::Tensor> d = into ? given() : std::vector<at::Tensor>{new_like(q), new_like(q), new_like(q)};
-    // (rows of no multiple of 8 elements have no parts of the queries to lend scratch for)
-    const size_t bytes = H * Dh % 8 ? cacti_hip_attention_bwd_workspace(S, H) : cacti_hip_attention_bwd_workspace_best(S, H, Dh);
+    const size_t bytes = cacti_hip_attention_bwd_workspace_used(S, H, Dh, H * Dh);
     const at::Tensor ws = empty({(int64_t)bytes}, q, at::kByte);
     void *st = stream();
     run([&] {

@@ -326,10 +326,12 @@ size_t cacti_hip_attention_stats_bytes(int64_t S, int64_t H);
 int cacti_hip_attention_fwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,
                             const void *v, int64_t ld, void *o, void *stats, void *stream);
 size_t cacti_hip_attention_bwd_workspace(int64_t S, int64_t H);
-/* As much as the adjoint can have a use for in the arithmetic that is set: with it (16-byte aligned) the default arithmetic sums
- * the dK / dV of few heads in parts of the queries, on more of the device, where the tensors allow the faster form above
- * (ld % 8 == 0 and the rest) and a walk over all queries takes longer.  Any workspace of at least
- * cacti_hip_attention_bwd_workspace(S, H) bytes is enough in either. */
+/* As much as the adjoint has a use for in the arithmetic that is set, with 16-byte aligned tensors of row stride ld: given it
+ * (16-byte aligned) the default arithmetic sums the dK / dV of few heads in parts of the queries, on more of the device, where the
+ * tensors allow the faster form above and a walk over all queries takes longer (1531 positions of 4 heads of 100: 24.5 MB; 1000
+ * of them: the least).  Any workspace of at least cacti_hip_attention_bwd_workspace(S, H) bytes is enough in either. */
+size_t cacti_hip_attention_bwd_workspace_used(int64_t S, int64_t H, int64_t Dh, int64_t ld);
+/* An upper bound of that for any ld: the room of the parts wherever there could be some, also where the walk is taken. */
 size_t cacti_hip_attention_bwd_workspace_best(int64_t S, int64_t H, int64_t Dh);
 int cacti_hip_attention_bwd(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k,
                             const void *v, const void *o, const void *dO, int64_t ld, const void *stats,

@@ -1106,6 +1106,36 @@ def test_attention_bwd_scratch_of_rows_without_parts(ops):
     assert taken <= room
 
 
+# with parts, then with a walk over all queries although a device of so few workgroups had room for parts, rows without direct tiles
+# (heads off the 16-byte grid, a window beyond the row's end), and shapes without parts
+@pytest.mark.parametrize("S,H,Dh,ld,parts", [(1531, 4, 100, 400, 5), (1471, 4, 128, 520, 5), (4001, 1, 64, 64, 8),
+                                             (1000, 4, 100, 400, 0), (577, 2, 128, 256, 0), (2048, 8, 128, 1024, 0),
+                                             (1531, 3, 100, 300, 0), (1531, 3, 100, 304, 6), (1531, 4, 100, 404, 0), (2048, 32, 100, 3200, 0), (128, 4, 64, 256, 0)])
+def test_attention_bwd_scratch_is_what_its_kernels_use(ops, S, H, Dh, ld, parts):
+    """What the operator allocates and a context's pool lends beside the results: the statistics, and the fp32 planes of the parts
+    where the kernel with parts is the one that runs (256 compute units); the exact arithmetic has none."""
+    from cacti_amd import ffi
+    L = ffi.lib()
+    least = L.cacti_hip_attention_bwd_workspace(S, H)
+    want = -(-least // 16) * 16 + parts * 2 * H * S * Dh * 4 if parts else least
+    assert L.cacti_hip_attention_bwd_workspace_used(S, H, Dh, ld) == want <= L.cacti_hip_attention_bwd_workspace_best(S, H, Dh)
+    ffi.call("cacti_hip_attention_set_exact", 1)
+    try:
+        assert L.cacti_hip_attention_bwd_workspace_used(S, H, Dh, ld) == least
+    finally:
+        ffi.call("cacti_hip_attention_set_exact", 0)
+    if ld != H * Dh:
+        return
+    q, k, v, dO = (torch.randn(S, H, Dh, device="cuda").half() for _ in range(4))
+    o, stats = ops.attention_fwd(q, k, v, 0.1)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    ops.attention_bwd(q, k, v, dO, stats, 0.1, o=o)
+    # (the allocator leaves up to 1 MiB of a block with the tensor in it)
+    assert torch.cuda.max_memory_allocated() - before <= 3 * q.nbytes + want + (4 << 20)
+
+
 @pytest.mark.parametrize("S,H,Dh", [(577, 2, 128), (576, 2, 128), (611, 16, 64), (777, 16, 128), (449, 3, 100), (1000, 2, 128),
                                     (1025, 8, 100), (2048, 32, 100), (128, 4, 64)])
 def test_attention_bwd_parts_fill_this_device(S, H, Dh):

@@ -211,6 +211,26 @@ def test_attention_scratch_gives_way_to_a_capped_pool(oracle):
         assert rel_l2(g, got[0][1][n]) < 5e-4, n
 
 
+def test_attention_scratch_of_a_walk_over_all_queries_is_the_least():
+    """1000 positions of 4 heads of 100 have no parts of the queries although there is room for some: the pool of a cycle in the
+    default arithmetic is no larger than in the exact one, which never has parts (25.6 MB of fp32 sums)."""
+    from cacti_amd import ffi
+    cfg, flat, tok, lm_tok, scale = make_inputs(dict(S=1000, D=400, H=4, Dh=100, F=416, V=512, L=1, eps=1e-6), seed=5, norm_mean=1.0,
+                                                grad_scale=1024.0)
+    peaks = []
+    for exact in (1, 0):
+        ffi.call("cacti_hip_attention_set_exact", exact)
+        try:
+            ctx, m = _model(cfg, pool_bytes=1 << 30)
+            m.put_params_flat(flat)
+            m.step(tok, lm_tok, scale)
+            peaks.append(ctx.stats()["pool_peak"])
+            m.close(); ctx.close()
+        finally:
+            ffi.call("cacti_hip_attention_set_exact", 0)
+    assert peaks[1] == peaks[0]
+
+
 @pytest.mark.parametrize("capped", [False, True])
 def test_digests_of_parameters_and_gradients(oracle, capped):
     """abs_log2_hist8 and nan_count of every parameter and gradient after a cycle, as the
