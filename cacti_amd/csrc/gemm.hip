@@ -522,6 +522,13 @@ static GemmPlan pair_plan(int64_t n, int64_t S, int64_t N, int64_t K)
 
 CACTI_API int cacti_hip_gemm_f16_grads_one_launch(int64_t n, int64_t S, int64_t N, int64_t K) { return pair_plan(n, S, N, K).tile >= 0 ? 1 : 0; }
 
+// whether na f16 values at a and nb at b have one in common
+static bool overlap(const void *a, int64_t na, const void *b, int64_t nb)
+{
+    const uintptr_t p = (uintptr_t)a, q = (uintptr_t)b;
+    return na > 0 && nb > 0 && p < q + (uint64_t)nb * sizeof(half_t) && q < p + (uint64_t)na * sizeof(half_t);
+}
+
 CACTI_API int cacti_hip_gemm_f16_grads(int64_t n, int64_t S, int64_t N, int64_t K, const void *const *dy, const void *const *W, const void *x,
                                        float beta_x, void *dx, float beta_w, void *const *dW, void *stream)
 {
@@ -529,8 +536,19 @@ CACTI_API int cacti_hip_gemm_f16_grads(int64_t n, int64_t S, int64_t N, int64_t 
     for (int64_t z = 0; z < n; z++)
         CACTI_REQUIRE(dy[z] && W[z] && dW[z], CACTI_E_INVALID, "gemm_grads: null operand in product %lld", (long long)z);
     CACTI_REQUIRE((beta_x == 0.f || beta_x == 1.f) && (beta_w == 0.f || beta_w == 1.f), CACTI_E_INVALID, "gemm_grads: beta must be 0 or 1");
+    for (int64_t z = 0; z < n; z++) {
+        CACTI_REQUIRE(!overlap(dx, S * K, dy[z], S * N) && !overlap(dx, S * K, W[z], N * K), CACTI_E_INVALID,
+                      "gemm_grads: dx overlaps an operand of product %lld", (long long)z);
+        CACTI_REQUIRE(!overlap(dW[z], N * K, x, S * K) && !overlap(dW[z], N * K, dx, S * K), CACTI_E_INVALID,
+                      "gemm_grads: dW of product %lld overlaps x or dx", (long long)z);
+        for (int64_t y = 0; y < n; y++)
+            CACTI_REQUIRE(!overlap(dW[z], N * K, dy[y], S * N) && !overlap(dW[z], N * K, W[y], N * K) &&
+                              (y == z || !overlap(dW[z], N * K, dW[y], N * K)),
+                          CACTI_E_INVALID, "gemm_grads: dW of product %lld overlaps a tensor of product %lld", (long long)z, (long long)y);
+    }
     const GemmPlan plan = pair_plan(n, S, N, K);
     bool one = plan.tile >= 0 && (n == 1 || beta_x == 0.f) && aligned(x, 16) && aligned(dx, 16);
+    if (overlap(dx, S * K, x, S * K)) one = false;         // every weight gradient has read x before dx takes its place
     for (int64_t z = 0; z < n && one; z++) one = aligned(dy[z], 16) && aligned(W[z], 16) && aligned(dW[z], 16);
     if (!one) {
         for (int64_t z = 0; z < n; z += kMaxPtrBatch) {

@@ -160,11 +160,13 @@ int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M, int64_t 
                                float alpha, const void *const *A, int64_t lda, const void *const *B,
                                int64_t ldb, float beta, void *const *C, int64_t ldc, void *stream);
 /* C = f16(f16(A_0 B_0 + beta C) + A_1 B_1) .. : n products of row-major [M,K] and [K,N] operands that accumulate into one
- * matrix, with the bits of n calls of cacti_hip_gemm_f16 (beta 1 from the second on). */
+ * matrix, with the bits of n calls of cacti_hip_gemm_f16 (beta 1 from the second on).  No element of C is one of an operand. */
 int cacti_hip_gemm_f16_chain(int64_t n, int64_t M, int64_t N, int64_t K, const void *const *A, int64_t lda, const void *const *B,
                              int64_t ldb, float beta, void *C, int64_t ldc, void *stream);
 /* The gradients of n products y_i = x W_i^T with x [S,K], W_i [N,K], contiguous: dW_i = f16(dy_i^T x + beta_w dW_i) and dx the chain
- * above over dy_i W_i; in one launch where that is expected to pay (..._one_launch: 1), with the bits of separate calls. */
+ * above over dy_i W_i; in one launch where that is expected to pay (..._one_launch: 1), with the bits of separate calls, those of dW
+ * before those of dx.  dx may take the place of x (then never in one launch); any other overlap of an output with another tensor
+ * of the call is CACTI_E_INVALID. */
 int cacti_hip_gemm_f16_grads(int64_t n, int64_t S, int64_t N, int64_t K, const void *const *dy, const void *const *W, const void *x,
                              float beta_x, void *dx, float beta_w, void *const *dW, void *stream);
 int cacti_hip_gemm_f16_grads_one_launch(int64_t n, int64_t S, int64_t N, int64_t K);

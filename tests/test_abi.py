@@ -3,6 +3,8 @@ import ctypes
 import os
 import re
 
+import pytest
+
 from cacti_amd import ffi
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -40,6 +42,20 @@ def test_argument_validation_needs_no_gpu():
     rc = L.cacti_hip_silu_gate_fwd(16, None, None, None, None)
     assert rc == -1
     assert L.cacti_hip_rms_norm_bwd_workspace(2048, 3200) == 256 * 3200 * 4
+
+
+@pytest.mark.parametrize("what", ["dx dy0", "dx W1", "dW0 x", "dW1 dx", "dW0 dy1", "dW1 W0", "dW1 W1", "dW1 dW0"])
+@pytest.mark.parametrize("off", [0, 1, -1])
+def test_gradients_that_overlap_other_tensors_are_rejected(what, off):
+    """An output of the gradients in one call on top of a tensor of the call, or with their last and first 16 bytes in common: before any launch."""
+    L, (n, S, N, K) = ffi.lib(), (2, 64, 128, 256)
+    size = {"dy": 2 * S * N, "W": 2 * N * K, "x": 2 * S * K, "dx": 2 * S * K, "dW": 2 * N * K}
+    at = {t: (i + 1) << 24 for i, t in enumerate(["dy0", "dy1", "W0", "W1", "x", "dx", "dW0", "dW1"])}
+    out, other = what.split()
+    at[out] = at[other] + {0: 0, 1: size[other.rstrip("01")] - 16, -1: 16 - size[out.rstrip("01")]}[off]
+    table = lambda t: ctypes.cast((ctypes.c_void_p * n)(at[t + "0"], at[t + "1"]), ctypes.c_void_p)
+    assert L.cacti_hip_gemm_f16_grads(n, S, N, K, table("dy"), table("W"), at["x"], 0.0, at["dx"], 0.0, table("dW"), None) == -1
+    assert b"overlaps" in L.cacti_hip_last_error()
 
 
 def test_edge_shapes_are_rejected_with_a_message():

@@ -683,6 +683,26 @@ def test_gemm_grads_have_the_bits_of_products_one_by_one(ops, n, S, N, K, one, b
         assert_bits(host(dW[z]), host(want_w[z]), "dW %d" % z)
 
 
+@pytest.mark.parametrize("n,S,N,K", [(1, 611, 1024, 1024), (3, 128, 256, 256), (2, 611, 2816, 1024), (2, 600, 1000, 1024)])
+def test_gemm_grads_with_dx_in_place_of_x(ops, n, S, N, K):
+    """The weight gradients are those of x, whether or not the sizes would have one launch of all (the last ones have not)."""
+    import ctypes as C
+    from cacti_amd import ffi
+    say("gemm grads in place", n, S, N, K)
+    g = torch.Generator(device="cuda").manual_seed(n + S + N + K)
+    st = torch.cuda.current_stream().cuda_stream
+    new = lambda *s: torch.randn(*s, device="cuda", generator=g).half()
+    dy, W, x = [new(S, N) for _ in range(n)], [new(N, K) for _ in range(n)], new(S, K)
+    table = lambda ts: C.cast((C.c_void_p * n)(*[t.data_ptr() for t in ts]), C.c_void_p)
+    got = []
+    for dx in (torch.empty_like(x), x):                  # (the second call overwrites x)
+        dW = [torch.empty(N, K, device="cuda", dtype=torch.float16) for _ in range(n)]
+        ffi.call("cacti_hip_gemm_f16_grads", n, S, N, K, table(dy), table(W), x.data_ptr(), 0.0, dx.data_ptr(), 0.0, table(dW), st)
+        got.append([host(t) for t in [dx] + dW])
+    for i, (a, b) in enumerate(zip(*got)):
+        assert_bits(b, a, "dx" if i == 0 else "dW %d" % (i - 1))
+
+
 def test_gemm_colmajor_entry(ops, oracle):
     """The cuBLAS-shaped entry: row-major callers pass operands swapped (thunk/op.rs:4469-4491)."""
     import ctypes as C
