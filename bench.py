@@ -88,6 +88,9 @@ def gemm_traffic_bytes(label, table):
 # "...]x3": three products of that shape staged as one thunk and launched together
 GEMM_RE = re.compile(r"^(block_matmul|matmul)\[([NT])([NT]),(\d+)x(\d+)x(\d+)x(\d+)(,acc)?\](?:x(\d+))?$")
 
+# both gradients of x [S,K] W^T, W [N,K], of that many W in one launch
+GRADS_RE = re.compile(r"^matmul_grads\[(\d+)x(\d+)x(\d+)(,acc[0-9a-f]+)?\]x(\d+)$")
+
 
 def gemm_group(label):
     m = GEMM_RE.match(label)
@@ -95,6 +98,10 @@ def gemm_group(label):
 
 
 def gemm_flops(label):
+    m = GRADS_RE.match(label)
+    if m:
+        S, N, K, n = (int(m.group(i)) for i in (1, 2, 3, 5))
+        return 4.0 * S * N * K * n
     m = GEMM_RE.match(label)
     if not m:
         return None
@@ -140,6 +147,8 @@ def is_split(label):
     """True if the thunk issues two kernels (the columns beyond the full rounds of its tiles go to
     a second launch of smaller tiles): its event pair then brackets both, so it is left out of a
     single kernel's roofline sample."""
+    if GRADS_RE.match(label):                              # several products
+        return True
     ta, tb, H, M, N, K = gemm_dims(label)
     if gemm_group(label) > 1:                              # a grouped thunk: never one launch of one product
         return True

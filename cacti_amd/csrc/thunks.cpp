@@ -454,11 +454,13 @@ struct GradsNSpec : ThunkSpec {
         *in = {a[(size_t)(i % n)], a[(size_t)(i < n ? 2 * n : i)]};
         return make_matmul(i < n, false, 1.f);
     }
-    std::string key(const std::vector<CellType> &aty, uint32_t) const override
+    // ",acc" and the bits of the outputs (dx, dW_1 ..) that are added to, in hexadecimal
+    std::string key(const std::vector<CellType> &aty, uint32_t acc) const override
     {
-        char buf[128];
-        snprintf(buf, sizeof(buf), "matmul_grads[%lldx%lldx%lld]x%d", (long long)aty[0].shape[0], (long long)aty[0].shape[1],
-                 (long long)aty[n].shape[1], n);
+        char buf[128], mode[16] = "";
+        if (acc) snprintf(mode, sizeof(mode), ",acc%x", acc);
+        snprintf(buf, sizeof(buf), "matmul_grads[%lldx%lldx%lld%s]x%d", (long long)aty[0].shape[0], (long long)aty[0].shape[1],
+                 (long long)aty[n].shape[1], mode, n);
         return buf;
     }
 };

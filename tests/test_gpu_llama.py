@@ -191,6 +191,27 @@ def test_grouped_products_run_one_by_one_in_a_pool_too_small_for_the_group():
         assert np.array_equal(g.view(np.uint16), got[0][1][n].view(np.uint16)), n
 
 
+def test_timing_labels_of_gradients_in_one_launch():
+    """The first micro-batch writes the weights' gradients and the second adds to them: timing entries of their own, with the operand
+    bytes of each; the benchmark takes them for the products they are."""
+    import bench
+    S, D, F = 128, 256, 256
+    cfg, flat, tok, lm_tok, scale = make_inputs(dict(S=S, D=D, H=4, Dh=64, F=F, V=512, L=1, eps=1e-6), seed=3, norm_mean=1.0, grad_scale=1024.0)
+    ctx, m = _model(cfg, pool_bytes=1 << 30)
+    m.put_params_flat(flat)
+    ctx.set_timing(2)
+    m.step(tok, lm_tok, scale)
+    m.step(tok, lm_tok, scale, accumulate=True)
+    rep = ctx.timing_report()
+    first, more = "matmul_grads[%dx%dx%d]x3" % (S, D, D), "matmul_grads[%dx%dx%d,acce]x3" % (S, D, D)
+    assert rep[first][0] == 1 and rep[more][0] == 1, sorted(rep)
+    # dy, W and x are read, dx and dW written, the latter read first as well
+    least = 2 * (3 * S * D + 3 * D * D + S * D + S * D + 3 * D * D)
+    assert ctx.operand_bytes[first] == least and ctx.operand_bytes[more] == least + 2 * 3 * D * D
+    assert bench.gemm_flops(first) == bench.gemm_flops(more) == 3 * 2 * 2.0 * S * D * D and bench.is_split(first) and bench.is_split(more)
+    m.close(); ctx.close()
+
+
 def test_attention_scratch_gives_way_to_a_capped_pool(oracle):
     """A pool with room for the least scratch of the attention adjoint, but not for what it is fastest with (26 MB of fp32
     partial sums at 1024 positions, 4 heads of 100): the cycle runs, with the results of the larger pool up to the
