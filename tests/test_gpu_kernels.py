@@ -783,8 +783,8 @@ def test_fused_attention(ops, oracle, S, H, Dh):
     (rows and keys beyond S are masked) and head dims 4 .. 128; accumulation into existing gradients.
     Both ways of loading tiles are covered: straight into LDS (even head counts with Dh % 8 = 4: every other
     head addressed 4 elements before its start, windows of 8, 13 and 16 chunks; Dh % 8 = 0) and through
-    registers (3 heads of 100, 1 head of 4); 448 rows give the dK, dV kernel whole tiles past the diagonal,
-    which run as its in-wave pipeline, and a last tile."""
+    registers (3 heads of 100, 1 head of 4).  On 256 compute units the direct ones are the kernels' of 32 rows per workgroup; the
+    tile kernels beyond those with tiles straight into LDS: TILE_SHAPES."""
     say("fused attention", S, H, Dh)
     r = rng(1200 + S + Dh)
     alpha = float(np.float32(1.0) / np.sqrt(np.float32(Dh)))
@@ -835,11 +835,18 @@ def test_fused_attention(ops, oracle, S, H, Dh):
 SHORT_SHAPES = [(1, 1, 8, 0), (31, 2, 100, 0), (32, 1, 64, 24), (33, 4, 60, 0), (127, 1, 128, 0), (129, 3, 64, 0), (255, 2, 68, 8),
                 (257, 1, 32, 0), (512, 16, 100, 0), (513, 16, 64, 0), (1023, 2, 12, 0), (1024, 8, 64, 0), (1025, 2, 128, 0), (2047, 8, 64, 0),
                 (2048, 2, 128, 8), (2080, 4, 64, 0), (97, 192, 12, 0), (128, 256, 72, 0), (128, 257, 72, 0), (700, 48, 64, 0)]
+# Just past those limits, tiles straight into LDS in the tile kernels (attention.hip), each of its forms for heads to 64, in windows
+# and beyond 112, whole tiles and a ragged last one: 64 rows forward and dQ, 64 keys; 128 rows, 128 keys (to 64: 64 keys, then
+# 128); 64 rows up to 1024 positions; 128 rows, 128 keys up to 128 positions.  Then parts of the queries
+# (default arithmetic) beside the dQ kernel of 32 rows, whole ones and a ragged last one
+TILE_SHAPES = [(1100, 20, 64, 8), (1057, 16, 100, 0), (1531, 16, 128, 0), (1090, 40, 64, 0), (1025, 64, 64, 0), (1090, 32, 100, 0),
+               (1100, 32, 128, 8), (1000, 26, 64, 0), (128, 264, 128, 0),
+               (4001, 1, 64, 0), (4096, 1, 64, 24), (1531, 4, 100, 0), (2001, 2, 100, 8), (1471, 4, 128, 8), (2048, 4, 128, 0)]
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("exact", [False, True])
-@pytest.mark.parametrize("S,H,Dh,gap", SHORT_SHAPES)
+@pytest.mark.parametrize("S,H,Dh,gap", SHORT_SHAPES + TILE_SHAPES)
 def test_attention_of_short_sequences_against_the_register_path(ops, S, H, Dh, gap, exact):
     """Tensors on 16-byte boundaries against the same ones 8 bytes off (tiles through registers, 128 rows): relative L2 to the
     chain in 64 bits of O, dQ, dK, dV no larger, but for the output's own rounding falling otherwise here and there (two sums of
@@ -970,10 +977,10 @@ def test_attention_infinity_in_the_last_row(ops, S, H, Dh, exact):
     assert masks["dv"][1][:, :, 4:8].all() and not masks["dv"][0].any()
 
 
-# The forward and the dQ kernel take 64 query rows per workgroup where their number is at most twice (forward, fast, up to
-# 1024 positions: 7/4 of) the CUs' of an MI355X, 256, and 128 beyond: rows one short of, on and one past the edges of both
-# at few heads, and the 128 rows' form at many small heads (480 workgroups of 64 rows: forward only; 528, 640: both), with
-# tiles straight into LDS, in windows (heads of 12, 100) and, exact, in the other arithmetic
+# Rows one short of, on and one past the edges of 64 and 128 query rows at few heads, which on 256 CUs are the kernels' of 32 rows;
+# at many small heads the tile kernels with 128 rows (64 for dQ at 480 workgroups of 64 rows, and forward in the exact
+# arithmetic; 528, 640: 128 for both), with tiles straight into LDS, in windows (heads of 12, 100) and, exact, in the other
+# arithmetic, all against the restatement of the chain
 @pytest.mark.gpu
 @pytest.mark.parametrize("exact", [False, True])
 @pytest.mark.parametrize("S,H,Dh", [(63, 2, 64), (64, 1, 128), (65, 2, 100), (127, 2, 128), (129, 4, 64), (191, 2, 100), (193, 1, 128),
@@ -1053,9 +1060,12 @@ def test_rope_on_two_tensors_in_one_launch(S, H, Dh):
 
 # dK / dV in parts of the queries (the workspace of ops) against one walk over all of them (the least workspace): parts that
 # begin on the diagonal or past it, of whole tiles and of a ragged last one alone, and accumulation; heads up to 64 (two
-# output tiles) and beyond, in windows too; 577: the fewest tiles that have parts
+# output tiles) and beyond, in windows too.  The first six have room for parts (577: the fewest tiles that have), and a walk that
+# is the better form with either workspace: the same kernel twice
 PART_SHAPES = [(577, 2, 128, True), (1000, 2, 128, False), (1025, 8, 100, False), (641, 4, 36, True), (705, 4, 64, False),
-               (1500, 10, 64, True)]
+               (1500, 10, 64, True),
+               (1531, 4, 100, True), (2001, 2, 100, False), (1471, 4, 128, False), (2048, 4, 128, True), (4001, 1, 64, True),
+               (4096, 1, 64, False)]
 
 
 @pytest.mark.parametrize("S,H,Dh,acc", PART_SHAPES)
@@ -1082,10 +1092,11 @@ def test_attention_bwd_in_parts(ops, S, H, Dh, acc):
         assert rel_l2(host(a), host(b)) < 2e-4 and exact_frac(host(a), host(b)) > 0.95
 
 
-@pytest.mark.parametrize("S,H,Dh", [(577, 2, 128), (1000, 4, 100), (705, 4, 64)])
+# (the last three: the default arithmetic has parts there; the others: room for some)
+@pytest.mark.parametrize("S,H,Dh", [(577, 2, 128), (1000, 4, 100), (705, 4, 64), (1531, 4, 100), (1471, 4, 128), (4001, 1, 64)])
 def test_attention_bwd_exact_has_no_parts(ops, S, H, Dh):
     """The exact arithmetic asks for no scratch for parts and takes the same kernels whatever the workspace: the same bits
-    with the least one and with one that the default arithmetic has parts in."""
+    with the least one and with one that the default arithmetic can have parts in."""
     from cacti_amd import ffi
     best = ffi.lib().cacti_hip_attention_bwd_workspace_best(S, H, Dh)
     least = ffi.lib().cacti_hip_attention_bwd_workspace(S, H)

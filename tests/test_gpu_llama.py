@@ -212,15 +212,17 @@ def test_timing_labels_of_gradients_in_one_launch():
     m.close(); ctx.close()
 
 
-def test_attention_scratch_gives_way_to_a_capped_pool(oracle):
-    """A pool with room for the least scratch of the attention adjoint, but not for what it is fastest with (26 MB of fp32
-    partial sums at 1024 positions, 4 heads of 100): the cycle runs, with the results of the larger pool up to the
+# (1024 positions have room for parts only; a walk over all queries is the better form, so that the smaller pool has what it wants)
+@pytest.mark.parametrize("S,cap,parts", [(1024, 24 << 20, False), (1531, 24400000, True)])
+def test_attention_scratch_gives_way_to_a_capped_pool(oracle, S, cap, parts):
+    """A pool with room for the least scratch of the attention adjoint, but not for what it is fastest with (24.5 MB of fp32
+    partial sums at 1531 positions, 4 heads of 100): the cycle runs, with the results of the larger pool up to the
     order of those sums (fp32, rounded once: rel-L2 below one f16 rounding, 2^-11, through the layer below)."""
     from cacti_amd import ffi
-    big = dict(S=1024, D=400, H=4, Dh=100, F=416, V=512, L=1, eps=1e-6)
+    big = dict(S=S, D=400, H=4, Dh=100, F=416, V=512, L=1, eps=1e-6)
     cfg, flat, tok, lm_tok, scale = make_inputs(big, seed=5, norm_mean=1.0, grad_scale=1024.0)
-    cap = 24 << 20
-    assert ffi.lib().cacti_hip_attention_bwd_workspace_best(1024, 4, 100) > cap > 2 * ffi.lib().cacti_hip_attention_bwd_workspace(1024, 4)
+    assert ffi.lib().cacti_hip_attention_bwd_workspace_best(S, 4, 100) > cap > 2 * ffi.lib().cacti_hip_attention_bwd_workspace(S, 4)
+    assert (ffi.lib().cacti_hip_attention_bwd_workspace_used(S, 4, 100, 400) > cap) == parts
     got = []
     for pool in (1 << 30, cap):
         ctx, m = _model(cfg, pool_bytes=pool)
