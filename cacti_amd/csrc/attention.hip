@@ -1186,11 +1186,11 @@ __global__ void __launch_bounds__(256) attn_bwd_dkv_sum_kernel(AttnArgs p)
 // A workgroup of the dK / dV kernel walks all query tiles from its keys on, 1.4 us each behind some 10 us of start, and
 // a short sequence has few workgroups for it (1000 positions of 4 heads: 32 of up to 16 tiles, on 256 CUs).  There the
 // query tiles of 128 keys go to several workgroups, as many as the device has room for, whose fp32 sums a second launch of
-// 4.6 to 6.6 us adds up.  What it is weighed against is one walk with 64 keys (few_keys: half the work per tile), so a part
-// has to be at least 8 tiles shorter than the walk.  Adjoint with 64 keys -> parts, us: 449 positions, 8 heads of 64 (6
-// tiles shorter) 27.7 -> 28.5; 611, 4 of 64 (8) 29.2 -> 27.8; 1000, 4 of 100 (14) 52 -> 44.6.  split = 1: not.  The exact
-// arithmetic has no parts, and is better with 64 keys than with 128 everywhere there (1000, 4 of 100: 91.5 -> 72.4 us).
-// (Most of these shapes are attention_short.hip's by now; parts are left long sequences of few heads: attention_short_dkv_takes.)
+// 4.6 to 6.6 us adds up.  Against one walk with 64 keys (few_keys: half the work per tile) a part has to be at least 8 tiles
+// shorter than the walk: adjoint with 64 keys -> parts, us, 449 positions, 8 heads of 64 (6 tiles shorter) 27.7 -> 28.5; 611, 4 of
+// 64 (8) 29.2 -> 27.8; 1000, 4 of 100 (14) 52 -> 44.6.  What it is weighed against where it runs is the walk of attention_short.hip,
+// which takes all of those and leaves parts the longest sequences of few heads: attention_short_dkv_takes.  split = 1: not.  The
+// exact arithmetic has no parts.
 struct DkvParts {
     int split, per;
 };
@@ -1224,25 +1224,27 @@ int set_smem(K kern, size_t bytes)
 // agree with the CPU restatement of the reference to 4.9e-5 .. 7.1e-5.
 std::atomic<int> g_exact{0};             // cacti_hip_attention_set_exact: launch the exactly rounded forms
 
-// Query rows per workgroup of the forward and the dQ kernel, 64 or 128, where attention_short.hip does not take the call (it
-// takes the smaller ones of the shapes below).  A workgroup has a CU to itself and walks its keys
+// Query rows per workgroup of the forward and the dQ kernel, 64 or 128, where attention_short.hip does not take the call.  A
+// workgroup has a CU to itself and walks its keys
 // 128 at a time; with 64 rows two waves share a tile's keys, so a step takes less time (one head of 128: 2.1 us against 2.85
 // forward) and there are twice as many workgroups, each of which reads all keys.  Worth it until they need a third round
-// over the CUs: 128 -> 64 rows, us, forward and adjoint, 611 positions, 16 heads of 64 19.2 -> 16.1 and 42.3 -> 35.4; 777,
-// 16 of 128 26.0 -> 20.7 and 62 -> 53; 1534, 16 of 100 41.3 -> 32.2 and 92 -> 85; 1984, 16 of 128 (496 workgroups) 50.8 ->
-// 46.2 and 115 -> 107; 1422, 24 of 100 (552) 38.4 -> 47.5 and 90 -> 94; 2048, 32 of 100 (1024) 68 -> 95 and 156 -> 168.
-// Exact arithmetic: 1531, 16 of 128 71.8 -> 43.7 and 172 -> 134.  Up to 128 positions there is a step or two either way.
-// The forward kernel's second round is short only if there are long sequences in the first: 901, 32 of 100 (480 workgroups)
-// 28.1 -> 29.2, 786 (416) 25.4 -> 25.6.
+// over the CUs: 128 -> 64 rows, us, forward and adjoint (its dQ alone), 1100 positions, 20 heads of 64 (360 workgroups) 30.0 -> 25.6
+// and 56 -> 50; 1531, 16 of 128 (384) 42.9 -> 34.7 and 93 -> 78; 1984, 16 of 128 (496) 54.2 -> 47.8 and 117 -> 107; 4096, 8 of 128
+// (512) 100 -> 84 and 199 -> 184; 1300, 26 of 64 (546) 33.1 -> 41.6 and 64 -> 65; 1422, 24 of 100 (552) 40.8 -> 49.6 and 100 -> 95;
+// 2048, 32 of 100 (1024) 68 -> 95 and 156 -> 168.  Exact arithmetic: 1531, 16 of 128 70.0 -> 45.4 and 143 -> 108; 1000, 26 of 64
+// (416) 45.6 -> 34.1 and 89 -> 70.  Up to 128 positions there is a step or two either way.
+// The forward kernel's second round is short only if there are long sequences in the first.  Up to 1024 positions it is left heads
+// to 64 between 3/2 and 2 workgroups per CU, where the default arithmetic is as good either way from 770 positions on (1000, 25 of
+// 64 28.2 -> 27.0; 832, 32 24.6 -> 24.3; 896, 32 25.7 -> 26.0; 1024, 28 27.8 -> 28.4) and better with 128 rows below (768, 36 of 64
+// 23.4 -> 25.1; 640, 40 21.2 -> 22.6; 450, 52 19.1 -> 21.9).
 int query_rows(int64_t S, int64_t H, bool forward, bool fast)
 {
-    const int64_t cus = device_cus(), wgs = (S + 63) / 64 * H;
-    return S > 128 && wgs <= (forward && fast && S <= 1024 ? cus + cus * 3 / 4 : 2 * cus) ? 64 : 128;
+    return S > (forward && fast ? 1024 : 128) && (S + 63) / 64 * H <= 2 * (int64_t)device_cus() ? 64 : 128;
 }
 
 // Whether the dK / dV kernel takes 64 keys per workgroup instead of 128: its workgroups then walk the same query tiles with
-// half of the work in each (two waves to 32 keys), but without the in-wave pipeline.  Adjoint with 128 -> 64 keys, us: 611
-// positions, 16 heads of 64 37.3 -> 32.2; 777, 16 of 128 53 -> 47; 1531, 16 of 128 (384 workgroups) 86 -> 75; 2048, 16 of 128
+// half of the work in each (two waves to 32 keys), but without the in-wave pipeline.  Adjoint with 128 -> 64 keys, us: 1531
+// positions, 16 heads of 128 (384 workgroups) 86 -> 75; 2048, 16 of 128
 // (512) 113 -> 108; 1051, 32 of 100 (544) 80 -> 87.  Heads to 64 leave registers for two workgroups per CU: 2048, 16 of 64
 // 94 -> 78; 2048, 32 of 64 (1024) 125 -> 117.  Parts of the query tiles, where there are any, are better (dkv_parts).
 bool few_keys(const AttnArgs &p, bool narrow)

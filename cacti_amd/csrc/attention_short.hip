@@ -6,8 +6,9 @@
 // the products are not one, and at 1000 positions of 4 heads 32 workgroups on 256 CUs.  Here a workgroup has 32 rows (keys, for
 // dK and dV), four times as many workgroups, and its 4 or 8 waves split what is walked, block by block of 32: each wave loads
 // its own blocks straight into its own LDS and waits for its own loads alone, so a walk is 1/4 or 1/8 as long and has no
-// barrier, and the waves' sums meet in LDS once at the end.  The rounded scores stay in registers (forward), so that the exact
-// maximum of a row is known before the first exponential: no product is formed twice and nothing is rescaled.
+// barrier, and the waves' sums meet in LDS once at the end.  The rounded scores stay in registers (forward), so that no product is
+// formed twice: a wave sums its exponentials against its own keys' maximum, those sums are rescaled once, where the waves'
+// statistics meet, and the probabilities are formed with the row's maximum and sum.
 // Times, and where the lines between the two lie: at the bottom.
 #include "attention_tile.h"
 

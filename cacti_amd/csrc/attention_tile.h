@@ -329,7 +329,8 @@ __device__ __forceinline__ void load_frags(half8_t (&f)[KS], gptr_t X, int64_t l
 
 // The same fragments out of an LDS tile that holds the operand's rows in window positions (a tile loaded
 // straight into LDS; row = the lane's row inside the tile): what lies outside the head there is the
-// neighbouring heads' data, cleared here.  Rows beyond S are zero in such a tile already.
+// neighbouring heads' data, cleared here.  Rows beyond S are zero in a tile of DmaTileLoader's; in a block of attention_short.hip
+// they are the last row once more, and nothing of theirs is written.
 template <int KS>
 __device__ __forceinline__ void frags_from_tile(half8_t (&f)[KS], const unsigned char *tile, int row, int Dh, int lh,
                                                 int shift)

@@ -837,7 +837,7 @@ SHORT_SHAPES = [(1, 1, 8, 0), (31, 2, 100, 0), (32, 1, 64, 24), (33, 4, 60, 0), 
                 (2048, 2, 128, 8), (2080, 4, 64, 0), (97, 192, 12, 0), (128, 256, 72, 0), (128, 257, 72, 0), (700, 48, 64, 0)]
 # Just past those limits, tiles straight into LDS in the tile kernels (attention.hip), each of its forms for heads to 64, in windows
 # and beyond 112, whole tiles and a ragged last one: 64 rows forward and dQ, 64 keys; 128 rows, 128 keys (to 64: 64 keys, then
-# 128); 64 rows up to 1024 positions; 128 rows, 128 keys up to 128 positions.  Then parts of the queries
+# 128); up to 1024 positions 128 rows forward (exact: 64); 128 rows, 128 keys up to 128 positions.  Then parts of the queries
 # (default arithmetic) beside the dQ kernel of 32 rows, whole ones and a ragged last one
 TILE_SHAPES = [(1100, 20, 64, 8), (1057, 16, 100, 0), (1531, 16, 128, 0), (1090, 40, 64, 0), (1025, 64, 64, 0), (1090, 32, 100, 0),
                (1100, 32, 128, 8), (1000, 26, 64, 0), (128, 264, 128, 0),
