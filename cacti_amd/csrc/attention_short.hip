@@ -209,7 +209,7 @@ __global__ void __launch_bounds__(NW * 64, 2) attn_short_fwd_kernel(AttnArgs p)
 #pragma unroll
     for (int w = 0; w < NW; w++) {
         const float mw = xs[w * 2 * kBlk + l32], lw = xs[(w * 2 + 1) * kBlk + l32];
-        l += mw == -INFINITY ? 0.f : lw * M::ex(mw, m);
+        l += mw == -INFINITY ? lw : lw * M::ex(mw, m);       // (0 then, or NaN of scores that are NaN)
     }
     if (myrow >= S) {
         m = 0.f;

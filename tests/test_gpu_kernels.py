@@ -957,6 +957,23 @@ def test_attention_rows_whose_every_score_overflows(ops, S, H, Dh, exact):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("S,H,Dh,keys", [(33, 2, 128, 1), (65, 3, 64, 1), (161, 2, 64, 1), (225, 1, 128, 1), (128, 4, 64, 32)])
+def test_attention_of_nan_scores_that_are_all_a_wave_has_of_a_row(ops, S, H, Dh, keys):
+    """The last keys of a head are NaN, in a block of 32 keys that is one wave's only one: the rows that see no other key of the
+    block have no softmax, and every gradient they reach is NaN, as in the chain of separate products (default arithmetic; in the
+    other heads nothing is)."""
+    import torch
+    say("attention, NaN scores", S, H, Dh, keys)
+    g = torch.Generator(device="cuda").manual_seed(S + H + Dh)
+    q, k, v, dO = (torch.randn(S, H, Dh, device="cuda", generator=g).half() for _ in range(4))
+    k[S - keys:, 0] = float("nan")
+    masks = _attention_masks(q, k, v, dO, Dh ** -0.5, 0, False)
+    for n, (nan, inf) in masks.items():
+        first = S - keys if n in ("o", "dq") else 0
+        assert nan[first:, 0].all() and nan.sum() == (S - first) * Dh and not inf.any(), n
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("exact", [False, True])
 @pytest.mark.parametrize("S,H,Dh", NOT_FINITE_SHAPES)
 def test_attention_infinity_in_the_last_row(ops, S, H, Dh, exact):
