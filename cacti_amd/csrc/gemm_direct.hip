@@ -961,10 +961,14 @@ GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K)
 }
 
 // What a launch of both is expected to take: the workgroups that the device holds at a time share them all, unless one of the
-// longer product takes longer than that.  Separate launches -> one, us: S = 611, N = K = 1024 12.3 -> 8.0; three of those 23.0 ->
-// 16.9; two of N = 2816 35.9 -> 27.6; 2048, 2048, 2048 40.5 -> 35.0; 333, 3200, 8640 60.2 -> 48.8; three of 128, 256, 256 (four
-// launches) 17.0 -> 6.5.  Larger ones fill the device by themselves, with tiles of their own: three of 2048, 3200, 3200 are 229 us,
-// two of 777, 5504, 2048 99.
+// longer product takes longer than that.  Separate launches -> one, us: S = 611, N = K = 1024 12.0 -> 8.7; three of those 23.7 ->
+// 17.9; two of N = 2816 35.9 -> 28.4; 2048, 2048, 2048 41.4 -> 34.8; 333, 3200, 8640 61.7 -> 49.4; three of 128, 256, 256 (four
+// launches) 16.3 -> 6.5.  Larger ones fill the device by themselves, with tiles of their own, and the long sums of the input
+// gradient share their CUs with the other product's workgroups, which this estimate leaves out: two of 603, 9280, 3200 214 -> 246,
+// two of 777, 8640, 3200 215 -> 233, 1351, 24104, 2048 292 -> 322.  So none beyond 150 us, where 49 products took 0.99 of the time
+// apart in the mean and every third longer, and from 40 us on, where the tile costs are 2 to 3 us off, a gain of 8 % is asked for
+// (1854, 2984, 3200 73 -> 80).  Of 1500 others (S 33 .. 2048, widths 256 .. 3200) 13 are 2 % to 8 % slower as one, by 2 us each at
+// most but for one of 3.5; all 1500 together 6800 us less.
 GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n)
 {
     const int64_t cus = device_cus(), kt_nn = (N + BK - 1) / BK * n, kt_tn = (S + BK - 1) / BK;
@@ -983,7 +987,8 @@ GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n)
         }
     }
     const GemmPlan nn = n > 1 ? gemm_plan_chain(S, K, N, n) : gemm_plan(S, K, N, 1, false), tn = gemm_plan(N, K, S, n, false);
-    if (best.us >= 0.95 * (nn.us + tn.us)) best.tile = -1;
+    const double apart = nn.us + tn.us;
+    if (apart > 150.0 || best.us >= (apart < 40.0 ? 0.95 : 0.92) * apart) best.tile = -1;
     return best;
 }
 

@@ -41,6 +41,14 @@ def test_kernel_names_tell_the_kernels_of_one_tile_shape_apart(M, N, K, how):
     assert bench.kernel_symbol("matmul[NT,1x%dx%dx%d]" % (M, N, K)) == "gemm_direct_kernel<false, true, %s, false>" % how
 
 
+@pytest.mark.parametrize("n,S,N,K,one", [(1, 611, 1024, 1024, 1), (3, 611, 1024, 1024, 1), (2, 611, 2816, 1024, 1), (1, 2048, 2048, 2048, 1),
+                                         (2, 603, 9280, 3200, 0), (1, 1267, 17088, 1600, 0), (2, 777, 8640, 3200, 0), (1, 1351, 24104, 2048, 0),
+                                         (1, 1854, 2984, 3200, 0), (3, 2048, 3200, 3200, 0)])
+def test_all_gradients_in_one_launch_where_that_is_quicker(n, S, N, K, one):
+    """Not where the launches apart are as quick: those of 200 us and more, and one of 73, measured 4 to 15 % slower as one."""
+    assert ffi.lib().cacti_hip_gemm_f16_grads_one_launch(n, S, N, K) == one
+
+
 def test_a_kernel_name_needs_its_room():
     name = C.create_string_buffer(128)
     assert ffi.lib().cacti_hip_gemm_kernel_name(1, 0, 2048, 8640, 3200, 1, name, 20) == -1
