@@ -123,36 +123,34 @@ def gemm_dims(label):
     return (m.group(2) == "T", m.group(3) == "T") + tuple(int(m.group(i)) for i in (4, 5, 6, 7))
 
 
-def gemm_plan(M, N, K):
-    """((tile rows, columns) of the first launch, launches) of a dense product of 16-byte aligned operands."""
+def gemm_launches(label):
+    """(kernel instantiation of the first launch as rocprofv3 prints it, launches) of a label of dense products of 16-byte
+    aligned operands: one product, a group of independent ones, or a chain of input gradients (the groups of that layout).
+    A launch more takes the columns beyond the full rounds of the first one's tiles.  ("", 0): several launches by another rule."""
     import ctypes as C
     from cacti_amd import ffi
-    out = (C.c_int64 * 6)()
-    ffi.call("cacti_hip_gemm_plan", M, N, K, 1, out)
-    return (out[0], out[1]), out[5]
+    ta, tb, H, M, N, K = gemm_dims(label)
+    n, acc = gemm_group(label), ",acc" in label
+    name = C.create_string_buffer(128)
+    if n > 1 and not ta and not tb:
+        count = C.c_int(0)
+        if not acc:
+            ffi.call("cacti_hip_gemm_chain_kernel_name", n, M, N, K, name, len(name), C.byref(count))
+        return name.value.decode(), count.value
+    if H > 1:
+        return "", 0
+    plan = (C.c_int64 * 6)()
+    ffi.call("cacti_hip_gemm_plan", M, N, K, n, plan)
+    ffi.call("cacti_hip_gemm_kernel_name", int(ta), int(tb), M, N, K, n, name, len(name))
+    return name.value.decode(), plan[5]
 
 
 def kernel_symbol(label):
-    """Name of the HIP kernel instantiation a dense GEMM label runs on (its first launch), as
-    rocprofv3 prints it, for 16-byte aligned operands."""
-    import ctypes as C
-    from cacti_amd import ffi
-    ta, tb, H, M, N, K = gemm_dims(label)
-    name = C.create_string_buffer(128)
-    ffi.call("cacti_hip_gemm_kernel_name", int(ta), int(tb), M, N, K, 1, name, len(name))
-    return name.value.decode()
-
-
-def is_split(label):
-    """True if the thunk issues two kernels (the columns beyond the full rounds of its tiles go to
-    a second launch of smaller tiles): its event pair then brackets both, so it is left out of a
-    single kernel's roofline sample."""
-    if GRADS_RE.match(label):                              # several products
-        return True
-    ta, tb, H, M, N, K = gemm_dims(label)
-    if gemm_group(label) > 1:                              # a grouped thunk: never one launch of one product
-        return True
-    return H == 1 and gemm_plan(M, N, K)[1] > 1
+    """Name of the kernel that all of the thunk's work is one launch of, or None: an event pair around several brackets them all."""
+    if not GEMM_RE.match(label) or not label.startswith("matmul"):
+        return None                                        # (both gradients in one launch: products of two layouts)
+    name, launches = gemm_launches(label)
+    return name if launches == 1 else None
 
 
 def label_prefix(label):
@@ -291,7 +289,7 @@ def run_step(args):
         else:
             ent.update(bound="hbm", GBs=ent["bytes"] / sec / 1e9, frac=ent["bytes"] / sec / 1e9 / PEAK_HBM_GBS)
         if fl is not None:
-            if label.startswith("matmul") and not is_split(label):     # one thunk = one launch
+            if kernel_symbol(label):                                   # one thunk = one launch
                 s_ = by_sym.setdefault(kernel_symbol(label), [0.0, set()])
                 s_[0] += tot_ms
                 s_[1].add(label_prefix(label))
@@ -302,8 +300,8 @@ def run_step(args):
     prefix = next(iter(prefixes))
 
     # timed region: exactly K steps, events around every EVENT_STRIDE-th launch of the dominant
-    # kernel (the stride is coprime to the 2 such launches per layer and the 52 per step, so all
-    # shapes are sampled)
+    # kernel's layout (the stride is coprime to the 4 launches of input gradients per layer and the
+    # 105 per step, so all shapes are sampled)
     ctx.set_timing(0)
     ctx.set_timing_filter(prefix, EVENT_STRIDE)
     ctx.set_timing(2)
@@ -327,7 +325,7 @@ def run_step(args):
 
     # the filter matches by label prefix: keep the launches that are exactly one launch of the
     # dominant kernel
-    rep = {label: v for label, v in rep.items() if not is_split(label) and kernel_symbol(label) == sym}
+    rep = {label: v for label, v in rep.items() if kernel_symbol(label) == sym}
     assert rep, "no sampled launch of %s" % sym
     fl = sum(gemm_flops(label) * cnt for label, (cnt, _) in rep.items())
     sec = sum(tot_ms for _, tot_ms in rep.values()) * 1e-3
@@ -542,22 +540,31 @@ def run_mfma_power(args):
 
 
 def run_gemm_traffic(args):
-    """The dense products of the step, each launched gemm_traffic.LAUNCHES times in the order of
+    """The dense products of the step, each (group) launched gemm_traffic.LAUNCHES times in the order of
     gemm_traffic.STEP_PRODUCTS and nothing else: the dispatch sequence `python -m cacti_amd.gemm_traffic`
     expects in the counter files of a rocprofv3 --pmc run over this workload."""
+    import ctypes as C
     import torch
-    from cacti_amd import gemm_traffic, ops
+    from cacti_amd import ffi, gemm_traffic
     g = torch.Generator(device="cuda").manual_seed(0)
     rn = lambda *s: (torch.randn(*s, device="cuda", generator=g) * 0.05).half()
+    st = torch.cuda.current_stream().cuda_stream
+    table = lambda ts: C.cast((C.c_void_p * len(ts))(*[t.data_ptr() for t in ts]), C.c_void_p)
     n = 0
     for label in gemm_traffic.STEP_PRODUCTS:
         ta, tb, _, M, N, K = gemm_dims(label)
-        a = rn(K, M) if ta else rn(M, K)
-        b = rn(N, K) if tb else rn(K, N)
-        out = rn(M, N)
-        beta = 1.0 if label.endswith(",acc]") else 0.0
+        k = gemm_group(label)
+        chain = k > 1 and not ta and not tb
+        # forward the group shares its input (A), the weight gradients share it as B; a chain shares its output
+        a = [rn(K, M) if ta else rn(M, K) for _ in range(1 if tb else k)] * (k if tb else 1)
+        b = [rn(N, K) if tb else rn(K, N) for _ in range(1 if ta else k)] * (k if ta else 1)
+        out = [rn(M, N) for _ in range(1 if chain else k)]
         for _ in range(gemm_traffic.LAUNCHES):
-            ops.gemm(a, b, ta, tb, 1.0, beta, out)
+            if chain:
+                ffi.call("cacti_hip_gemm_f16_chain", k, M, N, K, table(a), K, table(b), N, 0.0, out[0].data_ptr(), N, st)
+            else:
+                ffi.call("cacti_hip_gemm_f16_batched", int(ta), int(tb), k, M, N, K, 1.0, table(a), M if ta else K, table(b), K if tb else N,
+                         0.0, table(out), N, st)
             n += 1
         torch.cuda.synchronize()
     return {"metric": "launches for the traffic counters", "value": n, "unit": "launches", "n_gpus": 1,

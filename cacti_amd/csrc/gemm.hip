@@ -479,32 +479,50 @@ CACTI_API int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M
     return 0;
 }
 
-// One launch where the tiles come straight from memory and every product is of whole k tiles, and where the plans expect less
-// of it than of the launches one by one, which is nearly everywhere: they spend 3.7 to 6 us each on their start and end.
+// Whether a chain of aligned operands goes as its plan says: where every product is of whole k tiles, and where the plans expect
+// less of it than of the launches one by one, which is nearly everywhere: they spend 3.7 to 6 us each on their start and end.
+static bool chain_pays(int64_t n, int64_t M, int64_t N, int64_t K, GemmPlan *plan)
+{
+    if (!(n > 1 && n <= kMaxPtrBatch && M > 0 && N > 0 && K >= 4 * 64 && mult(K, 64) && mult(N, 8))) return false;
+    *plan = gemm_plan_chain(M, N, K, (int)n);
+    return plan->us < (double)n * gemm_plan(M, N, K, 1, false).us;
+}
+
+CACTI_API int cacti_hip_gemm_chain_kernel_name(int64_t n, int64_t M, int64_t N, int64_t K, char *name, size_t bytes, int *launches)
+{
+    CACTI_REQUIRE(name && bytes && launches && n > 0 && M > 0 && N > 0 && K > 0, CACTI_E_INVALID, "gemm_chain_kernel_name: bad argument");
+    GemmPlan plan;
+    name[0] = 0;
+    *launches = 0;
+    if (!chain_pays(n, M, N, K, &plan)) return 0;
+    const int len = gemm_chain_kernel_name(plan, name, bytes);
+    CACTI_REQUIRE(len >= 0 && (size_t)len < bytes, CACTI_E_INVALID, "gemm_chain_kernel_name: %zu bytes are too few for the name", bytes);
+    *launches = plan.cols > 0 ? 2 : 1;
+    return 0;
+}
+
 CACTI_API int cacti_hip_gemm_f16_chain(int64_t n, int64_t M, int64_t N, int64_t K, const void *const *A, int64_t lda, const void *const *B,
                                        int64_t ldb, float beta, void *C, int64_t ldc, void *stream)
 {
     CACTI_REQUIRE(n > 0 && A && B, CACTI_E_INVALID, "gemm_chain: null pointer array or no product");
     for (int64_t z = 0; z < n; z++)
         CACTI_REQUIRE(A[z] && B[z], CACTI_E_INVALID, "gemm_chain: null operand in product %lld", (long long)z);
-    bool one = n > 1 && n <= kMaxPtrBatch && C && M > 0 && N > 0 && K >= 4 * 64 && beta == 0.f && mult(K, 64) && mult(N, 8) && mult(lda, 8) &&
-               mult(ldb, 8) && mult(ldc, 8) && lda >= K && ldb >= N && ldc >= N && lda < kMaxPitch && ldb < kMaxPitch && aligned(C, 16);
+    bool one = C && beta == 0.f && mult(lda, 8) && mult(ldb, 8) && mult(ldc, 8) && lda >= K && ldb >= N && ldc >= N && lda < kMaxPitch &&
+               ldb < kMaxPitch && aligned(C, 16);
     for (int64_t z = 0; z < n && one; z++) one = aligned(A[z], 16) && aligned(B[z], 16);
-    if (one) {
-        const GemmPlan plan = gemm_plan_chain(M, N, K, (int)n);
-        if (plan.us < (double)n * gemm_plan(M, N, K, 1, false).us) {
-            GemmArgs p = {};
-            p.M = M; p.N = N; p.K = K; p.alpha = 1.f;
-            p.A = (const half_t *)A[0]; p.lda = lda;
-            p.B = (const half_t *)B[0]; p.ldb = ldb;
-            p.C = (half_t *)C; p.ldc = ldc;
-            p.chain = (int)n;
-            for (int64_t z = 0; z < n; z++) {
-                p.za[z] = (const half_t *)A[z] - p.A;
-                p.zb[z] = (const half_t *)B[z] - p.B;
-            }
-            return gemm_direct_launch(0, 0, p, 1, plan, (hipStream_t)stream);
+    GemmPlan plan;
+    if (one && chain_pays(n, M, N, K, &plan)) {
+        GemmArgs p = {};
+        p.M = M; p.N = N; p.K = K; p.alpha = 1.f;
+        p.A = (const half_t *)A[0]; p.lda = lda;
+        p.B = (const half_t *)B[0]; p.ldb = ldb;
+        p.C = (half_t *)C; p.ldc = ldc;
+        p.chain = (int)n;
+        for (int64_t z = 0; z < n; z++) {
+            p.za[z] = (const half_t *)A[z] - p.A;
+            p.zb[z] = (const half_t *)B[z] - p.B;
         }
+        return gemm_direct_launch(0, 0, p, 1, plan, (hipStream_t)stream);
     }
     for (int64_t z = 0; z < n; z++) {
         const int rc = cacti_hip_gemm_f16(0, 0, M, N, K, 1.f, A[z], lda, B[z], ldb, z ? 1.f : beta, C, ldc, stream);

@@ -927,6 +927,13 @@ int gemm_kernel_name(int ta, int tb, const GemmPlan &plan, char *name, size_t by
                     s.res, small ? "true" : "false");
 }
 
+int gemm_chain_kernel_name(const GemmPlan &plan, char *name, size_t bytes)
+{
+    const bool small = plan.tile == T64_SMALL;
+    const Shape &s = kShapes[small ? T64 : plan.tile];
+    return snprintf(name, bytes, "gemm_chain_kernel<%d, %d, %d, %s>", s.bm, s.bn, s.res, small ? "true" : "false");
+}
+
 // A program has few shapes and calls them over and over; working one out takes some microseconds (hundreds of costs), so
 // each thread keeps the plans of the last ones by their sizes.
 static GemmPlan kept_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split, int chain)

@@ -123,6 +123,7 @@ GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K);        // for GemmArgs:
 void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn);
 // the kernel of the plan's (first) launch as a profiler prints it; returns what snprintf does
 int gemm_kernel_name(int ta, int tb, const GemmPlan &plan, char *name, size_t bytes);
+int gemm_chain_kernel_name(const GemmPlan &plan, char *name, size_t bytes);
 
 // Products of operands whose rows are at least 8-byte aligned (align = 4; 8: 16-byte aligned), with a triangular operand or
 // a column window among them.

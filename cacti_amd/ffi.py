@@ -59,6 +59,7 @@ SIGNATURES = {
     "cacti_hip_gemm_f16_batched": (ci, [ci, ci, i64, i64, i64, i64, f32, vp, i64, vp, i64, f32, vp, i64, vp]),
     "cacti_hip_gemm_f16_grads": (ci, [i64, i64, i64, i64, vp, vp, vp, f32, vp, f32, vp, vp]),
     "cacti_hip_gemm_f16_grads_one_launch": (ci, [i64, i64, i64, i64]),
+    "cacti_hip_gemm_chain_kernel_name": (ci, [i64, i64, i64, i64, C.c_char_p, sz, C.POINTER(ci)]),
     "cacti_hip_gemm_f16_chain": (ci, [i64, i64, i64, i64, vp, i64, vp, i64, f32, vp, i64, vp]),
     "cacti_hip_gemm_f16_strided_batched": (ci, [ci, ci, i64, i64, i64, i64, f32, vp, i64, i64, vp,
                                                 i64, i64, f32, vp, i64, i64, vp]),

@@ -3,8 +3,8 @@
     python bench.py --workload gemm-traffic          # under rocprofv3 --pmc FETCH_SIZE, then --pmc WRITE_SIZE
     python -m cacti_amd.gemm_traffic <fetch counter_collection.csv> <write counter_collection.csv>
 
-writes cacti_amd/gemm_traffic.json: per timing label of a product the mean FETCH_SIZE and WRITE_SIZE of
-its launches (KiB per dispatch; a product that runs as two launches adds them) and the bytes they stand
+writes cacti_amd/gemm_traffic.json: per timing label of a product, a group or a chain the mean FETCH_SIZE and WRITE_SIZE of
+its launches (KiB per dispatch; one that runs as two launches adds them) and the bytes they stand
 for, bytes = (FETCH_FACTOR * FETCH_SIZE + WRITE_FACTOR * WRITE_SIZE) * 1024: a streaming copy kernel of
 known size reads FETCH_SIZE = half its bytes and WRITE_SIZE = its bytes on this device.  The file also
 records the SHA-256 of csrc/gemm_direct.hip; load_current() returns the table only while that source is
@@ -22,13 +22,14 @@ KERNEL_SOURCE = os.path.join(HERE, "csrc", "gemm_direct.hip")
 LAUNCHES = 4
 FETCH_FACTOR, WRITE_FACTOR = 2.0, 1.0
 
-# timing labels of the dense products of one 3B-shaped step (S = 2048, D = 3200, F = 8640, V = 32000)
+# timing labels of the dense products of one 3B-shaped step (S = 2048, D = 3200, F = 8640, V = 32000); "]x3": a group in one thunk,
+# of the NN layout a chain that adds up in one output
 STEP_PRODUCTS = [
-    "matmul[NT,1x2048x3200x3200]", "matmul[NT,1x2048x8640x3200]", "matmul[NT,1x2048x3200x8640]",
+    "matmul[NT,1x2048x3200x3200]", "matmul[NT,1x2048x3200x3200]x3", "matmul[NT,1x2048x8640x3200]x2", "matmul[NT,1x2048x3200x8640]",
     "matmul[NT,1x2048x32000x3200]",
-    "matmul[NN,1x2048x3200x3200]", "matmul[NN,1x2048x3200x3200,acc]", "matmul[NN,1x2048x3200x8640]",
-    "matmul[NN,1x2048x3200x8640,acc]", "matmul[NN,1x2048x8640x3200]", "matmul[NN,1x2048x3200x32000]",
-    "matmul[TN,1x3200x3200x2048]", "matmul[TN,1x8640x3200x2048]", "matmul[TN,1x3200x8640x2048]",
+    "matmul[NN,1x2048x3200x3200]", "matmul[NN,1x2048x3200x3200]x3", "matmul[NN,1x2048x3200x8640]x2", "matmul[NN,1x2048x8640x3200]",
+    "matmul[NN,1x2048x3200x32000]",
+    "matmul[TN,1x3200x3200x2048]", "matmul[TN,1x3200x3200x2048]x3", "matmul[TN,1x8640x3200x2048]x2", "matmul[TN,1x3200x8640x2048]",
     "matmul[TN,1x32000x3200x2048]",
 ]
 
@@ -53,7 +54,7 @@ def _dispatches(path):
     rows = []
     with open(path) as f:
         for r in csv.DictReader(f):
-            if "gemm_direct_kernel" in r["Kernel_Name"]:
+            if "gemm_direct_kernel" in r["Kernel_Name"] or "gemm_chain_kernel" in r["Kernel_Name"]:
                 rows.append((int(r["Dispatch_Id"]), float(r["Counter_Value"]), r["Kernel_Name"]))
     rows.sort()
     return rows
@@ -81,7 +82,7 @@ def main(argv):
         sys.exit(__doc__)
     sys.path.insert(0, os.path.dirname(HERE))
     import bench
-    per = {l: 2 if bench.is_split(l) else 1 for l in STEP_PRODUCTS}
+    per = {l: bench.gemm_launches(l)[1] for l in STEP_PRODUCTS}
     t = build(argv[1], argv[2], per)
     with open(TABLE, "w") as f:
         json.dump(t, f, indent=1, sort_keys=True)

@@ -163,6 +163,9 @@ int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M, int64_t 
  * matrix, with the bits of n calls of cacti_hip_gemm_f16 (beta 1 from the second on).  No element of C is one of an operand. */
 int cacti_hip_gemm_f16_chain(int64_t n, int64_t M, int64_t N, int64_t K, const void *const *A, int64_t lda, const void *const *B,
                              int64_t ldb, float beta, void *C, int64_t ldc, void *stream);
+/* The kernel of such a chain of 16-byte aligned operands and beta 0 as a profiler prints it, and its launches (1 or 2); none and 0
+ * where the products run one by one. */
+int cacti_hip_gemm_chain_kernel_name(int64_t n, int64_t M, int64_t N, int64_t K, char *name, size_t bytes, int *launches);
 /* The gradients of n products y_i = x W_i^T with x [S,K], W_i [N,K], contiguous: dW_i = f16(dy_i^T x + beta_w dW_i) and dx the chain
  * above over dy_i W_i; in one launch where that is expected to pay (..._one_launch: 1), with the bits of separate calls, those of dW
  * before those of dx.  dx may take the place of x (then never in one launch); any other overlap of an output with another tensor

@@ -41,6 +41,18 @@ def test_kernel_names_tell_the_kernels_of_one_tile_shape_apart(M, N, K, how):
     assert bench.kernel_symbol("matmul[NT,1x%dx%dx%d]" % (M, N, K)) == "gemm_direct_kernel<false, true, %s, false>" % how
 
 
+@pytest.mark.parametrize("label,kernel", [("matmul[NN,1x2048x3200x8640]x2", "gemm_chain_kernel<160, 192, 1, false>"),
+                                          ("matmul[NN,1x128x256x256]x3", "gemm_chain_kernel<64, 64, 2, true>"),
+                                          ("matmul[TN,1x3200x3200x2048]x3", "gemm_direct_kernel<true, false, 256, 256, 1, false, false>"),
+                                          ("matmul[TN,1x8640x3200x2048]x2", None),
+                                          ("matmul[NN,1x2048x3200x8640,acc]x2", None), ("matmul[NN,1x600x1000x1004]x2", None),
+                                          ("matmul_grads[611x1024x1024]x3", None), ("block_matmul[NT,32x2048x2048x100]", None)])
+def test_the_kernel_of_a_group_or_a_chain(label, kernel):
+    """None: several launches, or products of two layouts in one."""
+    import bench
+    assert bench.kernel_symbol(label) == kernel
+
+
 @pytest.mark.parametrize("n,S,N,K,one", [(1, 611, 1024, 1024, 1), (3, 611, 1024, 1024, 1), (2, 611, 2816, 1024, 1), (1, 2048, 2048, 2048, 1),
                                          (2, 603, 9280, 3200, 0), (1, 1267, 17088, 1600, 0), (2, 777, 8640, 3200, 0), (1, 1351, 24104, 2048, 0),
                                          (1, 1854, 2984, 3200, 0), (3, 2048, 3200, 3200, 0)])
@@ -54,3 +66,6 @@ def test_a_kernel_name_needs_its_room():
     assert ffi.lib().cacti_hip_gemm_kernel_name(1, 0, 2048, 8640, 3200, 1, name, 20) == -1
     assert ffi.lib().cacti_hip_gemm_kernel_name(1, 0, 2048, 8640, 3200, 1, name, 128) == 0
     assert name.value == b"gemm_direct_kernel<true, false, 256, 256, 1, false, false>"
+    n = C.c_int(7)
+    assert ffi.lib().cacti_hip_gemm_chain_kernel_name(2, 2048, 3200, 8640, name, 20, C.byref(n)) == -1
+    assert ffi.lib().cacti_hip_gemm_chain_kernel_name(2, 2048, 3200, 8640, name, 128, C.byref(n)) == 0 and n.value == 1

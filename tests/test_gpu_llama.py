@@ -208,7 +208,7 @@ def test_timing_labels_of_gradients_in_one_launch():
     # dy, W and x are read, dx and dW written, the latter read first as well
     least = 2 * (3 * S * D + 3 * D * D + S * D + S * D + 3 * D * D)
     assert ctx.operand_bytes[first] == least and ctx.operand_bytes[more] == least + 2 * 3 * D * D
-    assert bench.gemm_flops(first) == bench.gemm_flops(more) == 3 * 2 * 2.0 * S * D * D and bench.is_split(first) and bench.is_split(more)
+    assert bench.gemm_flops(first) == bench.gemm_flops(more) == 3 * 2 * 2.0 * S * D * D and bench.kernel_symbol(first) is bench.kernel_symbol(more) is None
     m.close(); ctx.close()
 
 
