@@ -84,8 +84,8 @@ __device__ __forceinline__ void st8(half_t *p, const h8 &x) { *reinterpret_cast<
 // Lanes exchange without LDS: through DPP within a row of 16 (quad_perm, row_half_mirror, row_mirror), across the rows and the
 // halves by v_permlane16_swap / v_permlane32_swap of a register with itself, which give both sides in every lane (an exchange
 // through LDS is a hundred cycles and more, one behind another; an fp64 sum was six of two words each); every lane ends with the
-// full result.  32 tokens of 3 layers of 3200 7118 -> 6988 us, a prompt of 1531 and 16 tokens of 4 layers of 2048 3901 -> 3811,
-// against ds_swizzle and ds_bpermute for the last two steps.  T: 4 bytes
+// full result.  32 tokens of 3 layers of 3200 7083 -> 6968 us, a prompt of 1531 and 16 tokens of 4 layers of 2048 3916 -> 3822,
+// 32 tokens of 2 layers of 256 1.8 ms on either side, against ds_swizzle and ds_bpermute for the last two steps.  T: 4 bytes
 template <int CTRL, class T>
 __device__ __forceinline__ T dpp(T v)
 {

@@ -149,8 +149,9 @@ constexpr int kCeThreads = 1024;
 // differences from the maximum below -100 contribute nothing to an fp32 sum that is at least 1.
 // The kernels are bound by their arithmetic as much as by HBM (per element: convert, maximum,
 // exponential, sum, quotient, one-hot, scale, round), hence exp_nonpos and RowDivide, and nothing per element that one lane of a
-// row has a use for (the place of the maximum, the label): 2048 x 32000 forward 56.6 -> 41.2 us (3.2 TB/s),
-// adjoint 66.2 -> 55.5 (4.7 TB/s).
+// row has a use for (the place of the maximum, the label): 2048 x 32000 by itself forward 50.0 -> 37.9 us (3.5 TB/s), adjoint
+// 63.5 -> 52.9 (5.0 TB/s); between the products of an LM head 51.9 -> 36.6 and 61.1 -> 52.0 (trace).  The head as a whole keeps 9
+// of these 24 us: its three products, the same kernels on both sides, take 14 longer behind kernels that idle less.
 template <int CH>
 struct CeRow {
     float e[CH][8];
