@@ -974,8 +974,8 @@ GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K)
 // gradient share their CUs with the other product's workgroups, which this estimate leaves out: two of 603, 9280, 3200 214 -> 246,
 // two of 777, 8640, 3200 215 -> 233, 1351, 24104, 2048 292 -> 322.  So none beyond 150 us, where 49 products took 0.99 of the time
 // apart in the mean and every third longer, and from 40 us on, where the tile costs are 2 to 3 us off, a gain of 8 % is asked for
-// (1854, 2984, 3200 73 -> 80).  Of 1500 others (S 33 .. 2048, widths 256 .. 3200) 13 are 2 % to 8 % slower as one, by 2 us each at
-// most but for one of 3.5; all 1500 together 6800 us less.
+// (1854, 2984, 3200 73 -> 80).  Of 2500 others (S 33 .. 2048, widths 256 .. 3200) 22 are 2 to 13 % slower as one, 59 us together
+// (1961, 2672, 2048 53 -> 60; 80, 3200, 11120, bound by what it reads and writes, 49 -> 55); all of them 70.6 -> 59.2 ms.
 GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n)
 {
     const int64_t cus = device_cus(), kt_nn = (N + BK - 1) / BK * n, kt_tn = (S + BK - 1) / BK;
