@@ -1357,14 +1357,8 @@ int dispatch(int64_t span, bool exact, bool dma, const AttnArgs &p, hipStream_t 
     return dma ? by_size(std::true_type{}, std::true_type{}) : by_size(std::true_type{}, std::false_type{});
 }
 template <int KS, int DT, bool F, bool D> struct Fwd { static int run(const AttnArgs &p, hipStream_t st) { return launch_fwd<KS, DT, F, D>(p, st); } };
+template <int KS, int DT, bool F, bool D> struct BwdDq { static int run(const AttnArgs &p, hipStream_t st) { return launch_dq<KS, DT, F, D>(p, st); } };
 template <int KS, int DT, bool F, bool D> struct BwdDkv { static int run(const AttnArgs &p, hipStream_t st) { return launch_dkv<KS, DT, F, D>(p, st); } };
-template <int KS, int DT, bool F, bool D> struct Bwd {
-    static int run(const AttnArgs &p, hipStream_t st)
-    {
-        const int rc = launch_dq<KS, DT, F, D>(p, st);
-        return rc ? rc : launch_dkv<KS, DT, F, D>(p, st);
-    }
-};
 
 int check_shape(const char *who, int64_t S, int64_t H, int64_t Dh, int64_t ld)
 {
@@ -1494,9 +1488,8 @@ CACTI_API int cacti_hip_attention_bwd(int64_t S, int64_t H, int64_t Dh, float al
     hipStream_t st = (hipStream_t)stream;
     int64_t span;
     const bool dma = direct_tiles(H, Dh, ld, {q, k, v, dO, o, dq, dk, dv}, &span);     // o may be null: passes
-    if (dma && attention_short_dkv_takes(S, H, span, p.split > 1 ? p.per : 0))
-        return (rc = attention_short_dq(p, span, exact, st)) ? rc : attention_short_dkv(p, span, exact, st);
-    if (dma && attention_short_bwd_takes(S, H))
-        return (rc = attention_short_dq(p, span, exact, st)) ? rc : dispatch<BwdDkv>(span, exact, dma, p, st);
-    return dispatch<Bwd>(span, exact, dma, p, st);
+    rc = dma && attention_short_dq_takes(S, H, exact) ? attention_short_dq(p, span, exact, st) : dispatch<BwdDq>(span, exact, dma, p, st);
+    if (rc) return rc;
+    if (dma && attention_short_dkv_takes(S, H, span, p.split > 1 ? p.per : 0)) return attention_short_dkv(p, span, exact, st);
+    return dispatch<BwdDkv>(span, exact, dma, p, st);
 }

@@ -617,17 +617,31 @@ int dispatch(const AttnArgs &p, int64_t span, bool exact, hipStream_t st)
 //   25.8; 512, 64 of 64 (1024) 16.7 -> 17.1; 1024, 64 of 64 (2048) 34.9 -> 41.6.  To 2048: 1536, 4 of 128 (192) 30.4 -> 15.3;
 //   2048, 8 of 64 (512) 33.6 -> 23.4; 1531, 16 of 128 (768) 34.6 -> 32.9; 2048, 16 of 64 (1024) 40.7 -> 43.2.  Beyond 2048 the
 //   rounded scores of a wave's blocks have no room in its registers.
-//   dQ: 128, 4 of 64 10.8 -> 7.4; 3001, 2 of 128 (188) 43.6 -> 25.0; 611, 16 of 64 (320) 16.0 -> 14.3; 400, 32 of 128 (416) 16.0
-//   -> 16.5; 4096, 4 of 64 (512) 43.7 -> 37.3; 640, 32 of 100 (640) 23.0 -> 26.0; 1531, 16 of 128 (768) 34.5 -> 36.1.
-//   dK, dV, parts and their sum together: 128, 4 of 64 10.1 -> 6.2; 777, 16 of 128 (400) 26.4 -> 21.3; 1024, 16 of 64 (512) 27.6 ->
-//   19.3; 2048, 8 of 128 (512) 46.7 -> 41.3; 1000, 24 of 64 (768) 23.5 -> 27.3; 640, 32 of 100 (640) 22.5 -> 30.4.
-//   Exact arithmetic, (512): 512, 32 of 128 18.7 -> 15.0 forward, 44.8 -> 42.8 adjoint; 2048, 8 of 64 47.0 -> 34.5, 106.7 -> 74.1.
+//   The adjoint's workgroups have a CU to themselves, so beyond 256 they come in two rounds, and the second is worth it where the
+//   first one's walks are long (second_round): up to 256 0.54 to 0.90 of the time.
+//   dQ, break-even at 280 workgroups of 500 positions, 320 of 600, 360 of 700, 440 of 800 and 512 of 930: 128, 4 of 64 10.8 -> 7.4;
+//   3001, 2 of 128 (188) 43.6 -> 25.0; 289, 27 of 64 (270) 10.8 -> 13.5; 373, 29 of 128 (348) 12.8 -> 15.6; 504, 26 of 64 (416) 12.7 ->
+//   15.4; 593, 25 of 128 (475) 17.5 -> 20.4; on the other side 611, 16 of 64 (320) 1.00 of the time, 640 to 700 (257 .. 280) 0.93, 750 to
+//   800 (to 340) 0.90 to 0.97, 800 to 900 (to 400) 0.82 to 0.96; 4096, 4 of 64 (512) 43.7 -> 37.3; 640, 32 of 100 (640) 23.0 -> 26.0;
+//   1531, 16 of 128 (768) 34.5 -> 36.1.  Exact, where arithmetic takes more of a block: at 257 of 100 and 512 of 530 (168, 67 of 64 (402)
+//   12.4 -> 15.2; 64 to 200 (257 .. 512) 1.03 to 1.11, 200 to 300 (to 350) 0.96, 300 to 400 (to 450) 0.80 to 0.97).
+//   dK, dV, parts and their sum together, at 257 of 200 and 512 of 630: 128, 4 of 64 10.1 -> 6.2; 777, 16 of 128 (400) 26.4 -> 21.3;
+//   1024, 16 of 64 (512) 27.6 -> 19.3; 2048, 8 of 128 (512) 46.7 -> 41.3; 168, 67 of 64 (402) 9.8 -> 13.0; 64 to 200 (257 .. 450) 1.07 to
+//   1.17, 200 to 300 (to 400) 1.01 to 1.05, 300 to 400 (to 350) 0.86, 500 to 600 (to 450) 0.75 to 0.98, from there to 512 1.01; 1000, 24
+//   of 64 (768) 23.5 -> 27.3; 640, 32 of 100 (640) 22.5 -> 30.4.
+//   Exact arithmetic, (512): 512, 32 of 128 18.7 -> 15.0 forward; 2048, 8 of 64 47.0 -> 34.5, adjoint 106.7 -> 74.1.
 bool attention_short_fwd_takes(int64_t S, int64_t H, int64_t span)
 {
     const int64_t wgs = blocks(S) * H, cus = device_cus();
     return S <= 1024 ? wgs <= (span > 64 ? 4 : 3) * cus : S <= 2048 && wgs <= 2 * cus;
 }
-bool attention_short_bwd_takes(int64_t S, int64_t H) { return blocks(S) * H <= 2 * device_cus(); }
+// The second round of workgroups: as many as the positions beyond `from` are 1/430 of the CUs'.
+static bool second_round(int64_t S, int64_t H, int64_t from)
+{
+    const int64_t wgs = blocks(S) * H, cus = device_cus();
+    return wgs <= cus || (wgs <= 2 * cus && (wgs - cus) * 430 <= (S - from) * cus);
+}
+bool attention_short_dq_takes(int64_t S, int64_t H, bool exact) { return second_round(S, H, exact ? 100 : 500); }
 
 // Against the parts of attention.hip (`per` tiles of 64 queries each; 0: there are none): a wave's walk is blocks / waves long, at
 // 1.7 us each, a part's `per` at 1.5 behind a longer start and the sum's launch.  Workgroups there -> here, us: 1000, 4 of 100
@@ -636,7 +650,7 @@ bool attention_short_bwd_takes(int64_t S, int64_t H) { return blocks(S) * H <= 2
 bool attention_short_dkv_takes(int64_t S, int64_t H, int64_t span, int per)
 {
     const int waves = span <= 64 ? 8 : 4;
-    return attention_short_bwd_takes(S, H) && (per == 0 || (blocks(S) + waves - 1) / waves <= per + 6);
+    return second_round(S, H, 200) && (per == 0 || (blocks(S) + waves - 1) / waves <= per + 6);
 }
 
 int attention_short_fwd(const AttnArgs &p, int64_t span, bool exact, hipStream_t st) { return dispatch<Fwd>(p, span, exact, st); }

@@ -838,10 +838,12 @@ SHORT_SHAPES = [(1, 1, 8, 0), (31, 2, 100, 0), (32, 1, 64, 24), (33, 4, 60, 0), 
 # Just past those limits, tiles straight into LDS in the tile kernels (attention.hip), each of its forms for heads to 64, in windows
 # and beyond 112, whole tiles and a ragged last one: 64 rows forward and dQ, 64 keys; 128 rows, 128 keys (to 64: 64 keys, then
 # 128); up to 1024 positions 128 rows forward (exact: 64); 128 rows, 128 keys up to 128 positions.  Then parts of the queries
-# (default arithmetic) beside the dQ kernel of 32 rows, whole ones and a ragged last one
+# (default arithmetic) beside the dQ kernel of 32 rows, whole ones and a ragged last one.  Then more than one workgroup of 32 rows per
+# CU: the tile dQ kernel (default arithmetic) beside dK / dV of 32 keys, and the tile kernels for both
 TILE_SHAPES = [(1100, 20, 64, 8), (1057, 16, 100, 0), (1531, 16, 128, 0), (1090, 40, 64, 0), (1025, 64, 64, 0), (1090, 32, 100, 0),
                (1100, 32, 128, 8), (1000, 26, 64, 0), (128, 264, 128, 0),
-               (4001, 1, 64, 0), (4096, 1, 64, 24), (1531, 4, 100, 0), (2001, 2, 100, 8), (1471, 4, 128, 8), (2048, 4, 128, 0)]
+               (4001, 1, 64, 0), (4096, 1, 64, 24), (1531, 4, 100, 0), (2001, 2, 100, 8), (1471, 4, 128, 8), (2048, 4, 128, 0),
+               (450, 24, 64, 0), (385, 28, 100, 8), (699, 18, 128, 0), (300, 36, 64, 0), (500, 32, 100, 0), (420, 34, 128, 8)]
 
 
 @pytest.mark.gpu
