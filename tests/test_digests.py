@@ -120,3 +120,38 @@ def test_batched_digests_match_the_oracle_bit_for_bit(ops, oracle):
         assert int(c[i]) == oracle.nan_count(cases[k]), k
     h0, c0 = ops.digests([])
     assert h0.shape == (0, 256) and c0.shape == (0,)
+
+
+@pytest.mark.gpu
+def test_digests_where_a_wave_counts_in_registers(ops):
+    """One class throughout (counters that run as full as they get: 16 sweeps of 1024 pieces, two workgroups at the least number
+    of sweeps each), for each of the 40 classes; and first elements of one class with the classes at and beyond the edges of the
+    16 that a wave then counts in registers behind them, zeros, subnormals and NaNs among them."""
+    import torch
+    r = rng(23)
+    least = [1 << c if c < 10 else (c - 9) << 10 for c in range(40)]
+    n = 2 * 65536 + 8 * 300 + 3
+    xs = []
+    for c, b in enumerate(least):
+        top = (least[c + 1] if c < 39 else 0x7c00) - 1
+        xs.append(r.integers(b, top + 1, n).astype(np.uint16) | (r.integers(0, 2, n) << 15).astype(np.uint16))
+    for c in (0, 5, 9, 10, 14, 15, 16, 24, 38, 39):
+        x = np.full(n, least[c], np.uint16)
+        x[16384:] = [least[k] + (k == c + 1) for k in (c - 15, c - 14, c - 1, c + 1, c + 2) if 0 <= k < 40][0]
+        for k in (c - 15, c - 14, c, c + 1, c + 2):
+            if 0 <= k < 40:
+                x[r.integers(16384, n, 3000)] = least[k]
+        x[r.integers(16384, n, 40)] = 0
+        x[r.integers(16384, n, 40)] = 1
+        x[r.integers(16384, n, 40)] = 0x7e01
+        x[n // 2:n // 2 + 4096] = 0x8000
+        xs.append(x)
+    ds = [torch.from_numpy(x.view(np.int16)).cuda().view(torch.float16) for x in xs]
+    print("digests in registers", len(ds), n, flush=True)
+    h, c = (t.cpu().numpy() for t in ops.digests(ds))
+    for i, x in enumerate(xs):
+        want = np.bincount(bins_from_values(x), minlength=256)
+        assert np.array_equal(h[i], want), i
+        assert int(c[i]) == int(np.isnan(x.view(np.float16)).sum())
+    alone = ops.abs_log2_hist8(ds[-1]).cpu().numpy()
+    assert np.array_equal(alone, h[-1])
