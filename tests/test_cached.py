@@ -524,6 +524,41 @@ def test_full_size_decode_agrees_with_one_call_over_the_same_tokens():
     k.close(); m.close(); ctx.close()
 
 
+# The cut of the decoding attention inside a cached pass, whose projections clear the counters of its parts: up to 256 positions
+# (384 of heads to 64, one or two rows) in one workgroup, then parts of 64, from 1025 on of 128, from 2049 on of 256; one to four
+# rows, a last part of one position, heads that no wave's pieces fill
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Dh,T,cuts", [(8, 100, 1, (256, 257, 320, 321)), (3, 64, 1, (384, 385, 1024, 1025)), (16, 128, 1, (1023, 1025, 2048, 2050)),
+                                         (4, 36, 2, (384, 386, 1024, 1026)), (2, 128, 4, (256, 257, 1025, 2049)), (4, 64, 3, (258, 2048, 2049, 2306))])
+def test_decoding_attention_in_parts_of_a_cached_pass(H, Dh, T, cuts):
+    """Rows decoded at the given lengths against the same rows of one call over the whole text."""
+    from cacti_amd.runtime import Ctx, Llama, LlamaCached
+    D, n = H * Dh, max(cuts)
+    cap = (n + 7) // 8 * 8
+    ctx = Ctx(0, 2 << 30, True)
+    m = Llama(ctx, S=cap, D=D, H=H, Dh=Dh, F=2 * D, V=512, L=2, eps=1e-6)
+    r = np.random.default_rng(H + Dh)
+    for i, (name, shp) in enumerate(m.params):
+        w = r.standard_normal(shp, dtype=np.float32) * (1.0 if name == "embed" else D ** -0.5)
+        m.put_param(i, (w + 1.0 if name.endswith("norm") else w).astype(np.float16))
+    tok = r.integers(0, 512, cap).astype(np.uint16)
+    k = LlamaCached(m, cap)
+    k.set_tokens(tok)
+    k.apply(0, n)
+    ref = k.outputs()["logit"]
+    for c in cuts:
+        print("decode", H, Dh, T, c, flush=True)
+        for _ in range(2):
+            k.reset_state()
+            k.set_tokens(tok)
+            k.apply(0, c - T)
+            k.set_tokens(tok)
+            k.apply(c - T, c)
+            # two orders of the same fp32 sums, as above
+            assert_parity(k.outputs()["logit"], ref[c - T:c], "rows before %d" % c, l2=3e-3, mx=6e-2)
+    k.close(); m.close(); ctx.close()
+
+
 @pytest.mark.gpu
 def test_handles_of_freed_caches_stay_dead(oracle):
     """The caches are cells that live across cycles; once the cached model is closed their handles must name
