@@ -52,9 +52,6 @@ using namespace cacti;
 
 namespace {
 
-// The largest tile that parts of K are formed on (a product that needs a split has few tiles: small ones).
-constexpr int kMaxPartTile = 128 * 128;
-
 // Tile buffers in LDS: D of each operand and one more of the smaller one, as many as RES workgroups per CU leave room for.
 constexpr int buffers(int bm, int bn, int res)
 {
@@ -96,7 +93,8 @@ __device__ __forceinline__ void load_odd(half_t *lds, const half_t *c, int64_t l
 // next product's tiles on their way while the last one's are multiplied.  Launches apart cost a start and an end each (3.7 us
 // with 64 x 64, 5.7 with 160 x 192), the sum's way through memory and the gap between them: three of 611 x 1024 x 1024 21.0 ->
 // 14.2 us, of 777 x 2048 x 2048 41.0 -> 31.6, of 2048 x 3200 x 3200 132 -> 114; two of 2048 x 3200 x 8640 199 -> 195.
-template <bool TA, bool TB, int BM, int BN, int RES, bool M32, bool ANY, bool CHAIN>
+// PART: the sums of a range of k tiles, as fp32 (split_k).
+template <bool TA, bool TB, int BM, int BN, int RES, bool M32, bool ANY, bool CHAIN, bool PART>
 __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
 {
     // the whole argument block in scalar registers before anything else: read field by field where the control
@@ -109,7 +107,7 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
     static_assert(D >= 2 && BM % 32 == 0 && BN % 64 == 0 && (!M32 || (BM == 64 && BN == 64)), "tile shape");
     constexpr bool TR_A = TA, TR_B = !TB;                         // fragments by transposing reads
     constexpr int NA = BM / 32, NB = BN / 32;                     // fragments of a wave
-    constexpr bool PARTS = BM * BN <= kMaxPartTile && !M32 && !CHAIN;
+    static_assert(!PART || (!M32 && !CHAIN), "parts of one product");
     static_assert(!CHAIN || (!ANY && D <= 4), "the first D tiles are of the first product");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     half_t *As = reinterpret_cast<half_t *>(smem_raw);            // [NBA][BM * BK]
@@ -122,7 +120,7 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
     const int product = nk;                                       // CHAIN: k tiles of one
     if constexpr (CHAIN) nk *= p.chain;
     const int part = bz;
-    if (PARTS && p.part) {
+    if constexpr (PART) {
         // the "blocks of the batch" are the parts of K: the same operands, a range of k tiles each
         const int per = p.split_tiles;
         kt0 = part * per;
@@ -491,7 +489,7 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
     }
     sums_done();
 
-    if (PARTS && p.part) {
+    if constexpr (PART) {
         // a lane's 4 consecutive columns of a row are 16 bytes of the part, four lanes a 64-byte run
         float *out = p.part + part * p.M * p.ldp;
 #pragma unroll
@@ -612,12 +610,17 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
 template <bool TA, bool TB, int BM, int BN, int RES, bool M32, bool ANY>
 __global__ void __launch_bounds__(256, RES) gemm_direct_kernel(GemmArgs p)
 {
-    gemm_direct_tile<TA, TB, BM, BN, RES, M32, ANY, false>(p, blockIdx.x);
+    gemm_direct_tile<TA, TB, BM, BN, RES, M32, ANY, false, false>(p, blockIdx.x);
+}
+template <bool TA, bool TB, int BM, int BN, int RES, bool ANY>
+__global__ void __launch_bounds__(256, RES) gemm_part_kernel(GemmArgs p)
+{
+    gemm_direct_tile<TA, TB, BM, BN, RES, false, ANY, false, true>(p, blockIdx.x);
 }
 template <int BM, int BN, int RES, bool M32>
 __global__ void __launch_bounds__(256, RES) gemm_chain_kernel(GemmArgs p)
 {
-    gemm_direct_tile<false, false, BM, BN, RES, M32, false, true>(p, blockIdx.x);
+    gemm_direct_tile<false, false, BM, BN, RES, M32, false, true, false>(p, blockIdx.x);
 }
 // Two products that wait for nothing of each other, in one launch: a gradient of the inputs (NN, of a chain perhaps) and those of
 // the weights (TN).  The one with the longer sums has the first workgroups, so that none of them begins when the others end; the
@@ -633,15 +636,15 @@ __global__ void __launch_bounds__(256, RES) gemm_pair_kernel(PairArgs p)
     const bool first = blockIdx.x < p.second;
     const uint32_t wg = first ? blockIdx.x : blockIdx.x - p.second;
     if (first == (p.tn_first != 0)) {
-        if (wg < (uint32_t)p.tn.walk.wgs) gemm_direct_tile<true, false, BM, BN, RES, M32, false, false>(p.tn, wg);
+        if (wg < (uint32_t)p.tn.walk.wgs) gemm_direct_tile<true, false, BM, BN, RES, M32, false, false, false>(p.tn, wg);
     } else {
-        if (wg < (uint32_t)p.nn.walk.wgs) gemm_direct_tile<false, false, BM, BN, RES, M32, false, CHAIN>(p.nn, wg);
+        if (wg < (uint32_t)p.nn.walk.wgs) gemm_direct_tile<false, false, BM, BN, RES, M32, false, CHAIN, false>(p.nn, wg);
     }
 }
 
 // C = f16(alpha sum of the parts + beta C), four columns per lane; the parts are added in order.  VEC: N and the rows
-// of C allow 8-byte accesses.
-template <bool VEC>
+// of C allow 8-byte accesses.  MOST: parts at most, requested together.
+template <bool VEC, int MOST>
 __global__ void __launch_bounds__(256)
 reduce_parts_kernel(int64_t M, int64_t N, int64_t ldp, int split, const float *__restrict__ part, float alpha, float beta,
                     half_t *__restrict__ C, int64_t ldc)
@@ -649,8 +652,13 @@ reduce_parts_kernel(int64_t M, int64_t N, int64_t ldp, int split, const float *_
     const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= M * ldp) return;
     const int64_t m = i / ldp, n = i - m * ldp;
-    float4_t s = *reinterpret_cast<const float4_t *>(part + i);
-    for (int k = 1; k < split; k++) s += *reinterpret_cast<const float4_t *>(part + k * M * ldp + i);
+    float4_t v[MOST];
+#pragma unroll
+    for (int k = 0; k < MOST; k++) v[k] = *reinterpret_cast<const float4_t *>(part + min(k, split - 1) * M * ldp + i);
+    float4_t s = v[0];
+#pragma unroll
+    for (int k = 1; k < MOST; k++)
+        if (k < split) s += v[k];
     half_t *cp = C + m * ldc + n;
     half4_t o, old = {0, 0, 0, 0};
     const bool has_beta = beta != 0.f;
@@ -701,13 +709,14 @@ __global__ void __launch_bounds__(256) repack_kernel(RepackArgs p)
     *reinterpret_cast<int4_t *>(p.dst[z] + i * 8) = v;
 }
 
-template <bool TA, bool TB, int BM, int BN, int RES, bool M32 = false, bool ANY = false, bool CHAIN = false>
+template <bool TA, bool TB, int BM, int BN, int RES, bool M32 = false, bool ANY = false, bool CHAIN = false, bool PART = false>
 int launch(GemmArgs p, int64_t nblk, hipStream_t st)
 {
     const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     constexpr size_t smem = (size_t)(ANY ? 2 * (BM + BN) : buffers(BM, BN, RES) * (BM + BN) + (BM < BN ? BM : BN)) * BK * sizeof(half_t);
     void (*kern)(GemmArgs);
     if constexpr (CHAIN) kern = gemm_chain_kernel<BM, BN, RES, M32>;
+    else if constexpr (PART) kern = gemm_part_kernel<TA, TB, BM, BN, RES, ANY>;
     else kern = gemm_direct_kernel<TA, TB, BM, BN, RES, M32, ANY>;
     static DeviceOnce attr_set;                   // one per instantiation
     if (!attr_set.fresh()) {
@@ -786,6 +795,37 @@ int launch_pair(const PairArgs &args, int64_t nblk, hipStream_t st)
 // The tiles of a pair, both products' the same.
 constexpr int kPairShapes[] = {T64_SMALL, 0, 3, 5, 7};     // 64 x 64 twice, 64 x 128, 128 x 128, 160 x 128
 
+// The tiles that parts of K are formed on.  The others would be expected to take 0.2 % less in the mean (10 % at most) of the
+// products that have parts.
+constexpr bool has_parts(int tile)
+{
+    for (int t : {0, 1, 4, 6, 7, 9, 12, 13})
+        if (t == tile) return true;
+    return false;
+}
+
+template <bool TA, bool TB, int... I>
+int launch_part_shape(int shape, const GemmArgs &p, int split, hipStream_t st, std::integer_sequence<int, I...>)
+{
+    if (p.any) return launch<TA, TB, 64, 64, 2, false, true, false, true>(p, split, st);
+    int rc = CACTI_E_STATE;
+    auto one = [&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        if constexpr (has_parts(i))
+            if (shape == i) rc = launch<TA, TB, kShapes[i].bm, kShapes[i].bn, kShapes[i].res, false, false, false, true>(p, split, st);
+    };
+    (one(std::integral_constant<int, I>{}), ...);
+    return rc;
+}
+int launch_parts(int ta, int tb, int shape, const GemmArgs &p, int split, hipStream_t st)
+{
+    const auto all = std::make_integer_sequence<int, kNumShapes>();
+    if (!ta && !tb) return launch_part_shape<false, false>(shape, p, split, st, all);
+    if (!ta && tb) return launch_part_shape<false, true>(shape, p, split, st, all);
+    if (ta && !tb) return launch_part_shape<true, false>(shape, p, split, st, all);
+    return launch_part_shape<true, true>(shape, p, split, st, all);
+}
+
 template <bool TA, bool TB, int... I>
 int launch_shape(int shape, const GemmArgs &p, int64_t nblk, hipStream_t st, std::integer_sequence<int, I...>)
 {
@@ -825,19 +865,22 @@ double tile_cost(int64_t cus, int tile, int64_t M, int64_t N, int64_t nz, int64_
 
 constexpr int64_t kSmallOutput = 1 << 18;
 constexpr double kAnyPerTile = 1.45;
+constexpr int kMostParts = 8;
 
-// `best` in up to 8 parts of K on tile t, if that costs less; per_tile: factor on the time per k tile
+// `best` in up to kMostParts parts of K on tile t, if that costs less; per_tile: factor on the time per k tile.  The parts and their
+// sum cost a launch of 3 to 13 us, 2 us per million fp32 values while they are few and half of that beyond.  A gain of 4 % is asked
+// of tiles above 128 x 128, whose time per k tile with a part of the CUs is the least certain (1719 x 1024 x 8256 39.2 -> 43.4 us
+// without).
 void split_k(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, double per_tile, GemmPlan &best, double &best_cost)
 {
-    for (int s = 2; s <= 8; s++) {
+    for (int s = 2; s <= kMostParts; s++) {
         const int64_t per = (kt + s - 1) / s;
         if (per < 4 || (kt + per - 1) / per != s) continue;               // parts of some length, none empty
-        const double fixed = kShapes[t].fixed;
-        const double c = fixed + per_tile * (tile_cost(cus, t, M, N, s, per) - fixed) + 4.0 + (double)(M * N) * s * 8.0 / 4e6;
-        if (c < best_cost) {
+        const double fixed = kShapes[t].fixed, x = (double)(M * N) * s / 1e6;
+        const double c = fixed + per_tile * (tile_cost(cus, t, M, N, s, per) - fixed) + 4.0 + (x < 4.0 ? 2.0 * x : 4.0 + x);
+        if (c * (kShapes[t].bm * kShapes[t].bn > 128 * 128 ? 1.04 : 1.0) < best_cost) {
             best_cost = c;
-            const double us = c;
-            best = {t, T64, 0, s, us};
+            best = {t, T64, 0, s, c};
         }
     }
 }
@@ -847,7 +890,10 @@ void split_k(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, double per_ti
 // columns of the full sets in one launch and the rest on other tiles in a second (2048 x 8640 x 3200: 256 tiles of 256 x
 // 256 and 448 columns); and, where the caller has a workspace (may_split), up to 8 parts of K for products with fewer
 // tiles than CUs and a long K, whose workgroups would otherwise run 100 k tiles one after another on a fraction of the CUs
-// (37 x 3200 x 8640: 25 tiles; the parts and their sum cost a launch and 8 bytes per part and element).
+// (37 x 3200 x 8640: 25 tiles of 64 x 64), or on small tiles, whose operands come over and over again from L2.  With parts on tiles
+// to 256 x 256 and not to 128 x 128 alone, us: 2048 x 3200 x 32000 405 -> 371 (2 parts of 256 x 256 against 160 x 192), of 50000
+// 656 -> 544, 2048 x 2048 x 32000 279 -> 215, 1531 x 2048 x 32000 255 -> 171, 1024 x 3200 x 32000 241 -> 192, 319 x 3200 x 27944
+// 113 -> 79; of 1576 products with up to 4000 rows, widths of models and K to 50000 it changes the parts of 36, 3304 -> 2865 us.
 GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split, int shapes = kNumShapes)
 {
     const int64_t kt = (K + BK - 1) / BK;
@@ -883,7 +929,7 @@ GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, boo
     }
     if (may_split && nz == 1)
         for (int t = T64; t < kNumShapes; t++)
-            if (kShapes[t].bm * kShapes[t].bn <= kMaxPartTile) split_k(cus, t, M, N, kt, 1.0, best, best_cost);
+            if (has_parts(t)) split_k(cus, t, M, N, kt, 1.0, best, best_cost);
     best.us = best_cost;
     return best;
 }
@@ -1016,10 +1062,12 @@ int gemm_direct_launch(int ta, int tb, const GemmArgs &p, int64_t nblk, const Ge
     if (plan.split > 1) {
         GemmArgs q = p;
         q.split_tiles = (int)(((p.K + BK - 1) / BK + plan.split - 1) / plan.split);
-        const int rc = launch_tile(ta, tb, plan.tile, q, plan.split, st);
+        const int rc = launch_parts(ta, tb, plan.tile, q, plan.split, st);
         if (rc) return rc;
         const unsigned grid = (unsigned)((p.M * p.ldp + 1023) / 1024);
-        const auto reduce = p.N % 4 == 0 && p.ldc % 4 == 0 && aligned(p.C, 8) ? reduce_parts_kernel<true> : reduce_parts_kernel<false>;
+        const bool vec = p.N % 4 == 0 && p.ldc % 4 == 0 && aligned(p.C, 8);
+        const auto reduce = plan.split <= 4 ? (vec ? reduce_parts_kernel<true, 4> : reduce_parts_kernel<false, 4>)
+                                            : (vec ? reduce_parts_kernel<true, kMostParts> : reduce_parts_kernel<false, kMostParts>);
         hipLaunchKernelGGL(reduce, dim3(grid), dim3(256), 0, st, p.M, p.N, p.ldp, plan.split, p.part, p.alpha, p.beta, p.C, p.ldc);
         return launch_status("gemm_reduce_parts");
     }

@@ -771,8 +771,11 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
         for (;;) {
             const int r = cacti_hip_gemm_f16_ws(0, 1, T, N, K, 1.f, a, K, w, K, 0.f, y, N, gws, gws_bytes, &need, st);
             if (r || need <= gws_bytes) return r;
-            gws = tmp((int64_t)need, 1);
-            if (!gws) return rc;
+            size_t off;
+            // (a pool without the room: the product as it is without a workspace)
+            if ((off = c.pool_try(need)) == kNoOffset) return cacti_hip_gemm_f16(0, 1, T, N, K, 1.f, a, K, w, K, 0.f, y, N, st);
+            temps.push_back(off);
+            gws = static_cast<char *>(c.dev_ptr(off));
             gws_bytes = need;
         }
     };

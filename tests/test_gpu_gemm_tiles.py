@@ -132,6 +132,21 @@ def test_parts_of_k(M, N, K):
     check(A, B, False, True, ops.gemm(A, B, tb=True))
 
 
+# parts on 96 x 64, 128 x 128, 96 x 128, 160 x 128, 160 x 192, 192 x 256 and 256 x 256 tiles (256 compute units), with rows, columns and
+# a K that no tile divides
+@pytest.mark.gpu
+@pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(1001, 520, 8200), (600, 1000, 16008), (400, 808, 20000), (520, 2008, 20000), (1184, 1352, 7048), (1500, 1000, 12008),
+                                   (1505, 3208, 20000)])
+def test_parts_of_k_on_large_tiles(M, N, K, ta, tb):
+    if ta:
+        M = (M + 7) // 8 * 8
+    A, B, a, b = operands(M, N, K, ta, tb)
+    check(A, B, False, True, ops.gemm(a, b, ta=ta, tb=tb))
+    old = torch.randn(M, N, device="cuda", dtype=torch.float16)
+    check(A, B, False, True, ops.gemm(a, b, ta=ta, tb=tb, beta=1.0, out=old.clone()), old)
+
+
 def test_every_tile_is_some_products():
     """(No GPU.)  The sizes above are looked for; at the largest depth each tile has to be found."""
     assert all(size_for(t, DEPTHS[-1]) for t in TILES)
