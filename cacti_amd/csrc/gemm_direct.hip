@@ -131,8 +131,8 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
     const half_t *B = p.B + (p.ztab ? p.zb[bz] : (int64_t)bz * p.sb);
     half_t *C = p.C + (p.ztab ? p.zc[bz] : (int64_t)bz * p.sc);
     // tile origins: &op[row0][0] for a k-contiguous operand, &op[0][row0] for a strided one
-    const half_t *Ao = TA ? A + m0 : A + m0 * p.lda;
-    const half_t *Bo = TB ? B + n0 * p.ldb : B + n0;
+    const half_t *Ao = TA ? A + m0 : A + (uint64_t)(uint32_t)m0 * (uint32_t)p.lda;
+    const half_t *Bo = TB ? B + (uint64_t)(uint32_t)n0 * (uint32_t)p.ldb : B + n0;
 
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wid & 1, wn = wid >> 1;
@@ -626,13 +626,16 @@ __global__ void __launch_bounds__(256, RES) gemm_chain_kernel(GemmArgs p)
 // the weights (TN).  The one with the longer sums has the first workgroups, so that none of them begins when the others end; the
 // other's begin at a number that keeps their XCDs.
 struct PairArgs {
-    GemmArgs nn, tn;
     uint32_t second;
     int tn_first;
+    GemmArgs nn, tn;
 };
 template <int BM, int BN, int RES, bool M32, bool CHAIN>
 __global__ void __launch_bounds__(256, RES) gemm_pair_kernel(PairArgs p)
 {
+    // a field of each cache line of the argument block, all requested at once: the product's own are read behind a branch
+    asm volatile("" ::"s"(p.second), "s"(p.tn_first), "s"(p.nn.M), "s"(p.nn.B), "s"(p.nn.walk.full), "s"(p.nn.ztab), "s"(p.nn.zc[0]),
+                 "s"(p.nn.part), "s"(p.tn.M), "s"(p.tn.B), "s"(p.tn.walk.full), "s"(p.tn.ztab), "s"(p.tn.zc[0]), "s"(p.tn.part));
     const bool first = blockIdx.x < p.second;
     const uint32_t wg = first ? blockIdx.x : blockIdx.x - p.second;
     if (first == (p.tn_first != 0)) {
@@ -1047,7 +1050,7 @@ GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n)
 
 int gemm_pair_launch(const GemmArgs &nn, const GemmArgs &tn, int64_t nblk, const GemmPlan &plan, hipStream_t st)
 {
-    const PairArgs p = {nn, tn, 0};
+    const PairArgs p = {0, 0, nn, tn};
     switch (plan.tile) {
         case T64_SMALL: return launch_pair<T64_SMALL>(p, nblk, st);
         case 0: return launch_pair<0>(p, nblk, st);

@@ -46,22 +46,33 @@ struct TileWalk {
     }
     __host__ __device__ __forceinline__ void locate(uint32_t wg, int &tm, int &tn, int &bz) const
     {
-        const uint32_t per = (uint32_t)wgs >> 3, rem = wgs & 7, xcd = wg & 7;
+        TileWalk w = *this;
+#ifdef __HIP_DEVICE_COMPILE__
+        // as values, all fetched at once: fields that are read where the control flow first wants them, or by a selected address,
+        // cost up to three dependent reads of the argument block, the first of a cache line that nothing has touched yet
+        asm volatile("" : "+s"(w.wgs), "+s"(w.nz), "+s"(w.ztab), "+s"(w.tiles), "+s"(w.rows), "+s"(w.full), "+s"(w.rest), "+s"(w.per_group),
+                     "+s"(w.by_group.m), "+s"(w.by_group.shift), "+s"(w.by_rows.m), "+s"(w.by_rows.shift), "+s"(w.by_rest.m),
+                     "+s"(w.by_rest.shift));
+        asm volatile("" : "+s"(w.by_tiles.m), "+s"(w.by_tiles.shift), "+s"(w.by_nz.m), "+s"(w.by_nz.shift));
+#endif
+        const uint32_t per = (uint32_t)w.wgs >> 3, rem = w.wgs & 7, xcd = wg & 7;
         uint32_t id = xcd * per + (xcd < rem ? xcd : rem) + (wg >> 3);
         bz = 0;
-        if (ztab) {
-            const uint32_t q = by_nz.div(id);
-            bz = (int)(id - q * nz);
+        if (w.ztab) {
+            const uint32_t q = w.by_nz.div(id);
+            bz = (int)(id - q * w.nz);
             id = q;
-        } else if (nz > 1) {
-            bz = (int)by_tiles.div(id);
-            id -= (uint32_t)bz * tiles;
+        } else if (w.nz > 1) {
+            bz = (int)w.by_tiles.div(id);
+            id -= (uint32_t)bz * w.tiles;
         }
-        const uint32_t group = by_group.div(id), in = id - group * per_group;
-        const int first = (int)group * rows;
-        const uint32_t col = first < full ? by_rows.div(in) : by_rest.div(in);
+        const uint32_t group = w.by_group.div(id), in = id - group * w.per_group;
+        const int first = (int)group * w.rows;
+        const bool whole = first < w.full;
+        const FastDiv by = {whole ? w.by_rows.m : w.by_rest.m, whole ? w.by_rows.shift : w.by_rest.shift};
+        const uint32_t col = by.div(in);
         tn = (int)col;
-        tm = first + (int)(in - col * (first < full ? rows : rest));
+        tm = first + (int)(in - col * (whole ? w.rows : w.rest));
     }
 };
 
