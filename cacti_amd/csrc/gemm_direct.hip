@@ -127,9 +127,19 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
         nk = min(nk, kt0 + per);
         bz = 0;
     }
-    const half_t *A = p.A + (p.ztab ? p.za[bz] : (int64_t)bz * p.sa);
-    const half_t *B = p.B + (p.ztab ? p.zb[bz] : (int64_t)bz * p.sb);
-    half_t *C = p.C + (p.ztab ? p.zc[bz] : (int64_t)bz * p.sc);
+    int64_t za, zb, zc;
+    if (__builtin_expect(p.ztab, 0)) {
+        za = p.za[bz];
+        zb = p.zb[bz];
+        zc = p.zc[bz];
+    } else {
+        za = (int64_t)bz * p.sa;
+        zb = (int64_t)bz * p.sb;
+        zc = (int64_t)bz * p.sc;
+    }
+    const half_t *A = p.A + za;
+    const half_t *B = p.B + zb;
+    half_t *C = p.C + zc;
     // tile origins: &op[row0][0] for a k-contiguous operand, &op[0][row0] for a strided one
     const half_t *Ao = TA ? A + m0 : A + (uint64_t)(uint32_t)m0 * (uint32_t)p.lda;
     const half_t *Bo = TB ? B + (uint64_t)(uint32_t)n0 * (uint32_t)p.ldb : B + n0;

@@ -58,7 +58,7 @@ struct TileWalk {
         const uint32_t per = (uint32_t)w.wgs >> 3, rem = w.wgs & 7, xcd = wg & 7;
         uint32_t id = xcd * per + (xcd < rem ? xcd : rem) + (wg >> 3);
         bz = 0;
-        if (w.ztab) {
+        if (__builtin_expect(w.ztab, 0)) {
             const uint32_t q = w.by_nz.div(id);
             bz = (int)(id - q * w.nz);
             id = q;
