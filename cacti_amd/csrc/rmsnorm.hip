@@ -7,7 +7,7 @@
 //   c1 = f16(dt / r); dr = -sum(dt x)/r^2; ds = dr/(r+r); dsq = ds/D;
 //   c2 = f16(dsq (x+x)); dx = f16(f16(dx_old + c1) + c2)   (or f16(c1 + c2))
 // (rms_norm closure src/librarium/llama.rs:442-451 and its adjoint chain).
-#include "common.h"
+#include "rmsnorm.h"
 #include "softmax_math.h"
 
 using namespace cacti;
@@ -199,9 +199,20 @@ rms_norm_bwd_kernel(int64_t N, int D, const half_t *__restrict__ x, const half_t
 // requested together, as the launch is a chain of latencies (256 rows of 3200 4.6 -> 4.3 us, 77 of 1024 4.6 -> 4.2; norms,
 // rotation and gate of 2048 rows in both directions 98.5 -> 96.9).
 constexpr int kFinCols = 32, kFinSlices = 32, kFinRows = 8;
+// The weights' gradients that a launch sums, one to a row of its grid: a training cycle's norms together, as each sum alone is all
+// latency (two micro-batches of 611 positions, 4 layers of 1024, 18 launches -> 2: 2680 -> 2637 us; 128 positions, 2 layers of
+// 256: 699 -> 686).
+struct DwSums {
+    const float *part[kRmsNormDwSums];
+    half_t *dw[kRmsNormDwSums];
+    uint32_t acc;                              // bit i: dw[i] is added to
+};
 __global__ void __launch_bounds__(kFinCols / 4 * kFinSlices)
-rms_norm_dw_finalize_kernel(int G, int D, const float *__restrict__ part, half_t *dw, int acc)
+rms_norm_dw_finalize_kernel(int G, int D, DwSums p)
 {
+    const float *__restrict__ part = p.part[blockIdx.y];
+    half_t *dw = p.dw[blockIdx.y];
+    const bool acc = p.acc >> blockIdx.y & 1;
     __shared__ float red[kFinSlices][kFinCols];
     const int cg = threadIdx.x & (kFinCols / 4 - 1), slice = threadIdx.x / (kFinCols / 4);
     const int col = blockIdx.x * kFinCols + cg * 4;            // D % 8 == 0: a float4 is whole
@@ -301,11 +312,26 @@ CACTI_API size_t cacti_hip_rms_norm_bwd_workspace(int64_t N, int64_t D)
     return (size_t)((N + kWaves - 1) / kWaves) * (size_t)D * sizeof(float);
 }
 
-CACTI_API int cacti_hip_rms_norm_bwd(int64_t N, int64_t D, const void *x, const void *w, float eps,
-                                     const void *dy, void *dx, int dx_acc, void *dw, int dw_acc,
-                                     void *workspace, size_t workspace_bytes, void *stream)
+namespace cacti {
+int rms_norm_dw_sums(int n, int64_t G, int64_t D, const void *const *part, void *const *dw, uint32_t acc, hipStream_t st)
 {
-    CACTI_REQUIRE(N > 0 && D > 0 && x && w && dy && dx && dw && workspace, CACTI_E_INVALID,
+    CACTI_REQUIRE(n > 0 && n <= kRmsNormDwSums, CACTI_E_INVALID, "rms_norm_dw: %d sums", n);
+    DwSums p = {};
+    for (int i = 0; i < n; i++) {
+        p.part[i] = (const float *)part[i];
+        p.dw[i] = (half_t *)dw[i];
+    }
+    p.acc = acc;
+    hipLaunchKernelGGL(rms_norm_dw_finalize_kernel, dim3((unsigned)((D + kFinCols - 1) / kFinCols), (unsigned)n),
+                       dim3(kFinCols / 4 * kFinSlices), 0, st, (int)G, (int)D, p);
+    return launch_status("rms_norm_dw_finalize");
+}
+}  // namespace cacti
+
+static int rms_norm_bwd(int64_t N, int64_t D, const void *x, const void *w, float eps, const void *dy, void *dx, int dx_acc, void *dw,
+                        int dw_acc, void *workspace, size_t workspace_bytes, void *stream)
+{
+    CACTI_REQUIRE(N > 0 && D > 0 && x && w && dy && dx && workspace, CACTI_E_INVALID,
                   "rms_norm_bwd: null pointer or empty shape");
     CACTI_REQUIRE(D % 8 == 0 && D <= 8192, CACTI_E_NOTIMPL,
                   "rms_norm_bwd: need D %% 8 == 0 and D <= 8192 (D=%lld)", (long long)D);
@@ -320,14 +346,25 @@ CACTI_API int cacti_hip_rms_norm_bwd(int64_t N, int64_t D, const void *x, const 
                       launch_bwd<CH>(N, (int)D, (const half_t *)x, (const half_t *)w, eps,
                                      (const half_t *)dy, (half_t *)dx, dx_acc, (float *)workspace,
                                      st));
-    int rc = launch_status("rms_norm_bwd");
-    if (rc) return rc;
-    const int G = (int)((N + kWaves - 1) / kWaves);
-    hipLaunchKernelGGL(rms_norm_dw_finalize_kernel, dim3((unsigned)((D + kFinCols - 1) / kFinCols)),
-                       dim3(kFinCols / 4 * kFinSlices), 0, st, G, (int)D, (const float *)workspace,
-                       (half_t *)dw, dw_acc);
-    return launch_status("rms_norm_dw_finalize");
+    const int rc = launch_status("rms_norm_bwd");
+    return rc || !dw ? rc : rms_norm_dw_sums(1, (N + kWaves - 1) / kWaves, D, (const void *const *)&workspace, &dw, dw_acc ? 1 : 0, st);
 }
+
+CACTI_API int cacti_hip_rms_norm_bwd(int64_t N, int64_t D, const void *x, const void *w, float eps,
+                                     const void *dy, void *dx, int dx_acc, void *dw, int dw_acc,
+                                     void *workspace, size_t workspace_bytes, void *stream)
+{
+    CACTI_REQUIRE(dw, CACTI_E_INVALID, "rms_norm_bwd: null pointer or empty shape");
+    return rms_norm_bwd(N, D, x, w, eps, dy, dx, dx_acc, dw, dw_acc, workspace, workspace_bytes, stream);
+}
+
+namespace cacti {
+int rms_norm_bwd_parts(int64_t N, int64_t D, const void *x, const void *w, float eps, const void *dy, void *dx, int dx_acc, void *part,
+                       size_t part_bytes, hipStream_t st)
+{
+    return rms_norm_bwd(N, D, x, w, eps, dy, dx, dx_acc, nullptr, 0, part, part_bytes, st);
+}
+}  // namespace cacti
 
 // ---- the same adjoint for callers that cannot allocate ----------------------------------------
 // The fp32 dw partial rows go to a file-scope device array instead of a caller workspace.  The

@@ -11,6 +11,8 @@
 
 #include "../../include/cacti_hip_runtime.h"
 #include "common.h"
+#include "rmsnorm.h"
+#include "thunks.h"
 
 namespace cacti {
 
@@ -1024,6 +1026,7 @@ void Ctx::reset()
     kept_.clear();
     adj_.clear();
     adj_wr_.clear();
+    sums_.clear();
     pc_ = 0;
     compiled_ = false;
     fwd_end_ = 0;
@@ -1121,13 +1124,15 @@ bool Ctx::adj_written(CellPtr primal)
 }
 
 int Ctx::adj_add(const std::vector<CellPtr> &primals, std::unique_ptr<ThunkSpec> spec,
-                 const std::vector<CellPtr> &args)
+                 const std::vector<CellPtr> &args, const std::vector<CellPtr> &more, bool wanted)
 {
     std::vector<CellPtr> outs;
     uint32_t mask = 0;
-    bool any = false;
+    bool any = wanted;
     for (size_t k = 0; k < primals.size(); k++) {
         CellPtr a = adj_of(primals[k]);
+        const int rc = stage_sums_of(a);
+        if (rc) return rc;
         if (a == 0) {
             // no adjoint wanted for this argument: the fused thunk still needs a target
             a = cell_new(cells_[primals[k]].ty, false, "d:unused");
@@ -1139,8 +1144,46 @@ int Ctx::adj_add(const std::vector<CellPtr> &primals, std::unique_ptr<ThunkSpec>
         outs.push_back(a);
     }
     if (!any) return 0;
+    outs.insert(outs.end(), more.begin(), more.end());
     int t = add_thunk(std::move(spec));
     return stage_into(t, args, outs, mask);
+}
+
+int Ctx::adj_sum_later(CellPtr primal, CellPtr rows)
+{
+    const CellPtr a = adj_of(primal);
+    if (a == 0) return 0;
+    int rc = stage_sums_of(a);
+    if (rc) return rc;
+    const CellType &ty = cells_[rows].ty;
+    if (!sums_.empty() && (!(cells_[sums_[0].rows].ty == ty) || sums_.size() == kRmsNormDwSums || (sums_.size() + 1) * ty.bytes() > kSumBytes))
+        if ((rc = stage_sums())) return rc;
+    sums_.push_back({rows, a, adj_wr_[a]});
+    adj_wr_[a] = true;
+    return 0;
+}
+
+int Ctx::stage_sums()
+{
+    if (sums_.empty()) return 0;
+    std::vector<CellPtr> args, outs;
+    std::vector<CellType> ty;
+    uint32_t mask = 0;
+    for (const RowSum &s : sums_) {
+        if (s.acc) mask |= 1u << outs.size();
+        args.push_back(s.rows);
+        outs.push_back(s.adj);
+        ty.push_back(cells_[s.adj].ty);
+    }
+    sums_.clear();
+    return stage_into(add_thunk(make_row_sums(std::move(ty))), args, outs, mask);
+}
+
+int Ctx::stage_sums_of(CellPtr adj)
+{
+    for (const RowSum &s : sums_)
+        if (s.adj == adj) return stage_sums();
+    return 0;
 }
 
 int Ctx::vadd_vjp()
@@ -1159,10 +1202,13 @@ int Ctx::vadd_vjp()
             }
         }
         if (!any) continue;
-        int rc = thunks_[e.thunk]->pop_adj(*this, e, out_adj);
+        int rc = 0;
+        for (const CellPtr a : out_adj)
+            if (a && !rc) rc = stage_sums_of(a);
+        if (!rc) rc = thunks_[e.thunk]->pop_adj(*this, e, out_adj);
         if (rc) return rc;
     }
-    return 0;
+    return stage_sums();
 }
 
 // Liveness: a non-stable, non-kept cell dies after its last use; an Unlive entry frees it

@@ -212,8 +212,13 @@ class Ctx {
     CellPtr adj_of(CellPtr primal);                              // 0 for const cells
     bool adj_written(CellPtr primal);
     // arg_adj[..] += thunk(args): Apply on first write, Accumulate afterwards (src/op.rs:20-188)
+    // `more`: outputs behind the adjoints that are written, not added to; wanted: staged also where no adjoint is
     int adj_add(const std::vector<CellPtr> &primals, std::unique_ptr<ThunkSpec> spec,
-                const std::vector<CellPtr> &args);
+                const std::vector<CellPtr> &args, const std::vector<CellPtr> &more = {}, bool wanted = false);
+    // primal's adjoint += the sum of the rows of `rows` (f32 [G,D], of this cycle).  Such sums are launches of 4 us for some KB of
+    // work, so they wait for others of their shape and go as one thunk: before anything else reads or writes one of the adjoints,
+    // when kRmsNormDwSums of them or kSumBytes of rows have come together, and at the end of the pass.
+    int adj_sum_later(CellPtr primal, CellPtr rows);
     int vadd_vjp();
     int compile();                                               // liveness, src/spine.rs:1435-1478
     int resume(CellPtr *yield_cell);                             // src/spine.rs:1484-1991
@@ -256,6 +261,11 @@ class Ctx {
     const std::map<std::string, std::pair<double, uint64_t>> &timings() const { return times_; }
 
    private:
+    struct RowSum { CellPtr rows, adj; bool acc; };
+    static constexpr size_t kSumBytes = (size_t)32 << 20;
+    std::vector<RowSum> sums_;                       // that wait
+    int stage_sums();
+    int stage_sums_of(CellPtr adj);                  // if adj's is among them
     int run_entry(const Entry &e);
     int run_thunk(const ThunkSpec &sp, const std::vector<CellPtr> &args, const std::vector<CellPtr> &outs, uint32_t acc_mask);
     int host_alloc(Cell &c);

@@ -1,6 +1,7 @@
 #include "thunks.h"
 
 #include "common.h"
+#include "rmsnorm.h"
 
 namespace cacti {
 namespace {
@@ -112,26 +113,63 @@ struct RmsNormBwdSpec : ThunkSpec {
     float eps;
     explicit RmsNormBwdSpec(float e) : eps(e) {}
     const char *name() const override { return "rms_norm_bwd"; }
-    int arity() const override { return 3; }                       // (x, w, dy) -> dx, dw
+    int arity() const override { return 3; }                       // (x, w, dy) -> dx, partial rows of dw
     int nout() const override { return 2; }
+    static CellType parts(const CellType &x)
+    {
+        const size_t bytes = cacti_hip_rms_norm_bwd_workspace(x.shape[0], x.shape[1]);
+        return CellType({(int64_t)(bytes / sizeof(float)) / x.shape[1], x.shape[1]}, F32);
+    }
     int out_ty(const std::vector<CellType> &a, std::vector<CellType> &o) const override
     {
         TY_REQUIRE(a[0] == a[2] && a[0].shape.size() == 2 && a[1].numel() == a[0].shape[1],
                    "rms_norm_bwd: shape mismatch");
-        o = {a[0], a[1]};
+        o = {a[0], parts(a[0])};
         return 0;
     }
-    size_t workspace(const std::vector<CellType> &a) const override
+    int run(Ctx &c, const std::vector<CellType> &aty, void *const *a, const std::vector<CellType> &oty,
+            void *const *o, uint32_t acc, void *, size_t) const override
     {
-        return cacti_hip_rms_norm_bwd_workspace(a[0].shape[0], a[0].shape[1]);
-    }
-    int run(Ctx &c, const std::vector<CellType> &aty, void *const *a, const std::vector<CellType> &,
-            void *const *o, uint32_t acc, void *ws, size_t wsb) const override
-    {
-        return cacti_hip_rms_norm_bwd(aty[0].shape[0], aty[0].shape[1], a[0], a[1], eps, a[2], o[0],
-                                      acc & 1, o[1], (acc >> 1) & 1, ws, wsb, S(c));
+        return rms_norm_bwd_parts(aty[0].shape[0], aty[0].shape[1], a[0], a[1], eps, a[2], o[0], acc & 1, o[1], oty[1].bytes(), c.stream());
     }
 };
+
+// The sums of the partial rows of several norms, each an output like `ty[i]`
+struct RmsNormDwSpec : ThunkSpec {
+    std::vector<CellType> ty;
+    explicit RmsNormDwSpec(std::vector<CellType> t) : ty(std::move(t)) {}
+    const char *name() const override { return "rms_norm_dw"; }
+    int arity() const override { return (int)ty.size(); }
+    int nout() const override { return (int)ty.size(); }
+    int out_ty(const std::vector<CellType> &a, std::vector<CellType> &o) const override
+    {
+        for (size_t i = 0; i < a.size(); i++)
+            TY_REQUIRE(a[i] == a[0] && a[i].dtype == F32 && a[i].shape.size() == 2 && ty[i].dtype == F16 && ty[i].numel() == a[i].shape[1],
+                       "rms_norm_dw: shape mismatch");
+        o = ty;
+        return 0;
+    }
+    int run(Ctx &c, const std::vector<CellType> &aty, void *const *a, const std::vector<CellType> &,
+            void *const *o, uint32_t acc, void *, size_t) const override
+    {
+        return rms_norm_dw_sums((int)ty.size(), aty[0].shape[0], aty[0].shape[1], a, o, acc, c.stream());
+    }
+    int pieces() const override { return (int)ty.size(); }
+    std::unique_ptr<ThunkSpec> piece(int i, const std::vector<CellPtr> &args, std::vector<CellPtr> *of) const override
+    {
+        *of = {args[(size_t)i]};
+        return std::unique_ptr<ThunkSpec>(new RmsNormDwSpec({ty[(size_t)i]}));
+    }
+};
+
+// dx (+)= and the partial rows of dw now, their sum with those of the norms to come
+int norm_adjoint(Ctx &c, float eps, CellPtr x, CellPtr w, CellPtr dy)
+{
+    const bool sum = c.adj_of(w) != 0;
+    const CellPtr rows = c.cell_new(RmsNormBwdSpec::parts(c.cell(x).ty), false, "dw rows");
+    const int rc = c.adj_add({x}, std::unique_ptr<ThunkSpec>(new RmsNormBwdSpec(eps)), {x, w, dy}, {rows}, sum);
+    return rc || !sum ? rc : c.adj_sum_later(w, rows);
+}
 
 struct RmsNormSpec : ThunkSpec {
     float eps;
@@ -153,8 +191,7 @@ struct RmsNormSpec : ThunkSpec {
     }
     int pop_adj(Ctx &c, const Entry &e, const std::vector<CellPtr> &dy) const override
     {
-        return c.adj_add({e.args[0], e.args[1]}, std::unique_ptr<ThunkSpec>(new RmsNormBwdSpec(eps)),
-                         {e.args[0], e.args[1], dy[0]});
+        return norm_adjoint(c, eps, e.args[0], e.args[1], dy[0]);
     }
 };
 
@@ -186,8 +223,7 @@ struct AddRmsNormSpec : ThunkSpec {
     int pop_adj(Ctx &c, const Entry &e, const std::vector<CellPtr> &dy) const override
     {
         if (dy[1]) {
-            int rc = c.adj_add({e.outs[0], e.args[2]}, std::unique_ptr<ThunkSpec>(new RmsNormBwdSpec(eps)),
-                               {e.outs[0], e.args[2], dy[1]});
+            const int rc = norm_adjoint(c, eps, e.outs[0], e.args[2], dy[1]);
             if (rc) return rc;
         }
         if (!c.adj_written(e.outs[0])) return 0;
@@ -872,6 +908,7 @@ struct SoftmaxCeSpec : ThunkSpec {
 }  // namespace
 
 std::unique_ptr<ThunkSpec> make_embed() { return std::unique_ptr<ThunkSpec>(new EmbedSpec()); }
+std::unique_ptr<ThunkSpec> make_row_sums(std::vector<CellType> ty) { return std::unique_ptr<ThunkSpec>(new RmsNormDwSpec(std::move(ty))); }
 std::unique_ptr<ThunkSpec> make_rms_norm(float eps)
 {
     return std::unique_ptr<ThunkSpec>(new RmsNormSpec(eps));

@@ -9,6 +9,7 @@ namespace cacti {
 
 std::unique_ptr<ThunkSpec> make_embed();                              // (W, tok) -> y
 std::unique_ptr<ThunkSpec> make_rms_norm(float eps);                  // (x, w) -> y
+std::unique_ptr<ThunkSpec> make_row_sums(std::vector<CellType> ty);   // f32 [G,D] each -> f16 sums of their rows, of types ty
 std::unique_ptr<ThunkSpec> make_matmul(bool ta, bool tb, float alpha);   // (a, b) -> c, 2-d
 std::unique_ptr<ThunkSpec> make_block_matmul(bool ta, bool tb, float alpha, int64_t H);   // [R,H*C]
 std::unique_ptr<ThunkSpec> make_linear();                             // x W^T, both gradients in one launch where that pays

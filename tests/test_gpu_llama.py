@@ -115,6 +115,30 @@ def test_grouped_products_of_a_ragged_sequence_are_the_separate_thunks_bit_for_b
             assert np.array_equal(g.view(np.uint16), got[0][1][n].view(np.uint16)), (groups, n)
 
 
+@pytest.mark.parametrize("L,thunks", [(7, 1), (8, 2)])
+def test_norm_gradients_summed_together(oracle, L, thunks):
+    """The sums of the norms' weight gradients wait for one another, up to 16 (7 layers have 15 norms, 8 have 17): each no further
+    from the oracle than its own other summation orders are, and twice itself, bit for bit, once a second cycle of the same batch
+    has added to it."""
+    from tests.envelope import order_envelope
+    cfg, flat, tok, lm_tok, scale = make_inputs(dict(S=41, D=64, H=2, Dh=32, F=176, V=256, L=L, eps=1e-6), seed=L, norm_mean=1.0,
+                                                grad_scale=64.0)
+    ref = oracle.llama_step(cfg, flat, tok, lm_tok, scale)
+    ctx, m = _model(cfg)
+    m.put_params_flat(flat)
+    m.step(tok, lm_tok, scale)
+    assert ctx.log_names().count("rms_norm_dw") == thunks
+    _, env = order_envelope(oracle, cfg, flat, tok, lm_tok, scale)
+    once, want = m.grads(), oracle.split_params(cfg, ref["grad"])
+    for name in [n for n in once if n.endswith("norm")]:
+        assert rel_l2(once[name], want[name]) <= env[name][0], name
+    m.step(tok, lm_tok, scale, accumulate=True)
+    for name, g in m.grads().items():
+        if name.endswith("norm"):
+            assert np.array_equal(g, once[name] + once[name]), name
+    m.close(); ctx.close()
+
+
 def test_tiny_llama_literal_config(oracle):
     """The reference's small training configuration as written: every weight ~N(0, 0.02), loss scale 1/(S-1).
     The q/k/gate/up/down gradients (1e-8 .. 1e-11) underflow f16 in the reference's own
