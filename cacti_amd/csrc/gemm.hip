@@ -531,12 +531,16 @@ CACTI_API int cacti_hip_gemm_f16_chain(int64_t n, int64_t M, int64_t N, int64_t 
     return 0;
 }
 
-static GemmPlan pair_plan(int64_t n, int64_t S, int64_t N, int64_t K)
+static GemmPlan pair_plan(int64_t n, int64_t S, int64_t N, int64_t K, size_t lent = 0)
 {
     const bool fits = n >= 1 && n <= kMaxPtrBatch && S > 0 && N > 0 && K > 0 && mult(N, n > 1 ? 64 : 8) && (n == 1 || N >= 4 * 64) &&
                       mult(K, 8) && N < kMaxPitch && K < kMaxPitch;
-    return fits ? gemm_plan_pair(S, N, K, (int)n) : GemmPlan{-1, 0, 0, 1, 0};
+    return fits ? gemm_plan_pair(S, N, K, (int)n, lent) : GemmPlan{-1, 0, 0, 1, 0};
 }
+
+namespace cacti {
+bool gemm_pair_pays(int64_t S, int64_t N, int64_t K, int n, size_t lent) { return pair_plan(n, S, N, K, lent).tile >= 0; }
+}  // namespace cacti
 
 CACTI_API int cacti_hip_gemm_f16_grads_one_launch(int64_t n, int64_t S, int64_t N, int64_t K) { return pair_plan(n, S, N, K).tile >= 0 ? 1 : 0; }
 

@@ -1035,7 +1035,7 @@ GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K)
 // apart in the mean and every third longer, and from 40 us on, where the tile costs are 2 to 3 us off, a gain of 8 % is asked for
 // (1854, 2984, 3200 73 -> 80).  Of 2500 others (S 33 .. 2048, widths 256 .. 3200) 22 are 2 to 13 % slower as one, 59 us together
 // (1961, 2672, 2048 53 -> 60; 80, 3200, 11120, bound by what it reads and writes, 49 -> 55); all of them 70.6 -> 59.2 ms.
-GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n)
+GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n, size_t lent)
 {
     const int64_t cus = device_cus(), kt_nn = (N + BK - 1) / BK * n, kt_tn = (S + BK - 1) / BK;
     const bool small_nn = S * K <= kSmallOutput, small_tn = N * K <= kSmallOutput;
@@ -1052,7 +1052,9 @@ GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n)
             best.us = us;
         }
     }
-    const GemmPlan nn = n > 1 ? gemm_plan_chain(S, K, N, n) : gemm_plan(S, K, N, 1, false), tn = gemm_plan(N, K, S, n, false);
+    GemmPlan nn = n > 1 ? gemm_plan_chain(S, K, N, n) : gemm_plan(S, K, N, 1, lent > 0);
+    if ((size_t)nn.split * (size_t)S * (size_t)K * sizeof(float) > lent && nn.split > 1) nn = gemm_plan(S, K, N, 1, false);
+    const GemmPlan tn = gemm_plan(N, K, S, n, false);
     const double apart = nn.us + tn.us;
     if (apart > 150.0 || best.us >= (apart < 40.0 ? 0.95 : 0.92) * apart) best.tile = -1;
     return best;

@@ -128,8 +128,10 @@ struct GemmPlan {
 // nz: products of this shape in the launch
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split);
 GemmPlan gemm_plan_chain(int64_t M, int64_t N, int64_t K, int chain);       // chain <= kMaxPtrBatch products that add up
-// the gradients of n products x W_i^T, x [S,K], W_i [N,K], all in one launch (tile < 0: no better than two)
-GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n);
+// the gradients of n products x W_i^T, x [S,K], W_i [N,K], all in one launch (tile < 0: no better than two, the input gradient of a
+// single product among them with `lent` bytes for parts of K)
+GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n, size_t lent);
+bool gemm_pair_pays(int64_t S, int64_t N, int64_t K, int n, size_t lent);
 GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K);        // for GemmArgs::any (with parts of K)
 void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn);
 // the kernel of the plan's (first) launch as a profiler prints it; returns what snprintf does

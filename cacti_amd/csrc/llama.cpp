@@ -472,7 +472,7 @@ CACTI_API int cacti_llama_stage(cacti_llama *m, int want_prob, int want_grad)
         add_a = add_b = 0;
         return 0;
     };
-    auto linear = [&]() { return m->group_products >= 2 ? make_linear() : make_matmul(false, true, 1.f); };
+    auto linear = [&]() { return make_linear(m->group_products >= 2); };
     TRY(ap(c, make_embed(), {m->embed, m->in_tok}, &stream));
     for (size_t l = 0; l < m->layers.size(); l++) {
         const LayerCells &w = m->layers[l];

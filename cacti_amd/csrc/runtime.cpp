@@ -154,6 +154,7 @@ Ctx::~Ctx()
     }
     staging_give_back(&staging_);
     if (base_) hipFree(base_);
+    if (product_scratch_) hipFree(product_scratch_);
     if (own_stream_ && stream_) hipStreamDestroy(stream_);
     if (counted_) live_contexts_add(dev_, -1);
 }
@@ -923,6 +924,17 @@ int Ctx::spill_eagerly(const Entry &e)
         if (rc) return rc;
     }
     return 0;
+}
+
+void *Ctx::product_scratch(size_t bytes)
+{
+    if (bytes > kProductScratch || no_product_scratch_) return nullptr;
+    if (!product_scratch_ && hipMalloc(&product_scratch_, kProductScratch) != hipSuccess) {
+        (void)hipGetLastError();
+        product_scratch_ = nullptr;
+        no_product_scratch_ = true;
+    }
+    return product_scratch_;
 }
 
 size_t Ctx::pinned_bytes() const

@@ -178,6 +178,11 @@ class Ctx {
     int pool_alloc(size_t bytes, size_t *off, bool high = false);                   // with soft-OOM eviction
     size_t pool_try(size_t bytes, bool high = false);            // likewise; kNoOffset and no report when it does not fit
     void pool_free(size_t off) { pool_.free(off); }              // later reuse is ordered on the stream
+    // Device memory beside the pool for the parts of products, so that how a product is cut, and with it its bits, does not depend
+    // on what the pool has room for: taken when the first product asks for it, kept until the context goes.  Thunks run one
+    // after another on the stream, so one serves them all.  Null: beyond kProductScratch, or the device has no more memory.
+    static constexpr size_t kProductScratch = (size_t)64 << 20;
+    void *product_scratch(size_t bytes);
     size_t pinned_bytes() const;                                 // of the cells of the running thunk
     int try_soft_oom(size_t need);
     int evict(CellPtr c);                                        // VMem -> Mem, drop VMem
@@ -330,6 +335,8 @@ class Ctx {
     std::map<std::string, std::pair<double, uint64_t>> times_;
     std::map<std::string, uint64_t> op_bytes_;                   // label -> operand bytes of one launch
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
+    void *product_scratch_ = nullptr;
+    bool no_product_scratch_ = false;
     Staging staging_;                                            // for read-backs
     // cell_ingest: two page-locked staging buffers and the event after the last upload from each
     void *ingest_host_[2] = {nullptr, nullptr};

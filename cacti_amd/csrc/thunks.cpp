@@ -1,6 +1,7 @@
 #include "thunks.h"
 
 #include "common.h"
+#include "gemm_internal.h"
 #include "rmsnorm.h"
 
 namespace cacti {
@@ -251,6 +252,7 @@ struct MatMulSpec : ThunkSpec {
     bool blocked;
     float alpha;
     int causal;
+    bool lend = false;               // a workspace for parts of K (Ctx::product_scratch), where the product asks for one
     MatMulSpec(bool a, bool b, float al, int64_t h, int cz = CAUSAL_NONE)
         : ta(a), tb(b), nblk(h), blocked(h > 0), alpha(al), causal(cz) {}
     const char *name() const override { return blocked ? "block_matmul" : "matmul"; }
@@ -291,6 +293,16 @@ struct MatMulSpec : ThunkSpec {
         Dims d;
         int rc = dims(aty, d);
         if (rc) return rc;
+        if (lend && !blocked) {
+            size_t need = 0;
+            void *ws = nullptr;
+            auto product = [&]() {
+                return cacti_hip_gemm_f16_ws(ta, tb, d.M, d.N, d.K, alpha, a[0], d.lda, a[1], d.ldb, (acc & 1) ? 1.f : 0.f, o[0], d.ldc, ws,
+                                             need, &need, S(c));
+            };
+            if ((rc = product()) || need == 0) return rc;
+            if ((ws = c.product_scratch(need))) return product();
+        }
         const int tri = causal == CAUSAL_OUT ? 1 : causal == CAUSAL_A ? (ta ? 3 : 2) : 0;
         return cacti_hip_gemm_f16_strided_batched_tri(ta, tb, d.H, d.M, d.N, d.K, alpha, a[0],
                                                       d.lda, d.sa, a[1], d.ldb, d.sb,
@@ -500,12 +512,16 @@ struct GradsNSpec : ThunkSpec {
         return buf;
     }
 };
+// whether the gradients of n products x W_i^T are one launch (apart, a single one's input gradient is lent a workspace)
+static bool one_launch(const CellType &dy, const CellType &w, int n)
+{
+    return gemm_pair_pays(dy.shape[0], dy.shape[1], w.shape[1], n, n > 1 ? 0 : Ctx::kProductScratch);
+}
 // the gradients of y_i = x W_i^T for the dy in `dy`, last product first, as one thunk if one launch of them pays; *staged: it did
 static int stage_grads(Ctx &c, CellPtr x, const std::vector<CellPtr> &ws, const std::vector<CellPtr> &dy, bool *staged)
 {
-    const CellType &g = c.cell(dy[0]).ty, &w = c.cell(ws[0]).ty;
     const int n = (int)ws.size();
-    *staged = cacti_hip_gemm_f16_grads_one_launch(n, g.shape[0], g.shape[1], w.shape[1]) != 0;
+    *staged = one_launch(c.cell(dy[0]).ty, c.cell(ws[0]).ty, n);
     if (!*staged) return 0;
     std::vector<CellPtr> primals = {x}, in(dy.rbegin(), dy.rend());
     primals.insert(primals.end(), ws.rbegin(), ws.rend());
@@ -588,14 +604,22 @@ struct ProjNSpec : ThunkSpec {
 };
 
 // ---------------------------------------------------------------------------
-// y = x W^T whose gradients are one thunk where one launch of both pays
+// y = x W^T of a layer: its gradients are one thunk where one launch of both pays (`one`), and it and its input gradient are lent a
+// workspace, the sums of few rows over a long K being the work of a few CUs otherwise: cycles of 48 x 256 (vocabulary 21480) 958 ->
+// 934 us, 80 x 1024 (29848) 2907 -> 2769, 112 x 768 (31600) 819 -> 758, 160 x 2048 (31432) 1229 -> 1125, 2048 x 3200 (32000, 4
+// layers) 9238 -> 9125.  (Products that have a grouped form are lent
+// none: alone, they have the group's bits.  So has the input gradient where the launch of both would pay.)
 struct LinearSpec : MatMulSpec {
-    LinearSpec() : MatMulSpec(false, true, 1.f, 0) {}
+    bool one;
+    explicit LinearSpec(bool o) : MatMulSpec(false, true, 1.f, 0), one(o) { lend = true; }
     int pop_adj(Ctx &c, const Entry &e, const std::vector<CellPtr> &dy) const override
     {
         bool staged = false;
-        const int rc = stage_grads(c, e.args[0], {e.args[1]}, {dy[0]}, &staged);
-        return rc || staged ? rc : MatMulSpec::pop_adj(c, e, dy);
+        int rc = one ? stage_grads(c, e.args[0], {e.args[1]}, {dy[0]}, &staged) : 0;
+        if (rc || staged || (rc = c.adj_add({e.args[1]}, mm(true, false), {dy[0], e.args[0]}))) return rc;
+        std::unique_ptr<MatMulSpec> dx(new MatMulSpec(false, false, 1.f, 0));
+        dx->lend = !one_launch(c.cell(dy[0]).ty, c.cell(e.args[1]).ty, 1);
+        return c.adj_add({e.args[0]}, std::move(dx), {dy[0], e.args[1]});
     }
 };
 
@@ -917,7 +941,7 @@ std::unique_ptr<ThunkSpec> make_matmul(bool ta, bool tb, float alpha)
 {
     return std::unique_ptr<ThunkSpec>(new MatMulSpec(ta, tb, alpha, 0));
 }
-std::unique_ptr<ThunkSpec> make_linear() { return std::unique_ptr<ThunkSpec>(new LinearSpec()); }
+std::unique_ptr<ThunkSpec> make_linear(bool one) { return std::unique_ptr<ThunkSpec>(new LinearSpec(one)); }
 std::unique_ptr<ThunkSpec> make_projections(int n, bool group_adjoints)
 {
     return std::unique_ptr<ThunkSpec>(new ProjNSpec(n, group_adjoints));

@@ -12,7 +12,7 @@ std::unique_ptr<ThunkSpec> make_rms_norm(float eps);                  // (x, w) 
 std::unique_ptr<ThunkSpec> make_row_sums(std::vector<CellType> ty);   // f32 [G,D] each -> f16 sums of their rows, of types ty
 std::unique_ptr<ThunkSpec> make_matmul(bool ta, bool tb, float alpha);   // (a, b) -> c, 2-d
 std::unique_ptr<ThunkSpec> make_block_matmul(bool ta, bool tb, float alpha, int64_t H);   // [R,H*C]
-std::unique_ptr<ThunkSpec> make_linear();                             // x W^T, both gradients in one launch where that pays
+std::unique_ptr<ThunkSpec> make_linear(bool one);   // x W^T with a workspace; `one`: both gradients in one launch where that pays
 // n products x W_i^T of one shape in one launch: (x, W_1 .. W_n) -> (y_1 .. y_n), 2 <= n <= 4; group_adjoints: their weight
 // gradients, and their input gradients, as one thunk each, or all as one (else the adjoint thunks of n separate matmul thunks)
 std::unique_ptr<ThunkSpec> make_projections(int n, bool group_adjoints);

@@ -139,6 +139,32 @@ def test_norm_gradients_summed_together(oracle, L, thunks):
     m.close(); ctx.close()
 
 
+@pytest.mark.parametrize("S,V", [(64, 8192), (37, 4104)])
+def test_products_in_parts_of_k(oracle, S, V):
+    """The head's input gradient and the FFN's last product as sums of parts (one to two tiles of 64 x 64, K of 640 to 8192, a k tile
+    that ends inside K): every gradient no further from the oracle than its own other summation orders are, the same bits from
+    every staging of the products and in a pool that spills (the two V x 64 weights, their gradients and nothing else fit)."""
+    from tests.envelope import order_envelope
+    cfg, flat, tok, lm_tok, scale = make_inputs(dict(S=S, D=64, H=2, Dh=32, F=648, V=V, L=1, eps=1e-6), seed=S, norm_mean=1.0,
+                                                grad_scale=64.0)
+    ref = oracle.llama_step(cfg, flat, tok, lm_tok, scale)
+    _, env = order_envelope(oracle, cfg, flat, tok, lm_tok, scale)
+    want, first = oracle.split_params(cfg, ref["grad"]), None
+    for groups, pool in ((2, 1 << 30), (1, 1 << 30), (0, 1 << 30), (2, 512 * V)):
+        ctx, m = _model(cfg, pool_bytes=pool)
+        m.set_product_groups(groups)
+        m.put_params_flat(flat)
+        assert_parity(m.step(tok, lm_tok, scale), ref["loss"], "loss", l2=1e-4, mx=1e-3)
+        got = m.grads()
+        if pool < 1 << 30:
+            assert ctx.stats()["n_evict"] > 0
+        m.close(); ctx.close()
+        first = first or got
+        for name, g in got.items():
+            assert rel_l2(g, want[name]) <= env[name][0], name
+            assert np.array_equal(g.view(np.uint16), first[name].view(np.uint16)), (groups, pool, name)
+
+
 def test_tiny_llama_literal_config(oracle):
     """The reference's small training configuration as written: every weight ~N(0, 0.02), loss scale 1/(S-1).
     The q/k/gate/up/down gradients (1e-8 .. 1e-11) underflow f16 in the reference's own
