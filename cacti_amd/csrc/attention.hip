@@ -7,16 +7,15 @@
 // (pop_adj :4882-4912, InnerSoftmaxPostAdj :3386-3457) without the sequence x sequence tensors
 // ever reaching memory.  Every rounding point of the chain is kept, in registers: scores and
 // probabilities are rounded to f16 before they are used, each product accumulates in fp32 and is
-// rounded once.  (attn_fwd_kernel rounds the probabilities before the division by the row's sum, see below.)
+// rounded once.
 //
 // Layout: q, k, v, o and their adjoints are [S, H, Dh] (row stride ld), 8-byte aligned.
 //
-// Forward (a workgroup = 128 or 64 query rows of one head, 32 rows to a wave; keys in tiles of 64): in the exact
-// arithmetic, and on tensors whose tiles come through registers, the scores are computed twice.  Pass 1 keeps a running row maximum m and sum l of exp(S16 - m);
-// pass 2 recomputes S16 (same instructions, same bits), forms P16 = f16(exp(S16 - m) / l) and accumulates
-// O += P16 V.  Else once (attn_fwd_kernel), O += f16(exp(S16 - r)) V with a reference r per row and one division
-// at the end: the same number of roundings, closer to 64 bits, and for whole steps of long sequences as close to
-// the reference's chain as its own runs in other orders of summation.  Only (m, l) per row are kept for the adjoint.
+// Forward (a workgroup = 128 or 64 query rows of one head, 32 rows to a wave; keys in tiles of 64):
+// the scores are computed twice.  Pass 1 keeps a running row maximum m and sum l of exp(S16 - m);
+// pass 2 recomputes S16 (same instructions, same bits), forms P16 = f16(exp(S16 - m) / l) -- the
+// reference's probabilities, not an unnormalised stand-in -- and accumulates O += P16 V.  Only
+// (m, l) per row are kept for the adjoint.
 //
 // Adjoint: two kernels, each deterministic (no atomics).  The dQ kernel has the forward's shape
 // (queries fixed, loop over keys); the dK/dV kernel fixes 128 or 64 keys and loops over the queries at
@@ -107,11 +106,10 @@ __device__ __forceinline__ void merge_partials(float16_t (&acc)[DT], unsigned ch
 }
 
 // ---------------------------------------------------------------------------------------------
-// Forward with the scores twice (see the top): the exact arithmetic, and the default one on tensors whose tiles come through
-// registers.  Workgroups take the tiles in descending order of their key count; a CU holds one workgroup at a
+// Workgroups take the tiles in descending order of their key count; a CU holds one workgroup at a
 // time (LDS), so the dispatcher hands the next tile to whichever CU is done first.
 template <int KS, int DT, bool FAST, bool DMA, int QR>
-__global__ void __launch_bounds__(kNT2, 2) attn_fwd_twice_kernel(AttnArgs p)
+__global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
 {
     // the whole argument block in scalar registers at once (read field by field where the control flow first
     // wants it, it costs several dependent round trips to memory before the first tile is requested)
@@ -338,7 +336,56 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_twice_kernel(AttnArgs p)
             tv.store(tm, Vs);
         }
         tile_sync<DMA>();
-        for (int it = 0; it < niter; it++) {
+        int it2 = 0;
+        if constexpr (FAST && DMA && KP == 1) {
+            // The key tiles wholly below the diagonal for every wave, as in pass 1, with the vector arithmetic of a
+            // block between the MFMAs of its neighbours: per tile, the scores of its second block are formed while
+            // the probabilities of the first are, the first block's P V products run while the second's
+            // probabilities are formed, then the second's P V; the first scores of the next tile follow the barrier
+            // that publishes it (the P V products read the V tile, which the next iteration's loads overwrite, so
+            // they cannot move behind the barrier).  The same operations on the same values in the same order as the
+            // general loop below.
+            const int nfull = min(qt, niter);
+            if (nfull > 0) {
+                half2v_t sp[8];
+                float pe[16];
+                half8_t pk[2][2];                               // packed probabilities of the tile's two blocks
+                auto prob_piece = [&](const float16_t &acc, half8_t (&out)[2], auto i_c) __attribute__((always_inline)) {
+                    constexpr int i = decltype(i_c)::value;
+                    if constexpr (i == 0) {
+#pragma unroll
+                        for (int e = 0; e < 8; e++)
+                            sp[e] = __builtin_convertvector(float2v_t{scaled(p.alpha, acc[2 * e]), scaled(p.alpha, acc[2 * e + 1])}, half2v_t);
+                    } else if constexpr (i < 5) {
+#pragma unroll
+                        for (int e = 4 * (i - 1); e < 4 * i; e++) pe[e] = exp2_mix(sp[e >> 1][e & 1], cs);
+                    } else {
+                        out[0] = pack8(pe);
+                        out[1] = pack8(pe + 8);
+                    }
+                };
+                float16_t accp = prod_direct<KS>(Ks, 0, qf, l32, lh);
+                for (int it = 0; it < nfull; it++) {
+                    const int jt = 2 * it + g, cur = it & 1;
+                    const bool nxt = jt + 2 < njt;
+                    if (nxt) {
+                        tk.load(tm, K + (int64_t)(jt + 2) * kTileRows * ld, S - (jt + 2) * kTileRows, Ks + (cur ^ 1) * kTileB);
+                        tv.load(tm, V + (int64_t)(jt + 2) * kTileRows * ld, S - (jt + 2) * kTileRows, Vs + (cur ^ 1) * kTileB);
+                    }
+                    const float16_t acc2 = prod_direct_with<KS, 6>(Ks + cur * kTileB, 32, qf, l32, lh,
+                                                                   [&](auto i_c) { prob_piece(accp, pk[0], i_c); });
+                    asm volatile("" : "+v"(pk[0][0]), "+v"(pk[0][1]));
+                    prod_tr_with<DT, 6>(oacc, Vs + cur * kTileB, 0, pk[0][0], pk[0][1], lane,
+                                        [&](auto i_c) { prob_piece(acc2, pk[1], i_c); });
+                    asm volatile("" : "+v"(pk[1][0]), "+v"(pk[1][1]));
+                    prod_tr<DT>(oacc, Vs + cur * kTileB, 32, pk[1][0], pk[1][1], lane);
+                    tile_sync<DMA>();
+                    if (it + 1 < nfull) accp = prod_direct<KS>(Ks + (cur ^ 1) * kTileB, 0, qf, l32, lh);
+                }
+                it2 = nfull;
+            }
+        }
+        for (int it = it2; it < niter; it++) {
             const int jt = 2 * it + g, cur = it & 1;
             const bool nxt = jt + 2 < njt;
             if (nxt) {
@@ -403,235 +450,6 @@ __global__ void __launch_bounds__(kNT2, 2) attn_fwd_twice_kernel(AttnArgs p)
                 }
         }
     }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Forward, default arithmetic, tiles straight into LDS: the scores once.  A row's probabilities are exp(S16 - r), rounded to f16, with a reference r that
-// is the row's maximum up to kRaise (so that they stay below e^8) and the same for the row's keys so far: where a block of keys has
-// more, r moves there and the sums so far shrink accordingly.  O is divided by the row's sum at the end, in f32.  Against the
-// probabilities exp(S16 - m) / l the f16 rounding is the same share of each of them, and fewer fall below what f16 holds: O of
-// 2048 positions, 32 heads of 100, N(0, 1), 4.41e-4 off 64 bits (twice: 4.57e-4), of 1531, 16 of 128 4.32e-4 (4.50e-4).
-// Twice the scores were 66 exponentials and 44 products per wave and tile, now 33 and 30: the vector units bound the kernel
-// with some 1150 cycles a tile where the matrix units need 960.  In us: 2048 positions, 32 heads of 100 81 -> 59, of 64 61 -> 40.5; 1531,
-// 16 of 128 37 -> 27; 1200, 24 of 100 35.7 -> 26.8; 1000, 26 of 64 27.6 -> 19.0.
-constexpr float kRaise = 8.f;
-
-// As above: longest rows first, one workgroup per CU.
-template <int KS, int DT, int QR>
-__global__ void __launch_bounds__(kNT2, 2) attn_fwd_kernel(AttnArgs p)
-{
-    // the whole argument block in scalar registers at once (read field by field where the control flow first
-    // wants it, it costs several dependent round trips to memory before the first tile is requested)
-    asm volatile("" ::"s"(p.S), "s"(p.H), "s"(p.Dh), "s"(p.ld), "s"(p.alpha), "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.dO),
-                 "s"(p.o), "s"(p.out), "s"(p.dq), "s"(p.dk), "s"(p.dv), "s"(p.m), "s"(p.l), "s"(p.y), "s"(p.sig),
-                 "s"(p.acc_dq), "s"(p.acc_dk), "s"(p.acc_dv));
-    typedef AttnMath<true> M;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    // wave-uniform values kept in scalar registers, so that the branches on them are scalar branches
-    const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), tig = threadIdx.x & (kNT - 1);
-    unsigned char *Ks = smem + g * kGroupLds, *Vs = Ks + 2 * kTileB;
-    float *xs = reinterpret_cast<float *>(smem + kXsOff);
-    const int lane = tig & 63, wid = __builtin_amdgcn_readfirstlane(tig >> 6), l32 = lane & 31, lh = lane >> 5;
-    const int S = p.S, Dh = p.Dh;
-    const int64_t ld = p.ld;
-    const int nqt = (S + QR - 1) / QR;
-    const WaveShare<QR> ws(wid, g);
-    constexpr int KP = WaveShare<QR>::KP, NP = 2 * KP;
-    constexpr bool PIPE = KP == 1;
-    const int h = blockIdx.x % p.H, qt = nqt - 1 - blockIdx.x / p.H;
-    const int shift = (int)(((int64_t)h * Dh) & 7);                    // the head's first column in its window
-    const int64_t hoff = (int64_t)h * Dh - shift;
-    gptr_t Q = gp(p.q) + hoff, K = gp(p.k) + hoff, V = gp(p.v) + hoff;
-    const int i0 = qt * QR, qrow = ws.qb * 32 + l32, r0 = i0 + ws.qb * 32, myrow = r0 + l32;
-    const int kend = min(i0 + QR, S);                     // keys [0, kend) are visible to the tile
-    const int njt = (kend + kTileRows - 1) / kTileRows, niter = (njt + 1) / 2;
-    // the iterations whose key tiles lie wholly below the diagonal for every wave, as a pipeline
-    const int nfull = PIPE ? min(qt, niter) : 0;
-
-    const DmaTileMap tm(ld, Dh, shift);
-    DmaTileLoader tk;
-    auto load = [&](gptr_t x, int jt, unsigned char *dst) __attribute__((always_inline)) {
-        tk.load(tm, x + (int64_t)jt * kTileRows * ld, S - jt * kTileRows, dst);
-    };
-    if (g < njt) {
-        load(K, g, Ks);
-        load(V, g, Vs);
-    }
-    // rows 64 g .. 64 g + 63 of the workgroup's queries into this group's second V buffer (a load in which every lane
-    // addresses its own row is served at one lane per clock); every wave then takes its fragments from the tile that
-    // holds its rows
-    if (QR > 64 || g == 0) tk.load(tm, Q + (int64_t)(i0 + g * kTileRows) * ld, S - (i0 + g * kTileRows), Vs + kTileB);
-    if (nfull > 0 && g + 2 < njt) load(K, g + 2, Ks + kTileB);
-    zero_pads(smem, 2 * kGroupLds / kRowB, (Dh + shift + 7) >> 3);
-    tile_sync<true>();
-    half8_t qf[KS];
-    frags_from_tile<KS>(qf, smem + (ws.qb >> 1) * kGroupLds + 3 * kTileB, (ws.qb & 1) * 32 + l32, Dh, lh, shift);
-
-    float16_t oacc[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) oacc[dt][r] = 0.f;
-    // the row's maximum and reference so far (the same in both lanes of the row), the reference as an exponent, and the
-    // lane's sum
-    float m_run = -INFINITY, ref = -INFINITY, cref = 0.f, l_run = 0.f;
-    // bm: the row's maximum over the keys that follow
-    auto raise = [&](float bm) __attribute__((always_inline)) {
-        m_run = fmaxf(m_run, bm);
-        const bool up = bm > ref + kRaise;
-        if (__any(up)) {
-            const float to = up ? bm : ref;
-            const float f = ref == -INFINITY ? 0.f : M::ex(ref, to);
-            ref = to;
-            cref = ref == -INFINITY ? 0.f : ref * kLog2e;
-            l_run *= f;
-#pragma unroll
-            for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) oacc[dt][r] *= f;
-        }
-    };
-    int it0 = 0;
-    if constexpr (PIPE) {
-        // Per tile: its exponentials between the score products of the next tile, the rounding and the maximum of the next
-        // tile's scores between its own products with V.  K tiles are an iteration ahead of V tiles.
-        if (nfull > 0) {
-            half2v_t sp[2][8], mx[2];
-            float pe[16];
-            half8_t pk[2][2];
-            auto round_piece = [&](const float16_t (&s)[2], auto i_c) __attribute__((always_inline)) {      // 8 pieces
-                constexpr int b = decltype(i_c)::value / 4, e0 = 2 * (decltype(i_c)::value % 4);
-#pragma unroll
-                for (int e = e0; e < e0 + 2; e++)
-                    sp[b][e] = __builtin_convertvector(float2v_t{scaled(p.alpha, s[b][2 * e]), scaled(p.alpha, s[b][2 * e + 1])}, half2v_t);
-            };
-            float bm;
-            auto max_piece = [&](auto i_c) __attribute__((always_inline)) {                                 // 3 pieces
-                constexpr int b = decltype(i_c)::value;
-                if constexpr (b < 2) {
-                    mx[b] = sp[b][0];
-#pragma unroll
-                    for (int e = 1; e < 8; e++) mx[b] = __builtin_elementwise_max(mx[b], sp[b][e]);
-                } else {
-                    const half2v_t t = __builtin_elementwise_max(mx[0], mx[1]);
-                    bm = with32((float)__builtin_fmaxf16(t[0], t[1]), OpMax());
-                }
-            };
-            auto exp_piece = [&](auto b_c, auto i_c) __attribute__((always_inline)) {                       // 9 pieces
-                constexpr int b = decltype(b_c)::value, i = decltype(i_c)::value;
-                if constexpr (i < 8) {
-                    pe[2 * i] = exp2_mix(sp[b][i][0], cref);
-                    pe[2 * i + 1] = exp2_mix(sp[b][i][1], cref);
-                    l_run += pe[2 * i];
-                    l_run += pe[2 * i + 1];
-                } else {
-                    pk[b][0] = pack8(pe);
-                    pk[b][1] = pack8(pe + 8);
-                }
-            };
-            const std::integral_constant<int, 0> b0;
-            const std::integral_constant<int, 1> b1;
-            float16_t s[2];
-            s[0] = prod_direct<KS>(Ks, 0, qf, l32, lh);
-            s[1] = prod_direct<KS>(Ks, 32, qf, l32, lh);
-            static_for<0, 8>([&](auto i_c) __attribute__((always_inline)) { round_piece(s, i_c); });
-            static_for<0, 3>(max_piece);
-            raise(bm);
-            __syncthreads();                              // every wave holds its queries: their buffers are free
-            for (int it = 0; it + 1 < nfull; it++) {
-                const int jt = 2 * it + g, cur = it & 1;
-                const unsigned char *Kn = Ks + (cur ^ 1) * kTileB, *Vc = Vs + cur * kTileB;
-                if (jt + 4 < njt) load(K, jt + 4, Ks + cur * kTileB);
-                load(V, jt + 2, Vs + (cur ^ 1) * kTileB);
-                s[0] = prod_direct_with<KS, 9>(Kn, 0, qf, l32, lh, [&](auto i_c) { exp_piece(b0, i_c); });
-                s[1] = prod_direct_with<KS, 9>(Kn, 32, qf, l32, lh, [&](auto i_c) { exp_piece(b1, i_c); });
-                asm volatile("" : "+v"(pk[0][0]), "+v"(pk[0][1]), "+v"(pk[1][0]), "+v"(pk[1][1]));
-                prod_tr_with<DT, 8>(oacc, Vc, 0, pk[0][0], pk[0][1], lane, [&](auto i_c) { round_piece(s, i_c); });
-                prod_tr_with<DT, 3>(oacc, Vc, 32, pk[1][0], pk[1][1], lane, max_piece);
-                raise(bm);
-                tile_sync<true>();
-            }
-            const int jt = 2 * (nfull - 1) + g, cur = (nfull - 1) & 1;
-            if (jt + 2 < njt) load(V, jt + 2, Vs + (cur ^ 1) * kTileB);
-            static_for<0, 9>([&](auto i_c) __attribute__((always_inline)) { exp_piece(b0, i_c); });
-            static_for<0, 9>([&](auto i_c) __attribute__((always_inline)) { exp_piece(b1, i_c); });
-            prod_tr<DT>(oacc, Vs + cur * kTileB, 0, pk[0][0], pk[0][1], lane);
-            prod_tr<DT>(oacc, Vs + cur * kTileB, 32, pk[1][0], pk[1][1], lane);
-            tile_sync<true>();
-            it0 = nfull;
-        }
-    }
-    if (it0 == 0) __syncthreads();                        // every wave holds its queries: their buffers are free
-    for (int it = it0; it < niter; it++) {
-        const int jt = 2 * it + g, cur = it & 1;
-        const bool nxt = jt + 2 < njt;
-        if (nxt) {
-            load(K, jt + 2, Ks + (cur ^ 1) * kTileB);
-            load(V, jt + 2, Vs + (cur ^ 1) * kTileB);
-        }
-        if (jt < njt) {
-#pragma unroll
-            for (int k2 = 0; k2 < 2 / KP; k2++) {
-                const int kt = KP == 1 ? k2 : ws.kp, kb = jt * kTileRows + 32 * kt;
-                if (kb > r0 + 31) continue;              // every key of the block is beyond every row of the wave
-                const float16_t acc = prod_direct<KS>(Ks + cur * kTileB, 32 * kt, qf, l32, lh);
-                half_t sh[16];
-                float pe[16];
-                if (kb + 31 <= r0) {
-#pragma unroll
-                    for (int e = 0; e < 16; e++) sh[e] = f2h(scaled(p.alpha, acc[e]));
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 16; e++) {
-                        const int key = kb + 8 * (e >> 2) + 4 * lh + (e & 3);
-                        sh[e] = key <= myrow ? f2h(scaled(p.alpha, acc[e])) : (half_t)-INFINITY;
-                    }
-                }
-                raise(with32(max16(sh), OpMax()));
-#pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    pe[e] = exp2_mix(sh[e], cref);
-                    l_run += pe[e];
-                }
-                prod_tr<DT>(oacc, Vs + cur * kTileB, 32 * kt, pack8(pe), pack8(pe + 8), lane);
-            }
-        }
-        tile_sync<true>();
-    }
-
-    // the parts of a row (NP waves): their maxima and sums, in one fixed order by every lane that needs the result
-    const float lw = with32(l_run, OpSum());
-    if (lh == 0) {
-        xs[(ws.part * 2 + 0) * QR + qrow] = m_run;
-        xs[(ws.part * 2 + 1) * QR + qrow] = m_run == -INFINITY ? lw : lw * M::ex(ref, m_run);
-    }
-    __syncthreads();
-    float m = xs[qrow], l = 0.f;
-#pragma unroll
-    for (int n = 1; n < NP; n++) m = fmaxf(m, xs[2 * n * QR + qrow]);
-#pragma unroll
-    for (int n = 0; n < NP; n++) {
-        // (a part without a finite score adds 0, or NaN where one of its scores is)
-        const float mn = xs[2 * n * QR + qrow], ln = xs[(2 * n + 1) * QR + qrow];
-        l += mn == -INFINITY ? ln : ln * M::ex(mn, m);
-    }
-    if (myrow >= S) {
-        m = 0.f;
-        l = 1.f;
-    }
-    if (ws.part == 0 && lh == 0 && myrow < S) {
-        p.m[(int64_t)h * S + myrow] = m;
-        p.l[(int64_t)h * S + myrow] = l;
-    }
-    const float y = recip_refined(l), w = ref == -INFINITY ? 0.f : M::ex(ref, m);
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) oacc[dt][r] *= w;
-    merge_partials<QR, DT>(oacc, smem, ws, tig);
-    if (ws.part == 0) stage_rows<DT>(smem, oacc, qrow, lh, y);
-    __syncthreads();
-    write_rows(smem, p.out + (int64_t)i0 * ld + hoff, ld, min(QR, S - i0), Dh, shift, threadIdx.x, kNT2);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1401,7 +1219,7 @@ int set_smem(K kern, size_t bytes)
 }
 
 // Which arithmetic the kernels are launched with (AttnMath).  Measured at 32 heads x 2048 x 100 on MI355X, in a hot loop:
-// forward 51 us / adjoint 145 us with the fast form, 101 / 251 us with the exact one, which has no in-wave pipelines, no short
+// forward 64 us / adjoint 145 us with the fast form, 101 / 251 us with the exact one, which has no in-wave pipelines, no short
 // form of sigma and no parts; the two differ by 3e-5 .. 4e-5 relative L2 in O, dQ, dK, dV, and O, dQ, dK, dV of the fast form
 // agree with the CPU restatement of the reference to 4.9e-5 .. 7.1e-5.
 std::atomic<int> g_exact{0};             // cacti_hip_attention_set_exact: launch the exactly rounded forms
@@ -1410,15 +1228,15 @@ std::atomic<int> g_exact{0};             // cacti_hip_attention_set_exact: launc
 // workgroup has a CU to itself and walks its keys
 // 128 at a time; with 64 rows two waves share a tile's keys, so a step takes less time (one head of 128: 2.1 us against 2.85
 // forward) and there are twice as many workgroups, each of which reads all keys.  Worth it until they need a third round
-// over the CUs: 128 -> 64 rows, us, forward, 1100 positions, 22 heads of 128 (396 workgroups) 24.7 -> 23.7; 1531, 16 of 128 (384) 30.0 ->
-// 25.1; 2048, 16 of 128 (512) 37.9 -> 35.0, of 64 30.2 -> 29.7; 1531, 21 of 64 (504) 25.4 -> 25.7, of 128 32.1 -> 34.3; 1100, 29 of 64 (522)
-// 21.0 -> 27.3; 1531, 22 of 100 (528) 32.5 -> 38.2; 2048, 24 of 100 (768) 40.6 -> 56.7.  Adjoint (its dQ alone), 1100, 20 of 64 (360) 56 ->
-// 50; 1531, 16 of 128 (384) 93 -> 78; 1984, 16 of 128 (496) 117 -> 107; 4096, 8 of 128 (512) 199 -> 184; 1300, 26 of 64 (546) 64 -> 65; 1422,
-// 24 of 100 (552) 100 -> 95; 2048, 32 of 100 (1024) 156 -> 168.  Exact arithmetic: 1531, 16 of 128 70.0 -> 45.4 and 143 -> 108; 1000, 26 of 64
+// over the CUs: 128 -> 64 rows, us, forward and adjoint (its dQ alone), 1100 positions, 20 heads of 64 (360 workgroups) 30.0 -> 25.6
+// and 56 -> 50; 1531, 16 of 128 (384) 42.9 -> 34.7 and 93 -> 78; 1984, 16 of 128 (496) 54.2 -> 47.8 and 117 -> 107; 4096, 8 of 128
+// (512) 100 -> 84 and 199 -> 184; 1300, 26 of 64 (546) 33.1 -> 41.6 and 64 -> 65; 1422, 24 of 100 (552) 40.8 -> 49.6 and 100 -> 95;
+// 2048, 32 of 100 (1024) 68 -> 95 and 156 -> 168.  Exact arithmetic: 1531, 16 of 128 70.0 -> 45.4 and 143 -> 108; 1000, 26 of 64
 // (416) 45.6 -> 34.1 and 89 -> 70.  Up to 128 positions there is a step or two either way.
-// The forward kernel's second round is short only if there are long sequences in the first: to 1024 positions the default arithmetic
-// is left more than 2 workgroups of 32 rows per CU, and is better with 128 rows (777, 31 of 128 24.4 -> 21.4; 512, 48 of 64 15.7 -> 12.7;
-// 1000, 32 of 100 25.9 -> 24.0).
+// The forward kernel's second round is short only if there are long sequences in the first.  Up to 1024 positions it is left heads
+// to 64 between 3/2 and 2 workgroups per CU, where the default arithmetic is as good either way from 770 positions on (1000, 25 of
+// 64 28.2 -> 27.0; 832, 32 24.6 -> 24.3; 896, 32 25.7 -> 26.0; 1024, 28 27.8 -> 28.4) and better with 128 rows below (768, 36 of 64
+// 23.4 -> 25.1; 640, 40 21.2 -> 22.6; 450, 52 19.1 -> 21.9).
 int query_rows(int64_t S, int64_t H, bool forward, bool fast)
 {
     return S > (forward && fast ? 1024 : 128) && (S + 63) / 64 * H <= 2 * (int64_t)device_cus() ? 64 : 128;
@@ -1435,29 +1253,22 @@ bool few_keys(const AttnArgs &p, bool narrow)
     return p.S > 128 && tiles * p.H <= (narrow ? 4 : 2) * (int64_t)device_cus() && p.split < 2;
 }
 
-template <int KS, int DT, bool FAST, bool DMA, int QR>
-constexpr auto fwd_kernel()
-{
-    if constexpr (FAST && DMA) return attn_fwd_kernel<KS, DT, QR>;
-    else return attn_fwd_twice_kernel<KS, DT, FAST, DMA, QR>;
-}
-
 template <int KS, int DT, bool FAST, bool DMA>
 int launch_fwd(const AttnArgs &p, hipStream_t st)
 {
     static DeviceOnce ready;
     if (!ready.fresh()) {
-        int rc = set_smem(fwd_kernel<KS, DT, FAST, DMA, 128>(), kQmSmem);
+        int rc = set_smem(attn_fwd_kernel<KS, DT, FAST, DMA, 128>, kQmSmem);
         if (rc) return rc;
         if constexpr (DMA)
-            if ((rc = set_smem(fwd_kernel<KS, DT, FAST, DMA, 64>(), kQmSmem))) return rc;
+            if ((rc = set_smem(attn_fwd_kernel<KS, DT, FAST, DMA, 64>, kQmSmem))) return rc;
         ready.mark();
     }
     const int rows = DMA ? query_rows(p.S, p.H, true, FAST) : 128, nqt = (p.S + rows - 1) / rows;
     const dim3 grid((unsigned)(nqt * p.H));
     if constexpr (DMA)
-        if (rows == 64) hipLaunchKernelGGL((fwd_kernel<KS, DT, FAST, DMA, 64>()), grid, dim3(kNT2), kQmSmem, st, p);
-    if (rows == 128) hipLaunchKernelGGL((fwd_kernel<KS, DT, FAST, DMA, 128>()), grid, dim3(kNT2), kQmSmem, st, p);
+        if (rows == 64) hipLaunchKernelGGL((attn_fwd_kernel<KS, DT, FAST, DMA, 64>), grid, dim3(kNT2), kQmSmem, st, p);
+    if (rows == 128) hipLaunchKernelGGL((attn_fwd_kernel<KS, DT, FAST, DMA, 128>), grid, dim3(kNT2), kQmSmem, st, p);
     return launch_status("attention_fwd");
 }
 
@@ -1598,7 +1409,7 @@ static int attention_fwd(int64_t S, int64_t H, int64_t Dh, float alpha, const vo
     p.l = p.m + S * H;
     int64_t span = Dh;
     const bool dma = (windows || Dh % 8 == 0) && direct_tiles(H, Dh, ld, {q, k, v, o}, &span);
-    if (dma && attention_short_fwd_takes(S, H, span, exact)) return attention_short_fwd(p, span, exact, st);
+    if (dma && attention_short_fwd_takes(S, H, span)) return attention_short_fwd(p, span, exact, st);
     return dispatch<Fwd>(span, exact, dma, p, st);
 }
 

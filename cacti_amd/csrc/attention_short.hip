@@ -612,11 +612,10 @@ int dispatch(const AttnArgs &p, int64_t span, bool exact, hipStream_t st)
 // A workgroup of these kernels takes 32 rows, so each reads a head's keys (or queries) for a quarter of the rows that one of
 // attention.hip reads them for: with many workgroups per CU that traffic is what they take, and the larger tiles are better.
 // Where the lines lie, kernel times in us, attention.hip -> here, workgroups of 32 rows in brackets, 256 CUs:
-//   forward, default arithmetic (there its scores once), to 1024 positions: 128 positions of 32 heads of 64 (128) 7.8 -> 6.6; 1000, 8 of
-//   100 (256) 21.4 -> 13.2; 512, 32 of 100 (512) 15.3 -> 12.3; 400, 40 of 100 (520) 13.7 -> 13.6; 512, 48 of 64 (768) 12.7 -> 15.9; 400, 60
-//   of 100 (780) 15.8 -> 17.8; 777, 31 of 128 (775) 21.4 -> 25.2; 1000, 24 of 128 (768) 22.9 -> 22.2; 1024, 32 of 100 (1024) 24.1 -> 27.
-//   To 2048: 1531, 8 of 128 (384) 22.2 -> 17.5; 2048, 8 of 64 (512) 23.3 -> 22.6; 1531, 11 of 64 (528) 19.9 -> 23.4.  Exact, its scores twice
-//   there: 1024, 32 of 128 (1024) and 1000, 24 of 64 (768) are still better here.  Beyond 2048 the
+//   forward, to 1024 positions: 128 positions of 4 heads of 64 (16) 8.9 -> 5.9; 1000, 4 of 100 (128) 23.0 -> 12.0; 512, 16 of
+//   100 (256) 15.8 -> 9.7; 1024, 16 of 128 (512) 25.2 -> 17.5; 1000, 24 of 64 (768) 24.0 -> 20.5; 1024, 32 of 128 (1024) 30.6 ->
+//   25.8; 512, 64 of 64 (1024) 16.7 -> 17.1; 1024, 64 of 64 (2048) 34.9 -> 41.6.  To 2048: 1536, 4 of 128 (192) 30.4 -> 15.3;
+//   2048, 8 of 64 (512) 33.6 -> 23.4; 1531, 16 of 128 (768) 34.6 -> 32.9; 2048, 16 of 64 (1024) 40.7 -> 43.2.  Beyond 2048 the
 //   rounded scores of a wave's blocks have no room in its registers.
 //   The adjoint's workgroups have a CU to themselves, so beyond 256 they come in two rounds, and the second is worth it where the
 //   first one's walks are long (second_round): up to 256 0.54 to 0.90 of the time.
@@ -631,11 +630,10 @@ int dispatch(const AttnArgs &p, int64_t span, bool exact, hipStream_t st)
 //   1.17, 200 to 300 (to 400) 1.01 to 1.05, 300 to 400 (to 350) 0.86, 500 to 600 (to 450) 0.75 to 0.98, from there to 512 1.01; 1000, 24
 //   of 64 (768) 23.5 -> 27.3; 640, 32 of 100 (640) 22.5 -> 30.4.
 //   Exact arithmetic, (512): 512, 32 of 128 18.7 -> 15.0 forward; 2048, 8 of 64 47.0 -> 34.5, adjoint 106.7 -> 74.1.
-bool attention_short_fwd_takes(int64_t S, int64_t H, int64_t span, bool exact)
+bool attention_short_fwd_takes(int64_t S, int64_t H, int64_t span)
 {
     const int64_t wgs = blocks(S) * H, cus = device_cus();
-    if (S > 1024) return S <= 2048 && wgs <= 2 * cus;
-    return exact ? wgs <= (span > 64 ? 4 : 3) * cus : wgs <= (S > 900 ? 3 * cus : cus * 9 / 4);
+    return S <= 1024 ? wgs <= (span > 64 ? 4 : 3) * cus : S <= 2048 && wgs <= 2 * cus;
 }
 // The second round of workgroups: as many as the positions beyond `from` are 1/430 of the CUs'.
 static bool second_round(int64_t S, int64_t H, int64_t from)

@@ -640,7 +640,7 @@ __device__ __forceinline__ void write_rows(const unsigned char *stage, half_t *d
 // attention_short.hip, for tensors whose tiles can be loaded straight into LDS; span: window positions of a head, at most 128.
 // The launches come after the question whether they take it.  dq and dkv together are an adjoint, as is either with
 // attention.hip's other half.
-bool attention_short_fwd_takes(int64_t S, int64_t H, int64_t span, bool exact);
+bool attention_short_fwd_takes(int64_t S, int64_t H, int64_t span);
 bool attention_short_dq_takes(int64_t S, int64_t H, bool exact);
 bool attention_short_dkv_takes(int64_t S, int64_t H, int64_t span, int per);
 int attention_short_fwd(const AttnArgs &p, int64_t span, bool exact, hipStream_t st);
