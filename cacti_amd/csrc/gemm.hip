@@ -427,6 +427,16 @@ CACTI_API int cacti_hip_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, i
     return 0;
 }
 
+CACTI_API int cacti_hip_gemm_plan_ws(int64_t M, int64_t N, int64_t K, int parts, int64_t out[3], double *us)
+{
+    CACTI_REQUIRE(out && us && M > 0 && N > 0 && K > 0 && parts >= 0 && parts <= 8, CACTI_E_INVALID, "gemm_plan_ws: bad argument");
+    const GemmPlan plan = parts > 1 ? gemm_plan_parts(M, N, K, parts) : gemm_plan(M, N, K, 1, parts == 0);
+    out[0] = plan.tile < 0 ? 0 : plan.split;
+    gemm_tile_dims(plan.tile < 0 ? 0 : plan.tile, out + 1, out + 2);
+    *us = plan.us;
+    return 0;
+}
+
 CACTI_API int cacti_hip_gemm_kernel_name(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t nz, char *name, size_t bytes)
 {
     CACTI_REQUIRE(name && M > 0 && N > 0 && K > 0 && nz > 0, CACTI_E_INVALID, "gemm_kernel_name: bad argument");

@@ -880,21 +880,25 @@ constexpr int64_t kSmallOutput = 1 << 18;
 constexpr double kAnyPerTile = 1.45;
 constexpr int kMostParts = 8;
 
-// `best` in up to kMostParts parts of K on tile t, if that costs less; per_tile: factor on the time per k tile.  The parts and their
-// sum cost a launch of 3 to 13 us, 2 us per million fp32 values while they are few and half of that beyond.  A gain of 4 % is asked
-// of tiles above 128 x 128, whose time per k tile with a part of the CUs is the least certain (1719 x 1024 x 8256 39.2 -> 43.4 us
-// without).
-void split_k(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, double per_tile, GemmPlan &best, double &best_cost)
+// What s parts of K on tile t are expected to take (negative: there are no such parts); per_tile: factor on the time per k tile.  The
+// parts and their sum cost a launch of 3 to 13 us, 2 us per million fp32 values while they are few and half of that beyond.
+double part_cost(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, int s, double per_tile)
 {
+    const int64_t per = (kt + s - 1) / s;
+    if (per < 4 || (kt + per - 1) / per != s) return -1.0;                // parts of some length, none empty
+    const double fixed = kShapes[t].fixed, x = (double)(M * N) * s / 1e6;
+    return fixed + per_tile * (tile_cost(cus, t, M, N, s, per) - fixed) + 4.0 + (x < 4.0 ? 2.0 * x : 4.0 + x);
+}
+
+// `best` in up to kMostParts parts of K on tile t, if that costs less, whichever tile it was on.  A gain of 4 % on the whole product
+// (`whole`) is asked of tiles above 128 x 128, whose time per k tile with a part of the CUs is the least certain (1719 x 1024 x 8256
+// 39.2 -> 43.4 us without).
+void split_k(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, double per_tile, double whole, GemmPlan &best)
+{
+    const double margin = kShapes[t].bm * kShapes[t].bn > 128 * 128 ? 1.04 : 1.0;
     for (int s = 2; s <= kMostParts; s++) {
-        const int64_t per = (kt + s - 1) / s;
-        if (per < 4 || (kt + per - 1) / per != s) continue;               // parts of some length, none empty
-        const double fixed = kShapes[t].fixed, x = (double)(M * N) * s / 1e6;
-        const double c = fixed + per_tile * (tile_cost(cus, t, M, N, s, per) - fixed) + 4.0 + (x < 4.0 ? 2.0 * x : 4.0 + x);
-        if (c * (kShapes[t].bm * kShapes[t].bn > 128 * 128 ? 1.04 : 1.0) < best_cost) {
-            best_cost = c;
-            best = {t, T64, 0, s, c};
-        }
+        const double c = part_cost(cus, t, M, N, kt, s, per_tile);
+        if (c >= 0 && c * margin < whole && c < best.us) best = {t, T64, 0, s, c};
     }
 }
 
@@ -940,10 +944,10 @@ GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, boo
             }
         }
     }
+    best.us = best_cost;
     if (may_split && nz == 1)
         for (int t = T64; t < kNumShapes; t++)
-            if (has_parts(t)) split_k(cus, t, M, N, kt, 1.0, best, best_cost);
-    best.us = best_cost;
+            if (has_parts(t)) split_k(cus, t, M, N, kt, 1.0, best_cost, best);
     return best;
 }
 
@@ -1013,6 +1017,16 @@ static GemmPlan kept_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split) { return kept_plan(M, N, K, nz, may_split, 1); }
 GemmPlan gemm_plan_chain(int64_t M, int64_t N, int64_t K, int chain) { return kept_plan(M, N, K, 1, false, chain); }
 
+GemmPlan gemm_plan_parts(int64_t M, int64_t N, int64_t K, int parts)
+{
+    GemmPlan best = {-1, T64, 0, parts, 0};
+    for (int t = T64; t < kNumShapes; t++) {
+        const double c = has_parts(t) ? part_cost(device_cus(), t, M, N, (K + BK - 1) / BK, parts, 1.0) : -1.0;
+        if (c >= 0 && (best.tile < 0 || c < best.us)) best = {t, T64, 0, parts, c};
+    }
+    return best;
+}
+
 // The same for operands that are loaded through registers whatever their alignment: 64 x 64 tiles, whose k tiles take some
 // half longer than the direct ones' (64 x 128 and 128 x 128 took twice and three times as long as that: their loads have
 // no room in the registers to be far enough ahead).
@@ -1022,7 +1036,7 @@ GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K)
     const double fixed = kShapes[T64].fixed;
     GemmPlan best = {T64, T64, 0, 1, 0};
     best.us = fixed + kAnyPerTile * (tile_cost(cus, T64, M, N, 1, kt) - fixed);
-    split_k(cus, T64, M, N, kt, kAnyPerTile, best, best.us);
+    split_k(cus, T64, M, N, kt, kAnyPerTile, best.us, best);
     return best;
 }
 

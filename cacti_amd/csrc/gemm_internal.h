@@ -127,6 +127,7 @@ struct GemmPlan {
 };
 // nz: products of this shape in the launch
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split);
+GemmPlan gemm_plan_parts(int64_t M, int64_t N, int64_t K, int parts);       // in exactly that many parts, 2 .. 8 (tile < 0: K has none)
 GemmPlan gemm_plan_chain(int64_t M, int64_t N, int64_t K, int chain);       // chain <= kMaxPtrBatch products that add up
 // the gradients of n products x W_i^T, x [S,K], W_i [N,K], all in one launch (tile < 0: no better than two, the input gradient of a
 // single product among them with `lent` bytes for parts of K)

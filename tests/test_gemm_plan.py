@@ -1,5 +1,6 @@
 """How products are cut into tiles (cacti_hip_gemm_plan; no GPU: the device is taken to have 256 CUs then)."""
 import ctypes as C
+import random
 
 import pytest
 
@@ -69,3 +70,29 @@ def test_a_kernel_name_needs_its_room():
     n = C.c_int(7)
     assert ffi.lib().cacti_hip_gemm_chain_kernel_name(2, 2048, 3200, 8640, name, 20, C.byref(n)) == -1
     assert ffi.lib().cacti_hip_gemm_chain_kernel_name(2, 2048, 3200, 8640, name, 128, C.byref(n)) == 0 and n.value == 1
+
+
+def parts_plan(M, N, K, parts=0):
+    """((parts of K, rows and columns of the tile), expected us); parts 0: as a product with a workspace is cut, 1: whole."""
+    out, us = (C.c_int64 * 3)(), C.c_double()
+    assert ffi.lib().cacti_hip_gemm_plan_ws(M, N, K, parts, out, C.byref(us)) == 0
+    return tuple(out), us.value
+
+
+def test_parts_of_k_are_the_cheapest_that_gain():
+    """Whatever the order in which tiles and numbers of parts are looked at: none of those that gain the 4 % asked of large tiles on the
+    whole product is expected to take less than the cut that is taken."""
+    r = random.Random(5)
+    drawn = [(round(33 * (2048 / 33) ** r.random()), 8 * round(32 * (400 / 32) ** r.random()), 8 * round(125 * 32 ** r.random())) for _ in range(1500)]
+    split = 0
+    for M, N, K in drawn + [(1378, 768, 19288), (1325, 3200, 24392), (2048, 3200, 32000)]:
+        (parts, _, _), us = parts_plan(M, N, K)
+        _, whole = parts_plan(M, N, K, 1)
+        assert us <= whole, (M, N, K)
+        split += parts > 1
+        for s in range(2, 9):
+            (n, bm, bn), cost = parts_plan(M, N, K, s)
+            assert n in (0, s)
+            if n and cost * 1.04 < whole:
+                assert us <= cost, (M, N, K, parts, us, s, bm, bn, cost)
+    assert split > 300
