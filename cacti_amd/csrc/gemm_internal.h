@@ -174,12 +174,8 @@ struct RowSource {
     int64_t vocab;
     int *status;
 };
-// clear: nclear words, kClearPitch apart, that it sets to 0 for the launch behind it (attn_decode.hip: counters that workgroups add to
-// from all sides, each in a cache line of its own: 16 of them side by side cost 4 us)
-constexpr int kClearPitch = 32;
 int rows_qkv_launch(int64_t M, int64_t H, int64_t Dh, const RowSource &x, void *sum_out, const void *Wq, const void *Wk, const void *Wv,
-                    const void *cos16, const void *sin16, void *q_rot, void *k_cache_rows, void *v_cache_rows, void *clear, int64_t nclear,
-                    hipStream_t st);
+                    const void *cos16, const void *sin16, void *q_rot, void *k_cache_rows, void *v_cache_rows, hipStream_t st);
 int rows_gate_launch(int64_t M, int64_t N, int64_t K, const RowSource &x, void *sum_out, const void *B, const void *B_mul, void *C,
                      hipStream_t st);
 int rows_norm_launch(int64_t M, int64_t N, int64_t K, const RowSource &x, const void *B, void *C, hipStream_t st);

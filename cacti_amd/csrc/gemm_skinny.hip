@@ -53,11 +53,6 @@ struct SkinnyArgs {
     half_t *kc, *vc;
     int H, Dh;
     FastDiv half_head;       // by Dh / 2
-    // QKV: words, kClearPitch apart, that the first workgroup sets to 0, for the launch behind this one.  (Here, among what is
-    // read at once anyway, and set to 0 behind the loads instead of at the end: q, k, v of 256 3.30 -> 3.2 us, 3.13
-    // without any.)
-    int nclear;
-    uint32_t *clear;
     // NORM: with tok, row m of x is row tok[m] of A (the embedding of `vocab` rows); an id out of range raises
     // *status to m + 1 and reads the last row
     const uint16_t *tok;
@@ -103,7 +98,7 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
     if (NORM && EPI != E_PLAIN) asm volatile("" ::"s"(p.B2));
     if (EPI == E_QKV)
         asm volatile("" ::"s"(p.B3), "s"(p.cos16), "s"(p.sin16), "s"(p.kc), "s"(p.vc), "s"(p.H), "s"(p.Dh), "s"(p.half_head.m),
-                     "s"(p.half_head.shift), "s"(p.clear), "s"(p.nclear));
+                     "s"(p.half_head.shift));
     constexpr int kThreads = W * 64;
     constexpr bool GATE = EPI == E_GATE;
     constexpr int NB = GATE ? 2 : 1;
@@ -210,8 +205,6 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
             ecos = p.cos16[em * p.Dh + d];
             esin = p.sin16[em * p.Dh + d];
             ecell = (blockIdx.y == 1 ? p.kc : p.vc)[em * p.ldc + ecol];
-            if (__builtin_expect(p.nclear > 0, 0) && blockIdx.x == 0 && blockIdx.y == 0)
-                for (int i = tid; i < p.nclear; i += kThreads) p.clear[i * kClearPitch] = 0;
         }
         if (NORM) __builtin_amdgcn_sched_barrier(0);
         if (NORM) {
@@ -443,13 +436,10 @@ SkinnyArgs norm_args(const RowSource &x, int64_t N, int64_t K, void *sum_out)
 }  // namespace
 
 int rows_qkv_launch(int64_t M, int64_t H, int64_t Dh, const RowSource &x, void *sum_out, const void *Wq, const void *Wk, const void *Wv,
-                    const void *cos16, const void *sin16, void *q_rot, void *k_cache_rows, void *v_cache_rows, void *clear, int64_t nclear,
-                    hipStream_t st)
+                    const void *cos16, const void *sin16, void *q_rot, void *k_cache_rows, void *v_cache_rows, hipStream_t st)
 {
     const int64_t D = H * Dh;
     SkinnyArgs p = norm_args(x, D, D, sum_out);
-    p.clear = static_cast<uint32_t *>(clear);
-    p.nclear = (int)nclear;
     p.B = (const half_t *)Wq; p.B2 = (const half_t *)Wk; p.B3 = (const half_t *)Wv;
     p.C = (half_t *)q_rot;
     p.cos16 = (const half_t *)cos16; p.sin16 = (const half_t *)sin16;
@@ -532,5 +522,5 @@ CACTI_API int cacti_hip_rows_qkv_rope_cache_f16(int64_t M, int64_t H, int64_t Dh
                       aligned(k_cache_rows, 2) && aligned(v_cache_rows, 2),
                   CACTI_E_INVALID, "rows_qkv: rows and weights must be 16-byte aligned");
     return rows_qkv_launch(M, H, Dh, RowSource{x, x2, w_norm, eps, nullptr, 0, nullptr}, sum_out, Wq, Wk, Wv, cos16, sin16, q_rot,
-                           k_cache_rows, v_cache_rows, nullptr, 0, (hipStream_t)stream);
+                           k_cache_rows, v_cache_rows, (hipStream_t)stream);
 }

@@ -611,11 +611,6 @@ int rope_cache_launch(int64_t S, int64_t H, int64_t Dh, const void *q, const voi
 // csrc/attention.hip
 int attention_fwd_exact(int64_t S, int64_t H, int64_t Dh, float alpha, const void *q, const void *k, const void *v, int64_t ld, void *o,
                         void *stats, hipStream_t st);
-// csrc/attn_decode.hip
-int64_t attn_decode_words(int64_t T, int64_t H, int64_t Dh, int64_t C);
-int attn_decode(int64_t T, int64_t H, int64_t Dh, int64_t C, int64_t initial_row, float alpha, const void *q, int64_t ldq, const void *k_cache,
-                const void *v_cache, int64_t ldkv, int64_t head_stride, void *out, int64_t ldo, void *workspace, size_t workspace_bytes, bool cleared,
-                hipStream_t st);
 }  // namespace cacti
 
 namespace {
@@ -749,7 +744,7 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
     char *x = tmp(T * D, 2), *pre = tmp(T * D, 2), *q = tmp(T * D, 2), *qr = tmp(T * D, 2), *kk = tmp(T * D, 2),
          *kr = tmp(T * D, 2), *v = tmp(T * D, 2), *attn = tmp(T * D, 2), *o = tmp(T * D, 2), *x1 = tmp(T * D, 2),
          *post = tmp(T * D, 2), *up = tmp(T * F, 2), *gate = tmp(T * F, 2), *h = tmp(T * F, 2), *down = tmp(T * D, 2);
-    // one to four rows: the decoding kernels, one launch per weight matrix (or pair, or triple) and one for
+    // one to four rows: the decoding kernels, one launch per weight matrix (or pair, or triple) and one or two for
     // attention.  More rows: the training kernels; a long prompt from position 0 is causal attention over its own rows of
     // the cache in one kernel (1531 rows, 16 heads of 128: 93 -> 40 us per layer), other rows take scores, softmax and P V
     // as three (up to 128 rows they are one tile of scores per head, 17 against 11 us, and the numbers of the training
@@ -820,9 +815,9 @@ CACTI_API int cacti_llama_cached_apply(cacti_llama_cached *k, int64_t prev, int6
                 char *kc = static_cast<char *>(P(k->k_cache[l])), *vc = static_cast<char *>(P(k->v_cache[l]));
                 // q, k, v projections of the normed stream, rotation, k_cache[prev ..] += k, v_cache[prev ..] += v
                 STEP(rows_qkv_launch(T, H, Dh, normed(xb, w.pre_norm), xb ? x : nullptr, P(w.q), P(w.k), P(w.v), cosr, sinr, qr,
-                                     kc + prev * D * 2, vc + prev * D * 2, aws, attn_decode_words(T, H, Dh, next), st));
+                                     kc + prev * D * 2, vc + prev * D * 2, st));
                 if (xb) xs = RowSource{x, nullptr, nullptr, g.eps, nullptr, 0, nullptr};
-                STEP(attn_decode(T, H, Dh, next, prev, alpha, qr, D, kc, vc, D, Dh, attn, D, aws, aws_bytes, true, st));
+                STEP(cacti_hip_attn_decode_f16(T, H, Dh, next, prev, alpha, qr, D, kc, vc, D, Dh, attn, D, aws, aws_bytes, st));
                 STEP(product(D, D, attn, P(w.o), o));
                 // x1 = stream + o; post = rms_norm(x1); h = silu(post gate^T) * (post up^T)
                 STEP(rows_gate_launch(T, F, D, normed(o, w.post_norm), x1, P(w.gate), P(w.up), h, st));

@@ -384,8 +384,7 @@ int cacti_hip_rows_qkv_rope_cache_f16(int64_t M, int64_t H, int64_t Dh, const vo
 /* Attention of T = 1..4 new positions over the key / value cache in one or two small launches: the chain
  * block_matmul_scale(q, k_cache^T, alpha) -> f32 -> row-causal mask -> softmax -> f16 ->
  * block_matmul(., v_cache) of src/librarium/llama.rs:895-915 with its rounding points (f16 scores
- * and, up to 480 positions or 960 of heads to 64, probabilities -- beyond, these stay f32 --, fp32 accumulation, one
- * rounding of the output).  q: [T, ldq] f16 with head h
+ * and probabilities, fp32 accumulation, one rounding of the output).  q: [T, ldq] f16 with head h
  * at columns h*Dh..; k_cache, v_cache: element (position j, head h, d) at j*ldkv + h*head_stride + d
  * (the reference's [C, H, Dh] layout is ldkv = H*Dh, head_stride = Dh; positions beyond
  * T + initial_row - 1 are not read); out: [T, ldo] f16.  Dh % 4 == 0, Dh <= 128; pointers 8-byte
