@@ -262,11 +262,11 @@ constexpr int64_t kMaxPitch = (int64_t)1 << 23;
 
 namespace {
 
-// ws_need null: the caller has no workspace.  Otherwise *ws_need is set to the bytes the chosen way needs, and if that is
-// more than ws_bytes nothing is launched.
+// ws_need null: the caller has no workspace.  Otherwise *ws_need is set to the bytes the chosen way needs (of those that need no
+// more than `most`), and if that is more than ws_bytes nothing is launched.
 int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, float alpha, const void *A, int64_t lda,
              int64_t stride_a, const void *B, int64_t ldb, int64_t stride_b, float beta, void *C, int64_t ldc,
-             int64_t stride_c, int tri, void *ws, size_t ws_bytes, size_t *ws_need, void *stream)
+             int64_t stride_c, int tri, size_t most, void *ws, size_t ws_bytes, size_t *ws_need, void *stream)
 {
     CACTI_REQUIRE(tri >= 0 && tri <= 3, CACTI_E_INVALID, "gemm: tri must be 0..3");
     CACTI_REQUIRE(tri == 0 || (tri == 1 && M == N) || (tri == 2 && !ta && M == K) ||
@@ -336,11 +336,11 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
         }
     }
     if (near && tri == 0 && vec == 8) {
-        const GemmPlan plan = gemm_plan(M, N, K, nblk, ws_need != nullptr);
+        const GemmPlan plan = gemm_plan(M, N, K, nblk, ws_need ? most : 0);
         if (plan.split > 1) {
-            p.ldp = (N + 3) / 4 * 4;
+            p.ldp = gemm_part_pitch(N);
             p.part = (float *)ws;
-            *ws_need = (size_t)plan.split * (size_t)M * (size_t)p.ldp * sizeof(float);
+            *ws_need = gemm_parts_bytes(M, N, plan.split);
             if (*ws_need > ws_bytes) return 0;
         }
         return gemm_direct_launch(ta, tb, p, nblk, plan, st);
@@ -351,21 +351,22 @@ int gemm_run(int ta, int tb, int64_t nblk, int64_t M, int64_t N, int64_t K, floa
     // mean than the better of the two, registers 3 %, this rule 0.2 % (19 % at worst: 687 x 3731 x 410).  Element-wise loads
     // in the kernel cost 1.6 us (both operands contiguous in K) to 3.4 us (both strided) per 32 values of K instead.
     const int64_t ra = ta ? K : M, rb = tb ? N : K, pa = (ca + 7) / 8 * 8, pb = (cb + 7) / 8 * 8;
-    if (ws_need && tri == 0 && nblk == 1 && K >= 8 && pa < kMaxPitch && pb < kMaxPitch) {
-        const bool ok_a = fits_a(8) && lda < kMaxPitch, ok_b = fits_b(8) && ldb < kMaxPitch;
-        size_t bytes_a = ok_a ? 0 : (size_t)ra * (size_t)pa * 2, bytes_b = ok_b ? 0 : (size_t)rb * (size_t)pb * 2;
-        GemmPlan plan = gemm_plan(M, N, K, 1, true);
-        if (near && ca >= 8 && cb >= 8) {
-            const GemmPlan as_is = gemm_plan_any(M, N, K);
+    const bool ok_a = fits_a(8) && lda < kMaxPitch, ok_b = fits_b(8) && ldb < kMaxPitch, as_it_is = near && ca >= 8 && cb >= 8;
+    size_t bytes_a = ok_a ? 0 : (size_t)ra * (size_t)pa * 2, bytes_b = ok_b ? 0 : (size_t)rb * (size_t)pb * 2;
+    const bool copied = bytes_a + bytes_b <= most;
+    if (ws_need && tri == 0 && nblk == 1 && K >= 8 && pa < kMaxPitch && pb < kMaxPitch && (copied || as_it_is)) {
+        GemmPlan plan = gemm_plan(M, N, K, 1, copied ? most - (bytes_a + bytes_b) : 0);
+        if (as_it_is) {
+            const GemmPlan as_is = gemm_plan_any(M, N, K, most);
             const double copy = bytes_a + bytes_b > 0 ? 3.5 + (double)(bytes_a + bytes_b) / 2.5e6 : 0;
-            if (as_is.us < plan.us + copy) {
+            if (!copied || as_is.us < plan.us + copy) {
                 plan = as_is;
                 p.any = 1;
                 bytes_a = bytes_b = 0;
             }
         }
-        p.ldp = (N + 3) / 4 * 4;
-        const size_t bytes_part = plan.split > 1 ? (size_t)plan.split * (size_t)M * (size_t)p.ldp * sizeof(float) : 0;
+        p.ldp = gemm_part_pitch(N);
+        const size_t bytes_part = plan.split > 1 ? gemm_parts_bytes(M, N, plan.split) : 0;
         *ws_need = bytes_a + bytes_b + bytes_part;                // each a multiple of 16
         if (*ws_need > ws_bytes) return 0;
         char *w = static_cast<char *>(ws);
@@ -404,22 +405,30 @@ CACTI_API int cacti_hip_gemm_f16_strided_batched_tri(int ta, int tb, int64_t nbl
                                                      void *C, int64_t ldc, int64_t stride_c, int tri,
                                                      void *stream)
 {
-    return gemm_run(ta, tb, nblk, M, N, K, alpha, A, lda, stride_a, B, ldb, stride_b, beta, C, ldc, stride_c, tri, nullptr, 0,
+    return gemm_run(ta, tb, nblk, M, N, K, alpha, A, lda, stride_a, B, ldb, stride_b, beta, C, ldc, stride_c, tri, 0, nullptr, 0,
                     nullptr, stream);
 }
+
+namespace cacti {
+int gemm_f16_within(size_t most, int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const void *A, int64_t lda, const void *B, int64_t ldb,
+                    float beta, void *C, int64_t ldc, void *ws, size_t ws_bytes, size_t *ws_need, hipStream_t st)
+{
+    return gemm_run(ta, tb, 1, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, 0, most, ws, ws_bytes, ws_need, st);
+}
+}  // namespace cacti
 
 CACTI_API int cacti_hip_gemm_f16_ws(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const void *A, int64_t lda,
                                     const void *B, int64_t ldb, float beta, void *C, int64_t ldc, void *ws, size_t ws_bytes,
                                     size_t *ws_need, void *stream)
 {
     CACTI_REQUIRE(ws_need, CACTI_E_INVALID, "gemm_ws: null ws_need");
-    return gemm_run(ta, tb, 1, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, 0, ws, ws_bytes, ws_need, stream);
+    return gemm_f16_within(SIZE_MAX, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, ws, ws_bytes, ws_need, (hipStream_t)stream);
 }
 
 CACTI_API int cacti_hip_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, int64_t out[6])
 {
     CACTI_REQUIRE(out && M > 0 && N > 0 && K > 0 && nz > 0, CACTI_E_INVALID, "gemm_plan: bad argument");
-    const GemmPlan plan = gemm_plan(M, N, K, nz, false);
+    const GemmPlan plan = gemm_plan(M, N, K, nz, 0);
     gemm_tile_dims(plan.tile, out, out + 1);
     out[2] = plan.cols > 0 ? plan.cols : N;
     gemm_tile_dims(plan.rest, out + 3, out + 4);
@@ -427,10 +436,10 @@ CACTI_API int cacti_hip_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, i
     return 0;
 }
 
-CACTI_API int cacti_hip_gemm_plan_ws(int64_t M, int64_t N, int64_t K, int parts, int64_t out[3], double *us)
+CACTI_API int cacti_hip_gemm_plan_ws(int64_t M, int64_t N, int64_t K, size_t lent, int parts, int64_t out[3], double *us)
 {
     CACTI_REQUIRE(out && us && M > 0 && N > 0 && K > 0 && parts >= 0 && parts <= 8, CACTI_E_INVALID, "gemm_plan_ws: bad argument");
-    const GemmPlan plan = parts > 1 ? gemm_plan_parts(M, N, K, parts) : gemm_plan(M, N, K, 1, parts == 0);
+    const GemmPlan plan = parts > 1 ? gemm_plan_parts(M, N, K, parts) : gemm_plan(M, N, K, 1, parts == 0 ? lent : 0);
     out[0] = plan.tile < 0 ? 0 : plan.split;
     gemm_tile_dims(plan.tile < 0 ? 0 : plan.tile, out + 1, out + 2);
     *us = plan.us;
@@ -440,7 +449,7 @@ CACTI_API int cacti_hip_gemm_plan_ws(int64_t M, int64_t N, int64_t K, int parts,
 CACTI_API int cacti_hip_gemm_kernel_name(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t nz, char *name, size_t bytes)
 {
     CACTI_REQUIRE(name && M > 0 && N > 0 && K > 0 && nz > 0, CACTI_E_INVALID, "gemm_kernel_name: bad argument");
-    const int n = gemm_kernel_name(ta, tb, gemm_plan(M, N, K, nz, false), name, bytes);
+    const int n = gemm_kernel_name(ta, tb, gemm_plan(M, N, K, nz, 0), name, bytes);
     CACTI_REQUIRE(n >= 0 && (size_t)n < bytes, CACTI_E_INVALID, "gemm_kernel_name: %zu bytes are too few for the name", bytes);
     return 0;
 }
@@ -482,7 +491,7 @@ CACTI_API int cacti_hip_gemm_f16_batched(int ta, int tb, int64_t nblk, int64_t M
             p.zb[z] = (const half_t *)B[zz] - p.B;
             p.zc[z] = (half_t *)C[zz] - p.C;
         }
-        const GemmPlan plan = gemm_plan(M, N, K, cnt, false);
+        const GemmPlan plan = gemm_plan(M, N, K, cnt, 0);
         const int rc = gemm_direct_launch(ta, tb, p, cnt, plan, (hipStream_t)stream);
         if (rc) return rc;
     }
@@ -495,7 +504,7 @@ static bool chain_pays(int64_t n, int64_t M, int64_t N, int64_t K, GemmPlan *pla
 {
     if (!(n > 1 && n <= kMaxPtrBatch && M > 0 && N > 0 && K >= 4 * 64 && mult(K, 64) && mult(N, 8))) return false;
     *plan = gemm_plan_chain(M, N, K, (int)n);
-    return plan->us < (double)n * gemm_plan(M, N, K, 1, false).us;
+    return plan->us < (double)n * gemm_plan(M, N, K, 1, 0).us;
 }
 
 CACTI_API int cacti_hip_gemm_chain_kernel_name(int64_t n, int64_t M, int64_t N, int64_t K, char *name, size_t bytes, int *launches)

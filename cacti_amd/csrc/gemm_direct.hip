@@ -890,13 +890,13 @@ double part_cost(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, int s, do
     return fixed + per_tile * (tile_cost(cus, t, M, N, s, per) - fixed) + 4.0 + (x < 4.0 ? 2.0 * x : 4.0 + x);
 }
 
-// `best` in up to kMostParts parts of K on tile t, if that costs less, whichever tile it was on.  A gain of 4 % on the whole product
+// `best` in up to kMostParts parts of K of `lent` bytes at most on tile t, if that costs less, whichever tile it was on.  A gain of 4 % on the whole product
 // (`whole`) is asked of tiles above 128 x 128, whose time per k tile with a part of the CUs is the least certain (1719 x 1024 x 8256
 // 39.2 -> 43.4 us without).
-void split_k(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, double per_tile, double whole, GemmPlan &best)
+void split_k(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, double per_tile, double whole, size_t lent, GemmPlan &best)
 {
     const double margin = kShapes[t].bm * kShapes[t].bn > 128 * 128 ? 1.04 : 1.0;
-    for (int s = 2; s <= kMostParts; s++) {
+    for (int s = 2; s <= kMostParts && gemm_parts_bytes(M, N, s) <= lent; s++) {
         const double c = part_cost(cus, t, M, N, kt, s, per_tile);
         if (c >= 0 && c * margin < whole && c < best.us) best = {t, T64, 0, s, c};
     }
@@ -905,13 +905,13 @@ void split_k(int64_t cus, int t, int64_t M, int64_t N, int64_t kt, double per_ti
 // How a product is cut.  One workgroup takes one tile; a launch runs in sets of resident workgroups, and a nearly empty
 // last set costs as much as a full one.  Considered: every tile shape by itself; for those of one workgroup per CU also the
 // columns of the full sets in one launch and the rest on other tiles in a second (2048 x 8640 x 3200: 256 tiles of 256 x
-// 256 and 448 columns); and, where the caller has a workspace (may_split), up to 8 parts of K for products with fewer
+// 256 and 448 columns); and, where the caller has a workspace (of `lent` bytes at most), up to 8 parts of K for products with fewer
 // tiles than CUs and a long K, whose workgroups would otherwise run 100 k tiles one after another on a fraction of the CUs
 // (37 x 3200 x 8640: 25 tiles of 64 x 64), or on small tiles, whose operands come over and over again from L2.  With parts on tiles
 // to 256 x 256 and not to 128 x 128 alone, us: 2048 x 3200 x 32000 405 -> 371 (2 parts of 256 x 256 against 160 x 192), of 50000
 // 656 -> 544, 2048 x 2048 x 32000 279 -> 215, 1531 x 2048 x 32000 255 -> 171, 1024 x 3200 x 32000 241 -> 192, 319 x 3200 x 27944
 // 113 -> 79; of 1576 products with up to 4000 rows, widths of models and K to 50000 it changes the parts of 36, 3304 -> 2865 us.
-GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split, int shapes = kNumShapes)
+GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, size_t lent, int shapes = kNumShapes)
 {
     const int64_t kt = (K + BK - 1) / BK;
     // A small output has about 64 tiles of 64 x 64 (or one row or column of them), the shape that is best for it while they
@@ -945,9 +945,9 @@ GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, int64_t nz, boo
         }
     }
     best.us = best_cost;
-    if (may_split && nz == 1)
+    if (lent > 0 && nz == 1)
         for (int t = T64; t < kNumShapes; t++)
-            if (has_parts(t)) split_k(cus, t, M, N, kt, 1.0, best_cost, best);
+            if (has_parts(t)) split_k(cus, t, M, N, kt, 1.0, best_cost, lent, best);
     return best;
 }
 
@@ -999,23 +999,24 @@ int gemm_chain_kernel_name(const GemmPlan &plan, char *name, size_t bytes)
 
 // A program has few shapes and calls them over and over; working one out takes some microseconds (hundreds of costs), so
 // each thread keeps the plans of the last ones by their sizes.
-static GemmPlan kept_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split, int chain)
+static GemmPlan kept_plan(int64_t M, int64_t N, int64_t K, int64_t nz, size_t lent, int chain)
 {
     struct Kept {
-        int64_t M, N, K, nz, how;                 // how: compute units, chain and may_split; 0: none kept
+        int64_t M, N, K, nz, how;                 // how: compute units and chain; 0: none kept
+        size_t lent;
         GemmPlan plan;
     };
     static thread_local Kept kept[256] = {};
-    const int64_t cus = device_cus(), how = (cus * 8 + chain) * 2 + (may_split ? 1 : 0);
+    const int64_t cus = device_cus(), how = cus * 8 + chain;
     const uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15u ^ (uint64_t)N * 0xc2b2ae3d27d4eb4fu ^ (uint64_t)K * 0x165667b19e3779f9u) +
-                       (uint64_t)(nz * 2 + (may_split ? 1 : 0) + chain * 64) * 0x27d4eb2f165667c5u;
+                       (uint64_t)(nz * 2 + (lent > 0 ? 1 : 0) + chain * 64) * 0x27d4eb2f165667c5u;
     Kept &k = kept[h >> 56];
-    if (k.how != how || k.M != M || k.N != N || k.K != K || k.nz != nz)
-        k = {M, N, K, nz, how, make_plan(cus, M, N, K * chain, nz, may_split, chain > 1 ? kChainShapes : kNumShapes)};
+    if (k.how != how || k.M != M || k.N != N || k.K != K || k.nz != nz || k.lent != lent)
+        k = {M, N, K, nz, how, lent, make_plan(cus, M, N, K * chain, nz, lent, chain > 1 ? kChainShapes : kNumShapes)};
     return k.plan;
 }
-GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split) { return kept_plan(M, N, K, nz, may_split, 1); }
-GemmPlan gemm_plan_chain(int64_t M, int64_t N, int64_t K, int chain) { return kept_plan(M, N, K, 1, false, chain); }
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, size_t lent) { return kept_plan(M, N, K, nz, lent, 1); }
+GemmPlan gemm_plan_chain(int64_t M, int64_t N, int64_t K, int chain) { return kept_plan(M, N, K, 1, 0, chain); }
 
 GemmPlan gemm_plan_parts(int64_t M, int64_t N, int64_t K, int parts)
 {
@@ -1030,13 +1031,13 @@ GemmPlan gemm_plan_parts(int64_t M, int64_t N, int64_t K, int parts)
 // The same for operands that are loaded through registers whatever their alignment: 64 x 64 tiles, whose k tiles take some
 // half longer than the direct ones' (64 x 128 and 128 x 128 took twice and three times as long as that: their loads have
 // no room in the registers to be far enough ahead).
-GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K)
+GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K, size_t lent)
 {
     const int64_t kt = (K + BK - 1) / BK, cus = device_cus();
     const double fixed = kShapes[T64].fixed;
     GemmPlan best = {T64, T64, 0, 1, 0};
     best.us = fixed + kAnyPerTile * (tile_cost(cus, T64, M, N, 1, kt) - fixed);
-    split_k(cus, T64, M, N, kt, kAnyPerTile, best.us, best);
+    split_k(cus, T64, M, N, kt, kAnyPerTile, best.us, lent, best);
     return best;
 }
 
@@ -1066,9 +1067,7 @@ GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n, size_t lent)
             best.us = us;
         }
     }
-    GemmPlan nn = n > 1 ? gemm_plan_chain(S, K, N, n) : gemm_plan(S, K, N, 1, lent > 0);
-    if ((size_t)nn.split * (size_t)S * (size_t)K * sizeof(float) > lent && nn.split > 1) nn = gemm_plan(S, K, N, 1, false);
-    const GemmPlan tn = gemm_plan(N, K, S, n, false);
+    const GemmPlan nn = n > 1 ? gemm_plan_chain(S, K, N, n) : gemm_plan(S, K, N, 1, lent), tn = gemm_plan(N, K, S, n, 0);
     const double apart = nn.us + tn.us;
     if (apart > 150.0 || best.us >= (apart < 40.0 ? 0.95 : 0.92) * apart) best.tile = -1;
     return best;

@@ -125,15 +125,20 @@ struct GemmPlan {
     int split;           // parts of K
     double us;           // what it is expected to take
 };
-// nz: products of this shape in the launch
-GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, bool may_split);
+// nz: products of this shape in the launch; lent: the largest workspace that the parts of one may take (0: it stays whole)
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, size_t lent);
+inline int64_t gemm_part_pitch(int64_t N) { return (N + 3) / 4 * 4; }            // GemmArgs::ldp
+inline size_t gemm_parts_bytes(int64_t M, int64_t N, int split) { return (size_t)split * (size_t)M * (size_t)gemm_part_pitch(N) * sizeof(float); }
 GemmPlan gemm_plan_parts(int64_t M, int64_t N, int64_t K, int parts);       // in exactly that many parts, 2 .. 8 (tile < 0: K has none)
 GemmPlan gemm_plan_chain(int64_t M, int64_t N, int64_t K, int chain);       // chain <= kMaxPtrBatch products that add up
 // the gradients of n products x W_i^T, x [S,K], W_i [N,K], all in one launch (tile < 0: no better than two, the input gradient of a
 // single product among them with `lent` bytes for parts of K)
 GemmPlan gemm_plan_pair(int64_t S, int64_t N, int64_t K, int n, size_t lent);
 bool gemm_pair_pays(int64_t S, int64_t N, int64_t K, int n, size_t lent);
-GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K);        // for GemmArgs::any (with parts of K)
+// cacti_hip_gemm_f16_ws that asks for no more than `most` bytes, in fewer parts or without a copy if need be
+int gemm_f16_within(size_t most, int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const void *A, int64_t lda, const void *B, int64_t ldb,
+                    float beta, void *C, int64_t ldc, void *ws, size_t ws_bytes, size_t *ws_need, hipStream_t st);
+GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K, size_t lent);        // for GemmArgs::any (with parts of K)
 void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn);
 // the kernel of the plan's (first) launch as a profiler prints it; returns what snprintf does
 int gemm_kernel_name(int ta, int tb, const GemmPlan &plan, char *name, size_t bytes);

@@ -297,8 +297,8 @@ struct MatMulSpec : ThunkSpec {
             size_t need = 0;
             void *ws = nullptr;
             auto product = [&]() {
-                return cacti_hip_gemm_f16_ws(ta, tb, d.M, d.N, d.K, alpha, a[0], d.lda, a[1], d.ldb, (acc & 1) ? 1.f : 0.f, o[0], d.ldc, ws,
-                                             need, &need, S(c));
+                return gemm_f16_within(Ctx::kProductScratch, ta, tb, d.M, d.N, d.K, alpha, a[0], d.lda, a[1], d.ldb, (acc & 1) ? 1.f : 0.f,
+                                       o[0], d.ldc, ws, need, &need, c.stream());
             };
             if ((rc = product()) || need == 0) return rc;
             if ((ws = c.product_scratch(need))) return product();

@@ -55,7 +55,7 @@ SIGNATURES = {
     "cacti_hip_gemm_f16": (ci, [ci, ci, i64, i64, i64, f32, vp, i64, vp, i64, f32, vp, i64, vp]),
     "cacti_hip_gemm_f16_ws": (ci, [ci, ci, i64, i64, i64, f32, vp, i64, vp, i64, f32, vp, i64, vp, sz, C.POINTER(sz), vp]),
     "cacti_hip_gemm_plan": (ci, [i64, i64, i64, i64, C.POINTER(i64)]),
-    "cacti_hip_gemm_plan_ws": (ci, [i64, i64, i64, ci, C.POINTER(i64), C.POINTER(C.c_double)]),
+    "cacti_hip_gemm_plan_ws": (ci, [i64, i64, i64, sz, ci, C.POINTER(i64), C.POINTER(C.c_double)]),
     "cacti_hip_gemm_kernel_name": (ci, [ci, ci, i64, i64, i64, i64, C.c_char_p, sz]),
     "cacti_hip_gemm_f16_batched": (ci, [ci, ci, i64, i64, i64, i64, f32, vp, i64, vp, i64, f32, vp, i64, vp]),
     "cacti_hip_gemm_f16_grads": (ci, [i64, i64, i64, i64, vp, vp, vp, f32, vp, f32, vp, vp]),

@@ -121,9 +121,10 @@ int cacti_hip_gemm_f16_ws(int ta, int tb, int64_t M, int64_t N, int64_t K, float
  * launch): out = rows and columns of the output tile of the first launch, its columns of C, rows and columns of the
  * tile of the second launch, launches (1 or 2). */
 int cacti_hip_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nz, int64_t out[6]);
-/* How one product is cut with a workspace: out = parts of K (1: whole), rows and columns of the (first) launch's tile; us: what it is
- * expected to take.  parts 0: as cacti_hip_gemm_f16_ws cuts it; 1: whole; 2 to 8: in that many (out[0] = 0: K has none). */
-int cacti_hip_gemm_plan_ws(int64_t M, int64_t N, int64_t K, int parts, int64_t out[3], double *us);
+/* How one product is cut with a workspace of up to `lent` bytes: out = parts of K (1: whole), rows and columns of the (first) launch's
+ * tile; us: what it is expected to take.  parts 0: as cacti_hip_gemm_f16_ws cuts it; 1: whole; 2 to 8: in that many, whatever is lent
+ * (out[0] = 0: K has none).  A part takes M rows of N values, N rounded up to 4, of 4 bytes. */
+int cacti_hip_gemm_plan_ws(int64_t M, int64_t N, int64_t K, size_t lent, int parts, int64_t out[3], double *us);
 /* The kernel of the first launch of such a product, as a profiler prints it (a tile shape can have more than one). */
 int cacti_hip_gemm_kernel_name(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t nz, char *name, size_t bytes);
 

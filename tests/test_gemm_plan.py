@@ -72,27 +72,36 @@ def test_a_kernel_name_needs_its_room():
     assert ffi.lib().cacti_hip_gemm_chain_kernel_name(2, 2048, 3200, 8640, name, 128, C.byref(n)) == 0 and n.value == 1
 
 
-def parts_plan(M, N, K, parts=0):
-    """((parts of K, rows and columns of the tile), expected us); parts 0: as a product with a workspace is cut, 1: whole."""
+def parts_plan(M, N, K, parts=0, lent=2 ** 64 - 1):
+    """((parts of K, rows and columns of the tile), expected us); parts 0: as a product with a workspace of `lent` bytes is cut, 1: whole."""
     out, us = (C.c_int64 * 3)(), C.c_double()
-    assert ffi.lib().cacti_hip_gemm_plan_ws(M, N, K, parts, out, C.byref(us)) == 0
+    assert ffi.lib().cacti_hip_gemm_plan_ws(M, N, K, lent, parts, out, C.byref(us)) == 0
     return tuple(out), us.value
 
 
-def test_parts_of_k_are_the_cheapest_that_gain():
-    """Whatever the order in which tiles and numbers of parts are looked at: none of those that gain the 4 % asked of large tiles on the
+@pytest.mark.parametrize("lent", [2 ** 64 - 1, 64 << 20, 1 << 20])
+def test_parts_of_k_are_the_cheapest_that_gain(lent):
+    """Of those that fit in what is lent, whatever the order in which tiles and numbers of parts are looked at: none of those that gain the 4 % asked of large tiles on the
     whole product is expected to take less than the cut that is taken."""
     r = random.Random(5)
     drawn = [(round(33 * (2048 / 33) ** r.random()), 8 * round(32 * (400 / 32) ** r.random()), 8 * round(125 * 32 ** r.random())) for _ in range(1500)]
     split = 0
-    for M, N, K in drawn + [(1378, 768, 19288), (1325, 3200, 24392), (2048, 3200, 32000)]:
-        (parts, _, _), us = parts_plan(M, N, K)
+    for M, N, K in drawn + [(1378, 768, 19288), (1325, 3200, 24392), (2048, 3200, 32000), (2048, 2048, 32000), (2056, 2048, 32000)]:
+        (parts, _, _), us = parts_plan(M, N, K, lent=lent)
+        room = lambda s: s * M * ((N + 3) // 4 * 4) * 4 <= lent
+        assert parts == 1 or room(parts), (M, N, K, parts)
         _, whole = parts_plan(M, N, K, 1)
         assert us <= whole, (M, N, K)
         split += parts > 1
         for s in range(2, 9):
             (n, bm, bn), cost = parts_plan(M, N, K, s)
             assert n in (0, s)
-            if n and cost * 1.04 < whole:
+            if n and room(n) and cost * 1.04 < whole:
                 assert us <= cost, (M, N, K, parts, us, s, bm, bn, cost)
-    assert split > 300
+    assert split > (300 if lent > 1 << 20 else 50)
+
+
+def test_a_product_that_is_lent_too_little_for_its_best_parts_is_cut_into_fewer():
+    for M, N, K, most in ((2056, 2048, 32000, 270), (1325, 3200, 24392, 220)):
+        (parts, _, _), us = parts_plan(M, N, K, lent=64 << 20)
+        assert parts > 1 and us < most, (parts, us)
