@@ -178,9 +178,11 @@ class Ctx {
     int pool_alloc(size_t bytes, size_t *off, bool high = false);                   // with soft-OOM eviction
     size_t pool_try(size_t bytes, bool high = false);            // likewise; kNoOffset and no report when it does not fit
     void pool_free(size_t off) { pool_.free(off); }              // later reuse is ordered on the stream
-    // Device memory beside the pool for the parts of products, so that how a product is cut, and with it its bits, does not depend
+    // Device memory beside the pool for the parts of products, and for their operands laid out anew where those are not 16-byte
+    // aligned, so that how a product is cut, and with it its bits, does not depend
     // on what the pool has room for: taken when the first product asks for it, kept until the context goes.  Thunks run one
-    // after another on the stream, so one serves them all.  Null: beyond kProductScratch, or the device has no more memory.
+    // after another on the stream, so one serves them all.  Null: beyond kProductScratch, or the device has no more memory (the
+    // products are then whole).
     static constexpr size_t kProductScratch = (size_t)64 << 20;
     void *product_scratch(size_t bytes);
     size_t pinned_bytes() const;                                 // of the cells of the running thunk

@@ -252,7 +252,7 @@ struct MatMulSpec : ThunkSpec {
     bool blocked;
     float alpha;
     int causal;
-    bool lend = false;               // a workspace for parts of K (Ctx::product_scratch), where the product asks for one
+    bool lend = false;               // a workspace (Ctx::product_scratch) for parts of K and operands of any alignment, where it asks for one
     MatMulSpec(bool a, bool b, float al, int64_t h, int cz = CAUSAL_NONE)
         : ta(a), tb(b), nblk(h), blocked(h > 0), alpha(al), causal(cz) {}
     const char *name() const override { return blocked ? "block_matmul" : "matmul"; }
@@ -605,7 +605,8 @@ struct ProjNSpec : ThunkSpec {
 
 // ---------------------------------------------------------------------------
 // y = x W^T of a layer: its gradients are one thunk where one launch of both pays (`one`), and it and its input gradient are lent a
-// workspace, the sums of few rows over a long K being the work of a few CUs otherwise: cycles of 48 x 256 (vocabulary 21480) 958 ->
+// workspace, the sums of few rows over a long K being the work of a few CUs otherwise, and rows between 16-byte boundaries (an FFN
+// width that is no multiple of 8: 512 x 1024 x 2815 129 -> 21 us) loaded an element at a time: cycles of 48 x 256 (vocabulary 21480) 958 ->
 // 934 us, 80 x 1024 (29848) 2907 -> 2769, 112 x 768 (31600) 819 -> 758, 160 x 2048 (31432) 1229 -> 1125, 2048 x 3200 (32000, 4
 // layers) 9238 -> 9125.  (Products that have a grouped form are lent
 // none: alone, they have the group's bits.  So has the input gradient where the launch of both would pay.)

@@ -651,3 +651,39 @@ def test_full_depth_step_on_a_16_gib_pool():
         assert len(ref[cyc][1]) >= 12
         for n, g in ref[cyc][1].items():
             assert np.array_equal(g.view(np.uint16), got[cyc][1][n].view(np.uint16)), (cyc, n)
+
+
+# An FFN width that is no multiple of 8: the down projection and its input gradient, which a cycle lends a workspace, take operands
+# and results of any alignment; a K of 22 and of 79 k tiles, the latter in parts
+@pytest.mark.parametrize("S,D,H,F,V", [(256, 512, 8, 1367, 1024), (200, 256, 4, 1373, 512), (40, 256, 4, 5003, 512)])
+def test_ffn_width_of_any_alignment(oracle, S, D, H, F, V):
+    """Loss and every gradient of a cycle, and of a second one that adds to it, inside the oracle's envelope; the bits of the
+    separate thunks in every staging of the products."""
+    from tests.envelope import assert_inside_envelope, order_envelope
+    c = dict(S=S, D=D, H=H, Dh=D // H, F=F, V=V, L=1, eps=1e-6)
+    cfg, flat, tok, lm_tok, scale = make_inputs(c, seed=F, norm_mean=1.0, grad_scale=256.0)
+    _, _, tok2, lm_tok2, _ = make_inputs(c, seed=F + 1, norm_mean=1.0, grad_scale=256.0)
+    print("ffn width", F, flush=True)
+    one = oracle.llama_step(cfg, flat, tok, lm_tok, scale)
+    two = oracle.llama_step(cfg, flat, tok2, lm_tok2, scale, grad_cached=one["grad"])
+    _, env1 = order_envelope(oracle, cfg, flat, tok, lm_tok, scale)
+    _, env2 = order_envelope(oracle, cfg, flat, tok2, lm_tok2, scale, grad_cached=one["grad"])
+    env12 = {t: (env1[t][0] + env2[t][0], env1[t][1] + env2[t][1]) for t in env2}   # two free-running cycles
+    first = None
+    for groups in (0, 1, 2):
+        ctx, m = _model(cfg)
+        m.set_product_groups(groups)
+        m.put_params_flat(flat)
+        loss = m.step(tok, lm_tok, scale)
+        assert_parity(loss, one["loss"], "loss", l2=1e-4, mx=1e-3)
+        got = m.grads()
+        m.step(tok2, lm_tok2, scale, accumulate=True)
+        both = m.grads()
+        m.close(); ctx.close()
+        if first is None:
+            first = (got, both)
+            assert_inside_envelope(got, oracle.split_params(cfg, one["grad"]), env1, "ffn of %d" % F)
+            assert_inside_envelope(both, oracle.split_params(cfg, two["grad"]), env12, "ffn of %d, twice" % F)
+        for name, g in got.items():
+            assert np.array_equal(g.view(np.uint16), first[0][name].view(np.uint16)), (groups, name)
+            assert np.array_equal(both[name].view(np.uint16), first[1][name].view(np.uint16)), (groups, name)
