@@ -687,3 +687,23 @@ def test_ffn_width_of_any_alignment(oracle, S, D, H, F, V):
         for name, g in got.items():
             assert np.array_equal(g.view(np.uint16), first[0][name].view(np.uint16)), (groups, name)
             assert np.array_equal(both[name].view(np.uint16), first[1][name].view(np.uint16)), (groups, name)
+
+
+# Sequences that the forward kernel of whole tiles takes (more than 1024 positions and 512 workgroups of 32 of them), heads of one and
+# of two 64-column halves
+@pytest.mark.parametrize("S,H,Dh", [(1100, 16, 64), (1060, 16, 72)])
+def test_two_layers_of_a_long_sequence(oracle, S, H, Dh):
+    """What one layer's attention rounds goes through the next layer's: loss and gradients of two layers inside the oracle's envelope."""
+    from tests.envelope import assert_loss_inside_envelope, order_envelope
+    D = H * Dh
+    cfg, flat, tok, lm_tok, scale = make_inputs(dict(S=S, D=D, H=H, Dh=Dh, F=512, V=1024, L=2, eps=1e-6), seed=3, norm_mean=1.0,
+                                                grad_scale=1024.0)
+    print("two layers", S, H, Dh, flush=True)
+    ref = oracle.llama_step(cfg, flat, tok, lm_tok, scale)
+    _, env = order_envelope(oracle, cfg, flat, tok, lm_tok, scale, count=8)
+    print("envelope measured", flush=True)
+    ctx, m = _model(cfg, pool_bytes=4 << 30)
+    m.put_params_flat(flat)
+    assert_loss_inside_envelope(m.step(tok, lm_tok, scale), ref["loss"], env, "two layers")
+    _compare(oracle, cfg, m, ref, env, "two layers")
+    m.close(); ctx.close()
