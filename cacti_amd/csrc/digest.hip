@@ -6,10 +6,10 @@
 // Both stream the tensor once, 16 bytes per lane per step, and counting has to keep up with 6 TB/s: 8 elements per lane in
 // some 40 clocks of its SIMD.  An LDS add per element, into the dozen adjacent bins that the values of a weight or gradient
 // tensor fall into, did not (3.7 TB/s), nor did one per pair of elements (4.0).  So a lane counts in registers: 16 counters of
-// four bits, for 16 neighbouring classes (Window), take 8 elements before they move to bytes, and those go to LDS once per 31
-// steps, summed over the wave.  Where a wave's 16 classes lie its first elements say (the largest, and one class more); pieces of 8
-// elements with one beyond them, a zero among others or a NaN, one in a hundred of a normally distributed tensor, are
-// counted in LDS, by pairs: the two exponent fields of a 32-bit word are one of 1024 bins, so there are half as many adds and
+// four bits, for 16 neighbouring classes (Window), take 8 elements before they move to bytes, and those go to LDS once per 28
+// pieces, summed over the wave.  Where a wave's 16 classes lie its first elements say (the largest, and one class more); pieces of 8
+// elements with one beyond them, a zero among others or a NaN, one in 820 to 1130 of a normally distributed tensor (a wave has one
+// in 13 to 18 of its steps), are counted in LDS, by pairs: the two exponent fields of a 32-bit word are one of 1024 bins, so there are half as many adds and
 // they spread over a hundred addresses (four sets of bins, by lane & 3).  What an exponent field does not say, the
 // subnormals' highest mantissa bit and the NaNs, is looked for in two halves at a time there and counted apart where there is
 // any; zeros are the zero exponents that were not subnormal.  At the end of a workgroup the pairs are summed to exponents and
@@ -126,7 +126,7 @@ __device__ __forceinline__ Window window_for(uint32_t largest)
 }
 
 // A lane's counters: byte j of by[0], by[1] counts classes 2 j and 2 j + 8 modulo 16 of the f32 exponent, of by[2], by[3] the ones behind.
-// At most 31 pieces of 8 go in before they are flushed.
+// At most 31 pieces of 8 fit in (28: kUnroll at a time) before they are flushed.
 struct LaneCounts {
     uint32_t by[4], zeros;
 };

@@ -123,14 +123,14 @@ def test_batched_digests_match_the_oracle_bit_for_bit(ops, oracle):
 
 
 @pytest.mark.gpu
-def test_digests_where_a_wave_counts_in_registers(ops):
-    """One class throughout (counters that run as full as they get: 16 sweeps of 1024 pieces, two workgroups at the least number
-    of sweeps each), for each of the 40 classes; and first elements of one class with the classes at and beyond the edges of the
+@pytest.mark.parametrize("n", [65536 + 3, 2 * 65536 + 8 * 300 + 3])
+def test_digests_where_a_wave_counts_in_registers(ops, n):
+    """One class throughout, for each of the 40 classes (one workgroup of 8 sweeps of 1024 pieces, whose counters run as full as they
+    get, 28 pieces a lane, and begin again; and workgroups of 6, 5 and 5); and first elements of one class with the classes at and beyond the edges of the
     16 that a wave then counts in registers behind them, zeros, subnormals and NaNs among them."""
     import torch
     r = rng(23)
     least = [1 << c if c < 10 else (c - 9) << 10 for c in range(40)]
-    n = 2 * 65536 + 8 * 300 + 3
     xs = []
     for c, b in enumerate(least):
         top = (least[c + 1] if c < 39 else 0x7c00) - 1
@@ -155,3 +155,25 @@ def test_digests_where_a_wave_counts_in_registers(ops):
         assert int(c[i]) == int(np.isnan(x.view(np.float16)).sum())
     alone = ops.abs_log2_hist8(ds[-1]).cpu().numpy()
     assert np.array_equal(alone, h[-1])
+
+
+@pytest.mark.gpu
+def test_digests_of_long_walks(ops):
+    """16 sweeps to a workgroup and more, so that full counters move twice and begin a third time: one class throughout, and two that
+    share the counters of a byte's neighbours."""
+    import torch
+    n = 4 * torch.cuda.get_device_properties(0).multi_processor_count * 16 * 8192 + 5 * 8192 + 11
+    least = [1 << c if c < 10 else (c - 9) << 10 for c in range(40)]
+    for c in (1, 9, 10, 24, 25, 39):
+        for second in (c, c - 1):
+            print("digest walk", n, c, second, flush=True)
+            x = torch.full((n,), least[c], dtype=torch.int16, device="cuda")
+            x[1::2] = least[second]
+            pair = np.array([least[c], least[second]], np.uint16)
+            bins = bins_from_values(pair)
+            want = np.zeros(256, np.int64)
+            want[bins[0]] += (n + 1) // 2
+            want[bins[1]] += n // 2
+            h, nans = (t.cpu().numpy() for t in ops.digests([x.view(torch.float16)]))
+            assert np.array_equal(h[0], want) and int(nans[0]) == 0
+            assert np.array_equal(ops.abs_log2_hist8(x.view(torch.float16)).cpu().numpy(), want)
