@@ -161,6 +161,14 @@ struct RmsNormDwSpec : ThunkSpec {
         *of = {args[(size_t)i]};
         return std::unique_ptr<ThunkSpec>(new RmsNormDwSpec({ty[(size_t)i]}));
     }
+    // launches of another number of sums are others; ",acc" and the outputs that are added to, in hexadecimal
+    std::string key(const std::vector<CellType> &aty, uint32_t acc) const override
+    {
+        char buf[96], mode[16] = "";
+        if (acc) snprintf(mode, sizeof(mode), ",acc%x", acc);
+        snprintf(buf, sizeof(buf), "rms_norm_dw[%lldx%lld%s]x%zu", (long long)aty[0].shape[0], (long long)aty[0].shape[1], mode, ty.size());
+        return buf;
+    }
 };
 
 // dx (+)= and the partial rows of dw now, their sum with those of the norms to come

@@ -139,6 +139,25 @@ def test_norm_gradients_summed_together(oracle, L, thunks):
     m.close(); ctx.close()
 
 
+def test_sums_of_another_number_of_norms_are_timed_apart():
+    """17 norms are a launch of 16 and one of 1: a label each, whose bytes are those of its launches (G partial rows of D values, f32,
+    read and D written, f16, by each sum; read as well where they are added to)."""
+    cfg, flat, tok, lm_tok, scale = make_inputs(dict(S=41, D=64, H=2, Dh=32, F=176, V=256, L=8, eps=1e-6), seed=8, norm_mean=1.0)
+    ctx, m = _model(cfg)
+    m.put_params_flat(flat)
+    ctx.set_timing(2)
+    m.step(tok, lm_tok, scale)
+    m.step(tok, lm_tok, scale, accumulate=True)
+    ctx.sync()
+    rep = {k: v for k, v in ctx.timing_report().items() if k.startswith("rms_norm_dw")}
+    G = 6                                                   # eight rows to a workgroup of the adjoint
+    assert {k: (n, ctx.operand_bytes[k]) for k, (n, _) in rep.items()} == {
+        "rms_norm_dw[%dx64]x16" % G: (1, 16 * (G * 256 + 128)), "rms_norm_dw[%dx64]x1" % G: (1, G * 256 + 128),
+        "rms_norm_dw[%dx64,accffff]x16" % G: (1, 16 * (G * 256 + 256)), "rms_norm_dw[%dx64,acc1]x1" % G: (1, G * 256 + 256)}
+    ctx.set_timing(0)
+    m.close(); ctx.close()
+
+
 @pytest.mark.parametrize("S,V", [(64, 8192), (37, 4104)])
 def test_products_in_parts_of_k(oracle, S, V):
     """The head's input gradient and the FFN's last product as sums of parts (one to two tiles of 64 x 64, K of 640 to 8192, a k tile
