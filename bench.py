@@ -85,8 +85,8 @@ def gemm_traffic_bytes(label, table):
     return None if ent is None else float(ent["bytes"])
 
 
-# "...]x3": three products of that shape staged as one thunk and launched together
-GEMM_RE = re.compile(r"^(block_matmul|matmul)\[([NT])([NT]),(\d+)x(\d+)x(\d+)x(\d+)(,acc)?\](?:x(\d+))?$")
+# "...]x3": three products of that shape staged as one thunk and launched together; ",parts2": one in two parts of K
+GEMM_RE = re.compile(r"^(block_matmul|matmul)\[([NT])([NT]),(\d+)x(\d+)x(\d+)x(\d+)(,acc)?(,parts\d+)?\](?:x(\d+))?$")
 
 # both gradients of x [S,K] W^T, W [N,K], of that many W in one launch
 GRADS_RE = re.compile(r"^matmul_grads\[(\d+)x(\d+)x(\d+)(,acc[0-9a-f]+)?\]x(\d+)$")
@@ -94,7 +94,12 @@ GRADS_RE = re.compile(r"^matmul_grads\[(\d+)x(\d+)x(\d+)(,acc[0-9a-f]+)?\]x(\d+)
 
 def gemm_group(label):
     m = GEMM_RE.match(label)
-    return int(m.group(9) or 1) if m else 1
+    return int(m.group(10) or 1) if m else 1
+
+
+def gemm_parts(label):
+    m = GEMM_RE.match(label)
+    return int(m.group(9)[6:]) if m and m.group(9) else 1
 
 
 def gemm_flops(label):
@@ -126,11 +131,14 @@ def gemm_dims(label):
 def gemm_launches(label):
     """(kernel instantiation of the first launch as rocprofv3 prints it, launches) of a label of dense products of 16-byte
     aligned operands: one product, a group of independent ones, or a chain of input gradients (the groups of that layout).
-    A launch more takes the columns beyond the full rounds of the first one's tiles.  ("", 0): several launches by another rule."""
+    A launch more takes the columns beyond the full rounds of the first one's tiles, or adds up parts of K ("": no name looked up).
+    ("", 0): several launches by another rule."""
     import ctypes as C
     from cacti_amd import ffi
     ta, tb, H, M, N, K = gemm_dims(label)
     n, acc = gemm_group(label), ",acc" in label
+    if gemm_parts(label) > 1:
+        return "", 2
     name = C.create_string_buffer(128)
     if n > 1 and not ta and not tb:
         count = C.c_int(0)
@@ -545,7 +553,7 @@ def run_gemm_traffic(args):
     expects in the counter files of a rocprofv3 --pmc run over this workload."""
     import ctypes as C
     import torch
-    from cacti_amd import ffi, gemm_traffic
+    from cacti_amd import ffi, gemm_traffic, ops
     g = torch.Generator(device="cuda").manual_seed(0)
     rn = lambda *s: (torch.randn(*s, device="cuda", generator=g) * 0.05).half()
     st = torch.cuda.current_stream().cuda_stream
@@ -554,13 +562,15 @@ def run_gemm_traffic(args):
     for label in gemm_traffic.STEP_PRODUCTS:
         ta, tb, _, M, N, K = gemm_dims(label)
         k = gemm_group(label)
-        chain = k > 1 and not ta and not tb
+        chain, parts = k > 1 and not ta and not tb, gemm_parts(label)
         # forward the group shares its input (A), the weight gradients share it as B; a chain shares its output
         a = [rn(K, M) if ta else rn(M, K) for _ in range(1 if tb else k)] * (k if tb else 1)
         b = [rn(N, K) if tb else rn(K, N) for _ in range(1 if ta else k)] * (k if ta else 1)
         out = [rn(M, N) for _ in range(1 if chain else k)]
         for _ in range(gemm_traffic.LAUNCHES):
-            if chain:
+            if parts > 1:
+                ops.gemm(a[0], b[0], ta=ta, tb=tb, out=out[0])           # (which lends a workspace)
+            elif chain:
                 ffi.call("cacti_hip_gemm_f16_chain", k, M, N, K, table(a), K, table(b), N, 0.0, out[0].data_ptr(), N, st)
             else:
                 ffi.call("cacti_hip_gemm_f16_batched", int(ta), int(tb), k, M, N, K, 1.0, table(a), M if ta else K, table(b), K if tb else N,

@@ -415,6 +415,13 @@ int gemm_f16_within(size_t most, int ta, int tb, int64_t M, int64_t N, int64_t K
 {
     return gemm_run(ta, tb, 1, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, 0, most, ws, ws_bytes, ws_need, st);
 }
+
+int gemm_parts_within(size_t most, int ta, int tb, int64_t M, int64_t N, int64_t K, bool acc)
+{
+    if (!mult(N, 8) || !mult(ta ? M : K, 8) || !mult(tb ? K : N, 8) || (ta ? M : K) >= kMaxPitch || (tb ? K : N) >= kMaxPitch) return 1;
+    if (!ta && tb && M <= 4 && !acc) return 1;                    // a stream over B
+    return gemm_plan(M, N, K, 1, most).split;
+}
 }  // namespace cacti
 
 CACTI_API int cacti_hip_gemm_f16_ws(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const void *A, int64_t lda,

@@ -138,6 +138,8 @@ bool gemm_pair_pays(int64_t S, int64_t N, int64_t K, int n, size_t lent);
 // cacti_hip_gemm_f16_ws that asks for no more than `most` bytes, in fewer parts or without a copy if need be
 int gemm_f16_within(size_t most, int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const void *A, int64_t lda, const void *B, int64_t ldb,
                     float beta, void *C, int64_t ldc, void *ws, size_t ws_bytes, size_t *ws_need, hipStream_t st);
+// the parts of K that it takes of whole matrices that begin on 16 bytes (1: whole, or rows between 16-byte boundaries)
+int gemm_parts_within(size_t most, int ta, int tb, int64_t M, int64_t N, int64_t K, bool acc);
 GemmPlan gemm_plan_any(int64_t M, int64_t N, int64_t K, size_t lent);        // for GemmArgs::any (with parts of K)
 void gemm_tile_dims(int tile, int64_t *bm, int64_t *bn);
 // the kernel of the plan's (first) launch as a profiler prints it; returns what snprintf does

@@ -321,10 +321,13 @@ struct MatMulSpec : ThunkSpec {
     {
         Dims d;
         if (dims(aty, d)) return name();
-        char buf[128];
-        snprintf(buf, sizeof(buf), "%s[%c%c,%lldx%lldx%lldx%lld%s]", name(), ta ? 'T' : 'N',
+        // ",parts2": in two parts of K, a launch of the parts and one of their sum
+        char buf[128], parts[16] = "";
+        const int split = lend && !blocked ? gemm_parts_within(Ctx::kProductScratch, ta, tb, d.M, d.N, d.K, acc & 1) : 1;
+        if (split > 1) snprintf(parts, sizeof(parts), ",parts%d", split);
+        snprintf(buf, sizeof(buf), "%s[%c%c,%lldx%lldx%lldx%lld%s%s]", name(), ta ? 'T' : 'N',
                  tb ? 'T' : 'N', (long long)d.H, (long long)d.M, (long long)d.N, (long long)d.K,
-                 (acc & 1) ? ",acc" : "");
+                 (acc & 1) ? ",acc" : "", parts);
         return buf;
     }
     std::unique_ptr<ThunkSpec> mm(bool x, bool y, int cz = CAUSAL_NONE) const

@@ -23,12 +23,12 @@ LAUNCHES = 4
 FETCH_FACTOR, WRITE_FACTOR = 2.0, 1.0
 
 # timing labels of the dense products of one 3B-shaped step (S = 2048, D = 3200, F = 8640, V = 32000); "]x3": a group in one thunk,
-# of the NN layout a chain that adds up in one output
+# of the NN layout a chain that adds up in one output; ",parts2": in two parts of K and their sum
 STEP_PRODUCTS = [
     "matmul[NT,1x2048x3200x3200]", "matmul[NT,1x2048x3200x3200]x3", "matmul[NT,1x2048x8640x3200]x2", "matmul[NT,1x2048x3200x8640]",
     "matmul[NT,1x2048x32000x3200]",
     "matmul[NN,1x2048x3200x3200]", "matmul[NN,1x2048x3200x3200]x3", "matmul[NN,1x2048x3200x8640]x2", "matmul[NN,1x2048x8640x3200]",
-    "matmul[NN,1x2048x3200x32000]",
+    "matmul[NN,1x2048x3200x32000,parts2]",
     "matmul[TN,1x3200x3200x2048]", "matmul[TN,1x3200x3200x2048]x3", "matmul[TN,1x8640x3200x2048]x2", "matmul[TN,1x3200x8640x2048]",
     "matmul[TN,1x32000x3200x2048]",
 ]
@@ -54,14 +54,14 @@ def _dispatches(path):
     rows = []
     with open(path) as f:
         for r in csv.DictReader(f):
-            if "gemm_direct_kernel" in r["Kernel_Name"] or "gemm_chain_kernel" in r["Kernel_Name"]:
+            if any(k in r["Kernel_Name"] for k in ("gemm_direct_kernel", "gemm_chain_kernel", "gemm_part_kernel", "reduce_parts_kernel")):
                 rows.append((int(r["Dispatch_Id"]), float(r["Counter_Value"]), r["Kernel_Name"]))
     rows.sort()
     return rows
 
 
 def build(fetch_csv, write_csv, launches_per_product):
-    """launches_per_product: {label: 1 or 2} (2: the columns beyond the full rounds go to a second kernel)."""
+    """launches_per_product: {label: 1 or 2} (2: the columns beyond the full rounds go to a second kernel, or parts of K are added up by one)."""
     f, w = _dispatches(fetch_csv), _dispatches(write_csv)
     want = sum(LAUNCHES * launches_per_product[l] for l in STEP_PRODUCTS)
     assert len(f) == want and len(w) == want, "expected %d GEMM dispatches, found %d / %d" % (want, len(f), len(w))

@@ -46,6 +46,7 @@ def test_kernel_names_tell_the_kernels_of_one_tile_shape_apart(M, N, K, how):
                                           ("matmul[NN,1x128x256x256]x3", "gemm_chain_kernel<64, 64, 2, true>"),
                                           ("matmul[TN,1x3200x3200x2048]x3", "gemm_direct_kernel<true, false, 256, 256, 1, false, false>"),
                                           ("matmul[TN,1x8640x3200x2048]x2", None),
+                                          ("matmul[NN,1x2048x3200x32000,parts2]", None), ("matmul[NN,1x2048x3200x8640]", "gemm_direct_kernel<false, false, 160, 192, 1, false, false>"),
                                           ("matmul[NN,1x2048x3200x8640,acc]x2", None), ("matmul[NN,1x600x1000x1004]x2", None),
                                           ("matmul_grads[611x1024x1024]x3", None), ("block_matmul[NT,32x2048x2048x100]", None)])
 def test_the_kernel_of_a_group_or_a_chain(label, kernel):
@@ -105,3 +106,14 @@ def test_a_product_that_is_lent_too_little_for_its_best_parts_is_cut_into_fewer(
     for M, N, K, most in ((2056, 2048, 32000, 270), (1325, 3200, 24392, 220)):
         (parts, _, _), us = parts_plan(M, N, K, lent=64 << 20)
         assert parts > 1 and us < most, (parts, us)
+
+
+def test_the_products_of_the_traffic_table_are_cut_as_their_labels_say():
+    """In a training cycle, which lends 64 MiB to what has no grouped form and is no weight gradient."""
+    import bench
+    from cacti_amd.gemm_traffic import STEP_PRODUCTS
+    for label in STEP_PRODUCTS:
+        ta, tb, _, M, N, K = bench.gemm_dims(label)
+        lent = 0 if ta or bench.gemm_group(label) > 1 else 64 << 20
+        assert parts_plan(M, N, K, lent=lent)[0][0] == bench.gemm_parts(label), label
+        assert bench.gemm_launches(label)[1] in (1, 2) and bench.gemm_flops(label) == 2.0 * M * N * K * bench.gemm_group(label)

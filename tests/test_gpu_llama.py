@@ -158,22 +158,27 @@ def test_sums_of_another_number_of_norms_are_timed_apart():
     m.close(); ctx.close()
 
 
-@pytest.mark.parametrize("S,V", [(64, 8192), (37, 4104)])
-def test_products_in_parts_of_k(oracle, S, V):
-    """The head's input gradient and the FFN's last product as sums of parts (one to two tiles of 64 x 64, K of 640 to 8192, a k tile
-    that ends inside K): every gradient no further from the oracle than its own other summation orders are, the same bits from
-    every staging of the products and in a pool that spills (the two V x 64 weights, their gradients and nothing else fit)."""
+@pytest.mark.parametrize("S,V,D,F", [(64, 8192, 64, 648), (37, 4104, 64, 648), (40, 8192, 256, 3080)])
+def test_products_in_parts_of_k(oracle, S, V, D, F):
+    """The head's input gradient, and the last time the FFN's last product, as sums of parts (one to four tiles of 64 x 64, K of 3080 to
+    8192, a k tile that ends inside K): every gradient no further from the oracle than its own other summation orders are, the same bits from
+    every staging of the products and in a pool that spills (the two V x D weights, their gradients and nothing else fit)."""
     from tests.envelope import order_envelope
-    cfg, flat, tok, lm_tok, scale = make_inputs(dict(S=S, D=64, H=2, Dh=32, F=648, V=V, L=1, eps=1e-6), seed=S, norm_mean=1.0,
+    cfg, flat, tok, lm_tok, scale = make_inputs(dict(S=S, D=D, H=D // 32, Dh=32, F=F, V=V, L=1, eps=1e-6), seed=S, norm_mean=1.0,
                                                 grad_scale=64.0)
     ref = oracle.llama_step(cfg, flat, tok, lm_tok, scale)
     _, env = order_envelope(oracle, cfg, flat, tok, lm_tok, scale)
     want, first = oracle.split_params(cfg, ref["grad"]), None
-    for groups, pool in ((2, 1 << 30), (1, 1 << 30), (0, 1 << 30), (2, 512 * V)):
+    for groups, pool in ((2, 1 << 30), (1, 1 << 30), (0, 1 << 30), (2, 8 * D * V)):
         ctx, m = _model(cfg, pool_bytes=pool)
         m.set_product_groups(groups)
         m.put_params_flat(flat)
+        ctx.set_timing(2)
         assert_parity(m.step(tok, lm_tok, scale), ref["loss"], "loss", l2=1e-4, mx=1e-3)
+        ctx.sync()
+        labels = list(ctx.timing_report())
+        for name, K in (("NN", V), ("NT", F))[:1 if F == 648 else 2]:           # their labels say so
+            assert any(l.startswith("matmul[%s,1x%dx%dx%d,parts" % (name, S, D, K)) for l in labels), labels
         got = m.grads()
         if pool < 1 << 30:
             assert ctx.stats()["n_evict"] > 0
