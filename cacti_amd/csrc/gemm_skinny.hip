@@ -332,10 +332,9 @@ gemm_skinny_nt_kernel(SkinnyArgs p)
 }
 
 // The arg max of each row from the workgroups' candidates, in out_tok; the last row's token is added to in_tok[pos]
-// (pos < 0: nowhere), src/librarium/llama.rs:953-959.  One workgroup and a chain of latencies: a lane's candidates (8000 of a
-// vocabulary of 32000: eight each) are requested together; 32 tokens of 3
-// layers of 3200 6980 -> 6933 us, 16 of 4 layers of 2048 behind 1531 3786 -> 3760.
-constexpr int kFinish = 8;
+// (pos < 0: nowhere), src/librarium/llama.rs:953-959.  One workgroup and a chain of latencies.  (A lane's candidates
+// requested together, eight of a vocabulary of 32000: no difference, 4.42 and 4.44 us behind 3 layers of 3200, 4.13 and 4.04 behind
+// 4 of 2048 where traces of one kernel differ by 0.2.)
 __global__ void __launch_bounds__(1024)
 finish_rows_kernel(int M, int count, const uint32_t *__restrict__ cand, uint16_t *out_tok, uint16_t *in_tok, int64_t pos)
 {
@@ -343,15 +342,8 @@ finish_rows_kernel(int M, int count, const uint32_t *__restrict__ cand, uint16_t
     // (read up front: behind the arg max it would be one more round trip to memory)
     const uint16_t before = threadIdx.x == 0 && pos >= 0 ? in_tok[pos] : 0;
     for (int m = 0; m < M; m++) {
-        const uint32_t *c = cand + (int64_t)m * count;
         uint32_t k = 0;
-        for (int i = threadIdx.x; i < count; i += kFinish * 1024) {
-            uint32_t v[kFinish];
-#pragma unroll
-            for (int j = 0; j < kFinish; j++) v[j] = c[min(i + j * 1024, count - 1)];      // (the last one again behind the row)
-#pragma unroll
-            for (int j = 0; j < kFinish; j++) k = max(k, v[j]);
-        }
+        for (int i = threadIdx.x; i < count; i += 1024) k = max(k, cand[(int64_t)m * count + i]);
         k = wave_reduce(k, [](uint32_t a, uint32_t b) { return max(a, b); });
         __syncthreads();
         if ((threadIdx.x & 63) == 0) best[threadIdx.x >> 6] = k;
