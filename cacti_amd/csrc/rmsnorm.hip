@@ -196,12 +196,12 @@ rms_norm_bwd_kernel(int64_t N, int D, const half_t *__restrict__ x, const half_t
 
 // dw[d] (+)= f16(sum over block partials): a block owns 32 columns (8 lanes x float4) and
 // splits the partial rows over 32 slices, so D / 32 blocks share the read of the partials.  A lane's rows, up to 8 of them, are
-// requested together, as the launch is a chain of latencies (256 rows of 3200 4.6 -> 4.3 us, 77 of 1024 4.6 -> 4.2; norms,
-// rotation and gate of 2048 rows in both directions 98.5 -> 96.9).
+// requested together, as the launch is a chain of latencies (256 rows of 3200 4.59 -> 4.25 us, 98 of 2048 4.4 either way; norms,
+// rotation and gate of 2048 rows in both directions 98.5 -> 97.0).
 constexpr int kFinCols = 32, kFinSlices = 32, kFinRows = 8;
 // The weights' gradients that a launch sums, one to a row of its grid: a training cycle's norms together, as each sum alone is all
-// latency (two micro-batches of 611 positions, 4 layers of 1024, 18 launches -> 2: 2680 -> 2637 us; 128 positions, 2 layers of
-// 256: 699 -> 686).
+// latency (two micro-batches of 611 positions, 4 layers of 1024: 18 launches of 4.25 us -> 2 of 4.0; 128 positions, 2 layers of
+// 256: 5 of 2.5 -> 1 of 2.8; runs of the whole cycles differ by more than that).
 struct DwSums {
     const float *part[kRmsNormDwSums];
     half_t *dw[kRmsNormDwSums];

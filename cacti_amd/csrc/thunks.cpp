@@ -617,9 +617,10 @@ struct ProjNSpec : ThunkSpec {
 // ---------------------------------------------------------------------------
 // y = x W^T of a layer: its gradients are one thunk where one launch of both pays (`one`), and it and its input gradient are lent a
 // workspace, the sums of few rows over a long K being the work of a few CUs otherwise, and rows between 16-byte boundaries (an FFN
-// width that is no multiple of 8: 512 x 1024 x 2815 129 -> 21 us) loaded an element at a time: cycles of 48 x 256 (vocabulary 21480) 958 ->
-// 934 us, 80 x 1024 (29848) 2907 -> 2769, 112 x 768 (31600) 819 -> 758, 160 x 2048 (31432) 1229 -> 1125, 2048 x 3200 (32000, 4
-// layers) 9238 -> 9125.  (Products that have a grouped form are lent
+// width that is no multiple of 8: 512 x 1024 x 2815 129 -> 21 us) loaded an element at a time: the head's
+// input gradient of 48 x 256 (vocabulary 21480) 66 -> 16 us, 80 x 1024 (29848) 93 -> 21, 112 x 768 (31600) 114 -> 22, 160 x 2048 (31432)
+// 156 -> 51, 611 x 1024 (8192) 32 -> 23, 2048 x 3200 (32000) 352 -> 316, and cycles of one layer around them 240 -> 200, 360 -> 283,
+// 356 -> 266, 659 -> 527, 311 -> 299, 2906 -> 2849.  (Products that have a grouped form are lent
 // none: alone, they have the group's bits.  So has the input gradient where the launch of both would pay.)
 struct LinearSpec : MatMulSpec {
     bool one;

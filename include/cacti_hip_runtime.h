@@ -44,7 +44,12 @@ typedef struct {
  * 1377-2002.  pool_bytes = 0 reserves 90.01 % of the device (src/ctx.rs:43); otherwise the
  * cap in bytes (the CACTI_VMEM_SOFT_LIMIT analogue, src/pctx/nvgpu.rs:1434-1463).  The pool
  * is ONE hipMalloc; when it is exhausted live cells are spilled to host memory
- * (_try_soft_oom, src/pctx/nvgpu.rs:2004-2283) and re-uploaded on their next use.
+ * (_try_soft_oom, src/pctx/nvgpu.rs:2004-2283) and re-uploaded on their next use.  Beside the
+ * pool, the first training cycle with a product that gains from parts of K, or whose operands are
+ * not 16-byte aligned, takes 64 MiB of device memory, kept until the context is destroyed; where
+ * the device has no more, these products are as they are without.  In the pool, up to 32 MiB of
+ * partial rows of norm gradients wait during a backward pass to be summed together; they are
+ * cells like any other, and spill like them.
  * host_pagelocked: 1 = hipHostMalloc, 0 = malloc (CACTI_NVGPU_MEM_ALLOC, :995-1002),
  * -1 = what the environment says (cacti_env_host_pagelocked).  With pool_bytes = 0 the
  * environment variable CACTI_VMEM_SOFT_LIMIT, when set, gives the reserve
