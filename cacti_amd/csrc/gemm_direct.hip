@@ -808,11 +808,13 @@ int launch_pair(const PairArgs &args, int64_t nblk, hipStream_t st)
 // The tiles of a pair, both products' the same.
 constexpr int kPairShapes[] = {T64_SMALL, 0, 3, 5, 7};     // 64 x 64 twice, 64 x 128, 128 x 128, 160 x 128
 
-// The tiles that parts of K are formed on.  The others would be expected to take 0.2 % less in the mean (10 % at most) of the
-// products that have parts.
+// The tiles that parts of K are formed on.  Of 87 products that 160 x 64 or 64 x 128 are the best for, by the costs by 2 % only, these
+// take 2642 us and the next best of the others 2893 (3320 x 136 x 10176 28 and 34).  128 x 128 with two workgroups to a CU is not among
+// them: where the costs put it first by 2 % it takes 6 % longer than the next (122 products; 214 x 3872 x 13944 46 and 39).  The
+// remaining ones would be expected to take 0.1 % less in the mean.
 constexpr bool has_parts(int tile)
 {
-    for (int t : {0, 1, 4, 6, 7, 9, 12, 13})
+    for (int t : {0, 1, 2, 3, 4, 6, 7, 9, 12, 13})
         if (t == tile) return true;
     return false;
 }

@@ -102,6 +102,13 @@ def test_parts_of_k_are_the_cheapest_that_gain(lent):
     assert split > (300 if lent > 1 << 20 else 50)
 
 
+@pytest.mark.parametrize("size,cut", [((3320, 136, 10176), (8, 160, 64)), ((2953, 136, 12288), (8, 160, 64)), ((319, 1248, 19240), (5, 64, 128)),
+                                      ((109, 2264, 14936), (7, 64, 128))])
+def test_parts_on_long_narrow_tiles(size, cut):
+    """Few columns or few rows over a long K: 28 and 25 us, 34 and 27 on the tiles that are next by the costs."""
+    assert parts_plan(*size)[0] == cut
+
+
 def test_a_product_that_is_lent_too_little_for_its_best_parts_is_cut_into_fewer():
     for M, N, K, most in ((2056, 2048, 32000, 270), (1325, 3200, 24392, 220)):
         (parts, _, _), us = parts_plan(M, N, K, lent=64 << 20)

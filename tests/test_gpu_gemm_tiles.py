@@ -132,12 +132,23 @@ def test_parts_of_k(M, N, K):
     check(A, B, False, True, ops.gemm(A, B, tb=True))
 
 
-# parts on 96 x 64, 128 x 128, 96 x 128, 160 x 128, 160 x 192, 192 x 256 and 256 x 256 tiles (256 compute units), with rows, columns and
-# a K that no tile divides
+# a product for each tile that parts are formed on but 64 x 64 (above), with rows, columns and a K that no tile divides
+PARTS = [((1001, 520, 8200), (96, 64)), ((3321, 136, 10184), (160, 64)), ((109, 2264, 14936), (64, 128)), ((400, 808, 20000), (96, 128)),
+         ((227, 1656, 12664), (128, 128)), ((600, 1000, 16008), (160, 128)), ((520, 2008, 20000), (160, 128)), ((1184, 1352, 7048), (160, 192)),
+         ((1500, 1000, 12008), (192, 256)), ((1505, 3208, 20000), (256, 256))]
+
+
+def test_every_tile_of_parts_is_some_product_s():
+    """(No GPU: the device is taken to have 256 CUs then.)"""
+    out, us = (C.c_int64 * 3)(), C.c_double()
+    for size, tile in PARTS:
+        ffi.call("cacti_hip_gemm_plan_ws", *size, 2 ** 64 - 1, 0, out, C.byref(us))
+        assert out[0] > 1 and tuple(out[1:]) == tile, (size, list(out))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
-@pytest.mark.parametrize("M,N,K", [(1001, 520, 8200), (600, 1000, 16008), (400, 808, 20000), (520, 2008, 20000), (1184, 1352, 7048), (1500, 1000, 12008),
-                                   (1505, 3208, 20000)])
+@pytest.mark.parametrize("M,N,K", [size for size, _ in PARTS])
 def test_parts_of_k_on_large_tiles(M, N, K, ta, tb):
     if ta:
         M = (M + 7) // 8 * 8
