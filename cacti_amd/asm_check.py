@@ -139,10 +139,18 @@ def _check_function(name, instrs, out):
                 fault(i, b, "a load into LDS follows its address too early")
 
 
-def check(text, spills=True, fused=True):
+def check(text, spills=True, fused=True, registers=()):
     """The faults found in an assembly file, as texts; `spills`, `fused`: also registers kept in memory, and products rounded
-    to half in the instruction that forms them (v_fma_mixlo / mixhi: one rounding where the sources have two)."""
+    to half in the instruction that forms them (v_fma_mixlo / mixhi: one rounding where the sources have two); `registers`: pairs of
+    a pattern and the vector registers, of both files, that a kernel whose name it is found in may have (a CU holds one workgroup of
+    four waves less for them otherwise).  A pattern that no kernel has is a fault as well."""
     out, name, lines = [], None, []
+    used = re.findall(r"^\s*\.amdhsa_kernel (\S+)$.*?^\s*\.amdhsa_next_free_vgpr (\d+)$", text, re.M | re.S) if registers else []
+    for pattern, most in registers:
+        seen = [(k, int(n)) for k, n in used if re.search(pattern, k)]
+        out += ["%s: %d registers, %d at most" % (k, n, most) for k, n in seen if n > most]
+        if not seen:
+            out.append("no kernel is named like %s" % pattern)
     for nr, line in enumerate(text.splitlines(), 1):
         m = re.match(r"^([A-Za-z_$][\w$]*):", line)
         if m:

@@ -28,6 +28,8 @@ FLAGS = [
 # Sources with matrix instructions or loads into LDS in inline assembly: what the compiler made of them is checked.  In
 # gemm_direct.hip, whose kernels hold all of a wave's registers, a spill and a product rounded only once are faults too.
 CHECKED = ("attention.hip", "attention_short.hip", "gemm_direct.hip", "gemm_mfma.hip")
+# kernels of which a CU is to hold four workgroups: the products of many tiles and operands of any alignment
+REGISTERS = {"gemm_direct.hip": [(r"gemm_part_kernel.*Lb1EEEv", 128)]}
 
 
 def sources():
@@ -47,7 +49,8 @@ def _compile(src):
         if len(asm) != 1:
             raise RuntimeError("%s: no assembly to check among %s" % (src, sorted(os.listdir(tmp))))
         with open(os.path.join(tmp, asm[0])) as f:
-            faults = asm_check.check(f.read(), spills=src == "gemm_direct.hip", fused=src == "gemm_direct.hip")
+            faults = asm_check.check(f.read(), spills=src == "gemm_direct.hip", fused=src == "gemm_direct.hip",
+                                     registers=REGISTERS.get(src, ()))
         if faults:
             raise RuntimeError("%s: %d faults around inline assembly\n%s" % (src, len(faults), "\n".join(faults[:20])))
         shutil.move(made, obj)

@@ -93,7 +93,10 @@ __device__ __forceinline__ void load_odd(half_t *lds, const half_t *c, int64_t l
 // next product's tiles on their way while the last one's are multiplied.  Launches apart cost a start and an end each (3.7 us
 // with 64 x 64, 5.7 with 160 x 192), the sum's way through memory and the gap between them: three of 611 x 1024 x 1024 21.0 ->
 // 14.2 us, of 777 x 2048 x 2048 41.0 -> 31.6, of 2048 x 3200 x 3200 132 -> 114; two of 2048 x 3200 x 8640 199 -> 195.
-// PART: the sums of a range of k tiles, as fp32 (split_k).
+// PART: the sums of a range of k tiles, as fp32 (split_k).  With ANY also whole products (p.part null), those of more than three
+// workgroups to a CU: with this branch the compiler stays at 128 registers, of which a CU holds four (asm_check.py sees to it), and
+// takes 136 to 148 without.  1201 x 3001 x 65 8.9 us on three of those, 8.3 on four of these; 509 x 1003 x 770 in three layouts, one
+// to a CU, 23.7 and 24.4.
 template <bool TA, bool TB, int BM, int BN, int RES, bool M32, bool ANY, bool CHAIN, bool PART>
 __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
 {
@@ -108,6 +111,7 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
     constexpr bool TR_A = TA, TR_B = !TB;                         // fragments by transposing reads
     constexpr int NA = BM / 32, NB = BN / 32;                     // fragments of a wave
     static_assert(!PART || (!M32 && !CHAIN), "parts of one product");
+    const bool in_parts = PART && (!ANY || p.part);
     static_assert(!CHAIN || (!ANY && D <= 4), "the first D tiles are of the first product");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     half_t *As = reinterpret_cast<half_t *>(smem_raw);            // [NBA][BM * BK]
@@ -120,7 +124,7 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
     const int product = nk;                                       // CHAIN: k tiles of one
     if constexpr (CHAIN) nk *= p.chain;
     const int part = bz;
-    if constexpr (PART) {
+    if (in_parts) {
         // the "blocks of the batch" are the parts of K: the same operands, a range of k tiles each
         const int per = p.split_tiles;
         kt0 = part * per;
@@ -499,7 +503,7 @@ __device__ __forceinline__ void gemm_direct_tile(const GemmArgs &p, uint32_t wg)
     }
     sums_done();
 
-    if constexpr (PART) {
+    if (in_parts) {
         // a lane's 4 consecutive columns of a row are 16 bytes of the part, four lanes a 64-byte run
         float *out = p.part + part * p.M * p.ldp;
 #pragma unroll
@@ -853,6 +857,8 @@ int launch_shape(int shape, const GemmArgs &p, int64_t nblk, hipStream_t st, std
             return rc;
         }
     if (shape == T64_SMALL) return launch<TA, TB, 64, 64, 2, true>(p, nblk, st);
+    if (p.any && (p.M + 63) / 64 * ((p.N + 63) / 64) * nblk > 3 * (int64_t)device_cus())
+        return launch<TA, TB, 64, 64, 2, false, true, false, true>(p, nblk, st);
     if (p.any) return launch<TA, TB, 64, 64, 2, false, true>(p, nblk, st);
     int rc = CACTI_E_STATE;
     (void)((shape == I && (rc = launch<TA, TB, kShapes[I].bm, kShapes[I].bn, kShapes[I].res>(p, nblk, st), true)) || ...);

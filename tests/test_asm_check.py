@@ -71,3 +71,10 @@ def test_one_mistake_is_found(what, old, new, text):
         assert faults == []
     else:
         assert faults and text in faults[0], faults
+
+
+def test_kernels_that_hold_more_registers_than_they_may():
+    text = GOOD + "\t.amdhsa_kernel kernel\n\t\t.amdhsa_next_free_vgpr 136\n\t.end_amdhsa_kernel\n"
+    assert asm_check.check(text, registers=[("kern", 136)]) == []
+    assert asm_check.check(text, registers=[("kern", 128)]) == ["kernel: 136 registers, 128 at most"]
+    assert asm_check.check(text, registers=[("other", 128)]) == ["no kernel is named like other"]

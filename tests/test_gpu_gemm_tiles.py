@@ -101,7 +101,7 @@ def test_small_outputs(M, N, K, ta, tb):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
-@pytest.mark.parametrize("M,N,K", [(9, 11, 65), (509, 1003, 770), (130, 4099, 131), (1999, 3001, 203)])
+@pytest.mark.parametrize("M,N,K", [(9, 11, 65), (509, 1003, 770), (130, 4099, 131), (1999, 3001, 203), (1535, 2047, 75), (1537, 2047, 75)])
 def test_products_of_any_alignment(M, N, K, ta, tb):
     A, B, a, b = operands(M, N, K, ta, tb)
     old = torch.randn(M, N, device="cuda", dtype=torch.float16)
